@@ -581,6 +581,22 @@ int loken_moe_gemm_gguf_down_reduce_static(const float* inputs, const void* weig
                                            const float* topk_weights, float* outputs, int num_experts,
                                            int topk, int size_m, int size_n, int size_k, int gguf_dtype,
                                            const float* down_bias, const float* add_after, void* stream);
+/* A mixture layer's expert block in one call: out[t] = sum over the token's choices j of topk_weights[t, j] *
+ * down_e (silu(gate_e . x[t]) * (up_e . x[t])), e = choices[t, j]; f32 rows x [tokens, hidden] and out [tokens,
+ * hidden], stacks gate / up [experts, ffn, hidden] of wtype_gu and down [experts, hidden, ffn] of wtype_down, choices
+ * int32 and weights f32 [tokens, topk]. The launches are those of the entry points above, chosen by size as the layer
+ * code of the reference chooses (src/inference/generic_transformer/moe_weights.rs:2118-2152). LK_ERR_TYPE: a format
+ * the path does not take; LK_ERR_NOMEM: the scratch would have to grow while the stream records a graph. */
+int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
+                   const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
+                   int hidden, int ffn, void* stream);
+/* The rules it chooses by: whether the expert-batched launches pay at `rows` routed rows (wtype: the stacks' type where
+ * all have the same, else -1); the longest run an expert is expected to own (mmq_experts.rs:215-227); whether a stack
+ * then takes lk_moe_q4k_rows_grouped. */
+int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype);
+int lk_moe_longest_run(int tokens, int topk, int n_experts);
+int lk_moe_rows_launch_pays(int wtype, int k, int longest_run);
+
 /* outputs[t, c] += sum over k ascending of pairs[(t * topk + k), c] (cuda/moe/moe_gguf.cu:745-752). */
 void loken_moe_sum_topk(const float* pairs, float* outputs, int tokens, int topk, int cols, void* stream);
 /* Q4_K weight [size_n rows, size_k] x plain Q8_1 rows [size_m, size_k / 32 blocks] -> output

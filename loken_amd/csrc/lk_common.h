@@ -226,6 +226,26 @@ template <> __device__ __forceinline__ float to_f32<float>(float v) { return v; 
 template <> __device__ __forceinline__ float to_f32<__half>(__half v) { return __half2float(v); }
 template <> __device__ __forceinline__ float to_f32<__hip_bfloat16>(__hip_bfloat16 v) { return __bfloat162float(v); }
 
+// Four consecutive values as f32 from an address aligned to four of them.
+template <typename T> struct Load4;
+template <> struct Load4<float> {
+    static __device__ __forceinline__ float4 at(const float* p) { return *(const float4*)p; }
+};
+template <> struct Load4<__half> {
+    static __device__ __forceinline__ float4 at(const __half* p) {
+        const uint2 raw = *(const uint2*)p;
+        const __half2 a = *(const __half2*)&raw.x, b = *(const __half2*)&raw.y;
+        return make_float4(__low2float(a), __high2float(a), __low2float(b), __high2float(b));
+    }
+};
+template <> struct Load4<__hip_bfloat16> {
+    static __device__ __forceinline__ float4 at(const __hip_bfloat16* p) {
+        const uint2 raw = *(const uint2*)p;
+        return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u),
+                           __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u));
+    }
+};
+
 // Host side: device facts fetched once.
 struct LkDevice {
     int cus;

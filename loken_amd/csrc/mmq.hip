@@ -26,6 +26,7 @@
 // MFMA (v_mfma_f32_32x32x2_f32) straight into the accumulators, costing no per-element VALU.
 
 #include "mmq_problem.h"
+#include "moe_block.h"
 #include "legacy_blocks.h"
 #include "codebook_blocks.h"
 
@@ -40,26 +41,10 @@ constexpr int REC_BYTES = MMQ_REC_BYTES;
 // --------------------------------------------------------------------------------------------
 // Activation quantizer -> workspace records
 // --------------------------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void mmq_quantize_kernel(const T* __restrict__ x,
-                                                           const int32_t* __restrict__ ids,
-                                                           uint8_t* __restrict__ vy, int64_t ne00,
-                                                           int64_t s01, int64_t s02, int64_t s03,
-                                                           int64_t ne0, int ne1, int ne2) {
+// Four consecutive values (value i0 of row `row` and the three after it) into the row's record: the eight
+// lanes of a 32-value block call it together.
+static __device__ __forceinline__ void put_record_quad(float4 v, uint8_t* rec, int in_rec) {
 #pragma clang fp contract(off)
-    const int64_t i0 = ((int64_t)blockIdx.y * 256 + threadIdx.x) * 4;
-    if (i0 >= ne0) return;
-    const int row = blockIdx.x;
-    const int64_t channel = blockIdx.z % ne2, sample = blockIdx.z / ne2;
-    const int64_t src_row = ids ? ids[row] : row;
-    const T* xr = x + sample * s03 + channel * s02 + src_row * s01;
-
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i0 + 0 < ne00) v.x = to_f32<T>(xr[i0 + 0]);
-    if (i0 + 1 < ne00) v.y = to_f32<T>(xr[i0 + 1]);
-    if (i0 + 2 < ne00) v.z = to_f32<T>(xr[i0 + 2]);
-    if (i0 + 3 < ne00) v.w = to_f32<T>(xr[i0 + 3]);
-
     float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
     amax = max8(amax);
     const float d = amax / 127.0f;
@@ -68,11 +53,6 @@ __global__ __launch_bounds__(256) void mmq_quantize_kernel(const T* __restrict__
     const int q2 = (int)roundf(v.z * inv), q3 = (int)roundf(v.w * inv);
     int quad_sum;
     const int sum = sum8(q0 + q1 + q2 + q3, quad_sum);
-
-    const int64_t kb = i0 / 256;
-    const int64_t blocks_per_channel = (ne0 / 256) * ne1;
-    uint8_t* rec = vy + ((int64_t)blockIdx.z * blocks_per_channel + kb * ne1 + row) * REC_BYTES;
-    const int in_rec = (int)(i0 % 256);
     *(uint32_t*)(rec + in_rec) = (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) |
                                  ((uint32_t)(q2 & 0xFF) << 16) | ((uint32_t)(q3 & 0xFF) << 24);
     if ((in_rec & 31) == 0) {
@@ -80,6 +60,51 @@ __global__ __launch_bounds__(256) void mmq_quantize_kernel(const T* __restrict__
         *(uint16_t*)(rec + 256 + 2 * s) = __half_as_ushort(__float2half_rn(d));
         *(int16_t*)(rec + 272 + 2 * s) = (int16_t)sum;
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void mmq_quantize_kernel(const T* __restrict__ x,
+                                                           const int32_t* __restrict__ ids,
+                                                           uint8_t* __restrict__ vy, int64_t ne00,
+                                                           int64_t s01, int64_t s02, int64_t s03,
+                                                           int64_t ne0, int ne1, int ne2) {
+    const int64_t i0 = ((int64_t)blockIdx.y * 256 + threadIdx.x) * 4;
+    if (i0 >= ne0) return;
+    const int row = blockIdx.x;
+    const int64_t channel = blockIdx.z % ne2, sample = blockIdx.z / ne2;
+    const int64_t src_row = ids ? ids[row] : row;
+    const T* xr = x + sample * s03 + channel * s02 + src_row * s01;
+
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i0 + 3 < ne00 && ((uintptr_t)(xr + i0) & (4 * sizeof(T) - 1)) == 0) {
+        v = Load4<T>::at(xr + i0);
+    } else {
+        if (i0 + 0 < ne00) v.x = to_f32<T>(xr[i0 + 0]);
+        if (i0 + 1 < ne00) v.y = to_f32<T>(xr[i0 + 1]);
+        if (i0 + 2 < ne00) v.z = to_f32<T>(xr[i0 + 2]);
+        if (i0 + 3 < ne00) v.w = to_f32<T>(xr[i0 + 3]);
+    }
+
+    const int64_t kb = i0 / 256;
+    const int64_t blocks_per_channel = (ne0 / 256) * ne1;
+    put_record_quad(v, vy + ((int64_t)blockIdx.z * blocks_per_channel + kb * ne1 + row) * REC_BYTES, (int)(i0 % 256));
+}
+
+// The rows silu(gate) * up of an expert block's gate and up products (gu: [rows][gate | up], `width` a multiple
+// of 32) straight into the records: the row in f32 is never written. width padded to 512 as the plain form's rows
+// are. 8888 rows of 768: 13.6 us (62 MB, 4.6 TB/s) where the activation's launch and the quantizer's took 25.1.
+__global__ __launch_bounds__(256) void mmq_quantize_gated_kernel(const float* __restrict__ gu, uint8_t* __restrict__ vy,
+                                                                 int width, int width_padded, int rows) {
+    const int i0 = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (i0 >= width_padded) return;
+    const int row = blockIdx.x;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i0 < width) {
+        const float4 g = *(const float4*)(gu + (int64_t)row * 2 * width + i0), u = *(const float4*)(gu + (int64_t)row * 2 * width + width + i0);
+        v = make_float4(g.x / (1.0f + expf(-g.x)) * u.x, g.y / (1.0f + expf(-g.y)) * u.y, g.z / (1.0f + expf(-g.z)) * u.z,
+                        g.w / (1.0f + expf(-g.w)) * u.w);
+    }
+    put_record_quad(v, vy + ((int64_t)(i0 / 256) * rows + row) * REC_BYTES, i0 % 256);
 }
 
 static void launch_quantize(const void* x, const int32_t* ids, void* vy, int type_x, int64_t ne00,
@@ -1074,6 +1099,14 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
 }
 
 }  // namespace
+
+int lk_mmq_quantize_gated(const float* gu, void* y, int64_t rows, int width, hipStream_t s) {
+    if (!gu || !y || rows <= 0 || rows > INT32_MAX || width <= 0 || width % 32 != 0 || (uintptr_t)gu % 16 != 0) return LK_ERR_ARG;
+    const int padded = (width + 511) / 512 * 512;
+    hipLaunchKernelGGL(mmq_quantize_gated_kernel, dim3((unsigned)rows, (unsigned)((padded + 1023) / 1024)), dim3(256), 0, s, gu,
+                       (uint8_t*)y, width, padded, (int)rows);
+    return lk_launch_status();
+}
 
 int lk_mmq_split_sum(const float* part, int splits, const MmqProblem& pb, hipStream_t s) {
     const int64_t count = (int64_t)pb.m_end * pb.n;

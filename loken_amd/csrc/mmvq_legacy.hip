@@ -385,7 +385,7 @@ __global__ __launch_bounds__(LWG) void moe_rows_legacy_kernel(const uint8_t* __r
     const int pair = blockIdx.y;
     // the pair's routing and the live count in one round of scalar loads, the launch's fields in the
     // round before it (asked for where each is first used they arrive in many dependent rounds)
-    const int slot = sorted_token_ids[pair];
+    const int slot = sorted_token_ids ? sorted_token_ids[pair] : pair;
     const int e = expert_ids[pair];
     const unsigned int live = d.live != nullptr ? *d.live : 0xFFFFFFFFu;
     asm volatile("" ::"s"(slot), "s"(e), "s"(live), "s"(d.pairs), "s"(d.experts), "s"(d.cols), "s"(d.nb), "s"(d.k32),

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
 // output row (the conventions of loken_moe_gemm_gguf_gate_up_silu_mul, cuda/moe/moe_gguf.cu:896-1060
 // of the reference). Everything else is the pair kernel above.
 struct RegMoeArgs {
-    const int32_t* sorted_token_ids;
+    const int32_t* sorted_token_ids;   // null: pair i is slot i
     const int32_t* expert_ids;
     int experts, topk, pairs;
     int64_t slab_bytes;
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_moe_pair_kernel(const uint8_t* __r
 #pragma clang fp contract(off)
     __shared__ __align__(16) uint8_t lds[LDS_BYTES];
     const int pair = blockIdx.y;
-    const int slot = m.sorted_token_ids[pair], e = m.expert_ids[pair];
+    const int slot = m.sorted_token_ids ? m.sorted_token_ids[pair] : pair, e = m.expert_ids[pair];
     asm volatile("" ::"s"(slot), "s"(e), "s"(m.pairs), "s"(m.experts), "s"(m.topk), "s"(m.slab_bytes), "s"(gate), "s"(up),
                  "s"(acts), "s"(out), "s"(nb), "s"(n), "s"(waves), "s"(m.act.kind));
     if (slot < 0 || slot >= m.pairs || e < 0 || e >= m.experts) return;   // a pair the routing leaves out writes nothing

@@ -1,0 +1,22 @@
+// The steps of a mixture layer's expert block as lk_moe_forward (moe_forward.hip) puts them together: the
+// same launches the exported entry points make, with what only a caller of both halves can ask for.
+#pragma once
+
+#include "lk_common.h"
+
+// loken_moe_gemm_gguf_gate_up_silu_mul / loken_moe_gemm_gguf_down_reduce over pairs in slot order: pair i is
+// slot i of expert choices[i], so no sorted routing is needed, and the down side writes `out` instead of
+// adding to it. `wire`: the format's id of the reference's table.
+int lk_moe_pairs_gate_up(int wire, const float* x, const void* gate, const void* up, const int32_t* choices, float* h, int experts,
+                         int topk, int pairs, int ffn, int hidden, hipStream_t s);
+int lk_moe_pairs_down(int wire, const float* h, const void* down, const int32_t* choices, const float* weights, float* out,
+                      int experts, int topk, int pairs, int hidden, int ffn, hipStream_t s);
+
+// Groups the router's choices by expert (moe_mmq.hip): counts [experts] (nullable), bounds [experts + 1], slots and src_rows [n].
+int lk_moe_route(const int32_t* choices, int n, int topk, int experts, int32_t* counts, int32_t* bounds, int32_t* slots,
+                 int32_t* src_rows, hipStream_t s);
+// out[t] = sum over the token's slots of weights[slot] * pairs[slot]
+int lk_moe_fold_write(const float* pairs, const float* weights, float* out, int64_t tokens, int topk, int cols, hipStream_t s);
+// silu(gu[:, :width]) * gu[:, width:] of every row into the tile kernels' workspace (mmq.hip): the activation
+// and the quantizer in one pass, same bytes as the two one after the other.
+int lk_mmq_quantize_gated(const float* gu, void* y, int64_t rows, int width, hipStream_t s);

@@ -14,6 +14,8 @@
 // host path does (src/inference/moe_cuda_cpu/mod.rs:598).
 
 #include "mmvq_core.h"
+#include "moe_block.h"
+#include "stream_scratch.h"
 
 #include <mutex>
 #include <unordered_map>
@@ -26,51 +28,22 @@ extern "C" int lk_quantize_q8_1(const void* x, int x_type, void* vy, int kx, int
 int lk_moe_down_fold(int quant_type, const float* inputs, const void* weights, const int32_t* sorted_token_ids,
                      const int32_t* expert_ids, const float* topk_weights, float* outputs, int num_experts, int topk,
                      int size_m, int size_n, int size_k, const float* down_bias, const float* add_after,
-                     hipStream_t stream);
+                     bool write, hipStream_t stream);
 
 namespace {
 
-// ---------------------------------------------------------------- stream scratch
+// ---------------------------------------------------------------- stream scratch (stream_scratch.h)
 struct ScratchSlot {
     int device;
     hipStream_t stream;
+    LkScratchUse use;
     void* ptr = nullptr;
     size_t size = 0;
     std::vector<void*> kept;  // outgrown buffers: queued kernels may still read them
 };
-std::mutex g_scratch_mu;
 std::vector<ScratchSlot> g_scratch;
 
-// Caller holds g_scratch_mu from the reservation until its launches are on the stream: the
-// buffer belongs to the stream, and another thread's quantize landing between a launcher's
-// two kernels is what the second would then read.
-void* reserve_scratch(size_t bytes, hipStream_t stream) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    ScratchSlot* slot = nullptr;
-    for (auto& s : g_scratch)
-        if (s.device == dev && s.stream == stream) slot = &s;
-    if (!slot) {
-        g_scratch.push_back(ScratchSlot{dev, stream});
-        slot = &g_scratch.back();
-    }
-    if (slot->size >= bytes) return slot->ptr;
-    // growing allocates, which a stream under capture may not do
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return nullptr;
-    (void)hipGetLastError();
-    size_t want = bytes + bytes / 4;
-    want = (want + 255) & ~(size_t)255;
-    void* fresh = nullptr;
-    if (hipMalloc(&fresh, want) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (slot->ptr) slot->kept.push_back(slot->ptr);
-    slot->ptr = fresh;
-    slot->size = want;
-    return fresh;
-}
+void* reserve_scratch(size_t bytes, hipStream_t stream) { return lk_reserve_scratch(bytes, stream, LK_SCRATCH_LAUNCHER); }
 
 // ---------------------------------------------------------------- static scratch
 // Scratch of the entry point that allocates nothing (loken_moe_gemm_gguf_down_reduce_static): a
@@ -124,7 +97,7 @@ __global__ __launch_bounds__(WG) void moe_rows_kernel(const uint8_t* __restrict_
     const int pair = blockIdx.y;
     // The pair's routing and the live count in ONE round of scalar loads, and the launch's fields in
     // the round before it: asked for where each is first used they arrive in eight dependent rounds.
-    const int slot = sorted_token_ids[pair];
+    const int slot = sorted_token_ids ? sorted_token_ids[pair] : pair;
     const int e = expert_ids[pair];
     const unsigned int live = d.live != nullptr ? *d.live : 0xFFFFFFFFu;
     asm volatile("" ::"s"(slot), "s"(e), "s"(live), "s"(d.pairs), "s"(d.experts), "s"(d.cols), "s"(d.nb), "s"(d.k32),
@@ -163,13 +136,13 @@ __global__ __launch_bounds__(WG) void moe_rows_kernel(const uint8_t* __restrict_
 }
 
 // outputs[t] (+)= sum over k ascending of pairs[t * topk + k]; with `add` the result is written
-// as fold + add instead of accumulated (cuda/moe/moe_gguf.cu:591-625).
+// as fold + add instead of accumulated (cuda/moe/moe_gguf.cu:591-625), with `write` as the fold alone.
 __global__ void sum_topk_kernel(const float* __restrict__ pairs, const float* __restrict__ add,
-                                float* __restrict__ outputs, int tokens, int topk, int cols) {
+                                float* __restrict__ outputs, int tokens, int topk, int cols, int write) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)tokens * cols) return;
     const size_t token = i / cols, col = i % cols;
-    float acc = add ? 0.0f : outputs[i];
+    float acc = add || write ? 0.0f : outputs[i];
     const float* p = pairs + token * topk * cols + col;
     // four rows' loads in flight at a time; the additions stay in k order
     int k = 0;
@@ -282,6 +255,39 @@ static inline bool rows_stage_as_f32(const float* inputs, int size_k, int quant_
 
 }  // namespace
 
+std::recursive_mutex& lk_scratch_mutex() {
+    static std::recursive_mutex mu;
+    return mu;
+}
+
+void* lk_reserve_scratch(size_t bytes, hipStream_t stream, LkScratchUse use) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    ScratchSlot* slot = nullptr;
+    for (auto& s : g_scratch)
+        if (s.device == dev && s.stream == stream && s.use == use) slot = &s;
+    if (!slot) {
+        g_scratch.push_back(ScratchSlot{dev, stream, use});
+        slot = &g_scratch.back();
+    }
+    if (slot->size >= bytes) return slot->ptr;
+    // growing allocates, which a stream under capture may not do
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return nullptr;
+    (void)hipGetLastError();
+    size_t want = bytes + bytes / 4;
+    want = (want + 255) & ~(size_t)255;
+    void* fresh = nullptr;
+    if (hipMalloc(&fresh, want) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (slot->ptr) slot->kept.push_back(slot->ptr);
+    slot->ptr = fresh;
+    slot->size = want;
+    return fresh;
+}
+
 void lk_mmq_q4k_wide_release(int device);   // mmq_q4k_wide.hip: the token-side operand buffers of the wide Q4_K tiles
 
 extern "C" void loken_stream_scratch_release() {
@@ -289,7 +295,7 @@ extern "C" void loken_stream_scratch_release() {
     if (hipGetDevice(&dev) != hipSuccess) return;
     (void)hipDeviceSynchronize();   // queued kernels may still read what is freed below
     lk_mmq_q4k_wide_release(dev);
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
     for (auto it = g_scratch.begin(); it != g_scratch.end();) {
         if (it->device != dev) { ++it; continue; }
         if (it->ptr) (void)hipFree(it->ptr);
@@ -302,7 +308,7 @@ extern "C" void loken_moe_sum_topk(const float* pairs, float* outputs, int token
     if (tokens <= 0 || cols <= 0) return;
     const size_t total = (size_t)tokens * cols;
     hipLaunchKernelGGL(sum_topk_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, pairs,
-                       (const float*)nullptr, outputs, tokens, topk, cols);
+                       (const float*)nullptr, outputs, tokens, topk, cols, 0);
     (void)hipGetLastError();
 }
 
@@ -323,7 +329,7 @@ extern "C" int loken_moe_gemm_gguf(const float* inputs, const void* weights, con
         return launch_format<MODE_PLAIN>(quant_type, (const uint8_t*)weights, nullptr, (const uint8_t*)inputs,
                                          sorted_token_ids, expert_ids, topk_weights, nullptr, (float*)outputs, d, size_k, s);
     }
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
     uint8_t* acts = (uint8_t*)reserve_scratch((size_t)act_rows * (kp / 32) * Q81_BYTES, s);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, LK_TYPE_F32, acts, size_k, kp, act_rows, stream)) return rc;
@@ -353,7 +359,7 @@ extern "C" int loken_moe_gemm_gguf_prefill(const void* inputs, const uint8_t* we
     hipStream_t s = (hipStream_t)stream;
     const int kp = pad512(size_k);
     const int act_rows = topk_weights ? size_m : size_m / topk;
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
     uint8_t* acts = (uint8_t*)reserve_scratch((size_t)act_rows * (kp / 32) * Q81_BYTES, s);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, input_dtype == 0 ? LK_TYPE_F16 : LK_TYPE_BF16, acts, size_k, kp, act_rows, stream))
@@ -364,14 +370,16 @@ extern "C" int loken_moe_gemm_gguf_prefill(const void* inputs, const uint8_t* we
 }
 
 // The gated launch: act(gate . x, up . x) per routed pair. `slab_rows` = weight rows per expert in
-// both stacks (size_n, or 2 size_n when `up_weights` points size_n rows into the gate's tensor).
+// both stacks (size_n, or 2 size_n when `up_weights` points size_n rows into the gate's tensor). `identity`:
+// no sorted_token_ids, pair i is slot i.
 static int gate_up_impl(const float* inputs, const void* gate_weights, const void* up_weights,
                         const int32_t* sorted_token_ids, const int32_t* expert_ids, float* outputs, int num_experts,
                         int topk, int size_m, int size_n, int size_k, int quant_type, const LkGateAct& act,
-                        int slab_rows, void* stream, const unsigned int* live = nullptr, const LkMoeAlt& alt = LkMoeAlt{}) {
+                        int slab_rows, void* stream, const unsigned int* live = nullptr, const LkMoeAlt& alt = LkMoeAlt{},
+                        bool identity = false) {
     if (block_len_of_wire(quant_type) == 0) return LK_ERR_TYPE;
     if (size_m == 0) return LK_OK;
-    if (!inputs || !gate_weights || !up_weights || !sorted_token_ids || !expert_ids || !outputs ||
+    if (!inputs || !gate_weights || !up_weights || (!sorted_token_ids && !identity) || !expert_ids || !outputs ||
         bad_shape(quant_type, num_experts, topk, size_m, size_n, size_k)) return LK_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
     const int kp = pad512(size_k), act_rows = size_m / topk;
@@ -389,7 +397,7 @@ static int gate_up_impl(const float* inputs, const void* gate_weights, const voi
                                          (const uint8_t*)inputs, sorted_token_ids, expert_ids, nullptr, nullptr, outputs,
                                          d, size_k, s);
     }
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
     uint8_t* acts = (uint8_t*)reserve_scratch((size_t)act_rows * (kp / 32) * Q81_BYTES, s);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, LK_TYPE_F32, acts, size_k, kp, act_rows, stream)) return rc;
@@ -475,30 +483,31 @@ __global__ void zero_f32_kernel(float* __restrict__ p, size_t n) {
     if (i < n) p[i] = 0.f;
 }
 
+// `identity`: no sorted_token_ids, pair i is slot i. `write`: the sums replace what `outputs` holds.
 // Down per routed pair, then the fold over a token's pairs; with `pair_rows` the weighted rows go to
 // the caller's [size_m, size_n] buffer and the sum is the caller's (cuda/moe/moe_gguf.cu:755-820).
 static int down_impl(const float* inputs, const void* weights, const int32_t* sorted_token_ids,
                      const int32_t* expert_ids, const float* topk_weights, float* outputs, int num_experts, int topk,
                      int size_m, int size_n, int size_k, int gguf_dtype, const float* down_bias,
                      const float* add_after, const unsigned int* live, float* pair_rows, void* stream,
-                     const LkMoeAlt& alt = LkMoeAlt{}, bool from_static = false) {
+                     const LkMoeAlt& alt = LkMoeAlt{}, bool from_static = false, bool identity = false, bool write = false) {
     if (block_len_of_wire(gguf_dtype) == 0) return LK_ERR_TYPE;
     if (size_m == 0) return LK_OK;
-    if (!inputs || !weights || !sorted_token_ids || !expert_ids || !topk_weights || (!outputs && !pair_rows) ||
+    if (!inputs || !weights || (!sorted_token_ids && !identity) || !expert_ids || !topk_weights || (!outputs && !pair_rows) ||
         bad_shape(gguf_dtype, num_experts, topk, size_m, size_n, size_k)) return LK_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
     // a handful of tokens over short K-quant rows: one launch that needs no pair rows at all (the entry
     // point that allocates nothing keeps the two launches over its fixed array)
     if (!from_static && !live && !pair_rows && !alt.alt0 && !alt.alt_at) {
         const int rc = lk_moe_down_fold(gguf_dtype, inputs, weights, sorted_token_ids, expert_ids, topk_weights, outputs,
-                                        num_experts, topk, size_m, size_n, size_k, down_bias, add_after, s);
+                                        num_experts, topk, size_m, size_n, size_k, down_bias, add_after, write, s);
         if (rc >= 0) return rc;
     }
     const int kp = pad512(size_k);
     const bool as_f32 = rows_stage_as_f32(inputs, size_k, gguf_dtype);
     const size_t act_bytes = as_f32 ? 0 : (((size_t)size_m * (kp / 32) * Q81_BYTES) + 255) & ~(size_t)255;
     const size_t pair_bytes = pair_rows ? 0 : (size_t)size_m * size_n * sizeof(float);
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
     uint8_t* base = nullptr;
     if (from_static) {
         // nothing is allocated: the device's fixed array, or an error when the call does not fit it
@@ -529,8 +538,20 @@ static int down_impl(const float* inputs, const void* weights, const int32_t* so
     const int tokens = size_m / topk;
     const size_t total = (size_t)tokens * size_n;
     hipLaunchKernelGGL(sum_topk_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, (const float*)pairs,
-                       add_after, outputs, tokens, topk, size_n);
+                       add_after, outputs, tokens, topk, size_n, write ? 1 : 0);
     return lk_launch_status();
+}
+
+int lk_moe_pairs_gate_up(int wire, const float* x, const void* gate, const void* up, const int32_t* choices, float* h, int experts,
+                         int topk, int pairs, int ffn, int hidden, hipStream_t s) {
+    return gate_up_impl(x, gate, up, nullptr, choices, h, experts, topk, pairs, ffn, hidden, wire, LkGateAct{}, 0, s, nullptr,
+                        LkMoeAlt{}, true);
+}
+
+int lk_moe_pairs_down(int wire, const float* h, const void* down, const int32_t* choices, const float* weights, float* out,
+                      int experts, int topk, int pairs, int hidden, int ffn, hipStream_t s) {
+    return down_impl(h, down, nullptr, choices, weights, out, experts, topk, pairs, hidden, ffn, wire, nullptr, nullptr, nullptr,
+                     nullptr, s, LkMoeAlt{}, false, true, true);
 }
 
 extern "C" int loken_moe_gemm_gguf_down_reduce(const float* inputs, const void* weights,
@@ -628,7 +649,7 @@ extern "C" int loken_moe_q4k_imma_m8_down(const void* weights, const void* q8_1,
     if (!weights || !q8_1 || !sorted_token_ids || !expert_ids || !topk_weights || !output ||
         bad_shape(1, num_experts, topk, size_m, hidden, size_k) || (((uintptr_t)q8_1) & 3) != 0) return LK_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
     float* pairs = (float*)reserve_scratch((size_t)size_m * hidden * sizeof(float), s);
     if (!pairs) return LK_ERR_NOMEM;
     // a pair whose slot is out of range writes nothing: its row of the sum must read zero

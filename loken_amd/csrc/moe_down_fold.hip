@@ -124,9 +124,10 @@ struct LaneQ6K {   // q = 2 * (half of the super-block) + (which 16-byte run of 
 struct FoldDims {
     int experts, topk, pairs, cols, passes;
     int64_t slab_bytes;
+    int write;   // the sums replace what the output holds
 };
 
-constexpr int SCAN_ROUNDS = 2;              // routing entries a lane looks at: pairs <= 2 * 256
+constexpr int SCAN_ROUNDS = 2;              // sorted routing entries a lane looks at: pairs <= 2 * 256
 constexpr int MAX_PAIRS = SCAN_ROUNDS * WG;
 
 template <class L, int NB>
@@ -163,12 +164,18 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
     const int slot0 = token * d.topk;
 
     // ---- loads that depend on nothing: the routing, then the token's activation rows
+    const bool in_order = sorted_token_ids == nullptr;   // pair i is slot i: a slot's expert is read where it stands
     int s_at[SCAN_ROUNDS], e_at[SCAN_ROUNDS];
+    int e = -1;
+    if (in_order) {
+        if (j < d.topk) e = expert_ids[slot0 + j];
+    } else {
 #pragma unroll
-    for (int u = 0; u < SCAN_ROUNDS; ++u) {
-        const int i = min(tid + u * WG, d.pairs - 1);
-        s_at[u] = sorted_token_ids[i];
-        e_at[u] = expert_ids[i];
+        for (int u = 0; u < SCAN_ROUNDS; ++u) {
+            const int i = min(tid + u * WG, d.pairs - 1);
+            s_at[u] = sorted_token_ids[i];
+            e_at[u] = expert_ids[i];
+        }
     }
     const float scale = topk_weights[slot0 + min(j, d.topk - 1)];
     float4 x[ACT_LOADS];
@@ -181,27 +188,30 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
     load_fence(acts);
 
     // ---- the expert of each of the token's slots
-    if (tid < TKP) e_of[tid] = -1;
-    __syncthreads();
+    if (!in_order) {
+        if (tid < TKP) e_of[tid] = -1;
+        __syncthreads();
 #pragma unroll
-    for (int u = 0; u < SCAN_ROUNDS; ++u) {
-        const int rel = s_at[u] - slot0;
-        if (tid + u * WG < d.pairs && rel >= 0 && rel < d.topk) e_of[rel] = e_at[u];
+        for (int u = 0; u < SCAN_ROUNDS; ++u) {
+            const int rel = s_at[u] - slot0;
+            if (tid + u * WG < d.pairs && rel >= 0 && rel < d.topk) e_of[rel] = e_at[u];
+        }
+        __syncthreads();
+        e = e_of[j];
     }
-    __syncthreads();
-    const int e = e_of[j];
     const bool routed = e >= 0 && e < d.experts;   // a slot no pair names, or an expert out of range, adds nothing
 
     const gbytes_t slab = to_gbytes(w) + (int64_t)(routed ? e : 0) * d.slab_bytes;
     const int group0 = blockIdx.x * d.passes;
     const size_t out_at = (size_t)token * d.cols;
-    const float* before = add_after ? add_after : out;   // what the sum starts from / ends with
+    // what the sum starts from / ends with (nothing when the sums are to be written)
+    const float* before = add_after ? add_after : out;
     auto load = [&](FoldFrag<L, NB>& f, int p) {
         const int row = min((group0 + p) * RPG + wave * RPW + r, d.cols - 1);
         const uint8_t* bp = (const uint8_t*)(slab + (size_t)row * (NB * L::BYTES));
 #pragma unroll
         for (int b = 0; b < NB; ++b) L::load(f.w[b], bp + b * L::BYTES, q);
-        f.prev = before[out_at + row];
+        f.prev = d.write ? 0.f : before[out_at + row];
         f.bias = down_bias ? down_bias[(size_t)(routed ? e : 0) * d.cols + row] : 0.f;
     };
     FoldFrag<L, NB> fa, fb;
@@ -315,13 +325,13 @@ int launch_format(const FoldCall& c, const FoldDims& d, int nb) {
 int lk_moe_down_fold(int quant_type, const float* inputs, const void* weights, const int32_t* sorted_token_ids,
                      const int32_t* expert_ids, const float* topk_weights, float* outputs, int num_experts, int topk,
                      int size_m, int size_n, int size_k, const float* down_bias, const float* add_after,
-                     hipStream_t stream) {
+                     bool write, hipStream_t stream) {
     if (lk_tune_env("LK_TUNE_DOWN_FOLD_OFF")) return -1;
-    if (size_k % 256 != 0 || topk < 1 || topk > 8 || size_m > MAX_PAIRS || size_m % topk != 0) return -1;
+    if (size_k % 256 != 0 || topk < 1 || topk > 8 || (sorted_token_ids && size_m > MAX_PAIRS) || size_m % topk != 0) return -1;
     if (((uintptr_t)inputs) & 15) return -1;
     const int tokens = size_m / topk;
     if (tokens < 1 || tokens > 65535) return -1;
-    const FoldDims d{num_experts, topk, size_m, size_n, 1, 0};
+    const FoldDims d{num_experts, topk, size_m, size_n, 1, 0, write && !add_after ? 1 : 0};
     const FoldCall c{(const uint8_t*)weights, inputs, sorted_token_ids, expert_ids, topk_weights, down_bias, add_after,
                      outputs, tokens, stream};
     switch (quant_type) {

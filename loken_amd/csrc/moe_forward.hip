@@ -1,0 +1,153 @@
+// The expert block of a mixture layer as one call: every launch from the router's choices to the block's
+// output, chosen by size as the reference's layer code chooses (src/inference/generic_transformer/
+// moe_weights.rs:2118-2152; MmqRouting, src/inference/moe_cuda/mmq_experts.rs:108-736): expert-batched
+// products over a grouped routing from about a routed row per expert on, a mat-vec per routed pair below.
+//
+// What it adds to the entry points it is made of: nothing is sorted, copied or cleared that the kernels do not
+// read (pairs stay in slot order, sums are written instead of added to zeros), the activation between the two
+// tiled products is quantized where it is computed, and the host does one call instead of eight to fifteen
+// (a one-token block of 128 experts: 80 us with torch's sort, copies and fills around the two kernels).
+
+#include "moe_block.h"
+#include "stream_scratch.h"
+
+#include <math.h>
+
+namespace {
+
+struct Format {
+    int type, block_len, block_bytes, wire;   // wire: id of the per-pair launchers, -1: they do not take it
+    int (*grouped)(const void*, const void*, int64_t, const void*, void*, const int*, const int*, int64_t, int64_t, int64_t, int64_t,
+                   int64_t, int64_t, int, int64_t, int64_t, int, int, int64_t, int, void*);
+};
+constexpr Format FORMATS[] = {
+    {LK_TYPE_Q8_0, 32, 34, 0, launch_mmq_moe_gguf_q8_0},       {LK_TYPE_Q4_K, 256, 144, 1, launch_mmq_moe_gguf_q4_k},
+    {LK_TYPE_Q2_K, 256, 84, 2, launch_mmq_moe_gguf_q2_k},      {LK_TYPE_Q3_K, 256, 110, 3, launch_mmq_moe_gguf_q3_k},
+    {LK_TYPE_Q5_K, 256, 176, 4, launch_mmq_moe_gguf_q5_k},     {LK_TYPE_Q6_K, 256, 210, 5, launch_mmq_moe_gguf_q6_k},
+    {LK_TYPE_Q5_0, 32, 22, 6, launch_mmq_moe_gguf_q5_0},       {LK_TYPE_MXFP4, 32, 17, 7, launch_mmq_moe_gguf_mxfp4},
+    {LK_TYPE_Q5_1, 32, 24, 8, launch_mmq_moe_gguf_q5_1},       {LK_TYPE_IQ4_NL, 32, 18, 9, launch_mmq_moe_gguf_iq4_nl},
+    {LK_TYPE_IQ4_XS, 256, 136, 10, launch_mmq_moe_gguf_iq4_xs}, {LK_TYPE_IQ3_XXS, 256, 98, 11, launch_mmq_moe_gguf_iq3_xxs},
+    {LK_TYPE_IQ3_S, 256, 110, 12, launch_mmq_moe_gguf_iq3_s},  {LK_TYPE_IQ2_S, 256, 82, 13, launch_mmq_moe_gguf_iq2_s},
+    {LK_TYPE_Q2_0, 64, 18, 14, launch_mmq_moe_gguf_q2_0},      {LK_TYPE_IQ2_XXS, 256, 66, 15, nullptr},
+    {LK_TYPE_Q4_0, 32, 18, -1, launch_mmq_moe_gguf_q4_0},      {LK_TYPE_Q4_1, 32, 20, -1, launch_mmq_moe_gguf_q4_1},
+};
+const Format* format_of(int type) {
+    for (const Format& f : FORMATS)
+        if (f.type == type) return &f;
+    return nullptr;
+}
+
+bool grouped_serves(const Format& f, int k) { return f.grouped && k % 256 == 0; }
+
+size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+size_t workspace_bytes(int64_t rows, int k) { return (size_t)rows * ((k + 511) / 512 * 4) * 144 + 128 * 144; }
+
+}  // namespace
+
+// Routed rows from which the expert-batched launches beat a mat-vec per routed pair. The reference breaks even
+// at one routed row per expert (mmq_experts.rs:72-86); here, measured on MI355X (128 experts of 2048 -> 768 -> 2048, top-8), the
+// mat-vec per routed pair stays ahead of the tiled products up to three rows per expert (117 us against 162 at 32
+// tokens, 176 against 168 at 48), and of the matrix-unit rows launch that Q4_K stacks take at short runs up to
+// 1.625 (16 tokens: 51 us against 74; 24: 81 against 83; 32: 92 against 88; 48: 139 against 106). `wtype`: the stacks' type where both
+// have the same, else -1.
+extern "C" int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype) {
+    const int64_t experts = n_experts > 1 ? n_experts : 1;
+    return wtype == LK_TYPE_Q4_K ? 8 * rows >= 13 * experts : rows >= 3 * experts;
+}
+
+// The longest run of rows an expert is expected to own, every choice equally likely: mean + sqrt(2 ln experts)
+// deviations of a binomial count (mmq_experts.rs:215-227).
+extern "C" int lk_moe_longest_run(int tokens, int topk, int n_experts) {
+    const double experts = n_experts > 1 ? n_experts : 1;
+    const double p = topk / experts < 1.0 ? topk / experts : 1.0;
+    const double mean = tokens * p, dev = sqrt(mean * (1.0 - p));
+    const double longest = ceil(n_experts > 1 ? mean + dev * sqrt(2.0 * log(experts)) : mean);
+    const double most = tokens > 1 ? tokens : 1;
+    return (int)(longest < 1.0 ? 1.0 : longest > most ? most : longest);
+}
+
+// Whether a stack takes the matrix-unit rows launch (weights straight from HBM into the operand, a wave per
+// 16-row tile, a pass per 8, 16 or 48 rows) rather than the tiled one (weights expanded into LDS per 32 tokens).
+// Measured on MI355X at 128 experts of 2048 -> 768 -> 2048, top-8: 64 tokens 112 us against 173, 128 tokens 121
+// against 170, 256 tokens 159 against 183, 512 tokens 228 against 271, 1024 tokens 394 against 408, 1536 tokens
+// 537 against 463 (the expected longest run is 17 at 128 tokens, 29 at 256, 88 at 1024, 126 at 1536).
+extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
+    return wtype == LK_TYPE_Q4_K && k % 256 == 0 && longest_run <= 90;
+}
+
+extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
+                              const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
+                              int hidden, int ffn, void* stream) {
+    const Format *fg = format_of(wtype_gu), *fd = format_of(wtype_down);
+    if (!fg || !fd) return LK_ERR_TYPE;
+    if (tokens == 0) return LK_OK;
+    if (!x || !gate || !up || !down || !choices || !topk_weights || !out || tokens < 0 || topk <= 0 || n_experts <= 0 || hidden <= 0 ||
+        ffn <= 0 || hidden % fg->block_len != 0 || ffn % fd->block_len != 0 || (int64_t)tokens * topk > INT32_MAX)
+        return LK_ERR_ARG;
+    hipStream_t s = (hipStream_t)stream;
+    const int rows = tokens * topk;
+    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
+
+    if (!(lk_moe_grouped_pays(rows, n_experts, wtype_gu == wtype_down ? wtype_gu : -1) && grouped_serves(*fg, hidden) &&
+          grouped_serves(*fd, ffn))) {
+        if (fg->wire < 0 || fd->wire < 0) return LK_ERR_TYPE;
+        float* h = (float*)lk_reserve_scratch((size_t)rows * ffn * 4, s, LK_SCRATCH_BLOCK);
+        if (!h) return LK_ERR_NOMEM;
+        if (int rc = lk_moe_pairs_gate_up(fg->wire, x, gate, up, choices, h, n_experts, topk, rows, ffn, hidden, s)) return rc;
+        return lk_moe_pairs_down(fd->wire, h, down, choices, topk_weights, out, n_experts, topk, rows, hidden, ffn, s);
+    }
+
+    const int longest = lk_moe_longest_run(tokens, topk, n_experts);
+    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest), rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
+    const bool gated_later = !rows_gu && !rows_down && ffn % 32 == 0;   // the activation rides the second product's quantizer
+    // the buffer's pieces
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const size_t p = at; at += up256(bytes); return p; };
+    const size_t bounds_at = take((size_t)(n_experts + 1) * 4), slots_at = take((size_t)rows * 4), src_at = take((size_t)rows * 4);
+    const size_t y_at = take(rows_gu ? (size_t)tokens * (hidden / 32) * Q81_BYTES : workspace_bytes(rows, hidden));
+    const size_t gu_at = take(rows_gu ? 0 : (size_t)rows * 2 * ffn * 4);
+    const size_t h_at = take(gated_later ? 0 : (size_t)rows * ffn * 4);
+    const size_t y2_at = take(rows_down ? (size_t)rows * (ffn / 32) * Q81_BYTES : workspace_bytes(rows, ffn));
+    const size_t pairs_at = take((size_t)rows * hidden * 4);
+    uint8_t* base = (uint8_t*)lk_reserve_scratch(at, s, LK_SCRATCH_BLOCK);
+    if (!base) return LK_ERR_NOMEM;
+    int32_t *bounds = (int32_t*)(base + bounds_at), *slots = (int32_t*)(base + slots_at), *src = (int32_t*)(base + src_at);
+    float *gu = (float*)(base + gu_at), *h = (float*)(base + h_at), *pairs = (float*)(base + pairs_at);
+    uint8_t *y = base + y_at, *y2 = base + y2_at;
+
+    auto grouped = [&](const Format& f, const void* w, const void* w2, int64_t second_at, const uint8_t* acts, float* dst, const int32_t* ids,
+                       int n, int k, int stride) {
+        const int64_t blocks = k / f.block_len;
+        return f.grouped(w, w2, second_at, acts, dst, bounds, ids, n * blocks * f.block_bytes, k, n, rows, blocks, stride, n_experts, longest,
+                         longest, 0, 0, 0, 0, stream) != 0
+                   ? LK_OK
+                   : LK_ERR_ARG;
+    };
+    auto quantize = [&](const float* from, const int32_t* gather, uint8_t* to, int k) {   // (one record layout serves every format)
+        launch_mmq_quantize_q8_1_DS4(from, gather, to, LK_TYPE_F32, k, k, 0, 0, (k + 511) / 512 * 512, rows, 1, 1, stream);
+    };
+
+    if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, s)) return rc;
+    if (rows_gu) {
+        if (int rc = lk_quantize_q8_1(x, LK_TYPE_F32, y, hidden, hidden, tokens, stream)) return rc;
+        if (int rc = lk_moe_q4k_rows_grouped(gate, up, 0, y, hidden / 32, bounds, src, nullptr, h, ffn, n_experts,
+                                             (int64_t)ffn * (hidden / 256) * Q4K_BYTES, ffn, hidden, longest, stream)) return rc;
+    } else {
+        quantize(x, src, y, hidden);
+        if (int rc = grouped(*fg, gate, up, ffn, y, gu, nullptr, ffn, hidden, 2 * ffn)) return rc;
+        if (gated_later) {
+            if (int rc = lk_mmq_quantize_gated(gu, y2, rows, ffn, s)) return rc;
+        } else {
+            loken_moe_mmq_silu_mul(gu, h, rows, ffn, stream);
+        }
+    }
+    if (rows_down) {
+        if (int rc = lk_quantize_q8_1(h, LK_TYPE_F32, y2, ffn, ffn, rows, stream)) return rc;
+        if (int rc = lk_moe_q4k_rows_grouped(down, nullptr, 0, y2, ffn / 32, bounds, nullptr, slots, pairs, hidden, n_experts,
+                                             (int64_t)hidden * (ffn / 256) * Q4K_BYTES, hidden, ffn, longest, stream)) return rc;
+    } else {
+        if (!gated_later) quantize(h, nullptr, y2, ffn);
+        if (int rc = grouped(*fd, down, nullptr, 0, y2, pairs, slots, hidden, ffn, hidden)) return rc;
+    }
+    return lk_moe_fold_write(pairs, topk_weights, out, tokens, topk, hidden, s);
+}

@@ -18,25 +18,6 @@
 
 namespace {
 
-template <typename T> struct Load4;
-template <> struct Load4<float> {
-    static __device__ __forceinline__ float4 at(const float* p) { return *(const float4*)p; }
-};
-template <> struct Load4<__half> {
-    static __device__ __forceinline__ float4 at(const __half* p) {
-        const uint2 raw = *(const uint2*)p;
-        const __half2 a = *(const __half2*)&raw.x, b = *(const __half2*)&raw.y;
-        return make_float4(__low2float(a), __high2float(a), __low2float(b), __high2float(b));
-    }
-};
-template <> struct Load4<__hip_bfloat16> {
-    static __device__ __forceinline__ float4 at(const __hip_bfloat16* p) {
-        const uint2 raw = *(const uint2*)p;
-        return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u),
-                           __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u));
-    }
-};
-
 static __device__ __forceinline__ int round_code(float v) {
     // roundf is half away from zero, as f32::round.
     return (int)roundf(v);

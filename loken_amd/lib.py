@@ -90,6 +90,10 @@ SIGNATURES.update({
     "loken_moe_gemm_gguf_down_pairs_two": (_i, [_vp] * 3 + [_i] + [_vp] * 5 + [_i] * 6 + [_vp]),
     "loken_moe_gemm_gguf_down_reduce": (_i, [_vp] * 6 + [_i] * 6 + [_vp, _vp, _vp]),
     "loken_moe_gemm_gguf_down_reduce_static": (_i, [_vp] * 6 + [_i] * 6 + [_vp, _vp, _vp]),
+    "lk_moe_forward": (_i, [_i, _i] + [_vp] * 7 + [_i] * 5 + [_vp]),
+    "lk_moe_grouped_pays": (_i, [_i64, _i, _i]),
+    "lk_moe_longest_run": (_i, [_i, _i, _i]),
+    "lk_moe_rows_launch_pays": (_i, [_i, _i, _i]),
     "loken_moe_sum_topk": (None, [_vp, _vp, _i, _i, _i, _vp]),
     "loken_stream_scratch_release": (None, []),
     "lk_rmsnorm_q8_1": (_i, [_vp, _vp, _vp, _vp, _f, _i, _i, _vp]),

@@ -5,8 +5,6 @@ token's slots in slot order. torch holds the buffers; every computation is a C-A
 """
 from __future__ import annotations
 
-import math
-
 import torch
 
 from . import lib as _lib
@@ -87,12 +85,7 @@ class MmqRouting:
 
     def longest_run_expected(self) -> int:
         """mmq_experts.rs:215-227: mean + sqrt(2 ln experts) deviations of a binomial count."""
-        experts = float(max(self.experts, 1))
-        p = min(self.topk / experts, 1.0)
-        mean = self.tokens * p
-        dev = math.sqrt(mean * (1.0 - p))
-        longest = mean + dev * math.sqrt(2.0 * math.log(experts)) if experts > 1 else mean
-        return max(1, min(int(math.ceil(longest)), max(self.tokens, 1)))
+        return _lib.load().lk_moe_longest_run(self.tokens, self.topk, self.experts)
 
     def _matmul(self, wtype: int, stack: torch.Tensor, second: torch.Tensor | None, second_offset: int,
                 n: int, k: int, y: torch.Tensor, dst: torch.Tensor, stride: int, ids_dst: torch.Tensor | None):
@@ -110,17 +103,10 @@ class MmqRouting:
         if launched == 0:
             raise _lib.LokenError(MMQ_MOE_LAUNCHER[wtype], _lib.LK_ERR_ARG)
 
-    # Rows an expert is expected to own up to which the matrix-unit rows launch (weights straight from
-    # HBM into the operand, a wave per 16-row tile, a pass per 8, 16 or 48 rows) beats the tiled one
-    # (weights expanded into LDS per 32 tokens). Measured on MI355X at 128 experts of 2048 -> 768 -> 2048,
-    # top-8: 64 tokens 112 us against 173, 128 tokens 121 against 170, 256 tokens 159 against 183, 512
-    # tokens 228 against 271, 1024 tokens 394 against 408, 1536 tokens 537 against 463 (the expected
-    # longest run is 17 at 128 tokens, 29 at 256, 88 at 1024, 126 at 1536).
-    ROWS_LAUNCH_MAX_RUN = 90
-
     def takes_rows_launch(self, wtype: int, k: int) -> bool:
-        return (self.path != "tiled" and wtype == _lib.TYPE_Q4_K and k % 256 == 0
-                and (self.path == "rows" or self.longest_run_expected() <= self.ROWS_LAUNCH_MAX_RUN))
+        if self.path == "tiled" or wtype != _lib.TYPE_Q4_K or k % 256:
+            return False
+        return self.path == "rows" or bool(_lib.load().lk_moe_rows_launch_pays(wtype, k, self.longest_run_expected()))
 
     def _rows_launch(self, weights: torch.Tensor, second: torch.Tensor | None, q: torch.Tensor, src, dst_map,
                      out: torch.Tensor, n: int, k: int):
@@ -436,16 +422,9 @@ def stable_sort_u32(keys: torch.Tensor, small: bool = False):
 
 
 def moe_mmq_pays(rows: int, experts: int, wtype: int | None = None) -> bool:
-    """Routed rows from which the expert-batched launches beat the per-pair kernels. The reference
-    breaks even at one routed row per expert (mmq_experts.rs:72-86); on MI355X, with this
-    library's kernels, the mat-vec per routed pair stays ahead of the tiled matmul up to three rows
-    per expert (Qwen3-30B-A3B shapes: 117 us against 162 us at 32 tokens, 176 against 168 at 48), and
-    of the matrix-unit rows launch that Q4_K stacks take at short runs up to 1.625 (per block inside
-    a step's graph, 16 tokens: 51 us against 74; 24: 81 against 83; 32: 92 against 88; 48: 139
-    against 106)."""
-    if wtype == _lib.TYPE_Q4_K:
-        return 8 * rows >= 13 * max(experts, 1)
-    return rows >= 3 * max(experts, 1)
+    """Whether the expert-batched launches beat the per-pair kernels at this many routed rows (``wtype``: the
+    stacks' type where all have the same)."""
+    return bool(_lib.load().lk_moe_grouped_pays(rows, experts, -1 if wtype is None else wtype))
 
 
 def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor,
@@ -457,6 +436,15 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
     `return_rows`: also the gated rows the second product read, in slot order (token * topk + choice)."""
     tokens, hidden = x.shape
     topk = choices.shape[1]
+    if (not return_rows and x.dtype == topk_weights.dtype == torch.float32 and choices.dtype == torch.int32 and x.is_contiguous()
+            and choices.shape[0] == tokens and choices.is_contiguous() and topk_weights.is_contiguous()
+            and topk_weights.numel() == choices.numel()):
+        # the whole block in one call; what it does not take goes on below, launch by launch
+        out = torch.empty((tokens, hidden), dtype=torch.float32, device=x.device)
+        if _lib.load().lk_moe_forward(wtype_gu, wtype_down, x.data_ptr(), gate.data_ptr(), up.data_ptr(), down.data_ptr(),
+                                      choices.data_ptr(), topk_weights.data_ptr(), out.data_ptr(), tokens, topk, n_experts, hidden, ffn,
+                                      _stream()) == _lib.LK_OK:
+            return out
     if (moe_mmq_pays(tokens * topk, n_experts, wtype_gu if wtype_gu == wtype_down else None)
             and moe_mmq_serves(wtype_gu, hidden) and moe_mmq_serves(wtype_down, ffn)):
         plan = MmqRouting.from_choices(choices, n_experts)

@@ -569,6 +569,33 @@ def test_layer_entry_picks_a_path_and_both_agree(tokens):
                 tokens=sample)
 
 
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,dn", [
+    (1, 2, 4, 512, 256, lib.TYPE_Q4_K, lib.TYPE_Q4_K), (7, 4, 60, 1024, 768, lib.TYPE_Q4_K, lib.TYPE_Q6_K),
+    (3, 2, 8, 512, 1280, lib.TYPE_MXFP4, lib.TYPE_MXFP4), (70, 8, 512, 256, 512, lib.TYPE_Q4_K, lib.TYPE_Q4_K),
+    (33, 4, 8, 512, 256, lib.TYPE_Q8_0, lib.TYPE_Q8_0), (129, 2, 8, 512, 768, lib.TYPE_Q4_K, lib.TYPE_Q4_K),
+    (301, 8, 16, 256, 512, lib.TYPE_Q5_K, lib.TYPE_Q6_K)])
+def test_block_in_one_call_is_the_block_launch_by_launch(tokens, topk, n_experts, hidden, ffn, gu, dn):
+    """lk_moe_forward (pairs in slot order, sums written, the activation in the second quantizer) against the
+    launches it is made of, sorted and summed into zeros: the same bits, two calls in a row."""
+    gate, up = (dev(synth.weight(gu, n_experts * ffn, hidden, seed=62, stream=i)) for i in (1, 2))
+    down = dev(synth.weight(dn, n_experts * hidden, ffn, seed=62, stream=3))
+    for seed in (63, 64):
+        x = dev(synth.activation(tokens, hidden, seed=seed))
+        ids, w = oracle.topk_softmax(synth.activation(tokens, n_experts, seed=seed, stream=7), topk)
+        args = (gu, dn, x, gate, up, down, dev(ids), dev(w), n_experts, ffn)
+        assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
+
+
+@pytest.mark.parametrize("n,n_experts,topk", [(1, 3, 1), (63, 5, 3), (64, 1, 1), (1025, 130, 5), (4097, 512, 1), (8888, 128, 8)])
+def test_routing_is_a_stable_grouping(n, n_experts, topk):
+    choices = synth.rand_ints(23, n, n, n_experts).astype(np.int32).reshape(-1, topk)
+    plan = MmqRouting.from_choices(dev(choices), n_experts)
+    order = np.argsort(choices.reshape(-1), kind="stable")
+    assert np.array_equal(plan.slots.cpu().numpy(), order)
+    assert np.array_equal(plan.src_rows.cpu().numpy(), order // topk)
+    assert np.array_equal(plan.bounds.cpu().numpy(), np.searchsorted(np.sort(choices.reshape(-1)), np.arange(n_experts + 1)))
+
+
 # ---------------------------------------------------------------- router
 @pytest.mark.parametrize("tokens,experts,topk,renorm", [(1, 128, 8, True), (16, 128, 8, True), (256, 128, 8, False),
                                                         (7, 60, 4, True), (5, 512, 64, True), (3, 8, 8, False)])
