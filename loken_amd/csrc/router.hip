@@ -8,6 +8,7 @@
 // arg-max rounds are wave reductions; rows are tiny (128 logits), so the launch is latency only.
 
 #include "lk_common.h"
+#include "stream_scratch.h"
 
 namespace {
 
@@ -26,22 +27,21 @@ static __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 
-// Softmax over `x[0 .. n_experts)` and the k largest, by the 64 lanes of one wave.
-static __device__ __forceinline__ void select_topk_softmax(const float* x, float* __restrict__ weights,
+// Softmax over the logits a lane brings (p[i]: expert lane + 64 i, -INFINITY past n_experts) and the k largest, by
+// the 64 lanes of one wave; PER = experts / 64 rounded up to a power of two. A round finds the largest
+// probability through lane moves of the vector unit and scalar registers, and the lowest expert that has it by
+// ballots (a permute through LDS per step of the reduction costs four times as much).
+template <int PER>
+static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], float* __restrict__ weights,
                                                            uint32_t* __restrict__ ids, int n_experts, int topk,
                                                            int with_norm, int lane) {
-    float p[MAX_PER_LANE];
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < MAX_PER_LANE; ++i) {
-        const int e = lane + 64 * i;
-        p[i] = e < n_experts ? x[e] : -INFINITY;
-        mx = fmaxf(mx, p[i]);
-    }
+    for (int i = 0; i < PER; ++i) mx = fmaxf(mx, p[i]);
     mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < MAX_PER_LANE; ++i) {
+    for (int i = 0; i < PER; ++i) {
         const int e = lane + 64 * i;
         p[i] = e < n_experts ? expf(p[i] - mx) : -1.f;   // -1: never chosen, probabilities are >= 0
         sum += e < n_experts ? p[i] : 0.f;
@@ -50,32 +50,35 @@ static __device__ __forceinline__ void select_topk_softmax(const float* x, float
     float picked_sum = 0.f, my_weight = 0.f;
     uint32_t my_id = 0;
     for (int j = 0; j < topk; ++j) {
-        // the lane's best: largest probability, lowest expert id among equals
-        float best = -1.f;
-        int best_e = 0x7FFFFFFF;
+        float best = p[0];
 #pragma unroll
-        for (int i = 0; i < MAX_PER_LANE; ++i)
-            if (p[i] > best) { best = p[i]; best_e = lane + 64 * i; }
-        // the wave's best, same order
-        float w_best = best;
-        int w_e = best_e;
+        for (int i = 1; i < PER; ++i) best = fmaxf(best, p[i]);
+        best = wave_max(best);
+        int e = 0x7FFFFFFF;   // stays so only where a logit is not a number and nothing compares equal
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const float ob = __shfl_xor(w_best, o);
-            const int oe = __shfl_xor(w_e, o);
-            if (ob > w_best || (ob == w_best && oe < w_e)) { w_best = ob; w_e = oe; }
+        for (int i = PER - 1; i >= 0; --i) {
+            const unsigned long long at = __ballot(p[i] == best);
+            if (at) e = 64 * i + __ffsll((long long)at) - 1;
         }
-        const float prob = w_best / sum;
+        const float prob = best / sum;
         picked_sum += prob;
-        if (lane == j) { my_weight = prob; my_id = (uint32_t)w_e; }
+        if (lane == j) { my_weight = prob; my_id = (uint32_t)e; }
 #pragma unroll
-        for (int i = 0; i < MAX_PER_LANE; ++i)
-            if (lane + 64 * i == w_e) p[i] = -1.f;
+        for (int i = 0; i < PER; ++i)
+            if (lane + 64 * i == e) p[i] = -1.f;
     }
     if (lane < topk) {
         weights[lane] = with_norm ? my_weight / picked_sum : my_weight;
         ids[lane] = my_id;
     }
+}
+
+static __device__ __forceinline__ void select_topk_softmax(const float* x, float* __restrict__ weights, uint32_t* __restrict__ ids,
+                                                           int n_experts, int topk, int with_norm, int lane) {
+    float p[MAX_PER_LANE];
+#pragma unroll
+    for (int i = 0; i < MAX_PER_LANE; ++i) p[i] = lane + 64 * i < n_experts ? x[lane + 64 * i] : -INFINITY;
+    select_topk_softmax<MAX_PER_LANE>(p, weights, ids, n_experts, topk, with_norm, lane);
 }
 
 __global__ __launch_bounds__(64) void topk_softmax_kernel(const float* __restrict__ logits, float* __restrict__ weights,
@@ -87,15 +90,169 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------------------------------------
-// The gate mat-vec, softmax and top-k of a token in one launch (loken_gate_topk_softmax,
-// cuda/moe/gate_topk.cu:253-295, 366-403). The reference gives a token one warp and each lane
-// whole weight rows, read four floats at a time at a stride of a row; here a token has a
-// workgroup of 16 waves, a wave takes experts w, w + 16, ... and its lanes walk the row together
-// (consecutive lanes read consecutive 16-byte pieces), so a one-token launch pulls the 1 MB of a
-// 128 x 2048 gate at the rate one CU can stream rather than one lane's. Each logit is then
-// a 64-lane sum instead of a serial one: same value up to f32 summation order. The selection is
-// the wave-wide one above, run by wave 0 over the logits left in LDS.
+// The gate product, softmax and top-k of every token (loken_gate_topk_softmax, cuda/moe/gate_topk.cu:253-295,
+// 366-403), in two launches: the logits as an f32 product on the matrix unit, then a wave per token that adds
+// the partial sums and selects. One workgroup per token (the kernel after these, still the one for rows that do
+// not start on 16 bytes and for streams that record a graph before their scratch exists) reads the whole gate
+// for each token through one CU: 28 us at one token of 2048 x 128, where the bytes take a microsecond, and 69 us
+// at 1111.
+//
+// The logits: v_mfma_f32_{16x16x4,32x32x2}_f32 (f32 operands and sums), a tile of tokens x experts per
+// workgroup. A lane takes four consecutive values of its token's row and of its expert's row at once, one component per
+// instruction (any order of K serves as long as both operands agree). The four waves of a workgroup and the
+// grid's z axis split K until the launch covers the chip; partial sums meet in LDS and in part[z].
 // ---------------------------------------------------------------------------------------------
+constexpr int LOGIT_WAVES = 4;
+constexpr int LOGIT_SPREAD = 768;   // workgroups a launch aims at: loads wait a microsecond each, so three per CU
+
+// Up to sixteen tokens: 16 x 16 tiles, rows straight from memory.
+__global__ __launch_bounds__(64 * LOGIT_WAVES) void gate_logits16_kernel(const float* __restrict__ x_in, const float* __restrict__ gate_w,
+                                                                         float* __restrict__ part, int hidden, int n_rows,
+                                                                         int n_experts) {
+    constexpr int M = 16, UNIT = 16, AHEAD = 4;   // UNIT: values of K a load of the wave covers; AHEAD: loads per operand in flight
+    __shared__ __align__(16) float meet[LOGIT_WAVES - 1][M * M];
+    const int lane = threadIdx.x & 63, at = lane % M, grp = lane / M;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e0 = blockIdx.y * M;
+    const int units = (hidden + UNIT - 1) / UNIT, shares = gridDim.z * LOGIT_WAVES, share = blockIdx.z * LOGIT_WAVES + wave;
+    const int u0 = (int)((int64_t)units * share / shares), u1 = (int)((int64_t)units * (share + 1) / shares);
+    const float* xr = x_in + (size_t)min(at, n_rows - 1) * hidden;
+    const float* wr = gate_w + (size_t)min(e0 + at, n_experts - 1) * hidden;
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    for (int u = u0; u < u1; u += AHEAD) {
+        float4 a[AHEAD], b[AHEAD];
+        bool live[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            // past the share (or the row's end, in its last unit): a repeat of the row's start, multiplied by zero
+            const int k = (u + i) * UNIT + 4 * grp;
+            live[i] = u + i < u1 && k < hidden;
+            a[i] = *(const float4*)(xr + (live[i] ? k : 0));
+            b[i] = *(const float4*)(wr + (live[i] ? k : 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);   // all of them out before the first is waited for
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            if (!live[i]) a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].x, b[i].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].y, b[i].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].z, b[i].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].w, b[i].w, acc, 0, 0, 0);
+        }
+    }
+    if (wave > 0) *(v4f*)(meet[wave - 1] + lane * 4) = acc;
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < LOGIT_WAVES - 1; ++w) acc += *(const v4f*)(meet[w] + lane * 4);
+    // lane (group, column), register v: token 4 grp + v, expert `at` of the tile
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (4 * grp + v < n_rows && e0 + at < n_experts) part[((size_t)blockIdx.z * n_rows + 4 * grp + v) * n_experts + e0 + at] = acc[v];
+}
+
+// More tokens: 32 x 32 tiles. Taken from memory in operand order (a lane per row) a load touches 32 cache lines
+// and the launch is bound by the address unit (1111 tokens: 22 us); here a wave copies 32 rows x 128 bytes of
+// each operand into its own piece of LDS, eight lanes to a row, and reads the operands from there (row pitch 144 bytes:
+// no bank conflicts). The next copy is in flight while this one is multiplied; waves share nothing until
+// their sums meet.
+__global__ __launch_bounds__(64 * LOGIT_WAVES) void gate_logits32_kernel(const float* __restrict__ x_in, const float* __restrict__ gate_w,
+                                                                         float* __restrict__ part, int hidden, int n_rows,
+                                                                         int n_experts) {
+    constexpr int M = 32, UNIT = 32, PITCH = UNIT + 4, ROUNDS = M * UNIT / 4 / 64;
+    __shared__ __align__(16) float stage[LOGIT_WAVES][2][M * PITCH];
+    const int lane = threadIdx.x & 63, at = lane % M, grp = lane / M;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = blockIdx.x * M, e0 = blockIdx.y * M;
+    const int units = (hidden + UNIT - 1) / UNIT, shares = gridDim.z * LOGIT_WAVES, share = blockIdx.z * LOGIT_WAVES + wave;
+    const int u0 = (int)((int64_t)units * share / shares), u1 = (int)((int64_t)units * (share + 1) / shares);
+    const int row8 = lane >> 3, k4 = 4 * (lane & 7);
+    float *sx = stage[wave][0], *sw = stage[wave][1];
+    float4 xv[ROUNDS], wv[ROUNDS];
+    auto fetch = [&](int u) {
+        const int k = u * UNIT + k4;
+        const bool live = k < hidden;   // in the row's last unit; past it: a repeat of the row's start, as zeros
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            xv[r] = *(const float4*)(x_in + (size_t)min(t0 + 8 * r + row8, n_rows - 1) * hidden + (live ? k : 0));
+            wv[r] = *(const float4*)(gate_w + (size_t)min(e0 + 8 * r + row8, n_experts - 1) * hidden + (live ? k : 0));
+            if (!live) xv[r] = wv[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    v16f acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    if (u0 < u1) fetch(u0);
+    for (int u = u0; u < u1; ++u) {
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            *(float4*)(sx + (8 * r + row8) * PITCH + k4) = xv[r];
+            *(float4*)(sw + (8 * r + row8) * PITCH + k4) = wv[r];
+        }
+        __builtin_amdgcn_wave_barrier();   // a wave's LDS operations are served in order: the reads below see the writes
+        if (u + 1 < u1) fetch(u + 1);
+#pragma unroll
+        for (int i = 0; i < UNIT / 8; ++i) {
+            const float4 a = *(const float4*)(sx + at * PITCH + 8 * i + 4 * grp), b = *(const float4*)(sw + at * PITCH + 8 * i + 4 * grp);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    float* meet = &stage[0][0][0] + wave * M * M;
+    __syncthreads();   // the pieces of LDS are read for the last time
+    if (wave > 0) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) meet[v * 64 + lane] = acc[v];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    // lane (group, column), register v: token 8 (v / 4) + 4 grp + v % 4, expert `at` of the tile
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        float sum = acc[v];
+#pragma unroll
+        for (int w = 1; w < LOGIT_WAVES; ++w) sum += meet[w * M * M + v * 64 + lane];
+        const int t = t0 + 8 * (v / 4) + 4 * grp + v % 4, e = e0 + at;
+        if (t < n_rows && e < n_experts) part[((size_t)blockIdx.z * n_rows + t) * n_experts + e] = sum;
+    }
+}
+
+template <int PER>
+__global__ __launch_bounds__(256) void gate_select_kernel(const float* __restrict__ part, int splits, float* __restrict__ weights,
+                                                          uint32_t* __restrict__ ids, int n_rows, int n_experts, int topk,
+                                                          int with_norm) {
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= n_rows) return;
+    float p[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) p[i] = 0.f;
+    constexpr int AHEAD = 8;   // partial sums in flight (one after the other they took 10 us of a one-token call)
+    for (int z0 = 0; z0 < splits; z0 += AHEAD) {
+        float v[AHEAD][PER];
+#pragma unroll
+        for (int z = 0; z < AHEAD; ++z)
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                v[z][i] = part[((size_t)min(z0 + z, splits - 1) * n_rows + row) * n_experts + min(lane + 64 * i, n_experts - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int z = 0; z < AHEAD; ++z)
+#pragma unroll
+            for (int i = 0; i < PER; ++i) p[i] += z0 + z < splits ? v[z][i] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (lane + 64 * i >= n_experts) p[i] = -INFINITY;
+    select_topk_softmax<PER>(p, weights + row * topk, ids + row * topk, n_experts, topk, with_norm, lane);
+}
+
+// The same for one token per workgroup of 16 waves: a wave takes experts w, w + 16, ... and its lanes walk the
+// row together (consecutive lanes read consecutive 16-byte pieces); the selection is run by wave 0 over the
+// logits left in LDS.
 constexpr int GATE_WAVES = 16;
 
 __global__ __launch_bounds__(64 * GATE_WAVES) void gate_topk_softmax_kernel(const float* __restrict__ x_in,
@@ -230,8 +387,32 @@ extern "C" void loken_gate_topk_softmax(const float* x_in, const float* gate_w, 
                                         void* stream) {
     if (!x_in || !gate_w || !weights_out || !ids_out || hidden <= 0 || hidden > 8192) return;   // the caller falls back
     if (!router_sizes_ok(n_rows, n_experts, n_expert_used)) return;
+    hipStream_t s = (hipStream_t)stream;
+    if (hidden % 4 == 0 && (((uintptr_t)x_in | (uintptr_t)gate_w) & 15) == 0) {
+        const int m = n_rows <= 16 ? 16 : 32;
+        const int t_tiles = (n_rows + m - 1) / m, e_tiles = (n_experts + m - 1) / m;
+        // K split until the launch has LOGIT_SPREAD workgroups, while a wave keeps at least two units of K
+        const int units = hidden / m;
+        int splits = LOGIT_SPREAD / (t_tiles < LOGIT_SPREAD ? t_tiles * e_tiles : LOGIT_SPREAD);
+        if (splits > units / (2 * LOGIT_WAVES)) splits = units / (2 * LOGIT_WAVES);
+        if (splits > 16) splits = 16;
+        if (splits < 1) splits = 1;
+        std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
+        float* part = (float*)lk_reserve_scratch((size_t)splits * n_rows * n_experts * 4, s, LK_SCRATCH_ROUTER);
+        if (part) {
+            auto logits = m == 16 ? gate_logits16_kernel : gate_logits32_kernel;
+            hipLaunchKernelGGL(logits, dim3(t_tiles, e_tiles, splits), dim3(64 * LOGIT_WAVES), 0, s, x_in, gate_w, part, hidden, n_rows,
+                               n_experts);
+            const dim3 waves((n_rows + 3) / 4);
+            auto select = n_experts <= 64 ? gate_select_kernel<1> : n_experts <= 128 ? gate_select_kernel<2> : n_experts <= 256 ? gate_select_kernel<4> : gate_select_kernel<8>;
+            hipLaunchKernelGGL(select, waves, dim3(256), 0, s, (const float*)part, splits, weights_out, ids_out, n_rows, n_experts,
+                               n_expert_used, with_norm);
+            (void)hipGetLastError();
+            return;
+        }
+    }
     const int lds = (((hidden + 3) & ~3) + n_experts) * 4;
-    hipLaunchKernelGGL(gate_topk_softmax_kernel, dim3(n_rows), dim3(64 * GATE_WAVES), lds, (hipStream_t)stream, x_in,
+    hipLaunchKernelGGL(gate_topk_softmax_kernel, dim3(n_rows), dim3(64 * GATE_WAVES), lds, s, x_in,
                        gate_w, weights_out, ids_out, hidden, n_experts, n_expert_used, with_norm);
     (void)hipGetLastError();
 }

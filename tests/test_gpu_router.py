@@ -18,7 +18,8 @@ def dev(a):
 @pytest.mark.parametrize("tokens,hidden,experts,k,renorm", [(1, 2048, 128, 8, True), (16, 2048, 128, 8, True),
                                                             (256, 2048, 128, 8, False), (3, 4096, 64, 4, True),
                                                             (2, 1030, 32, 2, True), (5, 8192, 256, 8, True),
-                                                            (2, 514, 40, 3, False)])
+                                                            (2, 514, 40, 3, False), (17, 1028, 33, 4, True), (16, 36, 65, 5, True),
+                                                            (97, 2048, 129, 8, True), (1111, 768, 512, 8, True)])
 def test_gate_topk_softmax_matches_the_two_step_path(tokens, hidden, experts, k, renorm):
     x = synth.normal(20, 1, tokens * hidden).reshape(tokens, hidden)
     gate = (synth.normal(20, 2, experts * hidden) * (1.5 / np.sqrt(hidden))).reshape(experts, hidden).astype(np.float32)
