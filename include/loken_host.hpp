@@ -1,8 +1,7 @@
 /* Host side of the quantized linear above the C ABI of loken_gfx950.h, in C++: the mirror of
  * loken's QKernelMatMul for the card path (src/tensor/quantized/kernel_matmul.rs:1086-1714,
  * kernel_matmul/mmq.rs:21-159): which kernel family a call takes by its row count, the grow-only
- * per-device workspaces with the host mutex held across a quantize -> consume pair of launches,
- * and the event that orders workspace reuse between streams. Rust is what the reference's host is
+ * workspaces per stream with the host mutex held across a quantize -> consume pair of launches. Rust is what the reference's host is
  * written in; this is the same logic for a C++ caller, and what a Rust binding to this library
  * would keep doing on its own side.
  *
@@ -48,8 +47,8 @@ public:
     QKernelMatMul(int dtype, int n, int k, const void* blob, int device);
 
     /* x [rows, k] (LK_TYPE_F32, F16 or BF16) -> out [rows, n] in x's type, on `stream`. The
-     * matrix-unit kernels write f32 rows; for f16 / bf16 rows they write into a buffer of the device's
-     * slot and one more launch rounds them into `out` (the reference narrows the f32 rows its
+     * matrix-unit kernels write f32 rows; for f16 / bf16 rows they write into a buffer of the stream's
+     * scratch and one more launch rounds them into `out` (the reference narrows the f32 rows its
      * mmq_forward returns the same way, kernel_matmul.rs:1086-1714). `decode_order` keeps every row on the mat-vec
      * kernels whatever the count (DecodeOrder of the reference, kernel_matmul.rs:34-75).
      * Returns LK_OK or an LK_ERR_* code; never throws, never aborts. */

@@ -1,14 +1,13 @@
 // Host mirror of loken's QKernelMatMul for the card path: see include/loken_host.hpp.
 
 #include "../../include/loken_host.hpp"
+#include "stream_scratch.h"
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
-#include <map>
 #include <type_traits>
-#include <mutex>
 
 namespace loken {
 namespace {
@@ -18,100 +17,6 @@ constexpr size_t MMQ_RECORD = 144;                      // bytes per 128 padded 
 constexpr size_t FIXUP_BYTES = 256u * 128u * 128u * 4u;  // kernel_matmul/mmq.rs:42
 
 size_t pad_to(size_t v, size_t m) { return (v + m - 1) / m * m; }
-
-// One device's buffers. `mu` is held across a quantize -> consume pair so that two host threads
-// sharing the card's stream cannot interleave their pairs (fast_mmvq.rs:15-32,
-// kernel_matmul/mmq.rs:43-86); `last_use` orders a later user on ANOTHER stream behind the
-// kernels enqueued here (the host mutex alone orders only the enqueueing).
-struct Slot {
-    std::mutex mu;
-    void* act = nullptr;      // Q8_1 rows / tiled-matmul workspace
-    size_t act_bytes = 0;
-    void* fixup = nullptr;
-    void* out32 = nullptr;    // f32 result rows of a call whose rows came in f16 / bf16 (the matrix-unit kernels write f32)
-    size_t out32_bytes = 0;
-    hipEvent_t last_use = nullptr;
-    bool used = false;
-};
-
-std::mutex g_slots_mu;
-std::map<int, Slot*> g_slots;
-
-Slot& slot_of(int device) {
-    std::lock_guard<std::mutex> lock(g_slots_mu);
-    auto it = g_slots.find(device);
-    if (it != g_slots.end()) return *it->second;
-    Slot* s = new Slot();
-    g_slots.emplace(device, s);
-    return *s;
-}
-
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return st != hipStreamCaptureStatusNone;
-}
-
-// Grow-only, zero-filled. Never grows while `stream` records a graph (an allocation is not a
-// capturable operation): the caller warms the size up outside the capture, as with the MoE scratch.
-int reserve(Slot& slot, size_t bytes, bool want_fixup, hipStream_t stream) {
-    const bool rec = capturing(stream);
-    if (slot.act_bytes < bytes) {
-        if (rec) return LK_ERR_NOMEM;
-        if (slot.act) {   // release the smaller one first: no double peak (kernel_matmul/mmq.rs:49-53)
-            if (hipStreamSynchronize(stream) != hipSuccess || hipFree(slot.act) != hipSuccess) (void)hipGetLastError();
-            slot.act = nullptr;
-            slot.act_bytes = 0;
-        }
-        if (hipMalloc(&slot.act, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            slot.act = nullptr;
-            return LK_ERR_NOMEM;
-        }
-        slot.act_bytes = bytes;
-        if (hipMemsetAsync(slot.act, 0, bytes, stream) != hipSuccess) (void)hipGetLastError();
-    }
-    if (want_fixup && !slot.fixup) {
-        if (rec) return LK_ERR_NOMEM;
-        if (hipMalloc(&slot.fixup, FIXUP_BYTES) != hipSuccess) {
-            (void)hipGetLastError();
-            slot.fixup = nullptr;
-            return LK_ERR_NOMEM;
-        }
-        if (hipMemsetAsync(slot.fixup, 0, FIXUP_BYTES, stream) != hipSuccess) (void)hipGetLastError();
-    }
-    if (!slot.last_use && !rec) {
-        if (hipEventCreateWithFlags(&slot.last_use, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            slot.last_use = nullptr;
-        }
-    }
-    // queue behind whoever used the buffers last; a graph being recorded neither waits nor marks
-    if (slot.used && slot.last_use && !rec && hipStreamWaitEvent(stream, slot.last_use, 0) != hipSuccess)
-        (void)hipGetLastError();
-    return LK_OK;
-}
-
-// The f32 rows a half-precision call's kernels write before they are narrowed into the caller's buffer.
-int reserve_out32(Slot& slot, size_t bytes, hipStream_t stream) {
-    if (slot.out32_bytes >= bytes) return LK_OK;
-    if (capturing(stream)) return LK_ERR_NOMEM;
-    if (slot.out32) {
-        if (hipStreamSynchronize(stream) != hipSuccess || hipFree(slot.out32) != hipSuccess) (void)hipGetLastError();
-        slot.out32 = nullptr;
-        slot.out32_bytes = 0;
-    }
-    if (hipMalloc(&slot.out32, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        slot.out32 = nullptr;
-        return LK_ERR_NOMEM;
-    }
-    slot.out32_bytes = bytes;
-    return LK_OK;
-}
 
 template <typename T>
 __global__ __launch_bounds__(256) void narrow_rows_kernel(const float* __restrict__ from, T* __restrict__ to, size_t count) {
@@ -128,13 +33,6 @@ int narrow_rows(const float* from, void* to, int type, size_t count, hipStream_t
     if (type == LK_TYPE_F16) hipLaunchKernelGGL(narrow_rows_kernel<__half>, dim3(grid), dim3(256), 0, stream, from, (__half*)to, count);
     else hipLaunchKernelGGL(narrow_rows_kernel<__hip_bfloat16>, dim3(grid), dim3(256), 0, stream, from, (__hip_bfloat16*)to, count);
     return hipGetLastError() == hipSuccess ? LK_OK : LK_ERR_LAUNCH;
-}
-
-void mark_used(Slot& slot, hipStream_t stream) {
-    if (slot.last_use && !capturing(stream)) {
-        if (hipEventRecord(slot.last_use, stream) != hipSuccess) (void)hipGetLastError();
-        slot.used = true;
-    }
 }
 
 // The 32-value nibble formats and the two-bit K-quants: served by the plain mat-vec (four of them by the
@@ -235,7 +133,8 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
         return LK_ERR_ARG;   // "input on a different device" (kernel_matmul.rs:1499-1503)
     }
     const int mv_max = matvec_rows(dtype_, k_);
-    Slot& slot = slot_of(device_);
+    // a quantize -> consume pair holds the stream's scratch, so that two host threads sharing the stream cannot
+    // interleave their pairs (fast_mmvq.rs:15-32, kernel_matmul/mmq.rs:43-86)
 
     // --- mat-vec family: up to matvec_rows, or any count when every row must sum like a one-row call
     const bool rows_kernel_fits = k_ % 256 == 0 && ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q6_K ? 1 : 15)) == 0;
@@ -251,17 +150,18 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
             return lk_mmvq_fused(dtype_, 1, vx, (const float*)x, k_, dst, x_type, k_, nn, rows, n_, nullptr, stream);
         }
         const int k_padded = (int)pad_to((size_t)k_, 512), blocks = k_padded / 32;
-        std::lock_guard<std::mutex> pair(slot.mu);
-        if (int rc = reserve(slot, (size_t)rows * blocks * Q81_BLOCK, false, stream)) return rc;
-        if (int rc = lk_quantize_q8_1(x, x_type, slot.act, k_, k_padded, rows, stream)) return rc;
+        const auto scratch = lk_stream_scratch(stream);
+        std::lock_guard<std::recursive_mutex> pair(scratch->mu);
+        uint8_t* act = (uint8_t*)scratch->get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK, stream);
+        if (!act) return LK_ERR_NOMEM;
+        if (int rc = lk_quantize_q8_1(x, x_type, act, k_, k_padded, rows, stream)) return rc;
         for (int r0 = 0; r0 < rows; r0 += 8) {
             const int b = rows - r0 < 8 ? rows - r0 : 8;
-            const int rc = lk_mmvq(dtype_, blob_, (const uint8_t*)slot.act + (size_t)r0 * blocks * Q81_BLOCK,
+            const int rc = lk_mmvq(dtype_, blob_, act + (size_t)r0 * blocks * Q81_BLOCK,
                                    (uint8_t*)out + (size_t)r0 * n_ * elem_bytes(x_type), x_type, k_, n_, b, blocks, n_,
                                    nullptr, decode_order ? 1 : 0, stream);
             if (rc) return rc;
         }
-        mark_used(slot, stream);
         last_path_ = Path::MatVec;
         return LK_OK;
     };
@@ -270,7 +170,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     // The matrix-unit kernels write f32 rows. Rows that came in f16 / bf16 leave in that type, as the
     // reference's do (the f32 rows its mmq_forward returns are narrowed by the caller,
     // src/tensor/quantized/kernel_matmul.rs:1086-1714): the kernels write into a buffer of the
-    // device's slot and one more launch rounds them into `out`.
+    // stream's scratch and one more launch rounds them into `out`.
     const bool half_rows = x_type != LK_TYPE_F32;
     const size_t out_count = (size_t)rows * n_;
 
@@ -280,19 +180,18 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
         const int blocks = k_ / 32;
         int rc;
         {
-            std::lock_guard<std::mutex> pair(slot.mu);
-            if (int r = reserve(slot, (size_t)rows * blocks * Q81_BLOCK, false, stream)) return r;
-            if (half_rows)
-                if (int r = reserve_out32(slot, out_count * 4, stream)) return r;
-            float* dst = half_rows ? (float*)slot.out32 : (float*)out;
-            if (int r = lk_quantize_q8_1(x, x_type, slot.act, k_, k_, rows, stream)) return r;
+            const auto scratch = lk_stream_scratch(stream);
+            std::lock_guard<std::recursive_mutex> pair(scratch->mu);
+            void* act = scratch->get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK, stream);
+            float* dst = half_rows ? (float*)scratch->get(LK_SCRATCH_LINEAR_F32, out_count * 4, stream) : (float*)out;
+            if (!act || !dst) return LK_ERR_NOMEM;
+            if (int r = lk_quantize_q8_1(x, x_type, act, k_, k_, rows, stream)) return r;
             // the launchers with a status (the exported void forms drop it): rows too long for their scale
             // tables in LDS launch nothing, and the call goes on to the mat-vec or the tiled matmul below
-            rc = dtype_ == LK_TYPE_Q4_K   ? lk_dense_q4k_rows(blob_, slot.act, dst, rows, n_, k_, stream)
-                 : dtype_ == LK_TYPE_Q5_K ? lk_dense_q5k_rows(blob_, slot.act, dst, rows, n_, k_, stream)
-                                          : lk_dense_q6k_rows(blob_, slot.act, dst, rows, n_, k_, stream);
+            rc = dtype_ == LK_TYPE_Q4_K   ? lk_dense_q4k_rows(blob_, act, dst, rows, n_, k_, stream)
+                 : dtype_ == LK_TYPE_Q5_K ? lk_dense_q5k_rows(blob_, act, dst, rows, n_, k_, stream)
+                                          : lk_dense_q6k_rows(blob_, act, dst, rows, n_, k_, stream);
             if (rc == LK_OK && half_rows) rc = narrow_rows(dst, out, x_type, out_count, stream);
-            mark_used(slot, stream);
         }
         if (rc == LK_OK) {
             last_path_ = Path::RowsOnMatrixUnit;
@@ -306,17 +205,18 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     if (!tiled_serves(dtype_, k_)) return LK_ERR_TYPE;
     const size_t k_padded = pad_to(pad_to((size_t)k_, 512), 128);
     const size_t ws_bytes = (size_t)rows * (k_padded / 128) * MMQ_RECORD + 128 * MMQ_RECORD;
-    std::lock_guard<std::mutex> pair(slot.mu);
-    if (int rc = reserve(slot, ws_bytes, true, stream)) return rc;
-    if (half_rows)
-        if (int rc = reserve_out32(slot, out_count * 4, stream)) return rc;
-    void* dst = half_rows ? slot.out32 : out;
+    const auto scratch = lk_stream_scratch(stream);
+    std::lock_guard<std::recursive_mutex> pair(scratch->mu);
+    void* act = scratch->get(LK_SCRATCH_LINEAR, ws_bytes, stream);
+    void* fixup = scratch->get(LK_SCRATCH_FIXUP, FIXUP_BYTES, stream);
+    void* dst = half_rows ? scratch->get(LK_SCRATCH_LINEAR_F32, out_count * 4, stream) : out;
+    if (!act || !fixup || !dst) return LK_ERR_NOMEM;
     // the layouts of the reference's table (quantized/mmq.rs:274-285)
     auto quantizer = dtype_ == LK_TYPE_Q2_K ? launch_mmq_quantize_q8_1_D2S6
                      : dtype_ == LK_TYPE_Q6_K || dtype_ == LK_TYPE_Q8_0 || dtype_ == LK_TYPE_Q5_0 || dtype_ == LK_TYPE_Q3_K
                          ? launch_mmq_quantize_q8_1_D4
                          : launch_mmq_quantize_q8_1_DS4;
-    quantizer(x, nullptr, slot.act, x_type, k_, k_, 0, 0, (int64_t)k_padded, rows, 1, 1, stream);
+    quantizer(x, nullptr, act, x_type, k_, k_, 0, 0, (int64_t)k_padded, rows, 1, 1, stream);
     auto launcher = dtype_ == LK_TYPE_Q4_K   ? launch_mmq_gguf_q4_k
                     : dtype_ == LK_TYPE_Q5_K ? launch_mmq_gguf_q5_k
                     : dtype_ == LK_TYPE_Q6_K ? launch_mmq_gguf_q6_k
@@ -329,11 +229,10 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
                                              : launch_mmq_gguf_q8_0;
     int abi = 0, cus = 0, lds = 0, wave = 0;
     (void)lk_device_info(&abi, &cus, &lds, &wave);
-    const int tile = launcher(slot.fixup, blob_, slot.act, dst, k_, n_, rows, k_ / block_len, n_, 0x1000950, cus, lds, wave,
+    const int tile = launcher(fixup, blob_, act, dst, k_, n_, rows, k_ / block_len, n_, 0x1000950, cus, lds, wave,
                               stream);
     int narrowed = LK_OK;
     if (tile != 0 && half_rows) narrowed = narrow_rows((const float*)dst, out, x_type, out_count, stream);
-    mark_used(slot, stream);
     if (tile == 0) return LK_ERR_ARG;   // "no tile fits, nothing ran": the reference falls back to dequantized
     if (narrowed != LK_OK) return narrowed;
     last_path_ = Path::Tiled;
@@ -422,29 +321,7 @@ int QKernelMatMul::forward_quantized_pair(QKernelMatMul& other, const QuantizedA
     return LK_OK;
 }
 
-void release_workspaces() {
-    std::lock_guard<std::mutex> lock(g_slots_mu);
-    int current = 0;
-    (void)hipGetDevice(&current);
-    for (auto& kv : g_slots) {
-        Slot& s = *kv.second;
-        std::lock_guard<std::mutex> pair(s.mu);
-        if (hipSetDevice(kv.first) != hipSuccess) { (void)hipGetLastError(); continue; }
-        (void)hipDeviceSynchronize();
-        if (s.act) (void)hipFree(s.act);
-        if (s.fixup) (void)hipFree(s.fixup);
-        if (s.out32) (void)hipFree(s.out32);
-        s.out32 = nullptr;
-        s.out32_bytes = 0;
-        if (s.last_use) (void)hipEventDestroy(s.last_use);
-        s.act = s.fixup = nullptr;
-        s.act_bytes = 0;
-        s.last_use = nullptr;
-        s.used = false;
-    }
-    (void)hipSetDevice(current);
-    (void)hipGetLastError();
-}
+void release_workspaces() { lk_stream_scratch_release(-1); }
 
 }  // namespace loken
 

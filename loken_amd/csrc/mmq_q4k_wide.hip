@@ -16,8 +16,8 @@
 // and everything else, and the per-sub-block fma is 16 vector instructions against two matrix
 // instructions, so the kernel is bound by vector issue and every other vector instruction counts:
 //   * the token side is expanded ONCE per call by `q4k_tokens_f16_kernel` into operand order (f16
-//     codes, f32 scales, the bf16 pieces of d8 * S): 74 KiB per (128-token tile, block), in memory
-//     the library keeps per stream. The tile kernel then spends nothing on tokens.
+//     codes, f32 scales, the bf16 pieces of d8 * S): 74 KiB per (128-token tile, block), in the
+//     stream's scratch. The tile kernel then spends nothing on tokens.
 //   * a wave owns 32 weight rows x 128 tokens (four tiles of v_mfma_f32_32x32x16_f16, registers <->
 //     weight rows, lanes <-> tokens), so the nibble expansion of its rows is shared by four token
 //     tiles instead of two.
@@ -32,10 +32,9 @@
 //     expansion and the previous block's d / dmin update spread over the slots.
 
 #include "mmq_problem.h"
+#include "stream_scratch.h"
 
-#include <mutex>
 #include <utility>
-#include <vector>
 
 namespace {
 
@@ -456,58 +455,11 @@ __global__ __launch_bounds__(Wd::THREADS, 1) void q4k_wide_dense_kernel(MmqProbl
     wide_tile(pb, units + (int64_t)m_tile * pb.nb * Wd::UNIT, n_tile * Wd::TN, pb.m_begin + m_tile * Wd::TM, lds);
 }
 
-// ------------------------------------------------------------------ the units' memory
-// Grow-only, one buffer per (device, stream), as the MoE decode launchers keep theirs; released by
-// loken_stream_scratch_release. A call whose tokens need more than the cap runs in several passes
-// of token tiles over the same buffer (stream order keeps them apart).
-struct UnitSlot {
-    int device;
-    hipStream_t stream;
-    void* ptr = nullptr;
-    size_t size = 0;
-    std::vector<void*> kept;   // outgrown buffers: queued kernels may still read them
-};
-std::mutex g_units_mu;
-std::vector<UnitSlot> g_units;
+// The units live in the stream's scratch. A call whose tokens need more than the cap runs in several passes of
+// token tiles over the same buffer (stream order keeps them apart).
 constexpr size_t UNITS_CAP = (size_t)256 << 20;
 
-void* reserve_units(size_t bytes, hipStream_t stream) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    UnitSlot* slot = nullptr;
-    for (auto& s : g_units)
-        if (s.device == dev && s.stream == stream) slot = &s;
-    if (!slot) {
-        g_units.push_back(UnitSlot{dev, stream});
-        slot = &g_units.back();
-    }
-    if (slot->size >= bytes) return slot->ptr;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;   // growing allocates, which a recording stream may not do
-    if (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return nullptr;
-    (void)hipGetLastError();
-    void* fresh = nullptr;
-    const size_t want = (bytes + 255) & ~(size_t)255;
-    if (hipMalloc(&fresh, want) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (slot->ptr) slot->kept.push_back(slot->ptr);
-    slot->ptr = fresh;
-    slot->size = want;
-    return fresh;
-}
-
 }  // namespace
-
-void lk_mmq_q4k_wide_release(int device) {
-    std::lock_guard<std::mutex> lock(g_units_mu);
-    for (auto it = g_units.begin(); it != g_units.end();) {
-        if (it->device != device) { ++it; continue; }
-        if (it->ptr) (void)hipFree(it->ptr);
-        for (void* p : it->kept) (void)hipFree(p);
-        it = g_units.erase(it);
-    }
-}
 
 int lk_mmq_q4k_wide_dense(const MmqProblem& pb, hipStream_t s) {
     using C = Wd;
@@ -520,8 +472,9 @@ int lk_mmq_q4k_wide_dense(const MmqProblem& pb, hipStream_t s) {
     const size_t tile_bytes = (size_t)pb.nb * C::UNIT;
     if (tile_bytes > UNITS_CAP) return -1;
     const int tiles_per_pass = (int)std::min<size_t>((size_t)m_tiles, UNITS_CAP / tile_bytes);
-    std::lock_guard<std::mutex> lock(g_units_mu);   // the buffer is the stream's from here until the launches are queued
-    uint8_t* units = (uint8_t*)reserve_units(tile_bytes * tiles_per_pass, s);
+    const auto scratch = lk_stream_scratch(s);
+    std::lock_guard<std::recursive_mutex> lock(scratch->mu);   // the buffer is the stream's from here until the launches are queued
+    uint8_t* units = (uint8_t*)scratch->get(LK_SCRATCH_TOKENS, tile_bytes * tiles_per_pass, s);
     if (!units) return -1;
     for (int t0 = 0; t0 < m_tiles; t0 += tiles_per_pass) {
         const int tiles = std::min(tiles_per_pass, m_tiles - t0);

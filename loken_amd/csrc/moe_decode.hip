@@ -6,8 +6,8 @@
 //   expert_ids[i] its expert; gate/up read activation row slot / topk and write row slot; down
 //   reads row slot, scales by topk_weights[slot] and writes row slot of a scratch that a fold
 //   then sums per token IN SLOT ORDER (no atomics, the same sum on every run).
-// The launchers quantize the activation themselves into a per-(device, stream) grow-only
-// scratch, as the reference's do; loken_stream_scratch_release frees it.
+// The launchers quantize the activation themselves into the stream's scratch (stream_scratch.h), as the
+// reference's do; loken_stream_scratch_release frees it.
 //
 // Kernels: grid (row tiles, pairs); each workgroup stages its pair's Q8_1 row into LDS and runs
 // the shared mat-vec row engine on the pair's expert slab. SiLU uses the accurate expf, as the
@@ -31,19 +31,6 @@ int lk_moe_down_fold(int quant_type, const float* inputs, const void* weights, c
                      bool write, hipStream_t stream);
 
 namespace {
-
-// ---------------------------------------------------------------- stream scratch (stream_scratch.h)
-struct ScratchSlot {
-    int device;
-    hipStream_t stream;
-    LkScratchUse use;
-    void* ptr = nullptr;
-    size_t size = 0;
-    std::vector<void*> kept;  // outgrown buffers: queued kernels may still read them
-};
-std::vector<ScratchSlot> g_scratch;
-
-void* reserve_scratch(size_t bytes, hipStream_t stream) { return lk_reserve_scratch(bytes, stream, LK_SCRATCH_LAUNCHER); }
 
 // ---------------------------------------------------------------- static scratch
 // Scratch of the entry point that allocates nothing (loken_moe_gemm_gguf_down_reduce_static): a
@@ -255,53 +242,9 @@ static inline bool rows_stage_as_f32(const float* inputs, int size_k, int quant_
 
 }  // namespace
 
-std::recursive_mutex& lk_scratch_mutex() {
-    static std::recursive_mutex mu;
-    return mu;
-}
-
-void* lk_reserve_scratch(size_t bytes, hipStream_t stream, LkScratchUse use) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    ScratchSlot* slot = nullptr;
-    for (auto& s : g_scratch)
-        if (s.device == dev && s.stream == stream && s.use == use) slot = &s;
-    if (!slot) {
-        g_scratch.push_back(ScratchSlot{dev, stream, use});
-        slot = &g_scratch.back();
-    }
-    if (slot->size >= bytes) return slot->ptr;
-    // growing allocates, which a stream under capture may not do
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return nullptr;
-    (void)hipGetLastError();
-    size_t want = bytes + bytes / 4;
-    want = (want + 255) & ~(size_t)255;
-    void* fresh = nullptr;
-    if (hipMalloc(&fresh, want) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (slot->ptr) slot->kept.push_back(slot->ptr);
-    slot->ptr = fresh;
-    slot->size = want;
-    return fresh;
-}
-
-void lk_mmq_q4k_wide_release(int device);   // mmq_q4k_wide.hip: the token-side operand buffers of the wide Q4_K tiles
-
 extern "C" void loken_stream_scratch_release() {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return;
-    (void)hipDeviceSynchronize();   // queued kernels may still read what is freed below
-    lk_mmq_q4k_wide_release(dev);
-    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
-    for (auto it = g_scratch.begin(); it != g_scratch.end();) {
-        if (it->device != dev) { ++it; continue; }
-        if (it->ptr) (void)hipFree(it->ptr);
-        for (void* p : it->kept) (void)hipFree(p);
-        it = g_scratch.erase(it);
-    }
+    if (hipGetDevice(&dev) == hipSuccess) lk_stream_scratch_release(dev);
 }
 
 extern "C" void loken_moe_sum_topk(const float* pairs, float* outputs, int tokens, int topk, int cols, void* stream) {
@@ -329,8 +272,9 @@ extern "C" int loken_moe_gemm_gguf(const float* inputs, const void* weights, con
         return launch_format<MODE_PLAIN>(quant_type, (const uint8_t*)weights, nullptr, (const uint8_t*)inputs,
                                          sorted_token_ids, expert_ids, topk_weights, nullptr, (float*)outputs, d, size_k, s);
     }
-    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
-    uint8_t* acts = (uint8_t*)reserve_scratch((size_t)act_rows * (kp / 32) * Q81_BYTES, s);
+    const auto scratch = lk_stream_scratch(s);
+    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
+    uint8_t* acts = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES, s);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, LK_TYPE_F32, acts, size_k, kp, act_rows, stream)) return rc;
     MoeDims d{num_experts, topk, size_m, size_n, 0, kp / 32, 0};
@@ -359,8 +303,9 @@ extern "C" int loken_moe_gemm_gguf_prefill(const void* inputs, const uint8_t* we
     hipStream_t s = (hipStream_t)stream;
     const int kp = pad512(size_k);
     const int act_rows = topk_weights ? size_m : size_m / topk;
-    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
-    uint8_t* acts = (uint8_t*)reserve_scratch((size_t)act_rows * (kp / 32) * Q81_BYTES, s);
+    const auto scratch = lk_stream_scratch(s);
+    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
+    uint8_t* acts = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES, s);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, input_dtype == 0 ? LK_TYPE_F16 : LK_TYPE_BF16, acts, size_k, kp, act_rows, stream))
         return rc;
@@ -397,8 +342,9 @@ static int gate_up_impl(const float* inputs, const void* gate_weights, const voi
                                          (const uint8_t*)inputs, sorted_token_ids, expert_ids, nullptr, nullptr, outputs,
                                          d, size_k, s);
     }
-    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
-    uint8_t* acts = (uint8_t*)reserve_scratch((size_t)act_rows * (kp / 32) * Q81_BYTES, s);
+    const auto scratch = lk_stream_scratch(s);
+    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
+    uint8_t* acts = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES, s);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, LK_TYPE_F32, acts, size_k, kp, act_rows, stream)) return rc;
     MoeDims d{num_experts, topk, size_m, size_n, 0, kp / 32, 0, 0, slab_rows, act, live, alt};
@@ -507,7 +453,8 @@ static int down_impl(const float* inputs, const void* weights, const int32_t* so
     const bool as_f32 = rows_stage_as_f32(inputs, size_k, gguf_dtype);
     const size_t act_bytes = as_f32 ? 0 : (((size_t)size_m * (kp / 32) * Q81_BYTES) + 255) & ~(size_t)255;
     const size_t pair_bytes = pair_rows ? 0 : (size_t)size_m * size_n * sizeof(float);
-    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
+    const auto scratch = lk_stream_scratch(s);
+    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
     uint8_t* base = nullptr;
     if (from_static) {
         // nothing is allocated: the device's fixed array, or an error when the call does not fit it
@@ -515,7 +462,7 @@ static int down_impl(const float* inputs, const void* weights, const int32_t* so
         base = static_scratch();
         if (!base) return LK_ERR_LAUNCH;
     } else if (act_bytes + pair_bytes) {
-        base = (uint8_t*)reserve_scratch(act_bytes + pair_bytes, s);
+        base = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, act_bytes + pair_bytes, s);
         if (!base) return LK_ERR_NOMEM;
     }
     float* pairs = pair_rows ? pair_rows : (float*)(base + act_bytes);
@@ -649,8 +596,9 @@ extern "C" int loken_moe_q4k_imma_m8_down(const void* weights, const void* q8_1,
     if (!weights || !q8_1 || !sorted_token_ids || !expert_ids || !topk_weights || !output ||
         bad_shape(1, num_experts, topk, size_m, hidden, size_k) || (((uintptr_t)q8_1) & 3) != 0) return LK_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
-    std::lock_guard<std::recursive_mutex> lock(lk_scratch_mutex());
-    float* pairs = (float*)reserve_scratch((size_t)size_m * hidden * sizeof(float), s);
+    const auto scratch = lk_stream_scratch(s);
+    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
+    float* pairs = (float*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)size_m * hidden * sizeof(float), s);
     if (!pairs) return LK_ERR_NOMEM;
     // a pair whose slot is out of range writes nothing: its row of the sum must read zero
     const size_t n = (size_t)size_m * hidden;

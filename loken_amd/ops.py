@@ -18,7 +18,8 @@ _X_TYPES = {torch.float32: _lib.TYPE_F32, torch.float16: _lib.TYPE_F16, torch.bf
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle alone: torch.cuda.current_stream() builds a Stream object around it, 2.9 us a call
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def pad_to(v: int, m: int) -> int:
