@@ -141,7 +141,7 @@ struct MmqQ45K {
     static constexpr int ALIGN = 4;   // whole-header reads
     static constexpr int BLOCK_BYTES = Q5 ? Q5K_BYTES : Q4K_BYTES;
     static constexpr int QS0 = Q5 ? 48 : 16;
-    static constexpr bool F16_TILES = !Q5;   // Q4_K above 32 tokens (dense) or 64 (expert-batched): the f16 tile kernels
+    static constexpr int F16_TYPE = Q5 ? LK_TYPE_Q5_K : LK_TYPE_Q4_K;   // the f16 tile kernels take it (mmq_f16.hip)
     static constexpr int WIDE_FROM = 384;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int NS = 8;          // one weight scale per 32 values
     static constexpr bool HAS_MIN = true;
@@ -226,7 +226,7 @@ struct MmqQ6K {
     static constexpr int NS = 16;
     static constexpr bool HAS_MIN = false;
     static constexpr int MIN_RANK = 0;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = LK_TYPE_Q6_K;
     static constexpr int WIDE_FROM = 384;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 1;
     static constexpr int QCH = TN * 8 / MMQ_WG;
@@ -292,7 +292,7 @@ struct MmqQ80 {
     static constexpr int NS = 8;
     static constexpr bool HAS_MIN = false;
     static constexpr int MIN_RANK = 0;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = -1;
     static constexpr int WIDE_FROM = 96;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 8;
     static constexpr int QCH = TN * 16 / MMQ_WG, DCH = TN * 8 / MMQ_WG;
@@ -344,7 +344,7 @@ struct MmqLegacy {
     static constexpr int NS = 8;
     static constexpr bool HAS_MIN = L::M_AT >= 0;
     static constexpr int MIN_RANK = HAS_MIN ? 8 : 0;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = -1;
     static constexpr int WIDE_FROM = 300;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 8;
     static constexpr int ALIGN = L::BYTES % 2 ? 1 : 2;
@@ -407,7 +407,7 @@ struct MmqQ3K {
     static constexpr int NS = 16;
     static constexpr bool HAS_MIN = false;
     static constexpr int MIN_RANK = 0;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = -1;
     static constexpr int WIDE_FROM = 384;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 1;
     static_assert(TN * 2 == MMQ_WG, "one (row, half) per thread");
@@ -476,7 +476,7 @@ struct MmqQ2K {
     static constexpr int NS = 16;
     static constexpr bool HAS_MIN = true;
     static constexpr int MIN_RANK = 16;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = -1;
     static constexpr int WIDE_FROM = 384;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 1;
     static_assert(TN * 2 == MMQ_WG, "one (row, half) per thread");
@@ -527,7 +527,7 @@ struct MmqIq4Xs {
     static constexpr int NS = 8;
     static constexpr bool HAS_MIN = false;
     static constexpr int MIN_RANK = 0;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = -1;
     static constexpr int WIDE_FROM = 300;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 1;
     static constexpr int PER = TN * 8 / MMQ_WG;
@@ -578,7 +578,7 @@ struct MmqCodebook {
     static constexpr int NS = ID == 22 ? 16 : 8;
     static constexpr bool HAS_MIN = false;
     static constexpr int MIN_RANK = 0;
-    static constexpr bool F16_TILES = false;
+    static constexpr int F16_TYPE = -1;
     static constexpr int WIDE_FROM = 300;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 8 / C::RUNS;
     static constexpr int PER = TN * 8 / MMQ_WG;
@@ -1001,11 +1001,14 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
     // (Q2_K stays on 64-token tiles: with the rank-16 minimum its 128-token tile spills and runs 512 x
     // 4096 -> 14336 in 344 us against 240, 2048 x 14336 -> 4096 in 1155 against 742; every other format
     // is 3 to 40 % faster on the wide tile)
-    // (Q4_K from 33 rows of a matrix of 2048 rows or more goes on to its 64-token f16 tiles: 14336 x 4096 at 64
-    // rows 40.5 us against 46.4 on the int8 tiles, 4096 x 14336 43.8 against 49.1, 4096 x 4096 the same 33)
-    const bool f16_from_33 = F::F16_TILES && nrows_x >= 2048 && !lk_env_flag("LK_MMQ_I8");
+    // (Q4_K, Q5_K and Q6_K from 33 rows of a matrix of 2048 rows or more go on to the 64-token f16 tiles, quantizer
+    // included against the int8 tiles: Q4_K 14336 x 4096 at 64 rows 40.5 us against 46.4, 4096 x 14336 43.8 against
+    // 49.1, 4096 x 4096 the same 33; Q5_K 14336 x 4096 at 64 / 512 / 2048 rows 33 / 138 / 495 against 36 / 169 / 631,
+    // 4096 x 4096 at 77 / 512 26 / 50 against 28 / 59; Q6_K 14336 x 4096 38 / 171 / 609 against 40 / 187 / 703,
+    // 4096 x 14336 at 2048 576 against 654, 4096 x 4096 at 64 / 512 28 / 59 against 26 / 66)
+    const bool f16_from_33 = F::F16_TYPE >= 0 && nrows_x >= 2048 && !lk_env_flag("LK_MMQ_I8");
     if ((ncols_y <= 64 && !f16_from_33) || F::MIN_RANK == 16) return launch_dense_tm<F, 64, 2>(pb, s, fixup);
-    if constexpr (F::F16_TILES) {   // Q4_K: scales folded into f16 operands
+    if constexpr (F::F16_TYPE >= 0) {   // Q4_K, Q5_K, Q6_K: scales folded into f16 operands
         // (under 2048 weight rows the 256-row f16 tiles are too few even with K cut: 1024 x 4096 at 512 / 1024 /
         // 2048 rows 48 / 63 / 93 us against 38 / 49 / 73 on the int8 tiles)
         if (!lk_env_flag("LK_MMQ_I8") && nrows_x >= 2048) {
@@ -1014,11 +1017,11 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
             // enough to occupy half the CUs (fewer: the 64-token tiles, which can cut K)
             const int64_t pad128 = (ncols_y + 127) / 128 * 128, pad64 = (ncols_y + 63) / 64 * 64;
             const int64_t wide_tiles = (nrows_x + 255) / 256 * (pad128 / 128);
-            if (ncols_y > 128 && 10 * pad128 <= 11 * pad64 && 2 * wide_tiles > lk_device().cus && !lk_env_flag("LK_MMQ_NO_WIDE")) {
+            if (F::F16_TYPE == LK_TYPE_Q4_K && ncols_y > 128 && 10 * pad128 <= 11 * pad64 && 2 * wide_tiles > lk_device().cus && !lk_env_flag("LK_MMQ_NO_WIDE")) {
                 const int tm = lk_mmq_q4k_wide_dense(pb, s);
                 if (tm >= 0) return tm;
             }
-            const int tm = lk_mmq_q4k_f16_dense(pb, s, fixup);
+            const int tm = lk_mmq_f16_dense(F::F16_TYPE, pb, s, fixup);
             if (tm >= 0) return tm;
         }
     }
@@ -1073,26 +1076,28 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
     const int64_t want = mmq_x > 0 ? mmq_x : (ncols_hint > 0 ? ncols_hint : ncols_max);
     if (want <= 32) return launch_moe_tm<F, 32, 1>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     if (want <= 64) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-    // The 128-token tile of this kernel (the routing's bounds and destination map on top of the dense
-    // tile's registers) runs out of registers for the formats with a minimum or two scales per sub-block
-    // and loses to the 64-token tile: 128 experts of 2048 -> 768 -> 2048, top-8, gate + up and down,
-    // 2048 tokens: Q6_K 954 us against 1352, Q5_K 739 against 1231; 4096 tokens: 1608 against 1991, 1297
-    // against 1787 (Q8_0 and Q4_0 go either way by a tenth and keep the wide tile).
-    if constexpr (!F::F16_TILES && (F::HAS_MIN || F::NS == 16))
+    // Runs of more than 64 rows: the f16 tiles for the formats that have them (128 experts of 2048 -> 768 -> 2048, top-8,
+    // Q4_K gate + up, 1111 / 1400 tokens, whole block, against the int8 tiles: Q4_K down 400 / 441 us against 512 / 542,
+    // Q5_K 430 / 464 against 518 / 540, Q6_K 464 / 500 against 573 / 599).
+    if constexpr (F::F16_TYPE >= 0) {
+        if (!lk_env_flag("LK_MMQ_I8")) {
+            const int tm = lk_mmq_f16_moe(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
+            if (tm >= 0) return tm;
+        }
+    }
+    // The 128-token int8 tile (the routing's bounds and destination map on top of the dense tile's registers) runs out
+    // of registers for the formats with a minimum or two scales per sub-block and loses to the 64-token tile (2048
+    // tokens, all three stacks: Q6_K 954 us against 1352, Q5_K 739 against 1231); Q8_0 and Q4_0 go either way by a
+    // tenth and keep the wide tile.
+    if constexpr (F::F16_TYPE != LK_TYPE_Q4_K && (F::HAS_MIN || F::NS == 16))
         return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     else {
         // Left to choose (no mmq_x), the narrower tile where it pads the expected longest run a fifth
         // less: a run of 150 rows is three tiles of 64 or two of 128, the second nearly empty (2048
         // tokens, as above: Q8_0 1198 us against 1300, Q4_0 742 against 983; at 1024 and 4096 tokens the
         // runs fill the wide tiles and those win by a tenth).
-        if (!F::F16_TILES && mmq_x <= 0 && 5 * ((want + 63) / 64 * 64) <= 4 * ((want + 127) / 128 * 128))
+        if (F::F16_TYPE < 0 && mmq_x <= 0 && 5 * ((want + 63) / 64 * 64) <= 4 * ((want + 127) / 128 * 128))
             return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-        if constexpr (F::F16_TILES) {
-            if (!lk_env_flag("LK_MMQ_I8")) {
-                const int tm = lk_mmq_q4k_f16_moe(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-                if (tm >= 0) return tm;
-            }
-        }
         constexpr int WAVES_M = 1;
         return launch_moe_tm<F, 128, WAVES_M>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     }

@@ -61,11 +61,10 @@ static inline int mmq_splits(const MmqProblem& pb, int64_t tiles, int64_t slots,
 // dst[token][c] = part[0][token][c] + part[1][token][c] + ..., part[i] m_end x n floats; LK_* status.
 int lk_mmq_split_sum(const float* part, int splits, const MmqProblem& pb, hipStream_t s);
 
-// Q4_K against 33 or more token rows (mmq_q4k_f16.hip); `fixup`: the caller's tmp_fixup or null. Return the token-tile width launched,
-// 0 when the launch failed, -1 when the operands do not suit these kernels (16-byte alignment,
-// 32-bit record offsets) and the caller should take the int8 tiles.
-int lk_mmq_q4k_f16_dense(const MmqProblem& pb, hipStream_t s, void* fixup);
+// Q4_K, Q5_K or Q6_K (`wtype`) against 33 or more token rows (mmq_f16.hip); `fixup`: the caller's tmp_fixup or null. Return the token-tile width launched,
+// 0 when the launch failed, -1 when the operands do not suit these kernels (alignment, 32-bit offsets) and the caller should take the int8 tiles.
+int lk_mmq_f16_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup);
 // Q4_K against 129 or more token rows on the f16 tiles with four token tiles per wave (mmq_q4k_wide.hip); same returns.
 int lk_mmq_q4k_wide_dense(const MmqProblem& pb, hipStream_t s);
-int lk_mmq_q4k_f16_moe(const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
-                       int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);
+int lk_mmq_f16_moe(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
+                   int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);

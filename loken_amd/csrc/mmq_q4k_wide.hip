@@ -1,11 +1,11 @@
-// Q4_K weight rows against 129 or more Q8_1 token rows: the f16-operand tiles of mmq_q4k_f16.hip
+// Q4_K weight rows against 129 or more Q8_1 token rows: the f16-operand tiles of mmq_f16.hip
 // with four token tiles per wave and every byte delivered to LDS without passing through registers.
 //
 //   out[token, n] = sum over 256-value blocks of
 //        d[n] * sum_s d8_s[token] * D_s[n, token]  -  dmin[n] * sum_s m_s[n] * (d8_s * S_s)[token]
 //   D_s[n, token] = sum over the 32 values of sub-block s of (sc_s[n] * q[n, k]) * a[token, k]
 //
-// The arithmetic is that of mmq_q4k_f16.hip, operation for operation (sc * q and the int8 codes are
+// The arithmetic is that of mmq_f16.hip, operation for operation (sc * q and the int8 codes are
 // exact in f16, D_s is an exact integer in the f32 accumulator, one fma by the token's d8 per element
 // and sub-block in ascending s, the block's d and dmin applied once per 256 values with the minimum
 // term as a rank-8 update on the bf16 matrix unit), so both kernels return the same bits: the integer

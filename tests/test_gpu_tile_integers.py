@@ -143,6 +143,40 @@ def test_q4k_int8_tiles_above_64_rows_emit_the_exact_integers(knobs):
     check(lambda w, x: ops.mmq_forward(Q4K, w, x, n), Q4K, n, k, m, seed=91)
 
 
+# the f16-operand tiles (33 token rows or more of a matrix of 2048 rows or more): one and two token tiles in the last
+# workgroup tile, a ragged last row tile, one block and several
+@pytest.mark.parametrize("wtype", [Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("m,k", [(33, 256), (64, 512), (65, 768), (97, 512)])
+def test_f16_tiles_emit_the_exact_subblock_integers(wtype, m, k):
+    n = 2051
+    check(lambda w, x: ops.mmq_forward(wtype, w, x, n), wtype, n, k, m, seed=140 + m, subs=[0, 7] if wtype != Q6K else [0, 6, 15])
+
+
+@pytest.mark.parametrize("sub", [0, 3, 6])
+def test_f16_tiles_carry_every_q6k_scale_exactly(sub):
+    # sc * (code - 32) reaches 128 * 32, one bit more than an f16 holds: both 16-value scales of one 32-value
+    # sub-block over all of int8, among the rows the largest products; |result| <= 128 * 32 * 127 * 32 < 2^24
+    n, k, m = 2050, 256, 40
+    w = synth.weight(Q6K, n, k, seed=150, stream=sub).copy()
+    rng = np.random.default_rng(150 + sub)
+    scales = rng.integers(-128, 128, (n, 1, 2))
+    scales[:4, 0] = [[-128, -128], [127, -128], [-128, 127], [127, 127]]
+    w[:2, :, 0:192] = 0       # codes -32
+    w[2:4, :, 0:192] = 0xFF   # codes 31
+    w[..., 192:208] = 0
+    w[..., 192 + 2 * sub:194 + 2 * sub] = scales.astype(np.int8).view(np.uint8)
+    w[..., 208:210] = ONE
+    x = grid_activation(m, k, 150)
+    x[1] = 127
+    x[2] = -127
+    x[2, ::32] = 127
+    got = ops.mmq_forward(Q6K, dev(w), dev(x), n).cpu().numpy().astype(np.float64)
+    for t in range(m):
+        dots, _ = oracle.ob_subdots(Q6K, k, n, w, oracle.quantize_q8_1(x[t]))
+        want = (dots.reshape(n, 16)[:, 2 * sub:2 * sub + 2].astype(np.int64) * scales[:, 0]).sum(axis=1)
+        assert np.array_equal(got[t], want), f"token {t}"
+
+
 # up to 8 rows: registers only; up to 16: the staged form; up to 32: weights straight into the operand
 @pytest.mark.parametrize("m", [3, 8, 12, 16, 24, 32])
 def test_rows_on_matrix_unit_emit_the_exact_subblock_integers(m):
