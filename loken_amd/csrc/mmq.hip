@@ -930,9 +930,10 @@ __global__ __launch_bounds__(MMQ_WG, 2) void mmq_dense_split_kernel(MmqProblem p
     mmq_tile<F, TM, WAVES_M>(pb, n_tile * TN, pb.m_begin + m_tile * TM, lds, kb0, kb1);
 }
 
-// dst[token][c] = part[0][token][c] + part[1][token][c] + ... in that order; four columns a thread.
+// dst[token][c] = part[0][token][c] + part[1][token][c] + ... in that order; four columns a thread. n4: floats between
+// the rows of a partial product, n rounded up to four (what lies in the pad is read and not stored).
 __global__ __launch_bounds__(256) void mmq_split_sum_kernel(const float* __restrict__ part, int splits, int64_t part_stride,
-                                                            float* __restrict__ dst, int64_t count, int n, int64_t ldd) {
+                                                            float* __restrict__ dst, int64_t count, int n, int n4, int64_t ldd) {
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= count) return;
     float4 a = *(const float4*)(part + i);
@@ -943,8 +944,17 @@ __global__ __launch_bounds__(256) void mmq_split_sum_kernel(const float* __restr
         a.z += b.z;
         a.w += b.w;
     }
-    const int64_t row = i / n, col = i - row * n;
-    *(float4*)(dst + row * ldd + col) = a;
+    const int64_t row = i / n4;
+    const int col = (int)(i - row * n4);
+    float* out = dst + row * ldd + col;
+    if (col + 3 < n && ((uintptr_t)out & 15) == 0) {
+        *(float4*)out = a;
+    } else {
+        out[0] = a.x;   // (col < n: the pad is less than four columns)
+        if (col + 1 < n) out[1] = a.y;
+        if (col + 2 < n) out[2] = a.z;
+        if (col + 3 < n) out[3] = a.w;
+    }
 }
 
 // Expert-batched product: expert e's slab against the sorted rows [bounds[e], bounds[e+1]).
@@ -1114,9 +1124,9 @@ int lk_mmq_quantize_gated(const float* gu, void* y, int64_t rows, int width, hip
 }
 
 int lk_mmq_split_sum(const float* part, int splits, const MmqProblem& pb, hipStream_t s) {
-    const int64_t count = (int64_t)pb.m_end * pb.n;
+    const int64_t n4 = mmq_part_stride(pb), count = pb.m_end * n4;
     hipLaunchKernelGGL(mmq_split_sum_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, s, part, splits, count,
-                       pb.dst, count, pb.n, pb.ldd);
+                       pb.dst, count, pb.n, (int)n4, pb.ldd);
     return lk_launch_status();
 }
 

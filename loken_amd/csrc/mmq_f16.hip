@@ -560,7 +560,7 @@ __global__ __launch_bounds__(Wide::THREADS, 1) void f16_dense_split_kernel(MmqPr
     pb.y += kb0 * pb.rows_total * MMQ_REC_BYTES;
     pb.nb = kb1 - kb0;
     pb.dst = part + split * part_stride;
-    pb.ldd = pb.n;
+    pb.ldd = mmq_part_stride(pb);
     f16_tile<F>(pb, n_tile * Wide::TN, pb.m_begin + m_tile * Wide::TM, lds);
 }
 
@@ -597,11 +597,11 @@ static int f16_dense(const MmqProblem& pb, hipStream_t s, void* fixup) {
     if (!f16_suits<F>(pb)) return -1;
     const int n_tiles = (pb.n + C::TN - 1) / C::TN;
     const int m_tiles = (pb.m_end - pb.m_begin + C::TM - 1) / C::TM;
-    const int splits = mmq_splits(pb, (int64_t)n_tiles * m_tiles, lk_device().cus, fixup);   // one workgroup a CU
+    const int splits = mmq_splits(pb, (int64_t)n_tiles * m_tiles, lk_device().cus, fixup, true);   // one workgroup a CU
     if (splits > 1) {
         if (mmq_prepare_kernel(f16_dense_split_kernel<F>, LDS) != LK_OK) return 0;
         hipLaunchKernelGGL(f16_dense_split_kernel<F>, dim3((n_tiles + 7) / 8 * 8 * m_tiles * splits), dim3(C::THREADS), LDS,
-                           s, pb, n_tiles, m_tiles, splits, (float*)fixup, (int64_t)pb.m_end * pb.n);
+                           s, pb, n_tiles, m_tiles, splits, (float*)fixup, pb.m_end * mmq_part_stride(pb));
         return lk_mmq_split_sum((const float*)fixup, splits, pb, s) == LK_OK ? C::TM : 0;
     }
     if (mmq_prepare_kernel(f16_dense_kernel<F>, LDS) != LK_OK) return 0;

@@ -135,6 +135,22 @@ def test_cut_k_on_the_f16_tiles_of_q4k_follows_the_oracle(m, k, n):
     assert (cut - plain).abs().max().item() <= 2e-5 * plain.abs().max().item()
 
 
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("m,k,n", [(33, 1024, 2049), (100, 1280, 2307), (40, 3584, 2050)])
+def test_cut_k_on_the_f16_tiles_takes_ragged_matrices(name, m, k, n):
+    # rows of an odd length: partial products are padded to whole 16-byte pieces, the result is not
+    wtype = DT[name]
+    w = dev(synth.weight(wtype, n, k, seed=49, stream=5))
+    xh = synth.activation(m, k, seed=49)
+    x = dev(xh)
+    cut = ops.mmq_forward(wtype, w, x, n)
+    whole = ops.mmq_forward(wtype, w, x, n, fixup=False)
+    assert not torch.equal(cut, whole)   # K was cut
+    # f32 sums of the same exact products in another order
+    assert (cut - whole).abs().max().item() <= 2e-5 * whole.abs().max().item()
+    assert_close(cut.cpu().numpy(), oracle.ob_matmul(wtype, xh, w.cpu().numpy(), n))
+
+
 @pytest.mark.parametrize("name,m,k,n", [("q6_k", 48, 2048, 260), ("q4_k", 100, 1792, 2304)])
 def test_cut_k_recorded_into_a_graph_replays_to_the_eager_bits(name, m, k, n):
     # The cut-K call is two launches and nothing else (no fill, no allocation): recorded into a HIP graph
