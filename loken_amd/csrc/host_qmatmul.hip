@@ -1,6 +1,7 @@
 // Host mirror of loken's QKernelMatMul for the card path: see include/loken_host.hpp.
 
 #include "../../include/loken_host.hpp"
+#include "lk_common.h"
 #include "stream_scratch.h"
 
 #include <hip/hip_runtime.h>
@@ -17,23 +18,6 @@ constexpr size_t MMQ_RECORD = 144;                      // bytes per 128 padded 
 constexpr size_t FIXUP_BYTES = 256u * 128u * 128u * 4u;  // kernel_matmul/mmq.rs:42
 
 size_t pad_to(size_t v, size_t m) { return (v + m - 1) / m * m; }
-
-template <typename T>
-__global__ __launch_bounds__(256) void narrow_rows_kernel(const float* __restrict__ from, T* __restrict__ to, size_t count) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= count) return;
-    if constexpr (sizeof(T) == 2 && std::is_same<T, __half>::value) to[i] = __float2half_rn(from[i]);
-    else to[i] = __float2bfloat16(from[i]);
-}
-
-// out (f16 / bf16) = the f32 rows, rounded to nearest: the conversion the reference applies to the
-// f32 rows mmq_forward returns (src/tensor/quantized/kernel_matmul.rs:1086-1714, output dtype follows input).
-int narrow_rows(const float* from, void* to, int type, size_t count, hipStream_t stream) {
-    const unsigned grid = (unsigned)((count + 255) / 256);
-    if (type == LK_TYPE_F16) hipLaunchKernelGGL(narrow_rows_kernel<__half>, dim3(grid), dim3(256), 0, stream, from, (__half*)to, count);
-    else hipLaunchKernelGGL(narrow_rows_kernel<__hip_bfloat16>, dim3(grid), dim3(256), 0, stream, from, (__hip_bfloat16*)to, count);
-    return hipGetLastError() == hipSuccess ? LK_OK : LK_ERR_LAUNCH;
-}
 
 // The 32-value nibble formats and the two-bit K-quants: served by the plain mat-vec (four of them by the
 // tiled matmul as well, and Q2_K / Q3_K, from the row counts of nibble_tiles_pay below).
@@ -167,13 +151,6 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     };
     if ((rows <= mv_max && !to_rows_kernel) || decode_order || (plain && !to_nibble_tiles)) return matvec();
 
-    // The matrix-unit kernels write f32 rows. Rows that came in f16 / bf16 leave in that type, as the
-    // reference's do (the f32 rows its mmq_forward returns are narrowed by the caller,
-    // src/tensor/quantized/kernel_matmul.rs:1086-1714): the kernels write into a buffer of the
-    // stream's scratch and one more launch rounds them into `out`.
-    const bool half_rows = x_type != LK_TYPE_F32;
-    const size_t out_count = (size_t)rows * n_;
-
     // --- a handful of rows (or a matrix too small to fill the chip with tiles): matrix unit, weights
     //     straight from HBM
     if (rows_kernel_serves(dtype_, n_, k_, rows) && rows_kernel_fits) {
@@ -183,15 +160,11 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
             const auto scratch = lk_stream_scratch(stream);
             std::lock_guard<std::recursive_mutex> pair(scratch->mu);
             void* act = scratch->get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK, stream);
-            float* dst = half_rows ? (float*)scratch->get(LK_SCRATCH_LINEAR_F32, out_count * 4, stream) : (float*)out;
-            if (!act || !dst) return LK_ERR_NOMEM;
+            if (!act) return LK_ERR_NOMEM;
             if (int r = lk_quantize_q8_1(x, x_type, act, k_, k_, rows, stream)) return r;
-            // the launchers with a status (the exported void forms drop it): rows too long for their scale
-            // tables in LDS launch nothing, and the call goes on to the mat-vec or the tiled matmul below
-            rc = dtype_ == LK_TYPE_Q4_K   ? lk_dense_q4k_rows(blob_, act, dst, rows, n_, k_, stream)
-                 : dtype_ == LK_TYPE_Q5_K ? lk_dense_q5k_rows(blob_, act, dst, rows, n_, k_, stream)
-                                          : lk_dense_q6k_rows(blob_, act, dst, rows, n_, k_, stream);
-            if (rc == LK_OK && half_rows) rc = narrow_rows(dst, out, x_type, out_count, stream);
+            // (rows too long for the kernels' scale tables in LDS launch nothing, and the call goes on to the
+            // mat-vec or the tiled matmul below)
+            rc = lk_rows_linear(dtype_, blob_, act, out, x_type, rows, n_, k_, stream);
         }
         if (rc == LK_OK) {
             last_path_ = Path::RowsOnMatrixUnit;
@@ -209,32 +182,15 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     std::lock_guard<std::recursive_mutex> pair(scratch->mu);
     void* act = scratch->get(LK_SCRATCH_LINEAR, ws_bytes, stream);
     void* fixup = scratch->get(LK_SCRATCH_FIXUP, FIXUP_BYTES, stream);
-    void* dst = half_rows ? scratch->get(LK_SCRATCH_LINEAR_F32, out_count * 4, stream) : out;
-    if (!act || !fixup || !dst) return LK_ERR_NOMEM;
+    if (!act || !fixup) return LK_ERR_NOMEM;
     // the layouts of the reference's table (quantized/mmq.rs:274-285)
     auto quantizer = dtype_ == LK_TYPE_Q2_K ? launch_mmq_quantize_q8_1_D2S6
                      : dtype_ == LK_TYPE_Q6_K || dtype_ == LK_TYPE_Q8_0 || dtype_ == LK_TYPE_Q5_0 || dtype_ == LK_TYPE_Q3_K
                          ? launch_mmq_quantize_q8_1_D4
                          : launch_mmq_quantize_q8_1_DS4;
     quantizer(x, nullptr, act, x_type, k_, k_, 0, 0, (int64_t)k_padded, rows, 1, 1, stream);
-    auto launcher = dtype_ == LK_TYPE_Q4_K   ? launch_mmq_gguf_q4_k
-                    : dtype_ == LK_TYPE_Q5_K ? launch_mmq_gguf_q5_k
-                    : dtype_ == LK_TYPE_Q6_K ? launch_mmq_gguf_q6_k
-                    : dtype_ == LK_TYPE_Q4_0 ? launch_mmq_gguf_q4_0
-                    : dtype_ == LK_TYPE_Q4_1 ? launch_mmq_gguf_q4_1
-                    : dtype_ == LK_TYPE_Q5_0 ? launch_mmq_gguf_q5_0
-                    : dtype_ == LK_TYPE_Q5_1 ? launch_mmq_gguf_q5_1
-                    : dtype_ == LK_TYPE_Q3_K ? launch_mmq_gguf_q3_k
-                    : dtype_ == LK_TYPE_Q2_K ? launch_mmq_gguf_q2_k
-                                             : launch_mmq_gguf_q8_0;
-    int abi = 0, cus = 0, lds = 0, wave = 0;
-    (void)lk_device_info(&abi, &cus, &lds, &wave);
-    const int tile = launcher(fixup, blob_, act, dst, k_, n_, rows, k_ / block_len, n_, 0x1000950, cus, lds, wave,
-                              stream);
-    int narrowed = LK_OK;
-    if (tile != 0 && half_rows) narrowed = narrow_rows((const float*)dst, out, x_type, out_count, stream);
-    if (tile == 0) return LK_ERR_ARG;   // "no tile fits, nothing ran": the reference falls back to dequantized
-    if (narrowed != LK_OK) return narrowed;
+    if (lk_mmq_linear(dtype_, fixup, blob_, act, out, x_type, k_, n_, rows, k_ / block_len, stream) == 0)
+        return LK_ERR_ARG;   // "no tile fits, nothing ran": the reference falls back to dequantized
     last_path_ = Path::Tiled;
     return LK_OK;
 }

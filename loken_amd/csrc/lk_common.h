@@ -254,8 +254,24 @@ struct LkDevice {
 const LkDevice& lk_device();
 
 // Q4_K x up to any number of Q8_1 rows on the matrix unit (rows_mfma.hip); LK_* status.
+// A matrix-unit kernel's f32 result as element `at` of a destination of `type` (f32, or f16 / bf16 rounded to nearest: the
+// conversion the reference applies to the f32 rows mmq_forward returns, src/tensor/quantized/kernel_matmul.rs:1086-1714).
+// The type is uniform over the launch. A second launch over f32 rows took 4 to 5 us a call.
+static __device__ __forceinline__ void lk_store_as(float* dst, size_t at, float v, int type) {
+    if (type == LK_TYPE_F32) dst[at] = v;
+    else if (type == LK_TYPE_F16) ((__half*)dst)[at] = __float2half_rn(v);
+    else ((__hip_bfloat16*)dst)[at] = __float2bfloat16(v);
+}
+// The dense launches of the matrix unit with a destination of f32, f16 or bf16 elements, for the host linear: a few rows
+// (rows_mfma.hip; Q4_K, Q5_K, Q6_K) and tiles (mmq.hip). lk_rows_linear: LK_* status; lk_mmq_linear: the token-tile
+// width launched, 0 when nothing ran.
+int lk_rows_linear(int wtype, const void* w, const void* q8_1, void* out, int out_type, int rows, int n, int k, hipStream_t stream);
+int lk_mmq_linear(int wtype, void* fixup, const void* w, const void* y, void* out, int out_type, int k, int n, int rows, int64_t row_blocks,
+                  hipStream_t stream);
 int lk_q4k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y,
                      int ldd, hipStream_t stream);
+int lk_q6k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y,
+                     int ldd, hipStream_t stream, int out_type);
 
 // Q4_K x one or two activation rows with the rows' codes held in registers (mmvq_reg.hip): weight rows of
 // at most 16 super-blocks. Up to four matrices over the activation; `act_f32` non-zero: `act` holds f32

@@ -870,7 +870,7 @@ static __device__ __forceinline__ void mmq_tile(const MmqProblem& pb, int n0, in
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
                         const int gn = n0 + (wn * JT + jt) * 32 + (v >> 2) * 8 + lh * 4 + (v & 3);
-                        if (gn < pb.n) pb.dst[drow * pb.ldd + gn] = acc[it][jt][v];
+                        if (gn < pb.n) lk_store_as(pb.dst, drow * pb.ldd + gn, acc[it][jt][v], pb.out_type);
                     }
                 }
             } else {
@@ -880,7 +880,7 @@ static __device__ __forceinline__ void mmq_tile(const MmqProblem& pb, int n0, in
                     const int col = m0 + (wm * IT + it) * 32 + (v >> 2) * 8 + lh * 4 + (v & 3);
                     if (gn < pb.n && col < pb.m_end) {
                         const int64_t drow = pb.ids_dst ? pb.ids_dst[col] : col;
-                        pb.dst[drow * pb.ldd + gn] = acc[it][jt][v];
+                        lk_store_as(pb.dst, drow * pb.ldd + gn, acc[it][jt][v], pb.out_type);
                     }
                 }
             }
@@ -926,14 +926,15 @@ __global__ __launch_bounds__(MMQ_WG, 2) void mmq_dense_split_kernel(MmqProblem p
     if (n_tile >= n_tiles) return;
     const int kb0 = (int)(pb.nb * split / splits), kb1 = (int)(pb.nb * (split + 1) / splits);
     pb.dst = part + split * part_stride;
-    pb.ldd = pb.n;
+    pb.ldd = mmq_part_stride(pb);
+    pb.out_type = LK_TYPE_F32;
     mmq_tile<F, TM, WAVES_M>(pb, n_tile * TN, pb.m_begin + m_tile * TM, lds, kb0, kb1);
 }
 
 // dst[token][c] = part[0][token][c] + part[1][token][c] + ... in that order; four columns a thread. n4: floats between
 // the rows of a partial product, n rounded up to four (what lies in the pad is read and not stored).
 __global__ __launch_bounds__(256) void mmq_split_sum_kernel(const float* __restrict__ part, int splits, int64_t part_stride,
-                                                            float* __restrict__ dst, int64_t count, int n, int n4, int64_t ldd) {
+                                                            MmqProblem pb, int64_t count, int n4) {
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= count) return;
     float4 a = *(const float4*)(part + i);
@@ -946,14 +947,13 @@ __global__ __launch_bounds__(256) void mmq_split_sum_kernel(const float* __restr
     }
     const int64_t row = i / n4;
     const int col = (int)(i - row * n4);
-    float* out = dst + row * ldd + col;
-    if (col + 3 < n && ((uintptr_t)out & 15) == 0) {
-        *(float4*)out = a;
+    const int64_t at = row * pb.ldd + col;
+    if (col + 3 < pb.n) {
+        mmq_store4(pb, at, a, pb.out_type == LK_TYPE_F32 && ((uintptr_t)(pb.dst + at) & 15) == 0);
     } else {
-        out[0] = a.x;   // (col < n: the pad is less than four columns)
-        if (col + 1 < n) out[1] = a.y;
-        if (col + 2 < n) out[2] = a.z;
-        if (col + 3 < n) out[3] = a.w;
+        lk_store_as(pb.dst, at, a.x, pb.out_type);   // (col < n: the pad is less than four columns)
+        if (col + 1 < pb.n) lk_store_as(pb.dst, at + 1, a.y, pb.out_type);
+        if (col + 2 < pb.n) lk_store_as(pb.dst, at + 2, a.z, pb.out_type);
     }
 }
 
@@ -985,7 +985,7 @@ static int launch_dense_tm(const MmqProblem& pb, hipStream_t s, void* fixup = nu
     if (splits > 1) {
         auto kernel = mmq_dense_split_kernel<F, TM, WAVES_M>;
         if (mmq_prepare_kernel(kernel, lds_bytes) != LK_OK) return 0;
-        const int64_t count = (int64_t)pb.m_end * pb.n;
+        const int64_t count = pb.m_end * mmq_part_stride(pb);
         hipLaunchKernelGGL(kernel, dim3(n_groups * 8 * m_tiles * splits), dim3(MMQ_WG), lds_bytes, s, pb, n_tiles, m_tiles,
                            splits, (float*)fixup, count);
         return lk_mmq_split_sum((const float*)fixup, splits, pb, s) == LK_OK ? TM : 0;
@@ -999,13 +999,13 @@ static int launch_dense_tm(const MmqProblem& pb, hipStream_t s, void* fixup = nu
 
 template <class F>
 static int launch_dense(void* fixup, const void* x, const void* y, void* dst, int64_t ncols_x, int64_t nrows_x,
-                        int64_t ncols_y, int64_t stride_row_x, int64_t stride_col_dst, void* stream) {
+                        int64_t ncols_y, int64_t stride_row_x, int64_t stride_col_dst, void* stream, int out_type = LK_TYPE_F32) {
     if (!x || !y || !dst || ncols_x <= 0 || nrows_x <= 0 || ncols_y <= 0) return 0;
     if ((uintptr_t)x % F::ALIGN != 0) return 0;
     if (ncols_x % 256 != 0 || stride_row_x < ncols_x / 256 * F::BLOCKS_PER_STEP) return 0;
     if (stride_col_dst < nrows_x || nrows_x > INT32_MAX || ncols_y > INT32_MAX) return 0;
     MmqProblem pb{(const uint8_t*)x, (const uint8_t*)y, (float*)dst, nullptr, ncols_x / 256, stride_row_x,
-                  ncols_y, stride_col_dst, (int)nrows_x, 0, (int)ncols_y};
+                  ncols_y, stride_col_dst, (int)nrows_x, 0, (int)ncols_y, out_type};
     hipStream_t s = (hipStream_t)stream;
     if (ncols_y <= 32) return launch_dense_tm<F, 32, 1>(pb, s, fixup);
     // (Q2_K stays on 64-token tiles: with the rank-16 minimum its 128-token tile spills and runs 512 x
@@ -1126,8 +1126,28 @@ int lk_mmq_quantize_gated(const float* gu, void* y, int64_t rows, int width, hip
 int lk_mmq_split_sum(const float* part, int splits, const MmqProblem& pb, hipStream_t s) {
     const int64_t n4 = mmq_part_stride(pb), count = pb.m_end * n4;
     hipLaunchKernelGGL(mmq_split_sum_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, s, part, splits, count,
-                       pb.dst, count, pb.n, (int)n4, pb.ldd);
+                       pb, count, (int)n4);
     return lk_launch_status();
+}
+
+int lk_mmq_linear(int wtype, void* fixup, const void* w, const void* y, void* out, int out_type, int k, int n, int rows, int64_t row_blocks,
+                  hipStream_t s) {
+    auto run = [&](auto format) {
+        return launch_dense<decltype(format)>(fixup, w, y, out, k, n, rows, row_blocks, n, s, out_type);
+    };
+    switch (wtype) {
+        case LK_TYPE_Q4_K: return run(MmqQ4K{});
+        case LK_TYPE_Q5_K: return run(MmqQ5K{});
+        case LK_TYPE_Q6_K: return run(MmqQ6K{});
+        case LK_TYPE_Q8_0: return run(MmqQ80{});
+        case LK_TYPE_Q4_0: return run(MmqQ40{});
+        case LK_TYPE_Q4_1: return run(MmqQ41{});
+        case LK_TYPE_Q5_0: return run(MmqQ50{});
+        case LK_TYPE_Q5_1: return run(MmqQ51{});
+        case LK_TYPE_Q3_K: return run(MmqQ3K{});
+        case LK_TYPE_Q2_K: return run(MmqQ2K{});
+        default: return 0;
+    }
 }
 
 extern "C" void launch_mmq_quantize_q8_1_D4(const void* x, const int32_t* ids, void* vy, int type_x,

@@ -503,22 +503,21 @@ static __device__ __forceinline__ void f16_tile_of(const MmqProblem& pb, int n0,
         __syncthreads();
     }
 
-    const bool vec_ok = ((uintptr_t)pb.dst % 16 == 0) && (pb.ldd % 4 == 0);
+    const bool vec_ok = pb.out_type == LK_TYPE_F32 && (uintptr_t)pb.dst % 16 == 0 && pb.ldd % 4 == 0;
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         const int col = m0 + 32 * tt + j;
         if (col >= pb.m_end) continue;
-        const int64_t drow = pb.ids_dst ? pb.ids_dst[col] : col;
-        float* out = pb.dst + drow * pb.ldd;
+        const int64_t out = (pb.ids_dst ? pb.ids_dst[col] : col) * pb.ldd;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int gn0 = n0 + 32 * wave + 8 * g + 4 * h;
-            if (vec_ok && gn0 + 3 < pb.n) {
-                *(float4*)(out + gn0) = make_float4(acc[tt][4 * g], acc[tt][4 * g + 1], acc[tt][4 * g + 2], acc[tt][4 * g + 3]);
+            if (gn0 + 3 < pb.n) {
+                mmq_store4(pb, out + gn0, make_float4(acc[tt][4 * g], acc[tt][4 * g + 1], acc[tt][4 * g + 2], acc[tt][4 * g + 3]), vec_ok);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (gn0 + e < pb.n) out[gn0 + e] = acc[tt][4 * g + e];
+                    if (gn0 + e < pb.n) lk_store_as(pb.dst, out + gn0 + e, acc[tt][4 * g + e], pb.out_type);
             }
         }
     }
@@ -565,6 +564,7 @@ __global__ __launch_bounds__(Wide::THREADS, 1) void f16_dense_split_kernel(MmqPr
     pb.nb = kb1 - kb0;
     pb.dst = part + split * part_stride;
     pb.ldd = mmq_part_stride(pb);
+    pb.out_type = LK_TYPE_F32;
     f16_tile<F>(pb, n_tile * Wide::TN, pb.m_begin + m_tile * Wide::TM, lds);
 }
 

@@ -19,7 +19,30 @@ struct MmqProblem {
     int64_t rows_total;    // rows the workspace was quantized with (record stride)
     int64_t ldd;           // floats between destination rows
     int n, m_begin, m_end;
+    int out_type = LK_TYPE_F32;   // element type of `dst` (lk_store_as)
 };
+
+// Four results of one row from element `at` of the destination on; `vec`: f32 and 16-byte pieces allowed.
+static __device__ __forceinline__ void mmq_store4(const MmqProblem& pb, int64_t at, const float4& v, bool vec) {
+    if (vec) {
+        *(float4*)(pb.dst + at) = v;
+    } else if (pb.out_type == LK_TYPE_F32) {
+        pb.dst[at] = v.x; pb.dst[at + 1] = v.y; pb.dst[at + 2] = v.z; pb.dst[at + 3] = v.w;
+    } else {
+        uint16_t h[4];
+        const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            h[e] = pb.out_type == LK_TYPE_F16 ? __half_as_ushort(__float2half_rn(f[e])) : __bfloat16_as_ushort(__float2bfloat16(f[e]));
+        uint16_t* out = (uint16_t*)pb.dst + at;
+        if (((uintptr_t)out & 7) == 0) {
+            *(uint2*)out = make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = h[e];
+        }
+    }
+}
 
 // Raises a kernel's dynamic LDS limit once per process; LK_ERR_ARG when the device has less.
 template <typename K>
@@ -55,7 +78,8 @@ __host__ __device__ static inline int64_t mmq_part_stride(const MmqProblem& pb) 
 static inline int mmq_splits(const MmqProblem& pb, int64_t tiles, int64_t slots, const void* fixup, bool ragged = false) {
     const int forced = lk_tune_env("LK_TUNE_MMQ_SPLITS");   // measurement runs: -1 never, n > 0 that many where they fit
     if (!fixup || forced < 0 || pb.ids_dst || pb.m_begin != 0) return 1;
-    if (!ragged && (pb.n % 4 != 0 || pb.ldd % 4 != 0 || (uintptr_t)pb.dst % 16 != 0)) return 1;
+    const bool f32 = pb.out_type == LK_TYPE_F32;
+    if (!ragged && (pb.n % 4 != 0 || (f32 && (pb.ldd % 4 != 0 || (uintptr_t)pb.dst % 16 != 0)))) return 1;
     if ((uintptr_t)fixup % 16 != 0) return 1;
     const int64_t fit = MMQ_FIXUP_BYTES / ((int64_t)pb.m_end * mmq_part_stride(pb) * 4);
     int64_t want = forced > 0 ? forced : slots / tiles;

@@ -421,22 +421,21 @@ static __device__ __forceinline__ void wide_tile(const MmqProblem& pb, const uin
     w.fold_block<2>(last & 1);
     w.fold_block<3>(last & 1);
 
-    const bool vec_ok = ((uintptr_t)pb.dst % 16 == 0) && (pb.ldd % 4 == 0);
+    const bool vec_ok = pb.out_type == LK_TYPE_F32 && (uintptr_t)pb.dst % 16 == 0 && pb.ldd % 4 == 0;
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
         const int col = m0 + 32 * tt + j;
         if (col >= pb.m_end) continue;
-        const int64_t drow = pb.ids_dst ? pb.ids_dst[col] : col;
-        float* out = pb.dst + drow * pb.ldd;
+        const int64_t out = (pb.ids_dst ? pb.ids_dst[col] : col) * pb.ldd;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int gn0 = n0 + 32 * wave + 8 * g + 4 * h;
-            if (vec_ok && gn0 + 3 < pb.n) {
-                *(float4*)(out + gn0) = make_float4(w.acc[tt][4 * g], w.acc[tt][4 * g + 1], w.acc[tt][4 * g + 2], w.acc[tt][4 * g + 3]);
+            if (gn0 + 3 < pb.n) {
+                mmq_store4(pb, out + gn0, make_float4(w.acc[tt][4 * g], w.acc[tt][4 * g + 1], w.acc[tt][4 * g + 2], w.acc[tt][4 * g + 3]), vec_ok);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (gn0 + e < pb.n) out[gn0 + e] = w.acc[tt][4 * g + e];
+                    if (gn0 + e < pb.n) lk_store_as(pb.dst, out + gn0 + e, w.acc[tt][4 * g + e], pb.out_type);
             }
         }
     }

@@ -13,6 +13,7 @@ struct LkRows16 {
     int gelu;              // `dual`: 0 SiLU, 1 tanh-form GELU
     uint8_t* q81_dst;      // `dual` only, when given: the result as Q8_1 rows (blocks of 32 consecutive output
     int q81_stride;        // rows, q81_stride blocks between rows) instead of f32 in dst[0]; n a multiple of 32
+    int out_type;          // element type of `dst` (lk_store_as), dense launches
 };
 // True when the launch takes `size_m` activation rows of `nb` super-blocks (their codes fit in LDS).
 bool lk_rows16_serves(int size_m, int nb);
@@ -38,4 +39,4 @@ int lk_rows16_launch_experts(const LkRows16& a, const LkRows16Experts& m, int n_
 // multiple of 2048, rows whose codes do not fit in LDS, above 16 rows a matrix of more than 64 MB or of more 16-row tiles than CUs, above 32 rows
 // anything but whole rounds of resident workgroups).
 int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
-                  hipStream_t stream);
+                  hipStream_t stream, int out_type);

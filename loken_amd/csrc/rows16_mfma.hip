@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256 * TW, TW == 4 ? 1 : 2) void q4k_rows16_kernel(L
                 const TileRef tr = tile_ref<DUAL>(p, vt);
                 const int out = DUAL ? 0 : tr.mat;
                 const int tok = (T16 ? 4 * (l >> 4) : 4 * ((l >> 4) & 1)) + v, row = tr.row0 + (l & 15);
-                if (tok < p.m && row < pick3(p.n, out)) pick3(p.dst, out)[(size_t)tok * pick3(p.ldd, out) + row] = sum;
+                if (tok < p.m && row < pick3(p.n, out)) lk_store_as(pick3(p.dst, out), (size_t)tok * pick3(p.ldd, out) + row, sum, p.out_type);
             }
         }
         __syncthreads();   // the partial tiles may be overwritten

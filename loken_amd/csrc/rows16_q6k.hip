@@ -57,7 +57,8 @@ struct Args {
     int n;                // weight rows
     int m;                // activation rows
     int stride_y;         // Q8_1 blocks between activation rows
-    int ldd;              // floats between output rows
+    int ldd;              // elements between output rows
+    int out_type;         // element type of `dst` (lk_store_as)
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -100,7 +101,6 @@ __global__ __launch_bounds__(D == 4 ? 512 : 1024, 1) void q6k_rows16_kernel(Args
     // grid.y: the activation rows in sets of TOKS, a set per workgroup (the weights are read once per set)
     const int set = (int)blockIdx.y;
     const uint8_t* const act_rows = p.y + (size_t)set * TOKS * p.stride_y * Q81_BYTES;
-    float* const out_rows = p.dst + (size_t)set * TOKS * p.ldd;
     const int m_rows = min(TOKS, p.m - set * TOKS);
     constexpr int ZERO_BYTES = TOKS * 256;   // the zero lanes' run: the largest offset a step adds, and 16
     constexpr int BLK = TOKS * 32;       // LDS bytes of one Q8_1 block's codes, all rows
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(D == 4 ? 512 : 1024, 1) void q6k_rows16_kernel(Args
             }
             const int tile = ((int)blockIdx.x + pass * stride) * tw + ts;
             const int tok = T16 ? 4 * (l >> 4) + v : T8 ? 4 * ((l >> 4) & 1) + v : v, row = tile * TILE + (l & 15);
-            if (tile < n_tiles && tok < m_rows && row < p.n) out_rows[(size_t)tok * p.ldd + row] = sum;
+            if (tile < n_tiles && tok < m_rows && row < p.n) lk_store_as(p.dst, (size_t)(set * TOKS + tok) * p.ldd + row, sum, p.out_type);
         }
         __syncthreads();   // the buffers may be overwritten
     };
@@ -438,12 +438,12 @@ int launch(const Args& a, hipStream_t stream, int sets = 1) {
 }  // namespace
 
 int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
-                  hipStream_t stream) {
+                  hipStream_t stream, int out_type) {
     if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256) return -1;
     // rows of whole granules, on 16-byte boundaries; a tile's granules within one workgroup
     if (size_k % (256 * GRAN) != 0 || size_k / (256 * GRAN) > MAX_WAVES || (((uintptr_t)w) & 15) != 0) return -1;
     if (lk_tune_env("LK_TUNE_ROWS16_OFF") != 0) return -1;
-    const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd};
+    const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
     if (size_m > 8 && lk_tune_env("LK_TUNE_ROWS16_MAX8") != 0) return -1;
     if (size_m <= 4) return launch<4>(a, stream);
     const int n_tiles = (size_n + TILE - 1) / TILE;

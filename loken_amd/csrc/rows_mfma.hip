@@ -69,6 +69,7 @@ struct Args {
     // block; q81_stride blocks between activation rows) instead of f32 in `dst`; n a multiple of 32
     uint8_t* q81_dst = nullptr;
     int q81_stride = 0;
+    int out_type = LK_TYPE_F32;   // one matrix, dense launch: element type of `dst` (lk_store_as)
 };
 
 // Row tile `t` of a launch: which matrix it belongs to, and which of that matrix's tiles it is.
@@ -141,9 +142,9 @@ struct PassRows {
         const int r = src ? src[first + i] : first + i;
         return y + (size_t)r * stride_y * Q81_BYTES;
     }
-    __device__ __forceinline__ float* out_row(int i) const {
+    __device__ __forceinline__ size_t out_row(int i) const {   // its first element
         const int r = dst_map ? dst_map[first + i] : first + i;
-        return dst + (size_t)r * ldd;
+        return (size_t)r * ldd;
     }
 };
 
@@ -322,7 +323,7 @@ static __device__ __forceinline__ void q4k_rows_pass(const Args& p, const PassRo
                     sum = lk_gated(act, gate_keep[v], sum, 0);
                 }
                 const int tok = (v >> 2) * 8 + lh * 4 + (v & 3), row = (DUAL ? t >> 1 : t) * 32 + l32;
-                if (tok < m_count && row < p.n) rows.out_row(tok)[row] = sum;
+                if (tok < m_count && row < p.n) lk_store_as(rows.dst, rows.out_row(tok) + row, sum, p.out_type);
             }
         };
         while (tile < n_vt) {
@@ -390,7 +391,7 @@ static __device__ __forceinline__ void q4k_rows_pass(const Args& p, const PassRo
                 if (tok < m_count && row < mr.n) mr.dst[(size_t)(rows.first + tok) * mr.ldd + row] = sum;
             } else {
                 const int row = (DUAL ? t >> 1 : t) * 32 + l32;
-                if (tok < m_count && row < p.n) rows.out_row(tok)[row] = sum;
+                if (tok < m_count && row < p.n) lk_store_as(rows.dst, rows.out_row(tok) + row, sum, p.out_type);
             }
         }
         __syncthreads();   // the partial tiles may be overwritten (and, past the last tile, the tables)
@@ -620,7 +621,7 @@ __global__ __launch_bounds__(WG, G == 1 ? 2 : 1) void q4k_rows_staged_kernel(Arg
                 sum = lk_gated(act, gate_keep[r], sum, 0);
             }
             const int tok = (v >> 2) * 8 + lh * 4 + (v & 3), row = tile_of(ordinal) * 32 + l32;
-            if (tok < m_count && row < p.n) p.dst[(size_t)tok * p.ldd + row] = sum;
+            if (tok < m_count && row < p.n) lk_store_as(p.dst, (size_t)tok * p.ldd + row, sum, p.out_type);
         }
         __syncthreads();   // the partial tiles may be overwritten
     };
@@ -778,6 +779,7 @@ int launch_any(const Args& a, hipStream_t stream) {
             r.dst[0] = a.dst;
             r.n[0] = r.n[1] = a.n;
             r.ldd[0] = a.ldd;
+            r.out_type = a.out_type;
             r.count = DUAL ? 2 : 1;
             r.y = a.y; r.nb = a.nb; r.m = a.m; r.stride_y = a.stride_y; r.gelu = a.gelu;
             return lk_rows16_launch(r, DUAL, Q5, stream);
@@ -803,17 +805,24 @@ bool bad_rows_call(const void* w, const void* q8_1, const float* output, int siz
 
 // Returns LK_OK, or the reason nothing was launched.
 static int rows_plain(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y,
-                      int ldd, bool q5, hipStream_t stream) {
+                      int ldd, bool q5, hipStream_t stream, int out_type = LK_TYPE_F32) {
     if (size_m == 0 || size_n == 0) return LK_OK;
     if (bad_rows_call(w, q8_1, output, size_m, size_n, size_k)) return LK_ERR_ARG;
     if (stride_y < size_k / 32 || ldd < size_n) return LK_ERR_ARG;
     Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, nullptr, 0};
+    a.out_type = out_type;
     return q5 ? launch_any<false, true>(a, stream) : launch_any<false, false>(a, stream);
 }
 
 int lk_q4k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k,
                      int stride_y, int ldd, hipStream_t stream) {
     return rows_plain(w, q8_1, output, size_m, size_n, size_k, stride_y, ldd, false, stream);
+}
+
+int lk_rows_linear(int wtype, const void* w, const void* q8_1, void* out, int out_type, int rows, int n, int k, hipStream_t stream) {
+    if (wtype == LK_TYPE_Q6_K) return lk_q6k_rows_mfma(w, q8_1, (float*)out, rows, n, k, k / 32, n, stream, out_type);
+    if (wtype != LK_TYPE_Q4_K && wtype != LK_TYPE_Q5_K) return LK_ERR_TYPE;
+    return rows_plain(w, q8_1, (float*)out, rows, n, k, k / 32, n, wtype == LK_TYPE_Q5_K, stream, out_type);
 }
 
 extern "C" int lk_dense_q4k_rows(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k,

@@ -44,7 +44,8 @@ struct Args {
     int n;                // weight rows
     int m;                // activation rows in all
     int stride_y;         // Q8_1 blocks between activation rows
-    int ldd;              // floats between output rows
+    int ldd;              // elements between output rows
+    int out_type;         // element type of `dst` (lk_store_as)
 };
 
 struct WFrag {
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
                 sum += (reduce[(4 * NV + v) * 64 + lane] + reduce[(5 * NV + v) * 64 + lane]) +
                        (reduce[(6 * NV + v) * 64 + lane] + reduce[(7 * NV + v) * 64 + lane]);
             const int tok = (v >> 2) * 8 + lh * 4 + (v & 3), row = ((int)blockIdx.x + ordinal * (int)gridDim.x) * 32 + l32;
-            if (tok < m_count && row < p.n) p.dst[(size_t)(m0 + tok) * p.ldd + row] = sum;
+            if (tok < m_count && row < p.n) lk_store_as(p.dst, (size_t)(m0 + tok) * p.ldd + row, sum, p.out_type);
         }
         __syncthreads();   // the partial tiles may be overwritten
     };
@@ -383,17 +384,17 @@ int launch(const Args& a, hipStream_t stream) {
 // [size_m, ldd floats apart] f32. LK_ERR_ARG (nothing launched) when the rows are too long for the
 // scale table in LDS.
 int lk_q6k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y,
-                     int ldd, hipStream_t stream) {
+                     int ldd, hipStream_t stream, int out_type) {
     if (size_m == 0 || size_n == 0) return LK_OK;
     if (!w || !q8_1 || !output || size_m < 0 || size_n < 0 || size_k <= 0 || size_k % 256 != 0) return LK_ERR_ARG;
     if (stride_y < size_k / 32 || ldd < size_n) return LK_ERR_ARG;
     if ((((uintptr_t)w) & 1) != 0 || (((uintptr_t)q8_1) & 3) != 0) return LK_ERR_ARG;
-    Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd};
+    Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
     int rc = -1;
     if (size_m <= 64) {
         // 16-row tiles (rows16_q6k.hip): a quarter of the matrix-unit time per weight, and every CU a tile
         // (above 16 rows: sets of eight rows, for a small matrix that L2 holds; the launcher declines the rest)
-        rc = lk_rows16_q6k(w, q8_1, output, size_m, size_n, size_k, stride_y, ldd, stream);
+        rc = lk_rows16_q6k(w, q8_1, output, size_m, size_n, size_k, stride_y, ldd, stream, out_type);
         if (rc >= 0) return rc;
     }
     if (size_m <= 8) {
@@ -410,5 +411,5 @@ int lk_q6k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m,
 
 extern "C" int lk_dense_q6k_rows(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k,
                                  void* stream) {
-    return lk_q6k_rows_mfma(w, q8_1, output, size_m, size_n, size_k, size_k / 32, size_n, (hipStream_t)stream);
+    return lk_q6k_rows_mfma(w, q8_1, output, size_m, size_n, size_k, size_k / 32, size_n, (hipStream_t)stream, LK_TYPE_F32);
 }

@@ -16,7 +16,6 @@ enum LkScratchUse {
     LK_SCRATCH_BLOCK,      // expert block: what passes between its launches
     LK_SCRATCH_ROUTER,     // gate logits
     LK_SCRATCH_LINEAR,     // host linear: quantized rows
-    LK_SCRATCH_LINEAR_F32, // host linear: f32 results of half-precision calls
     LK_SCRATCH_FIXUP,      // tiled matmul: partial products of a cut K
     LK_SCRATCH_TOKENS,     // wide tiles: token operands
     LK_SCRATCH_USES

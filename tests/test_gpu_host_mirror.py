@@ -111,6 +111,24 @@ def test_half_inputs_stay_in_their_type_on_the_matvec_family():
         lin.close()
 
 
+# every kernel that stores in the rows' type itself, at ragged row counts: 16- and 32-row tiles, int8 tiles whole and
+# with K cut, f16 tiles, the wide ones
+@pytest.mark.parametrize("half", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name,rows,n,k", [
+    ("q4_k", 12, 2050, 1024), ("q4_k", 12, 70, 1280), ("q5_k", 24, 2051, 1024), ("q6_k", 12, 1030, 2048), ("q6_k", 40, 601, 2048),
+    ("q6_k", 24, 601, 1280), ("q6_k", 9, 601, 1280), ("q8_0", 70, 1027, 512), ("q8_0", 70, 1028, 1024), ("q8_0", 200, 12289, 256),
+    ("q4_k", 150, 4099, 1024), ("q6_k", 200, 4099, 512), ("q5_k", 130, 16387, 256), ("q4_k", 512, 9001, 256), ("q4_1", 33, 201, 512)])
+def test_half_rows_are_the_f32_rows_rounded_once(name, rows, n, k, half):
+    w = dev(synth.weight(DT[name], n, k, seed=84, stream=rows))
+    lin = Linear(DT[name], w, n, k)
+    x = dev(synth.activation(rows, k, seed=84)).to(half)
+    want = lin(x.float())
+    path = lin.path
+    got = lin(x)
+    assert lin.path == path and torch.equal(got, want.to(half))
+    lin.close()
+
+
 @pytest.mark.parametrize("half", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name,rows,n,expect", [
     ("q6_k", 50, 64, "rows-on-matrix-unit"), ("q4_k", 20, 200, "rows-on-matrix-unit"), ("q4_k", 4, 4000, "rows-on-matrix-unit"),
