@@ -958,21 +958,23 @@ __global__ __launch_bounds__(256) void mmq_split_sum_kernel(const float* __restr
 }
 
 // Expert-batched product: expert e's slab against the sorted rows [bounds[e], bounds[e+1]).
-// grid = (n tiles, column tiles sized for the longest run the host expects, stacks * experts);
+// grid: mmq_moe_grid, column tiles sized for the longest run the host expects;
 // a run longer than the grid covers is walked by the same workgroups in further passes.
 template <class F, int TM, int WAVES_M>
 __global__ __launch_bounds__(MMQ_WG, 2) void mmq_moe_kernel(MmqProblem pb, const uint8_t* w_second,
                                                          int64_t dst_second, const int32_t* __restrict__ bounds,
-                                                         int64_t stride_expert, int n_experts) {
+                                                         int64_t stride_expert, int n_experts, int group) {
     extern __shared__ __align__(16) uint8_t lds[];
-    const int stack = blockIdx.z / n_experts, e = blockIdx.z % n_experts;
+    const int stack = blockIdx.y / n_experts, e = blockIdx.y % n_experts;
+    const int n_tiles = (pb.n + TN - 1) / TN, n_tile = blockIdx.x % n_tiles;
     pb.m_begin = bounds[e];
     pb.m_end = bounds[e + 1];
     if (pb.m_end <= pb.m_begin) return;
     pb.w = (stack ? w_second : pb.w) + (int64_t)e * stride_expert;
     if (stack) pb.dst += dst_second;
-    for (int m0 = pb.m_begin + blockIdx.y * TM; m0 < pb.m_end; m0 += gridDim.y * TM)
-        mmq_tile<F, TM, WAVES_M>(pb, blockIdx.x * TN, m0, lds, 0, (int)pb.nb);
+    pb.out_type = LK_TYPE_F32;   // known here: the tile's stores need no choice
+    for (int m0 = pb.m_begin + (blockIdx.z * group + blockIdx.x / n_tiles) * TM; m0 < pb.m_end; m0 += gridDim.z * group * TM)
+        mmq_tile<F, TM, WAVES_M>(pb, n_tile * TN, m0, lds, 0, (int)pb.nb);
 }
 
 template <class F, int TM, int WAVES_M>
@@ -1060,11 +1062,9 @@ static int launch_moe_tm(const MmqProblem& pb, const uint8_t* w_second, int64_t 
     auto kernel = mmq_moe_kernel<F, TM, WAVES_M>;
     constexpr int lds_bytes = mmq_lds_bytes<F, TM>();
     if (mmq_prepare_kernel(kernel, lds_bytes) != LK_OK) return 0;
-    const int64_t col_tiles = (ncols_max + TM - 1) / TM;
-    const dim3 grid((pb.n + TN - 1) / TN, (unsigned)(col_tiles < 1 ? 1 : (col_tiles > 65535 ? 65535 : col_tiles)),
-                    (unsigned)((w_second ? 2 : 1) * n_experts));
-    hipLaunchKernelGGL(kernel, grid, dim3(MMQ_WG), lds_bytes, s, pb, w_second, dst_second, bounds,
-                       stride_expert, n_experts);
+    const MmqMoeGrid g = mmq_moe_grid(pb, TN, TM, w_second ? 2 : 1, n_experts, ncols_max);
+    hipLaunchKernelGGL(kernel, g.grid, dim3(MMQ_WG), lds_bytes, s, pb, w_second, dst_second, bounds,
+                       stride_expert, n_experts, g.group);
     return hipGetLastError() == hipSuccess ? TM : 0;
 }
 
@@ -1085,15 +1085,21 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
     // the narrowest tile at or above what was asked for, else one sized for the expected run
     const int64_t want = mmq_x > 0 ? mmq_x : (ncols_hint > 0 ? ncols_hint : ncols_max);
     if (want <= 32) return launch_moe_tm<F, 32, 1>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-    if (want <= 64) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-    // Runs of more than 64 rows: the f16 tiles for the formats that have them (128 experts of 2048 -> 768 -> 2048, top-8,
+    const bool f16 = F::F16_TYPE >= 0 && !lk_env_flag("LK_MMQ_I8");
+    // (a caller that names a tile of 64 gets the int8 tile of 64; under 32 of the 256-row f16 tiles, an eighth of the
+    // CUs, the int8 tiles' twice as many workgroups stay)
+    const bool f16_short = f16 && mmq_x <= 0 && (w2 ? 2 : 1) * n_experts * ((nrows_x + 255) / 256) >= 32;
+    if (want <= 64 && !f16_short) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
+    // Runs of more than 32 rows: the f16 tiles for the formats that have them, a half tile for the experts that own 32
+    // rows or fewer (all three stacks of one format, average run 20 / 32 / 40, against the int8 tiles: Q6_K 248 / 287 /
+    // 308 us against 342 / 359 / 368, Q5_K 202 / 235 / 251 against 263 / 280 / 288; at 8 experts of 1024 -> 1536 80
+    // -> 72; under 33 rows the int8 tile of 32 stays: average 8 / 14, Q6_K 198 / 208 against 231 / 238; 128 experts of 2048 -> 768 -> 2048, top-8,
     // Q4_K gate + up, 1111 / 1400 tokens, whole block, against the int8 tiles: Q4_K down 400 / 441 us against 512 / 542,
     // Q5_K 430 / 464 against 518 / 540, Q6_K 464 / 500 against 573 / 599).
-    if constexpr (F::F16_TYPE >= 0) {
-        if (!lk_env_flag("LK_MMQ_I8")) {
-            const int tm = lk_mmq_f16_moe(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-            if (tm >= 0) return tm;
-        }
+    if (f16) {
+        const int tm = lk_mmq_f16_moe(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
+        if (tm >= 0) return tm;
+        if (want <= 64) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     }
     // The 128-token int8 tile (the routing's bounds and destination map on top of the dense tile's registers) runs out
     // of registers for the formats with a minimum or two scales per sub-block and loses to the 64-token tile (2048

@@ -568,20 +568,22 @@ __global__ __launch_bounds__(Wide::THREADS, 1) void f16_dense_split_kernel(MmqPr
     f16_tile<F>(pb, n_tile * Wide::TN, pb.m_begin + m_tile * Wide::TM, lds);
 }
 
-// Expert-batched: expert e's slab against the sorted rows [bounds[e], bounds[e+1]).
+// Expert-batched: expert e's slab against the sorted rows [bounds[e], bounds[e+1]); grid: mmq_moe_grid.
 template <class F>
 __global__ __launch_bounds__(Wide::THREADS, 1) void f16_moe_kernel(MmqProblem pb, const uint8_t* w_second, int64_t dst_second,
                                                                   const int32_t* __restrict__ bounds, int64_t stride_expert,
-                                                                  int n_experts) {
+                                                                  int n_experts, int group) {
     extern __shared__ __align__(16) uint8_t lds[];
-    const int stack = blockIdx.z / n_experts, e = blockIdx.z % n_experts;
+    const int stack = blockIdx.y / n_experts, e = blockIdx.y % n_experts;
+    const int n_tiles = (pb.n + Wide::TN - 1) / Wide::TN, n_tile = blockIdx.x % n_tiles;
     pb.m_begin = bounds[e];
     pb.m_end = bounds[e + 1];
     if (pb.m_end <= pb.m_begin) return;
     pb.w = (stack ? w_second : pb.w) + (int64_t)e * stride_expert;
     if (stack) pb.dst += dst_second;
-    for (int m0 = pb.m_begin + blockIdx.y * Wide::TM; m0 < pb.m_end; m0 += gridDim.y * Wide::TM) {
-        f16_tile<F>(pb, blockIdx.x * Wide::TN, m0, lds);
+    pb.out_type = LK_TYPE_F32;   // known here: the tile's stores need no choice
+    for (int m0 = pb.m_begin + (blockIdx.z * group + blockIdx.x / n_tiles) * Wide::TM; m0 < pb.m_end; m0 += gridDim.z * group * Wide::TM) {
+        f16_tile<F>(pb, n_tile * Wide::TN, m0, lds);
         __syncthreads();   // the next tile's prologue rewrites the first stages
     }
 }
@@ -621,11 +623,9 @@ static int f16_moe(const MmqProblem& pb, const uint8_t* w_second, int64_t dst_se
     constexpr int LDS = f16_lds_bytes<F>();
     if (!f16_suits<F>(pb) || (uintptr_t)w_second % F::ALIGN != 0 || stride_expert % F::ALIGN != 0) return -1;
     if (mmq_prepare_kernel(f16_moe_kernel<F>, LDS) != LK_OK) return 0;
-    const int64_t col_tiles = (ncols_max + C::TM - 1) / C::TM;
-    const dim3 grid((pb.n + C::TN - 1) / C::TN, (unsigned)(col_tiles < 1 ? 1 : (col_tiles > 65535 ? 65535 : col_tiles)),
-                    (unsigned)((w_second ? 2 : 1) * n_experts));
-    hipLaunchKernelGGL(f16_moe_kernel<F>, grid, dim3(C::THREADS), LDS, s, pb, w_second, dst_second, bounds,
-                       stride_expert, n_experts);
+    const MmqMoeGrid g = mmq_moe_grid(pb, C::TN, C::TM, w_second ? 2 : 1, n_experts, ncols_max);
+    hipLaunchKernelGGL(f16_moe_kernel<F>, g.grid, dim3(C::THREADS), LDS, s, pb, w_second, dst_second, bounds,
+                       stride_expert, n_experts, g.group);
     return hipGetLastError() == hipSuccess ? C::TM : 0;
 }
 

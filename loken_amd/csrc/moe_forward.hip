@@ -67,12 +67,13 @@ extern "C" int lk_moe_longest_run(int tokens, int topk, int n_experts) {
 }
 
 // Whether a stack takes the matrix-unit rows launch (weights straight from HBM into the operand, a wave per
-// 16-row tile, a pass per 8, 16 or 48 rows) rather than the tiled one (weights expanded into LDS per 32 tokens).
-// Measured on MI355X at 128 experts of 2048 -> 768 -> 2048, top-8: 64 tokens 112 us against 173, 128 tokens 121
-// against 170, 256 tokens 159 against 183, 512 tokens 228 against 271, 1024 tokens 394 against 408, 1536 tokens
-// 537 against 463 (the expected longest run is 17 at 128 tokens, 29 at 256, 88 at 1024, 126 at 1536).
+// 16-row tile, a pass per 8, 16 or 48 rows) rather than the tiled ones (weights expanded into LDS per 32 or 64 tokens),
+// by the longest expected run. Measured on MI355X, whole Q4_K block, rows launches against tiles: 128 experts of
+// 2048 -> 768 -> 2048, top-8, at 17 / 34 / 42 / 50 / 60 / 84 rows 113 / 154 / 179 / 210 / 287 / 349 us against 172 / 177 /
+// 186 / 206 / 230 / 323; rows of more than eight super-blocks (32-row tiles, four waves a tile): 32 experts of
+// 3072 -> 512, top-4, at 24 / 32 / 39 / 46 rows 55 / 64 / 82 / 92 against 69 / 72 / 82 / 84.
 extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
-    return wtype == LK_TYPE_Q4_K && k % 256 == 0 && longest_run <= 90;
+    return wtype == LK_TYPE_Q4_K && k % 256 == 0 && longest_run <= (k <= 2048 ? 44 : 40);
 }
 
 extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
@@ -99,7 +100,16 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     }
 
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
-    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest), rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
+    const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
+    // Gate and up also leave the rows launch where
+    //   * down is tiled, past 36 rows: tiles for both keep the rows between them in the tiles' layout and the activation in
+    //     their quantizer (128 experts as above with a Q6_K down, 26 / 34 / 42 / 50 rows: 175 / 209 / 234 / 241 us against
+    //     187 / 203 / 218 / 231)
+    //   * their rows are long and their tiles fill the chip, past 20 rows (60 experts of 2560 -> 1280, 600 tiles, at 16 /
+    //     25 / 33 / 41 rows 150 / 208 / 217 / 272 us against 161 / 168 / 175 / 190)
+    const bool tiles_fill = 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus;
+    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest) && (rows_down || longest <= 36) &&
+                         (hidden <= 2048 || !tiles_fill || longest <= 20);
     const bool gated_later = !rows_gu && !rows_down && ffn % 32 == 0;   // the activation rides the second product's quantizer
     // the buffer's pieces
     size_t at = 0;

@@ -157,6 +157,31 @@ def test_result_does_not_depend_on_tile_width():
     assert (outs[3] - outs[0]).abs().max().item() <= 1e-4 * scale
 
 
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("tokens,heavy", [(330, 40), (330, 150), (620, 260)])
+def test_f16_tiles_of_uneven_runs_agree_with_the_int8_tiles(name, tokens, heavy, knobs):
+    # expert 0 owns `heavy` rows more than its share, expert 1 none: full tiles, tiles of 32 tokens or fewer, and column
+    # tiles past what the grid's first two dimensions cover. Same integers either way, so two f32 orders of the sums of
+    # at most 16 sub-blocks of 512 values apart: 2e-5 of the largest result, as for the dense tiles.
+    dt = getattr(lib, "TYPE_" + name.upper())
+    hidden, ffn, n_experts, topk = 512, 512, 16, 2
+    rng = np.random.default_rng(tokens)
+    ids = np.stack([2 + rng.permutation(n_experts - 2)[:topk] for _ in range(tokens)]).astype(np.int32)
+    ids[rng.permutation(tokens)[:heavy], 0] = 0
+    gate, up, down = (dev(synth.weight(dt, n_experts * 512, 512, seed=58, stream=i)) for i in range(3))
+    x = dev(synth.activation(tokens, hidden, seed=58))
+    weights = torch.full((tokens * topk,), 0.5, device="cuda")
+    plan = MmqRouting.from_choices(dev(ids), n_experts).with_path("tiled")
+    assert plan.longest_run_expected() > 32
+    h = plan.gate_up_silu(dt, x, gate, up, ffn)
+    out = plan.down_fold(dt, h, down, hidden, weights)
+    knobs.set("LK_MMQ_I8")
+    h8 = plan.gate_up_silu(dt, x, gate, up, ffn)
+    out8 = plan.down_fold(dt, h, down, hidden, weights)
+    assert (h - h8).abs().max().item() <= 4e-5 * h8.abs().max().item()   # a product of two such results
+    assert (out - out8).abs().max().item() <= 2e-5 * out8.abs().max().item()
+
+
 def test_glu_kernels():
     rng = np.random.default_rng(55)
     rows, width, n_experts = 13, 40, 3
