@@ -31,7 +31,8 @@
 // The min term is a rank-8 update per block on the bf16 matrix unit, with d8 * S split into
 // three bf16 pieces (24 bits, nothing lost).
 // Bound by vector issue (expansion of a wave's weights over two token tiles, 16 fmas per item) and, Q6_K, the matrix
-// instructions' own time: 2048 rows of 14336 -> 4096 reach 395 TFLOP/s in Q6_K (int8 tiles 341), 505 in Q5_K (437).
+// instructions' own time: 2048 rows of 14336 -> 4096 in Q6_K reach 417 TFLOP/s (int8 tiles 341): the vector unit is
+// busy 60 % of the cycles, the matrix unit the rest, and the two do not overlap (counters; the sum is 100 %).
 //
 // K order inside a sub-block: lane half h (lane / 32) of MFMA hf holds values 16 h + 8 hf + i,
 // i in the order 0 2 1 3 4 6 5 7 (what masking a dword's even and odd bytes yields); weights and
@@ -74,6 +75,16 @@ struct Wide {
 // sub-block s, times the scale, as TERMS f16 operands.
 struct Scale16 { h2 scale, offset; };
 
+// A code of a format with a plane of high bits is put together as a byte, four to an instruction, and the bytes 0 | 2 and
+// 1 | 3 leave for the mantissas of two 1024.0 in one v_perm_b32 each (with the high bits masked and shifted per pair of
+// halves instead, 312 of the 863 vector instructions of a Q6_K block went there, now 184 of 735: 4096 x 14336 at 2048 rows 610 -> 577 us, Q5_K
+// 11003 x 4096 at 77 rows 43.3 -> 40.5).
+static __device__ __forceinline__ uint32_t bits_from(uint32_t w, int up, uint32_t mask) {
+    return (up >= 0 ? w << (up & 31) : w >> (-up & 31)) & mask;
+}
+static __device__ __forceinline__ uint32_t even_codes(uint32_t c, uint32_t h1024) { return __builtin_amdgcn_perm(h1024, c, 0x07020500u); }
+static __device__ __forceinline__ uint32_t odd_codes(uint32_t c, uint32_t h1024) { return __builtin_amdgcn_perm(h1024, c, 0x07030501u); }
+
 template <bool Q5>
 struct F16Q45K {
     static constexpr int BYTES = Q5 ? Q5K_BYTES : Q4K_BYTES, ROW = BYTES, ALIGN = 16, TERMS = 1;
@@ -92,28 +103,34 @@ struct F16Q45K {
     static __device__ __forceinline__ uint32_t min_of(const Header& hd, int s) {
         return s < 4 ? (hd.w.z >> (8 * s)) & 63u : ((hd.w.w >> (8 * (s - 4) + 4)) & 0xFu) | (((hd.w.z >> (8 * (s - 4) + 6)) & 3u) << 4);
     }
-    // (1024 + q) * sc - 1024 * sc for the low nibbles; the high nibbles sit four bits up,
-    // (1024 + 16 q) * (sc / 16) - 64 * sc. Both exact in f16 (sc <= 63).
+    // (1024 + q) * sc - 1024 * sc; Q4_K's high nibbles stay four bits up, (1024 + 16 q) * (sc / 16) - 64 * sc.
+    // Both exact in f16 (sc <= 63).
     static __device__ __forceinline__ Scale16 scale(const Header& hd, int s) {
         const float sc = (float)scale_of(hd, s);
-        const _Float16 a = (_Float16)(sc * ((s & 1) ? 0.0625f : 1.0f)), b = (_Float16)(sc * ((s & 1) ? -64.0f : -1024.0f));
+        const bool up = !Q5 && (s & 1);
+        const _Float16 a = (_Float16)(sc * (up ? 0.0625f : 1.0f)), b = (_Float16)(sc * (up ? -64.0f : -1024.0f));
         return {{a, a}, {b, b}};
     }
-    static __device__ __forceinline__ void operand(const Codes& c, int s, int hf, const Scale16& sc, uint32_t h1024, v8h a[TERMS]) {
-        const uint4 q = c.q[(s >> 1) & 1];
-        const uint32_t u[4] = {q.x, q.y, q.z, q.w}, b[4] = {c.qh.x, c.qh.y, c.qh.z, c.qh.w};
+    static __device__ __forceinline__ void operand(const Codes& cd, int s, int hf, const Scale16& sc, uint32_t h1024, v8h a[TERMS]) {
+        const uint4 q = cd.q[(s >> 1) & 1];
+        const uint32_t u[4] = {q.x, q.y, q.z, q.w}, b[4] = {cd.qh.x, cd.qh.y, cd.qh.z, cd.qh.w};
         const bool high = (s & 1) != 0;
-        const uint32_t mask = high ? 0x00F000F0u : 0x000F000Fu, bit = high ? 0x01000100u : 0x00100010u;
         uint32_t ab[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {   // even bytes, then odd ones, of two dwords
-            uint32_t x = ((u[2 * hf + (e >> 1)] >> (8 * (e & 1))) & mask) | h1024;
-            if (Q5) {   // bit s of the byte goes on top of the nibble
-                const int to = (high ? 8 : 4) - s - 8 * (e & 1);
-                const uint32_t w = b[2 * hf + (e >> 1)];
-                x |= (to >= 0 ? w << (to & 31) : w >> (-to & 31)) & bit;
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t x = u[2 * hf + e];
+            uint32_t even, odd;
+            if constexpr (Q5) {   // bit s of the byte goes on top of the nibble
+                const uint32_t c = bits_from(b[2 * hf + e], 4 - s, 0x10101010u) | ((high ? x >> 4 : x) & 0x0F0F0F0Fu);
+                even = even_codes(c, h1024);
+                odd = odd_codes(c, h1024);
+            } else {
+                const uint32_t mask = high ? 0x00F000F0u : 0x000F000Fu;
+                even = (x & mask) | h1024;
+                odd = ((x >> 8) & mask) | h1024;
             }
-            ab[e] = h2_bits(__builtin_elementwise_fma(as_h2(x), sc.scale, sc.offset));
+            ab[2 * e] = h2_bits(__builtin_elementwise_fma(as_h2(even), sc.scale, sc.offset));
+            ab[2 * e + 1] = h2_bits(__builtin_elementwise_fma(as_h2(odd), sc.scale, sc.offset));
         }
         a[0] = __builtin_bit_cast(v8h, make_uint4(ab[0], ab[1], ab[2], ab[3]));
     }
@@ -138,17 +155,17 @@ struct F16Q6K {
         const _Float16 b = (_Float16)-1056.0f;
         return {{a, a}, {b, b}};
     }
-    static __device__ __forceinline__ void operand(const Codes& c, int s, int hf, const Scale16& sc, uint32_t h1024, v8h a[TERMS]) {
+    static __device__ __forceinline__ void operand(const Codes& cd, int s, int hf, const Scale16& sc, uint32_t h1024, v8h a[TERMS]) {
         const int g = s & 3;
-        const uint4 q = c.q[g & 1];
-        const uint32_t u[4] = {q.x, q.y, q.z, q.w}, b[4] = {c.qh.x, c.qh.y, c.qh.z, c.qh.w};
-        uint32_t t0[4], t1[4];
+        const uint4 q = cd.q[g & 1];
+        const uint32_t u[4] = {q.x, q.y, q.z, q.w}, b[4] = {cd.qh.x, cd.qh.y, cd.qh.z, cd.qh.w};
+        uint32_t t0[4], t1[4], c[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            c[e] = bits_from(b[2 * hf + e], 4 - 2 * g, 0x30303030u) | ((g >= 2 ? u[2 * hf + e] >> 4 : u[2 * hf + e]) & 0x0F0F0F0Fu);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int down = (g >= 2 ? 4 : 0) + 8 * (e & 1), to = 4 - 2 * g - 8 * (e & 1);
-            const uint32_t w = b[2 * hf + (e >> 1)];
-            uint32_t x = ((u[2 * hf + (e >> 1)] >> down) & 0x000F000Fu) | h1024;
-            x |= (to >= 0 ? w << (to & 31) : w >> (-to & 31)) & 0x00300030u;
+            const uint32_t x = e & 1 ? odd_codes(c[e >> 1], h1024) : even_codes(c[e >> 1], h1024);
             const h2 code = as_h2(x) + sc.offset;   // 1024 + code - 1056: -32 .. 31
             const h2 v = code * sc.scale;
             t0[e] = h2_bits(v);
