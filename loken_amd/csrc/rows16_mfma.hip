@@ -83,8 +83,9 @@ static __device__ __forceinline__ TileRef tile_ref(const LkRows16& p, int vt) {
 // (live in groups 2, 3). Lane l, register v is (weight row l % 16, activation row 4 (l / 16) + v) for
 // both, so every lane unpacks all eight scales of its row and its sums are complete across sub-blocks.
 // Q81 (gate + up, four tiles per workgroup: the 32 consecutive output rows of a Q8_1 block): the result
-// leaves as the Q8_1 rows the next linear reads, with the quantizer's steps.
-template <bool DUAL, bool Q5, int STEPS, int TW, bool T16, bool Q81 = false>
+// leaves as the Q8_1 rows the next linear reads, with the quantizer's steps. HALF: results in p.out_type (a choice made
+// at run time in the f32 launches cost the 42-launch step of a small model's decode at 16 rows 1 %).
+template <bool DUAL, bool Q5, int STEPS, int TW, bool T16, bool Q81 = false, bool HALF = false>
 __global__ __launch_bounds__(256 * TW, TW == 4 ? 1 : 2) void q4k_rows16_kernel(LkRows16 p, int n_vt) {
     static_assert(!Q81 || (DUAL && TW == 4), "Q8_1 output: the dual launch with four tiles per workgroup");
     constexpr int WG = 256 * TW;
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(256 * TW, TW == 4 ? 1 : 2) void q4k_rows16_kernel(L
                 const TileRef tr = tile_ref<DUAL>(p, vt);
                 const int out = DUAL ? 0 : tr.mat;
                 const int tok = (T16 ? 4 * (l >> 4) : 4 * ((l >> 4) & 1)) + v, row = tr.row0 + (l & 15);
-                if (tok < p.m && row < pick3(p.n, out)) lk_store_as(pick3(p.dst, out), (size_t)tok * pick3(p.ldd, out) + row, sum, p.out_type);
+                if (tok < p.m && row < pick3(p.n, out)) lk_store_as(pick3(p.dst, out), (size_t)tok * pick3(p.ldd, out) + row, sum, HALF ? p.out_type : LK_TYPE_F32);
             }
         }
         __syncthreads();   // the partial tiles may be overwritten
@@ -244,7 +245,7 @@ __global__ __launch_bounds__(256 * TW, TW == 4 ? 1 : 2) void q4k_rows16_kernel(L
 }
 
 // Workgroups per CU the kernel can keep resident with `lds_bytes` of LDS each; 0: does not fit.
-template <bool DUAL, bool Q5, int STEPS, int TW, bool T16, bool Q81 = false>
+template <bool DUAL, bool Q5, int STEPS, int TW, bool T16, bool Q81 = false, bool HALF = false>
 int resident_cap(int lds_bytes) {
     static std::mutex mu;
     static std::unordered_map<int, int> by_lds;
@@ -255,11 +256,11 @@ int resident_cap(int lds_bytes) {
     if (lds_bytes > lk_device().lds_bytes) {
         r = 0;
     } else if (lds_bytes > 48 * 1024 &&
-               hipFuncSetAttribute((const void*)q4k_rows16_kernel<DUAL, Q5, STEPS, TW, T16, Q81>, hipFuncAttributeMaxDynamicSharedMemorySize,
+               hipFuncSetAttribute((const void*)q4k_rows16_kernel<DUAL, Q5, STEPS, TW, T16, Q81, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    lds_bytes) != hipSuccess) {
         (void)hipGetLastError();
         r = 0;
-    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q4k_rows16_kernel<DUAL, Q5, STEPS, TW, T16, Q81>, 256 * TW,
+    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q4k_rows16_kernel<DUAL, Q5, STEPS, TW, T16, Q81, HALF>, 256 * TW,
                                                             (size_t)lds_bytes) != hipSuccess || r < 1) {
         (void)hipGetLastError();
         r = 1;
@@ -268,10 +269,12 @@ int resident_cap(int lds_bytes) {
     return r;
 }
 
-template <bool DUAL, bool Q5, int STEPS, int TW, bool T16, bool Q81 = false>
+template <bool DUAL, bool Q5, int STEPS, int TW, bool T16, bool Q81 = false, bool HALF = false>
 int launch_shape(const LkRows16& a, int n_vt, hipStream_t stream) {
+    if constexpr (!DUAL && !Q81 && !HALF)
+        if (a.out_type != LK_TYPE_F32) return launch_shape<DUAL, Q5, STEPS, TW, T16, false, true>(a, n_vt, stream);
     const int lds_bytes = lds_bytes_for(a.nb, TW, T16 ? 16 : 8, Q81);
-    const int per_cu = resident_cap<DUAL, Q5, STEPS, TW, T16, Q81>(lds_bytes);
+    const int per_cu = resident_cap<DUAL, Q5, STEPS, TW, T16, Q81, HALF>(lds_bytes);
     if (per_cu == 0) return -1;
     const int units = (n_vt + TW - 1) / TW;   // tile groups
     // Every workgroup stages the activation, so a workgroup should walk a few tile groups; all of
@@ -281,7 +284,7 @@ int launch_shape(const LkRows16& a, int n_vt, hipStream_t stream) {
     if (forced > 0) cap = forced;
     const int passes = (units + cap - 1) / cap;
     const int wgs = (units + passes - 1) / passes;
-    hipLaunchKernelGGL((q4k_rows16_kernel<DUAL, Q5, STEPS, TW, T16, Q81>), dim3(wgs), dim3(256 * TW), lds_bytes, stream, a, n_vt);
+    hipLaunchKernelGGL((q4k_rows16_kernel<DUAL, Q5, STEPS, TW, T16, Q81, HALF>), dim3(wgs), dim3(256 * TW), lds_bytes, stream, a, n_vt);
     return lk_launch_status();
 }
 

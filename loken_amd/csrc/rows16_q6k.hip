@@ -95,7 +95,7 @@ static __host__ __device__ constexpr int lds_bytes_for(int nb, int waves) {
 // for each of the four groups, so a lane's sums are complete across groups).
 // D: super-blocks of loads a wave keeps in flight (4 in workgroups of at most eight waves, else 2).
 // tw: row tiles of a workgroup; a tile's nb / 8 granules go to as many waves.
-template <int TOKS, int D>
+template <int TOKS, int D, bool HALF = false>
 __global__ __launch_bounds__(D == 4 ? 512 : 1024, 1) void q6k_rows16_kernel(Args p, int n_tiles, int tw) {
     constexpr bool T8 = TOKS == 8, T16 = TOKS == 16;
     // grid.y: the activation rows in sets of TOKS, a set per workgroup (the weights are read once per set)
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(D == 4 ? 512 : 1024, 1) void q6k_rows16_kernel(Args
             }
             const int tile = ((int)blockIdx.x + pass * stride) * tw + ts;
             const int tok = T16 ? 4 * (l >> 4) + v : T8 ? 4 * ((l >> 4) & 1) + v : v, row = tile * TILE + (l & 15);
-            if (tile < n_tiles && tok < m_rows && row < p.n) lk_store_as(p.dst, (size_t)(set * TOKS + tok) * p.ldd + row, sum, p.out_type);
+            if (tile < n_tiles && tok < m_rows && row < p.n) lk_store_as(p.dst, (size_t)(set * TOKS + tok) * p.ldd + row, sum, HALF ? p.out_type : LK_TYPE_F32);
         }
         __syncthreads();   // the buffers may be overwritten
     };
@@ -391,8 +391,10 @@ __global__ __launch_bounds__(D == 4 ? 512 : 1024, 1) void q6k_rows16_kernel(Args
     }
 }
 
-template <int TOKS, int D>
+template <int TOKS, int D, bool HALF = false>
 int launch_shape(const Args& a, int tw, int sets, hipStream_t stream) {
+    if constexpr (!HALF)
+        if (a.out_type != LK_TYPE_F32) return launch_shape<TOKS, D, true>(a, tw, sets, stream);
     static std::mutex mu;
     static std::unordered_map<int, int> by_lds;
     const int waves = tw * (a.nb / GRAN);
@@ -404,7 +406,7 @@ int launch_shape(const Args& a, int tw, int sets, hipStream_t stream) {
         if (it == by_lds.end()) {
             int ok = 1;
             if (lds_bytes > 48 * 1024 &&
-                hipFuncSetAttribute((const void*)q6k_rows16_kernel<TOKS, D>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                hipFuncSetAttribute((const void*)q6k_rows16_kernel<TOKS, D, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     lds_bytes) != hipSuccess) {
                 (void)hipGetLastError();
                 ok = 0;
@@ -420,7 +422,7 @@ int launch_shape(const Args& a, int tw, int sets, hipStream_t stream) {
     if (forced > 0) cap = forced;
     const int passes = (groups + cap - 1) / cap;
     const int wgs = (groups + passes - 1) / passes;
-    hipLaunchKernelGGL((q6k_rows16_kernel<TOKS, D>), dim3(wgs, sets), dim3(64 * waves), lds_bytes, stream, a, n_tiles, tw);
+    hipLaunchKernelGGL((q6k_rows16_kernel<TOKS, D, HALF>), dim3(wgs, sets), dim3(64 * waves), lds_bytes, stream, a, n_tiles, tw);
     return lk_launch_status();
 }
 

@@ -156,7 +156,7 @@ struct PassRows {
 // row tiles, all of a row's super-blocks in turn, and nothing crosses waves but the tables: rows of
 // at most eight super-blocks, where a four-way split leaves a wave one or two blocks per tile and
 // most of its time in the reduction's barriers.
-template <int G, bool DUAL, bool Q5, bool KSPLIT = true, bool MULTI = false>
+template <int G, bool DUAL, bool Q5, bool KSPLIT = true, bool MULTI = false, bool HALF = false>
 static __device__ __forceinline__ void q4k_rows_pass(const Args& p, const PassRows& rows, int m_count, uint8_t* lds) {
     static_assert(!MULTI || (!DUAL && KSPLIT), "several matrices: the dense launch with the super-blocks split over the waves");
     constexpr int TW = 8 * G;   // activation rows a table row holds
@@ -323,7 +323,7 @@ static __device__ __forceinline__ void q4k_rows_pass(const Args& p, const PassRo
                     sum = lk_gated(act, gate_keep[v], sum, 0);
                 }
                 const int tok = (v >> 2) * 8 + lh * 4 + (v & 3), row = (DUAL ? t >> 1 : t) * 32 + l32;
-                if (tok < m_count && row < p.n) lk_store_as(rows.dst, rows.out_row(tok) + row, sum, p.out_type);
+                if (tok < m_count && row < p.n) lk_store_as(rows.dst, rows.out_row(tok) + row, sum, HALF ? p.out_type : LK_TYPE_F32);
             }
         };
         while (tile < n_vt) {
@@ -391,7 +391,7 @@ static __device__ __forceinline__ void q4k_rows_pass(const Args& p, const PassRo
                 if (tok < m_count && row < mr.n) mr.dst[(size_t)(rows.first + tok) * mr.ldd + row] = sum;
             } else {
                 const int row = (DUAL ? t >> 1 : t) * 32 + l32;
-                if (tok < m_count && row < p.n) lk_store_as(rows.dst, rows.out_row(tok) + row, sum, p.out_type);
+                if (tok < m_count && row < p.n) lk_store_as(rows.dst, rows.out_row(tok) + row, sum, HALF ? p.out_type : LK_TYPE_F32);
             }
         }
         __syncthreads();   // the partial tiles may be overwritten (and, past the last tile, the tables)
@@ -424,12 +424,12 @@ static __device__ __forceinline__ void q4k_rows_pass(const Args& p, const PassRo
 }
 
 // Dense: grid y walks the activation in passes of 32 rows.
-template <int G, bool DUAL, bool Q5, bool MULTI = false>
+template <int G, bool DUAL, bool Q5, bool MULTI = false, bool HALF = false>
 __global__ __launch_bounds__(WG, 2) void q4k_rows_mfma_kernel(Args p) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int m0 = blockIdx.y * TOK;
     const PassRows rows{p.y, p.dst, nullptr, nullptr, m0, p.stride_y, p.ldd};
-    q4k_rows_pass<G, DUAL, Q5, true, MULTI>(p, rows, min(TOK, p.m - m0), lds);
+    q4k_rows_pass<G, DUAL, Q5, true, MULTI, HALF>(p, rows, min(TOK, p.m - m0), lds);
 }
 
 // Expert-batched: grid y is the expert; its sorted rows [bounds[e], bounds[e + 1]) go through in
@@ -472,7 +472,7 @@ static __host__ __device__ constexpr int lds_bytes_staged(int nb) {
     return nb * 8 * 8 * G * 32 + 2 * nb * 8 * 8 * G * 4 + WAVES * 4 * G * 64 * 4;
 }
 
-template <int G, bool DUAL, bool Q5>
+template <int G, bool DUAL, bool Q5, bool HALF = false>
 __global__ __launch_bounds__(WG, G == 1 ? 2 : 1) void q4k_rows_staged_kernel(Args p) {
     constexpr int TW = 8 * G, NV = 4 * G;
     extern __shared__ __align__(16) uint8_t lds[];
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(WG, G == 1 ? 2 : 1) void q4k_rows_staged_kernel(Arg
                 sum = lk_gated(act, gate_keep[r], sum, 0);
             }
             const int tok = (v >> 2) * 8 + lh * 4 + (v & 3), row = tile_of(ordinal) * 32 + l32;
-            if (tok < m_count && row < p.n) lk_store_as(p.dst, (size_t)tok * p.ldd + row, sum, p.out_type);
+            if (tok < m_count && row < p.n) lk_store_as(p.dst, (size_t)tok * p.ldd + row, sum, HALF ? p.out_type : LK_TYPE_F32);
         }
         __syncthreads();   // the partial tiles may be overwritten
     };
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(WG, G == 1 ? 2 : 1) void q4k_rows_staged_kernel(Arg
     }
 }
 
-template <int G, bool DUAL, bool Q5, bool MULTI = false>
+template <int G, bool DUAL, bool Q5, bool MULTI = false, bool HALF = false>
 int resident_cap(int lds_bytes) {
     static std::mutex mu;
     static std::unordered_map<int, int> by_lds;
@@ -654,11 +654,11 @@ int resident_cap(int lds_bytes) {
     if (lds_bytes > lk_device().lds_bytes) {
         r = 0;
     } else if (lds_bytes > 48 * 1024 &&
-               hipFuncSetAttribute((const void*)q4k_rows_mfma_kernel<G, DUAL, Q5, MULTI>, hipFuncAttributeMaxDynamicSharedMemorySize,
+               hipFuncSetAttribute((const void*)q4k_rows_mfma_kernel<G, DUAL, Q5, MULTI, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    lds_bytes) != hipSuccess) {
         (void)hipGetLastError();
         r = 0;
-    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q4k_rows_mfma_kernel<G, DUAL, Q5, MULTI>, WG,
+    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q4k_rows_mfma_kernel<G, DUAL, Q5, MULTI, HALF>, WG,
                                                             (size_t)lds_bytes) != hipSuccess || r < 1) {
         (void)hipGetLastError();
         r = 1;
@@ -667,22 +667,26 @@ int resident_cap(int lds_bytes) {
     return r;
 }
 
-template <int G, bool DUAL, bool Q5, bool MULTI = false>
+template <int G, bool DUAL, bool Q5, bool MULTI = false, bool HALF = false>
 int launch_rows(const Args& a, hipStream_t stream) {
+    if constexpr (!DUAL && !MULTI && !HALF)
+        if (a.out_type != LK_TYPE_F32) return launch_rows<G, DUAL, Q5, false, true>(a, stream);
     const int lds_bytes = (lds_floats_table<G>(a.nb) + WAVES * 4 * G * 64) * (int)sizeof(float);
-    const int per_cu = resident_cap<G, DUAL, Q5, MULTI>(lds_bytes);
+    const int per_cu = resident_cap<G, DUAL, Q5, MULTI, HALF>(lds_bytes);
     if (per_cu == 0) return LK_ERR_ARG;   // rows too long for the scale tables
     const int n_tiles = (a.n + 31) / 32 + (MULTI ? (a.n_b + 31) / 32 + (a.n_c + 31) / 32 : 0), groups = (a.m + TOK - 1) / TOK;
     if (groups > 65535) return LK_ERR_ARG;
     int cap = lk_device().cus * per_cu / groups;
     if (cap < 1) cap = 1;
-    hipLaunchKernelGGL((q4k_rows_mfma_kernel<G, DUAL, Q5, MULTI>), dim3(n_tiles < cap ? n_tiles : cap, groups), dim3(WG), lds_bytes, stream, a);
+    hipLaunchKernelGGL((q4k_rows_mfma_kernel<G, DUAL, Q5, MULTI, HALF>), dim3(n_tiles < cap ? n_tiles : cap, groups), dim3(WG), lds_bytes, stream, a);
     return lk_launch_status();
 }
 
 // The staged kernel for `a.m` <= 8 G rows, if its LDS image fits; -1 when it does not.
-template <int G, bool DUAL, bool Q5>
+template <int G, bool DUAL, bool Q5, bool HALF = false>
 int launch_staged(const Args& a, hipStream_t stream) {
+    if constexpr (!DUAL && !HALF)
+        if (a.out_type != LK_TYPE_F32) return launch_staged<G, DUAL, Q5, true>(a, stream);
     static std::mutex mu;
     static std::unordered_map<int, int> by_lds;
     const int lds_bytes = lds_bytes_staged<G>(a.nb);
@@ -694,11 +698,11 @@ int launch_staged(const Args& a, hipStream_t stream) {
         if (it == by_lds.end()) {
             int r = 0;
             if (lds_bytes > 48 * 1024 &&
-                hipFuncSetAttribute((const void*)q4k_rows_staged_kernel<G, DUAL, Q5>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                hipFuncSetAttribute((const void*)q4k_rows_staged_kernel<G, DUAL, Q5, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     lds_bytes) != hipSuccess) {
                 (void)hipGetLastError();
                 r = 0;
-            } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q4k_rows_staged_kernel<G, DUAL, Q5>, WG,
+            } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q4k_rows_staged_kernel<G, DUAL, Q5, HALF>, WG,
                                                                     (size_t)lds_bytes) != hipSuccess || r < 1) {
                 (void)hipGetLastError();
                 r = 1;
@@ -709,7 +713,7 @@ int launch_staged(const Args& a, hipStream_t stream) {
     }
     if (per_cu == 0) return -1;
     const int n_tiles = (a.n + 31) / 32, cap = lk_device().cus * per_cu;
-    hipLaunchKernelGGL((q4k_rows_staged_kernel<G, DUAL, Q5>), dim3(n_tiles < cap ? n_tiles : cap), dim3(WG), lds_bytes, stream, a);
+    hipLaunchKernelGGL((q4k_rows_staged_kernel<G, DUAL, Q5, HALF>), dim3(n_tiles < cap ? n_tiles : cap), dim3(WG), lds_bytes, stream, a);
     return lk_launch_status();
 }
 

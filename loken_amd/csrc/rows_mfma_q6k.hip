@@ -152,7 +152,7 @@ static __host__ __device__ constexpr int lds_bytes_for(int nb) {
 // them once and a wave keeps DEPTH steps of weight loads in flight. Otherwise the lane reads its
 // activation row's codes from memory with every step's weights (two steps in flight), 32 rows per
 // pass, grid y over the passes.
-template <int G, bool STAGED, int WAVES>
+template <int G, bool STAGED, int WAVES, bool HALF = false>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kernel(Args p) {
     constexpr int TW = 8 * G, NV = 4 * G, WG = 64 * WAVES;
     extern __shared__ __align__(16) uint8_t lds[];
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
                 sum += (reduce[(4 * NV + v) * 64 + lane] + reduce[(5 * NV + v) * 64 + lane]) +
                        (reduce[(6 * NV + v) * 64 + lane] + reduce[(7 * NV + v) * 64 + lane]);
             const int tok = (v >> 2) * 8 + lh * 4 + (v & 3), row = ((int)blockIdx.x + ordinal * (int)gridDim.x) * 32 + l32;
-            if (tok < m_count && row < p.n) lk_store_as(p.dst, (size_t)(m0 + tok) * p.ldd + row, sum, p.out_type);
+            if (tok < m_count && row < p.n) lk_store_as(p.dst, (size_t)(m0 + tok) * p.ldd + row, sum, HALF ? p.out_type : LK_TYPE_F32);
         }
         __syncthreads();   // the partial tiles may be overwritten
     };
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
     }
 }
 
-template <int G, bool STAGED, int WAVES>
+template <int G, bool STAGED, int WAVES, bool HALF = false>
 int resident_cap(int lds_bytes) {
     static std::mutex mu;
     static std::unordered_map<int, int> by_lds;
@@ -335,11 +335,11 @@ int resident_cap(int lds_bytes) {
     if (lds_bytes > lk_device().lds_bytes) {
         r = 0;
     } else if (lds_bytes > 48 * 1024 &&
-               hipFuncSetAttribute((const void*)q6k_rows_kernel<G, STAGED, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize,
+               hipFuncSetAttribute((const void*)q6k_rows_kernel<G, STAGED, WAVES, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    lds_bytes) != hipSuccess) {
         (void)hipGetLastError();
         r = 0;
-    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q6k_rows_kernel<G, STAGED, WAVES>, 64 * WAVES,
+    } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)q6k_rows_kernel<G, STAGED, WAVES, HALF>, 64 * WAVES,
                                                             (size_t)lds_bytes) != hipSuccess || r < 1) {
         (void)hipGetLastError();
         r = 1;
@@ -349,16 +349,18 @@ int resident_cap(int lds_bytes) {
 }
 
 // -1: the kernel's LDS image does not fit (the caller tries the next form).
-template <int G, bool STAGED, int WAVES>
+template <int G, bool STAGED, int WAVES, bool HALF = false>
 int launch_waves(const Args& a, hipStream_t stream) {
+    if constexpr (!HALF)
+        if (a.out_type != LK_TYPE_F32) return launch_waves<G, STAGED, WAVES, true>(a, stream);
     const int lds_bytes = lds_bytes_for<G, STAGED, WAVES>(a.nb);
-    const int per_cu = resident_cap<G, STAGED, WAVES>(lds_bytes);
+    const int per_cu = resident_cap<G, STAGED, WAVES, HALF>(lds_bytes);
     if (per_cu == 0) return -1;
     const int n_tiles = (a.n + 31) / 32, groups = STAGED ? 1 : (a.m + TOK - 1) / TOK;
     if (groups > 65535) return LK_ERR_ARG;
     int cap = lk_device().cus * per_cu / groups;
     if (cap < 1) cap = 1;
-    hipLaunchKernelGGL((q6k_rows_kernel<G, STAGED, WAVES>), dim3(n_tiles < cap ? n_tiles : cap, groups), dim3(64 * WAVES), lds_bytes, stream, a);
+    hipLaunchKernelGGL((q6k_rows_kernel<G, STAGED, WAVES, HALF>), dim3(n_tiles < cap ? n_tiles : cap, groups), dim3(64 * WAVES), lds_bytes, stream, a);
     return lk_launch_status();
 }
 
