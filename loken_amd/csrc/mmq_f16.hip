@@ -30,9 +30,11 @@
 // expanded to f16 once per step into LDS, two stages deep, one barrier per step.
 // The min term is a rank-8 update per block on the bf16 matrix unit, with d8 * S split into
 // three bf16 pieces (24 bits, nothing lost).
-// Bound by vector issue (expansion of a wave's weights over two token tiles, 16 fmas per item) and, Q6_K, the matrix
-// instructions' own time: 2048 rows of 14336 -> 4096 in Q6_K reach 417 TFLOP/s (int8 tiles 341): the vector unit is
-// busy 60 % of the cycles, the matrix unit the rest, and the two do not overlap (counters; the sum is 100 %).
+// Bound by the issue of vector and matrix instructions, which do not overlap here (counters on Q6_K, 2048 rows of
+// 14336 -> 4096: vector unit 62 % of the cycles, matrix unit 39 %; the wide kernel 65 and 36): 16 fmas per item, the
+// expansion of a wave's weights shared by two token tiles, and twice the matrix instructions for Q6_K. 417 TFLOP/s
+// there (int8 tiles 341). Half as many rows per workgroup, two workgroups a CU, took 622 us for 577 there and 453 for 429 on
+// 128 experts at 1111 tokens (the token side is expanded twice as often), though few large tiles gain (8 experts 77 -> 67).
 //
 // K order inside a sub-block: lane half h (lane / 32) of MFMA hf holds values 16 h + 8 hf + i,
 // i in the order 0 2 1 3 4 6 5 7 (what masking a dword's even and odd bytes yields); weights and
@@ -77,8 +79,8 @@ struct Scale16 { h2 scale, offset; };
 
 // A code of a format with a plane of high bits is put together as a byte, four to an instruction, and the bytes 0 | 2 and
 // 1 | 3 leave for the mantissas of two 1024.0 in one v_perm_b32 each (with the high bits masked and shifted per pair of
-// halves instead, 312 of the 863 vector instructions of a Q6_K block went there, now 184 of 735: 4096 x 14336 at 2048 rows 610 -> 577 us, Q5_K
-// 11003 x 4096 at 77 rows 43.3 -> 40.5).
+// halves instead, 312 of the 863 vector instructions of a Q6_K block went there, now 184 of 735: 4096 x 14336 at 2048
+// rows 610 -> 577 us, Q5_K 11003 x 4096 at 77 rows 43.3 -> 40.5).
 static __device__ __forceinline__ uint32_t bits_from(uint32_t w, int up, uint32_t mask) {
     return (up >= 0 ? w << (up & 31) : w >> (-up & 31)) & mask;
 }
