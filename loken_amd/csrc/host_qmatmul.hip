@@ -81,6 +81,12 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     // costs them more than the cut K costs the tiled launch: 4096 x 14336 at 9 / 16 rows 42 / 46 us against 37,
     // Q5_K 44 / 48 against 38; 4096 x 8192 31 / 33 against 30. Q6_K keeps its 16-row tiles: 38 against 40)
     if (dtype != LK_TYPE_Q6_K && rows > 8 && rows <= 16 && k >= 8192 && n >= 2048) return false;
+    // Above 16 rows of 8192 values or more: Q4_K / Q5_K 4096 x 14336 at 20 rows 37 / 39 us against 27 / 28, 1024 x 14336 at
+    // 17 / 32 35 / 39 against 20 / 22, 2048 x 8192 23 / 25 against 18 / 19; above 32 rows, where the tiles are 256 rows
+    // high and K is cut further, from 12288 values (2048 x 14336 at 40 / 109 rows 40 / 43 against 28 / 33; 3072 x 11008
+    // 33 / 46 against 40 / 51). Q6_K keeps its sets of eight rows up to 32 (2048 x 8192 17 against 21) and leaves above
+    // (2048 x 14336 at 40 / 109 rows 50 / 53 against 31 / 38, 4096 x 8192 34 / 58 against 29 / 37).
+    if (rows > 16 && n >= 1024 && (dtype == LK_TYPE_Q6_K ? rows > 32 && k >= 8192 : k >= (rows > 32 ? 12288 : 8192))) return false;
     return rows <= 16 || (long long)n * rows * (k > 4096 ? k : 4096) <= 450000ll * 4096 * few;
 }
 

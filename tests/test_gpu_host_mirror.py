@@ -310,3 +310,18 @@ def test_long_rows_at_nine_to_sixteen_activation_rows(name, rows, expect):
         assert close(got.cpu().numpy()[:, pick], oracle.ob_matmul(wtype, x, w[pick], len(pick)))
     finally:
         lin.close()
+
+
+@pytest.mark.parametrize("name,k,rows,expect", [("q4_k", 8192, 17, "tiled"), ("q5_k", 8192, 32, "tiled"), ("q4_k", 8192, 33, "rows-on-matrix-unit"),
+                                                 ("q4_k", 12288, 33, "tiled"), ("q6_k", 8192, 32, "rows-on-matrix-unit"),
+                                                 ("q6_k", 8192, 33, "tiled")])
+def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
+    wtype, n = DT[name], 1100
+    w = synth.weight(wtype, n, k, seed=97, stream=1)
+    x = synth.activation(rows, k, seed=97)
+    lin = Linear(wtype, dev(w), n, k)
+    got = lin(dev(x))
+    assert lin.path == expect
+    lin.close()
+    pick = np.sort(np.random.default_rng(97).choice(n, 100, replace=False))
+    assert close(got.cpu().numpy()[:, pick], oracle.ob_matmul(wtype, x, w[pick], len(pick)))
