@@ -436,7 +436,9 @@ void loken_moe_mmq_plan(const int32_t* experts, const int32_t* slots, int n, int
                         int32_t* bounds, int32_t* slots_out, int32_t* src_rows, void* stream);
 /* From the router's choices [n = tokens * topk]: groups the pairs by expert on the device.
  * `counts` is n_experts ints of scratch. Rows of one expert come in ascending pair order (the
- * reference leaves that order unspecified). cuda/moe/moe_mmq.cu:57-99,190-198. */
+ * reference leaves that order unspecified); pairs whose choice names no expert come last, from row
+ * bounds[n_experts] on, so that every entry of slots and src_rows is written.
+ * cuda/moe/moe_mmq.cu:57-99,190-198. */
 void loken_moe_mmq_route(const int32_t* choices, int n, int topk, int n_experts, int32_t* counts,
                          int32_t* bounds, int32_t* slots, int32_t* src_rows, void* stream);
 /* out[r, c] = silu(gu[r, c]) * gu[r, width + c] over gu [rows, 2 * width]. moe_mmq.cu:101-114. */

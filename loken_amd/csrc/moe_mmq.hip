@@ -41,6 +41,9 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(const int32_t* __restrict
 // what makes the counting, the scan over experts and the placing of rows independent of one another: as three
 // launches, the middle one a single thread walking the experts, they took 17 us at 2048 pairs and 30 at 8888
 // over 128 experts.
+// A choice that names no expert (negative, or n_experts and more: what a router leaves for a token whose logits
+// are not numbers) counts as expert n_experts, whose workgroup puts those pairs behind all others. So `slots` is
+// always a permutation and every entry of `src_rows` a token: quantizers walk all n of them.
 constexpr int ROUTE_THREADS = 1024;
 __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(const int32_t* __restrict__ choices, int n, int topk, int run,
                                                               int n_experts, int32_t* __restrict__ counts,
@@ -52,10 +55,11 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(const int32_t* __r
     // `run` is a multiple of four: whole 16-byte pieces but for the last thread with pairs
     const int first = threadIdx.x * run, end = min(first + run, n);
     const bool vec = ((uintptr_t)choices & 15) == 0;
+    auto expert_of = [&](int c) { return (int)min((unsigned)c, (unsigned)n_experts); };
     int own = 0, less = 0;
     auto look = [&](int c) {
-        own += c == e;
-        less += c >= 0 && c < e;
+        own += expert_of(c) == e;
+        less += expert_of(c) < e;
     };
     int i = first;
     if (vec)
@@ -81,14 +85,13 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(const int32_t* __r
         before += w < wave ? wave_own[w] : 0;
     }
     if (threadIdx.x == 0) {
-        bounds[e] = base;
-        if (counts) counts[e] = total;
-        if (e == n_experts - 1) bounds[n_experts] = base + total;
+        bounds[e] = base;   // bounds[n_experts]: the rows that have an expert
+        if (counts && e < n_experts) counts[e] = total;
     }
     int row = base + before + upto - own;
     if (own == 0) return;
     auto place = [&](int c, int at) {
-        if (c != e) return;
+        if (expert_of(c) != e) return;
         slots[row] = at;
         src_rows[row] = at / topk;
         ++row;
@@ -236,7 +239,7 @@ int lk_moe_route(const int32_t* choices, int n, int topk, int experts, int32_t* 
                  int32_t* src_rows, hipStream_t s) {
     if (experts <= 0 || n < 0 || topk <= 0) return LK_ERR_ARG;
     const int run = ((n + ROUTE_THREADS - 1) / ROUTE_THREADS + 3) / 4 * 4;
-    hipLaunchKernelGGL(route_kernel, dim3(experts), dim3(ROUTE_THREADS), 0, s, choices, n, topk, run, experts, counts, bounds, slots,
+    hipLaunchKernelGGL(route_kernel, dim3(experts + 1), dim3(ROUTE_THREADS), 0, s, choices, n, topk, run, experts, counts, bounds, slots,
                        src_rows);
     return lk_launch_status();
 }

@@ -621,6 +621,25 @@ def test_routing_is_a_stable_grouping(n, n_experts, topk):
     assert np.array_equal(plan.bounds.cpu().numpy(), np.searchsorted(np.sort(choices.reshape(-1)), np.arange(n_experts + 1)))
 
 
+@pytest.mark.parametrize("n,n_experts,topk", [(1, 3, 1), (65, 5, 5), (1025, 130, 5), (4100, 64, 4)])
+@pytest.mark.parametrize("share", [0.2, 1.0])
+def test_pairs_without_an_expert_come_behind_all_others(n, n_experts, topk, share):
+    """Every entry of slots and src_rows is written whatever the choices hold: the quantizer gathers all of them."""
+    choices = synth.rand_ints(24, n, n, n_experts).astype(np.int32)
+    out = synth.rand_ints(25, n, n, 1000) < 1000 * share
+    choices[out] = np.array([-1, n_experts, 0x7FFFFFFF, -2 ** 31], np.int32)[synth.rand_ints(26, n, n, 4)[out]]
+    expert = np.where((choices < 0) | (choices >= n_experts), n_experts, choices)
+    order = np.argsort(expert, kind="stable")
+    cd = dev(choices)
+    counts, bounds, slots, src = (torch.full((m,), -9, dtype=torch.int32, device="cuda") for m in (n_experts, n_experts + 1, n, n))
+    lib.load().loken_moe_mmq_route(cd.data_ptr(), n, topk, n_experts, counts.data_ptr(), bounds.data_ptr(), slots.data_ptr(),
+                                   src.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert np.array_equal(slots.cpu().numpy(), order)
+    assert np.array_equal(src.cpu().numpy(), order // topk)
+    assert np.array_equal(bounds.cpu().numpy(), np.searchsorted(np.sort(expert), np.arange(n_experts + 1)))
+    assert np.array_equal(counts.cpu().numpy(), np.bincount(expert, minlength=n_experts + 1)[:n_experts])
+
+
 # ---------------------------------------------------------------- router
 @pytest.mark.parametrize("tokens,experts,topk,renorm", [(1, 128, 8, True), (16, 128, 8, True), (256, 128, 8, False),
                                                         (7, 60, 4, True), (5, 512, 64, True), (3, 8, 8, False)])
