@@ -449,10 +449,16 @@ void loken_moe_mmq_swiglu_oai(const float* gu, float* out, int64_t rows, int wid
                               const int32_t* bounds, int n_experts, const float* gate_bias,
                               const float* up_bias, float alpha, float limit, void* stream);
 /* out[t, c] += sum over k ascending of weights[p] * (pairs[p, c] + down_bias[choices[p], c]),
- * p = t * topk + k; bias and choices nullable together. moe_mmq.cu:155-176. */
+ * p = t * topk + k; bias and choices nullable together. A pair whose choice is negative or 0x7FFFFFFF
+ * (what loken_topk_softmax leaves where nothing can be chosen) adds nothing. moe_mmq.cu:155-176. */
 void loken_moe_mmq_fold(const float* pairs, const float* weights, const int32_t* choices,
                         const float* down_bias, float* out, int64_t tokens, int topk, int cols,
                         void* stream);
+/* The fold without a bias, over the pairs whose choice is in [0, n_experts): the expert-batched products
+ * write no row for the others. `choices` null: every pair. accumulate == 0: `out` is written, not added
+ * to. No counterpart in the reference. */
+int lk_moe_fold(const float* pairs, const float* weights, const int32_t* choices, int n_experts, float* out,
+                int64_t tokens, int topk, int cols, int accumulate, void* stream);
 
 /* ---------------------------------------------------------------------------------------
  * MoE decode: one mat-vec per routed pair (few rows per expert). Names, argument lists and row
@@ -586,7 +592,7 @@ int loken_moe_gemm_gguf_down_reduce_static(const float* inputs, const void* weig
 /* A mixture layer's expert block in one call: out[t] = sum over the token's choices j of topk_weights[t, j] *
  * down_e (silu(gate_e . x[t]) * (up_e . x[t])), e = choices[t, j]; f32 rows x [tokens, hidden] and out [tokens,
  * hidden], stacks gate / up [experts, ffn, hidden] of wtype_gu and down [experts, hidden, ffn] of wtype_down, choices
- * int32 and weights f32 [tokens, topk]. The launches are those of the entry points above, chosen by size as the layer
+ * int32 and weights f32 [tokens, topk]. A choice outside [0, n_experts) adds nothing, whatever its weight. The launches are those of the entry points above, chosen by size as the layer
  * code of the reference chooses (src/inference/generic_transformer/moe_weights.rs:2118-2152). LK_ERR_TYPE: a format
  * the path does not take; LK_ERR_NOMEM: the scratch would have to grow while the stream records a graph. */
 int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,

@@ -15,8 +15,6 @@ int lk_moe_pairs_down(int wire, const float* h, const void* down, const int32_t*
 // Groups the router's choices by expert (moe_mmq.hip): counts [experts] (nullable), bounds [experts + 1], slots and src_rows [n].
 int lk_moe_route(const int32_t* choices, int n, int topk, int experts, int32_t* counts, int32_t* bounds, int32_t* slots,
                  int32_t* src_rows, hipStream_t s);
-// out[t] = sum over the token's slots of weights[slot] * pairs[slot]
-int lk_moe_fold_write(const float* pairs, const float* weights, float* out, int64_t tokens, int topk, int cols, hipStream_t s);
 // silu(gu[:, :width]) * gu[:, width:] of every row into the tile kernels' workspace (mmq.hip): the activation
 // and the quantizer in one pass, same bytes as the two one after the other.
 int lk_mmq_quantize_gated(const float* gu, void* y, int64_t rows, int width, hipStream_t s);

@@ -160,5 +160,5 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
         if (!gated_later) quantize(h, nullptr, y2, ffn);
         if (int rc = grouped(*fd, down, nullptr, 0, y2, pairs, slots, hidden, ffn, hidden)) return rc;
     }
-    return lk_moe_fold_write(pairs, topk_weights, out, tokens, topk, hidden, s);
+    return lk_moe_fold(pairs, topk_weights, choices, n_experts, out, tokens, topk, hidden, 0, stream);
 }

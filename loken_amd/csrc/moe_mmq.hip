@@ -170,12 +170,13 @@ __global__ __launch_bounds__(THREADS) void swiglu_oai_kernel(const float* __rest
 }
 
 // out[t, c] += (`write`: =) sum over k ascending of weights[p] * (pairs[p, c] + down_bias[choices[p], c]),
-// p = t * topk + k. A workgroup column of the grid is one token; a thread owns four columns and
-// keeps four routed rows' loads in flight, adding them in k order.
+// p = t * topk + k, over the pairs whose choice names an expert (all of them without `choices`): the rows of
+// the others were written by nobody. A workgroup column of the grid is one token; a thread owns four columns
+// and keeps four routed rows' loads in flight, adding them in k order.
 constexpr int FOLD_AHEAD = 4;
 template <bool VEC>
 __global__ __launch_bounds__(THREADS) void fold_kernel(const float* __restrict__ pairs, const float* __restrict__ weights,
-                                                       const int32_t* __restrict__ choices,
+                                                       const int32_t* __restrict__ choices, int n_experts,
                                                        const float* __restrict__ down_bias, float* __restrict__ out,
                                                        int topk, int cols, int write) {
     constexpr int W = VEC ? 4 : 1;
@@ -204,16 +205,20 @@ __global__ __launch_bounds__(THREADS) void fold_kernel(const float* __restrict__
     };
     for (int k0 = 0; k0 < topk; k0 += FOLD_AHEAD) {
         float v[FOLD_AHEAD][W], b[FOLD_AHEAD][W], w[FOLD_AHEAD];
+        bool routed[FOLD_AHEAD];
 #pragma unroll
         for (int j = 0; j < FOLD_AHEAD; ++j) {
             const int64_t p = p0 + min(k0 + j, topk - 1);   // past the end: a repeat, dropped below
             row_at(pairs, p, v[j]);
             w[j] = weights[p];
-            if (down_bias != nullptr) row_at(down_bias, choices[p], b[j]);
+            const int e = choices != nullptr ? choices[p] : 0;
+            routed[j] = choices == nullptr || (unsigned)e < (unsigned)n_experts;
+            if (down_bias != nullptr && routed[j]) row_at(down_bias, e, b[j]);
         }
 #pragma unroll
         for (int j = 0; j < FOLD_AHEAD; ++j) {
             if (k0 + j >= topk) break;
+            if (!routed[j]) continue;
 #pragma unroll
             for (int e = 0; e < W; ++e) acc[e] += w[j] * (down_bias != nullptr ? v[j][e] + b[j][e] : v[j][e]);
         }
@@ -264,8 +269,8 @@ extern "C" void loken_moe_mmq_swiglu_oai(const float* gu, float* out, int64_t ro
     (void)hipGetLastError();
 }
 
-static int launch_fold(const float* pairs, const float* weights, const int32_t* choices, const float* down_bias, float* out,
-                       int64_t tokens, int topk, int cols, bool write, hipStream_t s) {
+static int launch_fold(const float* pairs, const float* weights, const int32_t* choices, int n_experts, const float* down_bias,
+                       float* out, int64_t tokens, int topk, int cols, bool write, hipStream_t s) {
     if (tokens <= 0 || cols <= 0 || topk <= 0 || tokens > 65535 * (int64_t)65535) return LK_ERR_ARG;
     const bool vec = cols % 4 == 0 && (((uintptr_t)pairs | (uintptr_t)out | (uintptr_t)down_bias) & 15) == 0;
     // tokens ride the grid's second axis, 65535 at a time
@@ -277,20 +282,24 @@ static int launch_fold(const float* pairs, const float* weights, const int32_t* 
         float* o = out + t0 * cols;
         if (vec)
             hipLaunchKernelGGL(fold_kernel<true>, dim3((unsigned)((cols / 4 + THREADS - 1) / THREADS), ty), dim3(THREADS), 0, s, p, w,
-                               ch, down_bias, o, topk, cols, write ? 1 : 0);
+                               ch, n_experts, down_bias, o, topk, cols, write ? 1 : 0);
         else
             hipLaunchKernelGGL(fold_kernel<false>, dim3((unsigned)((cols + THREADS - 1) / THREADS), ty), dim3(THREADS), 0, s, p, w,
-                               ch, down_bias, o, topk, cols, write ? 1 : 0);
+                               ch, n_experts, down_bias, o, topk, cols, write ? 1 : 0);
     }
     return lk_launch_status();
 }
 
-int lk_moe_fold_write(const float* pairs, const float* weights, float* out, int64_t tokens, int topk, int cols, hipStream_t s) {
-    return launch_fold(pairs, weights, nullptr, nullptr, out, tokens, topk, cols, true, s);
+extern "C" int lk_moe_fold(const float* pairs, const float* weights, const int32_t* choices, int n_experts, float* out, int64_t tokens,
+                           int topk, int cols, int accumulate, void* stream) {
+    if (tokens == 0) return LK_OK;
+    if (!pairs || !weights || !out || (choices && n_experts <= 0)) return LK_ERR_ARG;
+    return launch_fold(pairs, weights, choices, n_experts, nullptr, out, tokens, topk, cols, !accumulate, (hipStream_t)stream);
 }
 
 extern "C" void loken_moe_mmq_fold(const float* pairs, const float* weights, const int32_t* choices,
                                    const float* down_bias, float* out, int64_t tokens, int topk, int cols,
                                    void* stream) {
-    (void)launch_fold(pairs, weights, choices, down_bias, out, tokens, topk, cols, false, (hipStream_t)stream);
+    // the count of experts is not among the arguments: a negative choice names none, nor does 0x7FFFFFFF (loken_topk_softmax)
+    (void)launch_fold(pairs, weights, choices, 0x7FFFFFFF, down_bias, out, tokens, topk, cols, false, (hipStream_t)stream);
 }

@@ -159,6 +159,7 @@ SIGNATURES.update({
     "loken_moe_gemm_gguf_prefill": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "loken_rms_quantize_q8_1": (None, [_vp, _vp, _vp, _i, _f, _vp]),
     "loken_rms_quantize_q8_1_bf16": (None, [_vp, _vp, _vp, _i, _f, _vp]),
+    "lk_moe_fold": (_i, [_vp, _vp, _vp, _i, _vp, _i64, _i, _i, _i, _vp]),
     "loken_moe_mmq_fold": (None, [_vp, _vp, _vp, _vp, _vp, _i64, _i, _i, _vp]),
 })
 

@@ -54,6 +54,8 @@ class MmqRouting:
         _lib.load().loken_moe_mmq_plan(experts.data_ptr(), slots.data_ptr(), rows, topk, n_experts,
                                        plan.bounds.data_ptr(), plan.slots.data_ptr(),
                                        plan.src_rows.data_ptr(), _stream())
+        plan.choices = torch.empty_like(plan.slots)
+        plan.choices[slots.long()] = experts.to(torch.int32)
         return plan
 
     @classmethod
@@ -118,8 +120,9 @@ class MmqRouting:
             expert_bytes, n, k, self.longest_run_expected(), _stream()))
 
     def gate_up_silu(self, wtype: int, xs: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, width: int) -> torch.Tensor:
-        """``silu(gate . x) * (up . x)`` for every routed row, in sorted order: ``[rows, width]``
-        (mmq_experts.rs:300-435). ``gate`` / ``up`` are stacks of ``[experts, width, k]`` blocks."""
+        """``silu(gate . x) * (up . x)`` for every routed row, in sorted order: ``[rows, width]``, the rows from
+        ``bounds[experts]`` on (pairs without an expert) unspecified (mmq_experts.rs:300-435). ``gate`` / ``up`` are
+        stacks of ``[experts, width, k]`` blocks."""
         tokens, k = xs.shape
         if tokens != self.tokens:
             raise ValueError(f"moe mmq: {tokens} tokens against a plan of {self.tokens}")
@@ -140,7 +143,8 @@ class MmqRouting:
     def down_fold(self, wtype: int, hs: torch.Tensor, down: torch.Tensor, hidden: int, topk_weights: torch.Tensor,
                   residual: torch.Tensor | None = None) -> torch.Tensor:
         """Down projection of the sorted rows ``hs`` ``[rows, k]``, each scaled by its router
-        weight and folded into its token in slot order: ``[tokens, hidden]`` (mmq_experts.rs:440-557)."""
+        weight and folded into its token in slot order: ``[tokens, hidden]`` (mmq_experts.rs:440-557).
+        A pair without an expert adds nothing."""
         rows, k = hs.shape
         if rows != self.rows:
             raise ValueError(f"moe mmq: {rows} rows against a plan of {self.rows}")
@@ -153,12 +157,13 @@ class MmqRouting:
             y = mmq_quantize(wtype, hs.contiguous())
             self._matmul(wtype, down, None, 0, hidden, k, y, pairs, hidden, self.slots)
         out = (residual.reshape(self.tokens, hidden).to(torch.float32).clone() if residual is not None
-               else torch.zeros((self.tokens, hidden), dtype=torch.float32, device=hs.device))
+               else torch.empty((self.tokens, hidden), dtype=torch.float32, device=hs.device))
         w = topk_weights.to(torch.float32).contiguous()
         if w.numel() != rows:
             raise ValueError(f"moe mmq: {w.numel()} router weights for {rows} rows")
-        _lib.load().loken_moe_mmq_fold(pairs.data_ptr(), w.data_ptr(), None, None, out.data_ptr(), self.tokens,
-                                       self.topk, hidden, _stream())
+        _lib.check("lk_moe_fold", _lib.load().lk_moe_fold(
+            pairs.data_ptr(), w.data_ptr(), self.choices.data_ptr(), self.experts, out.data_ptr(), self.tokens, self.topk, hidden,
+            int(residual is not None), _stream()))
         return out
 
 
@@ -433,7 +438,9 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
     """The expert block of one layer, path chosen as the reference's layer code chooses it
     (src/inference/generic_transformer/moe_weights.rs:2118-2152): the expert-batched tiled
     matmuls when there is at least a routed row per expert, else one mat-vec per routed pair.
-    `return_rows`: also the gated rows the second product read, in slot order (token * topk + choice)."""
+    A choice outside ``[0, n_experts)`` adds nothing to its token.
+    `return_rows`: also the gated rows the second product read, in slot order (token * topk + choice), zeros where a
+    choice names no expert."""
     tokens, hidden = x.shape
     topk = choices.shape[1]
     if (not return_rows and x.dtype == topk_weights.dtype == torch.float32 and choices.dtype == torch.int32 and x.is_contiguous()
@@ -454,11 +461,15 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
             return out
         rows = torch.empty_like(h)
         rows[plan.slots.long()] = h   # sorted order -> slot order
-        return out, rows
+        flat = plan.choices.reshape(-1, 1)
+        return out, rows.masked_fill_((flat < 0) | (flat >= n_experts), 0.0)
     routing = ExpertRouting(choices)
     h = moe_gemm_gguf_gate_up_silu_mul(wtype_gu, x.contiguous(), gate, up, routing, n_experts, ffn)
     out = moe_gemm_gguf_down_reduce(wtype_down, h, down, routing, topk_weights.reshape(-1), n_experts, hidden)
-    return (out, h) if return_rows else out
+    if not return_rows:
+        return out
+    flat = choices.reshape(-1, 1)
+    return out, h.masked_fill_((flat < 0) | (flat >= n_experts), 0.0)
 
 
 def moe_q4k_imma_m8_gate_up(x: torch.Tensor, gate_up: torch.Tensor, sorted_token_ids: torch.Tensor,

@@ -640,6 +640,42 @@ def test_pairs_without_an_expert_come_behind_all_others(n, n_experts, topk, shar
     assert np.array_equal(counts.cpu().numpy(), np.bincount(expert, minlength=n_experts + 1)[:n_experts])
 
 
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,dn", [
+    (1, 2, 4, 512, 256, lib.TYPE_Q4_K, lib.TYPE_Q4_K),          # a mat-vec per pair
+    (3, 2, 8, 512, 1280, lib.TYPE_MXFP4, lib.TYPE_MXFP4),
+    (24, 4, 16, 512, 256, lib.TYPE_Q4_K, lib.TYPE_Q4_K),        # rows launches
+    (33, 4, 8, 512, 256, lib.TYPE_Q8_0, lib.TYPE_Q8_0),         # int8 tiles
+    (7, 4, 4, 1024, 768, lib.TYPE_Q4_K, lib.TYPE_Q6_K),         # rows, then tiles
+    (129, 2, 8, 512, 768, lib.TYPE_Q4_K, lib.TYPE_Q4_K),        # f16 tiles
+    (301, 8, 16, 256, 512, lib.TYPE_Q5_K, lib.TYPE_Q6_K)])
+def test_choices_that_name_no_expert_add_nothing(tokens, topk, n_experts, hidden, ffn, gu, dn):
+    """Left-out pairs (-1, the count itself, what the router leaves for a token that is not a number): the block's
+    output is that of the same choices with a weight of zero, bit for bit (a sum gains 0 x a finite row)."""
+    gate, up = (dev(synth.weight(gu, n_experts * ffn, hidden, seed=65, stream=i)) for i in (1, 2))
+    down = dev(synth.weight(dn, n_experts * hidden, ffn, seed=65, stream=3))
+    x = synth.activation(tokens, hidden, seed=65)
+    ids, w = oracle.topk_softmax(synth.activation(tokens, n_experts, seed=65, stream=7), topk)
+    left_out = synth.rand_ints(66, tokens, tokens * topk, 4).reshape(tokens, topk) == 0
+    left_out[-1] = True                                         # a token without any expert: the NaN row below
+    ids_out, w_zero = ids.copy(), w.copy()
+    ids_out[left_out] = np.resize(np.array([-1, n_experts, 0x7FFFFFFF], np.int32), left_out.sum())
+    w_zero[left_out] = 0.0
+    want = moe_forward(gu, dn, dev(x), gate, up, down, dev(ids), dev(w_zero), n_experts, ffn)
+    x_nan, w_nan = x.copy(), w.copy()
+    x_nan[-1] = np.nan
+    w_nan[-1] = np.nan
+    args = (gu, dn, dev(x_nan), gate, up, down, dev(ids_out), dev(w_nan), n_experts, ffn)
+    # the scratch the block works in, left full of values that are no indices and no numbers
+    junk = moe_forward(gu, dn, torch.full((2 * tokens, hidden), float("nan"), device="cuda"), gate, up, down,
+                       dev(np.concatenate([ids, ids])), dev(np.concatenate([w, w])), n_experts, ffn)
+    assert junk.shape == (2 * tokens, hidden)
+    got = moe_forward(*args)
+    assert torch.equal(got, want) and (got[-1] == 0).all()
+    by_launch, rows = moe_forward(*args, return_rows=True)
+    assert torch.equal(by_launch, got)
+    assert (rows[dev(left_out.reshape(-1))] == 0).all() and torch.isfinite(rows).all()
+
+
 # ---------------------------------------------------------------- router
 @pytest.mark.parametrize("tokens,experts,topk,renorm", [(1, 128, 8, True), (16, 128, 8, True), (256, 128, 8, False),
                                                         (7, 60, 4, True), (5, 512, 64, True), (3, 8, 8, False)])
