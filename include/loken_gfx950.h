@@ -710,7 +710,8 @@ int loken_moe_q4k_imma_m8_down(const void* weights, const void* q8_1, const int3
 /* The router step in front of the expert block: softmax over each row of logits [n_rows,
  * n_experts], the n_expert_used largest probabilities in descending order (ties to the lower
  * expert id) into weights / ids [n_rows, n_expert_used], divided by their sum when with_norm != 0.
- * Name and arguments of the reference's launcher (cuda/moe/gate_topk.cu:405-451; topk_softmax,
+ * An expert whose probability is not a number is never chosen; a choice for which none is left gets the id
+ * 0x7FFFFFFF. Name and arguments of the reference's launcher (cuda/moe/gate_topk.cu:405-451; topk_softmax,
  * src/inference/moe_cuda_cpu/mod.rs:2098-2113). Up to 512 experts, up to 64 used; nothing is
  * launched outside that (the caller falls back). */
 void loken_topk_softmax(const float* logits, float* weights, uint32_t* ids, int n_rows, int n_experts,

@@ -30,7 +30,8 @@ static __device__ __forceinline__ float wave_max(float v) {
 // Softmax over the logits a lane brings (p[i]: expert lane + 64 i, -INFINITY past n_experts) and the k largest, by
 // the 64 lanes of one wave; PER = experts / 64 rounded up to a power of two. A round finds the largest
 // probability through lane moves of the vector unit and scalar registers, and the lowest expert that has it by
-// ballots (a permute through LDS per step of the reduction costs four times as much).
+// ballots (a permute through LDS per step of the reduction costs four times as much). Experts of a row are
+// distinct; where nothing is left to choose the id is 0x7FFFFFFF and the weight not a number.
 template <int PER>
 static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], float* __restrict__ weights,
                                                            uint32_t* __restrict__ ids, int n_experts, int topk,
@@ -43,7 +44,7 @@ static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], floa
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int e = lane + 64 * i;
-        p[i] = e < n_experts ? expf(p[i] - mx) : -1.f;   // -1: never chosen, probabilities are >= 0
+        p[i] = e < n_experts ? expf(p[i] - mx) : -1.f;   // -1: never chosen, only probabilities >= 0 are
         sum += e < n_experts ? p[i] : 0.f;
     }
     sum = wave_sum(sum);
@@ -54,11 +55,15 @@ static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], floa
 #pragma unroll
         for (int i = 1; i < PER; ++i) best = fmaxf(best, p[i]);
         best = wave_max(best);
-        int e = 0x7FFFFFFF;   // stays so only where a logit is not a number and nothing compares equal
+        // Logits that are not numbers (and infinite ones, whose difference to the maximum is none) leave fewer
+        // probabilities than choices: `best` is then -1 or not a number itself, and the choice names no expert.
+        int e = 0x7FFFFFFF;
+        if (best >= 0.f) {
 #pragma unroll
-        for (int i = PER - 1; i >= 0; --i) {
-            const unsigned long long at = __ballot(p[i] == best);
-            if (at) e = 64 * i + __ffsll((long long)at) - 1;
+            for (int i = PER - 1; i >= 0; --i) {
+                const unsigned long long at = __ballot(p[i] == best);
+                if (at) e = 64 * i + __ffsll((long long)at) - 1;
+            }
         }
         const float prob = best / sum;
         picked_sum += prob;

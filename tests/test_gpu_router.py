@@ -41,6 +41,55 @@ def test_gate_topk_softmax_matches_the_two_step_path(tokens, hidden, experts, k,
     assert np.array_equal(ids2.cpu().numpy()[clear], ids[clear])
 
 
+NONE = 0x7FFFFFFF
+
+
+def chosen_of(logits, k):
+    """The selection's rule in numpy: probabilities that are numbers, largest first, ties to the lower id."""
+    with np.errstate(invalid="ignore"):
+        p = np.exp(logits - np.fmax.reduce(logits), dtype=np.float32)
+    ids = [e for e in np.argsort(-p, kind="stable") if not np.isnan(p[e])][:k]
+    return np.array(ids + [NONE] * (k - len(ids)), np.int32), bool(np.isnan(p).any())
+
+
+@pytest.mark.parametrize("experts,k", [(5, 5), (40, 3), (64, 8), (100, 64), (128, 8), (200, 16), (512, 64)])
+def test_logits_that_are_not_numbers_are_never_chosen_and_no_expert_twice(experts, k):
+    base = synth.normal(28, experts, 8 * experts).reshape(8, experts).astype(np.float32)
+    base[1, experts // 2] = np.nan
+    base[2] = np.nan
+    base[3, k // 2:] = np.nan                    # fewer numbers than choices
+    base[4, 0] = np.inf                          # inf - inf: not a probability
+    base[5] = -np.inf
+    base[6, 1:] = -np.inf                        # one expert and zeros
+    w, ids = moe.topk_softmax(dev(base), k, True)
+    w, ids = w.cpu().numpy(), ids.cpu().numpy()
+    for row in range(8):
+        want, not_a_number = chosen_of(base[row], k)
+        assert np.array_equal(ids[row], want), row
+        assert np.isnan(w[row]).all() if not_a_number else np.isfinite(w[row]).all(), row
+
+
+@pytest.mark.parametrize("tokens,experts,k", [(1, 40, 8), (16, 128, 8), (17, 33, 4), (40, 300, 8)])
+@pytest.mark.parametrize("aligned", [True, False])   # in two launches, or one (rows that do not start on 16 bytes)
+def test_gate_of_weights_and_tokens_that_are_not_numbers(tokens, experts, k, aligned):
+    hidden = 128
+    x = synth.normal(29, 1, tokens * hidden).reshape(tokens, hidden)
+    gate = (0.1 * synth.normal(29, 2, experts * hidden)).reshape(experts, hidden).astype(np.float32)
+    gate[k - 2:] = np.nan                        # fewer experts with a logit than choices
+    if tokens > 1:
+        x[3] = np.nan
+    xd = torch.empty(tokens * hidden + 1, device="cuda")[0 if aligned else 1:][:tokens * hidden].view(tokens, hidden)
+    xd.copy_(dev(x))
+    w, ids = moe.gate_topk_softmax(xd, dev(gate), k, True)
+    w, ids = w.cpu().numpy(), ids.cpu().numpy()
+    assert np.isnan(w).all() and (ids[:, k - 2:] == NONE).all()
+    for t in range(tokens):
+        if t == 3:
+            assert (ids[t] == NONE).all()
+        else:
+            assert sorted(ids[t, :k - 2].tolist()) == list(range(k - 2))
+
+
 @pytest.mark.parametrize("tokens,experts,k,renorm,scale,with_bias", [(1, 256, 8, True, 2.5, True), (33, 128, 8, True, 1.0, False),
                                                                      (7, 64, 6, False, 1.0, True), (4, 40, 3, True, 0.5, True),
                                                                      (2, 512, 10, True, 1.0, True)])
