@@ -448,10 +448,13 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
             and topk_weights.numel() == choices.numel()):
         # the whole block in one call; what it does not take goes on below, launch by launch
         out = torch.empty((tokens, hidden), dtype=torch.float32, device=x.device)
-        if _lib.load().lk_moe_forward(wtype_gu, wtype_down, x.data_ptr(), gate.data_ptr(), up.data_ptr(), down.data_ptr(),
-                                      choices.data_ptr(), topk_weights.data_ptr(), out.data_ptr(), tokens, topk, n_experts, hidden, ffn,
-                                      _stream()) == _lib.LK_OK:
+        status = _lib.load().lk_moe_forward(wtype_gu, wtype_down, x.data_ptr(), gate.data_ptr(), up.data_ptr(), down.data_ptr(),
+                                            choices.data_ptr(), topk_weights.data_ptr(), out.data_ptr(), tokens, topk, n_experts,
+                                            hidden, ffn, _stream())
+        if status == _lib.LK_OK:
             return out
+        if status not in (_lib.LK_ERR_TYPE, _lib.LK_ERR_ARG, _lib.LK_ERR_NOMEM):
+            raise _lib.LokenError("lk_moe_forward", status)
     if (moe_mmq_pays(tokens * topk, n_experts, wtype_gu if wtype_gu == wtype_down else None)
             and moe_mmq_serves(wtype_gu, hidden) and moe_mmq_serves(wtype_down, ffn)):
         plan = MmqRouting.from_choices(choices, n_experts)
