@@ -598,7 +598,15 @@ int loken_moe_gemm_gguf_down_reduce_static(const float* inputs, const void* weig
 int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
                    const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
                    int hidden, int ffn, void* stream);
-/* The rules it chooses by: whether the expert-batched launches pay at `rows` routed rows (wtype: the stacks' type where
+/* The launches it is made of at this size, as bits: LK_MOE_GROUPED (expert-batched products over a grouped
+ * routing; else a mat-vec per routed pair), and with it LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN where that
+ * product is lk_moe_q4k_rows_grouped rather than the tiled launch. For a caller that issues the launches
+ * itself and wants the block's bits. */
+#define LK_MOE_GROUPED 1
+#define LK_MOE_ROWS_GATE_UP 2
+#define LK_MOE_ROWS_DOWN 4
+int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int topk, int n_experts, int hidden, int ffn);
+/* The rules this goes by, each for one stack alone: whether the expert-batched launches pay at `rows` routed rows (wtype: the stacks' type where
  * all have the same, else -1); the longest run an expert is expected to own (mmq_experts.rs:215-227); whether a stack
  * then takes lk_moe_q4k_rows_grouped. */
 int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype);

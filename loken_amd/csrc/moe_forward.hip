@@ -76,6 +76,29 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
     return wtype == LK_TYPE_Q4_K && k % 256 == 0 && longest_run <= (k <= 2048 ? 44 : 40);
 }
 
+// Which launches the block is made of: LK_MOE_GROUPED (expert-batched products; else a mat-vec per routed pair),
+// and in it LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN (lk_moe_q4k_rows_grouped; else tiles). The one place that decides:
+// lk_moe_forward and a caller that issues the launches itself both ask here.
+// Gate and up also leave the rows launch where
+//   * down is tiled, past 36 rows: tiles for both keep the rows between them in the tiles' layout and the activation in
+//     their quantizer (128 experts as above with a Q6_K down, 26 / 34 / 42 / 50 rows: 175 / 209 / 234 / 241 us against
+//     187 / 203 / 218 / 231)
+//   * their rows are long and their tiles fill the chip, past 20 rows (60 experts of 2560 -> 1280, 600 tiles, at 16 /
+//     25 / 33 / 41 rows 150 / 208 / 217 / 272 us against 161 / 168 / 175 / 190)
+extern "C" int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int topk, int n_experts, int hidden, int ffn) {
+    const Format *fg = format_of(wtype_gu), *fd = format_of(wtype_down);
+    if (!fg || !fd || tokens <= 0 || topk <= 0 || n_experts <= 0) return 0;
+    if (!lk_moe_grouped_pays((int64_t)tokens * topk, n_experts, wtype_gu == wtype_down ? wtype_gu : -1) || !grouped_serves(*fg, hidden) ||
+        !grouped_serves(*fd, ffn))
+        return 0;
+    const int longest = lk_moe_longest_run(tokens, topk, n_experts);
+    const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
+    const bool tiles_fill = 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus;
+    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest) && (rows_down || longest <= 36) &&
+                         (hidden <= 2048 || !tiles_fill || longest <= 20);
+    return LK_MOE_GROUPED | (rows_gu ? LK_MOE_ROWS_GATE_UP : 0) | (rows_down ? LK_MOE_ROWS_DOWN : 0);
+}
+
 extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
                               const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
                               int hidden, int ffn, void* stream) {
@@ -90,8 +113,8 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     const auto scratch = lk_stream_scratch(s);
     std::lock_guard<std::recursive_mutex> lock(scratch->mu);
 
-    if (!(lk_moe_grouped_pays(rows, n_experts, wtype_gu == wtype_down ? wtype_gu : -1) && grouped_serves(*fg, hidden) &&
-          grouped_serves(*fd, ffn))) {
+    const int path = lk_moe_block_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn);
+    if (!(path & LK_MOE_GROUPED)) {
         if (fg->wire < 0 || fd->wire < 0) return LK_ERR_TYPE;
         float* h = (float*)scratch->get(LK_SCRATCH_BLOCK, (size_t)rows * ffn * 4, s);
         if (!h) return LK_ERR_NOMEM;
@@ -100,16 +123,7 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     }
 
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
-    const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
-    // Gate and up also leave the rows launch where
-    //   * down is tiled, past 36 rows: tiles for both keep the rows between them in the tiles' layout and the activation in
-    //     their quantizer (128 experts as above with a Q6_K down, 26 / 34 / 42 / 50 rows: 175 / 209 / 234 / 241 us against
-    //     187 / 203 / 218 / 231)
-    //   * their rows are long and their tiles fill the chip, past 20 rows (60 experts of 2560 -> 1280, 600 tiles, at 16 /
-    //     25 / 33 / 41 rows 150 / 208 / 217 / 272 us against 161 / 168 / 175 / 190)
-    const bool tiles_fill = 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus;
-    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest) && (rows_down || longest <= 36) &&
-                         (hidden <= 2048 || !tiles_fill || longest <= 20);
+    const bool rows_gu = path & LK_MOE_ROWS_GATE_UP, rows_down = path & LK_MOE_ROWS_DOWN;
     const bool gated_later = !rows_gu && !rows_down && ffn % 32 == 0;   // the activation rides the second product's quantizer
     // the buffer's pieces
     size_t at = 0;

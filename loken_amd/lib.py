@@ -12,6 +12,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libloken_gfx950.so"
 LK_OK, LK_ERR_ARG, LK_ERR_TYPE, LK_ERR_LAUNCH, LK_ERR_NOMEM, LK_ERR_SIZE, LK_NOT_TAKEN = 0, 1, 2, 3, 4, 5, 6
 _ERR_NAMES = {1: "LK_ERR_ARG", 2: "LK_ERR_TYPE", 3: "LK_ERR_LAUNCH", 4: "LK_ERR_NOMEM", 5: "LK_ERR_SIZE", 6: "LK_NOT_TAKEN"}
 STATIC_SCRATCH_BYTES = 8 << 20
+MOE_GROUPED, MOE_ROWS_GATE_UP, MOE_ROWS_DOWN = 1, 2, 4
 
 TYPE_F32, TYPE_F16, TYPE_BF16 = 0, 1, 30
 TYPE_Q4_0, TYPE_Q4_1, TYPE_Q5_0, TYPE_Q5_1 = 2, 3, 6, 7
@@ -91,6 +92,7 @@ SIGNATURES.update({
     "loken_moe_gemm_gguf_down_reduce": (_i, [_vp] * 6 + [_i] * 6 + [_vp, _vp, _vp]),
     "loken_moe_gemm_gguf_down_reduce_static": (_i, [_vp] * 6 + [_i] * 6 + [_vp, _vp, _vp]),
     "lk_moe_forward": (_i, [_i, _i] + [_vp] * 7 + [_i] * 5 + [_vp]),
+    "lk_moe_block_path": (_i, [_i] * 7),
     "lk_moe_grouped_pays": (_i, [_i64, _i, _i]),
     "lk_moe_longest_run": (_i, [_i, _i, _i]),
     "lk_moe_rows_launch_pays": (_i, [_i, _i, _i]),

@@ -455,11 +455,12 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
             return out
         if status not in (_lib.LK_ERR_TYPE, _lib.LK_ERR_ARG, _lib.LK_ERR_NOMEM):
             raise _lib.LokenError("lk_moe_forward", status)
-    if (moe_mmq_pays(tokens * topk, n_experts, wtype_gu if wtype_gu == wtype_down else None)
-            and moe_mmq_serves(wtype_gu, hidden) and moe_mmq_serves(wtype_down, ffn)):
+    path = _lib.load().lk_moe_block_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn)
+    if path & _lib.MOE_GROUPED:
         plan = MmqRouting.from_choices(choices, n_experts)
-        h = plan.gate_up_silu(wtype_gu, x, gate, up, ffn)
-        out = plan.down_fold(wtype_down, h, down, hidden, topk_weights.reshape(-1))
+        h = plan.with_path("rows" if path & _lib.MOE_ROWS_GATE_UP else "tiled").gate_up_silu(wtype_gu, x, gate, up, ffn)
+        out = plan.with_path("rows" if path & _lib.MOE_ROWS_DOWN else "tiled").down_fold(wtype_down, h, down, hidden,
+                                                                                       topk_weights.reshape(-1))
         if not return_rows:
             return out
         rows = torch.empty_like(h)

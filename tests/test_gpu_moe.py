@@ -611,6 +611,22 @@ def test_block_in_one_call_is_the_block_launch_by_launch(tokens, topk, n_experts
         assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
 
 
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,dn,rows_gu", [
+    (105, 2, 8, 512, 256, lib.TYPE_Q6_K, True), (115, 2, 8, 512, 256, lib.TYPE_Q6_K, False),   # longest run 36 / 39, down tiled
+    (500, 4, 128, 2304, 256, lib.TYPE_Q4_K, False), (115, 2, 8, 2304, 256, lib.TYPE_Q4_K, True)])   # long rows: tiles fill the chip, or not
+def test_block_launch_by_launch_makes_the_choices_of_the_one_call(tokens, topk, n_experts, hidden, ffn, dn, rows_gu):
+    """Where a product's launch depends on the other one, or on how many tiles there are: the same bits both ways."""
+    path = lib.load().lk_moe_block_path(lib.TYPE_Q4_K, dn, tokens, topk, n_experts, hidden, ffn)
+    assert path & lib.MOE_GROUPED and bool(path & lib.MOE_ROWS_GATE_UP) == rows_gu
+    assert MmqRouting(tokens, topk, n_experts, "cuda").takes_rows_launch(lib.TYPE_Q4_K, hidden)   # the stack's rule alone
+    gate, up = (dev(synth.weight(lib.TYPE_Q4_K, 2 * ffn, hidden, seed=67, stream=i)).repeat(n_experts // 2, 1, 1) for i in (1, 2))
+    down = dev(synth.weight(dn, 2 * hidden, ffn, seed=67, stream=3)).repeat(n_experts // 2, 1, 1)
+    x = dev(synth.activation(tokens, hidden, seed=67))
+    ids, w = oracle.topk_softmax(synth.activation(tokens, n_experts, seed=67, stream=7), topk)
+    args = (lib.TYPE_Q4_K, dn, x, gate, up, down, dev(ids), dev(w), n_experts, ffn)
+    assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
+
+
 @pytest.mark.parametrize("n,n_experts,topk", [(1, 3, 1), (63, 5, 3), (64, 1, 1), (1025, 130, 5), (4097, 512, 1), (8888, 128, 8)])
 def test_routing_is_a_stable_grouping(n, n_experts, topk):
     choices = synth.rand_ints(23, n, n, n_experts).astype(np.int32).reshape(-1, topk)
