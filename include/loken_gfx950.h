@@ -55,7 +55,7 @@ extern "C" {
 #define LK_ERR_ARG 1        /* a size, stride or pointer the kernels cannot take */
 #define LK_ERR_TYPE 2       /* weight / activation / output type not served */
 #define LK_ERR_LAUNCH 3     /* the HIP runtime refused the launch */
-#define LK_ERR_NOMEM 4      /* scratch could not be reserved (MoE decode launchers only) */
+#define LK_ERR_NOMEM 4      /* scratch could not be reserved (expert launchers, expert block, host linear) */
 #define LK_ERR_SIZE 5       /* the call needs more than the fixed scratch of an entry point that allocates nothing */
 #define LK_NOT_TAKEN 6      /* host mirror only: forward would serve this call another way (the reference's None) */
 
@@ -470,8 +470,11 @@ int lk_moe_fold(const float* pairs, const float* weights, const int32_t* choices
  * 10 = IQ4_XS, 11 = IQ3_XXS, 12 = IQ3_S, 13 = IQ2_S, 14 = Q2_0, 15 = IQ2_XXS: src/inference/moe_cuda/gemm.rs:23-39).
  * Weights are stacks [num_experts][size_n][size_k / block].
  * These launchers quantize the f32 activation themselves into a per-(device, stream)
- * grow-only scratch (the one allocation in this library; growing is refused with
- * LK_ERR_NOMEM while the stream is being captured). Return 0 or an LK_ERR_* code.
+ * grow-only scratch, the one allocation in this library. Calls recorded into a graph get scratch of
+ * that graph's own, which no call and no other graph uses, so that its replays need not be kept apart
+ * from anything; it is allocated while recording, where a call outside a capture has needed as much on
+ * any stream of the device before (else LK_ERR_NOMEM: warm up before recording), and lives until the
+ * release below. Return 0 or an LK_ERR_* code.
  * ------------------------------------------------------------------------------------- */
 
 /* out[slot, :] = expert(slot) . x[row], times topk_weights[slot] when given; with weights the
@@ -594,7 +597,7 @@ int loken_moe_gemm_gguf_down_reduce_static(const float* inputs, const void* weig
  * hidden], stacks gate / up [experts, ffn, hidden] of wtype_gu and down [experts, hidden, ffn] of wtype_down, choices
  * int32 and weights f32 [tokens, topk]. A choice outside [0, n_experts) adds nothing, whatever its weight. The launches are those of the entry points above, chosen by size as the layer
  * code of the reference chooses (src/inference/generic_transformer/moe_weights.rs:2118-2152). LK_ERR_TYPE: a format
- * the path does not take; LK_ERR_NOMEM: the scratch would have to grow while the stream records a graph. */
+ * the path does not take; LK_ERR_NOMEM: no scratch (while recording: none of that size outside a capture before). */
 int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
                    const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
                    int hidden, int ffn, void* stream);

@@ -140,9 +140,8 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
             return lk_mmvq_fused(dtype_, 1, vx, (const float*)x, k_, dst, x_type, k_, nn, rows, n_, nullptr, stream);
         }
         const int k_padded = (int)pad_to((size_t)k_, 512), blocks = k_padded / 32;
-        const auto scratch = lk_stream_scratch(stream);
-        std::lock_guard<std::recursive_mutex> pair(scratch->mu);
-        uint8_t* act = (uint8_t*)scratch->get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK, stream);
+        LkScratch scratch(stream);
+        uint8_t* act = (uint8_t*)scratch.get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK);
         if (!act) return LK_ERR_NOMEM;
         if (int rc = lk_quantize_q8_1(x, x_type, act, k_, k_padded, rows, stream)) return rc;
         for (int r0 = 0; r0 < rows; r0 += 8) {
@@ -163,9 +162,8 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
         const int blocks = k_ / 32;
         int rc;
         {
-            const auto scratch = lk_stream_scratch(stream);
-            std::lock_guard<std::recursive_mutex> pair(scratch->mu);
-            void* act = scratch->get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK, stream);
+            LkScratch scratch(stream);
+            void* act = scratch.get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK);
             if (!act) return LK_ERR_NOMEM;
             if (int r = lk_quantize_q8_1(x, x_type, act, k_, k_, rows, stream)) return r;
             // (rows too long for the kernels' scale tables in LDS launch nothing, and the call goes on to the
@@ -184,10 +182,9 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     if (!tiled_serves(dtype_, k_)) return LK_ERR_TYPE;
     const size_t k_padded = pad_to(pad_to((size_t)k_, 512), 128);
     const size_t ws_bytes = (size_t)rows * (k_padded / 128) * MMQ_RECORD + 128 * MMQ_RECORD;
-    const auto scratch = lk_stream_scratch(stream);
-    std::lock_guard<std::recursive_mutex> pair(scratch->mu);
-    void* act = scratch->get(LK_SCRATCH_LINEAR, ws_bytes, stream);
-    void* fixup = scratch->get(LK_SCRATCH_FIXUP, FIXUP_BYTES, stream);
+    LkScratch scratch(stream);
+    void* act = scratch.get(LK_SCRATCH_LINEAR, ws_bytes);
+    void* fixup = scratch.get(LK_SCRATCH_FIXUP, FIXUP_BYTES);
     if (!act || !fixup) return LK_ERR_NOMEM;
     // the layouts of the reference's table (quantized/mmq.rs:274-285)
     auto quantizer = dtype_ == LK_TYPE_Q2_K ? launch_mmq_quantize_q8_1_D2S6

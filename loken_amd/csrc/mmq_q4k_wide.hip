@@ -471,9 +471,8 @@ int lk_mmq_q4k_wide_dense(const MmqProblem& pb, hipStream_t s) {
     const size_t tile_bytes = (size_t)pb.nb * C::UNIT;
     if (tile_bytes > UNITS_CAP) return -1;
     const int tiles_per_pass = (int)std::min<size_t>((size_t)m_tiles, UNITS_CAP / tile_bytes);
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);   // the buffer is the stream's from here until the launches are queued
-    uint8_t* units = (uint8_t*)scratch->get(LK_SCRATCH_TOKENS, tile_bytes * tiles_per_pass, s);
+    LkScratch scratch(s);
+    uint8_t* units = (uint8_t*)scratch.get(LK_SCRATCH_TOKENS, tile_bytes * tiles_per_pass);
     if (!units) return -1;
     for (int t0 = 0; t0 < m_tiles; t0 += tiles_per_pass) {
         const int tiles = std::min(tiles_per_pass, m_tiles - t0);

@@ -272,9 +272,8 @@ extern "C" int loken_moe_gemm_gguf(const float* inputs, const void* weights, con
         return launch_format<MODE_PLAIN>(quant_type, (const uint8_t*)weights, nullptr, (const uint8_t*)inputs,
                                          sorted_token_ids, expert_ids, topk_weights, nullptr, (float*)outputs, d, size_k, s);
     }
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
-    uint8_t* acts = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES, s);
+    LkScratch scratch(s);
+    uint8_t* acts = (uint8_t*)scratch.get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, LK_TYPE_F32, acts, size_k, kp, act_rows, stream)) return rc;
     MoeDims d{num_experts, topk, size_m, size_n, 0, kp / 32, 0};
@@ -303,9 +302,8 @@ extern "C" int loken_moe_gemm_gguf_prefill(const void* inputs, const uint8_t* we
     hipStream_t s = (hipStream_t)stream;
     const int kp = pad512(size_k);
     const int act_rows = topk_weights ? size_m : size_m / topk;
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
-    uint8_t* acts = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES, s);
+    LkScratch scratch(s);
+    uint8_t* acts = (uint8_t*)scratch.get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, input_dtype == 0 ? LK_TYPE_F16 : LK_TYPE_BF16, acts, size_k, kp, act_rows, stream))
         return rc;
@@ -342,9 +340,8 @@ static int gate_up_impl(const float* inputs, const void* gate_weights, const voi
                                          (const uint8_t*)inputs, sorted_token_ids, expert_ids, nullptr, nullptr, outputs,
                                          d, size_k, s);
     }
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
-    uint8_t* acts = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES, s);
+    LkScratch scratch(s);
+    uint8_t* acts = (uint8_t*)scratch.get(LK_SCRATCH_LAUNCHER, (size_t)act_rows * (kp / 32) * Q81_BYTES);
     if (!acts) return LK_ERR_NOMEM;
     if (int rc = lk_quantize_q8_1(inputs, LK_TYPE_F32, acts, size_k, kp, act_rows, stream)) return rc;
     MoeDims d{num_experts, topk, size_m, size_n, 0, kp / 32, 0, 0, slab_rows, act, live, alt};
@@ -453,8 +450,7 @@ static int down_impl(const float* inputs, const void* weights, const int32_t* so
     const bool as_f32 = rows_stage_as_f32(inputs, size_k, gguf_dtype);
     const size_t act_bytes = as_f32 ? 0 : (((size_t)size_m * (kp / 32) * Q81_BYTES) + 255) & ~(size_t)255;
     const size_t pair_bytes = pair_rows ? 0 : (size_t)size_m * size_n * sizeof(float);
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
+    LkScratch scratch(s);
     uint8_t* base = nullptr;
     if (from_static) {
         // nothing is allocated: the device's fixed array, or an error when the call does not fit it
@@ -462,7 +458,7 @@ static int down_impl(const float* inputs, const void* weights, const int32_t* so
         base = static_scratch();
         if (!base) return LK_ERR_LAUNCH;
     } else if (act_bytes + pair_bytes) {
-        base = (uint8_t*)scratch->get(LK_SCRATCH_LAUNCHER, act_bytes + pair_bytes, s);
+        base = (uint8_t*)scratch.get(LK_SCRATCH_LAUNCHER, act_bytes + pair_bytes);
         if (!base) return LK_ERR_NOMEM;
     }
     float* pairs = pair_rows ? pair_rows : (float*)(base + act_bytes);
@@ -596,9 +592,8 @@ extern "C" int loken_moe_q4k_imma_m8_down(const void* weights, const void* q8_1,
     if (!weights || !q8_1 || !sorted_token_ids || !expert_ids || !topk_weights || !output ||
         bad_shape(1, num_experts, topk, size_m, hidden, size_k) || (((uintptr_t)q8_1) & 3) != 0) return LK_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
-    float* pairs = (float*)scratch->get(LK_SCRATCH_LAUNCHER, (size_t)size_m * hidden * sizeof(float), s);
+    LkScratch scratch(s);
+    float* pairs = (float*)scratch.get(LK_SCRATCH_LAUNCHER, (size_t)size_m * hidden * sizeof(float));
     if (!pairs) return LK_ERR_NOMEM;
     // a pair whose slot is out of range writes nothing: its row of the sum must read zero
     const size_t n = (size_t)size_m * hidden;

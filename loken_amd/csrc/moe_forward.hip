@@ -110,13 +110,12 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
         return LK_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
     const int rows = tokens * topk;
-    const auto scratch = lk_stream_scratch(s);
-    std::lock_guard<std::recursive_mutex> lock(scratch->mu);
+    LkScratch scratch(s);
 
     const int path = lk_moe_block_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn);
     if (!(path & LK_MOE_GROUPED)) {
         if (fg->wire < 0 || fd->wire < 0) return LK_ERR_TYPE;
-        float* h = (float*)scratch->get(LK_SCRATCH_BLOCK, (size_t)rows * ffn * 4, s);
+        float* h = (float*)scratch.get(LK_SCRATCH_BLOCK, (size_t)rows * ffn * 4);
         if (!h) return LK_ERR_NOMEM;
         if (int rc = lk_moe_pairs_gate_up(fg->wire, x, gate, up, choices, h, n_experts, topk, rows, ffn, hidden, s)) return rc;
         return lk_moe_pairs_down(fd->wire, h, down, choices, topk_weights, out, n_experts, topk, rows, hidden, ffn, s);
@@ -134,7 +133,7 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     const size_t h_at = take(gated_later ? 0 : (size_t)rows * ffn * 4);
     const size_t y2_at = take(rows_down ? (size_t)rows * (ffn / 32) * Q81_BYTES : workspace_bytes(rows, ffn));
     const size_t pairs_at = take((size_t)rows * hidden * 4);
-    uint8_t* base = (uint8_t*)scratch->get(LK_SCRATCH_BLOCK, at, s);
+    uint8_t* base = (uint8_t*)scratch.get(LK_SCRATCH_BLOCK, at);
     if (!base) return LK_ERR_NOMEM;
     int32_t *bounds = (int32_t*)(base + bounds_at), *slots = (int32_t*)(base + slots_at), *src = (int32_t*)(base + src_at);
     float *gu = (float*)(base + gu_at), *h = (float*)(base + h_at), *pairs = (float*)(base + pairs_at);

@@ -402,9 +402,8 @@ extern "C" void loken_gate_topk_softmax(const float* x_in, const float* gate_w, 
         if (splits > units / (2 * LOGIT_WAVES)) splits = units / (2 * LOGIT_WAVES);
         if (splits > 16) splits = 16;
         if (splits < 1) splits = 1;
-        const auto scratch = lk_stream_scratch(s);
-        std::lock_guard<std::recursive_mutex> lock(scratch->mu);
-        float* part = (float*)scratch->get(LK_SCRATCH_ROUTER, (size_t)splits * n_rows * n_experts * 4, s);
+        LkScratch scratch(s);
+        float* part = (float*)scratch.get(LK_SCRATCH_ROUTER, (size_t)splits * n_rows * n_experts * 4);
         if (part) {
             auto logits = m == 16 ? gate_logits16_kernel : gate_logits32_kernel;
             hipLaunchKernelGGL(logits, dim3(t_tiles, e_tiles, splits), dim3(64 * LOGIT_WAVES), 0, s, x_in, gate_w, part, hidden, n_rows,

@@ -1,125 +1,188 @@
 #include "stream_scratch.h"
 
 #include <thread>
+#include <utility>
+#include <vector>
 
 namespace {
 
-struct Entry {
-    hipStream_t stream;
-    std::thread::id thread;   // hipStreamPerThread is one handle for a stream of every thread
-    std::shared_ptr<LkStreamScratch> scratch;
+struct Block {
+    void* ptr = nullptr;
+    size_t size = 0;
 };
-std::mutex g_mu;
-std::vector<Entry>& g_entries = *new std::vector<Entry>;   // never destroyed: the process may end after its runtime
+
+// Who a pool belongs to. `capture`: the recording its graph comes from; 0, with `recording` false, for calls that run.
+struct Owner {
+    int device = 0;
+    hipStream_t stream = nullptr;
+    std::thread::id thread;   // hipStreamPerThread is one handle for a stream of every thread
+    bool recording = false;
+    unsigned long long capture = 0;
+    bool operator==(const Owner& o) const {
+        return device == o.device && stream == o.stream && thread == o.thread && recording == o.recording && capture == o.capture;
+    }
+};
+
+std::mutex g_mu;   // of what follows; taken inside a pool's lock, never around one
+std::vector<std::shared_ptr<LkScratchPool>>& g_streams = *new std::vector<std::shared_ptr<LkScratchPool>>;   // never destroyed: the
+std::vector<std::shared_ptr<LkScratchPool>>& g_graphs = *new std::vector<std::shared_ptr<LkScratchPool>>;    // process may end after its runtime
 unsigned long long g_clock = 0;
 
 }  // namespace
 
-struct LkStreamScratch::Block {
-    int device;
-    LkScratchUse use;
-    void* ptr;
-    size_t size;
-    ~Block() {   // hipFree waits for the device
-        int current = 0;
-        if (hipGetDevice(&current) == hipSuccess && hipSetDevice(device) == hipSuccess) {
-            (void)hipFree(ptr);
-            (void)hipSetDevice(current);
+struct LkScratchPool {
+    explicit LkScratchPool(const Owner& o) : owner(o) {}
+    ~LkScratchPool() { free_blocks(take_blocks()); }
+
+    std::vector<Block> take_blocks() {   // caller holds mu and g_mu, or has the last reference
+        std::vector<Block> all = std::move(kept);
+        kept.clear();
+        for (Block& b : now) {
+            if (b.ptr) all.push_back(b);
+            b = Block{};
         }
+        return all;
+    }
+    void free_blocks(const std::vector<Block>& blocks) const {   // hipFree waits for the device
+        int current = 0;
+        if (blocks.empty() || hipGetDevice(&current) != hipSuccess || hipSetDevice(owner.device) != hipSuccess) return;
+        for (const Block& b : blocks) (void)hipFree(b.ptr);
+        (void)hipSetDevice(current);
         (void)hipGetLastError();
     }
+
+    const Owner owner;
+    std::recursive_mutex mu;
+    unsigned long long used_at = 0;
+    bool retired = false;   // out of the table: the stream's next call gets another one
+    // written under mu and g_mu, so either is enough to read
+    Block now[LK_SCRATCH_USES];
+    std::vector<Block> kept;   // outgrown
 };
 
-std::vector<std::weak_ptr<LkStreamScratch::Block>>& LkStreamScratch::blocks() {
-    static auto& all = *new std::vector<std::weak_ptr<Block>>;
-    return all;
-}
+namespace {
 
-void LkStreamScratch::free_all() {
-    for (auto& b : now_) b.reset();
-    kept_.clear();
-}
-
-void* LkStreamScratch::get(LkScratchUse use, size_t bytes, hipStream_t stream) {
-    std::shared_ptr<Block>& own = now_[use];
-    const bool fits = own && own->size >= bytes;
-    if (fits && recorded) return own->ptr;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void)hipGetLastError();
-    if (cs != hipStreamCaptureStatusNone) recorded = true;
-    if (fits) return own->ptr;
-    if (cs != hipStreamCaptureStatusNone) {
-        std::lock_guard<std::mutex> lock(g_mu);
-        for (auto it = blocks().rbegin(); it != blocks().rend(); ++it)
-            if (auto b = it->lock(); b && b->device == device_ && b->use == use && b->size >= bytes) {
-                kept_.push_back(b);   // for the graph; calls of this stream outside it get their own
-                return b->ptr;
-            }
-        return nullptr;
-    }
-    void* fresh = nullptr;
-    const size_t want = (bytes + bytes / 4 + 255) & ~(size_t)255;
-    if (hipMalloc(&fresh, want) != hipSuccess) {
+Owner owner_of(hipStream_t stream) {
+    Owner o;
+    if (hipGetDevice(&o.device) != hipSuccess) (void)hipGetLastError();
+    o.stream = stream;
+    if (stream == hipStreamPerThread) o.thread = std::this_thread::get_id();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        status = hipStreamCaptureStatusNone;
     }
-    if (own) kept_.push_back(own);
-    own = std::shared_ptr<Block>(new Block{device_, use, fresh, want});
+    if (status != hipStreamCaptureStatusNone) {
+        o.recording = true;
+        o.capture = id;
+    }
+    return o;
+}
+
+std::shared_ptr<LkScratchPool> pool_of(const Owner& owner) {
+    std::shared_ptr<LkScratchPool> given_up;   // freed after the lock
     std::lock_guard<std::mutex> lock(g_mu);
-    auto& all = blocks();
-    for (size_t i = 0; i < all.size();) {
-        if (all[i].expired()) all.erase(all.begin() + (long)i);
-        else ++i;
+    auto& pools = owner.recording ? g_graphs : g_streams;
+    int held = 0;
+    size_t oldest = pools.size();
+    for (size_t i = pools.size(); i-- > 0;) {   // a capture's pool is among the last
+        LkScratchPool& p = *pools[i];
+        if (p.owner == owner) {
+            p.used_at = ++g_clock;
+            return pools[i];
+        }
+        if (p.owner.device != owner.device) continue;
+        ++held;
+        if (oldest == pools.size() || p.used_at < pools[oldest]->used_at) oldest = i;
     }
-    all.push_back(own);
+    if (!owner.recording && held >= LK_SCRATCH_STREAMS) {
+        given_up = std::move(pools[oldest]);
+        pools.erase(pools.begin() + (long)oldest);
+    }
+    pools.push_back(std::make_shared<LkScratchPool>(owner));
+    pools.back()->used_at = ++g_clock;
+    return pools.back();
+}
+
+// Whether a call outside any capture has reserved `bytes` for `use`, and the device's graphs have room for `want` more.
+bool graph_may_hold(int device, LkScratchUse use, size_t bytes, size_t want) {
+    std::lock_guard<std::mutex> lock(g_mu);
+    bool reserved = false;
+    for (const auto& p : g_streams) reserved = reserved || (p->owner.device == device && p->now[use].size >= bytes);
+    size_t held = 0;
+    for (const auto& p : g_graphs) {
+        if (p->owner.device != device) continue;
+        for (const Block& b : p->now) held += b.size;
+        for (const Block& b : p->kept) held += b.size;
+    }
+    return reserved && want <= LK_SCRATCH_GRAPH_BYTES && held <= LK_SCRATCH_GRAPH_BYTES - want;
+}
+
+void* allocate(size_t bytes) {
+    // An allocation is no operation of a stream and no part of a graph; in the relaxed mode it is allowed whatever
+    // streams are recording, this one or another thread's.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool switched = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* fresh = nullptr;
+    if (hipMalloc(&fresh, bytes) != hipSuccess) fresh = nullptr;
+    if (switched) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    (void)hipGetLastError();
     return fresh;
 }
 
-std::shared_ptr<LkStreamScratch> lk_stream_scratch(hipStream_t stream) {
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) (void)hipGetLastError();
-    const std::thread::id thread = stream == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
-    std::shared_ptr<LkStreamScratch> given_up;   // freed after the lock
+}  // namespace
+
+LkScratch::LkScratch(hipStream_t stream) {
+    const Owner owner = owner_of(stream);
+    do {
+        pool_ = pool_of(owner);
+        lock_ = std::unique_lock<std::recursive_mutex>(pool_->mu);
+        if (!pool_->retired) return;
+        lock_.unlock();
+    } while (true);
+}
+
+LkScratch::~LkScratch() = default;
+
+void* LkScratch::get(LkScratchUse use, size_t bytes) {
+    LkScratchPool& pool = *pool_;
+    Block& own = pool.now[use];
+    if (own.ptr && own.size >= bytes) return own.ptr;
+    const size_t want = ((use == LK_SCRATCH_FIXUP ? bytes : bytes + bytes / 4) + 255) & ~(size_t)255;   // (fixup: one size)
+    if (pool.owner.recording && !graph_may_hold(pool.owner.device, use, bytes, want)) return nullptr;
+    void* fresh = allocate(want);
+    if (!fresh) return nullptr;
     std::lock_guard<std::mutex> lock(g_mu);
-    int held = 0;
-    size_t oldest = g_entries.size();
-    for (size_t i = 0; i < g_entries.size(); ++i) {
-        Entry& e = g_entries[i];
-        if (e.scratch->device() != device) continue;
-        if (e.stream == stream && e.thread == thread) {
-            e.scratch->used_at = ++g_clock;
-            return e.scratch;
-        }
-        if (e.scratch->recorded) continue;
-        ++held;
-        if (oldest == g_entries.size() || e.scratch->used_at < g_entries[oldest].scratch->used_at) oldest = i;
-    }
-    if (held >= LK_SCRATCH_STREAMS) {
-        given_up = std::move(g_entries[oldest].scratch);
-        g_entries.erase(g_entries.begin() + (long)oldest);
-    }
-    g_entries.push_back(Entry{stream, thread, std::make_shared<LkStreamScratch>(device)});
-    g_entries.back().scratch->used_at = ++g_clock;
-    return g_entries.back().scratch;
+    if (own.ptr) pool.kept.push_back(own);
+    own = Block{fresh, want};
+    return fresh;
 }
 
 void lk_stream_scratch_release(int device) {
     int current = 0;
     if (hipGetDevice(&current) != hipSuccess) { (void)hipGetLastError(); return; }
-    std::vector<Entry> entries;
+    std::vector<std::shared_ptr<LkScratchPool>> pools;
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        for (size_t i = 0; i < g_entries.size();) {
-            if (device >= 0 && g_entries[i].scratch->device() != device) { ++i; continue; }
-            entries.push_back(std::move(g_entries[i]));
-            g_entries.erase(g_entries.begin() + (long)i);
-        }
+        for (auto* list : {&g_streams, &g_graphs})
+            for (size_t i = 0; i < list->size();) {
+                if (device >= 0 && (*list)[i]->owner.device != device) { ++i; continue; }
+                pools.push_back(std::move((*list)[i]));
+                list->erase(list->begin() + (long)i);
+            }
     }
-    for (Entry& e : entries) {
-        std::lock_guard<std::recursive_mutex> lock(e.scratch->mu);
-        if (hipSetDevice(e.scratch->device()) != hipSuccess) { (void)hipGetLastError(); continue; }
+    for (auto& p : pools) {
+        std::lock_guard<std::recursive_mutex> lock(p->mu);
+        if (hipSetDevice(p->owner.device) != hipSuccess) { (void)hipGetLastError(); continue; }
         (void)hipDeviceSynchronize();   // queued kernels may still read what is freed below
-        e.scratch->free_all();
+        p->retired = true;
+        std::vector<Block> blocks;
+        {
+            std::lock_guard<std::mutex> table(g_mu);
+            blocks = p->take_blocks();
+        }
+        p->free_blocks(blocks);
     }
     (void)hipSetDevice(current);
     (void)hipGetLastError();

@@ -1,0 +1,108 @@
+// Checks of the launchers' scratch memory (loken_amd/csrc/stream_scratch.hip) on the host, over the runtime of
+// hip_stub/: one case per run, named by the first argument. Exit status 0: the case holds.
+#include "stream_scratch.hip"
+
+#include <stdio.h>
+#include <string.h>
+
+#define CHECK(c)                                                                  \
+    do {                                                                          \
+        if (!(c)) { fprintf(stderr, "%s:%d: %s\n", __FILE__, __LINE__, #c); exit(1); } \
+    } while (0)
+
+static void* take(hipStream_t s, LkScratchUse use, size_t bytes) { return LkScratch(s).get(use, bytes); }
+struct Recording {   // `s` records into capture `id` while this lives
+    hipStream_t s;
+    Recording(hipStream_t stream, unsigned long long id) : s(stream) { s->capture = id; ++fake::captures; }
+    ~Recording() { s->capture = 0; --fake::captures; }
+};
+
+static void a_stream_keeps_its_buffers() {
+    ihipStream_t a, b;
+    void* p = take(&a, LK_SCRATCH_LINEAR, 1000);
+    CHECK(p && take(&a, LK_SCRATCH_LINEAR, 1000) == p && take(&a, LK_SCRATCH_LINEAR, 1) == p);
+    CHECK(take(&b, LK_SCRATCH_LINEAR, 1000) != p && take(&a, LK_SCRATCH_ROUTER, 1000) != p);
+    CHECK(take(hipStreamPerThread, LK_SCRATCH_LINEAR, 1000) != take(nullptr, LK_SCRATCH_LINEAR, 1000));
+    void* q = take(&a, LK_SCRATCH_LINEAR, 1 << 20);
+    CHECK(q && q != p && take(&a, LK_SCRATCH_LINEAR, 1000) == q);
+    fake::device = 1;
+    CHECK(take(&a, LK_SCRATCH_LINEAR, 1000) != q);
+    fake::device = 0;
+    fake::out_of_memory = true;
+    CHECK(!take(&a, LK_SCRATCH_BLOCK, 1000));
+}
+
+static void nothing_is_shared_with_a_graph() {
+    ihipStream_t a, b, c;
+    void* eager_a = take(&a, LK_SCRATCH_BLOCK, 4096);
+    void* eager_b = take(&b, LK_SCRATCH_BLOCK, 100);
+    void *first, *second, *own;
+    {
+        Recording r(&b, 7);
+        first = take(&b, LK_SCRATCH_BLOCK, 4096);
+        CHECK(first && first != eager_a && first != eager_b);          // nobody's from before
+        CHECK(take(&b, LK_SCRATCH_BLOCK, 4000) == first);              // one buffer through one recording of a stream
+        Recording forked(&c, 7);                                       // a second stream of the same capture runs beside it
+        CHECK(take(&c, LK_SCRATCH_BLOCK, 4096) != first);
+        CHECK(take(&a, LK_SCRATCH_BLOCK, 4096) == eager_a);            // another thread's calls go on meanwhile
+        CHECK(take(&a, LK_SCRATCH_LINEAR, 4096) != nullptr);           // and may grow
+    }
+    {
+        Recording r(&b, 8);                                            // the next graph of the same stream
+        second = take(&b, LK_SCRATCH_BLOCK, 4096);
+        CHECK(second && second != first && second != eager_a);
+    }
+    {
+        Recording r(&a, 9);                                            // recorded where the calls ran
+        own = take(&a, LK_SCRATCH_BLOCK, 4096);
+        CHECK(own && own != eager_a && own != first && own != second);
+    }
+    CHECK(take(&b, LK_SCRATCH_BLOCK, 4096) != first && take(&b, LK_SCRATCH_BLOCK, 4096) != second);
+    CHECK(take(&a, LK_SCRATCH_BLOCK, 4096) == eager_a);
+    for (void* p : {first, second, own}) CHECK(fake::live.count(p));   // theirs until the release
+}
+
+static void what_nothing_reserved_is_refused_while_recording() {
+    ihipStream_t a, b;
+    {
+        Recording r(&a, 1);
+        CHECK(!take(&a, LK_SCRATCH_LINEAR, 100));
+    }
+    CHECK(take(&b, LK_SCRATCH_LINEAR, 100));
+    {
+        Recording r(&a, 2);
+        CHECK(take(&a, LK_SCRATCH_LINEAR, 100));
+        CHECK(!take(&a, LK_SCRATCH_LINEAR, 1000) && !take(&a, LK_SCRATCH_ROUTER, 100));
+    }
+    lk_stream_scratch_release(-1);
+    CHECK(fake::held() == 0);
+    Recording r(&a, 3);
+    CHECK(!take(&a, LK_SCRATCH_LINEAR, 100));
+}
+
+static void graphs_together_stay_within_their_bound() {
+    ihipStream_t a;
+    const size_t big = LK_SCRATCH_GRAPH_BYTES / 4;   // a quarter more is reserved each time
+    CHECK(take(&a, LK_SCRATCH_TOKENS, big));
+    for (int i = 1; i <= 4; ++i) {
+        Recording r(&a, (unsigned long long)i);
+        CHECK((take(&a, LK_SCRATCH_TOKENS, big) != nullptr) == (i <= 3));
+    }
+    lk_stream_scratch_release(-1);
+    CHECK(take(&a, LK_SCRATCH_TOKENS, big));
+    Recording r(&a, 9);
+    CHECK(take(&a, LK_SCRATCH_TOKENS, big));
+}
+
+int main(int argc, char** argv) {
+    const struct { const char* name; void (*run)(); } cases[] = {
+#define CASE(f) {#f, f}
+        CASE(a_stream_keeps_its_buffers), CASE(nothing_is_shared_with_a_graph),
+        CASE(what_nothing_reserved_is_refused_while_recording), CASE(graphs_together_stay_within_their_bound),
+    };
+    for (auto& c : cases) {
+        if (argc < 2) puts(c.name);
+        else if (!strcmp(argv[1], c.name)) return c.run(), 0;
+    }
+    return argc < 2 ? 0 : 2;
+}

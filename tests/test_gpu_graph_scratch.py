@@ -1,0 +1,121 @@
+"""Calls that work in the library's scratch memory, recorded into graphs: replays beside calls and other graphs on
+streams that nothing orders against them, every one the eager bits."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import oracle
+from loken_amd import lib, moe, synth
+from test_gpu_host_mirror import Linear
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def record(fn, stream):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            out = fn()
+    return graph, out
+
+
+def check_replays(calls, stream):
+    """`calls`: functions of one operation over inputs of their own. The first two are recorded, both on `stream`, and
+    replayed on two more while the last runs eagerly where all were warmed up and where they were recorded."""
+    want = [fn() for fn in calls]
+    torch.cuda.synchronize()
+    graphs = [record(fn, stream) for fn in calls[:2]]
+    c, d = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for _, out in graphs:
+            out.zero_()
+        torch.cuda.synchronize()
+        for _ in range(5):
+            for (graph, _), s in zip(graphs, (c, d)):
+                with torch.cuda.stream(s):
+                    graph.replay()
+            here = calls[2]()
+            with torch.cuda.stream(stream):
+                there = calls[2]()
+        torch.cuda.synchronize()
+        for got, w in zip([out for _, out in graphs] + [here, there], [want[0], want[1], want[2], want[2]]):
+            assert torch.equal(got, w)
+
+
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,dn", [
+    (2, 2, 16, 1024, 512, lib.TYPE_Q8_0, lib.TYPE_Q8_0),         # mat-vec per pair
+    (64, 4, 16, 1024, 512, lib.TYPE_Q4_K, lib.TYPE_Q4_K),        # rows launches
+    (200, 4, 8, 1024, 768, lib.TYPE_Q4_K, lib.TYPE_Q6_K)])       # tiles
+def test_mixture_layer(tokens, topk, n_experts, hidden, ffn, gu, dn):
+    gate, up = (dev(synth.weight(gu, n_experts * ffn, hidden, seed=70, stream=i)) for i in (1, 2))
+    down = dev(synth.weight(dn, n_experts * hidden, ffn, seed=70, stream=3))
+    router = dev((synth.normal(70, 4, n_experts * hidden) * 0.05).reshape(n_experts, hidden).astype(np.float32))
+    L = lib.load()
+
+    def layer(seed):
+        x = dev(synth.activation(tokens, hidden, seed=seed))
+
+        def call():
+            w, ids = moe.gate_topk_softmax(x, router, topk)
+            out = torch.empty((tokens, hidden), device="cuda")
+            lib.check("lk_moe_forward", L.lk_moe_forward(
+                gu, dn, x.data_ptr(), gate.data_ptr(), up.data_ptr(), down.data_ptr(), ids.data_ptr(), w.data_ptr(), out.data_ptr(),
+                tokens, topk, n_experts, hidden, ffn, torch.cuda.current_stream().cuda_stream))
+            return out
+        return call
+
+    check_replays([layer(seed) for seed in (71, 72, 73)], torch.cuda.Stream())
+
+
+@pytest.mark.parametrize("wtype,n,k,rows,half", [(lib.TYPE_Q8_0, 300, 1024, 5, False), (lib.TYPE_Q4_K, 4096, 1024, 12, True),
+                                                  (lib.TYPE_Q5_K, 600, 4096, 77, True), (lib.TYPE_Q4_K, 4096, 1024, 200, False)])
+def test_linear(wtype, n, k, rows, half):
+    lin = Linear(wtype, dev(synth.weight(wtype, n, k, seed=74, stream=1)), n, k)
+
+    def call(seed):
+        x = dev(synth.activation(rows, k, seed=seed)).to(torch.float16 if half else torch.float32)
+        return lambda: lin(x)
+
+    try:
+        check_replays([call(seed) for seed in (75, 76, 77)], torch.cuda.Stream())
+    finally:
+        lin.close()
+
+
+def test_scratch_that_grows_after_a_recording():
+    """A graph keeps what it was recorded with, whatever the streams' buffers become."""
+    wtype, n, k = lib.TYPE_Q4_K, 640, 2048
+    lin = Linear(wtype, dev(synth.weight(wtype, n, k, seed=78, stream=1)), n, k)
+    x = dev(synth.activation(20, k, seed=78))
+    side = torch.cuda.Stream()
+    want = lin(x)
+    graph, out = record(lambda: lin(x), side)
+    for rows in (100, 300, 900):
+        big = dev(synth.activation(rows, k, seed=79))
+        with torch.cuda.stream(side):
+            there = lin(big)
+        here = lin(big)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(here, there)
+    lin.close()
+
+
+def test_router_recorded_before_any_call_takes_its_form_without_scratch():
+    lib.load().loken_stream_scratch_release()
+    x = dev(synth.activation(9, 512, seed=80))
+    gate = dev((synth.normal(80, 2, 64 * 512) * 0.05).reshape(64, 512).astype(np.float32))
+    graph, (w, ids) = record(lambda: moe.gate_topk_softmax(x, gate, 4), torch.cuda.Stream())
+    want_ids, want_w = oracle.topk_softmax((x.double() @ gate.double().T).float().cpu().numpy(), 4)
+    for _ in range(3):
+        ids.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(ids.cpu().numpy(), want_ids) and np.abs(w.cpu().numpy() - want_w).max() < 2e-5
