@@ -751,7 +751,9 @@ void loken_stable_sort_u32(const uint32_t* keys, uint32_t* sorted, uint32_t* ord
 /* The decode-size form (cuda/moe/gate_topk.cu:453-477; src/inference/moe_cuda/dense/gate.rs:185):
  * same result for m keys; the reference serves m <= 32, this m <= 256, nothing is launched above. */
 void loken_argsort_small_u32(const uint32_t* in, uint32_t* sorted_out, uint32_t* index_out, int m, void* stream);
-/* Frees the current device's MoE decode scratch (cuda/moe/moe_gguf.cu:104-118). Synchronizes. */
+/* Frees what the expert launchers, the expert block, the router and the wide tiles hold on the current device, for
+ * every stream and every recorded graph: none recorded over them may be replayed after. The host linears' workspaces
+ * stay (lkh_release_workspaces). Synchronizes the device (cuda/moe/moe_gguf.cu:104-118). */
 void loken_stream_scratch_release(void);
 
 /* Makes every LK_TUNE_* / LK_MMQ_* environment override (launch shapes and path choices of

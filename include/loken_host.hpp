@@ -90,7 +90,8 @@ private:
     Path last_path_ = Path::None;
 };
 
-/* Frees every workspace this layer holds on every device (synchronizes those devices). */
+/* Frees every workspace this layer holds on every device, those of recorded graphs of linears among them: none may be
+ * replayed after (synchronizes those devices). What the expert launchers hold stays (loken_stream_scratch_release). */
 void release_workspaces();
 
 /* ------------------------------------------------------------------------------------------

@@ -280,7 +280,7 @@ int QKernelMatMul::forward_quantized_pair(QKernelMatMul& other, const QuantizedA
     return LK_OK;
 }
 
-void release_workspaces() { lk_stream_scratch_release(-1); }
+void release_workspaces() { lk_stream_scratch_release(-1, LK_SCRATCH_OF_LINEARS); }
 
 }  // namespace loken
 

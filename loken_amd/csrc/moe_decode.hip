@@ -244,7 +244,7 @@ static inline bool rows_stage_as_f32(const float* inputs, int size_k, int quant_
 
 extern "C" void loken_stream_scratch_release() {
     int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) lk_stream_scratch_release(dev);
+    if (hipGetDevice(&dev) == hipSuccess) lk_stream_scratch_release(dev, LK_SCRATCH_OF_LAUNCHERS);
 }
 
 extern "C" void loken_moe_sum_topk(const float* pairs, float* outputs, int tokens, int topk, int cols, void* stream) {

@@ -52,5 +52,9 @@ class LkScratch {
 constexpr int LK_SCRATCH_STREAMS = 32;
 // What all recorded graphs of a device may hold together.
 constexpr size_t LK_SCRATCH_GRAPH_BYTES = (size_t)32 << 30;
-// Gives back what the streams and graphs of `device` hold (-1: of every device). Waits for the device.
-void lk_stream_scratch_release(int device);
+// The uses of the host linears, and those of everything else: each side gives back its own.
+constexpr unsigned LK_SCRATCH_OF_LINEARS = 1u << LK_SCRATCH_LINEAR | 1u << LK_SCRATCH_FIXUP;
+constexpr unsigned LK_SCRATCH_OF_LAUNCHERS = (1u << LK_SCRATCH_USES) - 1 - LK_SCRATCH_OF_LINEARS;
+// Gives back what the streams and graphs of `device` (-1: of every device) hold for `uses`, a bit per use. Waits for
+// the device; a graph recorded over any of it must not be replayed after.
+void lk_stream_scratch_release(int device, unsigned uses);

@@ -9,7 +9,9 @@ namespace {
 struct Block {
     void* ptr = nullptr;
     size_t size = 0;
+    LkScratchUse use = LK_SCRATCH_USES;
 };
+constexpr unsigned EVERY_USE = (1u << LK_SCRATCH_USES) - 1;
 
 // Who a pool belongs to. `capture`: the recording its graph comes from; 0, with `recording` false, for calls that run.
 struct Owner {
@@ -32,16 +34,23 @@ unsigned long long g_clock = 0;
 
 struct LkScratchPool {
     explicit LkScratchPool(const Owner& o) : owner(o) {}
-    ~LkScratchPool() { free_blocks(take_blocks()); }
+    ~LkScratchPool() { free_blocks(take_blocks(EVERY_USE)); }
 
-    std::vector<Block> take_blocks() {   // caller holds mu and g_mu, or has the last reference
-        std::vector<Block> all = std::move(kept);
-        kept.clear();
-        for (Block& b : now) {
-            if (b.ptr) all.push_back(b);
-            b = Block{};
-        }
-        return all;
+    std::vector<Block> take_blocks(unsigned uses) {   // caller holds mu and g_mu, or has the last reference
+        std::vector<Block> taken, stay;
+        for (const Block& b : kept) (uses >> b.use & 1 ? taken : stay).push_back(b);
+        kept = std::move(stay);
+        for (Block& b : now)
+            if (b.ptr && uses >> b.use & 1) {
+                taken.push_back(b);
+                b = Block{};
+            }
+        return taken;
+    }
+    bool empty() const {
+        for (const Block& b : now)
+            if (b.ptr) return false;
+        return kept.empty();
     }
     void free_blocks(const std::vector<Block>& blocks) const {   // hipFree waits for the device
         int current = 0;
@@ -155,32 +164,37 @@ void* LkScratch::get(LkScratchUse use, size_t bytes) {
     if (!fresh) return nullptr;
     std::lock_guard<std::mutex> lock(g_mu);
     if (own.ptr) pool.kept.push_back(own);
-    own = Block{fresh, want};
+    own = Block{fresh, want, use};
     return fresh;
 }
 
-void lk_stream_scratch_release(int device) {
+void lk_stream_scratch_release(int device, unsigned uses) {
     int current = 0;
     if (hipGetDevice(&current) != hipSuccess) { (void)hipGetLastError(); return; }
     std::vector<std::shared_ptr<LkScratchPool>> pools;
     {
         std::lock_guard<std::mutex> lock(g_mu);
         for (auto* list : {&g_streams, &g_graphs})
-            for (size_t i = 0; i < list->size();) {
-                if (device >= 0 && (*list)[i]->owner.device != device) { ++i; continue; }
-                pools.push_back(std::move((*list)[i]));
-                list->erase(list->begin() + (long)i);
-            }
+            for (const auto& p : *list)
+                if (device < 0 || p->owner.device == device) pools.push_back(p);
     }
     for (auto& p : pools) {
         std::lock_guard<std::recursive_mutex> lock(p->mu);
-        if (hipSetDevice(p->owner.device) != hipSuccess) { (void)hipGetLastError(); continue; }
-        (void)hipDeviceSynchronize();   // queued kernels may still read what is freed below
-        p->retired = true;
+        // queued kernels may still read what is freed: nothing is where they cannot be waited for
+        if (hipSetDevice(p->owner.device) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            continue;
+        }
         std::vector<Block> blocks;
         {
             std::lock_guard<std::mutex> table(g_mu);
-            blocks = p->take_blocks();
+            blocks = p->take_blocks(uses);
+            if (p->empty() && !p->retired) {
+                p->retired = true;
+                auto& list = p->owner.recording ? g_graphs : g_streams;
+                for (size_t i = 0; i < list.size(); ++i)
+                    if (list[i] == p) { list.erase(list.begin() + (long)i); break; }
+            }
         }
         p->free_blocks(blocks);
     }

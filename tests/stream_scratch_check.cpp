@@ -74,7 +74,7 @@ static void what_nothing_reserved_is_refused_while_recording() {
         CHECK(take(&a, LK_SCRATCH_LINEAR, 100));
         CHECK(!take(&a, LK_SCRATCH_LINEAR, 1000) && !take(&a, LK_SCRATCH_ROUTER, 100));
     }
-    lk_stream_scratch_release(-1);
+    lk_stream_scratch_release(-1, ~0u);
     CHECK(fake::held() == 0);
     Recording r(&a, 3);
     CHECK(!take(&a, LK_SCRATCH_LINEAR, 100));
@@ -88,10 +88,43 @@ static void graphs_together_stay_within_their_bound() {
         Recording r(&a, (unsigned long long)i);
         CHECK((take(&a, LK_SCRATCH_TOKENS, big) != nullptr) == (i <= 3));
     }
-    lk_stream_scratch_release(-1);
+    lk_stream_scratch_release(-1, ~0u);
     CHECK(take(&a, LK_SCRATCH_TOKENS, big));
     Recording r(&a, 9);
     CHECK(take(&a, LK_SCRATCH_TOKENS, big));
+}
+
+static void a_release_frees_its_own_part() {
+    ihipStream_t a;
+    void* held[2][LK_SCRATCH_USES][2];   // device, use, by a call / by a graph
+    for (int d = 0; d < 2; ++d) {
+        fake::device = d;
+        for (int u = 0; u < LK_SCRATCH_USES; ++u) held[d][u][0] = take(&a, (LkScratchUse)u, 1000);
+        Recording r(&a, 5);
+        for (int u = 0; u < LK_SCRATCH_USES; ++u) held[d][u][1] = take(&a, (LkScratchUse)u, 1000);
+    }
+    fake::device = 0;
+    void* outgrown = take(&a, LK_SCRATCH_LINEAR, 1000);
+    void* grown = take(&a, LK_SCRATCH_LINEAR, 10000);
+    auto lives = [&](int d, int u) { return fake::live.count(held[d][u][0]) + fake::live.count(held[d][u][1]); };
+    fake::sync_fails = true;             // a device that cannot be waited for keeps everything
+    lk_stream_scratch_release(-1, ~0u);
+    CHECK(fake::frees == 0);
+    fake::sync_fails = false;
+    lk_stream_scratch_release(1, LK_SCRATCH_OF_LAUNCHERS);
+    for (int u = 0; u < LK_SCRATCH_USES; ++u) {
+        const bool linears = u == LK_SCRATCH_LINEAR || u == LK_SCRATCH_FIXUP;
+        CHECK(lives(0, u) == 2 && lives(1, u) == (linears ? 2u : 0u));
+    }
+    CHECK(take(&a, LK_SCRATCH_LINEAR, 10000) == grown && outgrown == held[0][LK_SCRATCH_LINEAR][0]);
+    lk_stream_scratch_release(-1, LK_SCRATCH_OF_LINEARS);
+    for (int u = 0; u < LK_SCRATCH_USES; ++u) {
+        const bool linears = u == LK_SCRATCH_LINEAR || u == LK_SCRATCH_FIXUP;
+        CHECK(lives(0, u) == (linears ? 0u : 2u) && lives(1, u) == 0);
+    }
+    CHECK(!fake::live.count(grown) && fake::device == 0);
+    lk_stream_scratch_release(0, LK_SCRATCH_OF_LAUNCHERS);
+    CHECK(fake::held() == 0 && take(&a, LK_SCRATCH_BLOCK, 10));
 }
 
 int main(int argc, char** argv) {
@@ -99,6 +132,7 @@ int main(int argc, char** argv) {
 #define CASE(f) {#f, f}
         CASE(a_stream_keeps_its_buffers), CASE(nothing_is_shared_with_a_graph),
         CASE(what_nothing_reserved_is_refused_while_recording), CASE(graphs_together_stay_within_their_bound),
+        CASE(a_release_frees_its_own_part),
     };
     for (auto& c : cases) {
         if (argc < 2) puts(c.name);

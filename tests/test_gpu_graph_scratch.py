@@ -108,6 +108,25 @@ def test_scratch_that_grows_after_a_recording():
     lin.close()
 
 
+def test_dropping_the_linears_workspaces_leaves_the_mixtures_graph():
+    tokens, topk, n_experts, hidden, ffn = 64, 4, 8, 512, 256
+    gate, up = (dev(synth.weight(lib.TYPE_Q6_K, n_experts * ffn, hidden, seed=81, stream=i)) for i in (1, 2))
+    down = dev(synth.weight(lib.TYPE_Q6_K, n_experts * hidden, ffn, seed=81, stream=3))
+    ids, w = oracle.topk_softmax(synth.activation(tokens, n_experts, seed=81, stream=7), topk)
+    args = (lib.TYPE_Q6_K, lib.TYPE_Q6_K, dev(synth.activation(tokens, hidden, seed=81)), gate, up, down, dev(ids), dev(w), n_experts, ffn)
+    want = moe.moe_forward(*args)
+    graph, out = record(lambda: moe.moe_forward(*args), torch.cuda.Stream())
+    for _ in range(3):
+        lib.load().lkh_release_workspaces()
+        filler = torch.full((64 << 20,), 7.0, device="cuda")   # over what a release of too much would have given back
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and (filler == 7.0).all()
+        del filler
+        torch.cuda.empty_cache()
+
+
 def test_router_recorded_before_any_call_takes_its_form_without_scratch():
     lib.load().loken_stream_scratch_release()
     x = dev(synth.activation(9, 512, seed=80))
