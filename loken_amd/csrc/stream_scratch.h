@@ -6,6 +6,9 @@
 // A recorded graph replays on whatever stream its program picks, beside calls and graphs that stream order does
 // not keep apart from it. So what is recorded gets buffers of its own, per (capture, stream), that no call and no
 // other graph uses, and keeps them until the release.
+//
+// Past LK_SCRATCH_STREAMS streams of a device (destroyed ones count until the release) the further ones share one
+// set of buffers, ordered by such events.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -44,11 +47,12 @@ class LkScratch {
     void* get(LkScratchUse use, size_t bytes);
 
   private:
+    hipStream_t stream_;
     std::shared_ptr<LkScratchPool> pool_;
     std::unique_lock<std::recursive_mutex> lock_;
 };
 
-// At most LK_SCRATCH_STREAMS streams of a device hold some: past that the least recently used one gives its up.
+// Streams of a device with buffers of their own.
 constexpr int LK_SCRATCH_STREAMS = 32;
 // What all recorded graphs of a device may hold together.
 constexpr size_t LK_SCRATCH_GRAPH_BYTES = (size_t)32 << 30;

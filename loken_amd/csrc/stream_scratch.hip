@@ -13,28 +13,31 @@ struct Block {
 };
 constexpr unsigned EVERY_USE = (1u << LK_SCRATCH_USES) - 1;
 
-// Who a pool belongs to. `capture`: the recording its graph comes from; 0, with `recording` false, for calls that run.
+// Who a pool belongs to: a stream, what a stream records in one capture, or (`shared`) the streams without their own.
 struct Owner {
     int device = 0;
     hipStream_t stream = nullptr;
     std::thread::id thread;   // hipStreamPerThread is one handle for a stream of every thread
-    bool recording = false;
+    bool recording = false, shared = false;
     unsigned long long capture = 0;
     bool operator==(const Owner& o) const {
-        return device == o.device && stream == o.stream && thread == o.thread && recording == o.recording && capture == o.capture;
+        return device == o.device && stream == o.stream && thread == o.thread && recording == o.recording && shared == o.shared &&
+               capture == o.capture;
     }
 };
 
 std::mutex g_mu;   // of what follows; taken inside a pool's lock, never around one
 std::vector<std::shared_ptr<LkScratchPool>>& g_streams = *new std::vector<std::shared_ptr<LkScratchPool>>;   // never destroyed: the
 std::vector<std::shared_ptr<LkScratchPool>>& g_graphs = *new std::vector<std::shared_ptr<LkScratchPool>>;    // process may end after its runtime
-unsigned long long g_clock = 0;
 
 }  // namespace
 
 struct LkScratchPool {
     explicit LkScratchPool(const Owner& o) : owner(o) {}
-    ~LkScratchPool() { free_blocks(take_blocks(EVERY_USE)); }
+    ~LkScratchPool() {
+        free_blocks(take_blocks(EVERY_USE));
+        if (last_use && hipEventDestroy(last_use) != hipSuccess) (void)hipGetLastError();
+    }
 
     std::vector<Block> take_blocks(unsigned uses) {   // caller holds mu and g_mu, or has the last reference
         std::vector<Block> taken, stay;
@@ -62,11 +65,15 @@ struct LkScratchPool {
 
     const Owner owner;
     std::recursive_mutex mu;
-    unsigned long long used_at = 0;
     bool retired = false;   // out of the table: the stream's next call gets another one
     // written under mu and g_mu, so either is enough to read
     Block now[LK_SCRATCH_USES];
     std::vector<Block> kept;   // outgrown
+    // of a shared pool, under mu: how many of the thread's launchers hold it, whether they took a buffer, and the
+    // last kernels of those before them
+    int held = 0;
+    bool taken = false;
+    hipEvent_t last_use = nullptr;
 };
 
 namespace {
@@ -89,28 +96,25 @@ Owner owner_of(hipStream_t stream) {
     return o;
 }
 
-std::shared_ptr<LkScratchPool> pool_of(const Owner& owner) {
-    std::shared_ptr<LkScratchPool> given_up;   // freed after the lock
+std::shared_ptr<LkScratchPool> pool_of(Owner owner) {
     std::lock_guard<std::mutex> lock(g_mu);
     auto& pools = owner.recording ? g_graphs : g_streams;
-    int held = 0;
-    size_t oldest = pools.size();
+    int of_device = 0;
+    std::shared_ptr<LkScratchPool> shared;
     for (size_t i = pools.size(); i-- > 0;) {   // a capture's pool is among the last
-        LkScratchPool& p = *pools[i];
-        if (p.owner == owner) {
-            p.used_at = ++g_clock;
-            return pools[i];
-        }
-        if (p.owner.device != owner.device) continue;
-        ++held;
-        if (oldest == pools.size() || p.used_at < pools[oldest]->used_at) oldest = i;
+        if (pools[i]->owner == owner) return pools[i];
+        if (pools[i]->owner.device != owner.device) continue;
+        if (pools[i]->owner.shared) shared = pools[i];
+        else ++of_device;
     }
-    if (!owner.recording && held >= LK_SCRATCH_STREAMS) {
-        given_up = std::move(pools[oldest]);
-        pools.erase(pools.begin() + (long)oldest);
+    if (!owner.recording && of_device >= LK_SCRATCH_STREAMS) {
+        if (shared) return shared;
+        const int device = owner.device;
+        owner = Owner{};
+        owner.device = device;
+        owner.shared = true;
     }
     pools.push_back(std::make_shared<LkScratchPool>(owner));
-    pools.back()->used_at = ++g_clock;
     return pools.back();
 }
 
@@ -142,20 +146,35 @@ void* allocate(size_t bytes) {
 
 }  // namespace
 
-LkScratch::LkScratch(hipStream_t stream) {
+LkScratch::LkScratch(hipStream_t stream) : stream_(stream) {
     const Owner owner = owner_of(stream);
     do {
         pool_ = pool_of(owner);
         lock_ = std::unique_lock<std::recursive_mutex>(pool_->mu);
-        if (!pool_->retired) return;
+        if (!pool_->retired) break;
         lock_.unlock();
     } while (true);
+    ++pool_->held;
 }
 
-LkScratch::~LkScratch() = default;
+LkScratch::~LkScratch() {
+    LkScratchPool& pool = *pool_;
+    if (--pool.held > 0 || !pool.taken) return;
+    pool.taken = false;   // (set by a shared pool only)
+    if (!pool.last_use && hipEventCreateWithFlags(&pool.last_use, hipEventDisableTiming) != hipSuccess) pool.last_use = nullptr;
+    if (!pool.last_use || hipEventRecord(pool.last_use, stream_) != hipSuccess) (void)hipStreamSynchronize(stream_);
+    (void)hipGetLastError();
+}
 
 void* LkScratch::get(LkScratchUse use, size_t bytes) {
     LkScratchPool& pool = *pool_;
+    if (pool.owner.shared && !pool.taken) {
+        if (pool.last_use && hipStreamWaitEvent(stream_, pool.last_use, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        pool.taken = true;
+    }
     Block& own = pool.now[use];
     if (own.ptr && own.size >= bytes) return own.ptr;
     const size_t want = ((use == LK_SCRATCH_FIXUP ? bytes : bytes + bytes / 4) + 255) & ~(size_t)255;   // (fixup: one size)

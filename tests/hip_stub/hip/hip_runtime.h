@@ -25,7 +25,7 @@ namespace fake {
 inline std::mutex mu;
 inline std::map<void*, std::pair<int, size_t>> live;   // address -> device, bytes
 inline int frees = 0, allocations = 0, captures = 0;   // `captures`: recordings under way anywhere, in the global mode
-inline bool out_of_memory = false, sync_fails = false;
+inline bool out_of_memory = false, sync_fails = false, no_events = false;
 inline std::vector<std::string> log;                   // waits and records, in order
 inline thread_local int device = 0;
 inline thread_local hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
@@ -69,4 +69,21 @@ inline hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
     std::swap(*m, fake::mode);
     return hipSuccess;
 }
+inline void note(const char* what, const void* stream) {
+    std::lock_guard<std::mutex> lock(fake::mu);
+    fake::log.push_back(std::string(what) + " " + std::to_string((size_t)stream));
+}
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    if (fake::no_events) return hipErrorOutOfMemory;
+    *e = new ihipEvent_t;
+    return hipSuccess;
+}
+inline hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { e->recorded_on = s; note("record", s); return hipSuccess; }
+inline hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    if (!e->recorded_on) abort();
+    note("wait", s);
+    return hipSuccess;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t s) { note("synchronize", s); return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return fake::sync_fails || fake::refused() ? hipErrorStreamCaptureUnsupported : hipSuccess; }

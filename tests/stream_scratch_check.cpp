@@ -127,12 +127,78 @@ static void a_release_frees_its_own_part() {
     CHECK(fake::held() == 0 && take(&a, LK_SCRATCH_BLOCK, 10));
 }
 
+static void streams_past_the_bound_share_in_order() {
+    static ihipStream_t many[LK_SCRATCH_STREAMS + 3];
+    for (int round = 0; round < 3; ++round)
+        for (auto& s : many) CHECK(take(&s, LK_SCRATCH_LINEAR, 1000));
+    CHECK(fake::allocations == LK_SCRATCH_STREAMS + 1 && fake::frees == 0);   // round after round nothing is freed or allocated
+    ihipStream_t *x = &many[LK_SCRATCH_STREAMS], *y = x + 1;
+    CHECK(take(x, LK_SCRATCH_LINEAR, 1000) == take(y, LK_SCRATCH_LINEAR, 1000));
+    fake::log.clear();
+    CHECK(take(&many[0], LK_SCRATCH_LINEAR, 1000) != take(&many[1], LK_SCRATCH_LINEAR, 1000) && fake::log.empty());
+    {   // a launcher that calls others: one wait before its first buffer, one record behind its last launch
+        LkScratch outer(x);
+        CHECK(fake::log.empty());
+        CHECK(outer.get(LK_SCRATCH_BLOCK, 10) && LkScratch(x).get(LK_SCRATCH_LAUNCHER, 10) && outer.get(LK_SCRATCH_BLOCK, 10));
+        CHECK(fake::log.size() == 1 && fake::log[0] == "wait " + std::to_string((size_t)x));
+    }
+    CHECK(fake::log.size() == 2 && fake::log[1] == "record " + std::to_string((size_t)x));
+    CHECK(take(y, LK_SCRATCH_BLOCK, 10) && fake::log[2] == "wait " + std::to_string((size_t)y) && fake::log.size() == 4);
+    { LkScratch none(y); }               // took nothing: nothing to order
+    CHECK(fake::log.size() == 4);
+    {
+        Recording r(y, 3);               // a graph has its own, past the bound too
+        void* p = take(y, LK_SCRATCH_BLOCK, 10);
+        CHECK(p && fake::log.size() == 4);
+    }
+    lk_stream_scratch_release(-1, ~0u);  // and the streams that are still there get their own again
+    CHECK(fake::held() == 0);
+    CHECK(take(x, LK_SCRATCH_LINEAR, 1000) != take(y, LK_SCRATCH_LINEAR, 1000) && fake::log.size() == 4);
+}
+
+static void without_an_event_the_shared_buffers_wait_on_the_host() {
+    static ihipStream_t many[LK_SCRATCH_STREAMS + 1];
+    fake::no_events = true;
+    for (auto& s : many) CHECK(take(&s, LK_SCRATCH_LINEAR, 1000));
+    CHECK(fake::log.size() == 1 && fake::log[0] == "synchronize " + std::to_string((size_t)&many[LK_SCRATCH_STREAMS]));
+}
+
+static void threads_hold_what_they_use() {
+    // every thread marks the buffer it got while it holds it; on one stream, on streams of their own and past the bound
+    static ihipStream_t many[LK_SCRATCH_STREAMS + 2];
+    static std::map<void*, int> user;
+    static std::mutex mu;
+    for (int i = 0; i < LK_SCRATCH_STREAMS; ++i) take(&many[i], LK_SCRATCH_LINEAR, 10);
+    std::vector<std::thread> threads;
+    for (int t = 0; t < 8; ++t)
+        threads.emplace_back([t] {
+            for (int i = 0; i < 2000; ++i) {
+                LkScratch s(&many[t % 4 == 3 ? 0 : LK_SCRATCH_STREAMS - 2 + t % 4]);
+                void* p = s.get(LK_SCRATCH_LINEAR, 10 + (size_t)(i % 500) * 7);
+                CHECK(p);
+                { std::lock_guard<std::mutex> lock(mu); CHECK(user[p]++ == 0); }
+                { std::lock_guard<std::mutex> lock(mu); --user[p]; }
+                if (t == 0 && i % 97 == 0) {
+                    LkScratch other(&many[1]);
+                    (void)other;
+                }
+                if (t == 5 && i % 301 == 300) break;
+            }
+            if (t == 5)
+                for (int i = 0; i < 50; ++i) lk_stream_scratch_release(-1, i % 2 ? LK_SCRATCH_OF_LINEARS : LK_SCRATCH_OF_LAUNCHERS);
+        });
+    for (auto& t : threads) t.join();
+    lk_stream_scratch_release(-1, ~0u);
+    CHECK(fake::held() == 0);
+}
+
 int main(int argc, char** argv) {
     const struct { const char* name; void (*run)(); } cases[] = {
 #define CASE(f) {#f, f}
         CASE(a_stream_keeps_its_buffers), CASE(nothing_is_shared_with_a_graph),
         CASE(what_nothing_reserved_is_refused_while_recording), CASE(graphs_together_stay_within_their_bound),
-        CASE(a_release_frees_its_own_part),
+        CASE(a_release_frees_its_own_part), CASE(streams_past_the_bound_share_in_order),
+        CASE(without_an_event_the_shared_buffers_wait_on_the_host), CASE(threads_hold_what_they_use),
     };
     for (auto& c : cases) {
         if (argc < 2) puts(c.name);
