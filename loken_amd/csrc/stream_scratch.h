@@ -41,9 +41,9 @@ class LkScratch {
 
     // `bytes` for `use`, 256-byte aligned, not initialised; null when there is no memory. While the stream records a
     // graph, also null where no call of the device outside a capture has needed that much (the program warms up
-    // before it records, on any stream), and past LK_SCRATCH_GRAPH_BYTES. Outgrown buffers stay, for kernels and graphs
-    // that hold their addresses, until the release; a buffer that grows does by a quarter at least, so they add up to a
-    // few times the largest.
+    // before it records, on any stream), and past LK_SCRATCH_GRAPH_BYTES. A buffer grows by a quarter more than asked;
+    // the one it replaces is freed first, which waits for the device (so a launcher queues what reads a buffer before it
+    // asks for more of the same use), or kept until the release where a graph's nodes hold its address.
     void* get(LkScratchUse use, size_t bytes);
 
   private:

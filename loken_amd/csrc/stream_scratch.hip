@@ -68,7 +68,7 @@ struct LkScratchPool {
     bool retired = false;   // out of the table: the stream's next call gets another one
     // written under mu and g_mu, so either is enough to read
     Block now[LK_SCRATCH_USES];
-    std::vector<Block> kept;   // outgrown
+    std::vector<Block> kept;   // outgrown and not freed
     // of a shared pool, under mu: how many of the thread's launchers hold it, whether they took a buffer, and the
     // last kernels of those before them
     int held = 0;
@@ -132,17 +132,20 @@ bool graph_may_hold(int device, LkScratchUse use, size_t bytes, size_t want) {
     return reserved && want <= LK_SCRATCH_GRAPH_BYTES && held <= LK_SCRATCH_GRAPH_BYTES - want;
 }
 
-void* allocate(size_t bytes) {
-    // An allocation is no operation of a stream and no part of a graph; in the relaxed mode it is allowed whatever
-    // streams are recording, this one or another thread's.
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool switched = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    void* fresh = nullptr;
-    if (hipMalloc(&fresh, bytes) != hipSuccess) fresh = nullptr;
-    if (switched) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    (void)hipGetLastError();
-    return fresh;
-}
+// Allocating and freeing are no operations of a stream and no part of a graph; in the relaxed mode they are allowed
+// whatever streams are recording, this one or another thread's.
+class RelaxedCapture {
+  public:
+    RelaxedCapture() : switched_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {}
+    ~RelaxedCapture() {
+        if (switched_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+        (void)hipGetLastError();
+    }
+
+  private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    const bool switched_;
+};
 
 }  // namespace
 
@@ -179,10 +182,18 @@ void* LkScratch::get(LkScratchUse use, size_t bytes) {
     if (own.ptr && own.size >= bytes) return own.ptr;
     const size_t want = ((use == LK_SCRATCH_FIXUP ? bytes : bytes + bytes / 4) + 255) & ~(size_t)255;   // (fixup: one size)
     if (pool.owner.recording && !graph_may_hold(pool.owner.device, use, bytes, want)) return nullptr;
-    void* fresh = allocate(want);
-    if (!fresh) return nullptr;
+    RelaxedCapture relaxed;
+    if (own.ptr) {
+        // Outgrown. Kernels of this stream that still use it are waited for by hipFree; a graph's nodes keep theirs.
+        Block outgrown = own;
+        const bool freed = !pool.owner.recording && hipFree(outgrown.ptr) == hipSuccess;
+        std::lock_guard<std::mutex> lock(g_mu);
+        own = Block{};
+        if (!freed) pool.kept.push_back(outgrown);
+    }
+    void* fresh = nullptr;
+    if (hipMalloc(&fresh, want) != hipSuccess) return nullptr;
     std::lock_guard<std::mutex> lock(g_mu);
-    if (own.ptr) pool.kept.push_back(own);
     own = Block{fresh, want, use};
     return fresh;
 }
