@@ -272,6 +272,19 @@ def gemv_4096(args, dev):
 
 
 # ---------------------------------------------------------------------------- mmq
+def tile_kernel(wtype, n, m):
+    """Kernel, peak and operand type of a dense tiled call (launch_dense, mmq.hip). The K-quants of four to six bits form
+    their exact integer dots on the f16 matrix unit above 32 rows (scale folded into the weight operand), so that unit's
+    dense peak prices them; the int8 fraction is kept beside it because the target is quoted on the int8 peak."""
+    if wtype in (Q4K, lib.TYPE_Q5_K, Q6K) and m > 32 and n >= 2048:
+        pad128, pad64 = -(-m // 128) * 128, -(-m // 64) * 64
+        wide = wtype == Q4K and m > 128 and 10 * pad128 <= 11 * pad64 and 2 * -(-n // 256) * (pad128 // 128) > 256
+        kernel = ("q4k_wide_dense_kernel (+ q4k_tokens_f16_kernel once per call)" if wide
+                  else f"f16_dense_kernel, {NAMES[wtype]} (f16_dense_split_kernel where K is cut)")
+        return kernel, F16_PEAK_TFLOPS, "f16 operands (exact integers), f32 accumulate"
+    return f"mmq_dense_kernel, {NAMES[wtype]} tile policy (mmq_dense_split_kernel where K is cut)", INT8_PEAK_TOPS, "int8"
+
+
 def mmq(args, dev):
     L = lib.load()
     wtype, m, k, n = {"2a": (Q4K, 512, 4096, 14336), "2b": (Q6K, 2048, 14336, 4096)}[args.shape]
@@ -306,16 +319,7 @@ def mmq(args, dev):
     tops = lambda us: op_count / us / 1e6
     med = float(np.median(both))
     kern = float(np.median(mm))
-    # Q4_K above 64 rows forms its exact integer dots on the f16 matrix unit (scale folded into
-    # the weight operand), so that unit's dense peak prices it; the int8 fraction is kept beside
-    # it because the target is quoted on the int8 peak.
-    if wtype == Q4K:
-        kernel = "q4k_wide_dense_kernel (+ q4k_tokens_f16_kernel once per call)" if m > 128 else "q4k_f16_dense_kernel"
-        peak, dtype = F16_PEAK_TFLOPS, "f16 operands (exact integers), f32 accumulate"
-    elif wtype == Q6K:
-        kernel, peak, dtype = "mmq_dense_kernel<MmqQ6K,128,1>", INT8_PEAK_TOPS, "int8"
-    else:
-        kernel, peak, dtype = f"mmq_dense_kernel<{NAMES[wtype]} tile policy,128,1>", INT8_PEAK_TOPS, "int8"
+    kernel, peak, dtype = tile_kernel(wtype, n, m)
     roofline = {"bound": "mfma", "achieved": round(tops(kern), 1), "peak": peak, "unit": "TOP/s",
                 "frac": round(tops(kern) / peak, 4), "frac_of_int8_peak": round(tops(kern) / INT8_PEAK_TOPS, 4),
                 "traffic": None, "kernel": kernel, "avg_launch_us": round(float(mm.mean()), 3),
@@ -751,7 +755,7 @@ def brief_mmq(shape, launches=200):
     mm, both = float(np.median(mm_all)), float(np.median(both_all))
     op_count = 2.0 * m * k * n
     return {"workload": f"tiled matmul {m} rows x {k} -> {n}, {NAMES[wtype]}", "ops": int(op_count),
-            "kernel": "q4k_wide_dense_kernel after q4k_tokens_f16_kernel (exact integers on f16 operands)" if wtype == Q4K else "mmq_dense_kernel<MmqQ6K,128,1>",
+            "kernel": tile_kernel(wtype, n, m)[0],
             "matmul_us": round(mm, 2), "tops": round(op_count / mm / 1e6, 1), "matmul_launch": spread(mm_all),
             "call_two_launches": spread(both_all),
             "frac_of_int8_peak": round(op_count / mm / 1e6 / INT8_PEAK_TOPS, 4),
