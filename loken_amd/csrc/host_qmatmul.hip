@@ -84,8 +84,12 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     // Above 16 rows of 8192 values or more: Q4_K / Q5_K 4096 x 14336 at 20 rows 37 / 39 us against 27 / 28, 1024 x 14336 at
     // 17 / 32 35 / 39 against 20 / 22, 2048 x 8192 23 / 25 against 18 / 19; above 32 rows, where the tiles are 256 rows
     // high and K is cut further, from 12288 values (2048 x 14336 at 40 / 109 rows 40 / 43 against 28 / 33; 3072 x 11008
-    // 33 / 46 against 40 / 51). Q6_K keeps its sets of eight rows up to 32 (2048 x 8192 17 against 21) and leaves above
-    // (2048 x 14336 at 40 / 109 rows 50 / 53 against 31 / 38, 4096 x 8192 34 / 58 against 29 / 37).
+    // 33 / 46 against 40 / 51). Q6_K leaves above 32 rows (2048 x 14336 at 40 / 109 rows 50 / 53 against 31 / 38,
+    // 4096 x 8192 34 / 58 against 29 / 37); up to 32 its sets of eight rows are ahead at 1024 matrix rows and level at 2048
+    // (six matrices in turn in a graph, at 17 / 32 rows: 1024 x 8192 15.8 / 16.0 against 19.8 / 21.6, 1024 x 14336 19.7 / 20.5
+    // against 23.7 / 25.6, 2048 x 8192 22.1 / 18.8 against 21.4 / 22.8, 2048 x 14336 28.2 / 28.2 against 27.6 / 29.1), behind from
+    // 3072 on, which the line does not follow yet (3072 x 12288 34.5 / 34.6 against 28.8 / 30.7, 4096 x 8192 27.0 / 27.3 against
+    // 24.9 / 26.0, 8192 x 8192 33.4 / 38.0 against 32.1 / 35.2, 4096 x 14336 at 17 / 28 44.2 / 44.3 against 33.2 / 35.9).
     if (rows > 16 && n >= 1024 && (dtype == LK_TYPE_Q6_K ? rows > 32 && k >= 8192 : k >= (rows > 32 ? 12288 : 8192))) return false;
     return rows <= 16 || (long long)n * rows * (k > 4096 ? k : 4096) <= 450000ll * 4096 * few;
 }
