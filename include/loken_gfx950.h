@@ -595,9 +595,10 @@ int loken_moe_gemm_gguf_down_reduce_static(const float* inputs, const void* weig
 /* A mixture layer's expert block in one call: out[t] = sum over the token's choices j of topk_weights[t, j] *
  * down_e (silu(gate_e . x[t]) * (up_e . x[t])), e = choices[t, j]; f32 rows x [tokens, hidden] and out [tokens,
  * hidden], stacks gate / up [experts, ffn, hidden] of wtype_gu and down [experts, hidden, ffn] of wtype_down, choices
- * int32 and weights f32 [tokens, topk]. A choice outside [0, n_experts) adds nothing, whatever its weight. The launches are those of the entry points above, chosen by size as the layer
- * code of the reference chooses (src/inference/generic_transformer/moe_weights.rs:2118-2152). LK_ERR_TYPE: a format
- * the path does not take; LK_ERR_NOMEM: no scratch (while recording: none of that size outside a capture before). */
+ * int32 and weights f32 [tokens, topk]. A choice outside [0, n_experts) adds nothing, whatever its weight. The
+ * launches are those of the entry points above, chosen by size as the layer code of the reference chooses
+ * (src/inference/generic_transformer/moe_weights.rs:2118-2152). LK_ERR_TYPE: a format the path does not take;
+ * LK_ERR_NOMEM: no scratch (while recording: none of that size outside a capture before). */
 int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
                    const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
                    int hidden, int ffn, void* stream);
@@ -727,9 +728,10 @@ int loken_moe_q4k_imma_m8_down(const void* weights, const void* q8_1, const int3
  * launched outside that (the caller falls back). */
 void loken_topk_softmax(const float* logits, float* weights, uint32_t* ids, int n_rows, int n_experts,
                         int n_expert_used, int with_norm, void* stream);
-/* Gate mat-vec + softmax + top-k of each token in one launch: logits = gate_w [n_experts, hidden]
- * f32 . x [n_rows, hidden] f32, then the selection of loken_topk_softmax. A token has a workgroup
- * of 16 waves whose lanes walk each weight row together, so a logit is a 64-lane f32 sum (the
+/* Gate product + softmax + top-k of each token: logits = gate_w [n_experts, hidden] f32 .
+ * x [n_rows, hidden] f32, then the selection of loken_topk_softmax. Two launches, the logits as an f32
+ * product on the matrix unit with K split over the chip; one launch, a workgroup per token, where rows do
+ * not start on 16 bytes or a recording stream has no scratch. A logit is an f32 sum of partial sums (the
  * reference's is one lane's serial sum: same value up to summation order). Name and arguments of
  * the reference's launcher (cuda/moe/gate_topk.cu:366-403; called from
  * src/inference/moe_cuda/dense/gate.rs:51). hidden up to 8192, up to 512 experts (the reference:

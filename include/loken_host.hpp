@@ -34,8 +34,9 @@ enum class Path : int {
  * of the matrix-unit rows kernels from 3 f32 rows on (Q4_K / Q5_K: n x rows of 57344, or 8192 at
  * k <= 2048; Q6_K: n x k of 48 Mi with k a multiple of 2048); then the matrix-unit rows kernels up to
  * 16 rows, or while n x rows x max(k, 4096) / 4096 <= 450 000 (twice that for a matrix of 1024 rows, and so
- * on: few rows yield few tiles; Q4_K / Q5_K rows of 8192 values or more leave them from 9 rows; below that even a tiled launch with K cut
- * into ranges does not beat them), then the tiled matmul; Q8_0 mat-vec slices up to 16 rows, then the
+ * on: few rows yield few tiles; Q4_K / Q5_K rows of 8192 values or more over 2048 matrix rows leave them from
+ * 9 rows; above 16 rows a matrix of 1024 rows or more leaves them where its rows have 8192 values, Q4_K / Q5_K
+ * above 32 rows 12288, Q6_K only above 32), then the tiled matmul; Q8_0 mat-vec slices up to 16 rows, then the
  * tiled matmul; the 32-value nibble formats, Q3_K and Q2_K mat-vec slices up to 15 rows, or 8 over a
  * matrix of 48 Mi weights or more, then the tiled matmul). */
 int matvec_rows(int dtype, int k);
@@ -46,9 +47,8 @@ public:
      * Q6_K / Q8_0), owned by the caller, on device `device`. */
     QKernelMatMul(int dtype, int n, int k, const void* blob, int device);
 
-    /* x [rows, k] (LK_TYPE_F32, F16 or BF16) -> out [rows, n] in x's type, on `stream`. The
-     * matrix-unit kernels write f32 rows; for f16 / bf16 rows they write into a buffer of the stream's
-     * scratch and one more launch rounds them into `out` (the reference narrows the f32 rows its
+    /* x [rows, k] (LK_TYPE_F32, F16 or BF16) -> out [rows, n] in x's type, on `stream`: every kernel
+     * stores that type itself, its f32 sums rounded to nearest (the reference narrows the f32 rows its
      * mmq_forward returns the same way, kernel_matmul.rs:1086-1714). `decode_order` keeps every row on the mat-vec
      * kernels whatever the count (DecodeOrder of the reference, kernel_matmul.rs:34-75).
      * Returns LK_OK or an LK_ERR_* code; never throws, never aborts. */

@@ -253,7 +253,6 @@ struct LkDevice {
 };
 const LkDevice& lk_device();
 
-// Q4_K x up to any number of Q8_1 rows on the matrix unit (rows_mfma.hip); LK_* status.
 // A matrix-unit kernel's f32 result as element `at` of a destination of `type` (f32, or f16 / bf16 rounded to nearest: the
 // conversion the reference applies to the f32 rows mmq_forward returns, src/tensor/quantized/kernel_matmul.rs:1086-1714).
 // The type is uniform over the launch. A second launch over f32 rows took 4 to 5 us a call.
@@ -268,6 +267,7 @@ static __device__ __forceinline__ void lk_store_as(float* dst, size_t at, float 
 int lk_rows_linear(int wtype, const void* w, const void* q8_1, void* out, int out_type, int rows, int n, int k, hipStream_t stream);
 int lk_mmq_linear(int wtype, void* fixup, const void* w, const void* y, void* out, int out_type, int k, int n, int rows, int64_t row_blocks,
                   hipStream_t stream);
+// Q4_K / Q6_K x any number of Q8_1 rows on the matrix unit (rows_mfma.hip, rows_mfma_q6k.hip); LK_* status.
 int lk_q4k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y,
                      int ldd, hipStream_t stream);
 int lk_q6k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y,

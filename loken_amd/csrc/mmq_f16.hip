@@ -1,4 +1,4 @@
-// Q4_K, Q5_K and Q6_K weight rows against 33 or more Q8_1 token rows (65 or more where they are an expert's run): the
+// Q4_K, Q5_K and Q6_K weight rows against 33 or more Q8_1 token rows, a dense call's or those expected of an expert: the
 // sub-block dots on the f16 matrix unit.
 //
 //   out[token, n] = sum over 256-value blocks of

@@ -387,7 +387,7 @@ def _router_out(tokens: int, topk: int, device):
 
 
 def gate_topk_softmax(x: torch.Tensor, gate_w: torch.Tensor, topk: int, renorm: bool = True):
-    """Gate mat-vec + softmax + top-k in one launch: ``x [tokens, hidden]`` f32, ``gate_w [experts,
+    """Gate product + softmax + top-k in one call: ``x [tokens, hidden]`` f32, ``gate_w [experts,
     hidden]`` f32 -> (weights, choices) as ``topk_softmax`` (gate_topk_softmax,
     src/inference/moe_cuda/dense/gate.rs:20-75)."""
     tokens, hidden = x.shape
