@@ -57,13 +57,12 @@ static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], floa
         best = wave_max(best);
         // Logits that are not numbers (and infinite ones, whose difference to the maximum is none) leave fewer
         // probabilities than choices: `best` is then -1 or not a number itself, and the choice names no expert.
+        const float wanted = best >= 0.f ? best : NAN;   // equal to nothing
         int e = 0x7FFFFFFF;
-        if (best >= 0.f) {
 #pragma unroll
-            for (int i = PER - 1; i >= 0; --i) {
-                const unsigned long long at = __ballot(p[i] == best);
-                if (at) e = 64 * i + __ffsll((long long)at) - 1;
-            }
+        for (int i = PER - 1; i >= 0; --i) {
+            const unsigned long long at = __ballot(p[i] == wanted);
+            if (at) e = 64 * i + __ffsll((long long)at) - 1;
         }
         const float prob = best / sum;
         picked_sum += prob;
