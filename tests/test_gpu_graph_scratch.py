@@ -1,5 +1,7 @@
 """Calls that work in the library's scratch memory, recorded into graphs: replays beside calls and other graphs on
 streams that nothing orders against them, every one the eager bits."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -86,6 +88,24 @@ def test_linear(wtype, n, k, rows, half):
         check_replays([call(seed) for seed in (75, 76, 77)], torch.cuda.Stream())
     finally:
         lin.close()
+
+
+def test_every_capture_has_an_id_of_its_own():
+    """What the library tells one recording from the next by, on one stream and on another."""
+    hip = C.CDLL("libamdhip64.so")
+    x, sides, ids = torch.zeros(8, device="cuda"), [torch.cuda.Stream(), torch.cuda.Stream()], []
+
+    def body(stream):
+        x.add_(1.0)
+        for s in (stream, torch.cuda.default_stream()):
+            status, at = C.c_int(-1), C.c_ulonglong(0)
+            assert hip.hipStreamGetCaptureInfo(C.c_void_p(s.cuda_stream), C.byref(status), C.byref(at)) == 0
+            assert status.value == (1 if s is stream else 0)
+            if s is stream:
+                ids.append(at.value)
+
+    keep = [record(lambda: body(side), side) for side in sides + sides]
+    assert len(keep) == len(set(ids)) == 4
 
 
 def test_scratch_that_grows_after_a_recording():
