@@ -262,7 +262,8 @@ typedef struct {
     int workers;                 /* threads beside the caller */
     atomic_uint generation;      /* bumped once per job */
     atomic_size_t next, done;    /* next chunk to grab; chunks finished */
-    atomic_int active;           /* workers inside pool_drain: a job's state is not reused while one is */
+    atomic_int open;             /* a job's state is whole and its chunks may be grabbed */
+    atomic_int active;           /* workers that may be looking at a job: its state is not reused while one is */
     size_t n_chunks;
     chunk_fn fn;
     void* ctx;
@@ -303,12 +304,14 @@ static void* pool_worker(void* arg) {
             pthread_mutex_unlock(&p->mu);
         }
         if (atomic_load(&p->stop)) return NULL;
-        /* Entering is announced BEFORE the generation is read: pool_run bumps the generation and then
-         * waits for `active` to fall to zero, so either it sees this worker and waits for it, or this
-         * worker sees the new generation's state whole. */
+        /* Entering is announced BEFORE `open` is read, and pool_run closes a job BEFORE it waits for
+         * `active` to fall to zero: either it sees this worker and waits for it, or this worker, woken too
+         * late for its job, finds it closed and touches nothing. (A worker that could still grab from the
+         * counter of a finished job took a chunk of the next one between the resets of `next` and `done`:
+         * its finish was lost, and the caller waited for it for ever.) */
         atomic_fetch_add(&p->active, 1);
         seen = atomic_load(&p->generation);
-        pool_drain(p);
+        if (atomic_load(&p->open)) pool_drain(p);
         atomic_fetch_sub(&p->active, 1);
     }
 }
@@ -383,7 +386,8 @@ static void pool_run(size_t n_chunks, chunk_fn fn, void* ctx) {
     p->n_chunks = n_chunks;
     atomic_store(&p->next, 0);
     atomic_store(&p->done, 0);
-    atomic_fetch_add_explicit(&p->generation, 1, memory_order_release);
+    atomic_store(&p->open, 1);
+    atomic_fetch_add(&p->generation, 1);
     if (atomic_load(&p->sleepers) > 0) {
         pthread_mutex_lock(&p->mu);
         pthread_cond_broadcast(&p->wake);
@@ -391,10 +395,9 @@ static void pool_run(size_t n_chunks, chunk_fn fn, void* ctx) {
     }
     pool_drain(p);
     while (atomic_load_explicit(&p->done, memory_order_acquire) < n_chunks) _mm_pause();
-    /* A worker that woke late may still be inside pool_drain (its grab found no chunk left, or it is
-     * about to look): the next job's fn / ctx / counters are written only once nobody is in there,
-     * so a stale grab can never be compared against the next job's chunk count. */
-    while (atomic_load_explicit(&p->active, memory_order_acquire) != 0) _mm_pause();
+    /* the next job's fn / ctx / counters are written once nobody is in there any more */
+    atomic_store(&p->open, 0);
+    while (atomic_load(&p->active) != 0) _mm_pause();
 }
 
 /* ---------------------------------------------------------------------------------------------

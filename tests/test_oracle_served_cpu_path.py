@@ -8,6 +8,10 @@ columns, persistent worker pool) against the scalar oracle it is a faster statem
     1e-3 * max(|ref|, 1) (avx/parity.rs:50-56), for one row and for several;
   * the pool gives the same bits whatever its size (every output is one thread's own sum).
 """
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -231,3 +235,26 @@ def test_pooled_expert_block_is_the_scalar_block_token_by_token():
         want = oracle.moe_forward(family, Q4K, Q6K, x, gate, up, down, ids, weights, n_experts, ffn)
         got = oracle.moe_forward_pool(family, Q4K, Q6K, x, gate, up, down, ids, weights, n_experts, ffn)
         assert np.array_equal(got, want)
+
+
+def test_pool_outlives_many_short_jobs_with_more_workers_than_cores():
+    """Two jobs a call, shorter than a worker takes to wake: workers arrive when theirs is over and the next one is
+    being set up. In a process of its own, so that a pool that stops answering ends the test and not the run."""
+    body = """
+import os, time
+import numpy as np, oracle
+from loken_amd import synth
+w, x = synth.weight(oracle.Q4_K, 64, 256, seed=1), synth.activation(24, 256, seed=1)
+x8 = oracle.repack_q4k_x8(w, 64, 256)
+oracle.pool_start(min(64, 2 * len(os.sched_getaffinity(0)) + 4))
+want = oracle.oa_matmul_q4k_x8_tiled(x, x8, 64)
+end = time.time() + 4
+while time.time() < end:
+    for _ in range(200):
+        got = oracle.oa_matmul_q4k_x8_tiled(x, x8, 64)
+    assert np.array_equal(got, want)
+    time.sleep(0.001)   # the workers go to sleep now and then
+oracle.pool_start(1)
+"""
+    root = Path(__file__).resolve().parent.parent
+    subprocess.run([sys.executable, "-c", body], cwd=root, check=True, timeout=60)
