@@ -1013,30 +1013,14 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
     // (Q2_K stays on 64-token tiles: with the rank-16 minimum its 128-token tile spills and runs 512 x
     // 4096 -> 14336 in 344 us against 240, 2048 x 14336 -> 4096 in 1155 against 742; every other format
     // is 3 to 40 % faster on the wide tile)
-    // (Q4_K, Q5_K and Q6_K from 33 rows of a matrix of 2048 rows or more go on to the 64-token f16 tiles, quantizer
-    // included against the int8 tiles: Q4_K 14336 x 4096 at 64 rows 40.5 us against 46.4, 4096 x 14336 43.8 against
-    // 49.1, 4096 x 4096 the same 33; Q5_K 14336 x 4096 at 64 / 512 / 2048 rows 33 / 138 / 495 against 36 / 169 / 631,
-    // 4096 x 4096 at 77 / 512 26 / 50 against 28 / 59; Q6_K 14336 x 4096 38 / 171 / 609 against 40 / 187 / 703,
-    // 4096 x 14336 at 2048 576 against 654, 4096 x 4096 at 64 / 512 28 / 59 against 26 / 66)
-    const bool f16_from_33 = F::F16_TYPE >= 0 && nrows_x >= 2048 && !lk_env_flag("LK_MMQ_I8");
-    if ((ncols_y <= 64 && !f16_from_33) || F::MIN_RANK == 16) return launch_dense_tm<F, 64, 2>(pb, s, fixup);
-    if constexpr (F::F16_TYPE >= 0) {   // Q4_K, Q5_K, Q6_K: scales folded into f16 operands
-        // (under 2048 weight rows the 256-row f16 tiles are too few even with K cut: 1024 x 4096 at 512 / 1024 /
-        // 2048 rows 48 / 63 / 93 us against 38 / 49 / 73 on the int8 tiles)
-        if (!lk_env_flag("LK_MMQ_I8") && nrows_x >= 2048) {
-            // 128-token tiles with the token side expanded once per call, where they pad the rows at most a
-            // tenth more than the 64-token tiles would (512 x 4096 -> 14336: 105 us against 123) and are
-            // enough to occupy half the CUs (fewer: the 64-token tiles, which can cut K)
-            const int64_t pad128 = (ncols_y + 127) / 128 * 128, pad64 = (ncols_y + 63) / 64 * 64;
-            const int64_t wide_tiles = (nrows_x + 255) / 256 * (pad128 / 128);
-            if (F::F16_TYPE == LK_TYPE_Q4_K && ncols_y > 128 && 10 * pad128 <= 11 * pad64 && 2 * wide_tiles > lk_device().cus && !lk_env_flag("LK_MMQ_NO_WIDE")) {
-                const int tm = lk_mmq_q4k_wide_dense(pb, s);
-                if (tm >= 0) return tm;
-            }
-            const int tm = lk_mmq_f16_dense(F::F16_TYPE, pb, s, fixup);
+    // (Q4_K, Q5_K and Q6_K from 33 rows of a matrix of 2048 rows or more: the f16 tiles)
+    const bool f16 = F::F16_TYPE >= 0 && nrows_x >= 2048 && !lk_env_flag("LK_MMQ_I8");
+    if ((ncols_y <= 64 && !f16) || F::MIN_RANK == 16) return launch_dense_tm<F, 64, 2>(pb, s, fixup);
+    if constexpr (F::F16_TYPE >= 0)
+        if (f16) {
+            const int tm = lk_mmq_tiles_dense(F::F16_TYPE, pb, s, fixup);
             if (tm >= 0) return tm;
         }
-    }
     // 128-token tiles where there are F::WIDE_FROM of them or more, else 64-token tiles, twice as many and
     // with K cut where those are still few. Quantizer + matmul, 64- against 128-token tiles:
     //   Q6_K  4096 x 14336 at 128 / 512 / 1024 rows (32 / 128 / 256 tiles) 70 / 215 / 393 us against 99 / 307 /

@@ -551,42 +551,6 @@ static __device__ __forceinline__ void f16_tile(const MmqProblem& pb, int n0, in
     else f16_tile_of<F, 2>(pb, n0, m0, lds);
 }
 
-// Workgroup id -> (n tile, m tile): the m tiles of one n tile re-read the same weight rows, so
-// they are issued back to back on one XCD (ids are dealt round robin over the 8 XCDs).
-template <class F>
-__global__ __launch_bounds__(Wide::THREADS, 1) void f16_dense_kernel(MmqProblem pb, int n_tiles, int m_tiles) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int id = blockIdx.x;
-    const int xcd = id & 7, seq = id >> 3;
-    const int m_tile = seq % m_tiles;
-    const int n_tile = (seq / m_tiles) * 8 + xcd;
-    if (n_tile >= n_tiles) return;
-    f16_tile<F>(pb, n_tile * Wide::TN, pb.m_begin + m_tile * Wide::TM, lds);
-}
-
-// The same tiles over one of `splits` ranges of K each, the partial tile to part[range].
-template <class F>
-__global__ __launch_bounds__(Wide::THREADS, 1) void f16_dense_split_kernel(MmqProblem pb, int n_tiles, int m_tiles,
-                                                                          int splits, float* part, int64_t part_stride) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int id = blockIdx.x;
-    const int xcd = id & 7;
-    int seq = id >> 3;
-    const int m_tile = seq % m_tiles;
-    seq /= m_tiles;
-    const int split = seq % splits;
-    const int n_tile = (seq / splits) * 8 + xcd;
-    if (n_tile >= n_tiles) return;
-    const int64_t kb0 = pb.nb * split / splits, kb1 = pb.nb * (split + 1) / splits;
-    pb.w += kb0 * F::BYTES;
-    pb.y += kb0 * pb.rows_total * MMQ_REC_BYTES;
-    pb.nb = kb1 - kb0;
-    pb.dst = part + split * part_stride;
-    pb.ldd = mmq_part_stride(pb);
-    pb.out_type = LK_TYPE_F32;
-    f16_tile<F>(pb, n_tile * Wide::TN, pb.m_begin + m_tile * Wide::TM, lds);
-}
-
 // Expert-batched: expert e's slab against the sorted rows [bounds[e], bounds[e+1]); grid: mmq_moe_grid.
 template <class F>
 __global__ __launch_bounds__(Wide::THREADS, 1) void f16_moe_kernel(MmqProblem pb, const uint8_t* w_second, int64_t dst_second,
@@ -615,27 +579,6 @@ static bool f16_suits(const MmqProblem& pb) {
 }
 
 template <class F>
-static int f16_dense(const MmqProblem& pb, hipStream_t s, void* fixup) {
-    using C = Wide;
-    constexpr int LDS = f16_lds_bytes<F>();
-    static_assert(LDS <= 160 * 1024, "LDS of one CU");
-    if (!f16_suits<F>(pb)) return -1;
-    const int n_tiles = (pb.n + C::TN - 1) / C::TN;
-    const int m_tiles = (pb.m_end - pb.m_begin + C::TM - 1) / C::TM;
-    const int splits = mmq_splits(pb, (int64_t)n_tiles * m_tiles, lk_device().cus, fixup, true);   // one workgroup a CU
-    if (splits > 1) {
-        if (mmq_prepare_kernel(f16_dense_split_kernel<F>, LDS) != LK_OK) return 0;
-        hipLaunchKernelGGL(f16_dense_split_kernel<F>, dim3((n_tiles + 7) / 8 * 8 * m_tiles * splits), dim3(C::THREADS), LDS,
-                           s, pb, n_tiles, m_tiles, splits, (float*)fixup, pb.m_end * mmq_part_stride(pb));
-        return lk_mmq_split_sum((const float*)fixup, splits, pb, s) == LK_OK ? C::TM : 0;
-    }
-    if (mmq_prepare_kernel(f16_dense_kernel<F>, LDS) != LK_OK) return 0;
-    const int grid = (n_tiles + 7) / 8 * 8 * m_tiles;
-    hipLaunchKernelGGL(f16_dense_kernel<F>, dim3(grid), dim3(C::THREADS), LDS, s, pb, n_tiles, m_tiles);
-    return hipGetLastError() == hipSuccess ? C::TM : 0;
-}
-
-template <class F>
 static int f16_moe(const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
                    int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s) {
     using C = Wide;
@@ -649,13 +592,6 @@ static int f16_moe(const MmqProblem& pb, const uint8_t* w_second, int64_t dst_se
 }
 
 }  // namespace
-
-int lk_mmq_f16_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
-    return wtype == LK_TYPE_Q4_K   ? f16_dense<F16Q4K>(pb, s, fixup)
-           : wtype == LK_TYPE_Q5_K ? f16_dense<F16Q5K>(pb, s, fixup)
-           : wtype == LK_TYPE_Q6_K ? f16_dense<F16Q6K>(pb, s, fixup)
-                                   : -1;
-}
 
 int lk_mmq_f16_moe(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
                    int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s) {

@@ -110,10 +110,19 @@ static inline MmqMoeGrid mmq_moe_grid(const MmqProblem& pb, int tn, int tm, int 
     return {dim3((unsigned)(n_tiles * group), (unsigned)(stacks * n_experts), (unsigned)((col_tiles + group - 1) / group)), (int)group};
 }
 
-// Q4_K, Q5_K or Q6_K (`wtype`) against 33 or more token rows (mmq_f16.hip); `fixup`: the caller's tmp_fixup or null. Return the token-tile width launched,
-// 0 when the launch failed, -1 when the operands do not suit these kernels (alignment, 32-bit offsets) and the caller should take the int8 tiles.
-int lk_mmq_f16_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup);
-// Q4_K against 129 or more token rows on the f16 tiles with four token tiles per wave (mmq_q4k_wide.hip); same returns.
-int lk_mmq_q4k_wide_dense(const MmqProblem& pb, hipStream_t s);
+// Q4_K, Q5_K and Q6_K on the f16 tiles of mmq_tile.h. tt: token tiles of 32 a wave takes; waves: 4 (two workgroups a CU) or
+// 8 (tt = 4, one); splits: ranges of K, partial products as above.
+struct MmqTilePlan {
+    int tt, waves, splits;
+};
+struct LkTokenOperands;
+int lk_tile_dense_q4k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
+int lk_tile_dense_q5k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
+int lk_tile_dense_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
+// A dense product on them (mmq_tiles.hip), operands made from the workspace records; `fixup`: the caller's tmp_fixup or null.
+// Returns the token-tile width launched, 0 when the launch failed, -1 when the operands do not suit these kernels (alignment,
+// 32-bit offsets, no scratch) and the caller should take the int8 tiles.
+int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup);
+// The expert-batched product (mmq_f16.hip), same returns.
 int lk_mmq_f16_moe(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
                    int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);

@@ -1,0 +1,4 @@
+// The f16 tiles of one weight format (see mmq_tile.h).
+#include "mmq_tile.h"
+
+LK_DEFINE_TILES(q5k, mmq_tile::TileQ5K)

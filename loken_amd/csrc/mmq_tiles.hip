@@ -1,0 +1,104 @@
+// Dense products of Q4_K, Q5_K and Q6_K weights on the f16 tiles (mmq_tile.h): which tile a call takes, and the token operands.
+
+#include "mmq_operands.h"
+#include "mmq_problem.h"
+#include "stream_scratch.h"
+
+#include <algorithm>
+
+namespace {
+
+// Workspace records -> operands. grid (blocks, rows / 32), 256 threads: eight threads a row, a sub-block each.
+__global__ __launch_bounds__(256) void operands_from_records_kernel(const uint8_t* __restrict__ y, LkTokenOperands ops, int64_t rec_rows,
+                                                                    int row0, int rows) {
+    const int kb = blockIdx.x, s = threadIdx.x & 7;
+    const int r = blockIdx.y * 32 + (threadIdx.x >> 3);
+    if (r >= rows) return;
+    const uint8_t* rec = y + ((int64_t)kb * rec_rows + row0 + r) * MMQ_REC_BYTES;
+    uint8_t* to = ops.codes + ((int64_t)kb * ops.rows + r) * LK_OPERAND_CODES + 64 * s;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint4 c = *(const uint4*)(rec + 32 * s + 16 * h);
+        uint4 lo, hi;
+        operand_codes(c.x, lo.x, lo.y);
+        operand_codes(c.y, lo.z, lo.w);
+        operand_codes(c.z, hi.x, hi.y);
+        operand_codes(c.w, hi.z, hi.w);
+        *(uint4*)(to + 16 * h) = lo;
+        *(uint4*)(to + 32 + 16 * h) = hi;
+    }
+    operand_scales(ops.tabs + ((int64_t)kb * ops.rows + r) * LK_OPERAND_TAB, s, f16_bits_to_f32(*(const uint16_t*)(rec + 256 + 2 * s)),
+                   (int)*(const int16_t*)(rec + 272 + 2 * s));
+}
+
+// Nanoseconds an item (32 x 32 x 32 product) takes a SIMD: `full` with two workgroups on every CU, `alone` with one, by token
+// tiles; measured on MI355X, whole launches less the 5 us that starting and ending one takes. wide: eight waves, tt = 4.
+struct ItemTimes {
+    double full[4], alone[4], wide;
+};
+constexpr ItemTimes ONE_TERM = {{115, 98.6, 97, 90.7}, {177, 116, 104, 92}, 88}, TWO_TERMS = {{172, 145, 128.6, 121}, {240, 158, 136, 123}, 0};
+
+// The tile with the shortest estimated launch: rounds of workgroups, and what a cut K costs in partial products (written, read
+// and added at 4 TB/s by a launch of 3 us).
+MmqTilePlan plan_dense(int wtype, const MmqProblem& pb, const void* fixup) {
+    const ItemTimes& t = wtype == LK_TYPE_Q6_K ? TWO_TERMS : ONE_TERM;
+    const int cus = lk_device().cus;
+    MmqTilePlan best{1, 4, 1};
+    double least = 1e30;
+    for (int tt = 1; tt <= 4; ++tt) {
+        const int64_t tiles = ((pb.n + 127ll) / 128) * ((pb.m_end + 32ll * tt - 1) / (32 * tt));
+        const int splits = mmq_splits(pb, tiles, 2 * cus, fixup, true);
+        const int64_t groups = tiles * splits, rounds = groups / (2 * cus), rest = groups % (2 * cus);
+        const double items = 8.0 * tt * ((pb.nb + splits - 1) / splits), one = items * t.alone[tt - 1], two = 2 * items * t.full[tt - 1];
+        double ns = rounds * two;
+        if (rest > 0) ns += rest <= cus ? one : one + (two - one) * (rest - cus) / cus;
+        if (splits > 1) ns += 3000 + (splits + 1.0) * pb.m_end * pb.n * 4 / 4000.0;
+        if (ns < least) least = ns, best = {tt, 4, splits};
+    }
+    if (t.wide > 0) {
+        const int64_t tiles = ((pb.n + 255ll) / 256) * ((pb.m_end + 127ll) / 128);
+        if ((tiles + cus - 1) / cus * 64.0 * pb.nb * t.wide < least) best = {4, 8, 1};
+    }
+    return best;
+}
+
+int launch(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s) {
+    return wtype == LK_TYPE_Q4_K   ? lk_tile_dense_q4k(pb, ops, plan, part, s)
+           : wtype == LK_TYPE_Q5_K ? lk_tile_dense_q5k(pb, ops, plan, part, s)
+                                   : lk_tile_dense_q6k(pb, ops, plan, part, s);
+}
+
+// What the operands of one pass may take; a call with more goes in passes of token rows over the same buffer (stream order
+// keeps them apart).
+constexpr int64_t OPERANDS_CAP = 256ll << 20;
+
+}  // namespace
+
+int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
+    const int bytes = wtype == LK_TYPE_Q4_K ? Q4K_BYTES : wtype == LK_TYPE_Q5_K ? Q5K_BYTES : Q6K_BYTES;
+    const bool q6 = wtype == LK_TYPE_Q6_K;
+    if ((uintptr_t)pb.w % (q6 ? 2 : 16) != 0 || (uintptr_t)pb.y % 16 != 0 || (q6 && pb.n < 128)) return -1;
+    // lane offsets inside a tile are 32-bit
+    if (pb.row_blocks * bytes * 256 > (int64_t)INT32_MAX || pb.m_begin != 0) return -1;
+    const int64_t row_bytes = pb.nb * (LK_OPERAND_CODES + LK_OPERAND_TAB);
+    const int64_t fit = OPERANDS_CAP / row_bytes / 128 * 128 - LK_OPERAND_PAD;
+    if (fit < 128 || pb.nb > INT32_MAX / 2) return -1;
+    const int per_pass = (int)std::min<int64_t>(pb.m_end, fit);
+    LkScratch scratch(s);
+    void* buffer = scratch.get(LK_SCRATCH_TOKENS, lk_operand_bytes(per_pass, pb.nb));
+    if (!buffer) return -1;
+    int width = 0;
+    for (int m0 = 0; m0 < pb.m_end; m0 += per_pass) {
+        MmqProblem pass = pb;
+        pass.m_end = std::min(per_pass, pb.m_end - m0);
+        pass.dst = (float*)((uint8_t*)pb.dst + (int64_t)m0 * pb.ldd * (pb.out_type == LK_TYPE_F32 ? 4 : 2));
+        const LkTokenOperands ops = lk_operands_at(buffer, pass.m_end, pb.nb);
+        const MmqTilePlan plan = plan_dense(wtype, pass, fixup);
+        hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((pass.m_end + 31) / 32)), dim3(256), 0, s, pb.y, ops,
+                           pb.rows_total, m0, pass.m_end);
+        if (launch(wtype, pass, ops, plan, (float*)fixup, s) != LK_OK) return 0;
+        if (plan.splits > 1 && lk_mmq_split_sum((const float*)fixup, plan.splits, pass, s) != LK_OK) return 0;
+        width = std::max(width, 32 * plan.tt);
+    }
+    return width;
+}

@@ -277,10 +277,7 @@ def tile_kernel(wtype, n, m):
     their exact integer dots on the f16 matrix unit above 32 rows (scale folded into the weight operand), so that unit's
     dense peak prices them; the int8 fraction is kept beside it because the target is quoted on the int8 peak."""
     if wtype in (Q4K, lib.TYPE_Q5_K, Q6K) and m > 32 and n >= 2048:
-        pad128, pad64 = -(-m // 128) * 128, -(-m // 64) * 64
-        wide = wtype == Q4K and m > 128 and 10 * pad128 <= 11 * pad64 and 2 * -(-n // 256) * (pad128 // 128) > 256
-        kernel = ("q4k_wide_dense_kernel (+ q4k_tokens_f16_kernel once per call)" if wide
-                  else f"f16_dense_kernel, {NAMES[wtype]} (f16_dense_split_kernel where K is cut)")
+        kernel = f"tile_dense_kernel, {NAMES[wtype]} (+ operands_from_records_kernel once per call, mmq_split_sum_kernel where K is cut)"
         return kernel, F16_PEAK_TFLOPS, "f16 operands (exact integers), f32 accumulate"
     return f"mmq_dense_kernel, {NAMES[wtype]} tile policy (mmq_dense_split_kernel where K is cut)", INT8_PEAK_TOPS, "int8"
 

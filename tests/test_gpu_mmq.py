@@ -282,3 +282,25 @@ def test_full_benchmark_size_against_matvec_and_sampled_oracle(name, m, k, n):
     # 3. size-independent property: permuting token rows permutes output rows, bit for bit
     perm = torch.randperm(m, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
     assert torch.equal(ops.mmq_forward(wtype, wd, xd[perm].contiguous(), n), tiled[perm])
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("m,k,n", [(33, 256, 2048), (64, 512, 2049), (65, 768, 2175), (96, 2048, 2176), (97, 512, 2303), (128, 1280, 2051),
+                                   (129, 256, 4097), (384, 512, 16390), (515, 256, 16384)])
+@pytest.mark.parametrize("fixup", [True, False])
+def test_f16_tiles_at_every_width_and_edge(name, m, k, n, fixup, knobs):
+    # One to four token tiles a wave, four and eight waves; last tiles with one live row or token, one to eight blocks of K
+    # (shorter than the pipeline is deep), whole and cut. The integers are the int8 tiles' and the mat-vec's, so only the
+    # order of f32 sums differs: nb blocks of 8 roundings on each side, 2e-5 of the largest value as elsewhere here.
+    wtype = DT[name]
+    w = dev(synth.weight(wtype, n, k, seed=51, stream=10))
+    x = dev(synth.activation(m, k, seed=51))
+    got = ops.mmq_forward(wtype, w, x, n, fixup=fixup)
+    knobs.set("LK_MMQ_I8")
+    int8 = ops.mmq_forward(wtype, w, x, n, fixup=fixup)
+    knobs.clear("LK_MMQ_I8")
+    q = ops.quantize_q8_1_rows(x)
+    rows = torch.cat([ops.mmvq(wtype, w, q[i:i + 8], k, n) for i in range(0, m, 8)])
+    scale = rows.abs().max().item()
+    assert (got - int8).abs().max().item() <= 2e-5 * scale
+    assert (got - rows).abs().max().item() <= 2e-5 * scale
