@@ -1014,7 +1014,7 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
     // 4096 -> 14336 in 344 us against 240, 2048 x 14336 -> 4096 in 1155 against 742; every other format
     // is 3 to 40 % faster on the wide tile)
     // (Q4_K, Q5_K and Q6_K from 33 rows of a matrix of 2048 rows or more: the f16 tiles)
-    const bool f16 = F::F16_TYPE >= 0 && nrows_x >= 2048 && !lk_env_flag("LK_MMQ_I8");
+    const bool f16 = lk_mmq_tiles_take(F::F16_TYPE, nrows_x, ncols_y);
     if ((ncols_y <= 64 && !f16) || F::MIN_RANK == 16) return launch_dense_tm<F, 64, 2>(pb, s, fixup);
     if constexpr (F::F16_TYPE >= 0)
         if (f16) {

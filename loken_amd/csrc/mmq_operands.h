@@ -48,3 +48,25 @@ static __device__ __forceinline__ void operand_scales(uint8_t* tab, int s, float
     *(uint16_t*)(tab + 48 + 2 * s) = (uint16_t)(b1 >> 16);
     *(uint16_t*)(tab + 64 + 2 * s) = (uint16_t)(__float_as_uint(p2) >> 16);
 }
+
+// Four consecutive values of a 32-value sub-block, from value 4 l8 on, by each of the eight lanes of an aligned group: the
+// Q8_1 rule of the records' quantizer (d = amax / 127, codes = round_half_away(x * (1 / d)), d kept as f16), straight into
+// the operands of its row.
+static __device__ __forceinline__ void operand_quad(float4 v, uint8_t* codes, uint8_t* tab, int s, int l8) {
+    float d;
+    int sum;
+    {
+#pragma clang fp contract(off)
+        const float amax = max8(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        d = amax / 127.0f;
+        const float inv = d != 0.0f ? 1.0f / d : 0.0f;
+        const int q0 = (int)roundf(v.x * inv), q1 = (int)roundf(v.y * inv), q2 = (int)roundf(v.z * inv), q3 = (int)roundf(v.w * inv);
+        int quad_sum;
+        sum = sum8(q0 + q1 + q2 + q3, quad_sum);
+        uint2 o;
+        operand_codes((uint32_t)(q0 & 0xFF) | (uint32_t)(q1 & 0xFF) << 8 | (uint32_t)(q2 & 0xFF) << 16 | (uint32_t)(q3 & 0xFF) << 24, o.x, o.y);
+        // value 16 h + 8 hf + 4 i is half i of atom 2 hf + h
+        *(uint2*)(codes + 64 * s + 32 * ((l8 >> 1) & 1) + 16 * (l8 >> 2) + 8 * (l8 & 1)) = o;
+    }
+    if (l8 == 0) operand_scales(tab, s, __half2float(__float2half_rn(d)), sum);
+}

@@ -123,6 +123,10 @@ int lk_tile_dense_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const Mm
 // Returns the token-tile width launched, 0 when the launch failed, -1 when the operands do not suit these kernels (alignment,
 // 32-bit offsets, no scratch) and the caller should take the int8 tiles.
 int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup);
+// Whether a dense product takes them: 33 token rows or more and 2048 weight rows or more (LK_MMQ_I8 unset).
+bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows);
+// The same for `rows` rows of x, k values each, results in x's type: nothing between x and the operands.
+int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s);
 // The expert-batched product (mmq_f16.hip), same returns.
 int lk_mmq_f16_moe(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
                    int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);

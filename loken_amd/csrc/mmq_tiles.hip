@@ -31,6 +31,20 @@ __global__ __launch_bounds__(256) void operands_from_records_kernel(const uint8_
                    (int)*(const int16_t*)(rec + 272 + 2 * s));
 }
 
+// Rows of x -> operands, the quantizer and the expansion in one pass: grid (rows, k / 1024), four values a thread. Bound by
+// its bytes (2048 x 14336 f32: 185 MB); the records' quantizer and the expansion after it move 285.
+template <typename T>
+__global__ __launch_bounds__(256) void operands_quantize_kernel(const T* __restrict__ x, LkTokenOperands ops, int k) {
+    const int i0 = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (i0 >= k) return;
+    const int64_t row = blockIdx.x, at = (int64_t)(i0 / 256) * ops.rows + row;
+    const T* from = x + row * k + i0;
+    const float4 v = ((uintptr_t)from & (4 * sizeof(T) - 1)) == 0
+                         ? Load4<T>::at(from)
+                         : make_float4(to_f32<T>(from[0]), to_f32<T>(from[1]), to_f32<T>(from[2]), to_f32<T>(from[3]));
+    operand_quad(v, ops.codes + at * LK_OPERAND_CODES, ops.tabs + at * LK_OPERAND_TAB, (i0 / 32) & 7, (i0 / 4) & 7);
+}
+
 // Nanoseconds an item (32 x 32 x 32 product) takes a SIMD: `full` with two workgroups on every CU, `alone` with one, by token
 // tiles; measured on MI355X, whole launches less the 5 us that starting and ending one takes. wide: eight waves, tt = 4.
 struct ItemTimes {
@@ -72,12 +86,12 @@ int launch(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const Mm
 // keeps them apart).
 constexpr int64_t OPERANDS_CAP = 256ll << 20;
 
-}  // namespace
-
-int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
+// The product in passes; fill(operands, first row, rows) launches what writes a pass's operands. Returns as lk_mmq_tiles_dense.
+template <class Fill>
+int run_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup, Fill fill) {
     const int bytes = wtype == LK_TYPE_Q4_K ? Q4K_BYTES : wtype == LK_TYPE_Q5_K ? Q5K_BYTES : Q6K_BYTES;
     const bool q6 = wtype == LK_TYPE_Q6_K;
-    if ((uintptr_t)pb.w % (q6 ? 2 : 16) != 0 || (uintptr_t)pb.y % 16 != 0 || (q6 && pb.n < 128)) return -1;
+    if ((uintptr_t)pb.w % (q6 ? 2 : 16) != 0 || (q6 && pb.n < 128)) return -1;
     // lane offsets inside a tile are 32-bit
     if (pb.row_blocks * bytes * 256 > (int64_t)INT32_MAX || pb.m_begin != 0) return -1;
     const int64_t row_bytes = pb.nb * (LK_OPERAND_CODES + LK_OPERAND_TAB);
@@ -94,11 +108,36 @@ int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fix
         pass.dst = (float*)((uint8_t*)pb.dst + (int64_t)m0 * pb.ldd * (pb.out_type == LK_TYPE_F32 ? 4 : 2));
         const LkTokenOperands ops = lk_operands_at(buffer, pass.m_end, pb.nb);
         const MmqTilePlan plan = plan_dense(wtype, pass, fixup);
-        hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((pass.m_end + 31) / 32)), dim3(256), 0, s, pb.y, ops,
-                           pb.rows_total, m0, pass.m_end);
+        fill(ops, m0, pass.m_end);
         if (launch(wtype, pass, ops, plan, (float*)fixup, s) != LK_OK) return 0;
         if (plan.splits > 1 && lk_mmq_split_sum((const float*)fixup, plan.splits, pass, s) != LK_OK) return 0;
         width = std::max(width, 32 * plan.tt);
     }
     return width;
+}
+
+}  // namespace
+
+int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
+    if ((uintptr_t)pb.y % 16 != 0) return -1;
+    return run_dense(wtype, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int rows) {
+        hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((rows + 31) / 32)), dim3(256), 0, s, pb.y, ops,
+                           pb.rows_total, m0, rows);
+    });
+}
+
+bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows) {
+    return (wtype == LK_TYPE_Q4_K || wtype == LK_TYPE_Q5_K || wtype == LK_TYPE_Q6_K) && rows > 32 && n >= 2048 && !lk_env_flag("LK_MMQ_I8");
+}
+
+int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {
+    if (!lk_mmq_tiles_take(wtype, n, rows) || k % 256 != 0) return -1;
+    const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / 256, rows, n, n, 0, rows, type};
+    return run_dense(wtype, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
+        const dim3 grid((unsigned)count, (unsigned)((k + 1023) / 1024));
+        const int64_t at = (int64_t)m0 * k;
+        if (type == LK_TYPE_F16) hipLaunchKernelGGL(operands_quantize_kernel<__half>, grid, dim3(256), 0, s, (const __half*)x + at, ops, k);
+        else if (type == LK_TYPE_BF16) hipLaunchKernelGGL(operands_quantize_kernel<__hip_bfloat16>, grid, dim3(256), 0, s, (const __hip_bfloat16*)x + at, ops, k);
+        else hipLaunchKernelGGL(operands_quantize_kernel<float>, grid, dim3(256), 0, s, (const float*)x + at, ops, k);
+    });
 }

@@ -325,3 +325,22 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
     lin.close()
     pick = np.sort(np.random.default_rng(97).choice(n, 100, replace=False))
     assert close(got.cpu().numpy()[:, pick], oracle.ob_matmul(wtype, x, w[pick], len(pick)))
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("rows,n,k,shift", [(450, 2048, 256, 0), (180, 2561, 1280, 0), (33, 14336, 512, 1)])
+def test_operands_straight_from_the_rows_are_those_of_the_records(name, rows, n, k, shift):
+    # The tiled products' token operands written by the quantizer itself, or from the workspace records: one rule, so the same
+    # bits; rows that start off a 16-byte piece too. Zeros, the type's largest codes and tiny values among them.
+    w = dev(synth.weight(DT[name], n, k, seed=85, stream=2))
+    x = dev(synth.activation(rows, k, seed=85))
+    x[0] = 0
+    x[1, ::32] = 127
+    x[2] *= 1e-7
+    flat = torch.zeros(rows * k + shift, device="cuda")
+    flat[shift:] = x.reshape(-1)
+    x = flat[shift:].view(rows, k)
+    lin = Linear(DT[name], w, n, k)
+    got = lin(x)
+    assert lin.path == "tiled" and torch.equal(got, ops.mmq_forward(DT[name], w, x.clone(), n))
+    lin.close()
