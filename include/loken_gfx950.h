@@ -603,12 +603,14 @@ int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gat
                    const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts,
                    int hidden, int ffn, void* stream);
 /* The launches it is made of at this size, as bits: LK_MOE_GROUPED (expert-batched products over a grouped
- * routing; else a mat-vec per routed pair), and with it LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN where that
+ * routing; else a mat-vec per routed pair), and with it LK_MOE_TILES where both products run on the f16 tiles (the
+ * tiled launch asked for a tile of 128 has their bits), or LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN where that
  * product is lk_moe_q4k_rows_grouped rather than the tiled launch. For a caller that issues the launches
  * itself and wants the block's bits. */
 #define LK_MOE_GROUPED 1
 #define LK_MOE_ROWS_GATE_UP 2
 #define LK_MOE_ROWS_DOWN 4
+#define LK_MOE_TILES 8
 int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int topk, int n_experts, int hidden, int ffn);
 /* The rules this goes by, each for one stack alone: whether the expert-batched launches pay at `rows` routed rows (wtype: the stacks' type where
  * all have the same, else -1); the longest run an expert is expected to own (mmq_experts.rs:215-227); whether a stack
@@ -753,7 +755,7 @@ void loken_stable_sort_u32(const uint32_t* keys, uint32_t* sorted, uint32_t* ord
 /* The decode-size form (cuda/moe/gate_topk.cu:453-477; src/inference/moe_cuda/dense/gate.rs:185):
  * same result for m keys; the reference serves m <= 32, this m <= 256, nothing is launched above. */
 void loken_argsort_small_u32(const uint32_t* in, uint32_t* sorted_out, uint32_t* index_out, int m, void* stream);
-/* Frees what the expert launchers, the expert block, the router and the wide tiles hold on the current device, for
+/* Frees what the expert launchers, the expert block, the router and the f16 tiles hold on the current device, for
  * every stream and every recorded graph: none recorded over them may be replayed after. The host linears' workspaces
  * stay (lkh_release_workspaces). Synchronizes the device (cuda/moe/moe_gguf.cu:104-118). */
 void loken_stream_scratch_release(void);

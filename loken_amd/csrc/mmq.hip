@@ -141,7 +141,7 @@ struct MmqQ45K {
     static constexpr int ALIGN = 4;   // whole-header reads
     static constexpr int BLOCK_BYTES = Q5 ? Q5K_BYTES : Q4K_BYTES;
     static constexpr int QS0 = Q5 ? 48 : 16;
-    static constexpr int F16_TYPE = Q5 ? LK_TYPE_Q5_K : LK_TYPE_Q4_K;   // the f16 tile kernels take it (mmq_f16.hip)
+    static constexpr int F16_TYPE = Q5 ? LK_TYPE_Q5_K : LK_TYPE_Q4_K;   // the f16 tiles take it (mmq_tile.h)
     static constexpr int WIDE_FROM = 384;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int NS = 8;          // one weight scale per 32 values
     static constexpr bool HAS_MIN = true;
@@ -1074,14 +1074,11 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
     // CUs, the int8 tiles' twice as many workgroups stay)
     const bool f16_short = f16 && mmq_x <= 0 && (w2 ? 2 : 1) * n_experts * ((nrows_x + 255) / 256) >= 32;
     if (want <= 64 && !f16_short) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
-    // Runs of more than 32 rows: the f16 tiles for the formats that have them, a half tile for the experts that own 32
-    // rows or fewer (all three stacks of one format, average run 20 / 32 / 40, against the int8 tiles: Q6_K 248 / 287 /
-    // 308 us against 342 / 359 / 368, Q5_K 202 / 235 / 251 against 263 / 280 / 288; at 8 experts of 1024 -> 1536 80
-    // -> 72; under 33 rows the int8 tile of 32 stays: average 8 / 14, Q6_K 198 / 208 against 231 / 238; 128 experts of 2048 -> 768 -> 2048, top-8,
-    // Q4_K gate + up, 1111 / 1400 tokens, whole block, against the int8 tiles: Q4_K down 400 / 441 us against 512 / 542,
-    // Q5_K 430 / 464 against 518 / 540, Q6_K 464 / 500 against 573 / 599).
+    // Runs of more than 32 rows: the f16 tiles for the formats that have them, over operands made from the records (a block in
+    // one call makes them from the tokens and has its own, lower line: moe_forward.hip); under 33 rows the int8 tile of 32
+    // stays (128 experts of 2048 -> 768 -> 2048, Q6_K, average run 8 / 14: 198 / 208 us against 231 / 238).
     if (f16) {
-        const int tm = lk_mmq_f16_moe(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
+        const int tm = lk_mmq_tiles_moe_records(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
         if (tm >= 0) return tm;
         if (want <= 64) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     }

@@ -119,6 +119,24 @@ struct LkTokenOperands;
 int lk_tile_dense_q4k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
 int lk_tile_dense_q5k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
 int lk_tile_dense_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
+// Expert-batched: expert e's slab, `stride` bytes after the one before, against the sorted rows [bounds[e], bounds[e + 1]).
+// With `to`: gate (the problem's weights) and up (w_second) products of operand rows gather[sorted row], and silu(gate) * up as
+// the operands `to` of the next product, a row per sorted row. Else the products to dst, w_second's dst_second floats further.
+struct MmqTileExperts {
+    const int32_t *bounds, *gather;
+    const uint8_t* w_second;
+    int64_t dst_second, stride, longest;   // longest: expected longest run
+    int n_experts;
+    const LkTokenOperands* to;
+};
+int lk_tile_moe_q4k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+int lk_tile_moe_q5k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+int lk_tile_moe_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+// Whether an expert-batched product can take them (alignment, sizes); `gated`: as lk_tile_moe_* with `to`.
+bool lk_mmq_tiles_moe_fit(int wtype, const void* w, const void* w_second, int64_t stride, int64_t n, int64_t k, int64_t rows, bool gated);
+int lk_mmq_tiles_moe(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+// `rows` rows of x (k values each) as token operands.
+int lk_operands_quantize(const void* x, int type, const LkTokenOperands& ops, int k, int rows, hipStream_t s);
 // A dense product on them (mmq_tiles.hip), operands made from the workspace records; `fixup`: the caller's tmp_fixup or null.
 // Returns the token-tile width launched, 0 when the launch failed, -1 when the operands do not suit these kernels (alignment,
 // 32-bit offsets, no scratch) and the caller should take the int8 tiles.
@@ -127,6 +145,6 @@ int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fix
 bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows);
 // The same for `rows` rows of x, k values each, results in x's type: nothing between x and the operands.
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s);
-// The expert-batched product (mmq_f16.hip), same returns.
-int lk_mmq_f16_moe(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
-                   int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);
+// The expert-batched product over workspace records, same returns as the dense one.
+int lk_mmq_tiles_moe_records(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
+                             int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);

@@ -217,15 +217,17 @@ struct TileShape {
     // LDS: ring of quarters, two blocks' tables, each wave's weights, each wave's d of its rows for two blocks
     static constexpr int T_AT = 0, TAB_AT = NQ * QB, W_AT = TAB_AT + 2 * TABB, D_AT = W_AT + WAVES * W_BYTES, LDS = D_AT + WAVES * 256;
     static_assert(LDS <= (WAVES == 4 ? 80 : 160) * 1024, "LDS of a workgroup");
-    // Slots in which the next block's weights are loaded and, through registers, stored: with few token tiles a piece is in
-    // flight for a whole block (LONG: the block after the next), with many for 2 TT slots, which leaves registers.
+    // Slots in which weights are loaded: directly, a region's next pieces right after the slot that has read it (A, read in slot
+    // 7 TT - 1 for the next block: the block after that; B, in 3 TT - 1: the next block), so that they have almost a block's time.
+    // Through registers, with few token tiles a piece is in flight for a whole block (LONG: the block after the next), with
+    // many for 2 TT slots, which leaves registers; stored in commit_slot.
     static constexpr bool LONG = TT <= 2;
     static constexpr int commit_slot(int i) {
         const int c = (i < AC ? i + 2 : i + 1) * TT;
         return F::DMA ? -1 : c < NI ? c : NI - 1;
     }
     static constexpr int fetch_slot(int i) {
-        return F::DMA ? (i < AC ? i * TT / 2 : 4 * TT + (i - AC) * TT / 2) : LONG ? commit_slot(i) : commit_slot(i) - 2 * TT;
+        return F::DMA ? (i < AC ? 7 * TT + i * TT / AC : 3 * TT + (i - AC) * TT / BC) : LONG ? commit_slot(i) : commit_slot(i) - 2 * TT;
     }
     // Direct loads a wave issues in slot I. (Loads into registers, which the compiler places, are left out: `keep` then asks
     // for more than it has to and never for less.)
@@ -242,8 +244,9 @@ struct TileShape {
     static constexpr int keep(int q) {
         int last = (q + 1 - LEAD) * QI + CC - 1;                             // codes of quarter q + 1
         if (q == 3) last = later(last, QI + CC + RC - 1);                    // the next block's tables
-        if (F::DMA && q == 2) last = later(last, fetch_slot(AC - 1));        // the next block's A, read in slot 7 TT - 1
-        if (F::DMA && q == 0) last = later(last, fetch_slot(CH - 1) - NI);   // this block's B, read in slot 3 TT - 1
+        // the next block's A, read in slot 7 TT - 1, and this block's B, in 3 TT - 1: the last barriers before
+        if (F::DMA && q == (TT == 1 ? 3 : 2)) last = later(last, fetch_slot(AC - 1) - NI);
+        if (F::DMA && q == (TT == 1 ? 1 : 0)) last = later(last, fetch_slot(CH - 1) - NI);
         int n = 0;
         for (int I = last + 1; I < q * QI + QI - 2; ++I) n += direct(I);
         return n;
@@ -405,7 +408,8 @@ struct TileWave {
         }
         if constexpr (tt == TT - 1) operands<(s + 1) & 7>();
         if constexpr (I == 3 * TT - 1) { F::codes1(cd, rb, h, j); wave_order(); }
-        // the next block's weights into the stage this block has been read from for the last time
+        // weights into the region that the slot before has read (those reads are over here)
+        if constexpr (F::DMA && (I == 3 * TT || I == 7 * TT)) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         commits<I>(kb, next, next2, std::make_integer_sequence<int, S::CH>{});
         if constexpr (I == 7 * TT - 1) {
             wave_order();
@@ -441,7 +445,7 @@ struct TileWave {
     __device__ __forceinline__ void commits(int kb, int next, int next2, std::integer_sequence<int, C...>) {
         ([&] {
             if constexpr (!F::DMA && S::commit_slot(C) == I) commit(C);
-            if constexpr (S::fetch_slot(C) == I) fetch(!F::DMA && S::LONG ? next2 : next, C);
+            if constexpr (S::fetch_slot(C) == I) fetch((F::DMA ? C < S::AC : S::LONG) ? next2 : next, C);
         }(), ...);
     }
     template <int I, int... Q>
@@ -455,16 +459,19 @@ struct TileWave {
     }
 };
 
-// The tile of weight rows n0 .. n0 + 32 WAVES - 1 and tokens m0 .. m0 + 32 TT - 1. Row m0 + i of the operands is token
-// m0 + i, with GATHER row gather[m0 + i]. Formats through registers: all the tile's rows exist.
+// The products of a wave's 32 weight rows with tokens m0 .. m0 + 32 TT - 1, left in `t`: rows row0 .. row0 + 31 of the `live`
+// rows from `weights` on (formats through registers: they all exist; others re-read the last one, whose results are never
+// stored). Row m0 + i of the operands is token m0 + i, with GATHER row gather[m0 + i].
 template <class F, int TT, int WAVES, bool GATHER>
-static __device__ __forceinline__ void tile_of(const MmqProblem& pb, const LkTokenOperands& ops, const int32_t* gather, int n0, int m0, uint8_t* lds) {
+static __device__ __forceinline__ void multiply(TileWave<F, TT, WAVES, GATHER>& t, const MmqProblem& pb, const LkTokenOperands& ops,
+                                                const int32_t* gather, const uint8_t* weights, int row0, int live, int m0, uint8_t* lds) {
     using S = TileShape<F, TT, WAVES>;
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // a caller's loop over tiles keeps none of what follows from it in registers meanwhile
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int last = (int)pb.nb - 1;
     const int64_t row_bytes = pb.row_blocks * F::BYTES;
-    TileWave<F, TT, WAVES, GATHER> t;
     t.wave = wave;
     t.j = lane & 31;
     t.h = lane >> 5;
@@ -473,7 +480,7 @@ static __device__ __forceinline__ void tile_of(const MmqProblem& pb, const LkTok
     t.tab_slab = ops.rows * LK_OPERAND_TAB;
     t.codes = ops.codes;
     t.tabs = ops.tabs;
-    t.w = pb.w + (int64_t)n0 * row_bytes;
+    t.w = weights;
     // a chunk is eight tokens x 128 bytes; atom p of token t lands in place p ^ (t % 8), so that 32 tokens spread over the banks
     const uint32_t swz = 16 * ((lane & 7) ^ (lane >> 3));
     if constexpr (GATHER) {
@@ -499,15 +506,15 @@ static __device__ __forceinline__ void tile_of(const MmqProblem& pb, const LkTok
             const bool in_a = i < S::AC;
             const int per = in_a ? F::AP : F::BP;
             const int idx = min(lane + 64 * (in_a ? i : i - S::AC), 32 * per - 1), row = idx / per, p = idx % per;
-            t.from[i] = (uint32_t)min(32 * wave + row, pb.n - 1 - n0) * (uint32_t)row_bytes + (in_a ? F::a_src(p) : F::b_src(p, row));
+            t.from[i] = (uint32_t)min(row0 + row, live - 1) * (uint32_t)row_bytes + (in_a ? F::a_src(p) : F::b_src(p, row));
         }
     } else {
-        const uint32_t row = (uint32_t)(32 * wave + (lane >> 3)) * (uint32_t)row_bytes;
+        const uint32_t row = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)row_bytes;
         t.from[0] = row + F::a_src(min(lane & 7, F::AP - 1));
         t.from[1] = row + F::b_src(min(lane & 7, F::BP - 1), 0);
         t.row_bytes8 = 8 * row_bytes;
     }
-    t.d_from = (uint32_t)min(32 * wave + t.j, pb.n - 1 - n0) * (uint32_t)row_bytes + F::BYTES - 2;
+    t.d_from = (uint32_t)min(row0 + t.j, live - 1) * (uint32_t)row_bytes + F::BYTES - 2;
     t.d = 0;
 #pragma unroll
     for (int x = 0; x < 4; ++x) t.tb[x] = lds + S::T_AT + t.j * 128 + 16 * ((2 * x + t.h) ^ (t.j & 7));
@@ -536,19 +543,19 @@ static __device__ __forceinline__ void tile_of(const MmqProblem& pb, const LkTok
         for (int c = 0; c < S::CC; ++c) t.load_codes(0, q, c);
 #pragma unroll
     for (int c = 0; c < S::RC; ++c) t.load_tabs(0, c);
-    if constexpr (F::DMA) meet<0>();
-    else
+    if constexpr (!F::DMA)
 #pragma unroll
         for (int i = 0; i < S::CH; ++i) t.commit(i);
-    wave_order();
+    meet<0>();
     t.hd = F::header(t.ra, t.h);
     F::codes0(t.cd, t.ra, t.h);
     t.write_d(0);
+    wave_order();
     t.fetch_d(min(1, last));
-    meet<0>();
-    if constexpr (!F::DMA && S::LONG)
+    if constexpr (F::DMA) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if constexpr (F::DMA || S::LONG)
 #pragma unroll
-        for (int i = 0; i < S::CH; ++i) t.fetch(min(1, last), i);
+        for (int i = 0; i < (F::DMA ? S::AC : S::CH); ++i) t.fetch(min(1, last), i);
     t.template load_atom<0, 0>(); t.template load_atom<0, 1>(); t.template load_d8<0>(0);
     t.template load_atom<1, 0>(); t.template load_atom<1, 1>(); t.template load_d8<1>(0);
     t.template operands<0>();
@@ -560,8 +567,12 @@ static __device__ __forceinline__ void tile_of(const MmqProblem& pb, const LkTok
     for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) t.acc[tt][v] = fmaf(t.dv[v], t.part[tt][v], t.acc[tt][v]);
+}
 
-    const bool vec_ok = pb.out_type == LK_TYPE_F32 && (uintptr_t)pb.dst % 16 == 0 && pb.ldd % 4 == 0 && n0 % 4 == 0;
+// A wave's results to dst[token][row], or dst[ids_dst[token]][row]; `first` its first weight row.
+template <class F, int TT, int WAVES, bool GATHER>
+static __device__ __forceinline__ void store_rows(const TileWave<F, TT, WAVES, GATHER>& t, const MmqProblem& pb, int first, int m0) {
+    const bool vec_ok = pb.out_type == LK_TYPE_F32 && (uintptr_t)pb.dst % 16 == 0 && pb.ldd % 4 == 0 && first % 4 == 0;
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
         const int col = m0 + 32 * tt + t.j;
@@ -569,16 +580,55 @@ static __device__ __forceinline__ void tile_of(const MmqProblem& pb, const LkTok
         const int64_t out = (pb.ids_dst ? pb.ids_dst[col] : col) * pb.ldd;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int gn0 = n0 + 32 * wave + 8 * g + 4 * t.h;
-            if (gn0 + 3 < pb.n) {
-                mmq_store4(pb, out + gn0, make_float4(t.acc[tt][4 * g], t.acc[tt][4 * g + 1], t.acc[tt][4 * g + 2], t.acc[tt][4 * g + 3]), vec_ok);
+            const int row = first + 8 * g + 4 * t.h;
+            if (row + 3 < pb.n) {
+                mmq_store4(pb, out + row, make_float4(t.acc[tt][4 * g], t.acc[tt][4 * g + 1], t.acc[tt][4 * g + 2], t.acc[tt][4 * g + 3]), vec_ok);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (gn0 + e < pb.n) lk_store_as(pb.dst, out + gn0 + e, t.acc[tt][4 * g + e], pb.out_type);
+                    if (row + e < pb.n) lk_store_as(pb.dst, out + row + e, t.acc[tt][4 * g + e], pb.out_type);
             }
         }
     }
+}
+
+// silu(gate) * up of a token tile as the next product's operands. The 32 weight rows of a wave are one sub-block of them: lane
+// (j, h) holds 16 of token j's values, lane (j, 1 - h) the others; `first` their first row. The steps of operand_quad.
+static __device__ __forceinline__ void store_gated(const v16f& gate, const v16f& up, const LkTokenOperands& to, int first, int row, int h, bool live) {
+    const int64_t at = (int64_t)(first / 256) * to.rows + row;
+    const int s = (first / 32) & 7;
+    float v[16], amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        v[i] = gate[i] / (1.0f + expf(-gate[i])) * up[i];
+        amax = fmaxf(amax, fabsf(v[i]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    float d;
+    int sum = 0;
+    uint2 codes[4];
+    {
+#pragma clang fp contract(off)
+        d = amax / 127.0f;
+        const float inv = d != 0.0f ? 1.0f / d : 0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            uint32_t word = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int q = (int)roundf(v[4 * g + e] * inv);
+                sum += q;
+                word |= (uint32_t)(q & 0xFF) << (8 * e);
+            }
+            operand_codes(word, codes[g].x, codes[g].y);
+        }
+    }
+    sum += __shfl_xor(sum, 32);
+    if (!live) return;
+    uint8_t* out = to.codes + at * LK_OPERAND_CODES + 64 * s + 8 * h;   // row 8 g + 4 h + e is value 4 h + e of atom (g % 2, g / 2)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *(uint2*)(out + 32 * (g & 1) + 16 * (g >> 1)) = codes[g];
+    if (h == 0) operand_scales(to.tabs + at * LK_OPERAND_TAB, s, __half2float(__float2half_rn(d)), sum);
 }
 
 // Workgroup id -> (n tile, K range, m tile): the m tiles of one n tile re-read the same weight rows, so they are issued back
@@ -607,7 +657,108 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void tile_dense_ker
     }
     int n0 = n_tile * ROWS;
     if (!F::DMA) n0 = min(n0, pb.n - ROWS);   // (the last tile slides back over the one before: same rows, same results)
-    tile_of<F, TT, WAVES, false>(pb, ops, nullptr, n0, m_tile * 32 * TT, lds);
+    const int row0 = 32 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    TileWave<F, TT, WAVES, false> t;
+    multiply(t, pb, ops, nullptr, pb.w + n0 * (pb.row_blocks * F::BYTES), row0, pb.n - n0, m_tile * 32 * TT, lds);
+    store_rows(t, pb, n0 + row0, m_tile * 32 * TT);
+}
+
+// ------------------------------------------------------------------ experts
+// One tile of an expert's run. GATED: waves 0 and 1 take 64 rows of the gate, 2 and 3 the same rows of the up matrix (pb.w,
+// w_second), and the gated products leave as operands (`to`, a row per sorted row); else 128 rows of pb.w to pb.dst.
+template <class F, int TT, bool GATED>
+static __device__ __forceinline__ void expert_tile(const MmqProblem& pb, const LkTokenOperands& ops, const int32_t* gather, const uint8_t* w_second,
+                                                   const LkTokenOperands& to, int n_tile, int m0, uint8_t* lds) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row_bytes = pb.row_blocks * F::BYTES;
+    TileWave<F, TT, 4, GATED> t;
+    if constexpr (!GATED) {
+        int n0 = n_tile * 128;
+        if (!F::DMA) n0 = min(n0, pb.n - 128);
+        multiply(t, pb, ops, gather, pb.w + n0 * row_bytes, 32 * wave, pb.n - n0, m0, lds);
+        store_rows(t, pb, n0 + 32 * wave, m0);
+    } else {
+        const int n0 = n_tile * 64, row0 = 32 * (wave & 1);
+        const bool is_up = wave >= 2;
+        multiply(t, pb, ops, gather, (is_up ? w_second : pb.w) + n0 * row_bytes, row0, pb.n - n0, m0, lds);
+        meet<0>();
+        // the two waves of a row block trade token tiles through LDS: even ones are finished by the gate's wave, odd ones by the up's
+        float* mine = (float*)lds + (threadIdx.x & 63) * 4;
+        auto slab = [&](int tt) { return mine + ((wave & 1) * TT + tt) * 1024; };
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+            if ((tt & 1) != (int)is_up)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *(float4*)(slab(tt) + 256 * g) = make_float4(t.acc[tt][4 * g], t.acc[tt][4 * g + 1], t.acc[tt][4 * g + 2], t.acc[tt][4 * g + 3]);
+        meet<0>();
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+            if ((tt & 1) == (int)is_up) {
+                v16f other;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 o = *(const float4*)(slab(tt) + 256 * g);
+                    other[4 * g] = o.x; other[4 * g + 1] = o.y; other[4 * g + 2] = o.z; other[4 * g + 3] = o.w;
+                }
+                const int row = m0 + 32 * tt + t.j;
+                store_gated(is_up ? other : t.acc[tt], is_up ? t.acc[tt] : other, to, n0 + row0, row, t.h, row < pb.m_end);
+            }
+    }
+}
+
+// Expert e's slab against the sorted rows [bounds[e], bounds[e + 1]); grid: mmq_moe_grid. A run of c token tiles of 32 is cut
+// into as few tiles of at most MAX as hold it, of equal length up to one (MAX = 3, four: two and two).
+template <class F, bool GATED, int MAX>
+__global__ __launch_bounds__(256, MAX == 1 && F::DMA ? 3 : 2) void tile_moe_kernel(MmqProblem pb, LkTokenOperands ops, const int32_t* __restrict__ gather,
+                                                                         const uint8_t* w_second, int64_t dst_second, LkTokenOperands to,
+                                                                         const int32_t* __restrict__ bounds, int64_t stride_expert,
+                                                                         int n_experts, int group) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int stack = blockIdx.y / n_experts, e = blockIdx.y % n_experts;
+    const int n_tiles = GATED ? pb.n / 64 : (pb.n + 127) / 128, n_tile = blockIdx.x % n_tiles;
+    pb.m_begin = bounds[e];
+    pb.m_end = bounds[e + 1];
+    const int c = (pb.m_end - pb.m_begin + 31) / 32, tiles = (c + MAX - 1) / MAX;
+    if (c <= 0) return;
+    pb.w = (stack ? w_second : pb.w) + e * stride_expert;
+    if (GATED) w_second += e * stride_expert;
+    if (stack) pb.dst += dst_second;
+    pb.out_type = LK_TYPE_F32;   // known here: the stores need no choice
+    const int first = blockIdx.z * group + blockIdx.x / n_tiles, step = gridDim.z * group;
+    for (int i = first; i < tiles; i += step) {
+        if (i != first) meet<0>();   // the next tile's first loads go where this one's were
+        const int from = c * i / tiles, count = c * (i + 1) / tiles - from, m0 = pb.m_begin + 32 * from;
+        if (MAX == 1 || count == 1) expert_tile<F, 1, GATED>(pb, ops, gather, w_second, to, n_tile, m0, lds);
+        if constexpr (MAX >= 2) if (count == 2) expert_tile<F, 2, GATED>(pb, ops, gather, w_second, to, n_tile, m0, lds);
+        if constexpr (MAX >= 3) if (count == 3) expert_tile<F, 3, GATED>(pb, ops, gather, w_second, to, n_tile, m0, lds);
+        if constexpr (MAX >= 4) if (count == 4) expert_tile<F, 4, GATED>(pb, ops, gather, w_second, to, n_tile, m0, lds);
+    }
+}
+
+template <class F, int MAX>
+static constexpr int moe_lds() {
+    constexpr int a = TileShape<F, 1, 4>::LDS, b = MAX >= 2 ? TileShape<F, 2, 4>::LDS : 0, c = MAX >= 3 ? TileShape<F, 3, 4>::LDS : 0, d = MAX >= 4 ? TileShape<F, 4, 4>::LDS : 0;
+    constexpr int ab = a > b ? a : b, cd = c > d ? c : d;
+    return ab > cd ? ab : cd;
+}
+template <class F, bool GATED, int MAX>
+static int launch_moe(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {
+    auto kernel = tile_moe_kernel<F, GATED, MAX>;
+    constexpr int LDS = moe_lds<F, MAX>();
+    if (int rc = mmq_prepare_kernel(kernel, LDS)) return rc;
+    // (MAX = 1: a second column tile for the runs that turn out longer than expected, which would double the launch's end)
+    const MmqMoeGrid g = mmq_moe_grid(pb, GATED ? 64 : 128, 32 * MAX, !GATED && ex.w_second ? 2 : 1, ex.n_experts, ex.longest + (MAX == 1 ? 8 : 0));
+    hipLaunchKernelGGL(kernel, g.grid, dim3(256), LDS, s, pb, ops, ex.gather, ex.w_second, ex.dst_second, ex.to ? *ex.to : LkTokenOperands{},
+                       ex.bounds, ex.stride, ex.n_experts, g.group);
+    return lk_launch_status();
+}
+// Tiles of at most three token tiles (a fourth costs Q6_K 35 spilled registers and no format gains: runs of 69 rows 246 us
+// against 250, of 278 rows 118 against 120); runs of 32 rows and less leave registers for a third workgroup a CU (256 tokens over
+// 128 experts 138 -> 126 us).
+template <class F, bool GATED>
+static int launch_moe(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {
+    return ex.longest <= 32 ? launch_moe<F, GATED, 1>(pb, ops, ex, s) : launch_moe<F, GATED, 3>(pb, ops, ex, s);
 }
 
 template <class F, int TT, int WAVES>
@@ -640,4 +791,7 @@ static int launch_dense_plan(const MmqProblem& pb, const LkTokenOperands& ops, c
 #define LK_DEFINE_TILES(NAME, FORMAT)                                                                                             \
     int lk_tile_dense_##NAME(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s) { \
         return mmq_tile::launch_dense_plan<FORMAT>(pb, ops, plan, part, s);                                                       \
+    }                                                                                                                             \
+    int lk_tile_moe_##NAME(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {           \
+        return ex.to ? mmq_tile::launch_moe<FORMAT, true>(pb, ops, ex, s) : mmq_tile::launch_moe<FORMAT, false>(pb, ops, ex, s);  \
     }

@@ -134,10 +134,43 @@ int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, in
     if (!lk_mmq_tiles_take(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / 256, rows, n, n, 0, rows, type};
     return run_dense(wtype, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
-        const dim3 grid((unsigned)count, (unsigned)((k + 1023) / 1024));
-        const int64_t at = (int64_t)m0 * k;
-        if (type == LK_TYPE_F16) hipLaunchKernelGGL(operands_quantize_kernel<__half>, grid, dim3(256), 0, s, (const __half*)x + at, ops, k);
-        else if (type == LK_TYPE_BF16) hipLaunchKernelGGL(operands_quantize_kernel<__hip_bfloat16>, grid, dim3(256), 0, s, (const __hip_bfloat16*)x + at, ops, k);
-        else hipLaunchKernelGGL(operands_quantize_kernel<float>, grid, dim3(256), 0, s, (const float*)x + at, ops, k);
+        (void)lk_operands_quantize((const uint8_t*)x + (int64_t)m0 * k * (type == LK_TYPE_F32 ? 4 : 2), type, ops, k, count, s);
     });
+}
+
+int lk_operands_quantize(const void* x, int type, const LkTokenOperands& ops, int k, int rows, hipStream_t s) {
+    const dim3 grid((unsigned)rows, (unsigned)((k + 1023) / 1024));
+    if (type == LK_TYPE_F16) hipLaunchKernelGGL(operands_quantize_kernel<__half>, grid, dim3(256), 0, s, (const __half*)x, ops, k);
+    else if (type == LK_TYPE_BF16) hipLaunchKernelGGL(operands_quantize_kernel<__hip_bfloat16>, grid, dim3(256), 0, s, (const __hip_bfloat16*)x, ops, k);
+    else hipLaunchKernelGGL(operands_quantize_kernel<float>, grid, dim3(256), 0, s, (const float*)x, ops, k);
+    return lk_launch_status();
+}
+
+bool lk_mmq_tiles_moe_fit(int wtype, const void* w, const void* w_second, int64_t stride, int64_t n, int64_t k, int64_t rows, bool gated) {
+    if (wtype != LK_TYPE_Q4_K && wtype != LK_TYPE_Q5_K && wtype != LK_TYPE_Q6_K) return false;
+    const int bytes = wtype == LK_TYPE_Q4_K ? Q4K_BYTES : wtype == LK_TYPE_Q5_K ? Q5K_BYTES : Q6K_BYTES, align = wtype == LK_TYPE_Q6_K ? 2 : 16;
+    if (k % 256 != 0 || n > INT32_MAX || n < 128 || (gated && n % 64 != 0)) return false;
+    // operand row offsets inside a block, and row offsets inside a tile, are 32-bit
+    return ((uintptr_t)w | (uintptr_t)w_second | (uintptr_t)stride) % align == 0 && rows < (1 << 23) && k / 256 * bytes * 128 <= (int64_t)INT32_MAX;
+}
+
+int lk_mmq_tiles_moe(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {
+    return wtype == LK_TYPE_Q4_K   ? lk_tile_moe_q4k(pb, ops, ex, s)
+           : wtype == LK_TYPE_Q5_K ? lk_tile_moe_q5k(pb, ops, ex, s)
+                                   : lk_tile_moe_q6k(pb, ops, ex, s);
+}
+
+int lk_mmq_tiles_moe_records(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
+                             int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s) {
+    if ((uintptr_t)pb.y % 16 != 0 || pb.row_blocks > INT32_MAX / 256 || pb.nb > INT32_MAX / 256 ||
+        !lk_mmq_tiles_moe_fit(wtype, pb.w, w_second, stride_expert, pb.n, 256 * pb.row_blocks, pb.rows_total, false))
+        return -1;
+    LkScratch scratch(s);
+    void* buffer = scratch.get(LK_SCRATCH_TOKENS, lk_operand_bytes(pb.rows_total, pb.nb));
+    if (!buffer) return -1;
+    const LkTokenOperands ops = lk_operands_at(buffer, pb.rows_total, pb.nb);
+    hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((pb.rows_total + 31) / 32)), dim3(256), 0, s, pb.y, ops,
+                       pb.rows_total, 0, (int)pb.rows_total);
+    const MmqTileExperts ex{bounds, nullptr, w_second, dst_second, stride_expert, ncols_max, n_experts, nullptr};
+    return lk_mmq_tiles_moe(wtype, pb, ops, ex, s) == LK_OK ? 128 : 0;
 }

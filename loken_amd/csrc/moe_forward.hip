@@ -8,6 +8,8 @@
 // tiled products is quantized where it is computed, and the host does one call instead of eight to fifteen
 // (a one-token block of 128 experts: 80 us with torch's sort, copies and fills around the two kernels).
 
+#include "mmq_operands.h"
+#include "mmq_problem.h"
 #include "moe_block.h"
 #include "stream_scratch.h"
 
@@ -42,17 +44,48 @@ bool grouped_serves(const Format& f, int k) { return f.grouped && k % 256 == 0; 
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 size_t workspace_bytes(int64_t rows, int k) { return (size_t)rows * ((k + 511) / 512 * 4) * 144 + 128 * 144; }
 
+// The grouped block on the f16 tiles: the tokens quantized once, as operands (not once per routed pair), gathered by the gate +
+// up launch, which leaves silu(gate) * up as the operands of the down launch. 128 experts of 2048 -> 768 -> 2048, top-8, 1111
+// tokens, Q6_K down: 275 us, where records per pair, f32 products, a gated quantizer and tiles of 64 took 412.
+int block_on_tiles(const Format& fg, const Format& fd, const float* x, const void* gate, const void* up, const void* down,
+                   const int32_t* choices, const float* topk_weights, float* out, int tokens, int topk, int n_experts, int hidden, int ffn,
+                   int longest, LkScratch& scratch, hipStream_t s) {
+    const int rows = tokens * topk, nb = hidden / 256, nb2 = ffn / 256;
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const size_t p = at; at += up256(bytes); return p; };
+    const size_t bounds_at = take((size_t)(n_experts + 1) * 4), slots_at = take((size_t)rows * 4), src_at = take((size_t)rows * 4);
+    const size_t x_at = take(lk_operand_bytes(tokens, nb)), h_at = take(lk_operand_bytes(rows, nb2)), pairs_at = take((size_t)rows * hidden * 4);
+    uint8_t* base = (uint8_t*)scratch.get(LK_SCRATCH_BLOCK, at);
+    if (!base) return LK_ERR_NOMEM;
+    int32_t *bounds = (int32_t*)(base + bounds_at), *slots = (int32_t*)(base + slots_at), *src = (int32_t*)(base + src_at);
+    float* pairs = (float*)(base + pairs_at);
+    const LkTokenOperands tokens_in = lk_operands_at(base + x_at, tokens, nb), h = lk_operands_at(base + h_at, rows, nb2);
+
+    if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, s)) return rc;
+    if (int rc = lk_operands_quantize(x, LK_TYPE_F32, tokens_in, hidden, tokens, s)) return rc;
+    MmqProblem gu{(const uint8_t*)gate, nullptr, nullptr, nullptr, nb, nb, rows, 0, ffn, 0, 0};
+    const MmqTileExperts first{bounds, src, (const uint8_t*)up, 0, (int64_t)ffn * nb * fg.block_bytes, longest, n_experts, &h};
+    if (int rc = lk_mmq_tiles_moe(fg.type, gu, tokens_in, first, s)) return rc;
+    MmqProblem dn{(const uint8_t*)down, nullptr, pairs, slots, nb2, nb2, rows, hidden, hidden, 0, 0};
+    const MmqTileExperts second{bounds, nullptr, nullptr, 0, (int64_t)hidden * nb2 * fd.block_bytes, longest, n_experts, nullptr};
+    if (int rc = lk_mmq_tiles_moe(fd.type, dn, h, second, s)) return rc;
+    return lk_moe_fold(pairs, topk_weights, choices, n_experts, out, tokens, topk, hidden, 0, s);
+}
+
 }  // namespace
 
 // Routed rows from which the expert-batched launches beat a mat-vec per routed pair. The reference breaks even
 // at one routed row per expert (mmq_experts.rs:72-86); here, measured on MI355X (128 experts of 2048 -> 768 -> 2048, top-8), the
-// mat-vec per routed pair stays ahead of the tiled products up to three rows per expert (117 us against 162 at 32
-// tokens, 176 against 168 at 48), and of the matrix-unit rows launch that Q4_K stacks take at short runs up to
-// 1.625 (16 tokens: 51 us against 74; 24: 81 against 83; 32: 92 against 88; 48: 139 against 106). `wtype`: the stacks' type where both
-// have the same, else -1.
+// mat-vec per routed pair stays ahead of the int8 tiles up to three rows per expert, of the matrix-unit rows launch that
+// Q4_K stacks take at short runs up to 1.625 (16 tokens: 51 us against 74; 24: 81 against 83; 32: 92 against 88; 48: 139 against
+// 106), and of the f16 tiles up to two (Q5_K, 1.8 / 2.1 rows: 138 / 174 against 125 / 134) or two and a half (Q6_K, 2.4 / 2.9
+// rows: 55 / 227 against 60 / 199). `wtype`: the stacks' type where both have the same, else -1.
 extern "C" int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype) {
     const int64_t experts = n_experts > 1 ? n_experts : 1;
-    return wtype == LK_TYPE_Q4_K ? 8 * rows >= 13 * experts : rows >= 3 * experts;
+    return wtype == LK_TYPE_Q4_K   ? 8 * rows >= 13 * experts
+           : wtype == LK_TYPE_Q5_K ? rows >= 2 * experts
+           : wtype == LK_TYPE_Q6_K ? 2 * rows >= 5 * experts
+                                   : rows >= 3 * experts;
 }
 
 // The longest run of rows an expert is expected to own, every choice equally likely: mean + sqrt(2 ln experts)
@@ -76,22 +109,39 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
     return wtype == LK_TYPE_Q4_K && k % 256 == 0 && longest_run <= (k <= 2048 ? 44 : 40);
 }
 
+// Whether the block goes on the f16 tiles with nothing but operands between its launches (block_on_tiles), for two stacks of
+// Q4_K, Q5_K or Q6_K. Measured on MI355X, whole block, by the longest expected run, against the launches it replaces:
+//   Q5_K always (128 experts of 2048 -> 768 at 11 / 31 / 50 rows 137 / 147 / 182 us against 167 / 186 / 216)
+//   Q6_K likewise (64 of 1536 -> 1024 at 9 / 26 / 50 rows 99 / 105 / 125 against 104 / 112 / 150), but for short runs over 60 experts and
+//     more, whose int8 tiles of 32 tokens run two more workgroups a CU (128 of 2048 -> 768 at 11 / 22 rows 202 / 208 against 193 / 205)
+//   Q4_K, whose short runs have the rows launch, from 20 rows (128 of 2048 -> 768 at 19 / 26 / 42 rows 123 / 128 / 152 against 117 / 145 / 202,
+//     64 of 1536 -> 1024 at 15 / 22 / 42 rows 64 / 66 / 82 against 59 / 81 / 138); from 9 where that launch reads rows of more than
+//     eight super-blocks and the tiles fill the chip (60 of 2560 -> 1280 at 7 / 9 / 17 / 26 rows 116 / 120 / 117 / 123 against 114 / 141 / 195 / 182)
+// and with workgroups of 64 gate and up rows for a quarter of the CUs at least.
+static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int hidden, int ffn) {
+    auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K; };
+    if (!has_tiles(gu) || !has_tiles(down) || lk_env_flag("LK_MMQ_I8") || (int64_t)n_experts * (ffn / 64) < lk_device().cus / 4) return false;
+    if (gu == LK_TYPE_Q5_K || down == LK_TYPE_Q5_K) return true;
+    if (gu == LK_TYPE_Q6_K && down == LK_TYPE_Q6_K) return longest > 22 || n_experts < 60;
+    return longest >= 20 || (longest >= 9 && hidden > 2048 && 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus);
+}
+
 // Which launches the block is made of: LK_MOE_GROUPED (expert-batched products; else a mat-vec per routed pair),
-// and in it LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN (lk_moe_q4k_rows_grouped; else tiles). The one place that decides:
-// lk_moe_forward and a caller that issues the launches itself both ask here.
+// and in it LK_MOE_TILES (both products on the f16 tiles), or LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN
+// (lk_moe_q4k_rows_grouped; else the tiled launch). The one place that decides: lk_moe_forward and a caller that issues the
+// launches itself both ask here.
 // Gate and up also leave the rows launch where
 //   * down is tiled, past 36 rows: tiles for both keep the rows between them in the tiles' layout and the activation in
-//     their quantizer (128 experts as above with a Q6_K down, 26 / 34 / 42 / 50 rows: 175 / 209 / 234 / 241 us against
-//     187 / 203 / 218 / 231)
-//   * their rows are long and their tiles fill the chip, past 20 rows (60 experts of 2560 -> 1280, 600 tiles, at 16 /
-//     25 / 33 / 41 rows 150 / 208 / 217 / 272 us against 161 / 168 / 175 / 190)
+//     their quantizer
+//   * their rows are long and their tiles fill the chip, past 20 rows
 extern "C" int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int topk, int n_experts, int hidden, int ffn) {
     const Format *fg = format_of(wtype_gu), *fd = format_of(wtype_down);
     if (!fg || !fd || tokens <= 0 || topk <= 0 || n_experts <= 0) return 0;
-    if (!lk_moe_grouped_pays((int64_t)tokens * topk, n_experts, wtype_gu == wtype_down ? wtype_gu : -1) || !grouped_serves(*fg, hidden) ||
-        !grouped_serves(*fd, ffn))
-        return 0;
+    auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K; };
+    const int line = wtype_gu == wtype_down ? wtype_gu : has_tiles(wtype_gu) && has_tiles(wtype_down) ? LK_TYPE_Q6_K : -1;
+    if (!lk_moe_grouped_pays((int64_t)tokens * topk, n_experts, line) || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
+    if (block_takes_tiles(wtype_gu, wtype_down, longest, n_experts, hidden, ffn)) return LK_MOE_GROUPED | LK_MOE_TILES;
     const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
     const bool tiles_fill = 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus;
     const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest) && (rows_down || longest <= 36) &&
@@ -123,6 +173,10 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
 
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
     const bool rows_gu = path & LK_MOE_ROWS_GATE_UP, rows_down = path & LK_MOE_ROWS_DOWN;
+    if ((path & LK_MOE_TILES) &&
+        lk_mmq_tiles_moe_fit(wtype_gu, gate, up, (int64_t)ffn * (hidden / 256) * fg->block_bytes, ffn, hidden, tokens, true) &&
+        lk_mmq_tiles_moe_fit(wtype_down, down, nullptr, (int64_t)hidden * (ffn / 256) * fd->block_bytes, hidden, ffn, rows, false))
+        return block_on_tiles(*fg, *fd, x, gate, up, down, choices, topk_weights, out, tokens, topk, n_experts, hidden, ffn, longest, scratch, s);
     const bool gated_later = !rows_gu && !rows_down && ffn % 32 == 0;   // the activation rides the second product's quantizer
     // the buffer's pieces
     size_t at = 0;

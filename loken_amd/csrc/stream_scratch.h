@@ -23,7 +23,7 @@ enum LkScratchUse {
     LK_SCRATCH_ROUTER,     // gate logits
     LK_SCRATCH_LINEAR,     // host linear: quantized rows
     LK_SCRATCH_FIXUP,      // tiled matmul: partial products of a cut K
-    LK_SCRATCH_TOKENS,     // wide tiles: token operands
+    LK_SCRATCH_TOKENS,     // f16 tiles: token operands
     LK_SCRATCH_USES
 };
 

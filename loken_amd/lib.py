@@ -12,7 +12,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libloken_gfx950.so"
 LK_OK, LK_ERR_ARG, LK_ERR_TYPE, LK_ERR_LAUNCH, LK_ERR_NOMEM, LK_ERR_SIZE, LK_NOT_TAKEN = 0, 1, 2, 3, 4, 5, 6
 _ERR_NAMES = {1: "LK_ERR_ARG", 2: "LK_ERR_TYPE", 3: "LK_ERR_LAUNCH", 4: "LK_ERR_NOMEM", 5: "LK_ERR_SIZE", 6: "LK_NOT_TAKEN"}
 STATIC_SCRATCH_BYTES = 8 << 20
-MOE_GROUPED, MOE_ROWS_GATE_UP, MOE_ROWS_DOWN = 1, 2, 4
+MOE_GROUPED, MOE_ROWS_GATE_UP, MOE_ROWS_DOWN, MOE_TILES = 1, 2, 4, 8
 
 TYPE_F32, TYPE_F16, TYPE_BF16 = 0, 1, 30
 TYPE_Q4_0, TYPE_Q4_1, TYPE_Q5_0, TYPE_Q5_1 = 2, 3, 6, 7

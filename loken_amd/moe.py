@@ -457,7 +457,7 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
             raise _lib.LokenError("lk_moe_forward", status)
     path = _lib.load().lk_moe_block_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn)
     if path & _lib.MOE_GROUPED:
-        plan = MmqRouting.from_choices(choices, n_experts)
+        plan = MmqRouting.from_choices(choices, n_experts).with_tile_width(128 if path & _lib.MOE_TILES else 0)
         h = plan.with_path("rows" if path & _lib.MOE_ROWS_GATE_UP else "tiled").gate_up_silu(wtype_gu, x, gate, up, ffn)
         out = plan.with_path("rows" if path & _lib.MOE_ROWS_DOWN else "tiled").down_fold(wtype_down, h, down, hidden,
                                                                                        topk_weights.reshape(-1))

@@ -14,7 +14,7 @@ torch = pytest.importorskip("torch")
 import oracle
 from loken_amd import lib, moe, ops, synth
 from loken_amd.moe import MmqRouting
-from moe_block_check import check_block
+from moe_block_check import check_block, down_fold_from_rows
 
 pytestmark = pytest.mark.gpu
 RTOL, ATOL = 1e-3, 1e-4
@@ -625,6 +625,42 @@ def test_block_launch_by_launch_makes_the_choices_of_the_one_call(tokens, topk, 
     ids, w = oracle.topk_softmax(synth.activation(tokens, n_experts, seed=67, stream=7), topk)
     args = (lib.TYPE_Q4_K, dn, x, gate, up, down, dev(ids), dev(w), n_experts, ffn)
     assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
+
+
+# runs around every edge of the token tiles (one to three of 32, then several tiles), none at all, and one far longer than expected
+RUNS = [1, 32, 33, 64, 65, 96, 97, 128, 129, 0, 200, 31, 2, 95, 63, 34]
+
+
+@pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q4_K, lib.TYPE_Q4_K), (lib.TYPE_Q4_K, lib.TYPE_Q6_K), (lib.TYPE_Q6_K, lib.TYPE_Q6_K),
+                                   (lib.TYPE_Q5_K, lib.TYPE_Q5_K), (lib.TYPE_Q6_K, lib.TYPE_Q5_K)])
+@pytest.mark.parametrize("runs,hidden,ffn", [(RUNS, 256, 256), (RUNS, 768, 512), ([3] * 40 + [150] + [0, 1] * 11 + [12], 512, 256)])
+def test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn):
+    """Both products on the f16 tiles, operands gathered and handed on between them: the bits of the same launches through
+    workspace records and f32 rows, and the oracle's block."""
+    n_experts, tokens = len(runs), sum(runs)
+    ids = np.random.default_rng(68).permutation(np.repeat(np.arange(n_experts, dtype=np.int32), runs)).reshape(tokens, 1)
+    ids = np.concatenate([ids, np.roll(ids, 7, axis=0)], axis=1)
+    w = np.abs(synth.activation(tokens, 2, seed=68)) + np.float32(0.1)
+    if not lib.load().lk_moe_block_path(gu, dn, tokens, 2, n_experts, hidden, ffn) & lib.MOE_TILES:
+        pytest.skip("runs this short take other launches")
+    gate, up = (synth.weight(gu, n_experts * ffn, hidden, seed=68, stream=i) for i in (1, 2))
+    down = synth.weight(dn, n_experts * hidden, ffn, seed=68, stream=3)
+    x = synth.activation(tokens, hidden, seed=69)
+    args = (gu, dn, dev(x), dev(gate), dev(up), dev(down), dev(ids), dev(w), n_experts, ffn)
+    got, rows = moe_forward(*args, return_rows=True)
+    assert torch.equal(moe_forward(*args), got)
+    sample = np.arange(0, tokens, 9)
+    slabs = [np.ascontiguousarray(m).reshape(n_experts, -1) for m in (gate, up)]
+    pairs = (sample[:, None] * 2 + np.arange(2)).reshape(-1)
+    h = rows.cpu().numpy()[pairs]
+    for p, hp in zip(pairs, h):
+        e, row = ids[p // 2, p % 2], x[p // 2][None, :]
+        g, u = (oracle.ob_matmul(gu, row, s[e], ffn)[0].astype(np.float64) for s in slabs)
+        want = g / (1.0 + np.exp(-g)) * u
+        assert (np.abs(hp - want) <= 1e-3 * np.abs(want) + 1e-4 * max(1.0, np.abs(want).max())).all()
+    fed = down_fold_from_rows(dn, h, down, ids[sample], w[sample], n_experts, hidden)
+    bound = 1e-3 * np.abs(fed) + 1e-4 * max(1.0, np.abs(fed).max())
+    assert (np.abs(got.cpu().numpy()[sample] - fed) <= bound).all()
 
 
 @pytest.mark.parametrize("n,n_experts,topk", [(1, 3, 1), (63, 5, 3), (64, 1, 1), (1025, 130, 5), (4097, 512, 1), (8888, 128, 8)])
