@@ -75,17 +75,21 @@ constexpr int64_t MMQ_FIXUP_BYTES = 256ll * 128 * 128 * 4;
 // the kernel cuts K of a matrix whose row count is no multiple of four, or into a destination of any alignment, too
 // (11003 x 4096 at 77 rows, quantizer included: Q4_K 63 -> 40 us, Q5_K 73 -> 44, Q6_K 89 -> 51).
 __host__ __device__ static inline int64_t mmq_part_stride(const MmqProblem& pb) { return ((int64_t)pb.n + 3) / 4 * 4; }
-static inline int mmq_splits(const MmqProblem& pb, int64_t tiles, int64_t slots, const void* fixup, bool ragged = false) {
-    const int forced = lk_tune_env("LK_TUNE_MMQ_SPLITS");   // measurement runs: -1 never, n > 0 that many where they fit
-    if (!fixup || forced < 0 || pb.ids_dst || pb.m_begin != 0) return 1;
+// The most ranges K may be cut into: two blocks each, their partial products in the buffer; 1 where it stays whole.
+static inline int mmq_splits_most(const MmqProblem& pb, const void* fixup, bool ragged = false) {
+    if (!fixup || pb.ids_dst || pb.m_begin != 0) return 1;
     const bool f32 = pb.out_type == LK_TYPE_F32;
     if (!ragged && (pb.n % 4 != 0 || (f32 && (pb.ldd % 4 != 0 || (uintptr_t)pb.dst % 16 != 0)))) return 1;
     if ((uintptr_t)fixup % 16 != 0) return 1;
-    const int64_t fit = MMQ_FIXUP_BYTES / ((int64_t)pb.m_end * mmq_part_stride(pb) * 4);
-    int64_t want = forced > 0 ? forced : slots / tiles;
-    if (want > fit) want = fit;
-    if (want > pb.nb / 2) want = pb.nb / 2;
-    return want < 2 ? 1 : (int)want;
+    int64_t most = MMQ_FIXUP_BYTES / ((int64_t)pb.m_end * mmq_part_stride(pb) * 4);
+    if (most > pb.nb / 2) most = pb.nb / 2;
+    return most < 2 ? 1 : (int)most;
+}
+static inline int mmq_splits(const MmqProblem& pb, int64_t tiles, int64_t slots, const void* fixup) {
+    const int forced = lk_tune_env("LK_TUNE_MMQ_SPLITS");   // measurement runs: -1 never, n > 0 that many where they fit
+    if (forced < 0) return 1;
+    const int64_t want = forced > 0 ? forced : slots / tiles, most = mmq_splits_most(pb, fixup);
+    return want < 2 ? 1 : (int)(want < most ? want : most);
 }
 // dst[token][c] = part[0][token][c] + part[1][token][c] + ..., part[i] m_end x mmq_part_stride floats; LK_* status.
 int lk_mmq_split_sum(const float* part, int splits, const MmqProblem& pb, hipStream_t s);

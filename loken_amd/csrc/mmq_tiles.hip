@@ -45,33 +45,44 @@ __global__ __launch_bounds__(256) void operands_quantize_kernel(const T* __restr
     operand_quad(v, ops.codes + at * LK_OPERAND_CODES, ops.tabs + at * LK_OPERAND_TAB, (i0 / 32) & 7, (i0 / 4) & 7);
 }
 
-// Nanoseconds an item (32 x 32 x 32 product) takes a SIMD: `full` with two workgroups on every CU, `alone` with one, by token
-// tiles; measured on MI355X, whole launches less the 5 us that starting and ending one takes. wide: eight waves, tt = 4.
+// What a launch takes, fitted to 3000 calls on MI355X (7 shapes of 2048 x 2048 to 14336 x 4096 and 4096 x 14336, 33 to 2048 rows,
+// every tile width with K whole and cut into 2 to 12 ranges; the fit is off by 3 to 4 %, the plan it picks takes 1 to 2 % longer than
+// the best one of the sweep). alone / full: nanoseconds an item (32 x 32 x 32 product) takes a SIMD with one workgroup on its CU or two, by token
+// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items.
 struct ItemTimes {
-    double full[4], alone[4], wide;
+    double alone[4], full[4], wide, start;
 };
-constexpr ItemTimes ONE_TERM = {{115, 98.6, 97, 90.7}, {177, 116, 104, 92}, 88}, TWO_TERMS = {{172, 145, 128.6, 121}, {240, 158, 136, 123}, 0};
+constexpr ItemTimes ONE_TERM = {{164, 105, 104, 89}, {129, 98, 87.5, 82.7}, 80, 0.6}, TWO_TERMS = {{263, 144, 159, 143}, {194, 134, 122.5, 118}, 0, 3.1};
 
-// The tile with the shortest estimated launch: rounds of workgroups, and what a cut K costs in partial products (written, read
-// and added at 4 TB/s by a launch of 3 us).
+// The tile and the cut of K with the shortest estimated launch. Up to 2 * cus workgroups run at once, and a CU that holds two takes
+// nearly the time of a full chip; past that the rounds blur (0.6 of whole rounds, 0.4 of their share). A cut costs a launch and
+// its partial products, written, read and added.
 MmqTilePlan plan_dense(int wtype, const MmqProblem& pb, const void* fixup) {
     const ItemTimes& t = wtype == LK_TYPE_Q6_K ? TWO_TERMS : ONE_TERM;
     const int cus = lk_device().cus;
-    MmqTilePlan best{1, 4, 1};
+    const int forced_tt = lk_tune_env("LK_TUNE_MMQ_TT"), forced_splits = lk_tune_env("LK_TUNE_MMQ_SPLITS");   // measurement runs
+    const int most = forced_splits < 0 ? 1 : std::min(mmq_splits_most(pb, fixup, true), 12);
+    MmqTilePlan best{4, 4, 1};
     double least = 1e30;
     for (int tt = 1; tt <= 4; ++tt) {
+        if (forced_tt > 0 && tt != forced_tt) continue;
         const int64_t tiles = ((pb.n + 127ll) / 128) * ((pb.m_end + 32ll * tt - 1) / (32 * tt));
-        const int splits = mmq_splits(pb, tiles, 2 * cus, fixup, true);
-        const int64_t groups = tiles * splits, rounds = groups / (2 * cus), rest = groups % (2 * cus);
-        const double items = 8.0 * tt * ((pb.nb + splits - 1) / splits), one = items * t.alone[tt - 1], two = 2 * items * t.full[tt - 1];
-        double ns = rounds * two;
-        if (rest > 0) ns += rest <= cus ? one : one + (two - one) * (rest - cus) / cus;
-        if (splits > 1) ns += 3000 + (splits + 1.0) * pb.m_end * pb.n * 4 / 4000.0;
-        if (ns < least) least = ns, best = {tt, 4, splits};
+        for (int splits = forced_splits > 0 ? std::min(forced_splits, most) : 1; splits <= most; ++splits) {
+            const double items = 8e-3 * tt * ((pb.nb + splits - 1) / splits);
+            const double one = t.start + items * t.alone[tt - 1], two = t.start + 2 * items * t.full[tt - 1];
+            const int64_t groups = tiles * splits, rounds = groups / (2 * cus), rest = groups % (2 * cus);
+            double us = rounds * two;
+            if (rest > 0) us += rest <= cus ? one : one + (two - one) * (0.55 + 0.45 * (rest - cus) / cus);
+            if (rounds > 0) us = 0.6 * us + 0.4 * two * groups / (2 * cus);
+            if (splits > 1) us += 2.2 + 0.13e-6 * (splits + 1) * pb.m_end * pb.n * 4;
+            if (us < least) least = us, best = {tt, 4, splits};
+            if (forced_splits > 0) break;
+        }
     }
-    if (t.wide > 0) {
-        const int64_t tiles = ((pb.n + 255ll) / 256) * ((pb.m_end + 127ll) / 128);
-        if ((tiles + cus - 1) / cus * 64.0 * pb.nb * t.wide < least) best = {4, 8, 1};
+    if (t.wide > 0 && forced_splits <= 0 && (forced_tt <= 0 || forced_tt == 8)) {
+        const int64_t tiles = ((pb.n + 255ll) / 256) * ((pb.m_end + 127ll) / 128), rest = tiles % cus;
+        const double round = 64e-3 * pb.nb * t.wide;
+        if (round * (tiles / cus + (rest > 0 ? 0.85 + 0.15 * rest / cus : 0.0)) < least) best = {4, 8, 1};
     }
     return best;
 }
