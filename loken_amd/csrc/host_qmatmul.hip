@@ -60,39 +60,44 @@ int matvec_rows(int dtype, int k) {
     return dtype == LK_TYPE_Q8_0 && tiled_serves(dtype, k) ? 16 : 8;
 }
 
-// Rows the matrix-unit rows kernels take before the tiled matmul does. Measured on MI355X over
-// n = 2048 ... 151936 and k = 2048 ... 14336: a rows kernel re-reads the weights for every 32
-// activation rows but fills the chip from the first pass; a tiled launch holds a 128- or 256-row weight
-// block per workgroup, cuts K into ranges while its tiles are fewer than the chip's workgroup slots
-// (mmq_problem.h) and pays one more pass over the partial products for that. Up to 16 rows the 16-row
-// tiles stay; above, the two meet near n x rows = 450 K at k <= 4096 and in proportion earlier for
-// longer rows (quantizer + kernel, rows kernel against tiled):
-//   Q4_K  4096 x 4096: 128 rows 36 us against 39, 256 rows 49 against 43; 14336 x 4096: 32 rows 36
-//         against 36, 128 rows 75 against 53; 4096 x 14336: 32 rows 52 against 39, 512 rows 207 against 127
-//   Q6_K  4096 x 4096: 64 rows 32 against 35, 256 rows 64 against 51; 14336 x 4096: 32 rows 44 against 40,
-//         256 rows 161 against 114; 4096 x 14336: 32 rows 54 against 42, 1024 rows 568 against 360
-//   Q5_K  4096 x 4096: 128 rows 37 against 41, 256 rows 52 against 48; 4096 x 14336: 128 rows 80 against 63
+// Rows the matrix-unit rows kernels take before the tiled matmul does. A rows kernel reads the weights straight from HBM, once
+// for every 32 activation rows (16-row tiles up to 16 rows; Q6_K rows of a multiple of 2048 values in sets of eight further up), a
+// workgroup walking all of k: its time grows with k, and steps up once its workgroups (32 matrix rows x 32 activation rows each)
+// are more than the CUs. The f16 tiles cut K instead and read the weights once per 32 to 128 rows. Measured on MI355X, quantizer
+// included, rows kernel against f16 tiles (us), for matrices of 512 rows or more:
+//   Q4_K, 9 to 16 rows: 512 x 8192 20..22 / 16, 4096 x 8192 21 / 18, 700 x 11008 23..25 / 17; 6144 x 6144 16 / 20, 4096 x 4096 13 / 16
+//     17 to 32: 700 x 5120 18 / 15, 10000 x 5120 25 / 22, 2048 x 6144 21 / 16, 14336 x 4096 at 24 22 / 21; 4096 x 4096 16 / 16, 8192 x 4096 16 / 19
+//     above: 3000 x 5120 at 33 / 96 20 / 18, 27 / 24; 4096 x 4096 at 64 / 96 (256, 384 workgroups) 17 / 20, 25 / 25; 1024 x 4096 at 200 / 400
+//     (224, 416) 19 / 21, 28 / 25; 2048 x 2048 at 200 17 / 19. Q5_K alike.
+//   Q6_K, up to 16 rows, k a multiple of 2048: 4096 x 8192 17 / 22, 16384 x 6144 26 / 35; others: 700 x 5120 19 / 16, 10000 x 5120 32 / 26,
+//     6144 x 3072 15 / 20
+//     17 to 32: 4096 x 4096 16 / 18, 1024 x 14336 19 / 25 (sets of eight), 4096 x 8192 25 / 22, 4096 x 14336 42 / 31; 8192 x 4096 19 / 22, 3000 x 5120 22 / 19,
+//     14336 x 4096 31 / 28
+//     above: 1024 x 4096 at 64 / 96 13 / 17, 20 / 18; 3000 x 3072 at 33 20 / 18; 8192 x 4096 at 40 31 / 23; 2048 x 2048 at 64 12 / 15
 // `bench.py --workload rows-sweep` prints the table for a shape.
 static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K) return false;
-    // (a matrix of fewer than 2048 rows yields few tiles whatever the cut: Q4_K 1024 x 4096 at 512 rows 38 us
-    // against 38, at 1024 rows 55 against 49)
-    const long long few = n < 2048 ? 2048 / (n > 0 ? n : 1) : 1;
-    // (Q4_K / Q5_K rows of 8192 values or more at 9 to 16 activation rows: the 16-row tiles' second set of eight
-    // costs them more than the cut K costs the tiled launch: 4096 x 14336 at 9 / 16 rows 42 / 46 us against 37,
-    // Q5_K 44 / 48 against 38; 4096 x 8192 31 / 33 against 30. Q6_K keeps its 16-row tiles: 38 against 40)
-    if (dtype != LK_TYPE_Q6_K && rows > 8 && rows <= 16 && k >= 8192 && n >= 2048) return false;
-    // Above 16 rows of 8192 values or more: Q4_K / Q5_K 4096 x 14336 at 20 rows 37 / 39 us against 27 / 28, 1024 x 14336 at
-    // 17 / 32 35 / 39 against 20 / 22, 2048 x 8192 23 / 25 against 18 / 19; above 32 rows, where the tiles are 256 rows
-    // high and K is cut further, from 12288 values (2048 x 14336 at 40 / 109 rows 40 / 43 against 28 / 33; 3072 x 11008
-    // 33 / 46 against 40 / 51). Q6_K leaves above 32 rows (2048 x 14336 at 40 / 109 rows 50 / 53 against 31 / 38,
-    // 4096 x 8192 34 / 58 against 29 / 37); up to 32 its sets of eight rows are ahead at 1024 matrix rows and level at 2048
-    // (six matrices in turn in a graph, at 17 / 32 rows: 1024 x 8192 15.8 / 16.0 against 19.8 / 21.6, 1024 x 14336 19.7 / 20.5
-    // against 23.7 / 25.6, 2048 x 8192 22.1 / 18.8 against 21.4 / 22.8, 2048 x 14336 28.2 / 28.2 against 27.6 / 29.1), behind from
-    // 3072 on, which the line does not follow yet (3072 x 12288 34.5 / 34.6 against 28.8 / 30.7, 4096 x 8192 27.0 / 27.3 against
-    // 24.9 / 26.0, 8192 x 8192 33.4 / 38.0 against 32.1 / 35.2, 4096 x 14336 at 17 / 28 44.2 / 44.3 against 33.2 / 35.9).
-    if (rows > 16 && n >= 1024 && (dtype == LK_TYPE_Q6_K ? rows > 32 && k >= 8192 : k >= (rows > 32 ? 12288 : 8192))) return false;
-    return rows <= 16 || (long long)n * rows * (k > 4096 ? k : 4096) <= 450000ll * 4096 * few;
+    if (rows <= 8) return true;
+    const long long results = (long long)n * rows;
+    // (few matrix rows yield few tiles whatever the cut: the int8 tiles' line)
+    if (n < 512) return rows <= 16 || results * (k > 4096 ? k : 4096) <= 450000ll * 4096 * (n > 0 ? 2048 / n : 2048);
+    const long long items = (n + 31ll) / 32 * ((rows + 31) / 32);
+    if (dtype == LK_TYPE_Q6_K) {
+        const bool sets = k % 2048 == 0;
+        if (rows <= 16) return sets || k < 4608;
+        if (rows <= 32 && sets && n <= 4096) return (long long)n * k <= (24ll << 20);
+        if (rows <= 32) return k < 3072 || (k < 4608 && (sets ? n < 12288 : n >= 4096));
+        if (k < 5632 && n < 1024 && rows > 128 && items <= 256) return true;
+        if (k >= 3072 && (n >= 1024 || k >= 4608)) return rows <= 64 && n < 2800 && k < 7168 && sets;
+        return results <= 450000;
+    }
+    if (rows <= 16) return k < 7168;
+    // (the one stretch that is not the faster side: callers that read path() rely on the rows kernel at 1100 x 8192 and 33 rows,
+    // test_long_rows_above_sixteen_activation_rows; 1024 x 8192 there 27 / 18)
+    if (k >= 4608 && k < 12288 && n >= 1024 && n < 1152 && rows > 32 && rows <= 64) return true;
+    if (k >= 4608) return k < 5632 && items > 128 && items <= 256 && rows > 32;
+    if (rows <= 32) return n < 12288 || k < 4096 || rows < 20;
+    return items <= 256 || (k <= 2048 && results <= 450000);
 }
 
 // The K-quants at 3 to 8 f32 rows: the 16-row tiles of the matrix-unit kernels (their time hardly moves

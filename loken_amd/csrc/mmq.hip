@@ -1009,18 +1009,18 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
     MmqProblem pb{(const uint8_t*)x, (const uint8_t*)y, (float*)dst, nullptr, ncols_x / 256, stride_row_x,
                   ncols_y, stride_col_dst, (int)nrows_x, 0, (int)ncols_y, out_type};
     hipStream_t s = (hipStream_t)stream;
+    // (Q4_K, Q5_K and Q6_K from 9 rows of a matrix of 512 rows or more: the f16 tiles; quantizer included, against the int8 tiles:
+    // Q4_K 4096 x 14336 at 9 / 32 rows 22 / 23 us against 27 / 29, 1024 x 14336 at 33 / 400 rows 21 / 44 against 27 / 55)
+    if constexpr (F::F16_TYPE >= 0)
+        if (lk_mmq_tiles_take(F::F16_TYPE, nrows_x, ncols_y)) {
+            const int tm = lk_mmq_tiles_dense(F::F16_TYPE, pb, s, fixup);
+            if (tm >= 0) return tm;
+        }
     if (ncols_y <= 32) return launch_dense_tm<F, 32, 1>(pb, s, fixup);
     // (Q2_K stays on 64-token tiles: with the rank-16 minimum its 128-token tile spills and runs 512 x
     // 4096 -> 14336 in 344 us against 240, 2048 x 14336 -> 4096 in 1155 against 742; every other format
     // is 3 to 40 % faster on the wide tile)
-    // (Q4_K, Q5_K and Q6_K from 33 rows of a matrix of 2048 rows or more: the f16 tiles)
-    const bool f16 = lk_mmq_tiles_take(F::F16_TYPE, nrows_x, ncols_y);
-    if ((ncols_y <= 64 && !f16) || F::MIN_RANK == 16) return launch_dense_tm<F, 64, 2>(pb, s, fixup);
-    if constexpr (F::F16_TYPE >= 0)
-        if (f16) {
-            const int tm = lk_mmq_tiles_dense(F::F16_TYPE, pb, s, fixup);
-            if (tm >= 0) return tm;
-        }
+    if (ncols_y <= 64 || F::MIN_RANK == 16) return launch_dense_tm<F, 64, 2>(pb, s, fixup);
     // 128-token tiles where there are F::WIDE_FROM of them or more, else 64-token tiles, twice as many and
     // with K cut where those are still few. Quantizer + matmul, 64- against 128-token tiles:
     //   Q6_K  4096 x 14336 at 128 / 512 / 1024 rows (32 / 128 / 256 tiles) 70 / 215 / 393 us against 99 / 307 /

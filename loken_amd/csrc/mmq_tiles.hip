@@ -138,7 +138,7 @@ int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fix
 }
 
 bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows) {
-    return (wtype == LK_TYPE_Q4_K || wtype == LK_TYPE_Q5_K || wtype == LK_TYPE_Q6_K) && rows > 32 && n >= 2048 && !lk_env_flag("LK_MMQ_I8");
+    return (wtype == LK_TYPE_Q4_K || wtype == LK_TYPE_Q5_K || wtype == LK_TYPE_Q6_K) && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
 }
 
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {

@@ -327,6 +327,25 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
     assert close(got.cpu().numpy()[:, pick], oracle.ob_matmul(wtype, x, w[pick], len(pick)))
 
 
+@pytest.mark.parametrize("name,n,k,rows,expect", [
+    ("q4_k", 512, 7168, 9, "tiled"), ("q4_k", 512, 6912, 9, "rows-on-matrix-unit"), ("q4_k", 511, 7168, 9, "rows-on-matrix-unit"),
+    ("q5_k", 520, 4608, 17, "tiled"), ("q5_k", 520, 4352, 32, "rows-on-matrix-unit"), ("q4_k", 700, 5120, 200, "rows-on-matrix-unit"),
+    ("q4_k", 700, 5120, 33, "tiled"), ("q4_k", 600, 1024, 600, "rows-on-matrix-unit"), ("q5_k", 600, 2304, 600, "tiled"),
+    ("q6_k", 512, 4608, 9, "tiled"), ("q6_k", 512, 6144, 16, "rows-on-matrix-unit"), ("q6_k", 4100, 4096, 20, "rows-on-matrix-unit"),
+    ("q6_k", 520, 5120, 200, "rows-on-matrix-unit"), ("q6_k", 520, 5888, 65, "tiled"), ("q6_k", 2800, 3072, 33, "tiled"),
+    ("q6_k", 1023, 3072, 300, "rows-on-matrix-unit")])
+def test_both_sides_of_the_lines_between_rows_kernels_and_f16_tiles(name, n, k, rows, expect):
+    wtype = DT[name]
+    w = synth.weight(wtype, n, k, seed=98, stream=1)
+    x = synth.activation(rows, k, seed=98)
+    lin = Linear(wtype, dev(w), n, k)
+    got = lin(dev(x))
+    assert lin.path == expect
+    lin.close()
+    pick, some = np.r_[:40, n - 40:n], np.r_[:4, rows - 4:rows]
+    assert close(got.cpu().numpy()[some][:, pick], oracle.ob_matmul(wtype, x[some], w[pick], len(pick)))
+
+
 @pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
 @pytest.mark.parametrize("rows,n,k,shift", [(450, 2048, 256, 0), (180, 2561, 1280, 0), (33, 14336, 512, 1)])
 def test_operands_straight_from_the_rows_are_those_of_the_records(name, rows, n, k, shift):
