@@ -441,44 +441,29 @@ int launch(const Args& a, hipStream_t stream, int sets = 1) {
 
 int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                   hipStream_t stream, int out_type) {
-    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256) return -1;
+    if (size_m < 1 || size_m > 32 || size_n < 1 || size_k < 256) return -1;
     // rows of whole granules, on 16-byte boundaries; a tile's granules within one workgroup
     if (size_k % (256 * GRAN) != 0 || size_k / (256 * GRAN) > MAX_WAVES || (((uintptr_t)w) & 15) != 0) return -1;
     if (lk_tune_env("LK_TUNE_ROWS16_OFF") != 0) return -1;
     const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
     if (size_m > 8 && lk_tune_env("LK_TUNE_ROWS16_MAX8") != 0) return -1;
+    // (the short launch has taken the calls of few row tiles: rows16_q6k_short.hip)
     if (size_m <= 4) return launch<4>(a, stream);
     const int n_tiles = (size_n + TILE - 1) / TILE;
-    // 5..8 rows as two sets of four where that fills the chip sooner than eight at once: so few tiles that a
-    // workgroup per tile leaves half the CUs idle (2048 x 6144: 8.9 us against 10.7; 2048 x 14336 12.9 against
-    // 16.3), or a matrix small enough for its second reading to come from L2 at no cost (4096 x 4096 9.1 us
-    // against 10.3, 8192 x 2048 8.8 against 9.5, 6144 x 4096 11.7 against 12.7; 8192 x 4096, 27.5 MB, 12.2
-    // against 11.1 and stays with eight). (Sets: below.)
+    // 5..8 rows as two sets of four for a matrix small enough for its second reading to come from L2 at no cost (8192 x 2048 8.8 us
+    // against 9.5; 8192 x 4096, 27.5 MB, 12.2 against 11.1 and stays with eight). (Sets: below.)
     const size_t weight_bytes = (size_t)size_n * a.nb * Q6K_BYTES;
-    if (size_m <= 8)
-        return 2 * n_tiles <= lk_device().cus || weight_bytes <= ((size_t)22 << 20) ? launch<4>(a, stream, 2) : launch<8>(a, stream);
+    if (size_m <= 8) return weight_bytes <= ((size_t)22 << 20) ? launch<4>(a, stream, 2) : launch<8>(a, stream);
     // 9..32 rows. Sixteen at once when their codes fit LDS and the row tiles are several to the CU; else the
     // rows in sets of eight, a set per workgroup (grid.y), in one launch: rows too long for sixteen in LDS (k =
-    // 14336: 229 KB; 4096 x 14336 at 16 rows 25.7 us against 37.4 on the 32-row tiles that would take the
-    // call otherwise), up to two tiles to the CU, where twice the workgroups with half the staging each
-    // finish sooner (16 rows: 2048 x 6144 11.1 us against 15.9, 4096 x 4096 10.8 against 14.7, 8192 x 2048
-    // 10.4 against 13.2, 8192 x 4096 14.5 against 15.7; 11008 x 4096 28.2 against 23.8 and 14336 x 4096 27.2
-    // against 25.7 stay with sixteen at once), or 17..32 rows (2048 x 6144 at 32 rows 13.5 us against 22.4 on the 32-row
-    // tiles, 4096 x 4096 13.8 against 17.4, 4096 x 14336 42.7 against 47.4, 4096 x 8192 24.8 against 31.1).
-    // Every set reads the weights again, from L2 while they fit there, and three or four sets of more than a
+    // 14336: 229 KB), up to two tiles to the CU, where twice the workgroups with half the staging each
+    // finish sooner (16 rows: 8192 x 2048 10.4 us against 13.2, 8192 x 4096 14.5 against 15.7; 11008 x 4096 28.2 against 23.8 and 14336 x
+    // 4096 27.2 against 25.7 stay with sixteen at once), or 17..32 rows (4096 x 4096 13.8 against 17.4 on the 32-row tiles, 4096 x 8192
+    // 24.8 against 31.1). Every set reads the weights again, from L2 while they fit there, and three or four sets of more than a
     // tile to the CU are too many workgroups: above 16 rows a matrix of more than 64 MB or of more tiles
     // than CUs stays with the 32-row tiles (at 32 rows 151936 x 2048 173 us against 99, 6144 x 4096 25.8
     // against 18.4, 14336 x 4096 39.7 against 32.4).
     if (size_m > 16 && (n_tiles > lk_device().cus || weight_bytes > ((size_t)64 << 20))) return -1;
-    // 33..64 rows: only as whole rounds of workgroups that are all resident at two to the CU, one round or
-    // exactly two (2048 x 6144 at 64 rows, 128 tiles x 8 sets: 18.7 us against 22.3 on the 32-row tiles; at
-    // 40..56 rows, a second round partly filled, 24 against 22.2; 1024 x 2048, 64 tiles, 9.5 against 12.0 at 64
-    // rows and 10.3 against 11.8 at 40)
-    if (size_m > 32) {
-        const int total = n_tiles * ((size_m + 7) / 8), cus = lk_device().cus;
-        const bool two_per_cu = lds_bytes_for<8>(a.nb, a.nb / GRAN) <= lk_device().lds_bytes / 2 && a.nb / GRAN <= 8;
-        if (!two_per_cu || (total > 2 * cus && total != 4 * cus)) return -1;
-    }
     if (size_m <= 16 && n_tiles > 2 * lk_device().cus) {
         const int rc = launch<16>(a, stream);
         if (rc != -1) return rc;

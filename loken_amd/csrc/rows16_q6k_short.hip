@@ -1,0 +1,236 @@
+// Q6_K weights x at most sixteen Q8_1 activation rows (more as sets) where there are few 16-row tiles: the short launch of the
+// 16-row family (rows16_q6k.hip has the arithmetic's description: one instruction's four lane groups hold four 16-value groups
+// of a row, the activation live in the lanes of one group or of one of two).
+//
+// What bounds it: a `down` projection of a small model (2048 x 6144, 10 MB) is 128 row tiles, so a launch is over in about the
+// time of one load, one wave's arithmetic and one reduction, whatever the bytes. rows16_q6k.hip hands a wave a granule of eight
+// super-blocks, which makes that arithmetic eight steps long with three waves on a CU (11.1 us a launch at 16 rows in a
+// graph, of which 2 are a launch that does nothing; now 8.3). Here a tile's super-blocks go to up to twelve waves (168 registers each), every load of the first two in flight at once; nothing is staged for the workgroup, so no barrier stands before the
+// arithmetic: a wave reads the activation codes of its own super-blocks straight into the operand's lanes (sixteen bytes of one
+// row), and turns the weights and the eight scales per row through a buffer of its own.
+//
+// Any super-block may be a wave's, so its bytes start at any even phase of a 16-byte piece, another one for each row: the row's
+// fourteen pieces are written to the buffer so that the block starts at byte 16 or 18, and a lane shifts what it reads by its row's
+// zero or two bytes. Rows of any number of super-blocks are served.
+
+#include "lk_common.h"
+#include "rows16.h"
+
+namespace {
+
+constexpr int TILE = 16, MAX_WAVES = 12;
+constexpr int BLOCK_PIECES = 14;              // 16-byte pieces that hold a super-block, at any even phase
+constexpr int PITCH = 16 + 16 * BLOCK_PIECES + 32;   // bytes between the rows of a wave's buffer: 16 rows on 16 bank groups
+constexpr int ROWS_BYTES = TILE * PITCH;
+constexpr int WAVE_BYTES = ROWS_BYTES + 8 * 16 * 4;   // and d8 [8][TOKS] of the super-block
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+
+struct Args {
+    const uint8_t* w;     // 16-byte aligned
+    const uint8_t* y;     // Q8_1 rows
+    float* dst;
+    int nb, n, m;         // super-blocks per weight row, weight rows, activation rows
+    int stride_y;         // Q8_1 blocks between activation rows
+    int ldd;              // elements between output rows
+    int out_type;         // element type of `dst` (lk_store_as)
+};
+
+// grid (row tiles, sets of TOKS activation rows), 64 * waves threads: wave w takes super-blocks w, w + waves, ...
+template <int TOKS, bool HALF>
+__global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Args p) {
+    static_assert(TOKS == 8 || TOKS == 16, "sets of eight or sixteen activation rows");
+    constexpr bool T16 = TOKS == 16;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
+    const int tile = (int)blockIdx.x, m0 = (int)blockIdx.y * TOKS, m_rows = min(TOKS, p.m - m0);
+    const int last_row = min(TILE, p.n - tile * TILE) - 1;
+    const int row_bytes = p.nb * Q6K_BYTES;
+    uint8_t* buf = lds + wave * WAVE_BYTES;
+    float* table = (float*)(buf + ROWS_BYTES);
+
+    // ---- the weights: load u of a super-block is piece 64 u + lane of its 16 x 14 (sixteen rows are whole pieces: a tile is aligned)
+    constexpr int LOADS = (TILE * BLOCK_PIECES + 63) / 64;   // 4, the last half used
+    const uint8_t* w_tile = (const uint8_t*)(to_gbytes(p.w) + (size_t)tile * TILE * row_bytes);
+    uint32_t w_at[LOADS], w_piece[LOADS];
+    int w_to[LOADS];
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) {
+        const int id = min(64 * u + lane, TILE * BLOCK_PIECES - 1), row = id / BLOCK_PIECES;
+        w_piece[u] = (uint32_t)(16 * (id % BLOCK_PIECES));
+        w_at[u] = (uint32_t)(min(row, last_row) * row_bytes);
+        w_to[u] = row * PITCH + 16 * (id % BLOCK_PIECES) + 16;
+    }
+    const uint32_t my_at = (uint32_t)(min(l16, last_row) * row_bytes);   // of the lane's own row
+    // ---- the activation: the lane's sixteen codes of unit u (values 64 u + 16 grp ..), the scales it puts in the table
+    const int tok = l16 & (TOKS - 1), sel = l16 / TOKS;
+    const uint8_t* y0 = p.y + (size_t)m0 * p.stride_y * Q81_BYTES;
+    const uint32_t y_codes = (uint32_t)((min(tok, m_rows - 1) * p.stride_y + (grp >> 1)) * Q81_BYTES + 4 + 16 * (grp & 1));
+    constexpr int HEADS = T16 ? 2 : 1;
+    const int h_tok = lane & (TOKS - 1), h_sub = (lane / TOKS) & 7;
+    const uint32_t y_head = (uint32_t)((min(h_tok, m_rows - 1) * p.stride_y + h_sub) * Q81_BYTES);
+    const float h_real = h_tok < m_rows ? 1.f : 0.f;
+    // eight rows: the lanes whose codes the first and the second instruction see
+    const uint32_t keep0 = grp == sel ? ~0u : 0u, keep1 = grp == sel + 2 ? ~0u : 0u;
+    // the lane's results: eight rows: groups grp / 2 and 2 + grp / 2, rows 4 (grp % 2) + v; sixteen: every group, rows 4 grp + v
+    const float* t_lane = T16 ? table + 4 * grp : table + 4 * (grp & 1);
+    const int sh_sc = T16 ? 0 : 8 * (grp >> 1), sh_qh = 2 * (grp >> 1);
+
+    struct Block {
+        u32x4 w[LOADS], a[4];
+        uint32_t head[HEADS];
+    };
+    auto load = [&](Block& b, int kb) {
+        const uint32_t at = (uint32_t)(kb * Q6K_BYTES), ya = (uint32_t)(kb * 8 * Q81_BYTES);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b.a[u] = *(const u32x4_a4*)(y0 + (y_codes + ya) + 2 * u * Q81_BYTES);
+#pragma unroll
+        for (int h = 0; h < HEADS; ++h) b.head[h] = *(const uint32_t*)(y0 + (y_head + ya) + 4 * h * Q81_BYTES);
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) b.w[u] = *(const u32x4*)(w_tile + (((w_at[u] + at) & ~15u) + w_piece[u]));
+    };
+
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const Block& b, int kb) {
+        const uint32_t at = (uint32_t)(kb * Q6K_BYTES);
+        auto settle = [] {   // the wave's own LDS writes before its reads of other lanes' data
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+#pragma unroll
+        for (int h = 0; h < HEADS; ++h)
+            table[(h_sub + 4 * h) * TOKS + h_tok] = h_real * f16_bits_to_f32(b.head[h] & 0xFFFFu);
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u)
+            if (64 * u + lane < TILE * BLOCK_PIECES) *(u32x4_a4*)(buf + (w_to[u] - (int)((w_at[u] + at) & 12u))) = b.w[u];
+        settle();
+        const uint8_t* mine = buf + l16 * PITCH + 16;
+        const uint32_t sh = (my_at + at) & 2u;
+        auto piece_at = [&](int c, uint32_t& past) {   // sixteen bytes at byte c of the super-block; the four after them, unshifted
+            const u32x4 lo = *(const u32x4*)(mine + c);
+            past = *(const uint32_t*)(mine + c + 16);
+            return u32x4{__builtin_amdgcn_alignbyte(lo[1], lo[0], sh), __builtin_amdgcn_alignbyte(lo[2], lo[1], sh),
+                         __builtin_amdgcn_alignbyte(lo[3], lo[2], sh), __builtin_amdgcn_alignbyte(past, lo[3], sh)};
+        };
+        uint32_t past;
+        const u32x4 sc = piece_at(192, past);
+        const float d = f16_bits_to_f32((past >> (8 * sh)) & 0xFFFFu);
+        // (accumulators from the bit pattern of 1.5 * 2^23, the offset off again in the first fused multiply-add, exactly: rows16_q6k.hip)
+        constexpr int MAGIC_BITS = 0x4B400000;
+        constexpr float MAGIC = 12582912.0f;
+        const v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
+        auto fold = [&](const v4i& c, float dsc, int sub) {
+            const float off = -MAGIC * dsc;
+            const float4 t = *(const float4*)(t_lane + sub * TOKS);
+            acc[0] = fmaf(fmaf(__int_as_float(c[0]), dsc, off), t.x, acc[0]);
+            acc[1] = fmaf(fmaf(__int_as_float(c[1]), dsc, off), t.y, acc[1]);
+            acc[2] = fmaf(fmaf(__int_as_float(c[2]), dsc, off), t.z, acc[2]);
+            acc[3] = fmaf(fmaf(__int_as_float(c[3]), dsc, off), t.w, acc[3]);
+        };
+        u32x4 ql, qhp;
+#pragma unroll
+        for (int unit = 0; unit < 4; ++unit) {
+            if (unit % 2 == 0) {
+                ql = piece_at(32 * unit + 16 * grp, past);
+                qhp = piece_at(128 + 16 * unit + 16 * (grp & 1), past) >> (uint32_t)sh_qh;
+            }
+            v4i codes;   // the lane's sixteen signed codes: group 4 unit + grp of the row
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t nib = (unit & 1 ? ql[e] >> 4 : ql[e]) & 0x0F0F0F0Fu;
+                const uint32_t up = (unit & 1 ? qhp[e] : qhp[e] << 4) & 0x30303030u;
+                codes[e] = (int)(((nib | up) + 0x60606060u) ^ 0x80808080u);
+            }
+            const uint32_t scw = sc[unit] >> (uint32_t)sh_sc;
+            if constexpr (T16) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {   // the activation of group g alone
+                    v4i a;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) a[e] = grp == g ? (int)b.a[unit][e] : 0;
+                    const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, codes, magic, 0, 0, 0);
+                    fold(c, d * (float)(int)__builtin_amdgcn_sbfe(scw, 8 * g, 8), 2 * unit + (g >> 1));
+                }
+            } else {
+                v4i a0, a1;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a0[e] = (int)(b.a[unit][e] & keep0), a1[e] = (int)(b.a[unit][e] & keep1);
+                fold(__builtin_amdgcn_mfma_i32_16x16x64_i8(a0, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 0, 8), 2 * unit);
+                fold(__builtin_amdgcn_mfma_i32_16x16x64_i8(a1, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 16, 8), 2 * unit + 1);
+            }
+            // one unit at a time (left free, the compiler keeps all the result tiles alive and runs out of registers)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) asm volatile("" : "+v"(acc[v]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        settle();
+    };
+
+    Block ring[2];
+    load(ring[0], wave);
+    if (wave + waves < p.nb) load(ring[1], wave + waves);
+    for (int kb = wave; kb < p.nb; kb += 2 * waves) {
+        compute(ring[0], kb);
+        if (kb + 2 * waves < p.nb) load(ring[0], kb + 2 * waves);
+        if (kb + waves < p.nb) {
+            compute(ring[1], kb + waves);
+            if (kb + 3 * waves < p.nb) load(ring[1], kb + 3 * waves);
+        }
+    }
+
+    // the partial tiles, [4][64] floats at the start of each wave's buffer
+    float* part = (float*)buf;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) part[v * 64 + lane] = acc[v];
+    __syncthreads();
+    // sixteen rows: output (register v, lane l < 64) adds the waves' lanes l; eight: (v, l < 32) lanes l and l + 32
+    constexpr int LANES = 4 * TOKS;
+    for (int o = threadIdx.x; o < 4 * LANES; o += (int)blockDim.x) {
+        const int v = o / LANES, l = o % LANES;
+        float sum = 0.f;
+        for (int w = 0; w < waves; ++w) {
+            const float* col = (const float*)(lds + w * WAVE_BYTES) + v * 64 + l;
+            sum += T16 ? col[0] : col[0] + col[32];
+        }
+        const int t = 4 * (l >> 4) + v, row = l & 15;
+        if (t < m_rows && row <= last_row) lk_store_as(p.dst, (size_t)(m0 + t) * p.ldd + tile * TILE + row, sum, HALF ? p.out_type : LK_TYPE_F32);
+    }
+}
+
+template <int TOKS, bool HALF>
+int launch(const Args& a, int waves, hipStream_t stream) {
+    static const bool ok = hipFuncSetAttribute((const void*)q6k_rows16_short_kernel<TOKS, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               MAX_WAVES * WAVE_BYTES) == hipSuccess;
+    if (!ok) return -1;
+    hipLaunchKernelGGL((q6k_rows16_short_kernel<TOKS, HALF>), dim3((a.n + TILE - 1) / TILE, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
+                       waves * WAVE_BYTES, stream, a);
+    return lk_launch_status();
+}
+
+}  // namespace
+
+int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
+                        hipStream_t stream, int out_type) {
+    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || (((uintptr_t)w) & 15) != 0) return -1;
+    // One workgroup fits a CU (registers), and a second round of them costs what the first did, so the line is the number of
+    // workgroups. Eight rows to a set where that is one round, sixteen otherwise. Measured in a graph, us, the granules
+    // of rows16_q6k.hip (rows of a multiple of 2048 values; more rows than it takes: the 32-row tiles) against this:
+    //   up to 8 rows    1024 x 2048 7.3 / 4.2, 2048 x 6144 9.0 / 8.0, 4096 x 4096 9.3 / 7.1, 6144 x 2048 9.7 / 7.5, 8192 x 4096 12.1 / 12.7
+    //   9 to 16         1024 x 2048 9.2 / 4.3, 2048 x 6144 11.1 / 8.3, 4096 x 4096 10.8 / 8.4, 4096 x 14336 25.6 / 20.0, 8192 x 4096 15.0 / 15.1
+    //   17 to 32        1024 x 2048 9.3 / 4.4, 2048 x 6144 13.2 / 10.0, 4096 x 4096 13.3..13.8 / 12.9..14.5, 4096 x 14336 41 / 32..36 (over 64 MB)
+    //   33 to 64        1024 x 2048 10.1 / 5.0, 2048 x 6144 at 48 / 64 22.2, 18.1 / 17.9, 18.2, 2048 x 14336 46 / 34, 4096 x 4096 17.5 / 20.1
+    // and against the 32-row tiles where rows are no granules: 700 x 11008 at 8 / 16 / 32 / 64 rows 32, 37, 43, 43 / 10, 11, 11, 14;
+    // 10000 x 5120 at 8 / 16 / 32 25, 31, 37 / 21, 26, 41; 16384 x 3072 at 8 / 16 16.9, 20.3 / 17.9, 20.9; 3000 x 5120 at 32 / 64 19.8, 20.4 / 16.9, 24.4
+    const int nb = size_k / 256, tiles = (size_n + TILE - 1) / TILE, cus = lk_device().cus;
+    const bool granules = nb % 8 == 0, held = granules && tiles <= cus && (size_t)size_n * nb * Q6K_BYTES <= (64u << 20);
+    const int eights = (size_m + 7) / 8, sixteens = (size_m + 15) / 16;
+    const int64_t most = size_m <= 16 ? (granules ? 3 * cus / 2 : 3 * cus) : size_m > 32 ? 2 * cus : held ? cus : granules ? 2 * cus : 3 * cus;
+    const bool by_eight = size_m <= 8 || (int64_t)tiles * eights <= cus;
+    if ((int64_t)tiles * (by_eight ? eights : sixteens) > most) return -1;
+    const int steps = (nb + MAX_WAVES - 1) / MAX_WAVES, waves = (nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow
+    const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, nb, size_n, size_m, stride_y, ldd, out_type};
+    if (by_eight) return out_type == LK_TYPE_F32 ? launch<8, false>(a, waves, stream) : launch<8, true>(a, waves, stream);
+    return out_type == LK_TYPE_F32 ? launch<16, false>(a, waves, stream) : launch<16, true>(a, waves, stream);
+}

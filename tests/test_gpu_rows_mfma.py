@@ -315,6 +315,19 @@ def test_q6k_eight_rows_or_fewer_in_sixteen_row_tiles(m, k, n):
     assert_close(got, oracle.ob_matmul(Q6K, x, w, n))
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 3328, 5), (8, 3072, 16), (9, 3328, 31), (16, 6400, 100), (7, 2304, 6150), (16, 1792, 6100), (15, 4096, 2080),
+                                   (32, 4096, 1030), (20, 4096, 4000), (23, 2816, 5200), (64, 1280, 2048), (33, 11008, 700), (7, 4096, 8200),
+                                   (3, 2048, 8200)])
+def test_q6k_where_the_short_launch_takes_and_leaves(m, k, n):
+    """rows16_q6k_short.hip: super-blocks at every even phase of a 16-byte piece, one to four of them a wave, waves without a last one,
+    sets of eight and of sixteen rows with a last set of one, and both sides of its line in row tiles."""
+    w = synth.weight(Q6K, n, k, seed=79, stream=1)
+    x = synth.activation(m, k, seed=79)
+    got = ops.dense_q6k_rows(dev(w), dev(x), n).cpu().numpy()
+    pick = np.unique(np.r_[:min(n, 40), max(0, n - 40):n])
+    assert_close(got[:, pick], oracle.ob_matmul(Q6K, x, w[pick], len(pick)))
+
+
 @pytest.mark.parametrize("k", [1024, 4096])
 @pytest.mark.parametrize("m", [3, 4, 7, 11, 16, 21, 32])
 def test_q6k_few_rows_emit_the_exact_integers_on_crafted_inputs(m, k):
