@@ -18,6 +18,10 @@ struct LkRows16 {
 // True when the launch takes `size_m` activation rows of `nb` super-blocks (their codes fit in LDS).
 bool lk_rows16_serves(int size_m, int nb);
 int lk_rows16_launch(const LkRows16& a, bool dual, bool q5, hipStream_t stream);
+// The same (rows16_short.hip) for matrices of few row tiles: a tile to a workgroup, any number of super-blocks.
+// Its sums do not depend on what else the launch holds, nor on `dual`, so all launches over a matrix choose by lk_rows16_short_pays.
+int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream);
+bool lk_rows16_short_pays(int m, int n, int nb);
 
 // Q4_K per expert over a sorted routing, a wave per 16-row tile (rows16_moe.hip): expert e's matrices are
 // a.w[..] + e * expert_bytes (a.n[0] rows each, a.w[1] with `dual`), its rows the sorted rows

@@ -92,7 +92,9 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         for (int u = 0; u < LOADS; ++u) b.w[u] = *(const u32x4*)(w_tile + (((w_at[u] + at) & ~15u) + w_piece[u]));
     };
 
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    // eight rows: the lane's sums of groups 0 and 2 or 1 and 3 of each four; sixteen: of both, apart, so that either form adds the same
+    // numbers in the same order and a launch may choose
+    float acc[T16 ? 2 : 1][4] = {};
     auto compute = [&](const Block& b, int kb) {
         const uint32_t at = (uint32_t)(kb * Q6K_BYTES);
         auto settle = [] {   // the wave's own LDS writes before its reads of other lanes' data
@@ -121,13 +123,13 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         constexpr int MAGIC_BITS = 0x4B400000;
         constexpr float MAGIC = 12582912.0f;
         const v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
-        auto fold = [&](const v4i& c, float dsc, int sub) {
+        auto fold = [&](float (&sum)[4], const v4i& c, float dsc, int sub) {
             const float off = -MAGIC * dsc;
             const float4 t = *(const float4*)(t_lane + sub * TOKS);
-            acc[0] = fmaf(fmaf(__int_as_float(c[0]), dsc, off), t.x, acc[0]);
-            acc[1] = fmaf(fmaf(__int_as_float(c[1]), dsc, off), t.y, acc[1]);
-            acc[2] = fmaf(fmaf(__int_as_float(c[2]), dsc, off), t.z, acc[2]);
-            acc[3] = fmaf(fmaf(__int_as_float(c[3]), dsc, off), t.w, acc[3]);
+            sum[0] = fmaf(fmaf(__int_as_float(c[0]), dsc, off), t.x, sum[0]);
+            sum[1] = fmaf(fmaf(__int_as_float(c[1]), dsc, off), t.y, sum[1]);
+            sum[2] = fmaf(fmaf(__int_as_float(c[2]), dsc, off), t.z, sum[2]);
+            sum[3] = fmaf(fmaf(__int_as_float(c[3]), dsc, off), t.w, sum[3]);
         };
         u32x4 ql, qhp;
 #pragma unroll
@@ -151,18 +153,21 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
 #pragma unroll
                     for (int e = 0; e < 4; ++e) a[e] = grp == g ? (int)b.a[unit][e] : 0;
                     const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, codes, magic, 0, 0, 0);
-                    fold(c, d * (float)(int)__builtin_amdgcn_sbfe(scw, 8 * g, 8), 2 * unit + (g >> 1));
+                    fold(acc[T16 ? g & 1 : 0], c, d * (float)(int)__builtin_amdgcn_sbfe(scw, 8 * g, 8), 2 * unit + (g >> 1));
                 }
             } else {
                 v4i a0, a1;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) a0[e] = (int)(b.a[unit][e] & keep0), a1[e] = (int)(b.a[unit][e] & keep1);
-                fold(__builtin_amdgcn_mfma_i32_16x16x64_i8(a0, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 0, 8), 2 * unit);
-                fold(__builtin_amdgcn_mfma_i32_16x16x64_i8(a1, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 16, 8), 2 * unit + 1);
+                fold(acc[0], __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 0, 8), 2 * unit);
+                fold(acc[0], __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 16, 8), 2 * unit + 1);
             }
             // one unit at a time (left free, the compiler keeps all the result tiles alive and runs out of registers)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) asm volatile("" : "+v"(acc[v]));
+            for (int v = 0; v < 4; ++v) {
+                asm volatile("" : "+v"(acc[0][v]));
+                if constexpr (T16) asm volatile("" : "+v"(acc[1][v]));
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
         settle();
@@ -183,7 +188,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
     // the partial tiles, [4][64] floats at the start of each wave's buffer
     float* part = (float*)buf;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) part[v * 64 + lane] = acc[v];
+    for (int v = 0; v < 4; ++v) part[v * 64 + lane] = T16 ? acc[0][v] + acc[T16 ? 1 : 0][v] : acc[0][v];
     __syncthreads();
     // sixteen rows: output (register v, lane l < 64) adds the waves' lanes l; eight: (v, l < 32) lanes l and l + 32
     constexpr int LANES = 4 * TOKS;
@@ -213,7 +218,7 @@ int launch(const Args& a, int waves, hipStream_t stream) {
 
 int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                         hipStream_t stream, int out_type) {
-    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || (((uintptr_t)w) & 15) != 0) return -1;
+    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || size_k > 32768 || (((uintptr_t)w) & 15) != 0) return -1;   // (longer rows: the others' to take or refuse)
     // One workgroup fits a CU (registers), and a second round of them costs what the first did, so the line is the number of
     // workgroups. Eight rows to a set where that is one round, sixteen otherwise. Measured in a graph, us, the granules
     // of rows16_q6k.hip (rows of a multiple of 2048 values; more rows than it takes: the 32-row tiles) against this:

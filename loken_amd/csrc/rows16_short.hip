@@ -1,0 +1,307 @@
+// Q4_K / Q5_K weights x at most sixteen Q8_1 activation rows where there are few 16-row tiles: the short launch of the
+// 16-row family (rows16_core.h has the arithmetic's layout, rows16_mfma.hip the launches for many tiles).
+//
+// What bounds it: the o projection of a small model (2048 x 2048, 2.4 MB) is 128 row tiles. rows16_mfma.hip gives a workgroup of
+// eight waves two of them and stages the activation for both, so 64 CUs work, a barrier stands between the loads and the
+// arithmetic, and a wave has two super-blocks to walk. Here a workgroup is one tile, its super-blocks spread over up to sixteen waves, one
+// each up to k = 4096; a wave reads the activation codes of its own super-blocks straight into the operand's lanes (sixteen bytes of
+// one row), all its loads in flight at once, and forms the codes' sums itself from what it holds.
+
+#include "lk_common.h"
+#include "rows16.h"
+#include "rows16_core.h"
+
+namespace {
+
+using rows16::Blk;
+using rows16::TILE;
+using rows16::WFrag;
+
+constexpr int MAX_TOKS = 16;             // activation rows a launch serves
+constexpr int GROUPS = 16;               // of a tile's super-blocks at most, each summed by one wave
+constexpr int PART_BYTES = 4 * 64 * 4;   // a wave's partial tile; the first one holds its scales until then, [8][TOKS] floats
+enum Out { F32, ANY, DUAL_F32, DUAL_Q81 };   // plain: f32 or p.out_type; act(gate) * up: f32 or the Q8_1 rows that the next linear reads
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+
+template <typename T>
+static __device__ __forceinline__ T pick3(const T (&a)[3], int i) { return i == 0 ? a[0] : i == 1 ? a[1] : a[2]; }
+
+struct TileRef {
+    int mat, tile;
+};
+// Tile i of workgroup `wg`'s NT: plain: of the matrices' tiles one after another; dual: gate and up of the same rows by turns.
+template <int OUT, int NT>
+static __device__ __forceinline__ TileRef tile_of(const LkRows16& p, int wg, int i) {
+    if (OUT >= DUAL_F32) return {i & 1, wg * (NT / 2) + (i >> 1)};
+    int mat = 0, tile = wg * NT + i;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const int tiles = (p.n[m] + TILE - 1) / TILE;
+        if (mat == m && m + 1 < p.count && tile >= tiles) tile -= tiles, mat = m + 1;
+    }
+    return {mat, tile};
+}
+
+static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q81) { return waves * nt * PART_BYTES + (q81 ? MAX_TOKS * 32 * 4 : 0); }
+
+// grid.x workgroups of NT row tiles each (one; two where one would be more workgroups than CUs, and for a gate and its up; four for
+// the 32 rows of a Q8_1 block), 64 * waves threads: wave w takes super-blocks w, w + waves, ... of every one of them, against one reading of the
+// activation.
+template <bool Q5, int TOKS, int OUT, int NT>
+__global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows16 p, int n_tiles) {
+    static_assert(TOKS == 8 || TOKS == 16, "eight or sixteen activation rows");
+    static_assert(NT == 1 || NT == 2 || NT == 4, "tiles in turn through two sets of weight registers");
+    constexpr bool T16 = TOKS == 16, DUAL = OUT >= DUAL_F32;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4, half = grp & 1, par = grp >> 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
+    const int m0 = (int)blockIdx.y * TOKS, m_rows = min(TOKS, p.m - m0);
+    float* part = (float*)(lds + wave * NT * PART_BYTES);
+    float* table = part;   // d8 [8][TOKS] of the super-block in hand
+
+    const uint8_t* w_lane[NT];   // the lane's row of each tile (past the last tile: of the last)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const TileRef r = DUAL ? tile_of<OUT, NT>(p, blockIdx.x, i) : tile_of<OUT, 1>(p, min((int)blockIdx.x * NT + i, n_tiles - 1), 0);
+        w_lane[i] = (const uint8_t*)(to_gbytes(pick3(p.w, r.mat)) + (size_t)min(r.tile * TILE + l16, pick3(p.n, r.mat) - 1) * p.nb * Blk<Q5>::BYTES);
+    }
+    // (eight rows: lanes that neither the instruction nor the minimums see ask for what the lane before them does)
+    const int tok = !T16 && l16 >= 8 && par == 0 ? 7 : l16 & (TOKS - 1);
+    const uint8_t* y_row = p.y + (size_t)(m0 + min(tok, m_rows - 1)) * p.stride_y * Q81_BYTES;
+    const float real = tok < m_rows ? 1.f : 0.f;
+    // the lane's pieces (c2, nib): row tok, sub-block 4 c2 + nib + 2 par, codes 16 half ..; its scales (h): sub-block 4 h + grp
+    const uint8_t* y_codes = y_row + 2 * par * Q81_BYTES + 4 + 16 * half;
+    const uint8_t* y_head = y_row + grp * Q81_BYTES;
+    // lanes the instruction sees: sixteen rows: sub-block s in lane groups 0, 1 and, by the second one, s + 2 in groups 2, 3;
+    // eight: slots (sub-block, row)
+    const bool live = T16 ? par == 0 : (l16 >> 3) == par;
+    const float* t_lane = T16 ? table + 4 * grp : table + 2 * par * TOKS + 4 * half;
+    const int sh16 = T16 ? 0 : 16 * par, sh2 = 2 * par;
+
+    struct Act {
+        u32x4 a[4];
+        uint32_t head[2];
+    };
+    auto load_act = [&](Act& b, int kb) {
+        const uint8_t* yc = y_codes + (size_t)kb * 8 * Q81_BYTES;
+        const uint8_t* yh = y_head + (size_t)kb * 8 * Q81_BYTES;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) b.head[h] = *(const uint32_t*)(yh + 4 * h * Q81_BYTES);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b.a[u] = *(const u32x4_a4*)(yc + (4 * (u >> 1) + (u & 1)) * Q81_BYTES);
+    };
+    auto load_w = [&](WFrag& w, const uint8_t* row, int kb) {
+        const uint8_t* bp = row + (size_t)kb * Blk<Q5>::BYTES;
+        w.hdr = *(const uint4*)bp;
+        if (Q5) w.qh = *(const uint4*)(bp + 16 + 16 * half);
+        w.q[0] = *(const uint4*)(bp + Blk<Q5>::QS + 16 * grp);
+        w.q[1] = *(const uint4*)(bp + Blk<Q5>::QS + 64 + 16 * grp);
+    };
+
+    // eight rows: the lane's sums of sub-blocks 0, 1, 4, 5 or 2, 3, 6, 7; sixteen: of both, apart, so that either form adds the same
+    // numbers in the same order and a launch may choose
+    float acc[NT][T16 ? 2 : 1][4] = {};
+    float d8s[2];   // d8 * S of (row, sub-block 4 h + grp), for the minimums
+    auto settle = [] {   // between the wave's writes to its table and its reads of other lanes' entries
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto scales = [&](const Act& b) {
+        // the lane holds half the codes of sub-blocks 4 h + 2 par and + 1; its own is + half, the other half of whose codes is with the lane
+        // sixteen on
+        const uint4 ones = make_uint4(0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u);
+        settle();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float d8 = real * f16_bits_to_f32(b.head[h] & 0xFFFFu);
+            table[(4 * h + grp) * TOKS + tok] = d8;
+            int sums[2];
+#pragma unroll
+            for (int nib = 0; nib < 2; ++nib) {
+                const u32x4 v = b.a[2 * h + nib];
+                sums[nib] = dot16(ones, make_uint4(v[0], v[1], v[2], v[3]), 0);
+            }
+            const int other = __builtin_amdgcn_ds_swizzle(half ? sums[0] : sums[1], 0x401F);   // lane ^ 16
+            d8s[h] = d8 * (float)((half ? sums[1] : sums[0]) + other);
+        }
+        settle();
+    };
+    auto compute = [&](const Act& b, const WFrag& w, float (&sum)[T16 ? 2 : 1][4]) {
+        // (accumulators from the bit pattern of 1.5 * 2^23, the offset off again in the first fused multiply-add, exactly: rows16_core.h)
+        constexpr int MAGIC_BITS = 0x4B400000;
+        constexpr float MAGIC = 12582912.0f;
+        const v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
+        auto fold = [&](float (&s)[4], const v4i& c, float dsc, int sub) {
+            const float off = -MAGIC * dsc;
+            const float4 t = *(const float4*)(t_lane + sub * TOKS);
+            s[0] = fmaf(fmaf(__int_as_float(c[0]), dsc, off), t.x, s[0]);
+            s[1] = fmaf(fmaf(__int_as_float(c[1]), dsc, off), t.y, s[1]);
+            s[2] = fmaf(fmaf(__int_as_float(c[2]), dsc, off), t.z, s[2]);
+            s[3] = fmaf(fmaf(__int_as_float(c[3]), dsc, off), t.w, s[3]);
+        };
+        const uint32_t w1 = w.hdr.y, w2 = w.hdr.z, w3 = w.hdr.w;
+        const uint32_t sc_lo = (w1 & 0x3F3F3F3Fu) >> sh16, sc_hi = ((w3 & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u)) >> sh16;
+        const float d = f16_bits_to_f32(w.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(w.hdr.x >> 16);
+        const uint32_t hp[4] = {w.qh.x >> sh2, w.qh.y >> sh2, w.qh.z >> sh2, w.qh.w >> sh2};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c2 = u >> 1, nib = u & 1;
+            const uint32_t q[4] = {w.q[c2].x, w.q[c2].y, w.q[c2].z, w.q[c2].w};
+            v4i codes, a0, a1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t x = (nib ? q[e] >> 4 : q[e]) & 0x0F0F0F0Fu;
+                if (Q5) x |= ((hp[e] >> (4 * c2 + nib)) & 0x01010101u) << 4;
+                codes[e] = (int)x;
+                a0[e] = live ? (int)b.a[u][e] : 0;
+                a1[e] = live ? 0 : (int)b.a[u][e];
+            }
+            const uint32_t scw = c2 ? sc_hi : sc_lo;
+            fold(sum[0], __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, codes, magic, 0, 0, 0), d * (float)((scw >> (8 * nib)) & 0xFFu), 4 * c2 + nib);
+            if constexpr (T16)
+                fold(sum[1], __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, codes, magic, 0, 0, 0), d * (float)((scw >> (8 * nib + 16)) & 0xFFu),
+                     4 * c2 + 2 + nib);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {   // (one unit's result tiles at a time: registers)
+                asm volatile("" : "+v"(sum[0][v]));
+                if constexpr (T16) asm volatile("" : "+v"(sum[1][v]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the minimums: d8 * S [row, sub-block] x (-dmin * min) [sub-block, weight row], four sub-blocks an instruction
+        const uint32_t mins[2] = {w2 & 0x3F3F3F3Fu, ((w3 >> 4) & 0x0F0F0F0Fu) | ((w2 >> 2) & 0x30303030u)};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float bmin = -(dmin * (float)((mins[h] >> (8 * grp)) & 0xFFu));
+            v4f c = {sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(T16 || l16 < TOKS ? d8s[h] : 0.f, bmin, c, 0, 0, 0);
+            sum[0][0] = c[0], sum[0][1] = c[1], sum[0][2] = c[2], sum[0][3] = c[3];
+        }
+    };
+
+    if constexpr (NT == 1) {   // two super-blocks in flight
+        Act act[2];
+        WFrag w[2];
+        auto load = [&](int d, int kb) { load_act(act[d], kb), load_w(w[d], w_lane[0], kb); };
+        auto step = [&](int d) { scales(act[d]), compute(act[d], w[d], acc[0]); };
+        load(0, wave);
+        if (wave + waves < p.nb) load(1, wave + waves);
+        for (int kb = wave; kb < p.nb; kb += 2 * waves) {
+            step(0);
+            if (kb + 2 * waves < p.nb) load(0, kb + 2 * waves);
+            if (kb + waves < p.nb) {
+                step(1);
+                if (kb + 3 * waves < p.nb) load(1, kb + 3 * waves);
+            }
+        }
+    } else {   // two tiles' weights
+        Act act;
+        WFrag w[2];
+        load_act(act, wave);
+        load_w(w[0], w_lane[0], wave);
+        load_w(w[1], w_lane[1], wave);
+        for (int kb = wave; kb < p.nb; kb += waves) {
+            scales(act);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                compute(act, w[i & 1], acc[i]);
+                if (i + 2 < NT) load_w(w[i & 1], w_lane[(i + 2) % NT], kb);
+                else if (kb + waves < p.nb) load_w(w[i & 1], w_lane[(i + 2) % NT], kb + waves);
+            }
+            if (kb + waves < p.nb) load_act(act, kb + waves);
+        }
+    }
+
+    settle();
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[(4 * i + v) * 64 + lane] = T16 ? acc[i][0][v] + acc[i][T16 ? 1 : 0][v] : acc[i][0][v];
+    __syncthreads();
+    // sixteen rows: output (register v, lane l < 64) adds the waves' lanes l; eight: (v, l < 32) lanes l and l + 32
+    constexpr int LANES = 4 * TOKS, OUTS = DUAL ? NT / 2 : NT;
+    float* meet = (float*)(lds + waves * NT * PART_BYTES);   // Q8_1 output: [TOKS][32]
+    for (int o = threadIdx.x; o < OUTS * 4 * LANES; o += (int)blockDim.x) {
+        const int r = o / (4 * LANES), v = o / LANES & 3, l = o % LANES;
+        auto total = [&](int i) {
+            float sum = 0.f;
+            for (int w = 0; w < waves; ++w) {
+                const float* col = (const float*)(lds + (w * NT + i) * PART_BYTES) + v * 64 + l;
+                sum += T16 ? col[0] : col[0] + col[32];
+            }
+            return sum;
+        };
+        float sum = total(DUAL ? 2 * r : r);
+        if constexpr (DUAL) {
+            LkGateAct act;
+            act.kind = p.gelu ? LK_GATE_GELU : LK_GATE_SILU;
+            sum = lk_gated(act, sum, total(2 * r + 1), 0);
+        }
+        const int t = 4 * (l >> 4) + v;
+        if constexpr (OUT == DUAL_Q81) {
+            meet[t * 32 + 16 * r + (l & 15)] = sum;   // (n is a multiple of 32: both tiles are whole)
+        } else {
+            const TileRef at = tile_of<OUT, NT>(p, blockIdx.x, DUAL ? 2 * r : r);
+            const int row = at.tile * TILE + (l & 15), mat = DUAL ? 0 : at.mat;
+            if (t < m_rows && row < pick3(p.n, mat)) lk_store_as(pick3(p.dst, mat), (size_t)(m0 + t) * pick3(p.ldd, mat) + row, sum, OUT == ANY ? p.out_type : LK_TYPE_F32);
+        }
+    }
+    if constexpr (OUT == DUAL_Q81) {
+        __syncthreads();
+        // eight lanes per activation row write its block
+        const int l8 = threadIdx.x & 7;
+        for (int row = (int)threadIdx.x >> 3; row < m_rows; row += (int)blockDim.x / 8)
+            lk_store_q8_1_block(*(const float4*)(meet + row * 32 + 4 * l8), l8, (uint32_t*)(p.q81_dst + ((size_t)(m0 + row) * p.q81_stride + blockIdx.x) * Q81_BYTES));
+    }
+}
+
+template <bool Q5, int TOKS, int OUT, int NT>
+int launch(const LkRows16& a, int tiles, hipStream_t stream) {
+    static const bool ok = hipFuncSetAttribute((const void*)q4k_rows16_short_kernel<Q5, TOKS, OUT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               lds_bytes_for(GROUPS, NT, OUT == DUAL_Q81)) == hipSuccess;
+    if (!ok) return LK_ERR_ARG;
+    const int steps = (a.nb + GROUPS - 1) / GROUPS, waves = (a.nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow
+    const int per_wg = OUT >= DUAL_F32 ? NT / 2 : NT;
+    hipLaunchKernelGGL((q4k_rows16_short_kernel<Q5, TOKS, OUT, NT>), dim3((tiles + per_wg - 1) / per_wg, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
+                       lds_bytes_for(waves, NT, OUT == DUAL_Q81), stream, a, tiles);
+    return lk_launch_status();
+}
+
+template <bool Q5, int TOKS>
+int launch_out(const LkRows16& a, bool dual, int tiles, hipStream_t stream) {
+    if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 4>(a, tiles, stream);
+    const bool pairs = tiles > lk_device().cus;
+    if (dual) return pairs ? launch<Q5, TOKS, DUAL_F32, 4>(a, tiles, stream) : launch<Q5, TOKS, DUAL_F32, 2>(a, tiles, stream);
+    if (pairs) return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 2>(a, tiles, stream) : launch<Q5, TOKS, ANY, 2>(a, tiles, stream);
+    return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 1>(a, tiles, stream) : launch<Q5, TOKS, ANY, 1>(a, tiles, stream);
+}
+
+}  // namespace
+
+int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
+    if (a.m < 1 || a.m > MAX_TOKS || a.nb < 1 || a.count < 1 || a.count > 3) return LK_ERR_ARG;
+    if ((dual && (a.count != 2 || a.n[0] != a.n[1])) || (a.q81_dst && (!dual || a.n[0] % 32 != 0 || a.q81_stride < a.n[0] / 32))) return LK_ERR_ARG;
+    int tiles = 0;
+    for (int i = 0; i < (dual ? 1 : a.count); ++i) tiles += (a.n[i] + TILE - 1) / TILE;
+    if (tiles == 0) return LK_OK;
+    // more than eight rows: two sets of eight where both are resident at once (Q4_K 2048 x 6144 at 16 rows 8.5 us against 9.1)
+    const bool eight = a.m <= 8 || (!dual && 2 * tiles <= lk_device().cus);
+    if (eight) return q5 ? launch_out<true, 8>(a, dual, tiles, stream) : launch_out<false, 8>(a, dual, tiles, stream);
+    return q5 ? launch_out<true, 16>(a, dual, tiles, stream) : launch_out<false, 16>(a, dual, tiles, stream);
+}
+
+// Matrices of up to two row tiles to the CU: with more workgroups than CUs, or more tiles to a workgroup, the launches that stage the activation
+// once and walk many tiles are ahead; above a tile to the CU rows of 2048 values or more, and at most 8192 up to eight rows. A choice by the matrix
+// and the class of row counts alone, so that several matrices in one launch carry the bits of one launch each, and not above sixteen rows, where a row
+// carries the 32-row tiles' bits whatever rides with it. Measured in a graph, Q4_K, us, staged launches against this:
+//   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.8, 4.1; 4096 x 4096 7.7, 8.1 / 5.6, 6.2; 4096 x 14336 17.9, 19.4 / 13.2, 15.6; 6144 x 2048 5.5, 5.5 / 5.0, 5.4;
+//                8192 x 4096 8.9, 9.1 / 7.7, 8.3; 8192 x 1024 4.2, 4.1 / 4.0, 4.2; 5000 x 12288 16.7, 17.7 / 15.9, 18.3; 10000 x 5120 (three to the CU) 12.9, 13.6 / 13.2, 16.0
+//   9 / 16 rows  2048 x 2048 5.9, 6.4 / 4.5, 4.5; 4096 x 4096 9.4, 10.2 / 6.2, 6.9; 2048 x 6144 12.1, 13.2 / 8.4, 8.5; 4096 x 14336 28.8, 32.2 / 16, 19;
+//                8192 x 4096 10.3, 11.0 / 8.5, 9.3; 5000 x 12288 25.8, 28.7 / 18.4, 21.1; 8192 x 1024 4.2, 4.3 / 4.9, 5.1; 10000 x 5120 15.3, 16.3 / 16.3, 17.8
+// (Rows of up to 32768 values: longer ones are the other launches' to take or refuse.)
+bool lk_rows16_short_pays(int m, int n, int nb) {
+    const int tiles = (n + TILE - 1) / TILE, cus = lk_device().cus;
+    return m >= 1 && m <= MAX_TOKS && nb <= 128 && (tiles <= cus || (tiles <= 2 * cus && nb >= 8 && (m > 8 || nb <= 32)));
+}

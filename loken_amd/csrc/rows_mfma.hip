@@ -774,18 +774,20 @@ template <bool DUAL, bool Q5>
 int launch_any(const Args& a, hipStream_t stream) {
     // at most 8 / 16 activation rows in all: the fix-up runs on the registers those rows live in,
     // and the activation is staged in LDS when it fits there
+    LkRows16 r{};
+    r.w[0] = a.w; r.w[1] = a.w2;
+    r.dst[0] = a.dst;
+    r.n[0] = r.n[1] = a.n;
+    r.ldd[0] = a.ldd;
+    r.out_type = a.out_type;
+    r.count = DUAL ? 2 : 1;
+    r.y = a.y; r.nb = a.nb; r.m = a.m; r.stride_y = a.stride_y; r.gelu = a.gelu;
+    // few row tiles: each one's super-blocks over the waves of a workgroup (rows16_short.hip)
+    if (lk_rows16_short_pays(a.m, a.n, a.nb)) return lk_rows16_short(r, DUAL, Q5, stream);
     if (a.m <= 16) {
         // 16-row tiles (rows16_mfma.hip): half the matrix-unit time per weight, twice the tiles
         if (lk_rows16_serves(a.m, a.nb) && lk_tune_env("LK_TUNE_ROWS16_OFF") == 0 &&
             (a.m <= 8 || lk_tune_env("LK_TUNE_ROWS16_MAX8") == 0)) {
-            LkRows16 r{};
-            r.w[0] = a.w; r.w[1] = a.w2;
-            r.dst[0] = a.dst;
-            r.n[0] = r.n[1] = a.n;
-            r.ldd[0] = a.ldd;
-            r.out_type = a.out_type;
-            r.count = DUAL ? 2 : 1;
-            r.y = a.y; r.nb = a.nb; r.m = a.m; r.stride_y = a.stride_y; r.gelu = a.gelu;
             return lk_rows16_launch(r, DUAL, Q5, stream);
         }
     }
@@ -874,6 +876,31 @@ extern "C" int lk_dense_q4k_rows_multi(const void* const* weights, float* const*
     for (int i = 0; i < count; ++i)
         if (sizes_n[i] > 0 && bad_rows_call(weights[i], q8_1, outputs[i], size_m, sizes_n[i], size_k)) return LK_ERR_ARG;
     const int nb = size_k / 256;
+    // The matrices that a launch of their own takes to the short launch (lk_rows16_short_pays) go there together, the others as before:
+    // two launches where both kinds are, for the single launches' bits.
+    {
+        LkRows16 r{};
+        const void* rest_w[3];
+        float* rest_out[3];
+        int rest_n[3], rest = 0;
+        for (int i = 0; i < count; ++i) {
+            if (sizes_n[i] <= 0) continue;
+            if (!lk_rows16_short_pays(size_m, sizes_n[i], nb)) {
+                rest_w[rest] = weights[i], rest_out[rest] = outputs[i], rest_n[rest++] = sizes_n[i];
+                continue;
+            }
+            r.w[r.count] = (const uint8_t*)weights[i];
+            r.dst[r.count] = outputs[i];
+            r.n[r.count] = r.ldd[r.count] = sizes_n[i];
+            ++r.count;
+        }
+        if (r.count > 0) {
+            r.y = (const uint8_t*)q8_1; r.nb = nb; r.m = size_m; r.stride_y = size_k / 32;
+            const int rc = lk_rows16_short(r, false, q5 != 0, (hipStream_t)stream);
+            if (rc != LK_OK) return rc;
+            return rest > 0 ? lk_dense_q4k_rows_multi(rest_w, rest_out, rest_n, rest, q8_1, size_m, size_k, q5, stream) : LK_OK;
+        }
+    }
     if (lk_rows16_serves(size_m, nb) && lk_tune_env("LK_TUNE_ROWS16_OFF") == 0 &&
         (size_m <= 8 || lk_tune_env("LK_TUNE_ROWS16_MAX8") == 0)) {
         LkRows16 r{};
@@ -917,8 +944,7 @@ extern "C" int lk_dense_q4k_rows_multi(const void* const* weights, float* const*
 // Gate and up in one launch with the result handed on as Q8_1: q8_1_out[m][size_n / 32] blocks =
 // lk_quantize_q8_1(act(gate . x) * (up . x)), byte for byte, so the down projection of a layer reads it
 // without the f32 round trip and the quantizer launch in between (what lk_mmvq_pair_act_q8_1 is to the
-// mat-vec pair launch). Up to 16 rows the 16-row-tile kernel at four tiles per workgroup (rows of 2048 or
-// 4096 values), above them the 32-row tiles (a tile's rows are one block; any row length its tables hold);
+// mat-vec pair launch). Up to 16 rows the 16-row-tile kernels (few row tiles: rows16_short.hip), above them the 32-row tiles (a tile's rows are one block; any row length its tables hold). Up to 16 rows k is 2048 or 4096,
 // size_n a multiple of 32; anything else returns LK_ERR_ARG (take the f32 form and the quantizer). q5 != 0: Q5_K. No counterpart in the reference, whose dense_q4k_imma_m8_act_mul writes f32
 // (src/inference/moe_cuda/dense/imma.rs:320-400).
 extern "C" int lk_dense_q4k_rows_actmul_q8_1(const void* gate, const void* up, const void* q8_1, void* q8_1_out, int size_m,
@@ -929,6 +955,14 @@ extern "C" int lk_dense_q4k_rows_actmul_q8_1(const void* gate, const void* up, c
         ((((uintptr_t)q8_1) | ((uintptr_t)q8_1_out)) & 3) != 0)
         return LK_ERR_ARG;
     const int nb = size_k / 256;
+    if (size_m <= 16 && ((nb != 8 && nb != 16) || !lk_rows16_serves(size_m, nb))) return LK_ERR_ARG;
+    LkRows16 r{};
+    r.w[0] = (const uint8_t*)gate; r.w[1] = (const uint8_t*)up;
+    r.n[0] = r.n[1] = size_n;
+    r.count = 2;
+    r.y = (const uint8_t*)q8_1; r.nb = nb; r.m = size_m; r.stride_y = size_k / 32; r.gelu = use_gelu ? 1 : 0;
+    r.q81_dst = (uint8_t*)q8_1_out; r.q81_stride = size_n / 32;
+    if (lk_rows16_short_pays(size_m, size_n, nb)) return lk_rows16_short(r, true, q5 != 0, (hipStream_t)stream);
     if (size_m > 16) {   // the 32-row tiles: a tile's rows are one block
         Args a{(const uint8_t*)gate, (const uint8_t*)q8_1, nullptr, nb, size_n, size_m, size_k / 32, size_n,
                (const uint8_t*)up, use_gelu ? 1 : 0};
@@ -936,13 +970,6 @@ extern "C" int lk_dense_q4k_rows_actmul_q8_1(const void* gate, const void* up, c
         a.q81_stride = size_n / 32;
         return q5 ? launch_rows<4, true, true>(a, (hipStream_t)stream) : launch_rows<4, true, false>(a, (hipStream_t)stream);
     }
-    if ((nb != 8 && nb != 16) || !lk_rows16_serves(size_m, nb)) return LK_ERR_ARG;
-    LkRows16 r{};
-    r.w[0] = (const uint8_t*)gate; r.w[1] = (const uint8_t*)up;
-    r.n[0] = r.n[1] = size_n;
-    r.count = 2;
-    r.y = (const uint8_t*)q8_1; r.nb = nb; r.m = size_m; r.stride_y = size_k / 32; r.gelu = use_gelu ? 1 : 0;
-    r.q81_dst = (uint8_t*)q8_1_out; r.q81_stride = size_n / 32;
     return lk_rows16_launch(r, true, q5 != 0, (hipStream_t)stream);
 }
 

@@ -315,6 +315,24 @@ def test_q6k_eight_rows_or_fewer_in_sixteen_row_tiles(m, k, n):
     assert_close(got, oracle.ob_matmul(Q6K, x, w, n))
 
 
+@pytest.mark.parametrize("q5", [False, True])
+@pytest.mark.parametrize("m,k,n", [(1, 256, 1), (4, 768, 16), (5, 4352, 17), (8, 4096, 4096), (8, 2048, 4097), (9, 4096, 2048), (16, 8448, 2049),
+                                   (13, 12544, 40), (3, 2304, 4112), (11, 8192, 4000), (8, 8192, 4500), (9, 8448, 8192), (16, 2048, 8193), (17, 512, 100)])
+def test_few_row_tiles_take_the_short_launch(m, k, n, q5):
+    """rows16_short.hip: one to four super-blocks a wave, groups without a last one, sets of eight with a last set of one, two groups to a
+    wave, both sides of its line in row tiles; several matrices on both sides of it carry the single launches' bits."""
+    wtype, fn = lib.TYPE_Q5_K if q5 else Q4K, ops.dense_q4k_rows
+    w = synth.weight(wtype, n, k, seed=80, stream=1)
+    x = synth.activation(m, k, seed=80)
+    got = fn(dev(w), dev(x), n, q5=q5)
+    pick = np.unique(np.r_[:min(n, 40), max(0, n - 40):n])
+    assert_close(got.cpu().numpy()[:, pick], oracle.ob_matmul(wtype, x, w[pick], len(pick)))
+    small, big = dev(synth.weight(wtype, 33, k, seed=80, stream=2)), dev(synth.weight(wtype, 8200, k, seed=80, stream=3)) if k <= 1024 else None
+    ws, sizes = ([dev(w), small], (n, 33)) if big is None else ([dev(w), small, big], (n, 33, 8200))
+    for one, size, out in zip(ws, sizes, ops.dense_q4k_rows_multi(ws, dev(x), sizes, q5=q5)):
+        assert torch.equal(out, fn(one, dev(x), size, q5=q5))
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 3328, 5), (8, 3072, 16), (9, 3328, 31), (16, 6400, 100), (7, 2304, 6150), (16, 1792, 6100), (15, 4096, 2080),
                                    (32, 4096, 1030), (20, 4096, 4000), (23, 2816, 5200), (64, 1280, 2048), (33, 11008, 700), (7, 4096, 8200),
                                    (3, 2048, 8200)])
