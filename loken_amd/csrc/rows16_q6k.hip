@@ -450,10 +450,12 @@ int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, in
     // (the short launch has taken the calls of few row tiles: rows16_q6k_short.hip)
     if (size_m <= 4) return launch<4>(a, stream);
     const int n_tiles = (size_n + TILE - 1) / TILE;
-    // 5..8 rows as two sets of four for a matrix small enough for its second reading to come from L2 at no cost (8192 x 2048 8.8 us
-    // against 9.5; 8192 x 4096, 27.5 MB, 12.2 against 11.1 and stays with eight). (Sets: below.)
+    // 5..8 rows as two sets of four where that fills the chip sooner than eight at once: so few tiles that a
+    // workgroup per tile leaves half the CUs idle (2048 x 14336 12.9 us against 16.3), or a matrix small enough for its second reading to come
+    // from L2 at no cost (8192 x 2048 8.8 against 9.5; 8192 x 4096, 27.5 MB, 12.2 against 11.1 and stays with eight). (Sets: below.)
     const size_t weight_bytes = (size_t)size_n * a.nb * Q6K_BYTES;
-    if (size_m <= 8) return weight_bytes <= ((size_t)22 << 20) ? launch<4>(a, stream, 2) : launch<8>(a, stream);
+    if (size_m <= 8)
+        return 2 * n_tiles <= lk_device().cus || weight_bytes <= ((size_t)22 << 20) ? launch<4>(a, stream, 2) : launch<8>(a, stream);
     // 9..32 rows. Sixteen at once when their codes fit LDS and the row tiles are several to the CU; else the
     // rows in sets of eight, a set per workgroup (grid.y), in one launch: rows too long for sixteen in LDS (k =
     // 14336: 229 KB), up to two tiles to the CU, where twice the workgroups with half the staging each

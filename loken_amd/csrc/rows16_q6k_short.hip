@@ -5,9 +5,8 @@
 // What bounds it: a `down` projection of a small model (2048 x 6144, 10 MB) is 128 row tiles, so a launch is over in about the
 // time of one load, one wave's arithmetic and one reduction, whatever the bytes. rows16_q6k.hip hands a wave a granule of eight
 // super-blocks, which makes that arithmetic eight steps long with three waves on a CU (11.1 us a launch at 16 rows in a
-// graph, of which 2 are a launch that does nothing; now 8.3). Here a tile's super-blocks go to up to twelve waves (168 registers each), every load of the first two in flight at once; nothing is staged for the workgroup, so no barrier stands before the
-// arithmetic: a wave reads the activation codes of its own super-blocks straight into the operand's lanes (sixteen bytes of one
-// row), and turns the weights and the eight scales per row through a buffer of its own.
+// graph, of which 2 are a launch that does nothing; now 7.8). Here a tile's super-blocks go to up to twelve waves (168 registers each), every load of the first two in flight at once; nothing is staged for the workgroup, so no barrier stands before the
+// arithmetic: a wave reads the activation codes of its own super-blocks itself, and turns the weights and the eight scales per row through a buffer of its own.
 //
 // Any super-block may be a wave's, so its bytes start at any even phase of a 16-byte piece, another one for each row: the row's
 // fourteen pieces are written to the buffer so that the block starts at byte 16 or 18, and a lane shifts what it reads by its row's
@@ -64,14 +63,18 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         w_to[u] = row * PITCH + 16 * (id % BLOCK_PIECES) + 16;
     }
     const uint32_t my_at = (uint32_t)(min(l16, last_row) * row_bytes);   // of the lane's own row
-    // ---- the activation: the lane's sixteen codes of unit u (values 64 u + 16 grp ..), the scales it puts in the table
+    // ---- the activation, asked for in the order it lies in, a row's pieces by neighbouring lanes, and handed to the operand's lanes by a permutation
+    // (in the operand's order, neighbouring rows by neighbouring lanes, a load is a line a lane). Sixteen rows: load u is the four pieces of (row
+    // lane / 4, unit u: values 64 u ..); eight: load v the eight pieces of (row lane / 8, units 2 v and 2 v + 1)
     const int tok = l16 & (TOKS - 1), sel = l16 / TOKS;
+    constexpr int PER_ROW = 64 / TOKS, Y_LOADS = 16 / PER_ROW, HEADS = TOKS / 8;
+    const int y_tok = lane / PER_ROW, y_piece = lane % PER_ROW, h_tok = lane >> 3, h_sub = lane & 7;
     const uint8_t* y0 = p.y + (size_t)m0 * p.stride_y * Q81_BYTES;
-    const uint32_t y_codes = (uint32_t)((min(tok, m_rows - 1) * p.stride_y + (grp >> 1)) * Q81_BYTES + 4 + 16 * (grp & 1));
-    constexpr int HEADS = T16 ? 2 : 1;
-    const int h_tok = lane & (TOKS - 1), h_sub = (lane / TOKS) & 7;
-    const uint32_t y_head = (uint32_t)((min(h_tok, m_rows - 1) * p.stride_y + h_sub) * Q81_BYTES);
-    const float h_real = h_tok < m_rows ? 1.f : 0.f;
+    const uint32_t y_codes = (uint32_t)((min(y_tok, m_rows - 1) * p.stride_y + (y_piece >> 1)) * Q81_BYTES + 4 + 16 * (y_piece & 1));
+    uint32_t y_head[HEADS];   // scales: (row h_tok + 8 j, sub-block h_sub)
+#pragma unroll
+    for (int j = 0; j < HEADS; ++j) y_head[j] = (uint32_t)((min(h_tok + 8 * j, m_rows - 1) * p.stride_y + h_sub) * Q81_BYTES);
+    const int from = 4 * (tok * PER_ROW + grp);   // byte address of the lane that holds the operand's piece (eight rows: of even units)
     // eight rows: the lanes whose codes the first and the second instruction see
     const uint32_t keep0 = grp == sel ? ~0u : 0u, keep1 = grp == sel + 2 ? ~0u : 0u;
     // the lane's results: eight rows: groups grp / 2 and 2 + grp / 2, rows 4 (grp % 2) + v; sixteen: every group, rows 4 grp + v
@@ -79,15 +82,15 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
     const int sh_sc = T16 ? 0 : 8 * (grp >> 1), sh_qh = 2 * (grp >> 1);
 
     struct Block {
-        u32x4 w[LOADS], a[4];
+        u32x4 w[LOADS], y[Y_LOADS];
         uint32_t head[HEADS];
     };
     auto load = [&](Block& b, int kb) {
         const uint32_t at = (uint32_t)(kb * Q6K_BYTES), ya = (uint32_t)(kb * 8 * Q81_BYTES);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) b.a[u] = *(const u32x4_a4*)(y0 + (y_codes + ya) + 2 * u * Q81_BYTES);
+        for (int j = 0; j < HEADS; ++j) b.head[j] = *(const uint32_t*)(y0 + (y_head[j] + ya));
 #pragma unroll
-        for (int h = 0; h < HEADS; ++h) b.head[h] = *(const uint32_t*)(y0 + (y_head + ya) + 4 * h * Q81_BYTES);
+        for (int u = 0; u < Y_LOADS; ++u) b.y[u] = *(const u32x4_a4*)(y0 + (y_codes + ya) + u * (8 / Y_LOADS) * Q81_BYTES);
 #pragma unroll
         for (int u = 0; u < LOADS; ++u) b.w[u] = *(const u32x4*)(w_tile + (((w_at[u] + at) & ~15u) + w_piece[u]));
     };
@@ -102,8 +105,13 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
             __builtin_amdgcn_wave_barrier();
         };
 #pragma unroll
-        for (int h = 0; h < HEADS; ++h)
-            table[(h_sub + 4 * h) * TOKS + h_tok] = h_real * f16_bits_to_f32(b.head[h] & 0xFFFFu);
+        for (int j = 0; j < HEADS; ++j) table[h_sub * TOKS + h_tok + 8 * j] = h_tok + 8 * j < m_rows ? f16_bits_to_f32(b.head[j] & 0xFFFFu) : 0.f;
+        u32x4 act[4];   // the lane's sixteen codes of unit u: values 64 u + 16 grp ..
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                act[u][e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from + (T16 ? 0 : 16 * (u & 1)), (int)b.y[T16 ? u : u >> 1][e]);
 #pragma unroll
         for (int u = 0; u < LOADS; ++u)
             if (64 * u + lane < TILE * BLOCK_PIECES) *(u32x4_a4*)(buf + (w_to[u] - (int)((w_at[u] + at) & 12u))) = b.w[u];
@@ -151,14 +159,14 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
                 for (int g = 0; g < 4; ++g) {   // the activation of group g alone
                     v4i a;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) a[e] = grp == g ? (int)b.a[unit][e] : 0;
+                    for (int e = 0; e < 4; ++e) a[e] = grp == g ? (int)act[unit][e] : 0;
                     const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, codes, magic, 0, 0, 0);
                     fold(acc[T16 ? g & 1 : 0], c, d * (float)(int)__builtin_amdgcn_sbfe(scw, 8 * g, 8), 2 * unit + (g >> 1));
                 }
             } else {
                 v4i a0, a1;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a0[e] = (int)(b.a[unit][e] & keep0), a1[e] = (int)(b.a[unit][e] & keep1);
+                for (int e = 0; e < 4; ++e) a0[e] = (int)(act[unit][e] & keep0), a1[e] = (int)(act[unit][e] & keep1);
                 fold(acc[0], __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 0, 8), 2 * unit);
                 fold(acc[0], __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, codes, magic, 0, 0, 0), d * (float)(int)__builtin_amdgcn_sbfe(scw, 16, 8), 2 * unit + 1);
             }
@@ -222,14 +230,19 @@ int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size
     // One workgroup fits a CU (registers), and a second round of them costs what the first did, so the line is the number of
     // workgroups. Eight rows to a set where that is one round, sixteen otherwise. Measured in a graph, us, the granules
     // of rows16_q6k.hip (rows of a multiple of 2048 values; more rows than it takes: the 32-row tiles) against this:
-    //   up to 8 rows    1024 x 2048 7.3 / 4.2, 2048 x 6144 9.0 / 8.0, 4096 x 4096 9.3 / 7.1, 6144 x 2048 9.7 / 7.5, 8192 x 4096 12.1 / 12.7
-    //   9 to 16         1024 x 2048 9.2 / 4.3, 2048 x 6144 11.1 / 8.3, 4096 x 4096 10.8 / 8.4, 4096 x 14336 25.6 / 20.0, 8192 x 4096 15.0 / 15.1
-    //   17 to 32        1024 x 2048 9.3 / 4.4, 2048 x 6144 13.2 / 10.0, 4096 x 4096 13.3..13.8 / 12.9..14.5, 4096 x 14336 41 / 32..36 (over 64 MB)
-    //   33 to 64        1024 x 2048 10.1 / 5.0, 2048 x 6144 at 48 / 64 22.2, 18.1 / 17.9, 18.2, 2048 x 14336 46 / 34, 4096 x 4096 17.5 / 20.1
+    //   3 / 8 rows      1024 x 2048 7.4, 7.4 / 4.3, 4.3; 2048 x 6144 8.8, 9.1 / 7.8, 7.8; 4096 x 4096 8.9, 9.5 / 7.2, 7.2; 4096 x 14336 15.4, 19.3 / 16.2, 16.3;
+    //                   6144 x 2048 8.3, 9.8 / 7.0, 7.1; 8192 x 4096 10.5, 12.2 / 12.0, 12.3. Few tiles of long rows stay with the granules, whose waves have
+    //                   less to do in LDS a super-block (it is what a CU of twelve waves waits for here): 1024 x 8192 8.9, 9.2 / 9.4, 9.5; 2048 x 14336
+    //                   12.6, 13.4 / 14.1, 14.0
+    //   9 / 16          1024 x 2048 9.2, 9.3 / 4.3, 4.4; 2048 x 6144 11.0, 11.0 / 8.0, 7.8; 4096 x 4096 10.4, 10.8 / 8.2, 8.2; 4096 x 14336 26.1, 25.8 / 19.1, 19.1;
+    //                   2048 x 14336 16.7, 16.7 / 14.6, 14.3; 8192 x 4096 14.4, 15.0 / 14.4, 15.0
+    //   24 / 32         1024 x 2048 9.2, 9.3 / 4.4, 4.4; 2048 x 6144 14.6, 12.9 / 9.3, 9.4; 2048 x 14336 24.3, 24.7 / 17.4, 17.3; 4096 x 4096 13.9, 13.7 / 12.9, 14.3
+    //   48              1024 x 2048 10.1 / 5.0, 2048 x 6144 22.2 / 16.8, 2048 x 14336 46.0 / 31.2, 4096 x 4096 17.5 / 20.1
     // and against the 32-row tiles where rows are no granules: 700 x 11008 at 8 / 16 / 32 / 64 rows 32, 37, 43, 43 / 10, 11, 11, 14;
-    // 10000 x 5120 at 8 / 16 / 32 25, 31, 37 / 21, 26, 41; 16384 x 3072 at 8 / 16 16.9, 20.3 / 17.9, 20.9; 3000 x 5120 at 32 / 64 19.8, 20.4 / 16.9, 24.4
+    // 10000 x 5120 at 8 / 16 / 32 25.3, 31.6, 36.7 / 19.9, 24.4, 41; 16384 x 3072 at 8 / 16 17.1, 20.2 / 17.9, 20.9; 3000 x 5120 at 32 / 48 20.0, 20.2 / 16.1, 24.1
     const int nb = size_k / 256, tiles = (size_n + TILE - 1) / TILE, cus = lk_device().cus;
     const bool granules = nb % 8 == 0, held = granules && tiles <= cus && (size_t)size_n * nb * Q6K_BYTES <= (64u << 20);
+    if (granules && size_m <= 8 && nb >= 32 && (2 * tiles <= cus || (size_m <= 4 && nb >= 48))) return -1;
     const int eights = (size_m + 7) / 8, sixteens = (size_m + 15) / 16;
     const int64_t most = size_m <= 16 ? (granules ? 3 * cus / 2 : 3 * cus) : size_m > 32 ? 2 * cus : held ? cus : granules ? 2 * cus : 3 * cus;
     const bool by_eight = size_m <= 8 || (int64_t)tiles * eights <= cus;

@@ -4,8 +4,8 @@
 // What bounds it: the o projection of a small model (2048 x 2048, 2.4 MB) is 128 row tiles. rows16_mfma.hip gives a workgroup of
 // eight waves two of them and stages the activation for both, so 64 CUs work, a barrier stands between the loads and the
 // arithmetic, and a wave has two super-blocks to walk. Here a workgroup is one tile, its super-blocks spread over up to sixteen waves, one
-// each up to k = 4096; a wave reads the activation codes of its own super-blocks straight into the operand's lanes (sixteen bytes of
-// one row), all its loads in flight at once, and forms the codes' sums itself from what it holds.
+// each up to k = 4096; a wave reads the activation codes of its own super-blocks itself, all its loads in flight at
+// once, and forms the codes' sums from what it holds.
 
 #include "lk_common.h"
 #include "rows16.h"
@@ -61,19 +61,31 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     float* part = (float*)(lds + wave * NT * PART_BYTES);
     float* table = part;   // d8 [8][TOKS] of the super-block in hand
 
-    const uint8_t* w_lane[NT];   // the lane's row of each tile (past the last tile: of the last)
+    const uint8_t* w_base[NT];   // each tile's matrix, and the lane's row in it (past the last tile: of the last)
+    uint32_t w_row[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const TileRef r = DUAL ? tile_of<OUT, NT>(p, blockIdx.x, i) : tile_of<OUT, 1>(p, min((int)blockIdx.x * NT + i, n_tiles - 1), 0);
-        w_lane[i] = (const uint8_t*)(to_gbytes(pick3(p.w, r.mat)) + (size_t)min(r.tile * TILE + l16, pick3(p.n, r.mat) - 1) * p.nb * Blk<Q5>::BYTES);
+        w_base[i] = (const uint8_t*)to_gbytes(pick3(p.w, r.mat));
+        w_row[i] = (uint32_t)min(r.tile * TILE + l16, pick3(p.n, r.mat) - 1) * (uint32_t)(p.nb * Blk<Q5>::BYTES);
     }
-    // (eight rows: lanes that neither the instruction nor the minimums see ask for what the lane before them does)
-    const int tok = !T16 && l16 >= 8 && par == 0 ? 7 : l16 & (TOKS - 1);
-    const uint8_t* y_row = p.y + (size_t)(m0 + min(tok, m_rows - 1)) * p.stride_y * Q81_BYTES;
-    const float real = tok < m_rows ? 1.f : 0.f;
-    // the lane's pieces (c2, nib): row tok, sub-block 4 c2 + nib + 2 par, codes 16 half ..; its scales (h): sub-block 4 h + grp
-    const uint8_t* y_codes = y_row + 2 * par * Q81_BYTES + 4 + 16 * half;
-    const uint8_t* y_head = y_row + grp * Q81_BYTES;
+    const int tok = l16 & (TOKS - 1);
+    // The activation is asked for in the order it lies in, a row's pieces by neighbouring lanes, and handed to the operand's lanes by a
+    // permutation (in the operand's order, neighbouring rows by neighbouring lanes, a load is a line a lane). Sixteen rows: load u is the four pieces of
+    // (row lane / 4, unit u), unit u = 2 c2 + nib being sub-blocks 4 c2 + nib and + 2; eight: load c2 the eight pieces of (row lane / 8, units
+    // 2 c2 and 2 c2 + 1).
+    constexpr int PER_ROW = 64 / TOKS, LOADS = 16 / PER_ROW;
+    const int y_tok = lane / PER_ROW, y_piece = lane % PER_ROW;
+    const uint8_t* y_codes = p.y + ((size_t)(m0 + min(y_tok, m_rows - 1)) * p.stride_y + (T16 ? 2 * (y_piece >> 1) : y_piece >> 1)) * Q81_BYTES + 4 + 16 * (y_piece & 1);
+    int from[T16 ? 1 : 2];   // byte address of the lane that holds the operand's piece (eight rows: of units of nib 0 and 1)
+#pragma unroll
+    for (int nib = 0; nib < (T16 ? 1 : 2); ++nib) from[nib] = 4 * (tok * PER_ROW + (T16 ? grp : 2 * (nib + 2 * par) + half));
+    // scales: (row h_tok + 8 j, sub-block h_sub)
+    constexpr int HEADS = TOKS / 8;
+    const int h_tok = lane >> 3, h_sub = lane & 7;
+    const uint8_t* y_head[HEADS];
+#pragma unroll
+    for (int j = 0; j < HEADS; ++j) y_head[j] = p.y + ((size_t)(m0 + min(h_tok + 8 * j, m_rows - 1)) * p.stride_y + h_sub) * Q81_BYTES;
     // lanes the instruction sees: sixteen rows: sub-block s in lane groups 0, 1 and, by the second one, s + 2 in groups 2, 3;
     // eight: slots (sub-block, row)
     const bool live = T16 ? par == 0 : (l16 >> 3) == par;
@@ -81,23 +93,22 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     const int sh16 = T16 ? 0 : 16 * par, sh2 = 2 * par;
 
     struct Act {
-        u32x4 a[4];
-        uint32_t head[2];
+        u32x4 raw[LOADS];
+        uint32_t head[HEADS];
     };
     auto load_act = [&](Act& b, int kb) {
-        const uint8_t* yc = y_codes + (size_t)kb * 8 * Q81_BYTES;
-        const uint8_t* yh = y_head + (size_t)kb * 8 * Q81_BYTES;
+        const uint32_t at = (uint32_t)(kb * 8 * Q81_BYTES);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) b.head[h] = *(const uint32_t*)(yh + 4 * h * Q81_BYTES);
+        for (int j = 0; j < HEADS; ++j) b.head[j] = *(const uint32_t*)(y_head[j] + at);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) b.a[u] = *(const u32x4_a4*)(yc + (4 * (u >> 1) + (u & 1)) * Q81_BYTES);
+        for (int u = 0; u < LOADS; ++u) b.raw[u] = *(const u32x4_a4*)(y_codes + at + (T16 ? 4 * (u >> 1) + (u & 1) : 4 * u) * Q81_BYTES);
     };
-    auto load_w = [&](WFrag& w, const uint8_t* row, int kb) {
-        const uint8_t* bp = row + (size_t)kb * Blk<Q5>::BYTES;
-        w.hdr = *(const uint4*)bp;
-        if (Q5) w.qh = *(const uint4*)(bp + 16 + 16 * half);
-        w.q[0] = *(const uint4*)(bp + Blk<Q5>::QS + 16 * grp);
-        w.q[1] = *(const uint4*)(bp + Blk<Q5>::QS + 64 + 16 * grp);
+    auto load_w = [&](WFrag& w, int i, int kb) {
+        const uint32_t at = w_row[i] + (uint32_t)(kb * Blk<Q5>::BYTES), at_q = at + 16 * grp;
+        w.hdr = *(const uint4*)(w_base[i] + at);
+        if (Q5) w.qh = *(const uint4*)(w_base[i] + (at + 16 * half) + 16);
+        w.q[0] = *(const uint4*)(w_base[i] + at_q + Blk<Q5>::QS);
+        w.q[1] = *(const uint4*)(w_base[i] + at_q + Blk<Q5>::QS + 64);
     };
 
     // eight rows: the lane's sums of sub-blocks 0, 1, 4, 5 or 2, 3, 6, 7; sixteen: of both, apart, so that either form adds the same
@@ -108,27 +119,32 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
-    auto scales = [&](const Act& b) {
+    u32x4 a[4];   // the lane's pieces: unit (c2, nib): row tok, sub-block 4 c2 + nib + 2 par, codes 16 half ..
+    auto settle_act = [&](const Act& b) {
+        settle();
+#pragma unroll
+        for (int j = 0; j < HEADS; ++j) table[h_sub * TOKS + h_tok + 8 * j] = h_tok + 8 * j < m_rows ? f16_bits_to_f32(b.head[j] & 0xFFFFu) : 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[u][e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from[T16 ? 0 : u & 1], (int)b.raw[T16 ? u : u >> 1][e]);
+        settle();
         // the lane holds half the codes of sub-blocks 4 h + 2 par and + 1; its own is + half, the other half of whose codes is with the lane
         // sixteen on
         const uint4 ones = make_uint4(0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u);
-        settle();
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const float d8 = real * f16_bits_to_f32(b.head[h] & 0xFFFFu);
-            table[(4 * h + grp) * TOKS + tok] = d8;
             int sums[2];
 #pragma unroll
             for (int nib = 0; nib < 2; ++nib) {
-                const u32x4 v = b.a[2 * h + nib];
+                const u32x4 v = a[2 * h + nib];
                 sums[nib] = dot16(ones, make_uint4(v[0], v[1], v[2], v[3]), 0);
             }
             const int other = __builtin_amdgcn_ds_swizzle(half ? sums[0] : sums[1], 0x401F);   // lane ^ 16
-            d8s[h] = d8 * (float)((half ? sums[1] : sums[0]) + other);
+            d8s[h] = table[(4 * h + grp) * TOKS + tok] * (float)((half ? sums[1] : sums[0]) + other);
         }
-        settle();
     };
-    auto compute = [&](const Act& b, const WFrag& w, float (&sum)[T16 ? 2 : 1][4]) {
+    auto compute = [&](const WFrag& w, float (&sum)[T16 ? 2 : 1][4]) {
         // (accumulators from the bit pattern of 1.5 * 2^23, the offset off again in the first fused multiply-add, exactly: rows16_core.h)
         constexpr int MAGIC_BITS = 0x4B400000;
         constexpr float MAGIC = 12582912.0f;
@@ -155,8 +171,8 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
                 uint32_t x = (nib ? q[e] >> 4 : q[e]) & 0x0F0F0F0Fu;
                 if (Q5) x |= ((hp[e] >> (4 * c2 + nib)) & 0x01010101u) << 4;
                 codes[e] = (int)x;
-                a0[e] = live ? (int)b.a[u][e] : 0;
-                a1[e] = live ? 0 : (int)b.a[u][e];
+                a0[e] = live ? (int)a[u][e] : 0;
+                a1[e] = live ? 0 : (int)a[u][e];
             }
             const uint32_t scw = c2 ? sc_hi : sc_lo;
             fold(sum[0], __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, codes, magic, 0, 0, 0), d * (float)((scw >> (8 * nib)) & 0xFFu), 4 * c2 + nib);
@@ -181,11 +197,27 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
         }
     };
 
-    if constexpr (NT == 1) {   // two super-blocks in flight
+    WFrag w[2];   // NT 1: of two super-blocks; else of two tiles
+    if constexpr (NT == 1 && Q5 && T16) {   // (one activation set: registers. With two 4096 x 14336 takes 19.7 us against 17.5; the others lose 5 % with one)
+        Act act;
+        load_act(act, wave);
+        load_w(w[0], 0, wave);
+        if (wave + waves < p.nb) load_w(w[1], 0, wave + waves);
+        for (int kb = wave; kb < p.nb; kb += 2 * waves) {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                const int at = kb + d * waves;
+                if (at >= p.nb) break;
+                settle_act(act);
+                if (at + waves < p.nb) load_act(act, at + waves);
+                compute(w[d], acc[0]);
+                if (at + 2 * waves < p.nb) load_w(w[d], 0, at + 2 * waves);
+            }
+        }
+    } else if constexpr (NT == 1) {
         Act act[2];
-        WFrag w[2];
-        auto load = [&](int d, int kb) { load_act(act[d], kb), load_w(w[d], w_lane[0], kb); };
-        auto step = [&](int d) { scales(act[d]), compute(act[d], w[d], acc[0]); };
+        auto load = [&](int d, int kb) { load_act(act[d], kb), load_w(w[d], 0, kb); };
+        auto step = [&](int d) { settle_act(act[d]), compute(w[d], acc[0]); };
         load(0, wave);
         if (wave + waves < p.nb) load(1, wave + waves);
         for (int kb = wave; kb < p.nb; kb += 2 * waves) {
@@ -196,21 +228,20 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
                 if (kb + 3 * waves < p.nb) load(1, kb + 3 * waves);
             }
         }
-    } else {   // two tiles' weights
+    } else {
         Act act;
-        WFrag w[2];
         load_act(act, wave);
-        load_w(w[0], w_lane[0], wave);
-        load_w(w[1], w_lane[1], wave);
+        load_w(w[0], 0, wave);
+        load_w(w[1], 1, wave);
         for (int kb = wave; kb < p.nb; kb += waves) {
-            scales(act);
+            settle_act(act);
 #pragma unroll
             for (int i = 0; i < NT; ++i) {
-                compute(act, w[i & 1], acc[i]);
-                if (i + 2 < NT) load_w(w[i & 1], w_lane[(i + 2) % NT], kb);
-                else if (kb + waves < p.nb) load_w(w[i & 1], w_lane[(i + 2) % NT], kb + waves);
+                compute(w[i & 1], acc[i]);
+                if (i + 2 < NT) load_w(w[i & 1], i + 2, kb);
+                else if (kb + waves < p.nb) load_w(w[i & 1], i + 2 - NT, kb + waves);
             }
-            if (kb + waves < p.nb) load_act(act, kb + waves);
+            if (kb + waves < p.nb) load_act(act, kb + waves);   // (not before: registers)
         }
     }
 
@@ -286,7 +317,7 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
     int tiles = 0;
     for (int i = 0; i < (dual ? 1 : a.count); ++i) tiles += (a.n[i] + TILE - 1) / TILE;
     if (tiles == 0) return LK_OK;
-    // more than eight rows: two sets of eight where both are resident at once (Q4_K 2048 x 6144 at 16 rows 8.5 us against 9.1)
+    // more than eight rows: two sets of eight where both are resident at once (Q4_K 1024 x 2048 at 16 rows 4.2 us against 4.4 with sixteen)
     const bool eight = a.m <= 8 || (!dual && 2 * tiles <= lk_device().cus);
     if (eight) return q5 ? launch_out<true, 8>(a, dual, tiles, stream) : launch_out<false, 8>(a, dual, tiles, stream);
     return q5 ? launch_out<true, 16>(a, dual, tiles, stream) : launch_out<false, 16>(a, dual, tiles, stream);
@@ -296,9 +327,9 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
 // once and walk many tiles are ahead; above a tile to the CU rows of 2048 values or more, and at most 8192 up to eight rows. A choice by the matrix
 // and the class of row counts alone, so that several matrices in one launch carry the bits of one launch each, and not above sixteen rows, where a row
 // carries the 32-row tiles' bits whatever rides with it. Measured in a graph, Q4_K, us, staged launches against this:
-//   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.8, 4.1; 4096 x 4096 7.7, 8.1 / 5.6, 6.2; 4096 x 14336 17.9, 19.4 / 13.2, 15.6; 6144 x 2048 5.5, 5.5 / 5.0, 5.4;
+//   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.7, 3.7; 4096 x 4096 7.7, 8.1 / 5.1, 5.0; 4096 x 14336 17.9, 19.4 / 12.0, 11.9; 6144 x 2048 5.5, 5.5 / 5.0, 5.4;
 //                8192 x 4096 8.9, 9.1 / 7.7, 8.3; 8192 x 1024 4.2, 4.1 / 4.0, 4.2; 5000 x 12288 16.7, 17.7 / 15.9, 18.3; 10000 x 5120 (three to the CU) 12.9, 13.6 / 13.2, 16.0
-//   9 / 16 rows  2048 x 2048 5.9, 6.4 / 4.5, 4.5; 4096 x 4096 9.4, 10.2 / 6.2, 6.9; 2048 x 6144 12.1, 13.2 / 8.4, 8.5; 4096 x 14336 28.8, 32.2 / 16, 19;
+//   9 / 16 rows  2048 x 2048 5.9, 6.4 / 4.0, 3.9; 4096 x 4096 9.4, 10.2 / 5.6, 5.6; 2048 x 6144 12.1, 13.2 / 6.4, 6.4; 4096 x 14336 28.8, 32.2 / 13.6, 14.7;
 //                8192 x 4096 10.3, 11.0 / 8.5, 9.3; 5000 x 12288 25.8, 28.7 / 18.4, 21.1; 8192 x 1024 4.2, 4.3 / 4.9, 5.1; 10000 x 5120 15.3, 16.3 / 16.3, 17.8
 // (Rows of up to 32768 values: longer ones are the other launches' to take or refuse.)
 bool lk_rows16_short_pays(int m, int n, int nb) {
