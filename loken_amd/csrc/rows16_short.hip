@@ -44,7 +44,7 @@ static __device__ __forceinline__ TileRef tile_of(const LkRows16& p, int wg, int
     return {mat, tile};
 }
 
-static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q81) { return waves * nt * PART_BYTES + (q81 ? MAX_TOKS * 32 * 4 : 0); }
+static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q81) { return waves * nt * PART_BYTES + (q81 ? MAX_TOKS * nt / 4 * 32 * 4 : 0); }
 
 // grid.x workgroups of NT row tiles each (one; two where one would be more workgroups than CUs, and for a gate and its up; four for
 // the 32 rows of a Q8_1 block), 64 * waves threads: wave w takes super-blocks w, w + waves, ... of every one of them, against one reading of the
@@ -52,7 +52,7 @@ static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q
 template <bool Q5, int TOKS, int OUT, int NT>
 __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows16 p, int n_tiles) {
     static_assert(TOKS == 8 || TOKS == 16, "eight or sixteen activation rows");
-    static_assert(NT == 1 || NT == 2 || NT == 4, "tiles in turn through two sets of weight registers");
+    static_assert(NT == 1 || NT % 2 == 0, "tiles in turn through two sets of weight registers");
     constexpr bool T16 = TOKS == 16, DUAL = OUT >= DUAL_F32;
     extern __shared__ __align__(16) uint8_t lds[];
     const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4, half = grp & 1, par = grp >> 1;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     __syncthreads();
     // sixteen rows: output (register v, lane l < 64) adds the waves' lanes l; eight: (v, l < 32) lanes l and l + 32
     constexpr int LANES = 4 * TOKS, OUTS = DUAL ? NT / 2 : NT;
-    float* meet = (float*)(lds + waves * NT * PART_BYTES);   // Q8_1 output: [TOKS][32]
+    float* meet = (float*)(lds + waves * NT * PART_BYTES);   // Q8_1 output: [TOKS][8 NT]
     for (int o = threadIdx.x; o < OUTS * 4 * LANES; o += (int)blockDim.x) {
         const int r = o / (4 * LANES), v = o / LANES & 3, l = o % LANES;
         auto total = [&](int i) {
@@ -272,7 +272,7 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
         }
         const int t = 4 * (l >> 4) + v;
         if constexpr (OUT == DUAL_Q81) {
-            meet[t * 32 + 16 * r + (l & 15)] = sum;   // (n is a multiple of 32: both tiles are whole)
+            meet[t * (8 * NT) + 16 * r + (l & 15)] = sum;
         } else {
             const TileRef at = tile_of<OUT, NT>(p, blockIdx.x, DUAL ? 2 * r : r);
             const int row = at.tile * TILE + (l & 15), mat = DUAL ? 0 : at.mat;
@@ -281,10 +281,15 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     }
     if constexpr (OUT == DUAL_Q81) {
         __syncthreads();
-        // eight lanes per activation row write its block
+        // eight lanes per (activation row, block of 32 results) write it (n is a multiple of 32: a block's two tiles are whole or both missing)
+        constexpr int BLOCKS = NT / 4;
         const int l8 = threadIdx.x & 7;
-        for (int row = (int)threadIdx.x >> 3; row < m_rows; row += (int)blockDim.x / 8)
-            lk_store_q8_1_block(*(const float4*)(meet + row * 32 + 4 * l8), l8, (uint32_t*)(p.q81_dst + ((size_t)(m0 + row) * p.q81_stride + blockIdx.x) * Q81_BYTES));
+        for (int o = (int)threadIdx.x >> 3; o < m_rows * BLOCKS; o += (int)blockDim.x / 8) {
+            const int row = o / BLOCKS, at = o % BLOCKS, block = (int)blockIdx.x * BLOCKS + at;
+            if (32 * block < p.n[0])
+                lk_store_q8_1_block(*(const float4*)(meet + row * (8 * NT) + 32 * at + 4 * l8), l8,
+                                    (uint32_t*)(p.q81_dst + ((size_t)(m0 + row) * p.q81_stride + block) * Q81_BYTES));
+        }
     }
 }
 
@@ -300,12 +305,23 @@ int launch(const LkRows16& a, int tiles, hipStream_t stream) {
     return lk_launch_status();
 }
 
+// Tiles to a workgroup: as many as bring the launch to a workgroup to the CU; past two of a matrix to the CU only up to eight rows (registers).
 template <bool Q5, int TOKS>
 int launch_out(const LkRows16& a, bool dual, int tiles, hipStream_t stream) {
+    const int cus = lk_device().cus;
+    if constexpr (TOKS == 8) {
+        if (tiles > 2 * cus) {
+            if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 8>(a, tiles, stream);
+            if (dual) return launch<Q5, TOKS, DUAL_F32, 8>(a, tiles, stream);
+            return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 4>(a, tiles, stream) : launch<Q5, TOKS, ANY, 4>(a, tiles, stream);
+        }
+    }
     if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 4>(a, tiles, stream);
-    const bool pairs = tiles > lk_device().cus;
-    if (dual) return pairs ? launch<Q5, TOKS, DUAL_F32, 4>(a, tiles, stream) : launch<Q5, TOKS, DUAL_F32, 2>(a, tiles, stream);
-    if (pairs) return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 2>(a, tiles, stream) : launch<Q5, TOKS, ANY, 2>(a, tiles, stream);
+    if (tiles > cus) {
+        if (dual) return launch<Q5, TOKS, DUAL_F32, 4>(a, tiles, stream);
+        return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 2>(a, tiles, stream) : launch<Q5, TOKS, ANY, 2>(a, tiles, stream);
+    }
+    if (dual) return launch<Q5, TOKS, DUAL_F32, 2>(a, tiles, stream);
     return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 1>(a, tiles, stream) : launch<Q5, TOKS, ANY, 1>(a, tiles, stream);
 }
 
@@ -323,16 +339,17 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
     return q5 ? launch_out<true, 16>(a, dual, tiles, stream) : launch_out<false, 16>(a, dual, tiles, stream);
 }
 
-// Matrices of up to two row tiles to the CU: with more workgroups than CUs, or more tiles to a workgroup, the launches that stage the activation
-// once and walk many tiles are ahead; above a tile to the CU rows of 2048 values or more, and at most 8192 up to eight rows. A choice by the matrix
-// and the class of row counts alone, so that several matrices in one launch carry the bits of one launch each, and not above sixteen rows, where a row
-// carries the 32-row tiles' bits whatever rides with it. Measured in a graph, Q4_K, us, staged launches against this:
-//   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.7, 3.7; 4096 x 4096 7.7, 8.1 / 5.1, 5.0; 4096 x 14336 17.9, 19.4 / 12.0, 11.9; 6144 x 2048 5.5, 5.5 / 5.0, 5.4;
-//                8192 x 4096 8.9, 9.1 / 7.7, 8.3; 8192 x 1024 4.2, 4.1 / 4.0, 4.2; 5000 x 12288 16.7, 17.7 / 15.9, 18.3; 10000 x 5120 (three to the CU) 12.9, 13.6 / 13.2, 16.0
+// Matrices of up to four row tiles to the CU, two above eight rows: with more the launches that stage the activation once and walk many tiles are level
+// or ahead; above a tile to the CU rows of 2048 values or more. A choice by the matrix and the class of row counts alone, so that several
+// matrices in one launch carry the bits of one launch each, and not above sixteen rows, where a row carries the 32-row tiles' bits whatever rides with
+// it. Measured in a graph, Q4_K, us, staged launches against this:
+//   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.7, 3.7; 4096 x 4096 7.7, 8.1 / 5.1, 5.0; 4096 x 14336 17.9, 19.4 / 12.0, 11.9; 6144 x 2048 5.5, 5.5 / 4.9, 4.9;
+//                8192 x 4096 8.8, 9.1 / 7.3, 7.2; 5000 x 12288 16.7, 17.8 / 14.7, 15.0; 14336 x 4096 12.6, 13.3 / 10.6, 10.5; 8192 x 1024 4.2, 4.1 / 4.0, 4.2;
+//                18944 x 3584 (five to the CU) 14.1, 14.4 / 15.2, 15.4
 //   9 / 16 rows  2048 x 2048 5.9, 6.4 / 4.0, 3.9; 4096 x 4096 9.4, 10.2 / 5.6, 5.6; 2048 x 6144 12.1, 13.2 / 6.4, 6.4; 4096 x 14336 28.8, 32.2 / 13.6, 14.7;
-//                8192 x 4096 10.3, 11.0 / 8.5, 9.3; 5000 x 12288 25.8, 28.7 / 18.4, 21.1; 8192 x 1024 4.2, 4.3 / 4.9, 5.1; 10000 x 5120 15.3, 16.3 / 16.3, 17.8
+//                8192 x 4096 10.3, 11.0 / 7.9, 8.0; 5000 x 12288 25.9, 28.6 / 16.9, 16.9; 8192 x 1024 4.2, 4.3 / 4.9, 5.1; 14336 x 4096 14.4, 15.4 / 16.0, 16.6
 // (Rows of up to 32768 values: longer ones are the other launches' to take or refuse.)
 bool lk_rows16_short_pays(int m, int n, int nb) {
     const int tiles = (n + TILE - 1) / TILE, cus = lk_device().cus;
-    return m >= 1 && m <= MAX_TOKS && nb <= 128 && (tiles <= cus || (tiles <= 2 * cus && nb >= 8 && (m > 8 || nb <= 32)));
+    return m >= 1 && m <= MAX_TOKS && nb <= 128 && (tiles <= cus || (tiles <= (m <= 8 ? 4 : 2) * cus && nb >= 8));
 }

@@ -317,7 +317,7 @@ def test_q6k_eight_rows_or_fewer_in_sixteen_row_tiles(m, k, n):
 
 @pytest.mark.parametrize("q5", [False, True])
 @pytest.mark.parametrize("m,k,n", [(1, 256, 1), (4, 768, 16), (5, 4352, 17), (8, 4096, 4096), (8, 2048, 4097), (9, 4096, 2048), (16, 8448, 2049),
-                                   (13, 12544, 40), (3, 2304, 4112), (11, 8192, 4000), (8, 8192, 4500), (9, 8448, 8192), (16, 2048, 8193), (17, 512, 100)])
+                                   (13, 12544, 40), (3, 2304, 4112), (11, 8192, 4000), (8, 8192, 4500), (9, 8448, 8192), (16, 2048, 8193), (7, 2304, 8200), (5, 2048, 16384), (8, 4096, 16385), (17, 512, 100)])
 def test_few_row_tiles_take_the_short_launch(m, k, n, q5):
     """rows16_short.hip: one to four super-blocks a wave, groups without a last one, sets of eight with a last set of one, two groups to a
     wave, both sides of its line in row tiles; several matrices on both sides of it carry the single launches' bits."""
@@ -331,6 +331,22 @@ def test_few_row_tiles_take_the_short_launch(m, k, n, q5):
     ws, sizes = ([dev(w), small], (n, 33)) if big is None else ([dev(w), small, big], (n, 33, 8200))
     for one, size, out in zip(ws, sizes, ops.dense_q4k_rows_multi(ws, dev(x), sizes, q5=q5)):
         assert torch.equal(out, fn(one, dev(x), size, q5=q5))
+
+
+@pytest.mark.parametrize("q5", [False, True])
+@pytest.mark.parametrize("m,k,n", [(8, 2048, 8224), (3, 4096, 8256), (5, 2048, 16384), (16, 2048, 4128), (12, 4096, 8192), (8, 4096, 64), (8, 2048, 4128)])
+def test_gate_and_up_through_the_short_launch(m, k, n, q5):
+    """rows16_short.hip with two, four and eight tiles to a workgroup and a last group that is not whole: the plain launches' products (SiLU recomputed from
+    them differs by the device's exp alone) and, as Q8_1 rows, the quantizer's bytes."""
+    wtype = lib.TYPE_Q5_K if q5 else Q4K
+    gate, up = dev(synth.weight(wtype, n, k, seed=81, stream=1)), dev(synth.weight(wtype, n, k, seed=81, stream=2))
+    x = dev(synth.activation(m, k, seed=81))
+    g, u = ops.dense_q4k_rows(gate, x, n, q5=q5).double(), ops.dense_q4k_rows(up, x, n, q5=q5).double()
+    want = g / (1.0 + torch.exp(-g)) * u
+    got = ops.dense_q4k_rows_actmul(gate, up, x, n, False, q5=q5)
+    assert ((got.double() - want).abs() <= 2e-6 * want.abs() + 1e-30).all()
+    q81 = ops.dense_q4k_rows_actmul_q8_1(gate, up, x, n, False, q5=q5)
+    assert torch.equal(q81.reshape(-1), ops.quantize_q8_1_rows(got, k_padded=n).reshape(-1))
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 3328, 5), (8, 3072, 16), (9, 3328, 31), (16, 6400, 100), (7, 2304, 6150), (16, 1792, 6100), (15, 4096, 2080),
