@@ -61,13 +61,17 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     float* part = (float*)(lds + wave * NT * PART_BYTES);
     float* table = part;   // d8 [8][TOKS] of the super-block in hand
 
+    // The weights too are asked for in the order they lie in, four lanes to a row's 64 bytes, and handed to the operand's lanes, where the registers hold the
+    // code before and after (8192 x 14336 at 8 rows 19.1 us -> 17.5, 5000 x 12288 14.9 -> 12.4; sixteen rows with four tiles spill and go 7.5 -> 9.8)
+    constexpr bool IN_ORDER = !T16 || (NT == 2 && !Q5);
+    const int w_tile_row = IN_ORDER ? lane >> 2 : l16, w_piece = IN_ORDER ? lane & 3 : grp;
     const uint8_t* w_base[NT];   // each tile's matrix, and the lane's row in it (past the last tile: of the last)
     uint32_t w_row[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const TileRef r = DUAL ? tile_of<OUT, NT>(p, blockIdx.x, i) : tile_of<OUT, 1>(p, min((int)blockIdx.x * NT + i, n_tiles - 1), 0);
         w_base[i] = (const uint8_t*)to_gbytes(pick3(p.w, r.mat));
-        w_row[i] = (uint32_t)min(r.tile * TILE + l16, pick3(p.n, r.mat) - 1) * (uint32_t)(p.nb * Blk<Q5>::BYTES);
+        w_row[i] = (uint32_t)min(r.tile * TILE + w_tile_row, pick3(p.n, r.mat) - 1) * (uint32_t)(p.nb * Blk<Q5>::BYTES);
     }
     const int tok = l16 & (TOKS - 1);
     // The activation is asked for in the order it lies in, a row's pieces by neighbouring lanes, and handed to the operand's lanes by a
@@ -104,9 +108,9 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
         for (int u = 0; u < LOADS; ++u) b.raw[u] = *(const u32x4_a4*)(y_codes + at + (T16 ? 4 * (u >> 1) + (u & 1) : 4 * u) * Q81_BYTES);
     };
     auto load_w = [&](WFrag& w, int i, int kb) {
-        const uint32_t at = w_row[i] + (uint32_t)(kb * Blk<Q5>::BYTES), at_q = at + 16 * grp;
+        const uint32_t at = w_row[i] + (uint32_t)(kb * Blk<Q5>::BYTES), at_q = at + 16 * w_piece;
         w.hdr = *(const uint4*)(w_base[i] + at);
-        if (Q5) w.qh = *(const uint4*)(w_base[i] + (at + 16 * half) + 16);
+        if (Q5) w.qh = *(const uint4*)(w_base[i] + (at + 16 * (w_piece & 1)) + 16);
         w.q[0] = *(const uint4*)(w_base[i] + at_q + Blk<Q5>::QS);
         w.q[1] = *(const uint4*)(w_base[i] + at_q + Blk<Q5>::QS + 64);
     };
@@ -144,7 +148,13 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
             d8s[h] = table[(4 * h + grp) * TOKS + tok] * (float)((half ? sums[1] : sums[0]) + other);
         }
     };
-    auto compute = [&](const WFrag& w, float (&sum)[T16 ? 2 : 1][4]) {
+    auto to_lane = [&](const uint4& v) {
+        if constexpr (!IN_ORDER) return v;
+        const int w_from = 4 * (4 * l16 + grp);
+        return make_uint4((uint32_t)__builtin_amdgcn_ds_bpermute(w_from, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(w_from, (int)v.y),
+                          (uint32_t)__builtin_amdgcn_ds_bpermute(w_from, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(w_from, (int)v.w));
+    };
+    auto compute = [&](const WFrag& raw, float (&sum)[T16 ? 2 : 1][4]) {
         // (accumulators from the bit pattern of 1.5 * 2^23, the offset off again in the first fused multiply-add, exactly: rows16_core.h)
         constexpr int MAGIC_BITS = 0x4B400000;
         constexpr float MAGIC = 12582912.0f;
@@ -157,6 +167,11 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
             s[2] = fmaf(fmaf(__int_as_float(c[2]), dsc, off), t.z, s[2]);
             s[3] = fmaf(fmaf(__int_as_float(c[3]), dsc, off), t.w, s[3]);
         };
+        WFrag w;
+        w.hdr = to_lane(raw.hdr);
+        if (Q5) w.qh = to_lane(raw.qh);
+        w.q[0] = to_lane(raw.q[0]);
+        w.q[1] = to_lane(raw.q[1]);
         const uint32_t w1 = w.hdr.y, w2 = w.hdr.z, w3 = w.hdr.w;
         const uint32_t sc_lo = (w1 & 0x3F3F3F3Fu) >> sh16, sc_hi = ((w3 & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u)) >> sh16;
         const float d = f16_bits_to_f32(w.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(w.hdr.x >> 16);
