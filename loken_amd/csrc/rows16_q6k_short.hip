@@ -243,8 +243,9 @@ int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size
     const int nb = size_k / 256, tiles = (size_n + TILE - 1) / TILE, cus = lk_device().cus;
     const bool granules = nb % 8 == 0, held = granules && tiles <= cus && (size_t)size_n * nb * Q6K_BYTES <= (64u << 20);
     if (granules && size_m <= 8 && nb >= 32 && (2 * tiles <= cus || (size_m <= 4 && nb >= 48))) return -1;
+    if (granules && size_m <= 4 && nb > 8 && tiles > cus) return -1;   // (6144 x 6144 at 3 rows 12.6 / 15.0)
     const int eights = (size_m + 7) / 8, sixteens = (size_m + 15) / 16;
-    const int64_t most = size_m <= 16 ? (granules ? 3 * cus / 2 : 3 * cus) : size_m > 32 ? 2 * cus : held ? cus : granules ? 2 * cus : 3 * cus;
+    const int64_t most = size_m <= 16 ? (granules ? 3 * cus / 2 : 3 * cus) : size_m > 32 ? 2 * cus : held && nb < 32 ? cus : granules ? 2 * cus : 3 * cus;
     const bool by_eight = size_m <= 8 || (int64_t)tiles * eights <= cus;
     if ((int64_t)tiles * (by_eight ? eights : sixteens) > most) return -1;
     const int steps = (nb + MAX_WAVES - 1) / MAX_WAVES, waves = (nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow

@@ -55,6 +55,7 @@ struct WFrag {
     uint32_t d;    // f16 bits
 };
 
+// (the pieces of half `lh`)
 static __device__ __forceinline__ void load_weights(WFrag& f, const uint8_t* bp, int lh) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) f.ql[c] = *(const uint4_a2*)(bp + 32 * c + 16 * lh);
@@ -106,17 +107,32 @@ static __device__ __forceinline__ void fold_quarter(const v16i& c0, const v16i& 
 }
 
 // One super-block of the wave's 32 rows against the activation codes `a_of(quarter)` supplies.
+// Weights (and, unstaged, activation codes) are asked for in the order they lie in, two neighbouring lanes to 32 bytes of a row, and handed to the lanes the
+// matrix instruction wants them in (row l32, half lh) by a permutation: in that order itself every lane of a load has a line of its own, and the
+// loads cost more than the arithmetic. `from`: the byte address of the lane that asked for this lane's piece.
+static __device__ __forceinline__ uint4 to_lane(const uint4& v, int from) {
+    return make_uint4((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)v.y),
+                      (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)v.w));
+}
+
 template <int G, class AOf>
-static __device__ __forceinline__ void block_step(const WFrag& w, bool live, int sub0, const float* d8_table, int lh,
+static __device__ __forceinline__ void block_step(const WFrag& w, bool live, int sub0, const float* d8_table, int lh, int from,
                                                   uint32_t keep0, uint32_t keep1, AOf&& a_of, float acc[4 * G]) {
     constexpr int TW = 8 * G;
     constexpr int MAGIC_BITS = 0x4B400000;
-    const float d = live ? f16_bits_to_f32(w.d) : 0.f;
-    const uint32_t scd[4] = {w.sc.x, w.sc.y, w.sc.z, w.sc.w};
+    const float d = live ? f16_bits_to_f32((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)w.d)) : 0.f;
+    const uint4 sc = to_lane(w.sc, from);
+    const uint32_t scd[4] = {sc.x, sc.y, sc.z, sc.w};
+    uint4 ql[2], qh;   // of the half in hand
     auto quarter = [&](auto half_c, auto qt_c) {
         constexpr int HALF = decltype(half_c)::value, QT = decltype(qt_c)::value;
+        if constexpr (QT == 0) {
+            qh = to_lane(w.qh[HALF], from);
+            ql[0] = to_lane(w.ql[2 * HALF], from);
+            ql[1] = to_lane(w.ql[2 * HALF + 1], from);
+        }
         uint32_t z[4];
-        quarter_codes<QT>(w.ql[2 * HALF + (QT & 1)], w.qh[HALF], z);
+        quarter_codes<QT>(ql[QT & 1], qh, z);
         const v4i b0 = {(int)(z[0] & keep0), (int)(z[1] & keep0), (int)(z[2] & keep0), (int)(z[3] & keep0)};
         const v4i b1 = {(int)(z[0] & keep1), (int)(z[1] & keep1), (int)(z[2] & keep1), (int)(z[3] & keep1)};
         const v4i a = a_of(4 * HALF + QT);
@@ -163,6 +179,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
+    const int ld_row = lane >> 1, ld_half = lane & 1, from = 4 * (2 * l32 + lh);   // what the lane asks for, who has what it wants
     const uint32_t keep0 = lh ? 0u : 0xFFFFFFFFu, keep1 = ~keep0;
     const int m0 = STAGED ? 0 : blockIdx.y * TOK;
     const int m_count = min(STAGED ? TW : TOK, p.m - m0);
@@ -176,7 +193,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
     const int total = my_tiles * my_blocks;
     auto weights_at = [&](int j) {
         const int tile = blockIdx.x + (j / my_blocks) * gridDim.x, kb = wave + (j % my_blocks) * WAVES;
-        const int row = min(tile * 32 + l32, p.n - 1);
+        const int row = min(tile * 32 + ld_row, p.n - 1);
         return (const uint8_t*)(to_gbytes(p.w) + row * row_bytes + (size_t)kb * Q6K_BYTES);
     };
 
@@ -242,7 +259,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
         issue(threadIdx.x);
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d)
-            if (d < total) load_weights(f[d], weights_at(d), lh);
+            if (d < total) load_weights(f[d], weights_at(d), ld_half);
         place(threadIdx.x);
         for (int r = WG * PER; r < entries; r += WG * PER) {
             issue(r + threadIdx.x);
@@ -262,9 +279,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
                 const int j = j0 + d;
                 if (j < total) {
                     const int kb = wave + (j % my_blocks) * WAVES;
-                    block_step<G>(f[d], true, kb * 8, d8_table, lh, keep0, keep1,
+                    block_step<G>(f[d], true, kb * 8, d8_table, lh, from, keep0, keep1,
                                   [&](int q) { return *(const v4i*)(a_lane + (size_t)(kb * 8 + q) * TW * 32); }, acc);
-                    if (j + DEPTH < total) load_weights(f[d], weights_at(j + DEPTH), lh);
+                    if (j + DEPTH < total) load_weights(f[d], weights_at(j + DEPTH), ld_half);
                     if ((j + 1) % my_blocks == 0) finish_tile(j / my_blocks);
                 }
             }
@@ -286,14 +303,14 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
                 if (idx < entries) d8_table[idx] = idx % TW < m_count ? f16_bits_to_f32(bits[u]) : 0.f;
             }
         }
-        // The lane's activation row (a row past the end re-reads the last one; its scales are zero).
-        const uint8_t* y_lane = y0 + (size_t)min(l32, m_count - 1) * p.stride_y * Q81_BYTES + 4 + 16 * lh;
+        // The activation row the lane asks for (past the end the last one again; its scales are zero).
+        const uint8_t* y_lane = y0 + (size_t)min(ld_row, m_count - 1) * p.stride_y * Q81_BYTES + 4 + 16 * ld_half;
         struct Frag {
             WFrag w;
             v4i a[8];
         };
         auto load = [&](Frag& f, int j) {
-            load_weights(f.w, weights_at(j), lh);
+            load_weights(f.w, weights_at(j), ld_half);
             const int kb = wave + (j % my_blocks) * WAVES;
             const uint8_t* ap = y_lane + (size_t)kb * 8 * Q81_BYTES;
 #pragma unroll
@@ -311,7 +328,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void q6k_rows_kerne
         }
         auto step = [&](const Frag& f, int j) {
             const int kb = wave + (j % my_blocks) * WAVES;
-            block_step<G>(f.w, true, kb * 8, d8_table, lh, keep0, keep1, [&](int q) { return f.a[q]; }, acc);
+            block_step<G>(f.w, true, kb * 8, d8_table, lh, from, keep0, keep1, [&](int q) {
+                const uint4 v = to_lane(make_uint4((uint32_t)f.a[q][0], (uint32_t)f.a[q][1], (uint32_t)f.a[q][2], (uint32_t)f.a[q][3]), from);
+                return v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+            }, acc);
             if ((j + 1) % my_blocks == 0) finish_tile(j / my_blocks);
         };
         for (int j = 0; j < total; j += 2) {
