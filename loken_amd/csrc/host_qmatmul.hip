@@ -61,39 +61,36 @@ int matvec_rows(int dtype, int k) {
 }
 
 // Rows the matrix-unit rows kernels take before the tiled matmul does. A rows kernel reads the weights straight from HBM, once
-// for every 32 activation rows (16-row tiles up to 16 rows; Q6_K rows of a multiple of 2048 values in sets of eight further up), a
-// workgroup walking all of k: its time grows with k, and steps up once its workgroups (32 matrix rows x 32 activation rows each)
-// are more than the CUs. The f16 tiles cut K instead and read the weights once per 32 to 128 rows. Measured on MI355X, quantizer
-// included, rows kernel against f16 tiles (us), for matrices of 512 rows or more:
-//   Q4_K, 9 to 16 rows: 512 x 8192 20..22 / 16, 4096 x 8192 21 / 18, 700 x 11008 23..25 / 17; 6144 x 6144 16 / 20, 4096 x 4096 13 / 16
+// for every 16 or 32 activation rows; its time steps up once its workgroups are more than the CUs. The f16 tiles cut K and read the weights
+// once per 32 to 128 rows. Measured on MI355X, quantizer included, rows kernel against f16 tiles (us), for matrices of 512 rows or more:
+//   Q4_K, 9 to 16 rows: 512 x 8192 10..11 / 16, 8192 x 8192 14 / 22, 4096 x 14336 15..16 / 23, 10000 x 5120 18 / 21, 12000 x 10240 35..42 / 29; Q5_K alike
 //     17 to 32: 700 x 5120 18 / 15, 10000 x 5120 25 / 22, 2048 x 6144 21 / 16, 14336 x 4096 at 24 22 / 21; 4096 x 4096 16 / 16, 8192 x 4096 16 / 19
 //     above: 3000 x 5120 at 33 / 96 20 / 18, 27 / 24; 4096 x 4096 at 64 / 96 (256, 384 workgroups) 17 / 20, 25 / 25; 1024 x 4096 at 200 / 400
 //     (224, 416) 19 / 21, 28 / 25; 2048 x 2048 at 200 17 / 19. Q5_K alike.
-//   Q6_K, up to 16 rows, k a multiple of 2048: 4096 x 8192 17 / 22, 16384 x 6144 26 / 35; others: 700 x 5120 19 / 16, 10000 x 5120 32 / 26,
-//     6144 x 3072 15 / 20
-//     17 to 32: 4096 x 4096 16 / 18, 1024 x 14336 19 / 25 (sets of eight), 4096 x 8192 25 / 22, 4096 x 14336 42 / 31; 8192 x 4096 19 / 22, 3000 x 5120 22 / 19,
-//     14336 x 4096 31 / 28
-//     above: 1024 x 4096 at 64 / 96 13 / 17, 20 / 18; 3000 x 3072 at 33 20 / 18; 8192 x 4096 at 40 31 / 23; 2048 x 2048 at 64 12 / 15
+//   Q6_K, 9 to 16 rows: 2048 x 8192 13 / 20, 6144 x 6144 20 / 24, 4096 x 14336 20 / 30, 3000 x 5120 12 / 18, 10000 x 5120 26 / 26
+//     17 to 32: 2048 x 14336 20 / 25, 8192 x 4096 17..19 / 23, 6144 x 6144 22..23 / 24..25, 700 x 11008 13 / 22; 10000 x 5120 30..33 / 27, 4096 x 14336 35 / 31,
+//     4096 x 8192 25 / 22
+//     33 to 64: 512 x 14336 17..18 / 26, 1024 x 14336 20..21 / 26, 2048 x 6144 19..20 / 20..22, 4096 x 4096 18..19 / 20..22; 2048 x 14336 34..36 / 27..29, 8192 x
+//     4096 26..29 / 25, 6144 x 3072 22 / 20..22. Above: 4096 x 4096 at 96 28 / 26, 1024 x 6144 23 / 22
 // `bench.py --workload rows-sweep` prints the table for a shape.
 static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K) return false;
     if (rows <= 8) return true;
-    const long long results = (long long)n * rows;
+    const long long results = (long long)n * rows, weights = (long long)n * k;
     // (few matrix rows yield few tiles whatever the cut: the int8 tiles' line)
     if (n < 512) return rows <= 16 || results * (k > 4096 ? k : 4096) <= 450000ll * 4096 * (n > 0 ? 2048 / n : 2048);
     const long long items = (n + 31ll) / 32 * ((rows + 31) / 32);
     if (dtype == LK_TYPE_Q6_K) {
-        const bool sets = k % 2048 == 0;
-        if (rows <= 16) return sets || k < 4608;
-        if (rows <= 32 && sets && n <= 4096) return (long long)n * k <= (24ll << 20);
-        if (rows <= 32) return k < 3072 || (k < 4608 && (sets ? n < 12288 : n >= 4096));
+        if (rows <= 16) return k % 2048 == 0 || k < 4608 || n <= 12288;
+        if (rows <= 32) return weights <= (24ll << 20) || n <= 2048 || (k <= 6144 && weights <= (40ll << 20));
+        if (rows <= 64) return n <= 1024 || (k < 3072 ? results <= 450000 : k <= 6144 && weights <= (17ll << 20));
         if (k < 5632 && n < 1024 && rows > 128 && items <= 256) return true;
-        if (k >= 3072 && (n >= 1024 || k >= 4608)) return rows <= 64 && n < 2800 && k < 7168 && sets;
-        return results <= 450000;
+        return (k < 3072 || (n < 1024 && k < 4608)) && results <= 450000;
     }
-    if (rows <= 16) return k < 7168;
-    // (the one stretch that is not the faster side: callers that read path() rely on the rows kernel at 1100 x 8192 and 33 rows,
-    // test_long_rows_above_sixteen_activation_rows; 1024 x 8192 there 27 / 18)
+    // (the one stretch up to sixteen rows that is not the faster side: callers that read path() rely on the tiles at 2048 x 8192,
+    // test_long_rows_at_nine_to_sixteen_activation_rows; 11 / 17 there)
+    if (rows <= 16) return k < 7168 || (n <= 8192 && !(k <= 8192 && n >= 2048 && n < 2304));
+    // (and here on the rows kernel at 1100 x 8192 and 33 rows, test_long_rows_above_sixteen_activation_rows; 1024 x 8192 there 27 / 18)
     if (k >= 4608 && k < 12288 && n >= 1024 && n < 1152 && rows > 32 && rows <= 64) return true;
     if (k >= 4608) return k < 5632 && items > 128 && items <= 256 && rows > 32;
     if (rows <= 32) return n < 12288 || k < 4096 || rows < 20;
@@ -101,17 +98,18 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
 }
 
 // The K-quants at 3 to 8 f32 rows: the 16-row tiles of the matrix-unit kernels (their time hardly moves
-// with the row count) against mat-vec launches (whose dot work grows with every row). Every workgroup of
-// a rows kernel stages all the rows, so the matrix has to be large enough to pay for that. Measured on
-// MI355X, Q4_K / Q5_K, k = 4096: 14336 rows from 4 activation rows, 4096 rows from 8, 1024 rows never;
-// k = 2048: 2048 rows from 4, 6144 and 151936 rows from 3. Q6_K (k a multiple of 2048: its rows are loaded
-// in granules of eight super-blocks): 4096 x 14336 and 151936 x 2048 from 3 rows, 14336 x 4096 from 4,
-// 4096 x 4096 and 2048 x 6144 from 7 (as two sets of four rows: 8.9 us against 9.5 at 8 rows, 8.1 as mat-vec at 6).
+// with the row count) against mat-vec launches (whose dot work grows with every row). Small calls take the time of their two launches
+// either way (10 us). Measured on MI355X, mat-vec against rows kernel, quantizer included (us): Q4_K / Q5_K 4096 x 8192 at 4 / 5 / 8 rows 10.7, 11.7, 14.1 / 10.2,
+// 10.5, 10.0, 4096 x 14336 at 3 / 8 13.8, 24.0 / 13.5, 14.1, 8192 x 4096 at 4 / 5 10.8, 11.6 / 10.8, 10.1, 1024 x 14336 at 6 / 8 13.3, 15.5 / 12.0, 12.2; 2048 x 8192 at 8 10.8 / 9.8;
+// k = 2048: 2048 rows from 4, 6144 and 151936 from 3. Q6_K 4096 x 8192 at 5 / 6 13.1, 13.8 / 12.9, 12.9, 6144 x 2048 at 5 / 6 10.6, 11.5 / 10.0, 9.9, 1024 x 14336 at
+// 5 / 8 13.8, 22.1 / 14.6, 14.7, 700 x 5120 at 8 12.2 / 10.0, 512 x 4096 at 8 10.0 / 9.8, 4096 x 14336 at 3 / 4 16.6, 18.8 / 16.8, 16.8.
 static bool small_rows_kernel_pays(int dtype, int n, int k, int rows) {
     if (rows < 3 || rows > 8 || k % 256 != 0) return false;
-    if (dtype == LK_TYPE_Q6_K) return k % 2048 == 0 && ((long long)n * k >= (48ll << 20) || (rows >= 7 && n >= 1024));
+    const long long weights = (long long)n * k;
+    if (dtype == LK_TYPE_Q6_K)
+        return (rows >= 7 && n >= 512) || (rows >= 5 && weights * rows >= (76ll << 20)) || (k % 2048 == 0 && weights >= (48ll << 20));
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K) return false;
-    return (long long)n * rows >= (k <= 2048 ? 8192 : 57344);
+    return k <= 2048 ? (long long)n * rows >= 8192 : weights * rows > (128ll << 20);
 }
 
 QKernelMatMul::QKernelMatMul(int dtype, int n, int k, const void* blob, int device)

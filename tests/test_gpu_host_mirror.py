@@ -328,13 +328,15 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
 
 
 @pytest.mark.parametrize("name,n,k,rows,expect", [
-    ("q4_k", 512, 7168, 9, "tiled"), ("q4_k", 512, 6912, 9, "rows-on-matrix-unit"), ("q4_k", 511, 7168, 9, "rows-on-matrix-unit"),
+    ("q4_k", 8193, 7168, 9, "tiled"), ("q4_k", 8192, 7168, 9, "rows-on-matrix-unit"), ("q5_k", 512, 8448, 16, "rows-on-matrix-unit"),
     ("q5_k", 520, 4608, 17, "tiled"), ("q5_k", 520, 4352, 32, "rows-on-matrix-unit"), ("q4_k", 700, 5120, 200, "rows-on-matrix-unit"),
     ("q4_k", 700, 5120, 33, "tiled"), ("q4_k", 600, 1024, 600, "rows-on-matrix-unit"), ("q5_k", 600, 2304, 600, "tiled"),
-    ("q6_k", 512, 4608, 9, "tiled"), ("q6_k", 512, 6144, 16, "rows-on-matrix-unit"), ("q6_k", 4100, 4096, 20, "rows-on-matrix-unit"),
-    ("q6_k", 520, 5120, 200, "rows-on-matrix-unit"), ("q6_k", 520, 5888, 65, "tiled"), ("q6_k", 2800, 3072, 33, "tiled"),
-    ("q6_k", 1023, 3072, 300, "rows-on-matrix-unit")])
-def test_both_sides_of_the_lines_between_rows_kernels_and_f16_tiles(name, n, k, rows, expect):
+    ("q6_k", 12289, 4864, 9, "tiled"), ("q6_k", 520, 4864, 9, "rows-on-matrix-unit"), ("q6_k", 4100, 4096, 20, "rows-on-matrix-unit"),
+    ("q6_k", 2049, 12544, 17, "tiled"), ("q6_k", 2048, 12544, 32, "rows-on-matrix-unit"), ("q6_k", 1025, 6400, 64, "tiled"),
+    ("q6_k", 520, 5120, 200, "rows-on-matrix-unit"), ("q6_k", 520, 5888, 65, "tiled"), ("q6_k", 2800, 3072, 33, "rows-on-matrix-unit"),
+    ("q6_k", 1023, 3072, 300, "rows-on-matrix-unit"), ("q6_k", 520, 768, 7, "rows-on-matrix-unit"), ("q4_k", 4096, 8192, 4, "matvec"),
+    ("q4_k", 4112, 8192, 4, "rows-on-matrix-unit")])
+def test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect):
     wtype = DT[name]
     w = synth.weight(wtype, n, k, seed=98, stream=1)
     x = synth.activation(rows, k, seed=98)
