@@ -14,8 +14,11 @@
 
 #include "lk_common.h"
 #include "rows16.h"
+#include "rows16_direct.h"
 
 namespace {
+
+using namespace rows16_direct;
 
 constexpr int TILE = 16, MAX_WAVES = 12;
 constexpr int BLOCK_PIECES = 14;              // 16-byte pieces that hold a super-block, at any even phase
@@ -28,7 +31,7 @@ typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
 
 struct Args {
     const uint8_t* w;     // 16-byte aligned
-    const uint8_t* y;     // Q8_1 rows
+    const uint8_t* y;     // Q8_1 rows (rows of values: SRC's elements, nb * 256 of them each)
     float* dst;
     int nb, n, m;         // super-blocks per weight row, weight rows, activation rows
     int stride_y;         // Q8_1 blocks between activation rows
@@ -37,11 +40,12 @@ struct Args {
 };
 
 // grid (row tiles, sets of TOKS activation rows), 64 * waves threads: wave w takes super-blocks w, w + waves, ...
-template <int TOKS, bool HALF>
+template <int TOKS, bool HALF, int SRC>
 __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Args p) {
     static_assert(TOKS == 8 || TOKS == 16, "sets of eight or sixteen activation rows");
     constexpr bool T16 = TOKS == 16;
     extern __shared__ __align__(16) uint8_t lds[];
+    static_assert(SRC == Q81 || TOKS == 8, "rows of values: eight at a time");
     const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
     const int tile = (int)blockIdx.x, m0 = (int)blockIdx.y * TOKS, m_rows = min(TOKS, p.m - m0);
@@ -81,16 +85,27 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
     const float* t_lane = T16 ? table + 4 * grp : table + 4 * (grp & 1);
     const int sh_sc = T16 ? 0 : 8 * (grp >> 1), sh_qh = 2 * (grp >> 1);
 
+    // rows of values: load u is (row lane / 8, sub-block u, values 4 (lane % 8) ..), the quantizer's own layout
+    typedef typename SrcOf<SRC>::T T;
+    typedef typename SrcOf<SRC>::Raw Raw;
+    const T* x_row = (const T*)p.y + (size_t)(m0 + min(lane >> 3, m_rows - 1)) * p.nb * 256 + 4 * (lane & 7);
+    uint32_t* codes_of_rows = (uint32_t*)(lds + waves * WAVE_BYTES + wave * CODE_BYTES);   // [sub-block][row][8]
     struct Block {
         u32x4 w[LOADS], y[Y_LOADS];
         uint32_t head[HEADS];
+        Raw v[SRC == Q81 ? 1 : 8];
     };
     auto load = [&](Block& b, int kb) {
         const uint32_t at = (uint32_t)(kb * Q6K_BYTES), ya = (uint32_t)(kb * 8 * Q81_BYTES);
+        if constexpr (SRC != Q81) {
 #pragma unroll
-        for (int j = 0; j < HEADS; ++j) b.head[j] = *(const uint32_t*)(y0 + (y_head[j] + ya));
+            for (int u = 0; u < 8; ++u) b.v[u] = *(const Raw*)(x_row + kb * 256 + 32 * u);
+        } else {
 #pragma unroll
-        for (int u = 0; u < Y_LOADS; ++u) b.y[u] = *(const u32x4_a4*)(y0 + (y_codes + ya) + u * (8 / Y_LOADS) * Q81_BYTES);
+            for (int j = 0; j < HEADS; ++j) b.head[j] = *(const uint32_t*)(y0 + (y_head[j] + ya));
+#pragma unroll
+            for (int u = 0; u < Y_LOADS; ++u) b.y[u] = *(const u32x4_a4*)(y0 + (y_codes + ya) + u * (8 / Y_LOADS) * Q81_BYTES);
+        }
 #pragma unroll
         for (int u = 0; u < LOADS; ++u) b.w[u] = *(const u32x4*)(w_tile + (((w_at[u] + at) & ~15u) + w_piece[u]));
     };
@@ -104,18 +119,26 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
         };
-#pragma unroll
-        for (int j = 0; j < HEADS; ++j) table[h_sub * TOKS + h_tok + 8 * j] = h_tok + 8 * j < m_rows ? f16_bits_to_f32(b.head[j] & 0xFFFFu) : 0.f;
         u32x4 act[4];   // the lane's sixteen codes of unit u: values 64 u + 16 grp ..
+        if constexpr (SRC != Q81) {
+            quantize<T>(b.v, lane, m_rows, table, codes_of_rows);
+        } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+            for (int j = 0; j < HEADS; ++j) table[h_sub * TOKS + h_tok + 8 * j] = h_tok + 8 * j < m_rows ? f16_bits_to_f32(b.head[j] & 0xFFFFu) : 0.f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                act[u][e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from + (T16 ? 0 : 16 * (u & 1)), (int)b.y[T16 ? u : u >> 1][e]);
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    act[u][e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from + (T16 ? 0 : 16 * (u & 1)), (int)b.y[T16 ? u : u >> 1][e]);
+        }
 #pragma unroll
         for (int u = 0; u < LOADS; ++u)
             if (64 * u + lane < TILE * BLOCK_PIECES) *(u32x4_a4*)(buf + (w_to[u] - (int)((w_at[u] + at) & 12u))) = b.w[u];
         settle();
+        if constexpr (SRC != Q81) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) act[u] = *(const u32x4*)(codes_of_rows + ((2 * u + (grp >> 1)) * 8 + tok) * 8 + 4 * (grp & 1));
+        }
         const uint8_t* mine = buf + l16 * PITCH + 16;
         const uint32_t sh = (my_at + at) & 2u;
         auto piece_at = [&](int c, uint32_t& past) {   // sixteen bytes at byte c of the super-block; the four after them, unshifted
@@ -181,6 +204,10 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         settle();
     };
 
+    if constexpr (SRC != Q81) {   // one in flight (registers)
+        Block b;
+        for (int kb = wave; kb < p.nb; kb += waves) load(b, kb), compute(b, kb);
+    } else {
     Block ring[2];
     load(ring[0], wave);
     if (wave + waves < p.nb) load(ring[1], wave + waves);
@@ -191,6 +218,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
             compute(ring[1], kb + waves);
             if (kb + 3 * waves < p.nb) load(ring[1], kb + 3 * waves);
         }
+    }
     }
 
     // the partial tiles, [4][64] floats at the start of each wave's buffer
@@ -212,21 +240,20 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
     }
 }
 
-template <int TOKS, bool HALF>
-int launch(const Args& a, int waves, hipStream_t stream) {
-    static const bool ok = hipFuncSetAttribute((const void*)q6k_rows16_short_kernel<TOKS, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               MAX_WAVES * WAVE_BYTES) == hipSuccess;
+template <int TOKS, bool HALF, int SRC = Q81>
+int launch(const Args& a, hipStream_t stream) {
+    constexpr int bytes = WAVE_BYTES + (SRC == Q81 ? 0 : CODE_BYTES);
+    static const bool ok = hipFuncSetAttribute((const void*)q6k_rows16_short_kernel<TOKS, HALF, SRC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               MAX_WAVES * bytes) == hipSuccess;
     if (!ok) return -1;
-    hipLaunchKernelGGL((q6k_rows16_short_kernel<TOKS, HALF>), dim3((a.n + TILE - 1) / TILE, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
-                       waves * WAVE_BYTES, stream, a);
+    const int steps = (a.nb + MAX_WAVES - 1) / MAX_WAVES, waves = (a.nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow
+    hipLaunchKernelGGL((q6k_rows16_short_kernel<TOKS, HALF, SRC>), dim3((a.n + TILE - 1) / TILE, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
+                       waves * bytes, stream, a);
     return lk_launch_status();
 }
 
-}  // namespace
-
-int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
-                        hipStream_t stream, int out_type) {
-    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || size_k > 32768 || (((uintptr_t)w) & 15) != 0) return -1;   // (longer rows: the others' to take or refuse)
+// Whether the short launch takes the call, and the rows of a set.
+int set_rows(int size_m, int size_n, int size_k) {
     // One workgroup fits a CU (registers), and a second round of them costs what the first did, so the line is the number of
     // workgroups. Eight rows to a set where that is one round, sixteen otherwise. Measured in a graph, us, the granules
     // of rows16_q6k.hip (rows of a multiple of 2048 values; more rows than it takes: the 32-row tiles) against this:
@@ -242,14 +269,32 @@ int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size
     // 10000 x 5120 at 8 / 16 / 32 25.3, 31.6, 36.7 / 19.9, 24.4, 41; 16384 x 3072 at 8 / 16 17.1, 20.2 / 17.9, 20.9; 3000 x 5120 at 32 / 48 20.0, 20.2 / 16.1, 24.1
     const int nb = size_k / 256, tiles = (size_n + TILE - 1) / TILE, cus = lk_device().cus;
     const bool granules = nb % 8 == 0, held = granules && tiles <= cus && (size_t)size_n * nb * Q6K_BYTES <= (64u << 20);
-    if (granules && size_m <= 8 && nb >= 32 && (2 * tiles <= cus || (size_m <= 4 && nb >= 48))) return -1;
-    if (granules && size_m <= 4 && nb > 8 && tiles > cus) return -1;   // (6144 x 6144 at 3 rows 12.6 / 15.0)
+    if (granules && size_m <= 8 && nb >= 32 && (2 * tiles <= cus || (size_m <= 4 && nb >= 48))) return 0;
+    if (granules && size_m <= 4 && nb > 8 && tiles > cus) return 0;   // (6144 x 6144 at 3 rows 12.6 / 15.0)
     const int eights = (size_m + 7) / 8, sixteens = (size_m + 15) / 16;
     const int64_t most = size_m <= 16 ? (granules ? 3 * cus / 2 : 3 * cus) : size_m > 32 ? 2 * cus : held && nb < 32 ? cus : granules ? 2 * cus : 3 * cus;
     const bool by_eight = size_m <= 8 || (int64_t)tiles * eights <= cus;
-    if ((int64_t)tiles * (by_eight ? eights : sixteens) > most) return -1;
-    const int steps = (nb + MAX_WAVES - 1) / MAX_WAVES, waves = (nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow
-    const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, nb, size_n, size_m, stride_y, ldd, out_type};
-    if (by_eight) return out_type == LK_TYPE_F32 ? launch<8, false>(a, waves, stream) : launch<8, true>(a, waves, stream);
-    return out_type == LK_TYPE_F32 ? launch<16, false>(a, waves, stream) : launch<16, true>(a, waves, stream);
+    if ((int64_t)tiles * (by_eight ? eights : sixteens) > most) return 0;
+    return by_eight ? 8 : 16;
+}
+
+}  // namespace
+
+int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
+                        hipStream_t stream, int out_type) {
+    // (rows of more than 32768 values: the others' to take or refuse)
+    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || size_k > 32768 || (((uintptr_t)w) & 15) != 0) return -1;
+    const int rows = set_rows(size_m, size_n, size_k);
+    if (rows == 0) return -1;
+    const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
+    if (rows == 8) return out_type == LK_TYPE_F32 ? launch<8, false>(a, stream) : launch<8, true>(a, stream);
+    return out_type == LK_TYPE_F32 ? launch<16, false>(a, stream) : launch<16, true>(a, stream);
+}
+
+// Up to eight rows of up to 4096 values straight from them, as lk_rows16_short_rows.
+int lk_rows16_q6k_short_rows(const void* w, const void* x, float* output, int size_m, int size_n, int size_k, int x_type, hipStream_t stream) {
+    if (size_m < 1 || size_m > 8 || size_n < 1 || size_k < 256 || size_k > 4096 || (((uintptr_t)w) & 15) != 0 || set_rows(size_m, size_n, size_k) != 8) return -1;
+    const Args a{(const uint8_t*)w, (const uint8_t*)x, output, size_k / 256, size_n, size_m, 0, size_n, x_type};
+    if (x_type == LK_TYPE_F32) return launch<8, false, ROWS_F32>(a, stream);
+    return x_type == LK_TYPE_F16 ? launch<8, true, ROWS_F16>(a, stream) : launch<8, true, ROWS_BF16>(a, stream);
 }

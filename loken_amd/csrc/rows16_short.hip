@@ -10,10 +10,12 @@
 #include "lk_common.h"
 #include "rows16.h"
 #include "rows16_core.h"
+#include "rows16_direct.h"
 
 namespace {
 
 using rows16::Blk;
+using namespace rows16_direct;
 using rows16::TILE;
 using rows16::WFrag;
 
@@ -44,14 +46,17 @@ static __device__ __forceinline__ TileRef tile_of(const LkRows16& p, int wg, int
     return {mat, tile};
 }
 
-static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q81) { return waves * nt * PART_BYTES + (q81 ? MAX_TOKS * nt / 4 * 32 * 4 : 0); }
+static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q81, bool rows = false) {
+    return waves * (nt * PART_BYTES + (rows ? CODE_BYTES : 0)) + (q81 ? MAX_TOKS * nt / 4 * 32 * 4 : 0);
+}
 
 // grid.x workgroups of NT row tiles each (one; two where one would be more workgroups than CUs, and for a gate and its up; four for
 // the 32 rows of a Q8_1 block), 64 * waves threads: wave w takes super-blocks w, w + waves, ... of every one of them, against one reading of the
 // activation.
-template <bool Q5, int TOKS, int OUT, int NT>
+template <bool Q5, int TOKS, int OUT, int NT, int SRC>
 __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows16 p, int n_tiles) {
     static_assert(TOKS == 8 || TOKS == 16, "eight or sixteen activation rows");
+    static_assert(SRC == Q81 || (TOKS == 8 && OUT <= ANY), "rows of values: eight at a time, dense");
     static_assert(NT == 1 || NT % 2 == 0, "tiles in turn through two sets of weight registers");
     constexpr bool T16 = TOKS == 16, DUAL = OUT >= DUAL_F32;
     extern __shared__ __align__(16) uint8_t lds[];
@@ -96,11 +101,21 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     const float* t_lane = T16 ? table + 4 * grp : table + 2 * par * TOKS + 4 * half;
     const int sh16 = T16 ? 0 : 16 * par, sh2 = 2 * par;
 
+    // Rows of values: load u is (row lane / 8, sub-block u, values 4 (lane % 8) ..), the quantizer's own layout.
+    typedef typename SrcOf<SRC>::T T;
+    const T* x_row = (const T*)p.x + (size_t)(m0 + min(lane >> 3, m_rows - 1)) * p.nb * 256 + 4 * (lane & 7);
+    uint32_t* codes = (uint32_t*)(lds + waves * NT * PART_BYTES + wave * CODE_BYTES);   // [sub-block][row][8]
     struct Act {
         u32x4 raw[LOADS];
         uint32_t head[HEADS];
+        typename SrcOf<SRC>::Raw v[SRC == Q81 ? 1 : 8];
     };
     auto load_act = [&](Act& b, int kb) {
+        if constexpr (SRC != Q81) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) b.v[u] = *(const typename SrcOf<SRC>::Raw*)(x_row + kb * 256 + 32 * u);
+            return;
+        }
         const uint32_t at = (uint32_t)(kb * 8 * Q81_BYTES);
 #pragma unroll
         for (int j = 0; j < HEADS; ++j) b.head[j] = *(const uint32_t*)(y_head[j] + at);
@@ -126,6 +141,12 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     u32x4 a[4];   // the lane's pieces: unit (c2, nib): row tok, sub-block 4 c2 + nib + 2 par, codes 16 half ..
     auto settle_act = [&](const Act& b) {
         settle();
+        if constexpr (SRC != Q81) {
+            quantize<T>(b.v, lane, m_rows, table, codes);
+            settle();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[u] = *(const u32x4*)(codes + ((4 * (u >> 1) + (u & 1) + 2 * par) * 8 + tok) * 8 + 4 * half);
+        } else {
 #pragma unroll
         for (int j = 0; j < HEADS; ++j) table[h_sub * TOKS + h_tok + 8 * j] = h_tok + 8 * j < m_rows ? f16_bits_to_f32(b.head[j] & 0xFFFFu) : 0.f;
 #pragma unroll
@@ -133,6 +154,7 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[u][e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from[T16 ? 0 : u & 1], (int)b.raw[T16 ? u : u >> 1][e]);
         settle();
+        }
         // the lane holds half the codes of sub-blocks 4 h + 2 par and + 1; its own is + half, the other half of whose codes is with the lane
         // sixteen on
         const uint4 ones = make_uint4(0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u);
@@ -213,7 +235,18 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     };
 
     WFrag w[2];   // NT 1: of two super-blocks; else of two tiles
-    if constexpr (NT == 1 && Q5 && T16) {   // (one activation set: registers. With two 4096 x 14336 takes 19.7 us against 17.5; the others lose 5 % with one)
+    if constexpr (SRC != Q81) {   // (a super-block to a wave)
+        Act act;
+        load_act(act, wave);
+        load_w(w[0], 0, wave);
+        if constexpr (NT > 1) load_w(w[1], 1, wave);
+        settle_act(act);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            compute(w[i & 1], acc[i]);
+            if (i + 2 < NT) load_w(w[i & 1], i + 2, wave);
+        }
+    } else if constexpr (NT == 1 && Q5 && T16) {   // (one activation set: registers. With two 4096 x 14336 takes 19.7 us against 17.5; the others lose 5 % with one)
         Act act;
         load_act(act, wave);
         load_w(w[0], 0, wave);
@@ -308,15 +341,15 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     }
 }
 
-template <bool Q5, int TOKS, int OUT, int NT>
+template <bool Q5, int TOKS, int OUT, int NT, int SRC = Q81>
 int launch(const LkRows16& a, int tiles, hipStream_t stream) {
-    static const bool ok = hipFuncSetAttribute((const void*)q4k_rows16_short_kernel<Q5, TOKS, OUT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               lds_bytes_for(GROUPS, NT, OUT == DUAL_Q81)) == hipSuccess;
+    static const bool ok = hipFuncSetAttribute((const void*)q4k_rows16_short_kernel<Q5, TOKS, OUT, NT, SRC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               lds_bytes_for(GROUPS, NT, OUT == DUAL_Q81, SRC != Q81)) == hipSuccess;
     if (!ok) return LK_ERR_ARG;
     const int steps = (a.nb + GROUPS - 1) / GROUPS, waves = (a.nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow
     const int per_wg = OUT >= DUAL_F32 ? NT / 2 : NT;
-    hipLaunchKernelGGL((q4k_rows16_short_kernel<Q5, TOKS, OUT, NT>), dim3((tiles + per_wg - 1) / per_wg, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
-                       lds_bytes_for(waves, NT, OUT == DUAL_Q81), stream, a, tiles);
+    hipLaunchKernelGGL((q4k_rows16_short_kernel<Q5, TOKS, OUT, NT, SRC>), dim3((tiles + per_wg - 1) / per_wg, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
+                       lds_bytes_for(waves, NT, OUT == DUAL_Q81, SRC != Q81), stream, a, tiles);
     return lk_launch_status();
 }
 
@@ -338,6 +371,12 @@ int launch_out(const LkRows16& a, bool dual, int tiles, hipStream_t stream) {
     }
     if (dual) return launch<Q5, TOKS, DUAL_F32, 2>(a, tiles, stream);
     return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 1>(a, tiles, stream) : launch<Q5, TOKS, ANY, 1>(a, tiles, stream);
+}
+
+template <bool Q5, int OUT, int SRC>
+int launch_rows(const LkRows16& a, int tiles, hipStream_t stream) {
+    const int cus = lk_device().cus;
+    return tiles > 2 * cus ? launch<Q5, 8, OUT, 4, SRC>(a, tiles, stream) : tiles > cus ? launch<Q5, 8, OUT, 2, SRC>(a, tiles, stream) : launch<Q5, 8, OUT, 1, SRC>(a, tiles, stream);
 }
 
 }  // namespace
@@ -367,4 +406,15 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
 bool lk_rows16_short_pays(int m, int n, int nb) {
     const int tiles = (n + TILE - 1) / TILE, cus = lk_device().cus;
     return m >= 1 && m <= MAX_TOKS && nb <= 128 && (tiles <= cus || (tiles <= (m <= 8 ? 4 : 2) * cus && nb >= 8));
+}
+
+// Up to eight rows of up to 4096 values, a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the
+// chip (2 us), and the host is through with one launch where it was with two: up to 8192 x 4096 9.4 us a call -> 6.8, 14336 x 4096 11.1 -> 9.4. Not above eight
+// rows, where a call that records a graph without scratch is refused.
+int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream) {
+    const int tiles = (a.n[0] + TILE - 1) / TILE;
+    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || a.m > 8 || !lk_rows16_short_pays(a.m, a.n[0], a.nb)) return -1;
+    if (a.x_type == LK_TYPE_F32) return q5 ? launch_rows<true, F32, ROWS_F32>(a, tiles, stream) : launch_rows<false, F32, ROWS_F32>(a, tiles, stream);
+    if (a.x_type == LK_TYPE_F16) return q5 ? launch_rows<true, ANY, ROWS_F16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_F16>(a, tiles, stream);
+    return q5 ? launch_rows<true, ANY, ROWS_BF16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_BF16>(a, tiles, stream);
 }

@@ -831,6 +831,22 @@ int lk_rows_linear(int wtype, const void* w, const void* q8_1, void* out, int ou
     return rows_plain(w, q8_1, (float*)out, rows, n, k, k / 32, n, wtype == LK_TYPE_Q5_K, stream, out_type);
 }
 
+int lk_rows_linear_direct(int wtype, const void* w, const void* x, void* out, int x_type, int rows, int n, int k, hipStream_t stream) {
+    const int elem = x_type == LK_TYPE_F32 ? 4 : 2;
+    if (k % 256 != 0 || (((uintptr_t)w) & 15) != 0 || ((uintptr_t)x % (4 * elem)) != 0) return -1;
+    if (wtype == LK_TYPE_Q6_K) return lk_rows16_q6k_short_rows(w, x, (float*)out, rows, n, k, x_type, stream);
+    if (wtype != LK_TYPE_Q4_K && wtype != LK_TYPE_Q5_K) return -1;
+    LkRows16 r{};
+    r.w[0] = (const uint8_t*)w;
+    r.dst[0] = (float*)out;
+    r.n[0] = r.ldd[0] = n;
+    r.count = 1;
+    r.nb = k / 256; r.m = rows;
+    r.x = x;
+    r.x_type = r.out_type = x_type;
+    return lk_rows16_short_rows(r, wtype == LK_TYPE_Q5_K, stream);
+}
+
 extern "C" int lk_dense_q4k_rows(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k,
                                  void* stream) {
     return rows_plain(w, q8_1, output, size_m, size_n, size_k, size_k / 32, size_n, false, (hipStream_t)stream);

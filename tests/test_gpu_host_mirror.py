@@ -327,6 +327,32 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
     assert close(got.cpu().numpy()[:, pick], oracle.ob_matmul(wtype, x, w[pick], len(pick)))
 
 
+@pytest.mark.parametrize("half", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name,n,k,rows", [
+    ("q4_k", 260, 1280, 3), ("q5_k", 256, 4096, 8), ("q4_k", 4100, 2048, 7), ("q5_k", 8200, 2304, 5), ("q4_k", 16384, 2048, 8), ("q6_k", 270, 1280, 4),
+    ("q6_k", 300, 4096, 8), ("q6_k", 2050, 3072, 3), ("q6_k", 6144, 2048, 6)])
+def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n, k, rows, half):
+    # the same products from Q8_1 rows of the stand-alone quantizer: bit for bit, with zeros, a row's largest code everywhere, halves between two codes,
+    # tiny values and infinities among the rows; rows that start off a 16-byte piece go by way of the quantizer
+    w = dev(synth.weight(DT[name], n, k, seed=86, stream=3))
+    x = dev(synth.activation(rows, k, seed=86))
+    x[0, :64] = 0
+    x[1] = torch.arange(k, device="cuda").remainder(255) - 127.0
+    x[1, ::3] *= 0.5
+    x[2] *= 1e-6
+    x = x.to(half)
+    lin = Linear(DT[name], w, n, k)
+    fn = ops.dense_q6k_rows if name == "q6_k" else (lambda *a: ops.dense_q4k_rows(*a, q5=name == "q5_k"))
+    got = lin(x)
+    assert lin.path == "rows-on-matrix-unit" and torch.equal(got, fn(w, x.float(), n).to(half))
+    flat = torch.zeros(rows * k + 1, device="cuda", dtype=half)
+    flat[1:] = x.reshape(-1)
+    assert torch.equal(lin(flat[1:].view(rows, k)), got)
+    x[0, 5], x[rows - 1, k - 1] = float("inf"), float("nan")
+    assert torch.equal(torch.nan_to_num(lin(x)), torch.nan_to_num(fn(w, x.float(), n).to(half)))
+    lin.close()
+
+
 @pytest.mark.parametrize("name,n,k,rows,expect", [
     ("q4_k", 8193, 7168, 9, "tiled"), ("q4_k", 8192, 7168, 9, "rows-on-matrix-unit"), ("q5_k", 512, 8448, 16, "rows-on-matrix-unit"),
     ("q5_k", 520, 4608, 17, "tiled"), ("q5_k", 520, 4352, 32, "rows-on-matrix-unit"), ("q4_k", 700, 5120, 200, "rows-on-matrix-unit"),
@@ -335,7 +361,7 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
     ("q6_k", 2049, 12544, 17, "tiled"), ("q6_k", 2048, 12544, 32, "rows-on-matrix-unit"), ("q6_k", 1025, 6400, 64, "tiled"),
     ("q6_k", 520, 5120, 200, "rows-on-matrix-unit"), ("q6_k", 520, 5888, 65, "tiled"), ("q6_k", 2800, 3072, 33, "rows-on-matrix-unit"),
     ("q6_k", 1023, 3072, 300, "rows-on-matrix-unit"), ("q6_k", 520, 768, 7, "rows-on-matrix-unit"), ("q4_k", 4096, 8192, 4, "matvec"),
-    ("q4_k", 4112, 8192, 4, "rows-on-matrix-unit")])
+    ("q4_k", 4112, 8192, 4, "rows-on-matrix-unit"), ("q4_k", 255, 2048, 3, "matvec"), ("q6_k", 256, 1280, 3, "rows-on-matrix-unit")])
 def test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect):
     wtype = DT[name]
     w = synth.weight(wtype, n, k, seed=98, stream=1)
@@ -344,7 +370,7 @@ def test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expec
     got = lin(dev(x))
     assert lin.path == expect
     lin.close()
-    pick, some = np.r_[:40, n - 40:n], np.r_[:4, rows - 4:rows]
+    pick, some = np.r_[:40, n - 40:n], np.unique(np.r_[:min(4, rows), max(0, rows - 4):rows])
     assert close(got.cpu().numpy()[some][:, pick], oracle.ob_matmul(wtype, x[some], w[pick], len(pick)))
 
 
