@@ -408,12 +408,11 @@ bool lk_rows16_short_pays(int m, int n, int nb) {
     return m >= 1 && m <= MAX_TOKS && nb <= 128 && (tiles <= cus || (tiles <= (m <= 8 ? 4 : 2) * cus && nb >= 8));
 }
 
-// Up to eight rows of up to 4096 values, a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the
-// chip (2 us), and the host is through with one launch where it was with two: up to 8192 x 4096 9.4 us a call -> 6.8, 14336 x 4096 11.1 -> 9.4. Not above eight
-// rows, where a call that records a graph without scratch is refused.
+// Up to eight rows of up to 4096 values (sixteen as two sets where both are resident at once), a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the
+// chip (2 us), and the host is through with one launch where it was with two: up to 8192 x 4096 9.4 us a call -> 6.8, 14336 x 4096 11.1 -> 9.4.
 int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream) {
     const int tiles = (a.n[0] + TILE - 1) / TILE;
-    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || a.m > 8 || !lk_rows16_short_pays(a.m, a.n[0], a.nb)) return -1;
+    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || !lk_rows16_short_pays(a.m, a.n[0], a.nb) || (a.m > 8 && 2 * tiles > lk_device().cus)) return -1;
     if (a.x_type == LK_TYPE_F32) return q5 ? launch_rows<true, F32, ROWS_F32>(a, tiles, stream) : launch_rows<false, F32, ROWS_F32>(a, tiles, stream);
     if (a.x_type == LK_TYPE_F16) return q5 ? launch_rows<true, ANY, ROWS_F16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_F16>(a, tiles, stream);
     return q5 ? launch_rows<true, ANY, ROWS_BF16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_BF16>(a, tiles, stream);

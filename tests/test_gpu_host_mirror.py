@@ -330,7 +330,8 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
 @pytest.mark.parametrize("half", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name,n,k,rows", [
     ("q4_k", 260, 1280, 3), ("q5_k", 256, 4096, 8), ("q4_k", 4100, 2048, 7), ("q5_k", 8200, 2304, 5), ("q4_k", 16384, 2048, 8), ("q6_k", 270, 1280, 4),
-    ("q6_k", 300, 4096, 8), ("q6_k", 2050, 3072, 3), ("q6_k", 6144, 2048, 6)])
+    ("q6_k", 300, 4096, 8), ("q6_k", 2050, 3072, 3), ("q6_k", 6144, 2048, 6), ("q4_k", 2048, 4096, 16), ("q5_k", 2050, 2048, 9),
+    ("q6_k", 2030, 2816, 15)])
 def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n, k, rows, half):
     # the same products from Q8_1 rows of the stand-alone quantizer: bit for bit, with zeros, a row's largest code everywhere, halves between two codes,
     # tiny values and infinities among the rows; rows that start off a 16-byte piece go by way of the quantizer
