@@ -16,6 +16,7 @@
 #define Q5K_BYTES 176
 #define Q6K_BYTES 210
 #define Q80_BYTES 34
+#define Q40_BYTES 18
 #define Q81_BYTES 36
 
 // 16-byte loads from blocks that are only 2-byte aligned (Q6_K 210 B, Q8_0 34 B): global memory

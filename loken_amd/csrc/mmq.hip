@@ -292,7 +292,7 @@ struct MmqQ80 {
     static constexpr int NS = 8;
     static constexpr bool HAS_MIN = false;
     static constexpr int MIN_RANK = 0;
-    static constexpr int F16_TYPE = -1;
+    static constexpr int F16_TYPE = LK_TYPE_Q8_0;
     static constexpr int WIDE_FROM = 96;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 8;
     static constexpr int QCH = TN * 16 / MMQ_WG, DCH = TN * 8 / MMQ_WG;
@@ -344,7 +344,7 @@ struct MmqLegacy {
     static constexpr int NS = 8;
     static constexpr bool HAS_MIN = L::M_AT >= 0;
     static constexpr int MIN_RANK = HAS_MIN ? 8 : 0;
-    static constexpr int F16_TYPE = -1;
+    static constexpr int F16_TYPE = ID == LK_TYPE_Q4_0 ? ID : -1;
     static constexpr int WIDE_FROM = 300;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 8;
     static constexpr int ALIGN = L::BYTES % 2 ? 1 : 2;
@@ -1009,8 +1009,9 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
     MmqProblem pb{(const uint8_t*)x, (const uint8_t*)y, (float*)dst, nullptr, ncols_x / 256, stride_row_x,
                   ncols_y, stride_col_dst, (int)nrows_x, 0, (int)ncols_y, out_type};
     hipStream_t s = (hipStream_t)stream;
-    // (Q4_K, Q5_K and Q6_K from 9 rows of a matrix of 512 rows or more: the f16 tiles; quantizer included, against the int8 tiles:
-    // Q4_K 4096 x 14336 at 9 / 32 rows 22 / 23 us against 27 / 29, 1024 x 14336 at 33 / 400 rows 21 / 44 against 27 / 55)
+    // (Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 from 9 rows of a matrix of 512 rows or more: the f16 tiles; quantizer included, against the int8 tiles:
+    // Q4_K 4096 x 14336 at 9 / 32 rows 22 / 23 us against 27 / 29, 1024 x 14336 at 33 / 400 rows 21 / 44 against 27 / 55, Q8_0 and Q4_0
+    // 1024 x 2048 at 17 rows 16.7 and 15.8 against 20.6 and 18.2)
     if constexpr (F::F16_TYPE >= 0)
         if (lk_mmq_tiles_take(F::F16_TYPE, nrows_x, ncols_y)) {
             const int tm = lk_mmq_tiles_dense(F::F16_TYPE, pb, s, fixup);
@@ -1076,7 +1077,8 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
     if (want <= 64 && !f16_short) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     // Runs of more than 32 rows: the f16 tiles for the formats that have them, over operands made from the records (a block in
     // one call makes them from the tokens and has its own, lower line: moe_forward.hip); under 33 rows the int8 tile of 32
-    // stays (128 experts of 2048 -> 768 -> 2048, Q6_K, average run 8 / 14: 198 / 208 us against 231 / 238).
+    // stays (128 experts of 2048 -> 768 -> 2048, Q6_K, average run 8 / 14: 198 / 208 us against 231 / 238); Q8_0 of the same sizes at runs of 64,
+    // launch by launch, 774 us against 490).
     if (f16) {
         const int tm = lk_mmq_tiles_moe_records(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
         if (tm >= 0) return tm;
@@ -1085,7 +1087,7 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
     // The 128-token int8 tile (the routing's bounds and destination map on top of the dense tile's registers) runs out
     // of registers for the formats with a minimum or two scales per sub-block and loses to the 64-token tile (2048
     // tokens, all three stacks: Q6_K 954 us against 1352, Q5_K 739 against 1231); Q8_0 and Q4_0 go either way by a
-    // tenth and keep the wide tile.
+    // tenth and keep the wide tile (where they cannot take the f16 tiles).
     if constexpr (F::F16_TYPE != LK_TYPE_Q4_K && (F::HAS_MIN || F::NS == 16))
         return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     else {

@@ -114,7 +114,7 @@ static inline MmqMoeGrid mmq_moe_grid(const MmqProblem& pb, int tn, int tm, int 
     return {dim3((unsigned)(n_tiles * group), (unsigned)(stacks * n_experts), (unsigned)((col_tiles + group - 1) / group)), (int)group};
 }
 
-// Q4_K, Q5_K and Q6_K on the f16 tiles of mmq_tile.h. tt: token tiles of 32 a wave takes; waves: 4 (two workgroups a CU) or
+// Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 on the f16 tiles of mmq_tile.h. tt: token tiles of 32 a wave takes; waves: 4 (two workgroups a CU) or
 // 8 (tt = 4, one); splits: ranges of K, partial products as above.
 struct MmqTilePlan {
     int tt, waves, splits;
@@ -123,6 +123,8 @@ struct LkTokenOperands;
 int lk_tile_dense_q4k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
 int lk_tile_dense_q5k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
 int lk_tile_dense_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
+int lk_tile_dense_q80(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
+int lk_tile_dense_q40(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s);
 // Expert-batched: expert e's slab, `stride` bytes after the one before, against the sorted rows [bounds[e], bounds[e + 1]).
 // With `to`: gate (the problem's weights) and up (w_second) products of operand rows gather[sorted row], and silu(gate) * up as
 // the operands `to` of the next product, a row per sorted row. Else the products to dst, w_second's dst_second floats further.
@@ -136,6 +138,8 @@ struct MmqTileExperts {
 int lk_tile_moe_q4k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
 int lk_tile_moe_q5k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
 int lk_tile_moe_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+int lk_tile_moe_q80(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+int lk_tile_moe_q40(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
 // Whether an expert-batched product can take them (alignment, sizes); `gated`: as lk_tile_moe_* with `to`.
 bool lk_mmq_tiles_moe_fit(int wtype, const void* w, const void* w_second, int64_t stride, int64_t n, int64_t k, int64_t rows, bool gated);
 int lk_mmq_tiles_moe(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);

@@ -1,4 +1,4 @@
-// Q4_K, Q5_K and Q6_K weight rows against 33 or more Q8_1 token rows: the sub-block dots on the f16 matrix unit.
+// Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 weight rows against Q8_1 token rows: the sub-block dots on the f16 matrix unit.
 //
 //   out[token, n] = sum over 256-value blocks of
 //        d[n] * sum_s d8_s[token] * D_s[n, token]  -  dmin[n] * sum_s m_s[n] * (d8_s * S_s)[token]
@@ -14,6 +14,7 @@
 // Q6_K's signed scales meet six-bit codes: |sc * q| <= 128 * 32 has one bit more than f16 holds. The operand is the
 // product rounded to f16 and a second one carries what the rounding took (-1, 0 or 1, exact); both terms add up in the
 // same accumulator, still exactly (128 * 32 * 127 * 32 < 2^24), four matrix instructions per sub-block instead of two.
+// Q8_0 and Q4_0 have no integer scale: their codes are the operand (128 * 127 * 32 < 2^24), see TileSub.
 //
 // Shape: a wave owns 32 weight rows x TT token tiles of 32 (registers <-> weight rows, lanes <-> tokens,
 // v_mfma_f32_32x32x16_f16 called as weights x tokens), so that the expansion of its rows is shared by TT items. Four waves
@@ -48,7 +49,8 @@ constexpr uint32_t H1024 = 0x64006400u;   // two f16 1024.0: OR-ing an 8-bit int
 // ------------------------------------------------------------------ weight formats
 // A block reaches LDS in 16-byte pieces, in two regions per row that are each read once and free after that: A (AP pieces:
 // header or scales and the first half of the codes) and B (BP pieces: the second half), so that one stage is enough and the
-// next block's pieces have most of a block's time to arrive. a_src / b_src: where piece p lies in the block. DMA: blocks are
+// next block's pieces have most of a block's time to arrive. a_src / b_src: where piece p lies in the block, place: its place in the
+// row's region (formats through registers). UNIT: what `row_blocks` counts, in bytes. DMA: blocks are
 // 16-byte aligned and go to LDS directly; else through registers. Row strides are an odd number of pieces, or the pieces of
 // a row are exchanged by its number (B of Q4_K / Q5_K), so that 32 rows spread over the banks (Q6_K's six: two rows a bank).
 // Codes: what a lane needs of half a block (four sub-blocks). operand(): the lane's eight values of matrix instruction hf
@@ -66,8 +68,9 @@ static __device__ __forceinline__ uint32_t odd_codes(uint32_t c, uint32_t h1024)
 
 template <bool Q5>
 struct TileQ45K {
-    static constexpr int BYTES = Q5 ? Q5K_BYTES : Q4K_BYTES, ALIGN = 16, TERMS = 1;
-    static constexpr bool HAS_MIN = true;
+    static constexpr int BYTES = Q5 ? Q5K_BYTES : Q4K_BYTES, UNIT = BYTES, ALIGN = 16, TERMS = 1;
+    static constexpr bool HAS_MIN = true, D_PER_SUB = false;
+    static constexpr int TT_MOST = 4;
     static constexpr int AP = Q5 ? 7 : 5, BP = 4;
     static constexpr bool DMA = true;
     static __host__ __device__ constexpr int a_src(int p) { return 16 * p; }
@@ -75,7 +78,8 @@ struct TileQ45K {
     struct Header { uint4 w; };
     struct Codes { uint4 q[2], qh; };
     static __device__ __forceinline__ Header header(const uint8_t* ra, int h) { (void)h; return {*(const uint4*)ra}; }
-    static __device__ __forceinline__ void codes0(Codes& c, const uint8_t* ra, int h) {
+    static __device__ __forceinline__ void codes0(Codes& c, const uint8_t* ra, int h, int row) {
+        (void)row;
 #pragma unroll
         for (int p = 0; p < 2; ++p) c.q[p] = *(const uint4*)(ra + (Q5 ? 48 : 16) + 32 * p + 16 * h);
         if (Q5) c.qh = *(const uint4*)(ra + 16 + 16 * h);
@@ -124,26 +128,28 @@ struct TileQ45K {
 };
 
 struct TileQ6K {
-    static constexpr int BYTES = Q6K_BYTES, ALIGN = 2, TERMS = 2;   // its d, two bytes past the 13 pieces, travels by itself
-    static constexpr bool HAS_MIN = false;
+    static constexpr int BYTES = Q6K_BYTES, UNIT = BYTES, ALIGN = 2, TERMS = 2;   // its d, two bytes past the 13 pieces, travels by itself
+    static constexpr bool HAS_MIN = false, D_PER_SUB = false;
+    static constexpr int TT_MOST = 4;
     static constexpr int AP = 7, BP = 6;
     static constexpr bool DMA = false;
     static __host__ __device__ constexpr int a_src(int p) { return p < 4 ? 16 * p : p < 6 ? 128 + 16 * (p - 4) : 192; }
     static __device__ __forceinline__ int b_src(int p, int row) { (void)row; return p < 4 ? 64 + 16 * p : 160 + 16 * (p - 4); }
+    static __device__ __forceinline__ int place(int p, int row) { (void)row; return p; }
     struct Header { uint32_t sc[4]; };   // byte 2 * (s % 2) of word s / 2: the scale of the lane's 16 values of sub-block s
     struct Codes { uint4 q[2], qh; };
     static __device__ __forceinline__ Header header(const uint8_t* ra, int h) {
         const uint4 w = *(const uint4*)(ra + 96);
         return {{w.x >> (8 * h), w.y >> (8 * h), w.z >> (8 * h), w.w >> (8 * h)}};
     }
-    static __device__ __forceinline__ void codes0(Codes& c, const uint8_t* ra, int h) {
+    static __device__ __forceinline__ void codes0(Codes& c, const uint8_t* ra, int h, int row) {
+        (void)row;
 #pragma unroll
         for (int p = 0; p < 2; ++p) c.q[p] = *(const uint4*)(ra + 32 * p + 16 * h);
         c.qh = *(const uint4*)(ra + 64 + 16 * h);
     }
     static __device__ __forceinline__ void codes1(Codes& c, const uint8_t* rb, int h, int row) {
-        (void)row;
-        codes0(c, rb, h);
+        codes0(c, rb, h, row);
     }
     static __device__ __forceinline__ Scale16 scale(const Header& hd, int s) {
         const _Float16 a = (_Float16)(float)(int8_t)((hd.sc[s >> 1] >> (16 * (s & 1))) & 0xFFu);
@@ -172,6 +178,55 @@ struct TileQ6K {
 };
 using TileQ4K = TileQ45K<false>;
 using TileQ5K = TileQ45K<true>;
+
+// Q8_0 and Q4_0: eight 32-value blocks make a block here, each with a d of its own that no integer scale takes into the matrix
+// unit: the codes are the operand, and a sub-block's dots meet d8 and its rows' d (D_PER_SUB) on their way into the sums, two
+// vector instructions an element, as f32. An item costs 32 of them and the two matrix instructions, and nothing folds at a block's end. Measured
+// (us, a linear of f32 rows, against the int8 tiles): Q8_0 14336 x 4096 at 17 / 96 / 512 / 2048 rows 47 / 83 / 158 / 695 -> 32 / 52 / 146 / 521,
+// 11003 x 4096 at 40 rows 97 -> 40, Q4_0 4096 x 14336 at 512 rows 184 -> 134, 2048 x 4096 at 17 rows 17.4 -> 16.1. Pieces are placed by the row's number (their rows in LDS are 128 and 64 bytes).
+template <bool Q4>
+struct TileSub {
+    static constexpr int UNIT = Q4 ? Q40_BYTES : Q80_BYTES, BYTES = 8 * UNIT, ALIGN = 2, TERMS = 1;
+    static constexpr bool HAS_MIN = false, D_PER_SUB = true;
+    static constexpr int TT_MOST = Q4 ? 4 : 3;   // what LDS has room for
+    static constexpr int AP = Q4 ? 4 : 8, BP = AP;
+    static constexpr bool DMA = false;
+    static __host__ __device__ constexpr int a_src(int p) { return Q4 ? UNIT * p + 2 : UNIT * (p >> 1) + 2 + 16 * (p & 1); }
+    static __device__ __forceinline__ int b_src(int p, int row) { (void)row; return 4 * UNIT + a_src(p); }
+    static __device__ __forceinline__ int place(int p, int row) { return Q4 ? p ^ ((row >> 1) & 3) : p ^ (row & 7); }
+    struct Header {};
+    struct Codes { uint4 q[4]; };
+    static __device__ __forceinline__ Header header(const uint8_t* ra, int h) { (void)ra; (void)h; return {}; }
+    static __device__ __forceinline__ void codes0(Codes& c, const uint8_t* ra, int h, int row) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            c.q[p] = *(const uint4*)(ra + 16 * place(Q4 ? p : 2 * p + h, row));
+            if (Q4) {   // values 0 .. 15 are the low nibbles, 16 .. 31 the high ones
+                c.q[p].x >>= 4 * h; c.q[p].y >>= 4 * h; c.q[p].z >>= 4 * h; c.q[p].w >>= 4 * h;
+            }
+        }
+    }
+    static __device__ __forceinline__ void codes1(Codes& c, const uint8_t* rb, int h, int row) { codes0(c, rb, h, row); }
+    static __device__ __forceinline__ Scale16 scale(const Header& hd, int s) {
+        (void)hd; (void)s;
+        const _Float16 b = (_Float16)(Q4 ? -1032.0f : -1152.0f);
+        return {{b, b}, {b, b}};
+    }
+    static __device__ __forceinline__ void operand(const Codes& cd, int s, int hf, const Scale16& sc, uint32_t h1024, v8h a[TERMS]) {
+        const uint4 q = cd.q[s & 3];
+        const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+        uint32_t ab[4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t c = Q4 ? u[2 * hf + e] & 0x0F0F0F0Fu : u[2 * hf + e] ^ 0x80808080u;
+            ab[2 * e] = h2_bits(as_h2(even_codes(c, h1024)) + sc.offset);
+            ab[2 * e + 1] = h2_bits(as_h2(odd_codes(c, h1024)) + sc.offset);
+        }
+        a[0] = __builtin_bit_cast(v8h, make_uint4(ab[0], ab[1], ab[2], ab[3]));
+    }
+};
+using TileQ80 = TileSub<false>;
+using TileQ40 = TileSub<true>;
 
 // ------------------------------------------------------------------ movement
 // 64 lanes x 16 bytes from global memory straight into LDS: uniform base + the lane's 32-bit offset on the global side;
@@ -214,8 +269,9 @@ struct TileShape {
     static constexpr int AC = F::DMA ? (32 * F::AP + 63) / 64 : 4, BC = F::DMA ? (32 * F::BP + 63) / 64 : 4, CH = AC + BC;
     static constexpr int A_ROW = 16 * F::AP, B_ROW = 16 * F::BP;
     static constexpr int A_BYTES = F::DMA ? AC * 1024 : 32 * A_ROW, W_BYTES = A_BYTES + 32 * B_ROW;
-    // LDS: ring of quarters, two blocks' tables, each wave's weights, each wave's d of its rows for two blocks
-    static constexpr int T_AT = 0, TAB_AT = NQ * QB, W_AT = TAB_AT + 2 * TABB, D_AT = W_AT + WAVES * W_BYTES, LDS = D_AT + WAVES * 256;
+    // LDS: ring of quarters, two blocks' tables, each wave's weights, each wave's d of its rows for two blocks (D_PER_SUB: of one)
+    static constexpr int D_ROW = 36, D_BYTES = F::D_PER_SUB ? 8 * D_ROW * 4 : 256;   // d of a sub-block: 32 floats and 16 bytes to spread the banks
+    static constexpr int T_AT = 0, TAB_AT = NQ * QB, W_AT = TAB_AT + 2 * TABB, D_AT = W_AT + WAVES * W_BYTES, LDS = D_AT + WAVES * D_BYTES;
     static_assert(LDS <= (WAVES == 4 ? 80 : 160) * 1024, "LDS of a workgroup");
     // Slots in which weights are loaded: directly, a region's next pieces right after the slot that has read it (A, read in slot
     // 7 TT - 1 for the next block: the block after that; B, in 3 TT - 1: the next block), so that they have almost a block's time.
@@ -273,11 +329,11 @@ struct TileWave {
     uint8_t* wstage;
     float* wd;
 
-    v16f acc[TT], part[TT], dot[2];
+    v16f acc[TT], part[F::D_PER_SUB ? 1 : TT], dot[2];
     v8h a[2][TERMS], b[2][2];
-    float d8v[4], dv[16];
+    float d8v[4], dv[F::D_PER_SUB ? 2 : 1][16];
     uint4 data[S::CH];
-    uint16_t d;
+    uint16_t d[F::D_PER_SUB ? 4 : 1];
     typename F::Header hd;
     typename F::Codes cd;
     uint32_t mh[4], mm[4];      // -dmin * min of the row's eight sub-blocks: two bf16 that add up to it exactly
@@ -302,11 +358,16 @@ struct TileWave {
             data[i] = *(const piece*)(block + (i & 3) * row_bytes8 + from[i / 4]);
     }
     __device__ __forceinline__ void fetch_d(int kb) {
-        if constexpr (!F::DMA) d = *(const uint16_t*)(w + (int64_t)kb * F::BYTES + d_from);
+        const uint8_t* block = w + (int64_t)kb * F::BYTES;
+        if constexpr (F::D_PER_SUB) {   // eight rows a load, eight sub-blocks each
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i] = *(const uint16_t*)(block + i * row_bytes8 + d_from);
+        } else if constexpr (!F::DMA) d[0] = *(const uint16_t*)(block + d_from);
     }
     __device__ __forceinline__ void commit(int i) const {
         const int lane = threadIdx.x & 63, row = 8 * (i & 3) + (lane >> 3);
-        const int at = i < S::AC ? row * S::A_ROW + 16 * min(lane & 7, F::AP - 1) : S::A_BYTES + row * S::B_ROW + 16 * min(lane & 7, F::BP - 1);
+        const int at = i < S::AC ? row * S::A_ROW + 16 * F::place(min(lane & 7, F::AP - 1), row)
+                                : S::A_BYTES + row * S::B_ROW + 16 * F::place(min(lane & 7, F::BP - 1), row);
         *(uint4*)(wstage + at) = data[i];
     }
     template <int I, int HF>
@@ -326,16 +387,21 @@ struct TileWave {
         for (int hf = 0; hf < 2; ++hf) F::operand(cd, s, hf, sc, h1024, a[hf]);
     }
     __device__ __forceinline__ void write_d(int parity) {
-        if (h == 0) {
+        if constexpr (F::D_PER_SUB) {
+            const int lane = threadIdx.x & 63;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wd[(lane & 7) * S::D_ROW + 8 * i + (lane >> 3)] = f16_bits_to_f32(d[i]);
+        } else if (h == 0) {
             if constexpr (F::HAS_MIN) wd[parity * 32 + j] = f16_bits_to_f32(hd.w.x & 0xFFFFu);
-            else wd[parity * 32 + j] = f16_bits_to_f32(d);
+            else wd[parity * 32 + j] = f16_bits_to_f32(d[0]);
         }
     }
-    __device__ __forceinline__ void read_dv(int parity) {
+    template <int TO = 0>
+    __device__ __forceinline__ void read_dv(int at) {   // `at`: in rows' d
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const float4 t = *(const float4*)(wd + parity * 32 + 8 * g + 4 * h);
-            dv[4 * g] = t.x; dv[4 * g + 1] = t.y; dv[4 * g + 2] = t.z; dv[4 * g + 3] = t.w;
+            const float4 t = *(const float4*)(wd + at + 8 * g + 4 * h);
+            dv[TO][4 * g] = t.x; dv[TO][4 * g + 1] = t.y; dv[TO][4 * g + 2] = t.z; dv[TO][4 * g + 3] = t.w;
         }
     }
     // (11 + 6 bits: rounded to bf16 and what the rounding took, eight bits each)
@@ -354,12 +420,15 @@ struct TileWave {
         constexpr int pt = P % TT, ps = P / TT;
         const float d8p = d8v[P & 3];
 #pragma unroll
-        for (int v = FROM; v < TO; ++v) part[pt][v] = ps == 0 ? dot[P & 1][v] * d8p : fmaf(dot[P & 1][v], d8p, part[pt][v]);
+        for (int v = FROM; v < TO; ++v) {
+            if constexpr (F::D_PER_SUB) acc[pt][v] = fmaf(dv[ps & 1][v], dot[P & 1][v] * d8p, acc[pt][v]);
+            else part[pt][v] = ps == 0 ? dot[P & 1][v] * d8p : fmaf(dot[P & 1][v], d8p, part[pt][v]);
+        }
     }
     template <int T>
     __device__ __forceinline__ void fold() {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[T][v] = fmaf(dv[v], part[T][v], acc[T][v]);
+        for (int v = 0; v < 16; ++v) acc[T][v] = fmaf(dv[0][v], part[T][v], acc[T][v]);
     }
 
     static __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
@@ -414,11 +483,11 @@ struct TileWave {
         if constexpr (I == 7 * TT - 1) {
             wave_order();
             hd = F::header(ra, h);
-            F::codes0(cd, ra, h);
+            F::codes0(cd, ra, h, j);
         }
         if constexpr (I == 7 * TT) { write_d(par ^ 1); fetch_d(next2); wave_order(); }
         // the block before: tile I is complete since slot I at the latest and starts again in slot I + 1
-        if constexpr (I < TT) fold<I>();
+        if constexpr (I < TT && !F::D_PER_SUB) fold<I>();
         if constexpr (F::HAS_MIN) {
             mins<I>(std::make_integer_sequence<int, 4>{});
             if constexpr (I == 2 * TT - 1) {
@@ -435,10 +504,13 @@ struct TileWave {
             if constexpr (J >= -1 && J < 3 * TT - 1 && (J + 1) % 3 == 0) pb0 = *(const uint4*)(mp + par * S::TABB + (J + 1) / 3 * (32 * LK_OPERAND_TAB));
             if constexpr (J >= 0 && J < 3 * TT && J % 3 == 1) pb1 = *(const uint4*)(rp + par * S::TABB + J / 3 * (32 * LK_OPERAND_TAB) + 64);
         }
-        if constexpr (I == NI - 1) read_dv(par);
+        if constexpr (F::D_PER_SUB) {   // the next sub-block's, over those that this slot's fmas were the last to read
+            if constexpr (tt == 0) read_dv<(s + 1) & 1>((s + 1) % 8 * S::D_ROW);
+        } else if constexpr (I == NI - 1) read_dv(par * 32);
         // pins the slot's end for the instruction selector, which orders only what has side effects
-        asm volatile("" : "+v"(part[P % TT]), "+v"(a[0][0]));
-        if constexpr (I < TT) asm volatile("" : "+v"(acc[I % TT]));
+        if constexpr (F::D_PER_SUB) asm volatile("" : "+v"(acc[P % TT]), "+v"(a[0][0]));
+        else asm volatile("" : "+v"(part[P % TT]), "+v"(a[0][0]));
+        if constexpr (I < TT && !F::D_PER_SUB) asm volatile("" : "+v"(acc[I % TT]));
         fence();
     }
     template <int I, int... C>
@@ -471,7 +543,7 @@ static __device__ __forceinline__ void multiply(TileWave<F, TT, WAVES, GATHER>& 
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int last = (int)pb.nb - 1;
-    const int64_t row_bytes = pb.row_blocks * F::BYTES;
+    const int64_t row_bytes = pb.row_blocks * F::UNIT;
     t.wave = wave;
     t.j = lane & 31;
     t.h = lane >> 5;
@@ -514,8 +586,10 @@ static __device__ __forceinline__ void multiply(TileWave<F, TT, WAVES, GATHER>& 
         t.from[1] = row + F::b_src(min(lane & 7, F::BP - 1), 0);
         t.row_bytes8 = 8 * row_bytes;
     }
-    t.d_from = (uint32_t)min(row0 + t.j, live - 1) * (uint32_t)row_bytes + F::BYTES - 2;
-    t.d = 0;
+    t.d_from = F::D_PER_SUB ? (uint32_t)(row0 + (lane >> 3)) * (uint32_t)row_bytes + F::UNIT * (lane & 7)
+                            : (uint32_t)min(row0 + t.j, live - 1) * (uint32_t)row_bytes + F::BYTES - 2;
+#pragma unroll
+    for (int i = 0; i < (F::D_PER_SUB ? 4 : 1); ++i) t.d[i] = 0;
 #pragma unroll
     for (int x = 0; x < 4; ++x) t.tb[x] = lds + S::T_AT + t.j * 128 + 16 * ((2 * x + t.h) ^ (t.j & 7));
     t.rp = lds + S::TAB_AT + t.j * LK_OPERAND_TAB;
@@ -523,15 +597,15 @@ static __device__ __forceinline__ void multiply(TileWave<F, TT, WAVES, GATHER>& 
     t.wstage = lds + S::W_AT + wave * S::W_BYTES;
     t.ra = t.wstage + t.j * S::A_ROW;
     t.rb = t.wstage + S::A_BYTES + t.j * S::B_ROW;
-    t.wd = (float*)(lds + S::D_AT) + wave * 64;
+    t.wd = (float*)(lds + S::D_AT) + wave * (S::D_BYTES / 4);
     t.h1024 = H1024;   // in a vector register: (x & mask) | h1024 is then one v_and_or_b32 with the mask as its literal
     asm volatile("" : "+v"(t.h1024));
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) { t.acc[tt][v] = 0.f; t.part[tt][v] = 0.f; }
+        for (int v = 0; v < 16; ++v) { t.acc[tt][v] = 0.f; t.part[F::D_PER_SUB ? 0 : tt][v] = 0.f; }
 #pragma unroll
-    for (int v = 0; v < 16; ++v) { t.dot[(S::NI - 1) & 1][v] = 0.f; t.dv[v] = 0.f; }
+    for (int v = 0; v < 16; ++v) { t.dot[(S::NI - 1) & 1][v] = 0.f; t.dv[F::D_PER_SUB][v] = 0.f; }
     t.d8v[(S::NI - 1) & 3] = 0.f;   // "the item before the first": zeros times zero
 
 #pragma unroll
@@ -548,9 +622,10 @@ static __device__ __forceinline__ void multiply(TileWave<F, TT, WAVES, GATHER>& 
         for (int i = 0; i < S::CH; ++i) t.commit(i);
     meet<0>();
     t.hd = F::header(t.ra, t.h);
-    F::codes0(t.cd, t.ra, t.h);
+    F::codes0(t.cd, t.ra, t.h, t.j);
     t.write_d(0);
     wave_order();
+    if constexpr (F::D_PER_SUB) t.template read_dv<0>(0);
     t.fetch_d(min(1, last));
     if constexpr (F::DMA) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if constexpr (F::DMA || S::LONG)
@@ -563,10 +638,11 @@ static __device__ __forceinline__ void multiply(TileWave<F, TT, WAVES, GATHER>& 
     for (int kb = 0; kb <= last; ++kb) t.block(kb, last, std::make_integer_sequence<int, S::NI>{});
 
     t.template fix_up<0, 16, S::NI - 1>();
+    if constexpr (!F::D_PER_SUB)
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) t.acc[tt][v] = fmaf(t.dv[v], t.part[tt][v], t.acc[tt][v]);
+            for (int v = 0; v < 16; ++v) t.acc[tt][v] = fmaf(t.dv[0][v], t.part[tt][v], t.acc[tt][v]);
 }
 
 // A wave's results to dst[token][row], or dst[ids_dst[token]][row]; `first` its first weight row.
@@ -659,7 +735,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void tile_dense_ker
     if (!F::DMA) n0 = min(n0, pb.n - ROWS);   // (the last tile slides back over the one before: same rows, same results)
     const int row0 = 32 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     TileWave<F, TT, WAVES, false> t;
-    multiply(t, pb, ops, nullptr, pb.w + n0 * (pb.row_blocks * F::BYTES), row0, pb.n - n0, m_tile * 32 * TT, lds);
+    multiply(t, pb, ops, nullptr, pb.w + n0 * (pb.row_blocks * F::UNIT), row0, pb.n - n0, m_tile * 32 * TT, lds);
     store_rows(t, pb, n0 + row0, m_tile * 32 * TT);
 }
 
@@ -670,7 +746,7 @@ template <class F, int TT, bool GATED>
 static __device__ __forceinline__ void expert_tile(const MmqProblem& pb, const LkTokenOperands& ops, const int32_t* gather, const uint8_t* w_second,
                                                    const LkTokenOperands& to, int n_tile, int m0, uint8_t* lds) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t row_bytes = pb.row_blocks * F::BYTES;
+    const int64_t row_bytes = pb.row_blocks * F::UNIT;
     TileWave<F, TT, 4, GATED> t;
     if constexpr (!GATED) {
         int n0 = n_tile * 128;
@@ -738,9 +814,8 @@ __global__ __launch_bounds__(256, MAX == 1 && F::DMA ? 3 : 2) void tile_moe_kern
 
 template <class F, int MAX>
 static constexpr int moe_lds() {
-    constexpr int a = TileShape<F, 1, 4>::LDS, b = MAX >= 2 ? TileShape<F, 2, 4>::LDS : 0, c = MAX >= 3 ? TileShape<F, 3, 4>::LDS : 0, d = MAX >= 4 ? TileShape<F, 4, 4>::LDS : 0;
-    constexpr int ab = a > b ? a : b, cd = c > d ? c : d;
-    return ab > cd ? ab : cd;
+    if constexpr (MAX == 1) return TileShape<F, 1, 4>::LDS;
+    else return TileShape<F, MAX, 4>::LDS > moe_lds<F, MAX - 1>() ? TileShape<F, MAX, 4>::LDS : moe_lds<F, MAX - 1>();
 }
 template <class F, bool GATED, int MAX>
 static int launch_moe(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {
@@ -782,7 +857,9 @@ static int launch_dense_plan(const MmqProblem& pb, const LkTokenOperands& ops, c
         case 1: return launch_dense<F, 1, 4>(pb, ops, plan.splits, part, s);
         case 2: return launch_dense<F, 2, 4>(pb, ops, plan.splits, part, s);
         case 3: return launch_dense<F, 3, 4>(pb, ops, plan.splits, part, s);
-        default: return launch_dense<F, 4, 4>(pb, ops, plan.splits, part, s);
+        default:
+            if constexpr (F::TT_MOST == 4) return launch_dense<F, 4, 4>(pb, ops, plan.splits, part, s);
+            return LK_ERR_ARG;
     }
 }
 

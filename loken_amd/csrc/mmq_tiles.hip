@@ -1,4 +1,4 @@
-// Dense products of Q4_K, Q5_K and Q6_K weights on the f16 tiles (mmq_tile.h): which tile a call takes, and the token operands.
+// Products of Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 weights on the f16 tiles (mmq_tile.h): which tile a call takes, and the token operands.
 
 #include "mmq_operands.h"
 #include "mmq_problem.h"
@@ -45,26 +45,45 @@ __global__ __launch_bounds__(256) void operands_quantize_kernel(const T* __restr
     operand_quad(v, ops.codes + at * LK_OPERAND_CODES, ops.tabs + at * LK_OPERAND_TAB, (i0 / 32) & 7, (i0 / 4) & 7);
 }
 
+// The formats' kernels; unit: bytes that `row_blocks` counts, of `values` values; align: of the weights.
+struct Tiles {
+    int type, unit, values, align, tt_most;
+    int (*dense)(const MmqProblem&, const LkTokenOperands&, const MmqTilePlan&, float*, hipStream_t);
+    int (*moe)(const MmqProblem&, const LkTokenOperands&, const MmqTileExperts&, hipStream_t);
+};
+constexpr Tiles TILES[] = {{LK_TYPE_Q4_K, Q4K_BYTES, 256, 16, 4, lk_tile_dense_q4k, lk_tile_moe_q4k},
+                           {LK_TYPE_Q5_K, Q5K_BYTES, 256, 16, 4, lk_tile_dense_q5k, lk_tile_moe_q5k},
+                           {LK_TYPE_Q6_K, Q6K_BYTES, 256, 2, 4, lk_tile_dense_q6k, lk_tile_moe_q6k},
+                           {LK_TYPE_Q8_0, Q80_BYTES, 32, 2, 3, lk_tile_dense_q80, lk_tile_moe_q80},
+                           {LK_TYPE_Q4_0, Q40_BYTES, 32, 2, 4, lk_tile_dense_q40, lk_tile_moe_q40}};
+const Tiles* tiles_of(int wtype) {
+    for (const Tiles& t : TILES)
+        if (t.type == wtype) return &t;
+    return nullptr;
+}
+
 // What a launch takes, fitted to 3000 calls on MI355X (7 shapes of 2048 x 2048 to 14336 x 4096 and 4096 x 14336, 33 to 2048 rows,
 // every tile width with K whole and cut into 2 to 12 ranges; the fit is off by 3 to 4 %, the plan it picks takes 1 to 2 % longer than
 // the best one of the sweep). alone / full: nanoseconds an item (32 x 32 x 32 product) takes a SIMD with one workgroup on its CU or two, by token
-// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items.
+// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items. (Q8_ITEM, Q4_ITEM: Q8_0 and Q4_0, from
+// 14336 x 4096 at 33, 128 and 512 rows at every width.)
 struct ItemTimes {
     double alone[4], full[4], wide, start;
 };
-constexpr ItemTimes ONE_TERM = {{164, 105, 104, 89}, {129, 98, 87.5, 82.7}, 80, 0.6}, TWO_TERMS = {{263, 144, 159, 143}, {194, 134, 122.5, 118}, 0, 3.1};
+constexpr ItemTimes ONE_TERM = {{164, 105, 104, 89}, {129, 98, 87.5, 82.7}, 80, 0.6}, TWO_TERMS = {{263, 144, 159, 143}, {194, 134, 122.5, 118}, 0, 3.1},
+                    Q8_ITEM = {{340, 180, 178, 0}, {220, 148, 135, 0}, 0, 1.0}, Q4_ITEM = {{315, 170, 172, 142}, {190, 138, 121, 107}, 0, 1.0};
 
 // The tile and the cut of K with the shortest estimated launch. Up to 2 * cus workgroups run at once, and a CU that holds two takes
 // nearly the time of a full chip; past that the rounds blur (0.6 of whole rounds, 0.4 of their share). A cut costs a launch and
 // its partial products, written, read and added.
-MmqTilePlan plan_dense(int wtype, const MmqProblem& pb, const void* fixup) {
-    const ItemTimes& t = wtype == LK_TYPE_Q6_K ? TWO_TERMS : ONE_TERM;
+MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup) {
+    const ItemTimes& t = f.type == LK_TYPE_Q6_K ? TWO_TERMS : f.type == LK_TYPE_Q8_0 ? Q8_ITEM : f.type == LK_TYPE_Q4_0 ? Q4_ITEM : ONE_TERM;
     const int cus = lk_device().cus;
     const int forced_tt = lk_tune_env("LK_TUNE_MMQ_TT"), forced_splits = lk_tune_env("LK_TUNE_MMQ_SPLITS");   // measurement runs
     const int most = forced_splits < 0 ? 1 : std::min(mmq_splits_most(pb, fixup, true), 12);
-    MmqTilePlan best{4, 4, 1};
+    MmqTilePlan best{f.tt_most, 4, 1};
     double least = 1e30;
-    for (int tt = 1; tt <= 4; ++tt) {
+    for (int tt = 1; tt <= f.tt_most; ++tt) {
         if (forced_tt > 0 && tt != forced_tt) continue;
         const int64_t tiles = ((pb.n + 127ll) / 128) * ((pb.m_end + 32ll * tt - 1) / (32 * tt));
         for (int splits = forced_splits > 0 ? std::min(forced_splits, most) : 1; splits <= most; ++splits) {
@@ -87,24 +106,16 @@ MmqTilePlan plan_dense(int wtype, const MmqProblem& pb, const void* fixup) {
     return best;
 }
 
-int launch(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s) {
-    return wtype == LK_TYPE_Q4_K   ? lk_tile_dense_q4k(pb, ops, plan, part, s)
-           : wtype == LK_TYPE_Q5_K ? lk_tile_dense_q5k(pb, ops, plan, part, s)
-                                   : lk_tile_dense_q6k(pb, ops, plan, part, s);
-}
-
 // What the operands of one pass may take; a call with more goes in passes of token rows over the same buffer (stream order
 // keeps them apart).
 constexpr int64_t OPERANDS_CAP = 256ll << 20;
 
 // The product in passes; fill(operands, first row, rows) launches what writes a pass's operands. Returns as lk_mmq_tiles_dense.
 template <class Fill>
-int run_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup, Fill fill) {
-    const int bytes = wtype == LK_TYPE_Q4_K ? Q4K_BYTES : wtype == LK_TYPE_Q5_K ? Q5K_BYTES : Q6K_BYTES;
-    const bool q6 = wtype == LK_TYPE_Q6_K;
-    if ((uintptr_t)pb.w % (q6 ? 2 : 16) != 0 || (q6 && pb.n < 128)) return -1;
+int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, Fill fill) {
+    if ((uintptr_t)pb.w % f.align != 0 || (f.align != 16 && pb.n < 128)) return -1;
     // lane offsets inside a tile are 32-bit
-    if (pb.row_blocks * bytes * 256 > (int64_t)INT32_MAX || pb.m_begin != 0) return -1;
+    if (pb.row_blocks * f.unit * 256 > (int64_t)INT32_MAX || pb.m_begin != 0) return -1;
     const int64_t row_bytes = pb.nb * (LK_OPERAND_CODES + LK_OPERAND_TAB);
     const int64_t fit = OPERANDS_CAP / row_bytes / 128 * 128 - LK_OPERAND_PAD;
     if (fit < 128 || pb.nb > INT32_MAX / 2) return -1;
@@ -118,9 +129,9 @@ int run_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup, Fill 
         pass.m_end = std::min(per_pass, pb.m_end - m0);
         pass.dst = (float*)((uint8_t*)pb.dst + (int64_t)m0 * pb.ldd * (pb.out_type == LK_TYPE_F32 ? 4 : 2));
         const LkTokenOperands ops = lk_operands_at(buffer, pass.m_end, pb.nb);
-        const MmqTilePlan plan = plan_dense(wtype, pass, fixup);
+        const MmqTilePlan plan = plan_dense(f, pass, fixup);
         fill(ops, m0, pass.m_end);
-        if (launch(wtype, pass, ops, plan, (float*)fixup, s) != LK_OK) return 0;
+        if (f.dense(pass, ops, plan, (float*)fixup, s) != LK_OK) return 0;
         if (plan.splits > 1 && lk_mmq_split_sum((const float*)fixup, plan.splits, pass, s) != LK_OK) return 0;
         width = std::max(width, 32 * plan.tt);
     }
@@ -130,21 +141,22 @@ int run_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup, Fill 
 }  // namespace
 
 int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
-    if ((uintptr_t)pb.y % 16 != 0) return -1;
-    return run_dense(wtype, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int rows) {
+    const Tiles* f = tiles_of(wtype);
+    if (!f || (uintptr_t)pb.y % 16 != 0) return -1;
+    return run_dense(*f, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int rows) {
         hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((rows + 31) / 32)), dim3(256), 0, s, pb.y, ops,
                            pb.rows_total, m0, rows);
     });
 }
 
 bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows) {
-    return (wtype == LK_TYPE_Q4_K || wtype == LK_TYPE_Q5_K || wtype == LK_TYPE_Q6_K) && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
+    return tiles_of(wtype) && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
 }
 
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {
     if (!lk_mmq_tiles_take(wtype, n, rows) || k % 256 != 0) return -1;
-    const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / 256, rows, n, n, 0, rows, type};
-    return run_dense(wtype, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
+    const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
+    return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
         (void)lk_operands_quantize((const uint8_t*)x + (int64_t)m0 * k * (type == LK_TYPE_F32 ? 4 : 2), type, ops, k, count, s);
     });
 }
@@ -158,23 +170,20 @@ int lk_operands_quantize(const void* x, int type, const LkTokenOperands& ops, in
 }
 
 bool lk_mmq_tiles_moe_fit(int wtype, const void* w, const void* w_second, int64_t stride, int64_t n, int64_t k, int64_t rows, bool gated) {
-    if (wtype != LK_TYPE_Q4_K && wtype != LK_TYPE_Q5_K && wtype != LK_TYPE_Q6_K) return false;
-    const int bytes = wtype == LK_TYPE_Q4_K ? Q4K_BYTES : wtype == LK_TYPE_Q5_K ? Q5K_BYTES : Q6K_BYTES, align = wtype == LK_TYPE_Q6_K ? 2 : 16;
-    if (k % 256 != 0 || n > INT32_MAX || n < 128 || (gated && n % 64 != 0)) return false;
+    const Tiles* f = tiles_of(wtype);
+    if (!f || k % 256 != 0 || n > INT32_MAX || n < 128 || (gated && n % 64 != 0)) return false;
     // operand row offsets inside a block, and row offsets inside a tile, are 32-bit
-    return ((uintptr_t)w | (uintptr_t)w_second | (uintptr_t)stride) % align == 0 && rows < (1 << 23) && k / 256 * bytes * 128 <= (int64_t)INT32_MAX;
+    return ((uintptr_t)w | (uintptr_t)w_second | (uintptr_t)stride) % f->align == 0 && rows < (1 << 23) && k / f->values * f->unit * 128 <= (int64_t)INT32_MAX;
 }
 
 int lk_mmq_tiles_moe(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {
-    return wtype == LK_TYPE_Q4_K   ? lk_tile_moe_q4k(pb, ops, ex, s)
-           : wtype == LK_TYPE_Q5_K ? lk_tile_moe_q5k(pb, ops, ex, s)
-                                   : lk_tile_moe_q6k(pb, ops, ex, s);
+    return tiles_of(wtype)->moe(pb, ops, ex, s);
 }
 
 int lk_mmq_tiles_moe_records(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
                              int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s) {
     if ((uintptr_t)pb.y % 16 != 0 || pb.row_blocks > INT32_MAX / 256 || pb.nb > INT32_MAX / 256 ||
-        !lk_mmq_tiles_moe_fit(wtype, pb.w, w_second, stride_expert, pb.n, 256 * pb.row_blocks, pb.rows_total, false))
+        !lk_mmq_tiles_moe_fit(wtype, pb.w, w_second, stride_expert, pb.n, tiles_of(wtype)->values * pb.row_blocks, pb.rows_total, false))
         return -1;
     LkScratch scratch(s);
     void* buffer = scratch.get(LK_SCRATCH_TOKENS, lk_operand_bytes(pb.rows_total, pb.nb));

@@ -39,6 +39,7 @@ const Format* format_of(int type) {
     return nullptr;
 }
 
+int64_t stack_bytes(const Format& f, int n, int k) { return (int64_t)n * (k / f.block_len) * f.block_bytes; }   // of one expert
 bool grouped_serves(const Format& f, int k) { return f.grouped && k % 256 == 0; }
 
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -63,11 +64,11 @@ int block_on_tiles(const Format& fg, const Format& fd, const float* x, const voi
 
     if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, s)) return rc;
     if (int rc = lk_operands_quantize(x, LK_TYPE_F32, tokens_in, hidden, tokens, s)) return rc;
-    MmqProblem gu{(const uint8_t*)gate, nullptr, nullptr, nullptr, nb, nb, rows, 0, ffn, 0, 0};
-    const MmqTileExperts first{bounds, src, (const uint8_t*)up, 0, (int64_t)ffn * nb * fg.block_bytes, longest, n_experts, &h};
+    MmqProblem gu{(const uint8_t*)gate, nullptr, nullptr, nullptr, nb, hidden / fg.block_len, rows, 0, ffn, 0, 0};
+    const MmqTileExperts first{bounds, src, (const uint8_t*)up, 0, stack_bytes(fg, ffn, hidden), longest, n_experts, &h};
     if (int rc = lk_mmq_tiles_moe(fg.type, gu, tokens_in, first, s)) return rc;
-    MmqProblem dn{(const uint8_t*)down, nullptr, pairs, slots, nb2, nb2, rows, hidden, hidden, 0, 0};
-    const MmqTileExperts second{bounds, nullptr, nullptr, 0, (int64_t)hidden * nb2 * fd.block_bytes, longest, n_experts, nullptr};
+    MmqProblem dn{(const uint8_t*)down, nullptr, pairs, slots, nb2, ffn / fd.block_len, rows, hidden, hidden, 0, 0};
+    const MmqTileExperts second{bounds, nullptr, nullptr, 0, stack_bytes(fd, hidden, ffn), longest, n_experts, nullptr};
     if (int rc = lk_mmq_tiles_moe(fd.type, dn, h, second, s)) return rc;
     return lk_moe_fold(pairs, topk_weights, choices, n_experts, out, tokens, topk, hidden, 0, s);
 }
@@ -79,7 +80,7 @@ int block_on_tiles(const Format& fg, const Format& fd, const float* x, const voi
 // mat-vec per routed pair stays ahead of the int8 tiles up to three rows per expert, of the matrix-unit rows launch that
 // Q4_K stacks take at short runs up to 1.625 (16 tokens: 51 us against 74; 24: 81 against 83; 32: 92 against 88; 48: 139 against
 // 106), and of the f16 tiles up to two (Q5_K, 1.8 / 2.1 rows: 138 / 174 against 125 / 134) or two and a half (Q6_K, 2.4 / 2.9
-// rows: 55 / 227 against 60 / 199). `wtype`: the stacks' type where both have the same, else -1.
+// rows: 55 / 227 against 60 / 199), three of Q8_0 (2 / 4 rows: 226 / 399 against 257 / 266). `wtype`: the stacks' type where both have the same, else -1.
 extern "C" int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype) {
     const int64_t experts = n_experts > 1 ? n_experts : 1;
     return wtype == LK_TYPE_Q4_K   ? 8 * rows >= 13 * experts
@@ -110,8 +111,10 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
 }
 
 // Whether the block goes on the f16 tiles with nothing but operands between its launches (block_on_tiles), for two stacks of
-// Q4_K, Q5_K or Q6_K. Measured on MI355X, whole block, by the longest expected run, against the launches it replaces:
+// Q4_K, Q5_K, Q6_K, Q8_0 or Q4_0. Measured on MI355X, whole block, by the longest expected run, against the launches it replaces:
 //   Q5_K always (128 experts of 2048 -> 768 at 11 / 31 / 50 rows 137 / 147 / 182 us against 167 / 186 / 216)
+//   Q8_0 and Q4_0 likewise (Q8_0, 128 of 2048 -> 768, average run 4 / 16 / 64 rows: 266 / 274 / 365 us against 447 / 468 / 702, 8 of
+//     2560 -> 1536 at 8 / 32 / 256 rows 75 / 77 / 204 against 104 / 126 / 356)
 //   Q6_K likewise (64 of 1536 -> 1024 at 9 / 26 / 50 rows 99 / 105 / 125 against 104 / 112 / 150), but for short runs over 60 experts and
 //     more, whose int8 tiles of 32 tokens run two more workgroups a CU (128 of 2048 -> 768 at 11 / 22 rows 202 / 208 against 193 / 205)
 //   Q4_K, whose short runs have the rows launch, from 20 rows (128 of 2048 -> 768 at 19 / 26 / 42 rows 123 / 128 / 152 against 117 / 145 / 202,
@@ -119,9 +122,10 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
 //     eight super-blocks and the tiles fill the chip (60 of 2560 -> 1280 at 7 / 9 / 17 / 26 rows 116 / 120 / 117 / 123 against 114 / 141 / 195 / 182)
 // and with workgroups of 64 gate and up rows for a quarter of the CUs at least.
 static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int hidden, int ffn) {
-    auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K; };
+    auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K || type == LK_TYPE_Q8_0 || type == LK_TYPE_Q4_0; };
     if (!has_tiles(gu) || !has_tiles(down) || lk_env_flag("LK_MMQ_I8") || (int64_t)n_experts * (ffn / 64) < lk_device().cus / 4) return false;
-    if (gu == LK_TYPE_Q5_K || down == LK_TYPE_Q5_K) return true;
+    auto always = [](int type) { return type == LK_TYPE_Q5_K || type == LK_TYPE_Q8_0 || type == LK_TYPE_Q4_0; };
+    if (always(gu) || always(down)) return true;
     if (gu == LK_TYPE_Q6_K && down == LK_TYPE_Q6_K) return longest > 22 || n_experts < 60;
     return longest >= 20 || (longest >= 9 && hidden > 2048 && 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus);
 }
@@ -174,8 +178,8 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
     const bool rows_gu = path & LK_MOE_ROWS_GATE_UP, rows_down = path & LK_MOE_ROWS_DOWN;
     if ((path & LK_MOE_TILES) &&
-        lk_mmq_tiles_moe_fit(wtype_gu, gate, up, (int64_t)ffn * (hidden / 256) * fg->block_bytes, ffn, hidden, tokens, true) &&
-        lk_mmq_tiles_moe_fit(wtype_down, down, nullptr, (int64_t)hidden * (ffn / 256) * fd->block_bytes, hidden, ffn, rows, false))
+        lk_mmq_tiles_moe_fit(wtype_gu, gate, up, stack_bytes(*fg, ffn, hidden), ffn, hidden, tokens, true) &&
+        lk_mmq_tiles_moe_fit(wtype_down, down, nullptr, stack_bytes(*fd, hidden, ffn), hidden, ffn, rows, false))
         return block_on_tiles(*fg, *fd, x, gate, up, down, choices, topk_weights, out, tokens, topk, n_experts, hidden, ffn, longest, scratch, s);
     const bool gated_later = !rows_gu && !rows_down && ffn % 32 == 0;   // the activation rides the second product's quantizer
     // the buffer's pieces

@@ -304,3 +304,19 @@ def test_f16_tiles_at_every_width_and_edge(name, m, k, n, fixup, knobs):
     scale = rows.abs().max().item()
     assert (got - int8).abs().max().item() <= 2e-5 * scale
     assert (got - rows).abs().max().item() <= 2e-5 * scale
+
+
+@pytest.mark.parametrize("name", ["q8_0", "q4_0"])
+@pytest.mark.parametrize("m,k,n", [(9, 256, 512), (32, 512, 513), (33, 256, 639), (65, 768, 641), (96, 2048, 2176), (97, 512, 2303),
+                                   (129, 256, 4097), (384, 512, 16390)])
+@pytest.mark.parametrize("fixup", [True, False])
+def test_f16_tiles_of_blocks_with_a_scale_a_sub_block(name, m, k, n, fixup, knobs):
+    # As above for the formats whose 32-value blocks carry their own d (through registers, a last tile that slides back)
+    test_f16_tiles_at_every_width_and_edge(name, m, k, n, fixup, knobs)
+
+
+@pytest.mark.parametrize("name", ["q8_0", "q4_0"])
+@pytest.mark.parametrize("tt", [1, 2, 3, 4])
+def test_every_tile_width_of_blocks_with_a_scale_a_sub_block(name, tt, knobs):
+    knobs.set("LK_TUNE_MMQ_TT", str(tt))   # (a width a format has no room for takes its widest)
+    test_f16_tiles_at_every_width_and_edge(name, 131, 1280, 645, True, knobs)

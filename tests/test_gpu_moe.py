@@ -663,6 +663,12 @@ def test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn):
     assert (np.abs(got.cpu().numpy()[sample] - fed) <= bound).all()
 
 
+@pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q8_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_K, lib.TYPE_Q4_0)])
+@pytest.mark.parametrize("runs,hidden,ffn", [(RUNS, 256, 256), (RUNS, 768, 512)])
+def test_block_of_plain_blocks_on_the_f16_tiles(runs, hidden, ffn, gu, dn):
+    test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn)
+
+
 @pytest.mark.parametrize("n,n_experts,topk", [(1, 3, 1), (63, 5, 3), (64, 1, 1), (1025, 130, 5), (4097, 512, 1), (8888, 128, 8)])
 def test_routing_is_a_stable_grouping(n, n_experts, topk):
     choices = synth.rand_ints(23, n, n, n_experts).astype(np.int32).reshape(-1, topk)

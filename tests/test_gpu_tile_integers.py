@@ -152,6 +152,12 @@ def test_f16_tiles_emit_the_exact_subblock_integers(wtype, m, k):
     check(lambda w, x: ops.mmq_forward(wtype, w, x, n), wtype, n, k, m, seed=140 + m, subs=[0, 7] if wtype != Q6K else [0, 6, 15])
 
 
+@pytest.mark.parametrize("wtype", [Q80, lib.TYPE_Q4_0])
+@pytest.mark.parametrize("m,k", [(9, 256), (65, 768), (97, 512)])
+def test_f16_tiles_emit_the_exact_integers_of_plain_blocks(wtype, m, k):
+    test_f16_tiles_emit_the_exact_subblock_integers(wtype, m, k)
+
+
 @pytest.mark.parametrize("sub", [0, 3, 6])
 def test_f16_tiles_carry_every_q6k_scale_exactly(sub):
     # sc * (code - 32) reaches 128 * 32, one bit more than an f16 holds: both 16-value scales of one 32-value
