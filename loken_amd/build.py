@@ -24,7 +24,7 @@ FLAGS = [
 # MFMA results are consumed by VALU fix-ups right away: keep them in VGPRs instead of the
 # accumulator file, which would cost one v_accvgpr_read per value.
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-PER_FILE_FLAGS = {name: _VGPR_FORM for name in ("mmq.hip", *(f"mmq_tile_{w}.hip" for w in ("q4k", "q5k", "q6k", "q80", "q40")))}
+PER_FILE_FLAGS = {name: _VGPR_FORM for name in ("mmq.hip", *(f"mmq_tile_{w}.hip" for w in ("q4k", "q5k", "q6k", "q80", "q40", "iq4nl", "mxfp4")))}
 
 
 def sources() -> list[Path]:

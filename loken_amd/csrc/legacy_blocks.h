@@ -32,13 +32,12 @@ static __device__ __forceinline__ uint32_t levels_of(uint32_t codes) {
     return (high & top) | (low & ~top);
 }
 
-// The block's scale: an f16, or MXFP4's E8M0 byte as 0.5 * 2^(e - 127) (denormal patterns below 2).
+// MXFP4's E8M0 byte as 0.5 * 2^(e - 127) (denormal patterns below 2).
+static __device__ __forceinline__ float e8m0_half(uint32_t e) { return __uint_as_float(e < 2 ? (0x00200000u << e) : ((e - 1) << 23)); }
+// The block's scale: an f16, or MXFP4's.
 template <class F>
 static __device__ __forceinline__ float block_scale(const uint8_t* __restrict__ bp) {
-    if (F::TABLE == 2) {
-        const uint32_t e = bp[0];
-        return __uint_as_float(e < 2 ? (0x00200000u << e) : ((e - 1) << 23));
-    }
+    if (F::TABLE == 2) return e8m0_half(bp[0]);
     return f16_bits_to_f32(*(const uint16_t*)bp);
 }
 

@@ -344,7 +344,7 @@ struct MmqLegacy {
     static constexpr int NS = 8;
     static constexpr bool HAS_MIN = L::M_AT >= 0;
     static constexpr int MIN_RANK = HAS_MIN ? 8 : 0;
-    static constexpr int F16_TYPE = ID == LK_TYPE_Q4_0 ? ID : -1;
+    static constexpr int F16_TYPE = ID == LK_TYPE_Q4_0 || L::TABLE ? ID : -1;
     static constexpr int WIDE_FROM = 300;   // 128-token tiles from this many of them (launch_dense)
     static constexpr int BLOCKS_PER_STEP = 8;
     static constexpr int ALIGN = L::BYTES % 2 ? 1 : 2;
@@ -1077,7 +1077,7 @@ static int launch_moe(const void* x, const void* x_second, int64_t dst_second, c
     if (want <= 64 && !f16_short) return launch_moe_tm<F, 64, 2>(pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);
     // Runs of more than 32 rows: the f16 tiles for the formats that have them, over operands made from the records (a block in
     // one call makes them from the tokens and has its own, lower line: moe_forward.hip); under 33 rows the int8 tile of 32
-    // stays (128 experts of 2048 -> 768 -> 2048, Q6_K, average run 8 / 14: 198 / 208 us against 231 / 238); Q8_0 of the same sizes at runs of 64,
+    // stays (128 experts of 2048 -> 768 -> 2048, Q6_K, average run 8 / 14: 198 / 208 us against 231 / 238; Q8_0 of the same sizes at runs of 64,
     // launch by launch, 774 us against 490).
     if (f16) {
         const int tm = lk_mmq_tiles_moe_records(F::F16_TYPE, pb, w2, dst_second, expert_bounds, stride_expert_x, n_experts, ncols_max, s);

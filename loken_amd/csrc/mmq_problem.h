@@ -140,6 +140,8 @@ int lk_tile_moe_q5k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqT
 int lk_tile_moe_q6k(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
 int lk_tile_moe_q80(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
 int lk_tile_moe_q40(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+int lk_tile_moe_iq4nl(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
+int lk_tile_moe_mxfp4(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);
 // Whether an expert-batched product can take them (alignment, sizes); `gated`: as lk_tile_moe_* with `to`.
 bool lk_mmq_tiles_moe_fit(int wtype, const void* w, const void* w_second, int64_t stride, int64_t n, int64_t k, int64_t rows, bool gated);
 int lk_mmq_tiles_moe(int wtype, const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s);

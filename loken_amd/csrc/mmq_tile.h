@@ -14,7 +14,7 @@
 // Q6_K's signed scales meet six-bit codes: |sc * q| <= 128 * 32 has one bit more than f16 holds. The operand is the
 // product rounded to f16 and a second one carries what the rounding took (-1, 0 or 1, exact); both terms add up in the
 // same accumulator, still exactly (128 * 32 * 127 * 32 < 2^24), four matrix instructions per sub-block instead of two.
-// Q8_0 and Q4_0 have no integer scale: their codes are the operand (128 * 127 * 32 < 2^24), see TileSub.
+// Q8_0, Q4_0, IQ4_NL and MXFP4 have no integer scale: their codes or levels are the operand (128 * 127 * 32 < 2^24), see TileSub.
 //
 // Shape: a wave owns 32 weight rows x TT token tiles of 32 (registers <-> weight rows, lanes <-> tokens,
 // v_mfma_f32_32x32x16_f16 called as weights x tokens), so that the expansion of its rows is shared by TT items. Four waves
@@ -33,6 +33,7 @@
 // tokens use the same order, which is all a dot product asks. (A lane half holds one of Q6_K's 16-value groups.)
 #pragma once
 
+#include "legacy_blocks.h"
 #include "mmq_operands.h"
 #include "mmq_problem.h"
 
@@ -179,20 +180,25 @@ struct TileQ6K {
 using TileQ4K = TileQ45K<false>;
 using TileQ5K = TileQ45K<true>;
 
-// Q8_0 and Q4_0: eight 32-value blocks make a block here, each with a d of its own that no integer scale takes into the matrix
+// Q8_0, Q4_0, IQ4_NL and MXFP4: eight 32-value blocks make a block here, each with a d of its own that no integer scale takes into the matrix
 // unit: the codes are the operand, and a sub-block's dots meet d8 and its rows' d (D_PER_SUB) on their way into the sums, two
 // vector instructions an element, as f32. An item costs 32 of them and the two matrix instructions, and nothing folds at a block's end. Measured
 // (us, a linear of f32 rows, against the int8 tiles): Q8_0 14336 x 4096 at 17 / 96 / 512 / 2048 rows 47 / 83 / 158 / 695 -> 32 / 52 / 146 / 521,
 // 11003 x 4096 at 40 rows 97 -> 40, Q4_0 4096 x 14336 at 512 rows 184 -> 134, 2048 x 4096 at 17 rows 17.4 -> 16.1. Pieces are placed by the row's number (their rows in LDS are 128 and 64 bytes).
-template <bool Q4>
+template <int ID>
 struct TileSub {
-    static constexpr int UNIT = Q4 ? Q40_BYTES : Q80_BYTES, BYTES = 8 * UNIT, ALIGN = 2, TERMS = 1;
+    static constexpr bool Q4 = ID != LK_TYPE_Q8_0;   // 16 bytes of nibbles a sub-block
+    using L = Legacy<Q4 ? ID : LK_TYPE_Q4_0>;
+    static constexpr int UNIT = Q4 ? L::BYTES : Q80_BYTES, BYTES = 8 * UNIT, ALIGN = UNIT % 2 ? 1 : 2, TERMS = 1;
     static constexpr bool HAS_MIN = false, D_PER_SUB = true;
     static constexpr int TT_MOST = Q4 ? 4 : 3;   // what LDS has room for
     static constexpr int AP = Q4 ? 4 : 8, BP = AP;
     static constexpr bool DMA = false;
-    static __host__ __device__ constexpr int a_src(int p) { return Q4 ? UNIT * p + 2 : UNIT * (p >> 1) + 2 + 16 * (p & 1); }
+    static __host__ __device__ constexpr int a_src(int p) { return Q4 ? UNIT * p + L::QS_AT : UNIT * (p >> 1) + 2 + 16 * (p & 1); }
     static __device__ __forceinline__ int b_src(int p, int row) { (void)row; return 4 * UNIT + a_src(p); }
+    // d as it lies (one byte of MXFP4's E8M0, else f16), and its value
+    static __device__ __forceinline__ uint16_t scale_bits(const uint8_t* p) { return UNIT % 2 ? *p : *(const uint16_t*)p; }
+    static __device__ __forceinline__ float scale_value(uint16_t bits) { return L::TABLE == 2 ? e8m0_half(bits) : f16_bits_to_f32(bits); }
     static __device__ __forceinline__ int place(int p, int row) { return Q4 ? p ^ ((row >> 1) & 3) : p ^ (row & 7); }
     struct Header {};
     struct Codes { uint4 q[4]; };
@@ -209,7 +215,7 @@ struct TileSub {
     static __device__ __forceinline__ void codes1(Codes& c, const uint8_t* rb, int h, int row) { codes0(c, rb, h, row); }
     static __device__ __forceinline__ Scale16 scale(const Header& hd, int s) {
         (void)hd; (void)s;
-        const _Float16 b = (_Float16)(Q4 ? -1032.0f : -1152.0f);
+        const _Float16 b = (_Float16)(Q4 && !L::TABLE ? -1032.0f : -1152.0f);   // levels and Q8_0's codes are int8
         return {{b, b}, {b, b}};
     }
     static __device__ __forceinline__ void operand(const Codes& cd, int s, int hf, const Scale16& sc, uint32_t h1024, v8h a[TERMS]) {
@@ -218,15 +224,20 @@ struct TileSub {
         uint32_t ab[4];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const uint32_t c = Q4 ? u[2 * hf + e] & 0x0F0F0F0Fu : u[2 * hf + e] ^ 0x80808080u;
+            uint32_t c = u[2 * hf + e];
+            if (Q4) c &= 0x0F0F0F0Fu;
+            if (Q4 && L::TABLE) c = levels_of<L::TABLE>(c);
+            if (!Q4 || L::TABLE) c ^= 0x80808080u;
             ab[2 * e] = h2_bits(as_h2(even_codes(c, h1024)) + sc.offset);
             ab[2 * e + 1] = h2_bits(as_h2(odd_codes(c, h1024)) + sc.offset);
         }
         a[0] = __builtin_bit_cast(v8h, make_uint4(ab[0], ab[1], ab[2], ab[3]));
     }
 };
-using TileQ80 = TileSub<false>;
-using TileQ40 = TileSub<true>;
+using TileQ80 = TileSub<LK_TYPE_Q8_0>;
+using TileQ40 = TileSub<LK_TYPE_Q4_0>;
+using TileIq4Nl = TileSub<LK_TYPE_IQ4_NL>;
+using TileMxfp4 = TileSub<LK_TYPE_MXFP4>;
 
 // ------------------------------------------------------------------ movement
 // 64 lanes x 16 bytes from global memory straight into LDS: uniform base + the lane's 32-bit offset on the global side;
@@ -315,7 +326,7 @@ template <class F, int TT, int WAVES, bool GATHER>
 struct TileWave {
     using S = TileShape<F, TT, WAVES>;
     static constexpr int NI = S::NI, QI = S::QI, TERMS = F::TERMS;
-    using piece = typename std::conditional<F::ALIGN == 16, uint4, uint4_a2>::type;
+    using piece = typename std::conditional<F::ALIGN == 16, uint4, typename std::conditional<F::ALIGN == 1, uint4_a1, uint4_a2>::type>::type;
     // global side: uniform bases, lane offsets
     const uint8_t *codes, *tabs, *w;
     int64_t code_slab, tab_slab, row_bytes8;   // bytes of a block's codes, of its tables, of eight weight rows
@@ -361,7 +372,7 @@ struct TileWave {
         const uint8_t* block = w + (int64_t)kb * F::BYTES;
         if constexpr (F::D_PER_SUB) {   // eight rows a load, eight sub-blocks each
 #pragma unroll
-            for (int i = 0; i < 4; ++i) d[i] = *(const uint16_t*)(block + i * row_bytes8 + d_from);
+            for (int i = 0; i < 4; ++i) d[i] = F::scale_bits(block + i * row_bytes8 + d_from);
         } else if constexpr (!F::DMA) d[0] = *(const uint16_t*)(block + d_from);
     }
     __device__ __forceinline__ void commit(int i) const {
@@ -390,7 +401,7 @@ struct TileWave {
         if constexpr (F::D_PER_SUB) {
             const int lane = threadIdx.x & 63;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) wd[(lane & 7) * S::D_ROW + 8 * i + (lane >> 3)] = f16_bits_to_f32(d[i]);
+            for (int i = 0; i < 4; ++i) wd[(lane & 7) * S::D_ROW + 8 * i + (lane >> 3)] = F::scale_value(d[i]);
         } else if (h == 0) {
             if constexpr (F::HAS_MIN) wd[parity * 32 + j] = f16_bits_to_f32(hd.w.x & 0xFFFFu);
             else wd[parity * 32 + j] = f16_bits_to_f32(d[0]);
@@ -865,10 +876,12 @@ static int launch_dense_plan(const MmqProblem& pb, const LkTokenOperands& ops, c
 
 }  // namespace mmq_tile
 
-#define LK_DEFINE_TILES(NAME, FORMAT)                                                                                             \
-    int lk_tile_dense_##NAME(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s) { \
-        return mmq_tile::launch_dense_plan<FORMAT>(pb, ops, plan, part, s);                                                       \
-    }                                                                                                                             \
+#define LK_DEFINE_EXPERT_TILES(NAME, FORMAT)                                                                                      \
     int lk_tile_moe_##NAME(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTileExperts& ex, hipStream_t s) {           \
         return ex.to ? mmq_tile::launch_moe<FORMAT, true>(pb, ops, ex, s) : mmq_tile::launch_moe<FORMAT, false>(pb, ops, ex, s);  \
+    }
+#define LK_DEFINE_TILES(NAME, FORMAT)                                                                                             \
+    LK_DEFINE_EXPERT_TILES(NAME, FORMAT)                                                                                          \
+    int lk_tile_dense_##NAME(const MmqProblem& pb, const LkTokenOperands& ops, const MmqTilePlan& plan, float* part, hipStream_t s) { \
+        return mmq_tile::launch_dense_plan<FORMAT>(pb, ops, plan, part, s);                                                       \
     }

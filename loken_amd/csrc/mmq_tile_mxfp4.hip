@@ -1,0 +1,4 @@
+// The f16 tiles of one weight format, experts only (see mmq_tile.h).
+#include "mmq_tile.h"
+
+LK_DEFINE_EXPERT_TILES(mxfp4, mmq_tile::TileMxfp4)

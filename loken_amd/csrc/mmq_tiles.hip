@@ -55,7 +55,9 @@ constexpr Tiles TILES[] = {{LK_TYPE_Q4_K, Q4K_BYTES, 256, 16, 4, lk_tile_dense_q
                            {LK_TYPE_Q5_K, Q5K_BYTES, 256, 16, 4, lk_tile_dense_q5k, lk_tile_moe_q5k},
                            {LK_TYPE_Q6_K, Q6K_BYTES, 256, 2, 4, lk_tile_dense_q6k, lk_tile_moe_q6k},
                            {LK_TYPE_Q8_0, Q80_BYTES, 32, 2, 3, lk_tile_dense_q80, lk_tile_moe_q80},
-                           {LK_TYPE_Q4_0, Q40_BYTES, 32, 2, 4, lk_tile_dense_q40, lk_tile_moe_q40}};
+                           {LK_TYPE_Q4_0, Q40_BYTES, 32, 2, 4, lk_tile_dense_q40, lk_tile_moe_q40},
+                           {LK_TYPE_IQ4_NL, 18, 32, 2, 4, nullptr, lk_tile_moe_iq4nl},   // experts only
+                           {LK_TYPE_MXFP4, 17, 32, 1, 4, nullptr, lk_tile_moe_mxfp4}};
 const Tiles* tiles_of(int wtype) {
     for (const Tiles& t : TILES)
         if (t.type == wtype) return &t;
@@ -142,7 +144,7 @@ int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, 
 
 int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
     const Tiles* f = tiles_of(wtype);
-    if (!f || (uintptr_t)pb.y % 16 != 0) return -1;
+    if (!f || !f->dense || (uintptr_t)pb.y % 16 != 0) return -1;
     return run_dense(*f, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int rows) {
         hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((rows + 31) / 32)), dim3(256), 0, s, pb.y, ops,
                            pb.rows_total, m0, rows);
@@ -150,7 +152,8 @@ int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fix
 }
 
 bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows) {
-    return tiles_of(wtype) && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
+    const Tiles* f = tiles_of(wtype);
+    return f && f->dense && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
 }
 
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {

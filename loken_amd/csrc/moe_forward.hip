@@ -80,12 +80,13 @@ int block_on_tiles(const Format& fg, const Format& fd, const float* x, const voi
 // mat-vec per routed pair stays ahead of the int8 tiles up to three rows per expert, of the matrix-unit rows launch that
 // Q4_K stacks take at short runs up to 1.625 (16 tokens: 51 us against 74; 24: 81 against 83; 32: 92 against 88; 48: 139 against
 // 106), and of the f16 tiles up to two (Q5_K, 1.8 / 2.1 rows: 138 / 174 against 125 / 134) or two and a half (Q6_K, 2.4 / 2.9
-// rows: 55 / 227 against 60 / 199), three of Q8_0 (2 / 4 rows: 226 / 399 against 257 / 266). `wtype`: the stacks' type where both have the same, else -1.
+// rows: 55 / 227 against 60 / 199), three of Q8_0 (2 / 4 rows: 226 / 399 against 257 / 266). MXFP4's mat-vec is slower (2.5 rows: 270
+// against 191, 64 experts 142 against 121, 32 of 3072 -> 512 98 against 84); 8 experts, whose launches do not fill the chip, stay (54 against 70). `wtype`: the stacks' type where both have the same, else -1.
 extern "C" int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype) {
     const int64_t experts = n_experts > 1 ? n_experts : 1;
     return wtype == LK_TYPE_Q4_K   ? 8 * rows >= 13 * experts
            : wtype == LK_TYPE_Q5_K ? rows >= 2 * experts
-           : wtype == LK_TYPE_Q6_K ? 2 * rows >= 5 * experts
+           : wtype == LK_TYPE_Q6_K || (wtype == LK_TYPE_MXFP4 && experts >= 32) ? 2 * rows >= 5 * experts
                                    : rows >= 3 * experts;
 }
 
@@ -111,10 +112,12 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
 }
 
 // Whether the block goes on the f16 tiles with nothing but operands between its launches (block_on_tiles), for two stacks of
-// Q4_K, Q5_K, Q6_K, Q8_0 or Q4_0. Measured on MI355X, whole block, by the longest expected run, against the launches it replaces:
+// Q4_K, Q5_K, Q6_K, Q8_0, Q4_0, IQ4_NL or MXFP4. Measured on MI355X, whole block, by the longest expected run, against the launches it replaces:
 //   Q5_K always (128 experts of 2048 -> 768 at 11 / 31 / 50 rows 137 / 147 / 182 us against 167 / 186 / 216)
 //   Q8_0 and Q4_0 likewise (Q8_0, 128 of 2048 -> 768, average run 4 / 16 / 64 rows: 266 / 274 / 365 us against 447 / 468 / 702, 8 of
 //     2560 -> 1536 at 8 / 32 / 256 rows 75 / 77 / 204 against 104 / 126 / 356)
+//   IQ4_NL and MXFP4 from 33 rows, or over fewer than 60 experts (MXFP4, 128 of 2048 -> 768, average run 16 / 32 / 64 rows: 221 / 245 / 327 us against 206 /
+//     307 / 482, 64 of 1536 -> 1024 at 16 / 32 125 / 138 against 122 / 174, 8 of 2560 -> 1536 at 3 / 32 70 / 85 against 81 / 109; IQ4_NL alike)
 //   Q6_K likewise (64 of 1536 -> 1024 at 9 / 26 / 50 rows 99 / 105 / 125 against 104 / 112 / 150), but for short runs over 60 experts and
 //     more, whose int8 tiles of 32 tokens run two more workgroups a CU (128 of 2048 -> 768 at 11 / 22 rows 202 / 208 against 193 / 205)
 //   Q4_K, whose short runs have the rows launch, from 20 rows (128 of 2048 -> 768 at 19 / 26 / 42 rows 123 / 128 / 152 against 117 / 145 / 202,
@@ -122,10 +125,12 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
 //     eight super-blocks and the tiles fill the chip (60 of 2560 -> 1280 at 7 / 9 / 17 / 26 rows 116 / 120 / 117 / 123 against 114 / 141 / 195 / 182)
 // and with workgroups of 64 gate and up rows for a quarter of the CUs at least.
 static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int hidden, int ffn) {
-    auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K || type == LK_TYPE_Q8_0 || type == LK_TYPE_Q4_0; };
-    if (!has_tiles(gu) || !has_tiles(down) || lk_env_flag("LK_MMQ_I8") || (int64_t)n_experts * (ffn / 64) < lk_device().cus / 4) return false;
     auto always = [](int type) { return type == LK_TYPE_Q5_K || type == LK_TYPE_Q8_0 || type == LK_TYPE_Q4_0; };
+    auto of_levels = [](int type) { return type == LK_TYPE_IQ4_NL || type == LK_TYPE_MXFP4; };
+    auto has_tiles = [&](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q6_K || always(type) || of_levels(type); };
+    if (!has_tiles(gu) || !has_tiles(down) || lk_env_flag("LK_MMQ_I8") || (int64_t)n_experts * (ffn / 64) < lk_device().cus / 4) return false;
     if (always(gu) || always(down)) return true;
+    if (of_levels(gu) || of_levels(down)) return longest > 32 || n_experts < 60;
     if (gu == LK_TYPE_Q6_K && down == LK_TYPE_Q6_K) return longest > 22 || n_experts < 60;
     return longest >= 20 || (longest >= 9 && hidden > 2048 && 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus);
 }

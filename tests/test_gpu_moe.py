@@ -663,7 +663,8 @@ def test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn):
     assert (np.abs(got.cpu().numpy()[sample] - fed) <= bound).all()
 
 
-@pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q8_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_K, lib.TYPE_Q4_0)])
+@pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q8_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_K, lib.TYPE_Q4_0),
+                                   (lib.TYPE_MXFP4, lib.TYPE_MXFP4), (lib.TYPE_IQ4_NL, lib.TYPE_MXFP4), (lib.TYPE_Q5_K, lib.TYPE_IQ4_NL)])
 @pytest.mark.parametrize("runs,hidden,ffn", [(RUNS, 256, 256), (RUNS, 768, 512)])
 def test_block_of_plain_blocks_on_the_f16_tiles(runs, hidden, ffn, gu, dn):
     test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn)
