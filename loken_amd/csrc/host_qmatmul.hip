@@ -38,9 +38,21 @@ bool tiled_serves(int dtype, int k) {
            k % 256 == 0;
 }
 
+// Nine to sixteen rows of Q8_0 and Q4_0 on the f16 tiles, operands straight from the rows, against the quantizer and two mat-vec
+// launches (Q4_0 from 16 rows or 48 M weights: int8 tiles). us, before / tiles: Q8_0 14336 x 4096 at 9 / 16 rows 32 / 39 against 30 / 30,
+// 4096 x 14336 45 / 65 against 36 / 36, 64000 x 2048 72 / 93 against 55 / 55, 11003 x 3072 at 9 / 12 / 16 24 / 26 / 29 against 26 / 26 / 26, 4096 x 4096 17.5 / 18.7 /
+// 21 against 19 / 19 / 19, 2048 x 2048 15.5 / 15.8 / 16.0 against 15.8 / 17.0 / 15.8; Q4_0 512 x 14336 at 9 / 12 30 / 38 against 24 / 25, 11003 x 3072 26 / 30 against 22 / 22,
+// 1024 x 4096 17.4 / 16.5 against 16.4 / 16.5, 4096 x 4096 17.5 / 18.6 against 17.7 / 17.0.
+bool few_rows_to_tiles(int dtype, int n, int k, int rows, const void* blob) {
+    if (rows <= 8 || rows > 16 || n < 512 || k % 256 != 0 || ((uintptr_t)blob & 1) != 0) return false;
+    const long long weights = (long long)n * k;
+    if (dtype == LK_TYPE_Q8_0) return weights >= (48ll << 20) || (rows >= 12 && (weights >= (32ll << 20) || k >= 8192)) || (rows >= 14 && k >= 4096);
+    return dtype == LK_TYPE_Q4_0;
+}
+
 // Q4_0 / Q4_1 / Q5_0 / Q5_1, Q3_K and Q2_K above eight rows: one tiled launch (with K cut into ranges
 // where its tiles are few, mmq_problem.h) against mat-vec launches of eight rows each. Measured on MI355X,
-// quantizer included, mat-vec against tiled: Q4_0 4096 x 4096 at 9 / 16 / 32 rows 29 / 35 / 55 us against
+// quantizer included, mat-vec against tiled (int8): Q4_0 4096 x 4096 at 9 / 16 / 32 rows 29 / 35 / 55 us against
 // 31 / 27 / 29; 14336 x 4096 at 9 / 16 rows 42 / 58 against 37 / 38; 4096 x 14336 at 9 rows 57 against 41;
 // 1024 x 4096 at 9 / 16 rows 27 / 31 against 33 / 26. Q5_1, Q3_K and Q2_K alike (Q3_K 4096 x 4096 at 9 / 16
 // rows 31 / 40 against 29 / 27). So: from 16 rows, and from 9 on a matrix of 48 M weights or more.
@@ -55,8 +67,7 @@ size_t elem_bytes(int type) { return type == LK_TYPE_F32 ? 4 : 2; }
 
 int matvec_rows(int dtype, int k) {
     if ((dtype == LK_TYPE_Q4_K || dtype == LK_TYPE_Q5_K || dtype == LK_TYPE_Q6_K) && k % 256 == 0) return 8;
-    // Q8_0, mat-vec launches of eight rows against the tiled matmul: 4096 x 4096 at 16 / 24 / 32 rows 32 / 40 /
-    // 49 us against 32 / 32 / 32; 14336 x 4096 51 / 70 / 89 against 56 / 56 / 58
+    // Q8_0: mat-vec launches of eight rows up to 16 rows, but for few_rows_to_tiles
     return dtype == LK_TYPE_Q8_0 && tiled_serves(dtype, k) ? 16 : 8;
 }
 
@@ -138,7 +149,8 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     // --- mat-vec family: up to matvec_rows, or any count when every row must sum like a one-row call
     const bool rows_kernel_fits = k_ % 256 == 0 && ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q6_K ? 1 : 15)) == 0;
     const bool to_rows_kernel = rows_kernel_fits && small_rows_kernel_pays(dtype_, n_, k_, rows);
-    const bool to_nibble_tiles = !decode_order && nibble_tiles_pay(dtype_, n_, k_, rows) &&
+    const bool few_to_tiles = few_rows_to_tiles(dtype_, n_, k_, rows, blob_);
+    const bool to_nibble_tiles = !decode_order && (few_to_tiles || nibble_tiles_pay(dtype_, n_, k_, rows)) &&
                                  ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q2_K ? 3 : 1)) == 0;
     auto matvec = [&]() -> int {
         if (!plain && x_type == LK_TYPE_F32 && rows <= 2 && k_ <= 8192 && ((uintptr_t)x & 15) == 0 && k_ % 4 == 0) {
@@ -163,7 +175,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
         last_path_ = Path::MatVec;
         return LK_OK;
     };
-    if ((rows <= mv_max && !to_rows_kernel) || decode_order || (plain && !to_nibble_tiles)) return matvec();
+    if ((rows <= mv_max && !to_rows_kernel && !few_to_tiles) || decode_order || (plain && !to_nibble_tiles)) return matvec();
 
     // --- a handful of rows (or a matrix too small to fill the chip with tiles): matrix unit, weights
     //     straight from HBM
@@ -218,12 +230,13 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
 }
 
 // takes_matvec of the reference (kernel_matmul.rs:1069-1075) with this mirror's own exceptions: the
-// K-quants' few rows over a large matrix go to the 16-row tiles, and the formats with tiles leave the
+// K-quants' few rows go to the 16-row tiles where that pays, nine rows and more of Q8_0 and Q4_0 to the f16 tiles, and the formats with tiles leave the
 // mat-vec launches from nibble_tiles_pay's row counts.
 bool QKernelMatMul::takes_matvec(int rows, bool decode_order) const {
     if (!blob_ || rows < 1) return false;
     if (decode_order && rows > 1) return true;
     const bool plain = matvec_only(dtype_);
+    if (few_rows_to_tiles(dtype_, n_, k_, rows, blob_)) return false;
     if (plain) return !nibble_tiles_pay(dtype_, n_, k_, rows) || rows <= matvec_rows(dtype_, k_);
     if (rows > matvec_rows(dtype_, k_)) return false;
     const bool rows_kernel_fits = k_ % 256 == 0 && ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q6_K ? 1 : 15)) == 0;

@@ -375,6 +375,21 @@ def test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expec
     assert close(got.cpu().numpy()[some][:, pick], oracle.ob_matmul(wtype, x[some], w[pick], len(pick)))
 
 
+@pytest.mark.parametrize("name,n,k,rows,expect", [
+    ("q8_0", 12289, 4096, 9, "tiled"), ("q8_0", 12287, 4096, 11, "matvec"), ("q8_0", 8193, 4096, 12, "tiled"), ("q8_0", 513, 4096, 14, "tiled"), ("q8_0", 513, 4096, 13, "matvec"),
+    ("q8_0", 513, 8192, 12, "tiled"),
+    ("q8_0", 513, 3840, 16, "matvec"), ("q8_0", 511, 4096, 16, "matvec"), ("q8_0", 12289, 4096, 8, "matvec"), ("q4_0", 512, 256, 9, "tiled"),
+    ("q4_0", 511, 768, 15, "matvec"), ("q4_0", 645, 2304, 12, "tiled"), ("q4_0", 645, 2304, 8, "matvec")])
+def test_nine_to_sixteen_rows_of_plain_blocks(name, n, k, rows, expect):
+    test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
+    q81 = torch.empty(lib.load().lkh_quantized_activation_bytes(k, rows), dtype=torch.uint8, device="cuda")
+    lin = Linear(DT[name], dev(synth.weight(DT[name], 8, k, seed=98).reshape(8, -1).repeat((n + 7) // 8, axis=0)[:n]), n, k)
+    x = dev(synth.activation(rows, k, seed=98))
+    status = lib.load().lkh_qkernel_matmul_quantize_for_matvec(lin.h, x.data_ptr(), X_TYPES[x.dtype], rows, q81.data_ptr(), torch.cuda.current_stream().cuda_stream, 0)
+    assert (status == 0) == (expect == "matvec")   # follows forward
+    lin.close()
+
+
 @pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
 @pytest.mark.parametrize("rows,n,k,shift", [(450, 2048, 256, 0), (180, 2561, 1280, 0), (33, 14336, 512, 1)])
 def test_operands_straight_from_the_rows_are_those_of_the_records(name, rows, n, k, shift):
