@@ -291,6 +291,9 @@ struct LkRegMulti {
 bool lk_q4k_reg_serves(int nb);
 int lk_q4k_reg_multi(const LkRegMulti& m, const void* act, int act_f32, int nb, int dst_type, int batch, int act_stride,
                      int dst_stride, hipStream_t stream);
+// One matrix over one or two rows of f16 or bf16 values, quantized in the launch, results in their type; -1: not taken (row
+// length, alignment), nothing launched.
+int lk_q4k_half_linear(const void* w, const void* x, int type, void* out, int rows, int n, int k, hipStream_t stream);
 // The gate/up pair over the activation rows: dst = act(gate . x) * (up . x) as f32 / bf16 (`dst_q8_1`
 // false; rows dst_stride elements apart) or as Q8_1 blocks of 32 consecutive rows (true; n a multiple of
 // 32; rows dst_stride blocks apart).

@@ -81,11 +81,20 @@ static __device__ __forceinline__ float row_share(const RowFrag& f, const Slice&
 // issue order, so the small activation must go first and must not wait for weights.
 // unit = 4 * slot + p: which 72 bytes of the Q8_1 row (64 bytes of the LDS image) are the lane's.
 // B activation rows, `act_stride` bytes apart, into B slices (the f32 form: B images of LDS_BYTES).
-template <bool ACT_F32, int B, class First>
+// ACT: Q8_1 rows, or rows of values, quantized here: half rows stay two bytes a value in registers until the weights are under way.
+constexpr int ACT_Q81 = 0, ACT_VALUES = 1, ACT_HALF = 2, ACT_BF16 = 3;
+template <int ACT>
+static __device__ __forceinline__ float4 values_of(const float4& v) { return v; }
+template <int ACT>
+static __device__ __forceinline__ float4 values_of(const uint2& v) {
+    if (ACT == ACT_HALF) return Load4<__half>::at((const __half*)&v);
+    return Load4<__hip_bfloat16>::at((const __hip_bfloat16*)&v);
+}
+template <int ACT, int B, class First>
 static __device__ __forceinline__ void slice_load(Slice (&s)[B], gbytes_t act, size_t act_stride, int nb, int unit, bool valid,
                                                   uint8_t* lds, First&& first_loads) {
 #pragma clang fp contract(off)
-    if (!ACT_F32) {
+    if constexpr (ACT == ACT_Q81) {
         // (cast back from the global address space: the compiler keeps track of where it came from)
         uint32_t head0[B], head1[B];
 #pragma unroll
@@ -105,14 +114,15 @@ static __device__ __forceinline__ void slice_load(Slice (&s)[B], gbytes_t act, s
         for (int b = 0; b < B; ++b) slice_finish(s[b], f16_bits_to_f32(head0[b] & 0xFFFFu), f16_bits_to_f32(head1[b] & 0xFFFFu));
         return;
     }
-    // f32 row: item t is four values, eight consecutive items (lanes) are one Q8_1 block
+    // row of values: item t is four of them, eight consecutive items (lanes) are one Q8_1 block
+    using quad = typename std::conditional<ACT == ACT_VALUES, float4, uint2>::type;
     const int items = nb * 64;
-    float4 v[B][2];
+    quad v[B][2];
 #pragma unroll
     for (int b = 0; b < B; ++b)
 #pragma unroll
         for (int u = 0; u < 2; ++u)
-            v[b][u] = *(const float4*)(const uint8_t*)(act + b * act_stride + 16 * min((int)threadIdx.x + u * RT, items - 1));
+            v[b][u] = *(const quad*)(const uint8_t*)(act + b * act_stride + (int)sizeof(quad) * min((int)threadIdx.x + u * RT, items - 1));
     load_fence((const void*)lds);
     first_loads();
     load_fence((const void*)lds);
@@ -124,7 +134,7 @@ static __device__ __forceinline__ void slice_load(Slice (&s)[B], gbytes_t act, s
         for (int u = 0; u < 2; ++u) {
             const int item = threadIdx.x + u * RT;
             if (item < items) {   // whole waves: items is a multiple of 64
-                const float4 x = v[b][u];
+                const float4 x = values_of<ACT>(v[b][u]);
                 const float amax = max8(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
                 const float d = amax / 127.0f;
                 const float inv = d != 0.0f ? 1.0f / d : 0.0f;
@@ -180,10 +190,10 @@ struct Geo {
 // Up to four matrices over one activation row. A tile is R * RP consecutive rows of one matrix;
 // wave g of the grid takes tiles g, g + waves, ...
 // B: activation rows (1 or 2), act_stride bytes apart; their outputs dst_stride elements apart.
-template <int R, int RP, bool ACT_F32, int B>
+template <int R, int RP, int ACT, int B>
 __global__ __launch_bounds__(RT) void q4k_reg_kernel(RegArgs a, const uint8_t* __restrict__ act, int nb, int dst_type,
                                                      int waves, int act_stride, int dst_stride) {
-    __shared__ __align__(16) uint8_t lds[ACT_F32 ? B * LDS_BYTES : 16];
+    __shared__ __align__(16) uint8_t lds[ACT != ACT_Q81 ? B * LDS_BYTES : 16];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int TR = R * RP;
     uint32_t flip = 0x80808080u;
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_kernel(RegArgs a, const uint8_t* _
     // (a wave without a tile loads the last one rather than nothing: the count of loads ahead of
     // the weights stays the same for every wave)
     relocate(min(t, total - 1));
-    slice_load<ACT_F32, B>(s, act_g, (size_t)act_stride, nb, g.unit, g.valid, lds, [&] { load(min(t, total - 1)); });
+    slice_load<ACT, B>(s, act_g, (size_t)act_stride, nb, g.unit, g.valid, lds, [&] { load(min(t, total - 1)); });
     const bool odd = g.lane & 1;
     while (t < total) {
         void* dst = (void*)(uint8_t*)to_gbytes((uint64_t)cur_dst);
@@ -327,7 +337,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
         // tiles of RP rows, wave-strided
         const int tiles = (n + RP - 1) / RP, step = (int)gridDim.x * waves;
         int t = (int)blockIdx.x * waves + wave;
-        slice_load<ACT_F32, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds,
+        slice_load<ACT_F32 ? ACT_VALUES : ACT_Q81, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds,
                                [&] { load(min(t, tiles - 1) * RP + g.rp); });
         while (t < tiles) {
             const int row = t * RP + g.rp;
@@ -354,7 +364,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
         row_load(bg[slot], wg + at, g.hdr_off, g.qs_off);
         row_load(bu[slot], wu + at, g.hdr_off, g.qs_off);
     };
-    slice_load<ACT_F32, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds, [&] {
+    slice_load<ACT_F32 ? ACT_VALUES : ACT_Q81, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds, [&] {
 #pragma unroll
         for (int i = 0; i < D; ++i) load_pass(i, min(b, blocks - 1), i);
     });
@@ -471,7 +481,7 @@ static Shape shape_for(bool act_f32) {
 }
 
 template <int R, int RP, int B>
-static int launch_multi(const LkRegMulti& m, const void* act, int act_f32, int nb, int dst_type, int act_stride, int dst_stride,
+static int launch_multi(const LkRegMulti& m, const void* act, int act_form, int nb, int dst_type, int act_stride, int dst_stride,
                         hipStream_t s) {
     RegArgs a{};
     int total = 0;
@@ -485,16 +495,15 @@ static int launch_multi(const LkRegMulti& m, const void* act, int act_f32, int n
         }
         a.tile_end[i] = total;
     }
-    const Shape sh = shape_for(act_f32 != 0);
+    const Shape sh = shape_for(act_form != ACT_Q81);
     const int need = (total + sh.waves - 1) / sh.waves;
     const int forced_grid = lk_tune_env("LK_TUNE_REG_GRID");
     const dim3 grid(forced_grid > 0 ? (forced_grid < need ? forced_grid : need) : need < sh.cap ? need : sh.cap), block(sh.waves * 64);
-    if (act_f32)
-        hipLaunchKernelGGL((q4k_reg_kernel<R, RP, true, B>), grid, block, 0, s, a, (const uint8_t*)act, nb, dst_type, sh.waves,
-                           act_stride, dst_stride);
-    else
-        hipLaunchKernelGGL((q4k_reg_kernel<R, RP, false, B>), grid, block, 0, s, a, (const uint8_t*)act, nb, dst_type, sh.waves,
-                           act_stride, dst_stride);
+    auto kernel = act_form == ACT_Q81      ? q4k_reg_kernel<R, RP, ACT_Q81, B>
+                  : act_form == ACT_VALUES ? q4k_reg_kernel<R, RP, ACT_VALUES, B>
+                  : act_form == ACT_HALF   ? q4k_reg_kernel<R, RP, ACT_HALF, B>
+                                           : q4k_reg_kernel<R, RP, ACT_BF16, B>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, a, (const uint8_t*)act, nb, dst_type, sh.waves, act_stride, dst_stride);
     return lk_launch_status();
 }
 
@@ -535,7 +544,7 @@ bool lk_q4k_reg_serves(int nb) {
 }
 
 template <int B>
-static int multi_rows(const LkRegMulti& m, const void* act, int act_f32, int nb, int dst_type, int act_bytes, int dst_stride,
+static int multi_rows(const LkRegMulti& m, const void* act, int act_form, int nb, int dst_type, int act_bytes, int dst_stride,
                       hipStream_t stream) {
     const int rp = q4k_rows_per_pass(nb);
     // Two rows per wave tile while every wave still gets at most one tile (the launch is one round
@@ -543,19 +552,19 @@ static int multi_rows(const LkRegMulti& m, const void* act, int act_f32, int nb,
     int rows = 0;
     for (int i = 0; i < m.count; ++i) rows += m.n[i];
     const int forced = lk_tune_env("LK_TUNE_REG_R");
-    const Shape sh = shape_for(act_f32 != 0);
+    const Shape sh = shape_for(act_form != ACT_Q81);
     // (from f32 rows the bound is one workgroup per CU: q + k + v of a Llama-sized layer, 6144 rows, is
     // faster as single rows over two workgroups per CU, 5.7 against 6.1 us; o, 4096 rows, as pairs)
-    const int waves_at_once = (act_f32 ? lk_device().cus : sh.cap) * sh.waves;
+    const int waves_at_once = (act_form != ACT_Q81 ? lk_device().cus : sh.cap) * sh.waves;
     // (rows short enough to go side by side already give a wave two or four rows per pass: two such
     // tiles per wave measured slower, Qwen3-1.7B step 0.598 against 0.586 ms)
     const bool two = forced ? forced == 2 : rp == 1 && rows <= waves_at_once * 2;
     switch (rp) {
-        case 1: return two ? launch_multi<2, 1, B>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream)
-                           : launch_multi<1, 1, B>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream);
-        case 2: return two ? launch_multi<2, 2, B>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream)
-                           : launch_multi<1, 2, B>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream);
-        default: return launch_multi<1, 4, B>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream);
+        case 1: return two ? launch_multi<2, 1, B>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream)
+                           : launch_multi<1, 1, B>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream);
+        case 2: return two ? launch_multi<2, 2, B>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream)
+                           : launch_multi<1, 2, B>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream);
+        default: return launch_multi<1, 4, B>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream);
     }
 }
 
@@ -565,6 +574,20 @@ int lk_q4k_reg_multi(const LkRegMulti& m, const void* act, int act_f32, int nb, 
     const int act_bytes = act_stride * (act_f32 ? (int)sizeof(float) : Q81_BYTES);
     return batch == 1 ? multi_rows<1>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream)
                       : multi_rows<2>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream);
+}
+
+int lk_q4k_half_linear(const void* w, const void* x, int type, void* out, int rows, int n, int k, hipStream_t stream) {
+    if (type != LK_TYPE_F16 && type != LK_TYPE_BF16) return -1;
+    if (rows < 1 || rows > LK_REG_MAX_BATCH || n < 1 || k % 256 != 0 || !lk_q4k_reg_serves(k / 256) || (uintptr_t)w % 16 != 0 ||
+        (uintptr_t)x % 8 != 0)
+        return -1;
+    LkRegMulti m{};
+    m.vx[0] = (const uint8_t*)w;
+    m.dst[0] = out;
+    m.n[0] = n;
+    m.count = 1;
+    const int form = type == LK_TYPE_F16 ? ACT_HALF : ACT_BF16;
+    return rows == 1 ? multi_rows<1>(m, x, form, k / 256, type, 2 * k, n, stream) : multi_rows<2>(m, x, form, k / 256, type, 2 * k, n, stream);
 }
 
 template <int RP>

@@ -390,6 +390,31 @@ def test_nine_to_sixteen_rows_of_plain_blocks(name, n, k, rows, expect):
     lin.close()
 
 
+@pytest.mark.parametrize("half", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,n,k,shift,expect", [(1, 1, 256, 0, "matvec-fused"), (2, 7, 1024, 4, "matvec-fused"), (1, 301, 2048, 0, "matvec-fused"),
+                                                   (2, 4099, 4096, 8, "matvec-fused"), (1, 9001, 3840, 0, "matvec-fused"), (2, 2050, 2048, 0, "matvec-fused"),
+                                                   (1, 64, 1024, 2, "matvec"), (2, 64, 4352, 0, "matvec")])
+def test_half_rows_quantized_in_the_launch_carry_the_quantizers_codes(rows, n, k, shift, expect, half):
+    # One launch over one or two half rows of Q4_K: the bits of quantizer and mat-vec, rows from any 8-byte boundary; rows off it,
+    # and longer ones, go on as two launches. Zeros, the largest codes, tiny values, infinities and NaN among them.
+    w = dev(synth.weight(lib.TYPE_Q4_K, n, k, seed=99, stream=1))
+    x = dev(synth.activation(rows, k, seed=99))
+    x[0, :32] = 0
+    x[0, 32:64] *= 1e-6
+    x[rows - 1, 64] = 127
+    flat = torch.zeros(rows * k + shift, device="cuda", dtype=half)
+    flat[shift:] = x.reshape(-1).to(half)
+    x = flat[shift:].view(rows, k)
+    lin = Linear(lib.TYPE_Q4_K, w, n, k)
+    for _ in range(2):
+        got = lin(x)
+        assert lin.path == expect and got.dtype == half
+        want = ops.mmvq(lib.TYPE_Q4_K, w, ops.quantize_q8_1_rows(x.contiguous()), k, n, out_dtype=half)
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
+        x[0, 5], x[rows - 1, k - 1] = float("inf"), float("nan")
+    lin.close()
+
+
 @pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
 @pytest.mark.parametrize("rows,n,k,shift", [(450, 2048, 256, 0), (180, 2561, 1280, 0), (33, 14336, 512, 1)])
 def test_operands_straight_from_the_rows_are_those_of_the_records(name, rows, n, k, shift):
