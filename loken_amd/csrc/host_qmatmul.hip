@@ -38,6 +38,19 @@ bool tiled_serves(int dtype, int k) {
            k % 256 == 0;
 }
 
+// One or two rows in one launch, against the quantizer's launch and the mat-vec's (us): every workgroup quantizes the rows, which a matrix that keeps
+// the chip busy longer than the second launch costs pays for several times over. Two rows: 1024 x 4096 6.8 / 9.7, 4096 x 4096 Q4_K, Q6_K, Q8_0 7.0, 8.3, 7.9 / 9.8; 8192 x 4096 Q4_K,
+// Q5_K, Q6_K, Q8_0 7.9, 10.2, 11.2, 11.1 / 10.0, 14336 x 4096 Q4_K, Q8_0 9.6, 15.2 / 10.4, 13.3, 14336 x 2048 Q5_K, Q6_K, Q8_0 10.6, 11.9, 9.5 / 9.9, 10.5, 9.7; 1024 x 6144 7.8, 8.3, 9.6, 7.7 / 9.8, 2048 x 8192 8.2, 8.8, 10.2, 10.6 / 9.7,
+// 4096 x 8192 11.5, 12.6, 13.8, 13.3 / 10.0, 12288 x 6144 17.4, 19.4, 22.0, 20.2 / 12.8, 14.9, 17.4, 16.1. One row: up to 14336 x 4096 6.8 to
+// 11.1 / 9.6 to 12.8, 4096 x 8192 8.4, 8.8, 10.0, 10.0 / 9.9, 9.9, 10.0, 10.0, 12288 x 6144 12.5, 14.3, 16.2, 14.4 / 11.7, 13.3, 14.3, 15.3,
+// 28672 x 8192 25.8, 30.9, 38.5, 45.9 / 26.3, 31.5, 37.6, 46.0.
+bool pays_in_one_launch(int dtype, int n, int k, int rows) {
+    const long long weights = (long long)n * k;
+    if (rows == 1) return k <= 4096 || dtype == LK_TYPE_Q8_0 || weights <= (40ll << 20) || (dtype != LK_TYPE_Q6_K && weights >= (128ll << 20));
+    if (k <= 4096) return dtype == LK_TYPE_Q4_K || weights <= (dtype == LK_TYPE_Q8_0 ? 28ll << 20 : 24ll << 20);
+    return weights <= (dtype == LK_TYPE_Q4_K || dtype == LK_TYPE_Q5_K ? 16ll << 20 : 12ll << 20);
+}
+
 // Nine to sixteen rows of Q8_0 and Q4_0 on the f16 tiles, operands straight from the rows, against the quantizer and two mat-vec
 // launches (Q4_0 from 16 rows or 48 M weights: int8 tiles). us, before / tiles: Q8_0 14336 x 4096 at 9 / 16 rows 32 / 39 against 30 / 30,
 // 4096 x 14336 45 / 65 against 36 / 36, 64000 x 2048 72 / 93 against 55 / 55, 11003 x 3072 at 9 / 12 / 16 24 / 26 / 29 against 26 / 26 / 26, 4096 x 4096 17.5 / 18.7 /
@@ -153,25 +166,21 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     const bool to_nibble_tiles = !decode_order && (few_to_tiles || nibble_tiles_pay(dtype_, n_, k_, rows)) &&
                                  ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q2_K ? 3 : 1)) == 0;
     auto matvec = [&]() -> int {
-        if (!plain && x_type == LK_TYPE_F32 && rows <= 2 && k_ <= 8192 && ((uintptr_t)x & 15) == 0 && k_ % 4 == 0) {
+        // One or two rows quantized in the mat-vec launch itself
+        auto in_one_launch = [&]() -> int {
+            last_path_ = Path::MatVecFused;
+            if (x_type != LK_TYPE_F32) return lk_mmvq_half_rows(dtype_, blob_, x, x_type, out, rows, n_, k_, stream);
             const void* vx[1] = {blob_};
             void* dst[1] = {out};
             const int nn[1] = {n_};
-            last_path_ = Path::MatVecFused;
             return lk_mmvq_fused(dtype_, 1, vx, (const float*)x, k_, dst, x_type, k_, nn, rows, n_, nullptr, stream);
-        }
-        // (Q4_K, half rows in one launch too: 512 x 1024 to 14336 x 4096 at 1 and 2 rows 10.0..10.6 -> 7.1..7.6 us, two rows of 14336 x 4096 10.5 -> 9.6)
-        if (dtype_ == LK_TYPE_Q4_K && rows <= 2) {
-            const int rc = lk_q4k_half_linear(blob_, x, x_type, out, rows, n_, k_, stream);
-            if (rc >= 0) {
-                if (rc == LK_OK) last_path_ = Path::MatVecFused;
-                return rc;
-            }
-        }
+        };
+        const bool can_fuse = !plain && rows <= 2 && k_ <= 8192 && ((uintptr_t)x & (x_type == LK_TYPE_F32 ? 15 : 7)) == 0 && k_ % 4 == 0;
+        if (can_fuse && pays_in_one_launch(dtype_, n_, k_, rows)) return in_one_launch();
         const int k_padded = (int)pad_to((size_t)k_, 512), blocks = k_padded / 32;
         LkScratch scratch(stream);
         uint8_t* act = (uint8_t*)scratch.get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK);
-        if (!act) return LK_ERR_NOMEM;
+        if (!act) return can_fuse ? in_one_launch() : LK_ERR_NOMEM;   // (the same bits)
         if (int rc = lk_quantize_q8_1(x, x_type, act, k_, k_padded, rows, stream)) return rc;
         for (int r0 = 0; r0 < rows; r0 += 8) {
             const int b = rows - r0 < 8 ? rows - r0 : 8;

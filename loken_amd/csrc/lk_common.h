@@ -289,11 +289,11 @@ struct LkRegMulti {
     int count;
 };
 bool lk_q4k_reg_serves(int nb);
-int lk_q4k_reg_multi(const LkRegMulti& m, const void* act, int act_f32, int nb, int dst_type, int batch, int act_stride,
+enum { LK_REG_Q8_1 = 0, LK_REG_F32 = 1, LK_REG_F16 = 2, LK_REG_BF16 = 3 };   // what the activation rows hold
+int lk_q4k_reg_multi(const LkRegMulti& m, const void* act, int act_form, int nb, int dst_type, int batch, int act_stride,
                      int dst_stride, hipStream_t stream);
-// One matrix over one or two rows of f16 or bf16 values, quantized in the launch, results in their type; -1: not taken (row
-// length, alignment), nothing launched.
-int lk_q4k_half_linear(const void* w, const void* x, int type, void* out, int rows, int n, int k, hipStream_t stream);
+// One matrix over one or two rows of f16 or bf16 values (8-byte aligned, k apart), quantized in the launch, results in their type.
+int lk_mmvq_half_rows(int wtype, const void* w, const void* x, int type, void* out, int rows, int n, int k, void* stream);
 // The gate/up pair over the activation rows: dst = act(gate . x) * (up . x) as f32 / bf16 (`dst_q8_1`
 // false; rows dst_stride elements apart) or as Q8_1 blocks of 32 consecutive rows (true; n a multiple of
 // 32; rows dst_stride blocks apart).

@@ -161,9 +161,9 @@ static int check_weight(int wtype, const void* vx) {
 
 static int run_multi(int wtype, int count, const void* const* vx, const void* vy, void* const* dst, int dst_type,
                      int ncols_x, const int* nrows_x, int batch, int stride_col_y, int stride_col_dst,
-                     const float* const* bias, void* stream, int act_stride_f32 = 0) {
+                     const float* const* bias, void* stream, int act_stride_f32 = 0, bool half_rows = false) {
     if (int rc = check_common(wtype, vy, ncols_x, batch, act_stride_f32 ? ncols_x / 32 : stride_col_y)) return rc;
-    if (act_stride_f32 && (act_stride_f32 < ncols_x || act_stride_f32 % 4 != 0 || ((uintptr_t)vy & 15) != 0)) return LK_ERR_ARG;
+    if (act_stride_f32 && (act_stride_f32 < ncols_x || act_stride_f32 % 4 != 0 || ((uintptr_t)vy & (half_rows ? 7 : 15)) != 0)) return LK_ERR_ARG;
     if (count < 1 || count > MAX_MULTI) return LK_ERR_ARG;
     MmvqCall a{};
     a.vy = (const uint8_t*)vy;
@@ -171,6 +171,7 @@ static int run_multi(int wtype, int count, const void* const* vx, const void* vy
     a.stride_col_y = stride_col_y;
     a.stride_col_dst = stride_col_dst;
     a.act_stride_f32 = act_stride_f32;
+    a.half_rows = half_rows;
     a.stream = (hipStream_t)stream;
     int live = 0;
     for (int i = 0; i < count; ++i) {
@@ -197,7 +198,7 @@ static int run_multi(int wtype, int count, const void* const* vx, const void* vy
             m.bias[i] = a.m.bias[i];
             m.n[i] = a.m.n[i];
         }
-        return lk_q4k_reg_multi(m, vy, act_stride_f32 != 0, a.nb, dst_type, batch, act_stride_f32 ? act_stride_f32 : stride_col_y,
+        return lk_q4k_reg_multi(m, vy, !act_stride_f32 ? LK_REG_Q8_1 : !half_rows ? LK_REG_F32 : dst_type == LK_TYPE_F16 ? LK_REG_F16 : LK_REG_BF16, a.nb, dst_type, batch, act_stride_f32 ? act_stride_f32 : stride_col_y,
                                 stride_col_dst, a.stream);
     }
     // A launch stages all its activation rows in LDS; a batch that does not fit (long rows) goes
@@ -209,7 +210,7 @@ static int run_multi(int wtype, int count, const void* const* vx, const void* vy
     for (int b0 = 0; b0 < batch; b0 += share) {
         const int b = batch - b0 < share ? batch - b0 : share;
         MmvqCall c = a;
-        c.vy = a.vy + (act_stride_f32 ? (size_t)b0 * act_stride_f32 * sizeof(float) : (size_t)b0 * stride_col_y * Q81_BYTES);
+        c.vy = a.vy + (act_stride_f32 ? (size_t)b0 * act_stride_f32 * (half_rows ? 2 : sizeof(float)) : (size_t)b0 * stride_col_y * Q81_BYTES);
         for (int i = 0; i < live; ++i) c.m.dst[i] = (uint8_t*)a.m.dst[i] + (size_t)b0 * stride_col_dst * dst_elem;
         if (int rc = dispatch_plain(wtype, dst_type, b, c)) return rc;
     }
@@ -255,6 +256,11 @@ extern "C" int lk_mmvq_fused(int wtype, int count, const void* const* vx, const 
     if (!vx || !dst || !nrows_x || stride_x <= 0) return LK_ERR_ARG;
     return run_multi(wtype, count, vx, x, dst, dst_type, ncols_x, nrows_x, batch, 0, stride_col_dst, bias, stream,
                      stride_x);
+}
+
+int lk_mmvq_half_rows(int wtype, const void* w, const void* x, int type, void* out, int rows, int n, int k, void* stream) {
+    if ((type != LK_TYPE_F16 && type != LK_TYPE_BF16) || rows > 2) return LK_ERR_ARG;
+    return run_multi(wtype, 1, &w, x, &out, type, k, &n, rows, 0, n, nullptr, stream, k, true);
 }
 
 extern "C" int lk_mmvq_pair_act(int wtype, const void* gate, const void* up, const void* vy_q8_1, void* dst,

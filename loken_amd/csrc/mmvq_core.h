@@ -207,7 +207,6 @@ struct ActRegs {
     static constexpr int ROWS = B <= 2 ? B : 0;
     uint32_t head[ROWS ? ROWS : 1];   // a Q8_1 block: d and s, then the two halves of its codes
     uint4 lo[ROWS ? ROWS : 1], hi[ROWS ? ROWS : 1];
-    float4 x[ROWS ? ROWS : 1][4];
 };
 
 // One Q8_1 block (j-th of its row; `real` false past the row's end) into the LDS image of `row`.
@@ -331,27 +330,38 @@ static __device__ __forceinline__ void put_f32_quad(uint8_t* row, int n_iter, in
 constexpr int F32_ROUND = 4;  // float4 loads a thread issues together: the lane exchanges would
                               // otherwise serialize one memory latency per 1024 values
 
-template <class F, int B>
-static __device__ __forceinline__ void load_f32_round(float4 (&v)[F32_ROUND], const float* __restrict__ x, int t0,
+// Four values as they lie (half rows: two bytes each until they are quantized), and as f32.
+template <typename T> struct ValueQuad { typedef uint2 raw; };
+template <> struct ValueQuad<float> { typedef float4 raw; };
+template <typename T>
+static __device__ __forceinline__ float4 quad_values(const typename ValueQuad<T>::raw& v) { return Load4<T>::at((const T*)&v); }
+
+template <class F, int B, typename T>
+static __device__ __forceinline__ void load_f32_round(typename ValueQuad<T>::raw (&v)[F32_ROUND], const T* __restrict__ x, int t0,
                                                       int items, int k32) {
 #pragma unroll
     for (int u = 0; u < F32_ROUND; ++u) {
         // past the row's end: re-read its last quad (dropped by the caller), never a branch
         const int t = min(t0 + u * WG, k32 * 8 - 1);
-        v[u] = *(const float4*)(x + (size_t)t * 4);
+        v[u] = *(const typename ValueQuad<T>::raw*)(x + (size_t)t * 4);
     }
 }
 
-template <class F, int B>
-static __device__ __forceinline__ void stage_issue_f32(ActRegs<B>& ar, const float* __restrict__ x, int k32,
+template <int B, typename T>
+struct ValueRegs {
+    static constexpr int ROWS = ActRegs<B>::ROWS;
+    typename ValueQuad<T>::raw x[ROWS ? ROWS : 1][F32_ROUND];
+};
+template <class F, int B, typename T>
+static __device__ __forceinline__ void stage_issue_f32(ValueRegs<B, T>& ar, const T* __restrict__ x, int k32,
                                                        int n_iter, int x_stride) {
     const int items = n_iter * (F::VPI / 32) * 8;
 #pragma unroll
-    for (int c = 0; c < ActRegs<B>::ROWS; ++c) load_f32_round<F, B>(ar.x[c], x + (size_t)c * x_stride, threadIdx.x, items, k32);
+    for (int c = 0; c < ActRegs<B>::ROWS; ++c) load_f32_round<F, B, T>(ar.x[c], x + (size_t)c * x_stride, threadIdx.x, items, k32);
 }
 
-template <class F, int B>
-static __device__ __forceinline__ void stage_finish_f32(const ActRegs<B>& ar, uint8_t* lds, const float* __restrict__ x,
+template <class F, int B, typename T>
+static __device__ __forceinline__ void stage_finish_f32(const ValueRegs<B, T>& ar, uint8_t* lds, const T* __restrict__ x,
                                                         int k32, int n_iter, int x_stride) {
     const int items = n_iter * (F::VPI / 32) * 8;
     const int row_bytes = lds_bytes_per_row<F>(n_iter);
@@ -361,23 +371,23 @@ static __device__ __forceinline__ void stage_finish_f32(const ActRegs<B>& ar, ui
         for (int c = 0; c < ActRegs<B>::ROWS; ++c)
 #pragma unroll
             for (int u = 0; u < F32_ROUND; ++u)
-                if (t0 + u * WG < items) put_f32_quad<F>(lds + c * row_bytes, n_iter, k32, t0 + u * WG, ar.x[c][u]);
+                if (t0 + u * WG < items) put_f32_quad<F>(lds + c * row_bytes, n_iter, k32, t0 + u * WG, quad_values<T>(ar.x[c][u]));
         t0 += WG * F32_ROUND;
     }
     for (; t0 < items; t0 += WG * F32_ROUND) {
 #pragma unroll
         for (int c = 0; c < B; ++c) {
-            float4 v[F32_ROUND];
-            load_f32_round<F, B>(v, x + (size_t)c * x_stride, t0, items, k32);
+            typename ValueQuad<T>::raw v[F32_ROUND];
+            load_f32_round<F, B, T>(v, x + (size_t)c * x_stride, t0, items, k32);
 #pragma unroll
             for (int u = 0; u < F32_ROUND; ++u)
-                if (t0 + u * WG < items) put_f32_quad<F>(lds + c * row_bytes, n_iter, k32, t0 + u * WG, v[u]);
+                if (t0 + u * WG < items) put_f32_quad<F>(lds + c * row_bytes, n_iter, k32, t0 + u * WG, quad_values<T>(v[u]));
         }
     }
 }
 
 // What a workgroup computes: rows of `vx[0..NW)` against the B activation rows at `vy`.
-template <int NW>
+template <int NW, typename V = float>   // V: what rows of values hold where half_rows is set
 struct RowJob {
     gbytes_t vx[NW];
     const uint8_t* vy;
@@ -386,17 +396,18 @@ struct RowJob {
     int stride_col_y;  // Q8_1 blocks between activation rows
     int tile_stride;   // row tiles between a wave's consecutive tiles
     int tile_first;    // first row tile of wave 0 of this workgroup
-    int act_stride_f32 = 0;  // non-zero: `vy` holds f32 activation rows this many floats apart,
+    int act_stride_f32 = 0;  // non-zero: `vy` holds activation rows of values this many values apart (f32, or V where half_rows is set: two rows at most),
                              // quantized to Q8_1 by the workgroup itself while staging
     // A wave's tiles: it starts at tile_first + wave * wave_stride, walks run_len consecutive tiles
     // (a power of two; the run starts on a multiple of it) and then jumps tile_stride from the
     // run's last tile. The defaults give the plain round-robin tile, tile + tile_stride, ...
     int wave_stride = 1;
     int run_len = 1;
+    int half_rows = 0;
 };
 
-template <int NW>
-static __device__ __forceinline__ int next_tile(const RowJob<NW>& job, int t) {
+template <int NW, typename V>
+static __device__ __forceinline__ int next_tile(const RowJob<NW, V>& job, int t) {
     return (job.run_len > 1 && ((t + 1) & (job.run_len - 1))) ? t + 1 : t + job.tile_stride;
 }
 
@@ -416,16 +427,22 @@ static __device__ __forceinline__ void load_fence(const void* p) {
 // first weight loads) between the two halves. Each form runs `mid` in its own branch: merged
 // after the branch, the wait for the activation data could no longer tell how many loads are
 // ahead of the weights and would wait for part of them too.
-template <class F, int B, int NW, class Mid>
-static __device__ __forceinline__ void stage_around(uint8_t* lds, const RowJob<NW>& job, int k32, int n_iter, Mid&& mid) {
-    ActRegs<B> ar;
-    if (job.act_stride_f32) {
-        stage_issue_f32<F, B>(ar, (const float*)job.vy, k32, n_iter, job.act_stride_f32);
+template <class F, int B, int NW, class Mid, typename V>
+static __device__ __forceinline__ void stage_around(uint8_t* lds, const RowJob<NW, V>& job, int k32, int n_iter, Mid&& mid) {
+    auto values = [&](const auto* x) {
+        ValueRegs<B, std::remove_cv_t<std::remove_pointer_t<decltype(x)>>> ar;
+        stage_issue_f32<F, B>(ar, x, k32, n_iter, job.act_stride_f32);
         load_fence(job.vy);
         mid();
         load_fence(job.vy);
-        stage_finish_f32<F, B>(ar, lds, (const float*)job.vy, k32, n_iter, job.act_stride_f32);
+        stage_finish_f32<F, B>(ar, lds, x, k32, n_iter, job.act_stride_f32);
+    };
+    if constexpr (sizeof(V) == 2 && B <= 2)
+        if (job.half_rows) return values((const V*)job.vy);
+    if (job.act_stride_f32) {
+        values((const float*)job.vy);
     } else {
+        ActRegs<B> ar;
         stage_issue_q8_1<F, B>(ar, job.vy, k32, job.stride_col_y);
         load_fence(job.vy);
         mid();
@@ -460,8 +477,8 @@ static __device__ __forceinline__ void row16_sums(float v, float (&q)[4]) {
 // done(tile) runs on every lane of the wave once the tile's rows have been handed to epi.
 // PACK false: one row per pass, all of this a compile-time 1 / 16 (the long-row kernels pay
 // nothing for the short-row form); PACK true: rows per pass from the row length.
-template <int B, int R, int NW, bool PACK, bool Q5, class Epi, class Done>
-static __device__ __forceinline__ void rows_q4k(const RowJob<NW>& job, uint8_t* lds, Epi&& epi, Done&& done) {
+template <int B, int R, int NW, bool PACK, bool Q5, class Epi, class Done, typename V>
+static __device__ __forceinline__ void rows_q4k(const RowJob<NW, V>& job, uint8_t* lds, Epi&& epi, Done&& done) {
     // Q5_K: the Q4_K header, then 32 bytes of fifth bits, then the nibbles
     constexpr int BB = Q5 ? Q5K_BYTES : Q4K_BYTES, QS0 = Q5 ? 48 : 16;
     const int nb = job.nb, n = job.n;
@@ -627,8 +644,8 @@ static __device__ __forceinline__ void rows_q4k(const RowJob<NW>& job, uint8_t* 
 // fragments, and the very first loads go out between the two halves of the activation staging so
 // that the two memory latencies overlap.
 // ---------------------------------------------------------------------------------------------
-template <class Frag, int NW, class Stage, class Load, class Compute>
-static __device__ __forceinline__ void step_loop(const RowJob<NW>& job, int tile, int n_tiles, int n_iter, Stage&& stage,
+template <class Frag, int NW, class Stage, class Load, class Compute, typename V>
+static __device__ __forceinline__ void step_loop(const RowJob<NW, V>& job, int tile, int n_tiles, int n_iter, Stage&& stage,
                                                  Load&& load, Compute&& compute) {
     int it = 0;
     Frag fa, fb;
@@ -662,8 +679,8 @@ static __device__ __forceinline__ void step_loop(const RowJob<NW>& job, int tile
 // ---------------------------------------------------------------------------------------------
 // PACK: rows of at most 8 (4) super-blocks share a pass two (four) at a time, each in its own 32 (16)
 // lanes, as the short Q4_K rows do.
-template <int B, int R, int NW, bool PACK, class Epi, class Done>
-static __device__ __forceinline__ void rows_q6k(const RowJob<NW>& job, uint8_t* lds, Epi&& epi, Done&& done) {
+template <int B, int R, int NW, bool PACK, class Epi, class Done, typename V>
+static __device__ __forceinline__ void rows_q6k(const RowJob<NW, V>& job, uint8_t* lds, Epi&& epi, Done&& done) {
     const int nb = job.nb, n = job.n;
     const int n_iter_lds = (nb + 15) >> 4;   // passes of the staged activation (its layout)
     const int row_bytes = lds_bytes_per_row<FmtQ6K>(n_iter_lds);
@@ -787,8 +804,8 @@ static __device__ __forceinline__ void rows_q6k(const RowJob<NW>& job, uint8_t* 
 // ---------------------------------------------------------------------------------------------
 // Q8_0: 2 lanes per 32-value block, 32 blocks per wave pass.
 // ---------------------------------------------------------------------------------------------
-template <int B, int R, int NW, class Epi, class Done>
-static __device__ __forceinline__ void rows_q80(const RowJob<NW>& job, uint8_t* lds, Epi&& epi, Done&& done) {
+template <int B, int R, int NW, class Epi, class Done, typename V>
+static __device__ __forceinline__ void rows_q80(const RowJob<NW, V>& job, uint8_t* lds, Epi&& epi, Done&& done) {
     const int nb = job.nb, n = job.n;
     const int n_iter = (nb + 31) >> 5;
     const int row_bytes = lds_bytes_per_row<FmtQ80>(n_iter);
@@ -870,8 +887,8 @@ struct EngQ4K {
     static constexpr bool ONE_ROW_TILES = false;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 8;
     static __host__ __device__ int rows_per_pass(int) { return 1; }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q4k<B, R, NW, false, false>(j, lds, e, d);
     }
 };
@@ -881,8 +898,8 @@ struct EngQ4KShort {
     static constexpr bool ONE_ROW_TILES = false;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 8;
     static __host__ __device__ int rows_per_pass(int nb) { return q4k_rows_per_pass(nb); }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q4k<B, R, NW, true, false>(j, lds, e, d);
     }
 };
@@ -892,8 +909,8 @@ struct EngQ5K {
     static constexpr bool ONE_ROW_TILES = false;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 8;
     static __host__ __device__ int rows_per_pass(int) { return 1; }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q4k<B, R, NW, false, true>(j, lds, e, d);
     }
 };
@@ -902,8 +919,8 @@ struct EngQ5KShort {
     static constexpr bool ONE_ROW_TILES = false;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 8;
     static __host__ __device__ int rows_per_pass(int nb) { return q4k_rows_per_pass(nb); }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q4k<B, R, NW, true, true>(j, lds, e, d);
     }
 };
@@ -912,8 +929,8 @@ struct EngQ6K {
     static constexpr bool ONE_ROW_TILES = true;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 3;
     static __host__ __device__ int rows_per_pass(int) { return 1; }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q6k<B, R, NW, false>(j, lds, e, d);
     }
 };
@@ -923,8 +940,8 @@ struct EngQ6KShort {
     static constexpr bool ONE_ROW_TILES = false;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 8;
     static __host__ __device__ int rows_per_pass(int nb) { return q4k_rows_per_pass(nb); }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q6k<B, R, NW, true>(j, lds, e, d);
     }
 };
@@ -933,8 +950,8 @@ struct EngQ80 {
     static constexpr bool ONE_ROW_TILES = false;   // one row per wave tile at one activation row
     static constexpr int WGS_PER_CU_ONE_ROW = 8;
     static __host__ __device__ int rows_per_pass(int) { return 1; }
-    template <int B, int R, int NW, class Epi, class Done = NoTileHook>
-    static __device__ __forceinline__ void run(const RowJob<NW>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
+    template <int B, int R, int NW, class Epi, class Done = NoTileHook, typename V>
+    static __device__ __forceinline__ void run(const RowJob<NW, V>& j, uint8_t* lds, Epi&& e, Done&& d = Done()) {
         rows_q80<B, R, NW>(j, lds, e, d);
     }
 };

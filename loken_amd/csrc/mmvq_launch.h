@@ -26,7 +26,7 @@ struct MultiArgs {
 
 template <class E, int B, int R, typename T>
 __global__ __launch_bounds__(WG) void mmvq_kernel(MultiArgs m, const uint8_t* __restrict__ vy, int nb,
-                                                  int stride_col_y, int stride_col_dst, int act_stride_f32) {
+                                                  int stride_col_y, int stride_col_dst, int act_stride_f32, int half_rows) {
     extern __shared__ __align__(16) uint8_t lds[];
     // Which matrix this workgroup serves. Every field is read at a fixed index and picked with a
     // mask, so the kernel arguments the first loads need arrive in one round of scalar loads
@@ -67,8 +67,9 @@ __global__ __launch_bounds__(WG) void mmvq_kernel(MultiArgs m, const uint8_t* __
     T* dst = (T*)(uint8_t*)to_gbytes((uint64_t)dst_bits);
     const float* bias = (const float*)to_gbytes((uint64_t)bias_bits);
     const int n = (int)n_bits, wg_first = (int)first_bits, wg_end = (int)end_bits;
-    RowJob<1> job{{vx}, vy, nb, n, stride_col_y, (wg_end - wg_first) * WAVES, ((int)blockIdx.x - wg_first) * WAVES,
-                  act_stride_f32};
+    RowJob<1, T> job{{vx}, vy, nb, n, stride_col_y, (wg_end - wg_first) * WAVES, ((int)blockIdx.x - wg_first) * WAVES,
+                     act_stride_f32};
+    job.half_rows = half_rows;
     E::template run<B, R, 1>(job, lds, [&](int row, int c, const float* tot) {
         float v = tot[0];
         if (bias) v += bias[row];
@@ -213,7 +214,8 @@ struct MmvqCall {
     MultiArgs m;
     const uint8_t* vy;
     int nb, stride_col_y, stride_col_dst;
-    int act_stride_f32;  // non-zero: vy is f32 rows, quantized in the kernel
+    int act_stride_f32;  // non-zero: vy is rows of values, quantized in the kernel: f32, or
+    int half_rows;       // (at most two of them) of the outputs' half type
     hipStream_t stream;
 };
 
@@ -242,7 +244,7 @@ static int launch_plain_r(MmvqCall& a) {
     }
     for (int i = a.m.count; i < MAX_MULTI; ++i) a.m.wg_begin[i + 1] = a.m.wg_begin[i];
     hipLaunchKernelGGL(kernel, dim3(a.m.wg_begin[a.m.count]), dim3(WG), lds_bytes, a.stream, a.m, a.vy, a.nb,
-                       a.stride_col_y, a.stride_col_dst, a.act_stride_f32);
+                       a.stride_col_y, a.stride_col_dst, a.act_stride_f32, a.half_rows);
     return lk_launch_status();
 }
 

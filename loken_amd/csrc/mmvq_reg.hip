@@ -82,19 +82,18 @@ static __device__ __forceinline__ float row_share(const RowFrag& f, const Slice&
 // unit = 4 * slot + p: which 72 bytes of the Q8_1 row (64 bytes of the LDS image) are the lane's.
 // B activation rows, `act_stride` bytes apart, into B slices (the f32 form: B images of LDS_BYTES).
 // ACT: Q8_1 rows, or rows of values, quantized here: half rows stay two bytes a value in registers until the weights are under way.
-constexpr int ACT_Q81 = 0, ACT_VALUES = 1, ACT_HALF = 2, ACT_BF16 = 3;
 template <int ACT>
 static __device__ __forceinline__ float4 values_of(const float4& v) { return v; }
 template <int ACT>
 static __device__ __forceinline__ float4 values_of(const uint2& v) {
-    if (ACT == ACT_HALF) return Load4<__half>::at((const __half*)&v);
+    if (ACT == LK_REG_F16) return Load4<__half>::at((const __half*)&v);
     return Load4<__hip_bfloat16>::at((const __hip_bfloat16*)&v);
 }
 template <int ACT, int B, class First>
 static __device__ __forceinline__ void slice_load(Slice (&s)[B], gbytes_t act, size_t act_stride, int nb, int unit, bool valid,
                                                   uint8_t* lds, First&& first_loads) {
 #pragma clang fp contract(off)
-    if constexpr (ACT == ACT_Q81) {
+    if constexpr (ACT == LK_REG_Q8_1) {
         // (cast back from the global address space: the compiler keeps track of where it came from)
         uint32_t head0[B], head1[B];
 #pragma unroll
@@ -115,7 +114,7 @@ static __device__ __forceinline__ void slice_load(Slice (&s)[B], gbytes_t act, s
         return;
     }
     // row of values: item t is four of them, eight consecutive items (lanes) are one Q8_1 block
-    using quad = typename std::conditional<ACT == ACT_VALUES, float4, uint2>::type;
+    using quad = typename std::conditional<ACT == LK_REG_F32, float4, uint2>::type;
     const int items = nb * 64;
     quad v[B][2];
 #pragma unroll
@@ -193,7 +192,7 @@ struct Geo {
 template <int R, int RP, int ACT, int B>
 __global__ __launch_bounds__(RT) void q4k_reg_kernel(RegArgs a, const uint8_t* __restrict__ act, int nb, int dst_type,
                                                      int waves, int act_stride, int dst_stride) {
-    __shared__ __align__(16) uint8_t lds[ACT != ACT_Q81 ? B * LDS_BYTES : 16];
+    __shared__ __align__(16) uint8_t lds[ACT != LK_REG_Q8_1 ? B * LDS_BYTES : 16];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int TR = R * RP;
     uint32_t flip = 0x80808080u;
@@ -337,7 +336,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
         // tiles of RP rows, wave-strided
         const int tiles = (n + RP - 1) / RP, step = (int)gridDim.x * waves;
         int t = (int)blockIdx.x * waves + wave;
-        slice_load<ACT_F32 ? ACT_VALUES : ACT_Q81, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds,
+        slice_load<ACT_F32 ? LK_REG_F32 : LK_REG_Q8_1, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds,
                                [&] { load(min(t, tiles - 1) * RP + g.rp); });
         while (t < tiles) {
             const int row = t * RP + g.rp;
@@ -364,7 +363,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
         row_load(bg[slot], wg + at, g.hdr_off, g.qs_off);
         row_load(bu[slot], wu + at, g.hdr_off, g.qs_off);
     };
-    slice_load<ACT_F32 ? ACT_VALUES : ACT_Q81, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds, [&] {
+    slice_load<ACT_F32 ? LK_REG_F32 : LK_REG_Q8_1, B>(s, to_gbytes(act), (size_t)act_stride, nb, g.unit, g.valid, lds, [&] {
 #pragma unroll
         for (int i = 0; i < D; ++i) load_pass(i, min(b, blocks - 1), i);
     });
@@ -495,14 +494,14 @@ static int launch_multi(const LkRegMulti& m, const void* act, int act_form, int 
         }
         a.tile_end[i] = total;
     }
-    const Shape sh = shape_for(act_form != ACT_Q81);
+    const Shape sh = shape_for(act_form != LK_REG_Q8_1);
     const int need = (total + sh.waves - 1) / sh.waves;
     const int forced_grid = lk_tune_env("LK_TUNE_REG_GRID");
     const dim3 grid(forced_grid > 0 ? (forced_grid < need ? forced_grid : need) : need < sh.cap ? need : sh.cap), block(sh.waves * 64);
-    auto kernel = act_form == ACT_Q81      ? q4k_reg_kernel<R, RP, ACT_Q81, B>
-                  : act_form == ACT_VALUES ? q4k_reg_kernel<R, RP, ACT_VALUES, B>
-                  : act_form == ACT_HALF   ? q4k_reg_kernel<R, RP, ACT_HALF, B>
-                                           : q4k_reg_kernel<R, RP, ACT_BF16, B>;
+    auto kernel = act_form == LK_REG_Q8_1      ? q4k_reg_kernel<R, RP, LK_REG_Q8_1, B>
+                  : act_form == LK_REG_F32 ? q4k_reg_kernel<R, RP, LK_REG_F32, B>
+                  : act_form == LK_REG_F16   ? q4k_reg_kernel<R, RP, LK_REG_F16, B>
+                                           : q4k_reg_kernel<R, RP, LK_REG_BF16, B>;
     hipLaunchKernelGGL(kernel, grid, block, 0, s, a, (const uint8_t*)act, nb, dst_type, sh.waves, act_stride, dst_stride);
     return lk_launch_status();
 }
@@ -552,10 +551,10 @@ static int multi_rows(const LkRegMulti& m, const void* act, int act_form, int nb
     int rows = 0;
     for (int i = 0; i < m.count; ++i) rows += m.n[i];
     const int forced = lk_tune_env("LK_TUNE_REG_R");
-    const Shape sh = shape_for(act_form != ACT_Q81);
+    const Shape sh = shape_for(act_form != LK_REG_Q8_1);
     // (from f32 rows the bound is one workgroup per CU: q + k + v of a Llama-sized layer, 6144 rows, is
     // faster as single rows over two workgroups per CU, 5.7 against 6.1 us; o, 4096 rows, as pairs)
-    const int waves_at_once = (act_form != ACT_Q81 ? lk_device().cus : sh.cap) * sh.waves;
+    const int waves_at_once = (act_form != LK_REG_Q8_1 ? lk_device().cus : sh.cap) * sh.waves;
     // (rows short enough to go side by side already give a wave two or four rows per pass: two such
     // tiles per wave measured slower, Qwen3-1.7B step 0.598 against 0.586 ms)
     const bool two = forced ? forced == 2 : rp == 1 && rows <= waves_at_once * 2;
@@ -568,26 +567,12 @@ static int multi_rows(const LkRegMulti& m, const void* act, int act_form, int nb
     }
 }
 
-int lk_q4k_reg_multi(const LkRegMulti& m, const void* act, int act_f32, int nb, int dst_type, int batch, int act_stride,
+int lk_q4k_reg_multi(const LkRegMulti& m, const void* act, int act_form, int nb, int dst_type, int batch, int act_stride,
                      int dst_stride, hipStream_t stream) {
     if (!lk_q4k_reg_serves(nb) || m.count < 1 || m.count > 4 || batch < 1 || batch > LK_REG_MAX_BATCH) return LK_ERR_ARG;
-    const int act_bytes = act_stride * (act_f32 ? (int)sizeof(float) : Q81_BYTES);
-    return batch == 1 ? multi_rows<1>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream)
-                      : multi_rows<2>(m, act, act_f32, nb, dst_type, act_bytes, dst_stride, stream);
-}
-
-int lk_q4k_half_linear(const void* w, const void* x, int type, void* out, int rows, int n, int k, hipStream_t stream) {
-    if (type != LK_TYPE_F16 && type != LK_TYPE_BF16) return -1;
-    if (rows < 1 || rows > LK_REG_MAX_BATCH || n < 1 || k % 256 != 0 || !lk_q4k_reg_serves(k / 256) || (uintptr_t)w % 16 != 0 ||
-        (uintptr_t)x % 8 != 0)
-        return -1;
-    LkRegMulti m{};
-    m.vx[0] = (const uint8_t*)w;
-    m.dst[0] = out;
-    m.n[0] = n;
-    m.count = 1;
-    const int form = type == LK_TYPE_F16 ? ACT_HALF : ACT_BF16;
-    return rows == 1 ? multi_rows<1>(m, x, form, k / 256, type, 2 * k, n, stream) : multi_rows<2>(m, x, form, k / 256, type, 2 * k, n, stream);
+    const int act_bytes = act_stride * (act_form == LK_REG_Q8_1 ? Q81_BYTES : act_form == LK_REG_F32 ? 4 : 2);
+    return batch == 1 ? multi_rows<1>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream)
+                      : multi_rows<2>(m, act, act_form, nb, dst_type, act_bytes, dst_stride, stream);
 }
 
 template <int RP>

@@ -390,14 +390,17 @@ def test_nine_to_sixteen_rows_of_plain_blocks(name, n, k, rows, expect):
     lin.close()
 
 
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k", "q8_0"])
 @pytest.mark.parametrize("half", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,n,k,shift,expect", [(1, 1, 256, 0, "matvec-fused"), (2, 7, 1024, 4, "matvec-fused"), (1, 301, 2048, 0, "matvec-fused"),
                                                    (2, 4099, 4096, 8, "matvec-fused"), (1, 9001, 3840, 0, "matvec-fused"), (2, 2050, 2048, 0, "matvec-fused"),
-                                                   (1, 64, 1024, 2, "matvec"), (2, 64, 4352, 0, "matvec")])
-def test_half_rows_quantized_in_the_launch_carry_the_quantizers_codes(rows, n, k, shift, expect, half):
-    # One launch over one or two half rows of Q4_K: the bits of quantizer and mat-vec, rows from any 8-byte boundary; rows off it,
+                                                   (1, 64, 1024, 2, "matvec"), (2, 70, 8192, 0, "matvec-fused"),
+                                                   (1, 70, 4352, 4, "matvec-fused"), (2, 64, 8448, 0, "matvec"),
+                                                   (2, 4096, 4352, 0, "matvec"), (1, 9637, 4352, 0, "matvec-fused"), (2, 2890, 4352, 0, "matvec-fused")])
+def test_half_rows_quantized_in_the_launch_carry_the_quantizers_codes(name, rows, n, k, shift, expect, half):
+    # One launch over one or two half rows: the bits of quantizer and mat-vec, rows from any 8-byte boundary; rows off it,
     # and longer ones, go on as two launches. Zeros, the largest codes, tiny values, infinities and NaN among them.
-    w = dev(synth.weight(lib.TYPE_Q4_K, n, k, seed=99, stream=1))
+    w = dev(synth.weight(DT[name], n, k, seed=99, stream=1))
     x = dev(synth.activation(rows, k, seed=99))
     x[0, :32] = 0
     x[0, 32:64] *= 1e-6
@@ -405,11 +408,11 @@ def test_half_rows_quantized_in_the_launch_carry_the_quantizers_codes(rows, n, k
     flat = torch.zeros(rows * k + shift, device="cuda", dtype=half)
     flat[shift:] = x.reshape(-1).to(half)
     x = flat[shift:].view(rows, k)
-    lin = Linear(lib.TYPE_Q4_K, w, n, k)
+    lin = Linear(DT[name], w, n, k)
     for _ in range(2):
         got = lin(x)
         assert lin.path == expect and got.dtype == half
-        want = ops.mmvq(lib.TYPE_Q4_K, w, ops.quantize_q8_1_rows(x.contiguous()), k, n, out_dtype=half)
+        want = ops.mmvq(DT[name], w, ops.quantize_q8_1_rows(x.contiguous()), k, n, out_dtype=half)
         assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
         x[0, 5], x[rows - 1, k - 1] = float("inf"), float("nan")
     lin.close()
