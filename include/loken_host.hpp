@@ -22,7 +22,7 @@ namespace loken {
 /* Which launchers a forward call went through. */
 enum class Path : int {
     None = 0,
-    MatVecFused = 1,   /* lk_mmvq_fused: f32 rows quantized inside the mat-vec launch */
+    MatVecFused = 1,   /* one or two rows quantized inside the mat-vec launch */
     MatVec = 2,        /* lk_quantize_q8_1 + lk_mmvq (slices of eight rows) */
     RowsOnMatrixUnit = 3, /* lk_quantize_q8_1 + lk_dense_q4k_rows / lk_dense_q5k_rows / lk_dense_q6k_rows */
     Tiled = 4,         /* launch_mmq_quantize_q8_1_* + launch_mmq_gguf_* */
