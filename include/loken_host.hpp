@@ -66,13 +66,16 @@ public:
 
     /* quantize_for_matvec (kernel_matmul.rs:695-748): x [rows, k] into `q81` the way forward quantizes it
      * for the mat-vec kernels, so that several weights over the same rows quantize them once. LK_OK and `a`
-     * filled, or LK_NOT_TAKEN where forward would not take those kernels for this row count (the
-     * reference's None): more rows than matvec_rows without `decode_order`, or a matrix whose few rows go
-     * to the matrix-unit rows kernels. */
+     * filled, or LK_NOT_TAKEN (the reference's None): without `decode_order` more than matvec_rows rows (Q4_0, Q4_1,
+     * Q5_0, Q5_1, Q2_K and Q3_K: 16 rows, or 9 over 48 Mi weights; IQ4_NL, MXFP4 and IQ4_XS: never), or 3 to 8 rows of a
+     * K-quant over a large matrix (Q4_K / Q5_K: n x rows of 57344, or 8192 at k <= 2048; Q6_K with k a multiple of 2048: n x k of
+     * 48 Mi, or 7 rows and n of 1024). */
     int quantize_for_matvec(const void* x, int x_type, int rows, void* q81, void* stream, QuantizedActivation* a,
                             bool decode_order = false) const;
     /* forward_quantized (kernel_matmul.rs:750-812): out [rows, n] in a.x_type, the bits forward gives on the
-     * rows `a` was made from. LK_NOT_TAKEN where forward would take another path. */
+     * rows `a` was made from, out of the same kernels (last_path: MatVec, RowsOnMatrixUnit or Tiled). LK_NOT_TAKEN as
+     * quantize_for_matvec. Where forward takes tiles and there is no scratch for them (a capture at a size not warmed up), the
+     * mat-vec kernels serve the call: the same integer dots, summed in another order. */
     int forward_quantized(const QuantizedActivation& a, void* out, void* stream, bool decode_order = false);
     /* forward_quantized_pair (kernel_matmul.rs:814-876): this weight and `other` over ONE f32-born activation
      * row in one launch, each output with the bits of its own forward_quantized. LK_NOT_TAKEN where the pair
@@ -84,7 +87,7 @@ public:
     int k() const { return k_; }
 
 private:
-    bool takes_matvec(int rows, bool decode_order) const;
+    bool takes_quantized(int rows, bool decode_order) const;
     int dtype_, n_, k_, device_;
     const void* blob_;
     Path last_path_ = Path::None;

@@ -137,6 +137,18 @@ static bool small_rows_kernel_pays(int dtype, int n, int k, int rows) {
     return k <= 2048 ? (long long)n * rows >= 8192 : weights * rows > (128ll << 20);
 }
 
+// Matrices whose 3 to 8 rows are refused as rows quantized beforehand, as they have been since the 16-row tiles took them over; the
+// smaller ones small_rows_kernel_pays names are served from Q8_1 rows too.
+static bool large_for_few_rows(int dtype, int n, int k, int rows) {
+    if (dtype == LK_TYPE_Q6_K) return k % 2048 == 0 && ((long long)n * k >= (48ll << 20) || (rows >= 7 && n >= 1024));
+    return (long long)n * rows >= (k <= 2048 ? 8192 : 57344);
+}
+
+// The K-quants' weights as the rows kernels take them.
+static bool fits_rows_kernel(int dtype, int k, const void* blob) {
+    return k % 256 == 0 && ((uintptr_t)blob & (dtype == LK_TYPE_Q6_K ? 1 : 15)) == 0;
+}
+
 QKernelMatMul::QKernelMatMul(int dtype, int n, int k, const void* blob, int device)
     : dtype_(dtype), n_(n), k_(k), device_(device), blob_(blob) {}
 
@@ -160,7 +172,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     // interleave their pairs (fast_mmvq.rs:15-32, kernel_matmul/mmq.rs:43-86)
 
     // --- mat-vec family: up to matvec_rows, or any count when every row must sum like a one-row call
-    const bool rows_kernel_fits = k_ % 256 == 0 && ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q6_K ? 1 : 15)) == 0;
+    const bool rows_kernel_fits = fits_rows_kernel(dtype_, k_, blob_);
     const bool to_rows_kernel = rows_kernel_fits && small_rows_kernel_pays(dtype_, n_, k_, rows);
     const bool few_to_tiles = few_rows_to_tiles(dtype_, n_, k_, rows, blob_);
     const bool to_nibble_tiles = !decode_order && (few_to_tiles || nibble_tiles_pay(dtype_, n_, k_, rows)) &&
@@ -207,7 +219,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
             if (int r = lk_quantize_q8_1(x, x_type, act, k_, k_, rows, stream)) return r;
             // (rows too long for the kernels' scale tables in LDS launch nothing, and the call goes on to the
             // mat-vec or the tiled matmul below)
-            rc = lk_rows_linear(dtype_, blob_, act, out, x_type, rows, n_, k_, stream);
+            rc = lk_rows_linear(dtype_, blob_, act, blocks, out, x_type, rows, n_, k_, stream);
         }
         if (rc == LK_OK) {
             last_path_ = Path::RowsOnMatrixUnit;
@@ -246,18 +258,16 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     return LK_OK;
 }
 
-// takes_matvec of the reference (kernel_matmul.rs:1069-1075) with this mirror's own exceptions: the
-// K-quants' few rows go to the 16-row tiles where that pays, nine rows and more of Q8_0 and Q4_0 to the f16 tiles, and the formats with tiles leave the
-// mat-vec launches from nibble_tiles_pay's row counts.
-bool QKernelMatMul::takes_matvec(int rows, bool decode_order) const {
+// takes_matvec of the reference (kernel_matmul.rs:1069-1075), for rows quantized beforehand: mat-vec counts of rows, but for the K-quants'
+// 3 to 8 rows over a large matrix (large_for_few_rows) and the formats with tiles from nibble_tiles_pay's row counts. Which launch serves the call
+// is forward's choice all the same (forward_quantized). Three products over one activation, forward three times / quantized once (us): Q4_K 4096 x 4096
+// at 4 / 8 rows 18.9, 18.8 / 17.1, 17.2; Q6_K 2048 x 3072 at 8 rows 17.3 / 15.8; Q8_0 4096 x 8192 at 16 81 / 83, 14336 x 4096 at 9 105 / 107.
+bool QKernelMatMul::takes_quantized(int rows, bool decode_order) const {
     if (!blob_ || rows < 1) return false;
     if (decode_order && rows > 1) return true;
-    const bool plain = matvec_only(dtype_);
-    if (few_rows_to_tiles(dtype_, n_, k_, rows, blob_)) return false;
-    if (plain) return !nibble_tiles_pay(dtype_, n_, k_, rows) || rows <= matvec_rows(dtype_, k_);
+    if (matvec_only(dtype_)) return !nibble_tiles_pay(dtype_, n_, k_, rows) || rows <= matvec_rows(dtype_, k_);
     if (rows > matvec_rows(dtype_, k_)) return false;
-    const bool rows_kernel_fits = k_ % 256 == 0 && ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q6_K ? 1 : 15)) == 0;
-    return !(rows_kernel_fits && small_rows_kernel_pays(dtype_, n_, k_, rows));
+    return !(fits_rows_kernel(dtype_, k_, blob_) && small_rows_kernel_pays(dtype_, n_, k_, rows) && large_for_few_rows(dtype_, n_, k_, rows));
 }
 
 size_t QKernelMatMul::quantized_bytes(int k, int rows) {
@@ -273,7 +283,7 @@ int QKernelMatMul::quantize_for_matvec(const void* x, int x_type, int rows, void
         (void)hipGetLastError();
         return LK_ERR_ARG;
     }
-    if (!takes_matvec(rows, decode_order)) return LK_NOT_TAKEN;
+    if (!takes_quantized(rows, decode_order)) return LK_NOT_TAKEN;
     const int k_padded = (int)pad_to((size_t)k_, 512);
     if (int rc = lk_quantize_q8_1(x, x_type, q81, k_, k_padded, rows, stream)) return rc;
     a->q81 = q81;
@@ -287,13 +297,30 @@ int QKernelMatMul::quantize_for_matvec(const void* x, int x_type, int rows, void
 int QKernelMatMul::forward_quantized(const QuantizedActivation& a, void* out, void* stream, bool decode_order) {
     last_path_ = Path::None;
     if (!a.q81 || !out) return LK_ERR_ARG;
-    if (a.k != k_ || a.device != device_ || !takes_matvec(a.rows, decode_order)) return LK_NOT_TAKEN;
+    if (a.k != k_ || a.device != device_ || !takes_quantized(a.rows, decode_order)) return LK_NOT_TAKEN;
     int current = -1;
     if (hipGetDevice(&current) != hipSuccess || current != device_) {
         (void)hipGetLastError();
         return LK_ERR_ARG;
     }
     const int blocks = (int)pad_to((size_t)k_, 512) / 32;
+    // The launches forward takes at this row count, with its bits; where they decline, or the tiles have no scratch, the mat-vec launches
+    const bool one_order = decode_order && a.rows > 1;
+    if (!one_order && fits_rows_kernel(dtype_, k_, blob_) && small_rows_kernel_pays(dtype_, n_, k_, a.rows)) {
+        const int rc = lk_rows_linear(dtype_, blob_, a.q81, blocks, out, a.x_type, a.rows, n_, k_, (hipStream_t)stream);
+        if (rc == LK_OK) last_path_ = Path::RowsOnMatrixUnit;
+        if (rc != LK_ERR_ARG) return rc;
+    }
+    if (!one_order && few_rows_to_tiles(dtype_, n_, k_, a.rows, blob_)) {
+        LkScratch scratch((hipStream_t)stream);
+        void* fixup = scratch.get(LK_SCRATCH_FIXUP, FIXUP_BYTES);
+        const int width = fixup ? lk_mmq_tiles_linear_q8_1(dtype_, fixup, blob_, a.q81, blocks, a.x_type, out, k_, n_, a.rows, (hipStream_t)stream) : -1;
+        if (width == 0) return LK_ERR_ARG;
+        if (width > 0) {
+            last_path_ = Path::Tiled;
+            return LK_OK;
+        }
+    }
     for (int r0 = 0; r0 < a.rows; r0 += 8) {
         const int b = a.rows - r0 < 8 ? a.rows - r0 : 8;
         const int rc = lk_mmvq(dtype_, blob_, (const uint8_t*)a.q81 + (size_t)r0 * blocks * Q81_BLOCK,
@@ -310,7 +337,7 @@ int QKernelMatMul::forward_quantized_pair(QKernelMatMul& other, const QuantizedA
     last_path_ = other.last_path_ = Path::None;
     if (!a.q81 || !out0 || !out1) return LK_ERR_ARG;
     if (a.k != k_ || other.k_ != k_ || a.rows != 1 || a.x_type != LK_TYPE_F32 || dtype_ != other.dtype_ ||
-        device_ != other.device_ || a.device != device_ || !takes_matvec(1, false) || !other.takes_matvec(1, false))
+        device_ != other.device_ || a.device != device_ || !takes_quantized(1, false) || !other.takes_quantized(1, false))
         return LK_NOT_TAKEN;
     int current = -1;
     if (hipGetDevice(&current) != hipSuccess || current != device_) {

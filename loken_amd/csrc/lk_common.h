@@ -263,11 +263,11 @@ static __device__ __forceinline__ void lk_store_as(float* dst, size_t at, float 
     else ((__hip_bfloat16*)dst)[at] = __float2bfloat16(v);
 }
 // The dense launches of the matrix unit with a destination of f32, f16 or bf16 elements, for the host linear: a few rows
-// (rows_mfma.hip; Q4_K, Q5_K, Q6_K) and tiles (mmq.hip). lk_rows_linear: LK_* status; lk_mmq_linear: the token-tile
+// (rows_mfma.hip; Q4_K, Q5_K, Q6_K) and tiles (mmq.hip). lk_rows_linear (stride_y: Q8_1 blocks between rows): LK_* status; lk_mmq_linear: the token-tile
 // width launched, 0 when nothing ran.
 // lk_rows_linear_direct: the same straight from rows of `x_type` (results in it too), -1 where no launch takes them.
 int lk_rows_linear_direct(int wtype, const void* w, const void* x, void* out, int x_type, int rows, int n, int k, hipStream_t stream);
-int lk_rows_linear(int wtype, const void* w, const void* q8_1, void* out, int out_type, int rows, int n, int k, hipStream_t stream);
+int lk_rows_linear(int wtype, const void* w, const void* q8_1, int stride_y, void* out, int out_type, int rows, int n, int k, hipStream_t stream);
 int lk_mmq_linear(int wtype, void* fixup, const void* w, const void* y, void* out, int out_type, int k, int n, int rows, int64_t row_blocks,
                   hipStream_t stream);
 // Q4_K / Q6_K x any number of Q8_1 rows on the matrix unit (rows_mfma.hip, rows_mfma_q6k.hip); LK_* status.

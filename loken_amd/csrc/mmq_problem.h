@@ -155,6 +155,9 @@ int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fix
 bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows);
 // The same for `rows` rows of x, k values each, results in x's type: nothing between x and the operands.
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s);
+// The same from the rows' Q8_1 blocks, `stride` blocks between rows, with the same bits.
+int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
+                             hipStream_t s);
 // The expert-batched product over workspace records, same returns as the dense one.
 int lk_mmq_tiles_moe_records(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,
                              int64_t stride_expert, int n_experts, int64_t ncols_max, hipStream_t s);

@@ -8,17 +8,12 @@
 
 namespace {
 
-// Workspace records -> operands. grid (blocks, rows / 32), 256 threads: eight threads a row, a sub-block each.
-__global__ __launch_bounds__(256) void operands_from_records_kernel(const uint8_t* __restrict__ y, LkTokenOperands ops, int64_t rec_rows,
-                                                                    int row0, int rows) {
-    const int kb = blockIdx.x, s = threadIdx.x & 7;
-    const int r = blockIdx.y * 32 + (threadIdx.x >> 3);
-    if (r >= rows) return;
-    const uint8_t* rec = y + ((int64_t)kb * rec_rows + row0 + r) * MMQ_REC_BYTES;
-    uint8_t* to = ops.codes + ((int64_t)kb * ops.rows + r) * LK_OPERAND_CODES + 64 * s;
+// A sub-block's 32 codes as its four atoms; Vec: sixteen bytes as `codes` is aligned.
+template <class Vec>
+static __device__ __forceinline__ void operand_atoms(const uint8_t* codes, uint8_t* to) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const uint4 c = *(const uint4*)(rec + 32 * s + 16 * h);
+        const Vec c = *(const Vec*)(codes + 16 * h);
         uint4 lo, hi;
         operand_codes(c.x, lo.x, lo.y);
         operand_codes(c.y, lo.z, lo.w);
@@ -27,8 +22,32 @@ __global__ __launch_bounds__(256) void operands_from_records_kernel(const uint8_
         *(uint4*)(to + 16 * h) = lo;
         *(uint4*)(to + 32 + 16 * h) = hi;
     }
+}
+
+// Workspace records -> operands. grid (blocks, rows / 32), 256 threads: eight threads a row, a sub-block each.
+__global__ __launch_bounds__(256) void operands_from_records_kernel(const uint8_t* __restrict__ y, LkTokenOperands ops, int64_t rec_rows,
+                                                                    int row0, int rows) {
+    const int kb = blockIdx.x, s = threadIdx.x & 7;
+    const int r = blockIdx.y * 32 + (threadIdx.x >> 3);
+    if (r >= rows) return;
+    const uint8_t* rec = y + ((int64_t)kb * rec_rows + row0 + r) * MMQ_REC_BYTES;
+    operand_atoms<uint4>(rec + 32 * s, ops.codes + ((int64_t)kb * ops.rows + r) * LK_OPERAND_CODES + 64 * s);
     operand_scales(ops.tabs + ((int64_t)kb * ops.rows + r) * LK_OPERAND_TAB, s, f16_bits_to_f32(*(const uint16_t*)(rec + 256 + 2 * s)),
                    (int)*(const int16_t*)(rec + 272 + 2 * s));
+}
+
+// Q8_1 rows, `stride` blocks apart -> operands, on the same grid: the codes and scales the quantizer below makes of the rows
+// they came from, so the products carry its bits. A few rows a call: a launch's time, whatever the bytes.
+__global__ __launch_bounds__(256) void operands_from_q8_1_kernel(const uint8_t* __restrict__ y, LkTokenOperands ops, int stride, int rows) {
+    const int kb = blockIdx.x, s = threadIdx.x & 7;
+    const int r = blockIdx.y * 32 + (threadIdx.x >> 3);
+    if (r >= rows) return;
+    const uint8_t* block = y + ((int64_t)r * stride + 8 * kb + s) * Q81_BYTES;
+    operand_atoms<uint4_a4>(block + 4, ops.codes + ((int64_t)kb * ops.rows + r) * LK_OPERAND_CODES + 64 * s);
+    int sum = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum = __builtin_amdgcn_sdot4(*(const int*)(block + 4 + 4 * i), 0x01010101, sum, false);
+    operand_scales(ops.tabs + ((int64_t)kb * ops.rows + r) * LK_OPERAND_TAB, s, f16_bits_to_f32(*(const uint16_t*)block), sum);
 }
 
 // Rows of x -> operands, the quantizer and the expansion in one pass: grid (rows, k / 1024), four values a thread. Bound by
@@ -161,6 +180,16 @@ int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, in
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
     return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
         (void)lk_operands_quantize((const uint8_t*)x + (int64_t)m0 * k * (type == LK_TYPE_F32 ? 4 : 2), type, ops, k, count, s);
+    });
+}
+
+int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
+                             hipStream_t s) {
+    if (!lk_mmq_tiles_take(wtype, n, rows) || k % 256 != 0) return -1;
+    const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
+    return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
+        hipLaunchKernelGGL(operands_from_q8_1_kernel, dim3((unsigned)pb.nb, (unsigned)((count + 31) / 32)), dim3(256), 0, s,
+                           (const uint8_t*)q8_1 + (int64_t)m0 * stride * Q81_BYTES, ops, stride, count);
     });
 }
 

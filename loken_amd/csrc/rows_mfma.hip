@@ -825,10 +825,10 @@ int lk_q4k_rows_mfma(const void* w, const void* q8_1, float* output, int size_m,
     return rows_plain(w, q8_1, output, size_m, size_n, size_k, stride_y, ldd, false, stream);
 }
 
-int lk_rows_linear(int wtype, const void* w, const void* q8_1, void* out, int out_type, int rows, int n, int k, hipStream_t stream) {
-    if (wtype == LK_TYPE_Q6_K) return lk_q6k_rows_mfma(w, q8_1, (float*)out, rows, n, k, k / 32, n, stream, out_type);
+int lk_rows_linear(int wtype, const void* w, const void* q8_1, int stride_y, void* out, int out_type, int rows, int n, int k, hipStream_t stream) {
+    if (wtype == LK_TYPE_Q6_K) return lk_q6k_rows_mfma(w, q8_1, (float*)out, rows, n, k, stride_y, n, stream, out_type);
     if (wtype != LK_TYPE_Q4_K && wtype != LK_TYPE_Q5_K) return LK_ERR_TYPE;
-    return rows_plain(w, q8_1, (float*)out, rows, n, k, k / 32, n, wtype == LK_TYPE_Q5_K, stream, out_type);
+    return rows_plain(w, q8_1, (float*)out, rows, n, k, stride_y, n, wtype == LK_TYPE_Q5_K, stream, out_type);
 }
 
 int lk_rows_linear_direct(int wtype, const void* w, const void* x, void* out, int x_type, int rows, int n, int k, hipStream_t stream) {

@@ -385,8 +385,55 @@ def test_nine_to_sixteen_rows_of_plain_blocks(name, n, k, rows, expect):
     q81 = torch.empty(lib.load().lkh_quantized_activation_bytes(k, rows), dtype=torch.uint8, device="cuda")
     lin = Linear(DT[name], dev(synth.weight(DT[name], 8, k, seed=98).reshape(8, -1).repeat((n + 7) // 8, axis=0)[:n]), n, k)
     x = dev(synth.activation(rows, k, seed=98))
-    status = lib.load().lkh_qkernel_matmul_quantize_for_matvec(lin.h, x.data_ptr(), X_TYPES[x.dtype], rows, q81.data_ptr(), torch.cuda.current_stream().cuda_stream, 0)
-    assert (status == 0) == (expect == "matvec")   # follows forward
+    s = torch.cuda.current_stream().cuda_stream
+    # rows quantized beforehand are served whichever launch forward takes, with its bits
+    assert lib.load().lkh_qkernel_matmul_quantize_for_matvec(lin.h, x.data_ptr(), X_TYPES[x.dtype], rows, q81.data_ptr(), s, 0) == 0
+    out = torch.empty((rows, n), device="cuda")
+    assert lib.load().lkh_qkernel_matmul_forward_quantized(lin.h, q81.data_ptr(), X_TYPES[x.dtype], rows, out.data_ptr(), s, 0) == 0
+    assert lin.path == expect and torch.equal(out, lin(x))
+    lin.close()
+
+
+# three to eight rows of the K-quants on the rows kernels (rows whose padded length is more than their own among them), nine to
+# sixteen of Q8_0 and Q4_0 on the tiles
+@pytest.mark.parametrize("xt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name,rows,n,k,expect", [
+    ("q4_k", 3, 2100, 1280, "rows-on-matrix-unit"), ("q4_k", 8, 520, 2048, "rows-on-matrix-unit"), ("q5_k", 7, 1100, 4096, "rows-on-matrix-unit"),
+    ("q6_k", 5, 2050, 2048, "rows-on-matrix-unit"), ("q6_k", 8, 601, 1280, "rows-on-matrix-unit"), ("q6_k", 3, 4099, 2816, "rows-on-matrix-unit"),
+    ("q8_0", 14, 513, 4352, "tiled"), ("q8_0", 16, 1030, 8192, "tiled"), ("q4_0", 9, 512, 256, "tiled"), ("q4_0", 15, 645, 1280, "tiled")])
+def test_rows_quantized_beforehand_are_served_by_the_launches_of_forward(name, rows, n, k, expect, xt):
+    l, s = lib.load(), torch.cuda.current_stream().cuda_stream
+    w = synth.weight(DT[name], n, k, seed=95, stream=1)
+    lin = Linear(DT[name], dev(w), n, k)
+    q81 = torch.empty(l.lkh_quantized_activation_bytes(k, rows), dtype=torch.uint8, device="cuda")
+    x = dev(synth.activation(rows, k, seed=95)).to(xt)
+    x[0, :64] = 0
+    x[1] *= 1e-6
+    for bad in (False, True):
+        if bad:
+            x[0, 5], x[rows - 1, k - 1] = float("inf"), float("nan")
+        want = lin(x)
+        assert lin.path == expect
+        out = torch.empty((rows, n), dtype=xt, device="cuda")
+        assert l.lkh_qkernel_matmul_quantize_for_matvec(lin.h, x.data_ptr(), X_TYPES[xt], rows, q81.data_ptr(), s, 0) == 0
+        assert l.lkh_qkernel_matmul_forward_quantized(lin.h, q81.data_ptr(), X_TYPES[xt], rows, out.data_ptr(), s, 0) == 0
+        assert lin.path == expect and torch.equal(torch.nan_to_num(out), torch.nan_to_num(want))
+        if not bad:
+            pick = np.arange(0, n, 7)
+            eps = 0.0 if xt == torch.float32 else 2.0 ** -8   # one rounding to the narrow type
+            assert close(out.float().cpu().numpy()[:, pick], oracle.ob_matmul(DT[name], x.float().cpu().numpy(), w[pick], len(pick)), rtol=1e-3 + eps)
+    lin.close()
+
+
+@pytest.mark.parametrize("name,rows,n,k", [("q4_k", 3, 4096, 2048), ("q5_k", 4, 14336, 4096), ("q6_k", 7, 1024, 2048), ("q6_k", 3, 4096, 14336),
+                                           ("q8_0", 17, 513, 4096), ("q4_0", 16, 645, 1024)])
+def test_large_matrices_and_tiled_row_counts_refuse_rows_quantized_beforehand(name, rows, n, k):
+    l, s = lib.load(), torch.cuda.current_stream().cuda_stream
+    lin = Linear(DT[name], torch.zeros(1 << 26, dtype=torch.uint8, device="cuda"), n, k)
+    q81 = torch.zeros(l.lkh_quantized_activation_bytes(k, rows), dtype=torch.uint8, device="cuda")
+    x, out = torch.zeros((rows, k), device="cuda"), torch.zeros((rows, n), device="cuda")
+    assert l.lkh_qkernel_matmul_quantize_for_matvec(lin.h, x.data_ptr(), lib.TYPE_F32, rows, q81.data_ptr(), s, 0) == lib.LK_NOT_TAKEN
+    assert l.lkh_qkernel_matmul_forward_quantized(lin.h, q81.data_ptr(), lib.TYPE_F32, rows, out.data_ptr(), s, 0) == lib.LK_NOT_TAKEN
     lin.close()
 
 
