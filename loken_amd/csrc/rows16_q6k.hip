@@ -454,8 +454,10 @@ int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, in
     // workgroup per tile leaves half the CUs idle (2048 x 14336 12.9 us against 16.3), or a matrix small enough for its second reading to come
     // from L2 at no cost (8192 x 2048 8.8 against 9.5; 8192 x 4096, 27.5 MB, 12.2 against 11.1 and stays with eight). (Sets: below.)
     const size_t weight_bytes = (size_t)size_n * a.nb * Q6K_BYTES;
-    if (size_m <= 8)
-        return 2 * n_tiles <= lk_device().cus || weight_bytes <= ((size_t)22 << 20) ? launch<4>(a, stream, 2) : launch<8>(a, stream);
+    if (size_m <= 8) {
+        const int rc = 2 * n_tiles <= lk_device().cus || weight_bytes <= ((size_t)22 << 20) ? -1 : launch<8>(a, stream);
+        return rc != -1 ? rc : launch<4>(a, stream, 2);   // (eight rows too long for LDS: the sums four or fewer of them have)
+    }
     // 9..32 rows. Sixteen at once when their codes fit LDS and the row tiles are several to the CU; else the
     // rows in sets of eight, a set per workgroup (grid.y), in one launch: rows too long for sixteen in LDS (k =
     // 14336: 229 KB), up to two tiles to the CU, where twice the workgroups with half the staging each

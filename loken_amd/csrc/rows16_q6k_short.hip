@@ -252,7 +252,8 @@ int launch(const Args& a, hipStream_t stream) {
     return lk_launch_status();
 }
 
-// Whether the short launch takes the call, and the rows of a set.
+// Whether the short launch takes the call, and the rows of a set. By the matrix and the class of row counts alone (up to 8, 16, 32, 48,
+// 64): its sums are of another order than the other launches', and a row carries the same bits whatever rides with it in its class.
 int set_rows(int size_m, int size_n, int size_k) {
     // One workgroup fits a CU (registers), and a second round of them costs what the first did, so the line is the number of
     // workgroups. Eight rows to a set where that is one round, sixteen otherwise. Measured in a graph, us, the granules
@@ -269,8 +270,10 @@ int set_rows(int size_m, int size_n, int size_k) {
     // 10000 x 5120 at 8 / 16 / 32 25.3, 31.6, 36.7 / 19.9, 24.4, 41; 16384 x 3072 at 8 / 16 17.1, 20.2 / 17.9, 20.9; 3000 x 5120 at 32 / 48 20.0, 20.2 / 16.1, 24.1
     const int nb = size_k / 256, tiles = (size_n + TILE - 1) / TILE, cus = lk_device().cus;
     const bool granules = nb % 8 == 0, held = granules && tiles <= cus && (size_t)size_n * nb * Q6K_BYTES <= (64u << 20);
-    if (granules && size_m <= 8 && nb >= 32 && (2 * tiles <= cus || (size_m <= 4 && nb >= 48))) return 0;
-    if (granules && size_m <= 4 && nb > 8 && tiles > cus) return 0;   // (6144 x 6144 at 3 rows 12.6 / 15.0)
+    // More than a tile to the CU of rows longer than 4096 values stay too: 3 / 5 / 8 rows 5120 x 8192 15.4, 18.2, 18.7 / 19.3, 19.6, 20.3; 4608 x
+    // 14336 21.0, 24.5, 25.7 / 27.4, 27.9, 28.1; 6144 x 10240 23.1, 22.6, 23.2 / 23.0, 23.3, 23.6; 6144 x 6144 13.0, 15.7, 16.6 / 15.5, 15.6, 15.8
+    // (at 4096 values 6144 x 4096 11.3, 12.5, 13.0 / 12.3, 12.4, 12.5, and one launch with the quantizer in it).
+    if (granules && size_m <= 8 && (2 * tiles <= cus ? nb >= 32 : tiles > cus && nb > 16)) return 0;
     const int eights = (size_m + 7) / 8, sixteens = (size_m + 15) / 16;
     const int64_t most = size_m <= 16 ? (granules ? 3 * cus / 2 : 3 * cus) : size_m > 32 ? 2 * cus : held && nb < 32 ? cus : granules ? 2 * cus : 3 * cus;
     const bool by_eight = size_m <= 8 || (int64_t)tiles * eights <= cus;

@@ -72,6 +72,19 @@ def test_a_row_does_not_depend_on_its_company():
     assert (sixteen - full[8:24]).abs().max().item() <= 2e-6 * scale
 
 
+# matrices on either side of every choice between the Q6_K launches: row tiles up to half the CUs, up to the CUs and more, rows of
+# whole granules and others, rows so long that eight of them do not fit LDS
+@pytest.mark.parametrize("n,k", [(70, 256), (1030, 8192), (700, 2816), (2064, 12288), (4100, 4096), (4112, 6144), (4112, 16384), (6160, 2304)])
+def test_a_q6k_row_does_not_depend_on_its_company(n, k):
+    # up to 8, 16, 32, 48, 64 rows or more in all: within a class the launch is chosen by the matrix alone
+    w = dev(synth.weight(lib.TYPE_Q6_K, 64, k, seed=62, stream=5).reshape(64, -1).repeat((n + 63) // 64, axis=0)[:n])
+    x = dev(synth.activation(80, k, seed=62))
+    for most, counts in ((8, (1, 3, 4, 5, 7)), (16, (9, 12)), (32, (17, 25)), (48, (33, 40)), (64, (49, 57)), (80, (65,))):
+        full = ops.dense_q6k_rows(w, x[:most], n)
+        for m in counts:
+            assert torch.equal(ops.dense_q6k_rows(w, x[most - m:most].contiguous(), n), full[most - m:]), (most, m)
+
+
 def test_full_gate_shape_against_matvec_and_sampled_oracle():
     m, k, n = 16, 4096, 14336
     w = synth.weight(Q4K, n, k, seed=0, stream=30)
