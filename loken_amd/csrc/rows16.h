@@ -14,7 +14,7 @@ struct LkRows16 {
     uint8_t* q81_dst;      // `dual` only, when given: the result as Q8_1 rows (blocks of 32 consecutive output
     int q81_stride;        // rows, q81_stride blocks between rows) instead of f32 in dst[0]; n a multiple of 32
     int out_type;          // element type of `dst` (lk_store_as), dense launches
-    const void* x;         // short launches: the rows themselves instead of y (nb * 256 elements each, 16- or 8-byte aligned), quantized on the way in
+    const void* x;         // short launches: the rows themselves instead of y (nb * 256 elements each), quantized on the way in
     int x_type;
 };
 // True when the launch takes `size_m` activation rows of `nb` super-blocks (their codes fit in LDS).
@@ -51,5 +51,5 @@ int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, in
 // weights off a 16-byte boundary.
 int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                         hipStream_t stream, int out_type);
-// The same straight over rows of `x_type` (results in it too), 16- or 8-byte aligned. -1: a call it does not serve.
+// The same straight over rows of `x_type` (results in it too). -1: a call it does not serve.
 int lk_rows16_q6k_short_rows(const void* w, const void* x, float* output, int size_m, int size_n, int size_k, int x_type, hipStream_t stream);

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         const uint32_t at = (uint32_t)(kb * Q6K_BYTES), ya = (uint32_t)(kb * 8 * Q81_BYTES);
         if constexpr (SRC != Q81) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) b.v[u] = *(const Raw*)(x_row + kb * 256 + 32 * u);
+            for (int u = 0; u < 8; ++u) b.v[u] = *(const typename SrcOf<SRC>::Load*)(x_row + kb * 256 + 32 * u);
         } else {
 #pragma unroll
             for (int j = 0; j < HEADS; ++j) b.head[j] = *(const uint32_t*)(y0 + (y_head[j] + ya));

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     auto load_act = [&](Act& b, int kb) {
         if constexpr (SRC != Q81) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) b.v[u] = *(const typename SrcOf<SRC>::Raw*)(x_row + kb * 256 + 32 * u);
+            for (int u = 0; u < 8; ++u) b.v[u] = *(const typename SrcOf<SRC>::Load*)(x_row + kb * 256 + 32 * u);
             return;
         }
         const uint32_t at = (uint32_t)(kb * 8 * Q81_BYTES);

@@ -833,7 +833,7 @@ int lk_rows_linear(int wtype, const void* w, const void* q8_1, int stride_y, voi
 
 int lk_rows_linear_direct(int wtype, const void* w, const void* x, void* out, int x_type, int rows, int n, int k, hipStream_t stream) {
     const int elem = x_type == LK_TYPE_F32 ? 4 : 2;
-    if (k % 256 != 0 || (((uintptr_t)w) & 15) != 0 || ((uintptr_t)x % (4 * elem)) != 0) return -1;
+    if (k % 256 != 0 || (((uintptr_t)w) & 15) != 0 || ((uintptr_t)x % elem) != 0) return -1;
     if (wtype == LK_TYPE_Q6_K) return lk_rows16_q6k_short_rows(w, x, (float*)out, rows, n, k, x_type, stream);
     if (wtype != LK_TYPE_Q4_K && wtype != LK_TYPE_Q5_K) return -1;
     LkRows16 r{};

@@ -334,7 +334,7 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
     ("q6_k", 2030, 2816, 15)])
 def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n, k, rows, half):
     # the same products from Q8_1 rows of the stand-alone quantizer: bit for bit, with zeros, a row's largest code everywhere, halves between two codes,
-    # tiny values and infinities among the rows; rows that start off a 16-byte piece go by way of the quantizer
+    # tiny values and infinities among the rows; rows that start off a 16-byte piece too
     w = dev(synth.weight(DT[name], n, k, seed=86, stream=3))
     x = dev(synth.activation(rows, k, seed=86))
     x[0, :64] = 0
@@ -351,6 +351,31 @@ def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n,
     assert torch.equal(lin(flat[1:].view(rows, k)), got)
     x[0, 5], x[rows - 1, k - 1] = float("inf"), float("nan")
     assert torch.equal(torch.nan_to_num(lin(x)), torch.nan_to_num(fn(w, x.float(), n).to(half)))
+    lin.close()
+
+
+@pytest.mark.parametrize("half", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name,n,k,rows", [("q4_k", 260, 4096, 3), ("q5_k", 2030, 2048, 9), ("q6_k", 2050, 3072, 8), ("q6_k", 1030, 1024, 16)])
+def test_a_few_rows_off_a_vector_boundary_are_one_launch_without_a_workspace(name, n, k, rows, half):
+    # a recorded call with nothing reserved is refused where it needs a workspace; rows on any element need none
+    lin = Linear(DT[name], dev(synth.weight(DT[name], n, k, seed=88, stream=1)), n, k)
+    x = dev(synth.activation(rows, k, seed=88)).to(half)
+    want = lin(x)
+    flat = torch.zeros(rows * k + 1, device="cuda", dtype=half)
+    flat[1:] = x.reshape(-1)
+    lib.load().lkh_release_workspaces()
+    side, graph, out = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.zeros_like(want)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        rc = lib.load().lkh_qkernel_matmul_forward(lin.h, flat[1:].data_ptr(), X_TYPES[half], rows, out.data_ptr(), side.cuda_stream, 0)
+    assert rc == 0 and lin.path == "rows-on-matrix-unit"
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    # half an element off: no such rows
+    assert lib.load().lkh_qkernel_matmul_forward(lin.h, flat.data_ptr() + 1, X_TYPES[half], rows, out.data_ptr(), None, 0) == lib.LK_ERR_ARG
     lin.close()
 
 
