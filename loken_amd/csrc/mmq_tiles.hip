@@ -36,6 +36,12 @@ __global__ __launch_bounds__(256) void operands_from_records_kernel(const uint8_
                    (int)*(const int16_t*)(rec + 272 + 2 * s));
 }
 
+// The runs' share of the sorted rows [from, to), counted from `from`.
+__global__ __launch_bounds__(256) void bounds_of_pass_kernel(const int32_t* __restrict__ bounds, int32_t* __restrict__ pass, int count, int from, int to) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e < count) pass[e] = min(max(bounds[e], from), to) - from;
+}
+
 // Q8_1 rows, `stride` blocks apart -> operands, on the same grid: the codes and scales the quantizer below makes of the rows
 // they came from, so the products carry its bits. A few rows a call: a launch's time, whatever the bytes.
 __global__ __launch_bounds__(256) void operands_from_q8_1_kernel(const uint8_t* __restrict__ y, LkTokenOperands ops, int stride, int rows) {
@@ -131,14 +137,16 @@ MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup) 
 // keeps them apart).
 constexpr int64_t OPERANDS_CAP = 256ll << 20;
 
+// Rows of a pass over `blocks` 256-value blocks each; less than 128: rows too long for these kernels.
+int64_t rows_of_pass(int64_t blocks) { return OPERANDS_CAP / (blocks * (LK_OPERAND_CODES + LK_OPERAND_TAB)) / 128 * 128 - LK_OPERAND_PAD; }
+
 // The product in passes; fill(operands, first row, rows) launches what writes a pass's operands. Returns as lk_mmq_tiles_dense.
 template <class Fill>
 int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, Fill fill) {
     if ((uintptr_t)pb.w % f.align != 0 || (f.align != 16 && pb.n < 128)) return -1;
     // lane offsets inside a tile are 32-bit
     if (pb.row_blocks * f.unit * 256 > (int64_t)INT32_MAX || pb.m_begin != 0) return -1;
-    const int64_t row_bytes = pb.nb * (LK_OPERAND_CODES + LK_OPERAND_TAB);
-    const int64_t fit = OPERANDS_CAP / row_bytes / 128 * 128 - LK_OPERAND_PAD;
+    const int64_t fit = rows_of_pass(pb.nb);
     if (fit < 128 || pb.nb > INT32_MAX / 2) return -1;
     const int per_pass = (int)std::min<int64_t>(pb.m_end, fit);
     LkScratch scratch(s);
@@ -217,12 +225,30 @@ int lk_mmq_tiles_moe_records(int wtype, const MmqProblem& pb, const uint8_t* w_s
     if ((uintptr_t)pb.y % 16 != 0 || pb.row_blocks > INT32_MAX / 256 || pb.nb > INT32_MAX / 256 ||
         !lk_mmq_tiles_moe_fit(wtype, pb.w, w_second, stride_expert, pb.n, tiles_of(wtype)->values * pb.row_blocks, pb.rows_total, false))
         return -1;
+    // More sorted rows than a pass holds: pass by pass, every expert's run cut at the pass's ends (its weights are read again by the
+    // pass that goes on with it)
+    const int64_t fit = rows_of_pass(pb.nb);
+    if (fit < 128) return -1;
+    const int64_t per_pass = std::min(pb.rows_total, fit);
+    const size_t operand_bytes = lk_operand_bytes(per_pass, pb.nb);
+    const bool whole = per_pass == pb.rows_total;
     LkScratch scratch(s);
-    void* buffer = scratch.get(LK_SCRATCH_TOKENS, lk_operand_bytes(pb.rows_total, pb.nb));
+    uint8_t* buffer = (uint8_t*)scratch.get(LK_SCRATCH_TOKENS, operand_bytes + (whole ? 0 : (size_t)(n_experts + 1) * 4));
     if (!buffer) return -1;
-    const LkTokenOperands ops = lk_operands_at(buffer, pb.rows_total, pb.nb);
-    hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((pb.rows_total + 31) / 32)), dim3(256), 0, s, pb.y, ops,
-                       pb.rows_total, 0, (int)pb.rows_total);
-    const MmqTileExperts ex{bounds, nullptr, w_second, dst_second, stride_expert, ncols_max, n_experts, nullptr};
-    return lk_mmq_tiles_moe(wtype, pb, ops, ex, s) == LK_OK ? 128 : 0;
+    int32_t* cut = (int32_t*)(buffer + operand_bytes);
+    for (int64_t m0 = 0; m0 < pb.rows_total; m0 += per_pass) {
+        MmqProblem pass = pb;
+        pass.rows_total = std::min(per_pass, pb.rows_total - m0);
+        if (pass.ids_dst) pass.ids_dst += m0;
+        else pass.dst += m0 * pb.ldd;
+        const LkTokenOperands ops = lk_operands_at(buffer, pass.rows_total, pb.nb);
+        hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((pass.rows_total + 31) / 32)), dim3(256), 0, s, pb.y, ops,
+                           pb.rows_total, (int)m0, (int)pass.rows_total);
+        if (!whole)
+            hipLaunchKernelGGL(bounds_of_pass_kernel, dim3((unsigned)(n_experts / 256 + 1)), dim3(256), 0, s, bounds, cut, n_experts + 1, (int)m0,
+                               (int)(m0 + pass.rows_total));
+        const MmqTileExperts ex{whole ? bounds : cut, nullptr, w_second, dst_second, stride_expert, std::min(ncols_max, pass.rows_total), n_experts, nullptr};
+        if (lk_mmq_tiles_moe(wtype, pass, ops, ex, s) != LK_OK) return 0;
+    }
+    return 128;
 }

@@ -670,6 +670,46 @@ def test_block_of_plain_blocks_on_the_f16_tiles(runs, hidden, ffn, gu, dn):
     test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn)
 
 
+@pytest.mark.parametrize("wtype,second,mapped", [(lib.TYPE_Q4_K, True, False), (lib.TYPE_Q6_K, False, True)])
+def test_expert_product_of_more_rows_than_its_operands_buffer_holds(wtype, second, mapped):
+    """17000 rows of 14336 values: 564 MB of token operands, which the launch makes and multiplies in passes of 256 MB at most,
+    runs cut at their ends: the bits of calls over less than a pass each."""
+    l, k, n, stacks = lib.load(), 14336, 128, 2 if second else 1
+    runs, info, s = [5000, 0, 11963, 37], ops.MMQ_DEVICE_INFO, torch.cuda.current_stream().cuda_stream
+    w = dev(synth.weight(wtype, stacks * len(runs) * n, k, seed=70, stream=1))
+    half = w.numel() // stacks
+    base = dev(synth.activation(500, k, seed=70))
+    bounds = np.concatenate([[0], np.cumsum(runs)]).astype(np.int32)
+
+    def launch(y, rows, cut, dst, ids):
+        w2 = w.reshape(-1)[half:].data_ptr() if second else None
+        assert getattr(l, moe.MMQ_MOE_LAUNCHER[wtype])(
+            w.data_ptr(), w2, n, y.data_ptr(), dst.data_ptr(), cut.data_ptr(), ids.data_ptr() if ids is not None else None, half // len(runs), k, n, rows,
+            k // synth.BLOCK_LEN[wtype], stacks * n, len(runs), 12000, 12000, 0, info["cc"], info["smpbo"], info["warp_size"], s) != 0
+
+    total = int(bounds[-1])
+    x = base.repeat(total // 500 + 1, 1)[:total].contiguous()
+    y = ops.mmq_quantize(wtype, x)
+    ids = dev(np.random.default_rng(70).permutation(total).astype(np.int32)) if mapped else None
+    out = torch.full((total, stacks * n), float("nan"), device="cuda")
+    launch(ops.mmq_quantize(wtype, base), 500, dev(np.array([0, 500, 500, 500, 500], np.int32)), torch.empty_like(out[:500]), None)   # kernels loaded
+    l.loken_stream_scratch_release()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    launch(y, total, dev(bounds), out, ids)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 336 << 20   # 256 MB and the quarter more that a buffer grows by
+    if mapped:
+        out = out[ids.long()]
+    for m0 in range(0, total, 500):
+        m1 = min(m0 + 500, total)
+        part = torch.empty((m1 - m0, stacks * n), device="cuda")
+        y = ops.mmq_quantize(wtype, x[m0:m1])
+        launch(y, m1 - m0, dev(np.clip(bounds, m0, m1) - np.int32(m0)), part, None)
+        assert torch.equal(out[m0:m1], part), m0
+    l.loken_stream_scratch_release()
+
+
 @pytest.mark.parametrize("n,n_experts,topk", [(1, 3, 1), (63, 5, 3), (64, 1, 1), (1025, 130, 5), (4097, 512, 1), (8888, 128, 8)])
 def test_routing_is_a_stable_grouping(n, n_experts, topk):
     choices = synth.rand_ints(23, n, n, n_experts).astype(np.int32).reshape(-1, topk)
