@@ -295,11 +295,13 @@ def test_rows_that_forward_serves_another_way_are_not_quantized_for_the_matvec()
         big.close()
 
 
-@pytest.mark.parametrize("name,rows,expect", [("q4_k", 12, "tiled"), ("q5_k", 16, "tiled"), ("q6_k", 12, "rows-on-matrix-unit"),
-                                               ("q4_k", 8, "matvec")])
-def test_long_rows_at_nine_to_sixteen_activation_rows(name, rows, expect):
-    # rows of 8192 values: Q4_K / Q5_K leave the 16-row tiles for the tiled matmul (K cut into ranges) from nine rows
-    wtype, n, k = DT[name], 2048, 8192
+@pytest.mark.parametrize("name,rows,n,k,expect", [
+    ("q4_k", 12, 2048, 8192, "rows-on-matrix-unit"), ("q5_k", 16, 2048, 8192, "rows-on-matrix-unit"), ("q6_k", 12, 2048, 8192, "rows-on-matrix-unit"),
+    ("q4_k", 8, 2048, 8192, "matvec"), ("q5_k", 9, 2288, 7680, "rows-on-matrix-unit"), ("q4_k", 16, 8200, 8192, "tiled")])
+def test_long_rows_at_nine_to_sixteen_activation_rows(name, rows, n, k, expect):
+    # Q4_K / Q5_K: the 16-row tiles up to 8192 matrix rows (2048 x 8192 at 12 rows 9.2 us, the tiled matmul with K cut 17.0), the tiled
+    # matmul past them
+    wtype = DT[name]
     w = synth.weight(wtype, n, k, seed=96, stream=1)
     x = synth.activation(rows, k, seed=96)
     lin = Linear(wtype, dev(w), n, k)
