@@ -89,7 +89,7 @@ int matvec_rows(int dtype, int k) {
 // once per 32 to 128 rows. Measured on MI355X, quantizer included, rows kernel against f16 tiles (us), for matrices of 512 rows or more:
 //   Q4_K, 9 to 16 rows: 512 x 8192 10..11 / 16, 2048 x 8192 9..10 / 17..18, 8192 x 8192 14 / 22, 4096 x 14336 15..16 / 23, 10000 x 5120 18 / 21, 12000 x 10240 35..42 / 29; Q5_K alike
 //     17 to 32: 700 x 5120 18 / 15, 10000 x 5120 25 / 22, 2048 x 6144 21 / 16, 14336 x 4096 at 24 22 / 21; 4096 x 4096 16 / 16, 8192 x 4096 16 / 19
-//     above: 3000 x 5120 at 33 / 96 20 / 18, 27 / 24; 4096 x 4096 at 64 / 96 (256, 384 workgroups) 17 / 20, 25 / 25; 1024 x 4096 at 200 / 400
+//     above: 1024 x 4608 at 33 18 / 14, 1100 x 8192 at 33 / 64 26 / 18, 26 / 19; 3000 x 5120 at 33 / 96 20 / 18, 27 / 24; 4096 x 4096 at 64 / 96 (256, 384 workgroups) 17 / 20, 25 / 25; 1024 x 4096 at 200 / 400
 //     (224, 416) 19 / 21, 28 / 25; 2048 x 2048 at 200 17 / 19. Q5_K alike.
 //   Q6_K, 9 to 16 rows: 2048 x 8192 13 / 20, 6144 x 6144 20 / 24, 4096 x 14336 20 / 30, 3000 x 5120 12 / 18, 10000 x 5120 26 / 26
 //     17 to 32: 2048 x 14336 20 / 25, 8192 x 4096 17..19 / 23, 6144 x 6144 22..23 / 24..25, 700 x 11008 13 / 22; 10000 x 5120 30..33 / 27, 4096 x 14336 35 / 31,
@@ -112,8 +112,6 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
         return (k < 3072 || (n < 1024 && k < 4608)) && results <= 450000;
     }
     if (rows <= 16) return k < 7168 || n <= 8192;
-    // (and here on the rows kernel at 1100 x 8192 and 33 rows, test_long_rows_above_sixteen_activation_rows; 1024 x 8192 there 27 / 18)
-    if (k >= 4608 && k < 12288 && n >= 1024 && n < 1152 && rows > 32 && rows <= 64) return true;
     if (k >= 4608) return k < 5632 && items > 128 && items <= 256 && rows > 32;
     if (rows <= 32) return n < 12288 || k < 4096 || rows < 20;
     return items <= 256 || (k <= 2048 && results <= 450000);

@@ -314,7 +314,7 @@ def test_long_rows_at_nine_to_sixteen_activation_rows(name, rows, n, k, expect):
         lin.close()
 
 
-@pytest.mark.parametrize("name,k,rows,expect", [("q4_k", 8192, 17, "tiled"), ("q5_k", 8192, 32, "tiled"), ("q4_k", 8192, 33, "rows-on-matrix-unit"),
+@pytest.mark.parametrize("name,k,rows,expect", [("q4_k", 8192, 17, "tiled"), ("q5_k", 8192, 32, "tiled"), ("q4_k", 8192, 33, "tiled"),
                                                  ("q4_k", 12288, 33, "tiled"), ("q6_k", 8192, 32, "rows-on-matrix-unit"),
                                                  ("q6_k", 8192, 33, "tiled")])
 def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
