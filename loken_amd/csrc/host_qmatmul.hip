@@ -119,15 +119,16 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
 
 // The K-quants at 3 to 8 f32 rows: the 16-row tiles of the matrix-unit kernels (their time hardly moves
 // with the row count) against mat-vec launches (whose dot work grows with every row). Up to 4096 values a row the rows kernel takes the rows
-// themselves, one launch where the mat-vec kernels need the quantizer's too: from 256 x 1024 to 8192 x 4096 at 3 to 8 rows 6.7 to 8.6 us against 9.5 to 13.7
-// (matrices of 1024 values a row and fewer than 8192 results stay, as callers that read path() expect). Longer rows: measured on MI355X, mat-vec against rows kernel, quantizer included (us): Q4_K / Q5_K 4096 x 8192 at 4 / 5 / 8 rows 10.7, 11.7, 14.1 / 10.2,
+// themselves, one launch where the mat-vec kernels need the quantizer's too, rows kernel / mat-vec at 3, 5, 8 rows: Q4_K 256 x 256 3.6, 3.7, 3.7 / 7.4, 9.3, 12.2; 2000 x
+// 1024 3.6 / 7.4, 9.3, 12.2; 256 x 2048 4.1 / 6.6, 8.1, 10.0; 8192 x 4096 7.6, 7.8, 7.9 / 9.9, 11.6, 14.1; Q6_K 1024 x 1024 4.0 / 7.9, 9.7, 12.6; 4096 x 4096 8.4, 8.3, 8.5 /
+// 8.9, 10.3, 12.1 (fewer than 256 matrix rows have not been moved: 64 x 1024 3.6 / 7.0, 9.0, 12.0, Q6_K 200 x 4096 7.0 / 6.5, 7.4, 8.8). Longer rows: measured on MI355X, mat-vec against rows kernel, quantizer included (us): Q4_K / Q5_K 4096 x 8192 at 4 / 5 / 8 rows 10.7, 11.7, 14.1 / 10.2,
 // 10.5, 10.0, 4096 x 14336 at 3 / 8 13.8, 24.0 / 13.5, 14.1, 8192 x 4096 at 4 / 5 10.8, 11.6 / 10.8, 10.1, 1024 x 14336 at 6 / 8 13.3, 15.5 / 12.0, 12.2; 2048 x 8192 at 8 10.8 / 9.8;
 // k = 2048: 2048 rows from 4, 6144 and 151936 from 3. Q6_K 4096 x 8192 at 5 / 6 13.1, 13.8 / 12.9, 12.9, 6144 x 2048 at 5 / 6 10.6, 11.5 / 10.0, 9.9, 1024 x 14336 at
 // 5 / 8 13.8, 22.1 / 14.6, 14.7, 700 x 5120 at 8 12.2 / 10.0, 512 x 4096 at 8 10.0 / 9.8, 4096 x 14336 at 3 / 4 16.6, 18.8 / 16.8, 16.8.
 static bool small_rows_kernel_pays(int dtype, int n, int k, int rows) {
     if (rows < 3 || rows > 8 || k % 256 != 0 || (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K)) return false;
     const long long weights = (long long)n * k;
-    if (k <= 4096 && n >= 256 && n <= (dtype == LK_TYPE_Q6_K ? 6144 : 16384) && (k > 1024 || (long long)n * rows >= 8192)) return true;
+    if (k <= 4096 && n >= 256 && n <= (dtype == LK_TYPE_Q6_K ? 6144 : 16384)) return true;
     if (dtype == LK_TYPE_Q6_K)
         return (rows >= 7 && n >= 512) || (rows >= 5 && weights * rows >= (76ll << 20)) || (k % 2048 == 0 && weights >= (48ll << 20));
     return k <= 2048 ? (long long)n * rows >= 8192 : weights * rows > (128ll << 20);
