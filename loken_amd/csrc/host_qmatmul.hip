@@ -207,8 +207,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     //     straight from HBM
     if (rows_kernel_serves(dtype_, n_, k_, rows) && rows_kernel_fits) {
         const int blocks = k_ / 32;
-        // (few matrix rows at more than eight: by way of the scratch, without which a recorded call is refused)
-        int rc = rows <= 8 || n_ >= 256 ? lk_rows_linear_direct(dtype_, blob_, x, out, x_type, rows, n_, k_, stream) : -1;
+        int rc = lk_rows_linear_direct(dtype_, blob_, x, out, x_type, rows, n_, k_, stream);
         if (rc < 0) {
             LkScratch scratch(stream);
             void* act = scratch.get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK);

@@ -159,12 +159,13 @@ def test_half_rows_above_the_matvec_family_follow_the_oracle_and_leave_in_their_
 
 
 def test_workspace_grows_outside_a_capture_only_and_replays_then():
+    # twenty rows: up to sixteen over a matrix like this are quantized in the launch and need no workspace
     wtype, n, k = lib.TYPE_Q4_K, 128, 1024
     w = dev(synth.weight(wtype, n, k, seed=83, stream=1))
     lin = Linear(wtype, w, n, k)
     lib.load().lkh_release_workspaces()
     try:
-        x = dev(synth.activation(12, k, seed=83))
+        x = dev(synth.activation(20, k, seed=83))
         side = torch.cuda.Stream()
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.stream(side):
@@ -176,10 +177,10 @@ def test_workspace_grows_outside_a_capture_only_and_replays_then():
         eager = lin(x)                                       # reserves the workspace
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
-        out = torch.empty((12, n), device="cuda")
+        out = torch.empty((20, n), device="cuda")
         with torch.cuda.stream(side):
             with torch.cuda.graph(graph, stream=side):
-                rc = lib.load().lkh_qkernel_matmul_forward(lin.h, x.data_ptr(), lib.TYPE_F32, 12, out.data_ptr(),
+                rc = lib.load().lkh_qkernel_matmul_forward(lin.h, x.data_ptr(), lib.TYPE_F32, 20, out.data_ptr(),
                                                            side.cuda_stream, 0)
                 assert rc == 0
         for _ in range(3):
@@ -334,7 +335,7 @@ def test_long_rows_above_sixteen_activation_rows(name, k, rows, expect):
 @pytest.mark.parametrize("name,n,k,rows", [
     ("q4_k", 260, 1280, 3), ("q5_k", 256, 4096, 8), ("q4_k", 4100, 2048, 7), ("q5_k", 8200, 2304, 5), ("q4_k", 16384, 2048, 8), ("q6_k", 270, 1280, 4),
     ("q6_k", 300, 4096, 8), ("q6_k", 2050, 3072, 3), ("q6_k", 6144, 2048, 6), ("q4_k", 2048, 4096, 16), ("q5_k", 2050, 2048, 9),
-    ("q6_k", 2030, 2816, 15)])
+    ("q6_k", 2030, 2816, 15), ("q4_k", 1, 256, 9), ("q5_k", 200, 4096, 16), ("q6_k", 40, 1280, 12)])
 def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n, k, rows, half):
     # the same products from Q8_1 rows of the stand-alone quantizer: bit for bit, with zeros, a row's largest code everywhere, halves between two codes,
     # tiny values and infinities among the rows; rows that start off a 16-byte piece too
@@ -358,7 +359,8 @@ def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n,
 
 
 @pytest.mark.parametrize("half", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("name,n,k,rows", [("q4_k", 260, 4096, 3), ("q5_k", 2030, 2048, 9), ("q6_k", 2050, 3072, 8), ("q6_k", 1030, 1024, 16)])
+@pytest.mark.parametrize("name,n,k,rows", [("q4_k", 260, 4096, 3), ("q5_k", 2030, 2048, 9), ("q6_k", 2050, 3072, 8), ("q6_k", 1030, 1024, 16),
+                                           ("q4_k", 128, 1024, 12), ("q5_k", 17, 256, 9), ("q6_k", 255, 4096, 16)])
 def test_a_few_rows_off_a_vector_boundary_are_one_launch_without_a_workspace(name, n, k, rows, half):
     # a recorded call with nothing reserved is refused where it needs a workspace; rows on any element need none
     lin = Linear(DT[name], dev(synth.weight(DT[name], n, k, seed=88, stream=1)), n, k)
