@@ -146,6 +146,13 @@ static bool fits_rows_kernel(int dtype, int k, const void* blob) {
     return k % 256 == 0 && ((uintptr_t)blob & (dtype == LK_TYPE_Q6_K ? 1 : 15)) == 0;
 }
 
+// Three to eight rows go to the rows kernels by the lines of the 16-row tiles, which take weights from a 16-byte boundary on. Q6_K weights off it (a
+// matrix that starts at some row of another one) would get the 32-row tiles: 3 / 8 rows, those / mat-vec: 2048 x 3840 13.6, 14.0 / 7.1, 10.2; 4096 x 8448
+// at 5 / 8 24.8, 25.3 / 18.4, 23.6; 256 x 1280 at 3 / 8 7.9, 8.1 / 7.4, 11.4.
+static bool few_rows_to_kernel(int dtype, int n, int k, int rows, const void* blob) {
+    return ((uintptr_t)blob & 15) == 0 && small_rows_kernel_pays(dtype, n, k, rows);
+}
+
 QKernelMatMul::QKernelMatMul(int dtype, int n, int k, const void* blob, int device)
     : dtype_(dtype), n_(n), k_(k), device_(device), blob_(blob) {}
 
@@ -170,7 +177,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
 
     // --- mat-vec family: up to matvec_rows, or any count when every row must sum like a one-row call
     const bool rows_kernel_fits = fits_rows_kernel(dtype_, k_, blob_);
-    const bool to_rows_kernel = rows_kernel_fits && small_rows_kernel_pays(dtype_, n_, k_, rows);
+    const bool to_rows_kernel = few_rows_to_kernel(dtype_, n_, k_, rows, blob_);
     const bool few_to_tiles = few_rows_to_tiles(dtype_, n_, k_, rows, blob_);
     const bool to_nibble_tiles = !decode_order && (few_to_tiles || nibble_tiles_pay(dtype_, n_, k_, rows)) &&
                                  ((uintptr_t)blob_ & (dtype_ == LK_TYPE_Q2_K ? 3 : 1)) == 0;
@@ -302,7 +309,7 @@ int QKernelMatMul::forward_quantized(const QuantizedActivation& a, void* out, vo
     const int blocks = (int)pad_to((size_t)k_, 512) / 32;
     // The launches forward takes at this row count, with its bits; where they decline, or the tiles have no scratch, the mat-vec launches
     const bool one_order = decode_order && a.rows > 1;
-    if (!one_order && fits_rows_kernel(dtype_, k_, blob_) && small_rows_kernel_pays(dtype_, n_, k_, a.rows)) {
+    if (!one_order && few_rows_to_kernel(dtype_, n_, k_, a.rows, blob_)) {
         const int rc = lk_rows_linear(dtype_, blob_, a.q81, blocks, out, a.x_type, a.rows, n_, k_, (hipStream_t)stream);
         if (rc == LK_OK) last_path_ = Path::RowsOnMatrixUnit;
         if (rc != LK_ERR_ARG) return rc;

@@ -455,6 +455,21 @@ def test_rows_quantized_beforehand_are_served_by_the_launches_of_forward(name, r
     lin.close()
 
 
+@pytest.mark.parametrize("rows,n,k,expect", [(3, 1030, 2816, "matvec"), (8, 1030, 2816, "matvec"), (5, 2050, 4096, "matvec"),
+                                             (9, 1030, 2816, "rows-on-matrix-unit"), (20, 300, 1280, "rows-on-matrix-unit")])
+def test_q6k_weights_off_a_16_byte_boundary(rows, n, k, expect):
+    w = synth.weight(lib.TYPE_Q6_K, n, k, seed=89, stream=1)
+    flat = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda")
+    flat[2:2 + w.size] = dev(w).reshape(-1)
+    x = synth.activation(rows, k, seed=89)
+    lin = Linear(lib.TYPE_Q6_K, flat[2:], n, k)
+    got = lin(dev(x))
+    assert lin.path == expect
+    lin.close()
+    pick = np.arange(0, n, 5)
+    assert close(got.cpu().numpy()[:, pick], oracle.ob_matmul(lib.TYPE_Q6_K, x, w[pick], len(pick)))
+
+
 @pytest.mark.parametrize("name,rows,n,k", [("q4_k", 3, 4096, 2048), ("q5_k", 4, 14336, 4096), ("q6_k", 7, 1024, 2048), ("q6_k", 3, 4096, 14336),
                                            ("q8_0", 17, 513, 4096), ("q4_0", 16, 645, 1024)])
 def test_large_matrices_and_tiled_row_counts_refuse_rows_quantized_beforehand(name, rows, n, k):
