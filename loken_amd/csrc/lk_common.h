@@ -395,6 +395,9 @@ int lk_tune_read(LkTuneSite& site);
 static inline bool lk_env_flag_site(int v) { return v != 0; }
 #define lk_env_flag(NAME) lk_env_flag_site(lk_tune_env(NAME))
 
+// Measurement runs without the 16-row-tile kernels, or with them up to eight activation rows only.
+static inline bool lk_rows16_off(int rows) { return lk_tune_env("LK_TUNE_ROWS16_OFF") != 0 || (rows > 8 && lk_tune_env("LK_TUNE_ROWS16_MAX8") != 0); }
+
 static inline int lk_launch_status() {
     return hipGetLastError() == hipSuccess ? LK_OK : LK_ERR_LAUNCH;
 }

@@ -444,9 +444,8 @@ int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, in
     if (size_m < 1 || size_m > 32 || size_n < 1 || size_k < 256) return -1;
     // rows of whole granules, on 16-byte boundaries; a tile's granules within one workgroup
     if (size_k % (256 * GRAN) != 0 || size_k / (256 * GRAN) > MAX_WAVES || (((uintptr_t)w) & 15) != 0) return -1;
-    if (lk_tune_env("LK_TUNE_ROWS16_OFF") != 0) return -1;
+    if (lk_rows16_off(size_m)) return -1;
     const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
-    if (size_m > 8 && lk_tune_env("LK_TUNE_ROWS16_MAX8") != 0) return -1;
     // (the short launch has taken the calls of few row tiles: rows16_q6k_short.hip)
     if (size_m <= 4) return launch<4>(a, stream);
     const int n_tiles = (size_n + TILE - 1) / TILE;

@@ -286,7 +286,7 @@ int set_rows(int size_m, int size_n, int size_k) {
 int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                         hipStream_t stream, int out_type) {
     // (rows of more than 32768 values: the others' to take or refuse)
-    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || size_k > 32768 || (((uintptr_t)w) & 15) != 0) return -1;
+    if (size_m < 1 || size_m > 64 || size_n < 1 || size_k < 256 || size_k > 32768 || (((uintptr_t)w) & 15) != 0 || lk_rows16_off(size_m)) return -1;
     const int rows = set_rows(size_m, size_n, size_k);
     if (rows == 0) return -1;
     const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
@@ -296,7 +296,7 @@ int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size
 
 // Up to sixteen rows of up to 4096 values straight from them, as lk_rows16_short_rows.
 int lk_rows16_q6k_short_rows(const void* w, const void* x, float* output, int size_m, int size_n, int size_k, int x_type, hipStream_t stream) {
-    if (size_m < 1 || size_m > 16 || size_n < 1 || size_k < 256 || size_k > 4096 || (((uintptr_t)w) & 15) != 0 || set_rows(size_m, size_n, size_k) != 8) return -1;
+    if (size_m < 1 || size_m > 16 || size_n < 1 || size_k < 256 || size_k > 4096 || (((uintptr_t)w) & 15) != 0 || lk_rows16_off(size_m) || set_rows(size_m, size_n, size_k) != 8) return -1;
     const Args a{(const uint8_t*)w, (const uint8_t*)x, output, size_k / 256, size_n, size_m, 0, size_n, x_type};
     if (x_type == LK_TYPE_F32) return launch<8, false, ROWS_F32>(a, stream);
     return x_type == LK_TYPE_F16 ? launch<8, true, ROWS_F16>(a, stream) : launch<8, true, ROWS_BF16>(a, stream);

@@ -405,7 +405,7 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
 // (Rows of up to 32768 values: longer ones are the other launches' to take or refuse.)
 bool lk_rows16_short_pays(int m, int n, int nb) {
     const int tiles = (n + TILE - 1) / TILE, cus = lk_device().cus;
-    return m >= 1 && m <= MAX_TOKS && nb <= 128 && (tiles <= cus || (tiles <= (m <= 8 ? 4 : 2) * cus && nb >= 8));
+    return m >= 1 && m <= MAX_TOKS && !lk_rows16_off(m) && nb <= 128 && (tiles <= cus || (tiles <= (m <= 8 ? 4 : 2) * cus && nb >= 8));
 }
 
 // Up to eight rows of up to 4096 values (sixteen as two sets where both are resident at once), a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the

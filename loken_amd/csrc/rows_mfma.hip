@@ -786,10 +786,7 @@ int launch_any(const Args& a, hipStream_t stream) {
     if (lk_rows16_short_pays(a.m, a.n, a.nb)) return lk_rows16_short(r, DUAL, Q5, stream);
     if (a.m <= 16) {
         // 16-row tiles (rows16_mfma.hip): half the matrix-unit time per weight, twice the tiles
-        if (lk_rows16_serves(a.m, a.nb) && lk_tune_env("LK_TUNE_ROWS16_OFF") == 0 &&
-            (a.m <= 8 || lk_tune_env("LK_TUNE_ROWS16_MAX8") == 0)) {
-            return lk_rows16_launch(r, DUAL, Q5, stream);
-        }
+        if (lk_rows16_serves(a.m, a.nb) && !lk_rows16_off(a.m)) return lk_rows16_launch(r, DUAL, Q5, stream);
     }
     if (a.m <= 8) {
         const int rc = launch_staged<1, DUAL, Q5>(a, stream);
@@ -917,8 +914,7 @@ extern "C" int lk_dense_q4k_rows_multi(const void* const* weights, float* const*
             return rest > 0 ? lk_dense_q4k_rows_multi(rest_w, rest_out, rest_n, rest, q8_1, size_m, size_k, q5, stream) : LK_OK;
         }
     }
-    if (lk_rows16_serves(size_m, nb) && lk_tune_env("LK_TUNE_ROWS16_OFF") == 0 &&
-        (size_m <= 8 || lk_tune_env("LK_TUNE_ROWS16_MAX8") == 0)) {
+    if (lk_rows16_serves(size_m, nb) && !lk_rows16_off(size_m)) {
         LkRows16 r{};
         for (int i = 0; i < count; ++i) {
             if (sizes_n[i] <= 0) continue;

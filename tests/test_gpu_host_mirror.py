@@ -384,6 +384,26 @@ def test_a_few_rows_off_a_vector_boundary_are_one_launch_without_a_workspace(nam
     lin.close()
 
 
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("knob,rows,off", [("LK_TUNE_ROWS16_OFF", 5, True), ("LK_TUNE_ROWS16_OFF", 12, True), ("LK_TUNE_ROWS16_MAX8", 8, False),
+                                           ("LK_TUNE_ROWS16_MAX8", 12, True)])
+def test_the_overrides_turn_the_short_launches_off_too(name, knob, rows, off, knobs):
+    # without them the rows go by way of the quantizer and its workspace, without which a recorded call is refused
+    l, n, k = lib.load(), 520, 1024
+    w, x = synth.weight(DT[name], n, k, seed=87, stream=1), synth.activation(rows, k, seed=87)
+    lin, xd = Linear(DT[name], dev(w), n, k), dev(x)
+    knobs.set(knob)
+    l.lkh_release_workspaces()
+    side, graph, out = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.empty((rows, n), device="cuda")
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        rc = l.lkh_qkernel_matmul_forward(lin.h, xd.data_ptr(), lib.TYPE_F32, rows, out.data_ptr(), side.cuda_stream, 0)
+    assert rc == (lib.LK_ERR_NOMEM if off else 0)
+    got = lin(xd)
+    assert lin.path == "rows-on-matrix-unit" and close(got.cpu().numpy(), oracle.ob_matmul(DT[name], x, w, n))
+    lin.close()
+
+
 @pytest.mark.parametrize("name,n,k,rows,expect", [
     ("q4_k", 8193, 7168, 9, "tiled"), ("q4_k", 8192, 7168, 9, "rows-on-matrix-unit"), ("q5_k", 512, 8448, 16, "rows-on-matrix-unit"),
     ("q5_k", 520, 4608, 17, "tiled"), ("q5_k", 520, 4352, 32, "rows-on-matrix-unit"), ("q4_k", 700, 5120, 200, "rows-on-matrix-unit"),
