@@ -1013,7 +1013,7 @@ static int launch_dense(void* fixup, const void* x, const void* y, void* dst, in
     // Q4_K 4096 x 14336 at 9 / 32 rows 22 / 23 us against 27 / 29, 1024 x 14336 at 33 / 400 rows 21 / 44 against 27 / 55, Q8_0 and Q4_0
     // 1024 x 2048 at 17 rows 16.7 and 15.8 against 20.6 and 18.2)
     if constexpr (F::F16_TYPE >= 0)
-        if (lk_mmq_tiles_take(F::F16_TYPE, nrows_x, ncols_y)) {
+        if (lk_mmq_f16_tiles(F::F16_TYPE, nrows_x, ncols_y)) {
             const int tm = lk_mmq_tiles_dense(F::F16_TYPE, pb, s, fixup);
             if (tm >= 0) return tm;
         }

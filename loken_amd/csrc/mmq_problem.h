@@ -151,8 +151,7 @@ int lk_operands_quantize(const void* x, int type, const LkTokenOperands& ops, in
 // Returns the token-tile width launched, 0 when the launch failed, -1 when the operands do not suit these kernels (alignment,
 // 32-bit offsets, no scratch) and the caller should take the int8 tiles.
 int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup);
-// Whether a dense product takes them: 9 token rows or more and 512 weight rows or more (LK_MMQ_I8 unset).
-bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows);
+// lk_mmq_f16_tiles: whether a dense product takes them: 9 token rows or more and 512 weight rows or more (LK_MMQ_I8 unset).
 // The same for `rows` rows of x, k values each, results in x's type: nothing between x and the operands.
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s);
 // The same from the rows' Q8_1 blocks, `stride` blocks between rows, with the same bits.

@@ -178,13 +178,13 @@ int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fix
     });
 }
 
-bool lk_mmq_tiles_take(int wtype, int64_t n, int64_t rows) {
+extern "C" int lk_mmq_f16_tiles(int wtype, int64_t n, int64_t rows) {
     const Tiles* f = tiles_of(wtype);
     return f && f->dense && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
 }
 
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {
-    if (!lk_mmq_tiles_take(wtype, n, rows) || k % 256 != 0) return -1;
+    if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
     return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
         (void)lk_operands_quantize((const uint8_t*)x + (int64_t)m0 * k * (type == LK_TYPE_F32 ? 4 : 2), type, ops, k, count, s);
@@ -193,7 +193,7 @@ int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, in
 
 int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
                              hipStream_t s) {
-    if (!lk_mmq_tiles_take(wtype, n, rows) || k % 256 != 0) return -1;
+    if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
     return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
         hipLaunchKernelGGL(operands_from_q8_1_kernel, dim3((unsigned)pb.nb, (unsigned)((count + 31) / 32)), dim3(256), 0, s,

@@ -56,6 +56,7 @@ SIGNATURES = {
     "launch_mmq_gguf_q3_k": (_i, [_vp, _vp, _vp, _vp] + [_i64] * 5 + [_i, _i, _i64, _i, _vp]),
     "launch_mmq_gguf_q2_k": (_i, [_vp, _vp, _vp, _vp] + [_i64] * 5 + [_i, _i, _i64, _i, _vp]),
 }
+SIGNATURES["lk_mmq_f16_tiles"] = (_i, [_i, _i64, _i64])
 _MOE_MMQ = (_i, [_vp, _vp, _i64, _vp, _vp, _vp, _vp] + [_i64] * 6 + [_i, _i64, _i64, _i, _i, _i64, _i, _vp])
 SIGNATURES.update({
     "launch_mmq_moe_gguf_q4_k": _MOE_MMQ,

@@ -273,10 +273,10 @@ def gemv_4096(args, dev):
 
 # ---------------------------------------------------------------------------- mmq
 def tile_kernel(wtype, n, m):
-    """Kernel, peak and operand type of a dense tiled call (launch_dense, mmq.hip). The K-quants of four to six bits form
-    their exact integer dots on the f16 matrix unit above 32 rows (scale folded into the weight operand), so that unit's
-    dense peak prices them; the int8 fraction is kept beside it because the target is quoted on the int8 peak."""
-    if wtype in (Q4K, lib.TYPE_Q5_K, Q6K) and m > 32 and n >= 2048:
+    """Kernel, peak and operand type of a dense tiled call (launch_dense, mmq.hip). Where the exact integer dots are formed on
+    the f16 matrix unit, that unit's dense peak prices them; the int8 fraction is kept beside it because the target is
+    quoted on the int8 peak."""
+    if lib.load().lk_mmq_f16_tiles(wtype, n, m):
         kernel = f"tile_dense_kernel, {NAMES[wtype]} (+ operands_from_records_kernel once per call, mmq_split_sum_kernel where K is cut)"
         return kernel, F16_PEAK_TFLOPS, "f16 operands (exact integers), f32 accumulate"
     return f"mmq_dense_kernel, {NAMES[wtype]} tile policy (mmq_dense_split_kernel where K is cut)", INT8_PEAK_TOPS, "int8"
