@@ -641,8 +641,9 @@ def test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn):
     ids = np.random.default_rng(68).permutation(np.repeat(np.arange(n_experts, dtype=np.int32), runs)).reshape(tokens, 1)
     ids = np.concatenate([ids, np.roll(ids, 7, axis=0)], axis=1)
     w = np.abs(synth.activation(tokens, 2, seed=68)) + np.float32(0.1)
-    if not lib.load().lk_moe_block_path(gu, dn, tokens, 2, n_experts, hidden, ffn) & lib.MOE_TILES:
-        pytest.skip("runs this short take other launches")
+    # runs of a few rows over 64 experts: the rows launch of Q4_K and the int8 tiles of Q6_K, the same block
+    tiles = n_experts < 60 or lib.TYPE_Q5_K in (gu, dn)
+    assert bool(lib.load().lk_moe_block_path(gu, dn, tokens, 2, n_experts, hidden, ffn) & lib.MOE_TILES) == tiles
     gate, up = (synth.weight(gu, n_experts * ffn, hidden, seed=68, stream=i) for i in (1, 2))
     down = synth.weight(dn, n_experts * hidden, ffn, seed=68, stream=3)
     x = synth.activation(tokens, hidden, seed=69)
@@ -661,6 +662,39 @@ def test_block_on_the_f16_tiles_at_every_run_length(runs, hidden, ffn, gu, dn):
     fed = down_fold_from_rows(dn, h, down, ids[sample], w[sample], n_experts, hidden)
     bound = 1e-3 * np.abs(fed) + 1e-4 * max(1.0, np.abs(fed).max())
     assert (np.abs(got.cpu().numpy()[sample] - fed) <= bound).all()
+
+
+@pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q4_K, lib.TYPE_Q6_K), (lib.TYPE_Q5_K, lib.TYPE_Q5_K), (lib.TYPE_Q6_K, lib.TYPE_Q6_K),
+                                   (lib.TYPE_Q8_0, lib.TYPE_Q4_0), (lib.TYPE_MXFP4, lib.TYPE_IQ4_NL)])
+def test_block_on_the_f16_tiles_keeps_odd_tokens_and_missing_choices_to_themselves(gu, dn):
+    """Zeros, tiny and large values, infinities and NaN among the tokens, choices outside the expert range among the pairs: the
+    launches' own bits, every other token as without them, a missing pair as one of weight zero."""
+    hidden, ffn, n_experts, tokens, topk = 512, 256, 16, 300, 4
+    assert lib.load().lk_moe_block_path(gu, dn, tokens, topk, n_experts, hidden, ffn) & lib.MOE_TILES
+    gate, up = (dev(synth.weight(gu, n_experts * ffn, hidden, seed=71, stream=i)) for i in (1, 2))
+    down = dev(synth.weight(dn, n_experts * hidden, ffn, seed=71, stream=3))
+    x = dev(synth.activation(tokens, hidden, seed=71))
+    ids, w = (dev(a) for a in oracle.topk_softmax(synth.activation(tokens, n_experts, seed=71, stream=7), topk))
+    run = lambda x, ids, w, **how: moe_forward(gu, dn, x, gate, up, down, ids, w, n_experts, ffn, **how)
+    clean = run(x, ids, w)
+    odd = x.clone()
+    odd[3] = 0
+    odd[50] *= 1e-7
+    odd[51, ::32] = 30.0   # (a Q8_1 scale holds 65504 x 127: the gated products of larger values are infinite)
+    odd[77, 5], odd[130, 511], odd[299] = float("inf"), float("nan"), float("-inf")
+    got = run(odd, ids, w)
+    changed = torch.tensor([3, 50, 51, 77, 130, 299], device="cuda")
+    kept = torch.ones(tokens, dtype=torch.bool, device="cuda")
+    kept[changed] = False
+    assert torch.equal(got[kept], clean[kept]) and not got[3].any() and torch.isfinite(got[[50, 51]]).all()
+    assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(run(odd, ids, w, return_rows=True)[0]))
+    missing, weights = ids.clone(), w.clone()
+    for token, slot, to in ((0, 0, -1), (9, 3, n_experts), (64, 1, 2 ** 31 - 1), (64, 2, -2 ** 31), (298, 0, 1 << 20)):
+        missing[token, slot], weights[token, slot] = to, 0.0
+    missing[200], weights[200] = -1, 0.0   # a token without any expert
+    got = run(x, missing, w)
+    assert torch.equal(got, run(x, ids, weights)) and not got[200].any()
+    assert torch.equal(got, run(x, missing, w, return_rows=True)[0])
 
 
 @pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q8_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_0, lib.TYPE_Q8_0), (lib.TYPE_Q4_K, lib.TYPE_Q4_0),
