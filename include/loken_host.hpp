@@ -24,21 +24,23 @@ enum class Path : int {
     None = 0,
     MatVecFused = 1,   /* one or two rows quantized inside the mat-vec launch */
     MatVec = 2,        /* lk_quantize_q8_1 + lk_mmvq (slices of eight rows) */
-    RowsOnMatrixUnit = 3, /* lk_quantize_q8_1 + lk_dense_q4k_rows / lk_dense_q5k_rows / lk_dense_q6k_rows */
-    Tiled = 4,         /* launch_mmq_quantize_q8_1_* + launch_mmq_gguf_* */
+    RowsOnMatrixUnit = 3, /* lk_quantize_q8_1 + lk_dense_q4k_rows / lk_dense_q5k_rows / lk_dense_q6k_rows, or up to sixteen rows of
+                             up to 4096 values quantized inside that launch */
+    Tiled = 4,         /* launch_mmq_quantize_q8_1_* + launch_mmq_gguf_*, or the f16 tiles' operands straight from the rows */
 };
 
 /* The most rows the mat-vec family takes for this weight before the call moves to a matrix-unit
- * kernel (matvec_rows of the reference, kernel_matmul.rs:27-33, with the crossovers measured on
- * MI355X: the K-quants 8 rows, except that matrices large enough to pay for it go to the 16-row tiles
- * of the matrix-unit rows kernels from 3 f32 rows on (Q4_K / Q5_K: n x rows of 57344, or 8192 at
- * k <= 2048; Q6_K: n x k of 48 Mi with k a multiple of 2048); then the matrix-unit rows kernels up to
- * 16 rows, or while n x rows x max(k, 4096) / 4096 <= 450 000 (twice that for a matrix of 1024 rows, and so
- * on: few rows yield few tiles; Q4_K / Q5_K rows of 8192 values or more over 2048 matrix rows leave them from
- * 9 rows; above 16 rows a matrix of 1024 rows or more leaves them where its rows have 8192 values, Q4_K / Q5_K
- * above 32 rows 12288, Q6_K only above 32), then the tiled matmul; Q8_0 mat-vec slices up to 16 rows, then the
- * tiled matmul; the 32-value nibble formats, Q3_K and Q2_K mat-vec slices up to 15 rows, or 8 over a
- * matrix of 48 Mi weights or more, then the tiled matmul). */
+ * kernel (matvec_rows of the reference, kernel_matmul.rs:27-33): 16 for Q8_0, else 8. forward goes by lines
+ * measured on MI355X (host_qmatmul.hip has them with both sides' times):
+ *   Q4_K, Q5_K, Q6_K  one or two rows on the mat-vec kernels. From 3 rows the matrix-unit rows kernels over 256 matrix rows or
+ *                     more of up to 4096 values (Q6_K: up to 6144 of them; longer rows and larger matrices from a row count of
+ *                     their own); from 9 rows those or the tiled matmul, which takes the long rows, the large matrices and most
+ *                     calls of more than 32 to 128 rows.
+ *   Q8_0              mat-vec slices up to 16 rows, but from 9 the tiled matmul over a matrix of 48 Mi weights, from 12 over
+ *                     32 Mi or rows of 8192 values, from 14 of 4096 values (512 matrix rows or more); then the tiled matmul.
+ *   Q4_0, Q4_1, Q5_0, Q5_1, Q2_K, Q3_K   mat-vec slices up to 15 rows, or 8 over a matrix of 48 Mi weights or more (Q4_0: 8 over
+ *                     512 matrix rows or more), then the tiled matmul.
+ *   IQ4_NL, MXFP4, IQ4_XS   mat-vec slices at any count. */
 int matvec_rows(int dtype, int k);
 
 class QKernelMatMul {
@@ -50,7 +52,8 @@ public:
     /* x [rows, k] (LK_TYPE_F32, F16 or BF16) -> out [rows, n] in x's type, on `stream`: every kernel
      * stores that type itself, its f32 sums rounded to nearest (the reference narrows the f32 rows its
      * mmq_forward returns the same way, kernel_matmul.rs:1086-1714). `decode_order` keeps every row on the mat-vec
-     * kernels whatever the count (DecodeOrder of the reference, kernel_matmul.rs:34-75).
+     * kernels whatever the count (DecodeOrder of the reference, kernel_matmul.rs:34-75); without it the order of a
+     * row's sums is that of the kernel its row count takes, so that its last bits may change with the count.
      * Returns LK_OK or an LK_ERR_* code; never throws, never aborts. */
     int forward(const void* x, int x_type, int rows, void* out, void* stream, bool decode_order = false);
 

@@ -38,12 +38,23 @@ bool tiled_serves(int dtype, int k) {
            k % 256 == 0;
 }
 
-// One or two rows in one launch, against the quantizer's launch and the mat-vec's (us): every workgroup quantizes the rows, which a matrix that keeps
-// the chip busy longer than the second launch costs pays for several times over. Two rows: 1024 x 4096 6.8 / 9.7, 4096 x 4096 Q4_K, Q6_K, Q8_0 7.0, 8.3, 7.9 / 9.8; 8192 x 4096 Q4_K,
-// Q5_K, Q6_K, Q8_0 7.9, 10.2, 11.2, 11.1 / 10.0, 14336 x 4096 Q4_K, Q8_0 9.6, 15.2 / 10.4, 13.3, 14336 x 2048 Q5_K, Q6_K, Q8_0 10.6, 11.9, 9.5 / 9.9, 10.5, 9.7; 1024 x 6144 7.8, 8.3, 9.6, 7.7 / 9.8, 2048 x 8192 8.2, 8.8, 10.2, 10.6 / 9.7,
-// 4096 x 8192 11.5, 12.6, 13.8, 13.3 / 10.0, 12288 x 6144 17.4, 19.4, 22.0, 20.2 / 12.8, 14.9, 17.4, 16.1. One row: up to 14336 x 4096 6.8 to
-// 11.1 / 9.6 to 12.8, 4096 x 8192 8.4, 8.8, 10.0, 10.0 / 9.9, 9.9, 10.0, 10.0, 12288 x 6144 12.5, 14.3, 16.2, 14.4 / 11.7, 13.3, 14.3, 15.3,
-// 28672 x 8192 25.8, 30.9, 38.5, 45.9 / 26.3, 31.5, 37.6, 46.0.
+// One or two rows quantized in the mat-vec launch, against the quantizer's launch and the mat-vec's: every workgroup quantizes the
+// rows, which a matrix that keeps the chip busy longer than the second launch costs pays for several times over. One launch / two
+// (us; one figure on the right: all formats alike):
+//   two rows         Q4_K          Q5_K          Q6_K          Q8_0
+//   1024 x 4096      6.8 / 9.7
+//   4096 x 4096      7.0 / 9.8                   8.3 / 9.8     7.9 / 9.8
+//   8192 x 4096      7.9 / 10.0    10.2 / 10.0   11.2 / 10.0   11.1 / 10.0
+//   14336 x 4096     9.6 / 10.4                                15.2 / 13.3
+//   14336 x 2048                   10.6 / 9.9    11.9 / 10.5   9.5 / 9.7
+//   1024 x 6144      7.8 / 9.8     8.3 / 9.8     9.6 / 9.8     7.7 / 9.8
+//   2048 x 8192      8.2 / 9.7     8.8 / 9.7     10.2 / 9.7    10.6 / 9.7
+//   4096 x 8192      11.5 / 10.0   12.6 / 10.0   13.8 / 10.0   13.3 / 10.0
+//   12288 x 6144     17.4 / 12.8   19.4 / 14.9   22.0 / 17.4   20.2 / 16.1
+//   one row          (up to 14336 x 4096 6.8 to 11.1 / 9.6 to 12.8)
+//   4096 x 8192      8.4 / 9.9     8.8 / 9.9     10.0 / 10.0   10.0 / 10.0
+//   12288 x 6144     12.5 / 11.7   14.3 / 13.3   16.2 / 14.3   14.4 / 15.3
+//   28672 x 8192     25.8 / 26.3   30.9 / 31.5   38.5 / 37.6   45.9 / 46.0
 bool pays_in_one_launch(int dtype, int n, int k, int rows) {
     const long long weights = (long long)n * k;
     if (rows == 1) return k <= 4096 || dtype == LK_TYPE_Q8_0 || weights <= (40ll << 20) || (dtype != LK_TYPE_Q6_K && weights >= (128ll << 20));
@@ -51,11 +62,19 @@ bool pays_in_one_launch(int dtype, int n, int k, int rows) {
     return weights <= (dtype == LK_TYPE_Q4_K || dtype == LK_TYPE_Q5_K ? 16ll << 20 : 12ll << 20);
 }
 
-// Nine to sixteen rows of Q8_0 and Q4_0 on the f16 tiles, operands straight from the rows, against the quantizer and two mat-vec
-// launches (Q4_0 from 16 rows or 48 M weights: int8 tiles). us, before / tiles: Q8_0 14336 x 4096 at 9 / 16 rows 32 / 39 against 30 / 30,
-// 4096 x 14336 45 / 65 against 36 / 36, 64000 x 2048 72 / 93 against 55 / 55, 11003 x 3072 at 9 / 12 / 16 24 / 26 / 29 against 26 / 26 / 26, 4096 x 4096 17.5 / 18.7 /
-// 21 against 19 / 19 / 19, 2048 x 2048 15.5 / 15.8 / 16.0 against 15.8 / 17.0 / 15.8; Q4_0 512 x 14336 at 9 / 12 30 / 38 against 24 / 25, 11003 x 3072 26 / 30 against 22 / 22,
-// 1024 x 4096 17.4 / 16.5 against 16.4 / 16.5, 4096 x 4096 17.5 / 18.6 against 17.7 / 17.0.
+// Nine to sixteen rows of Q8_0 and Q4_0 on the f16 tiles, operands straight from the rows, against what served them else: the
+// quantizer and two mat-vec launches, for Q4_0 from 16 rows or 48 M weights the int8 tiles. Those / f16 tiles (us):
+//                         9 rows        12 rows       16 rows
+//   Q8_0  14336 x 4096    32 / 30                     39 / 30
+//         4096 x 14336    45 / 36                     65 / 36
+//         64000 x 2048    72 / 55                     93 / 55
+//         11003 x 3072    24 / 26       26 / 26       29 / 26
+//         4096 x 4096     17.5 / 19     18.7 / 19     21 / 19
+//         2048 x 2048     15.5 / 15.8   15.8 / 17.0   16.0 / 15.8
+//   Q4_0  512 x 14336     30 / 24       38 / 25
+//         11003 x 3072    26 / 22       30 / 22
+//         4096 x 4096     17.5 / 17.7   18.6 / 17.0
+//         1024 x 4096     17.4 / 16.4   16.5 / 16.5
 bool few_rows_to_tiles(int dtype, int n, int k, int rows, const void* blob) {
     if (rows <= 8 || rows > 16 || n < 512 || k % 256 != 0 || ((uintptr_t)blob & 1) != 0) return false;
     const long long weights = (long long)n * k;
@@ -84,24 +103,34 @@ int matvec_rows(int dtype, int k) {
     return dtype == LK_TYPE_Q8_0 && tiled_serves(dtype, k) ? 16 : 8;
 }
 
-// Rows the matrix-unit rows kernels take before the tiled matmul does. A rows kernel reads the weights straight from HBM, once
-// for every 16 or 32 activation rows; its time steps up once its workgroups are more than the CUs. The f16 tiles cut K and read the weights
-// once per 32 to 128 rows. Measured on MI355X, quantizer included, rows kernel against f16 tiles (us), for matrices of 512 rows or more:
-//   Q4_K, 9 to 16 rows: 512 x 8192 10..11 / 16, 2048 x 8192 9..10 / 17..18, 8192 x 8192 14 / 22, 4096 x 14336 15..16 / 23, 10000 x 5120 18 / 21, 12000 x 10240 35..42 / 29; Q5_K alike
-//     17 to 32: 700 x 5120 18 / 15, 10000 x 5120 25 / 22, 2048 x 6144 21 / 16, 14336 x 4096 at 24 22 / 21; 4096 x 4096 16 / 16, 8192 x 4096 16 / 19
-//     above: 1024 x 4608 at 33 18 / 14, 1100 x 8192 at 33 / 64 26 / 18, 26 / 19; 3000 x 5120 at 33 / 96 20 / 18, 27 / 24; 4096 x 4096 at 64 / 96 (256, 384 workgroups) 17 / 20, 25 / 25; 1024 x 4096 at 200 / 400
-//     (224, 416) 19 / 21, 28 / 25; 2048 x 2048 at 200 17 / 19. Q5_K alike.
-//   Q6_K, 9 to 16 rows: 2048 x 8192 13 / 20, 6144 x 6144 20 / 24, 4096 x 14336 20 / 30, 3000 x 5120 12 / 18, 10000 x 5120 26 / 26
-//     17 to 32: 2048 x 14336 20 / 25, 8192 x 4096 17..19 / 23, 6144 x 6144 22..23 / 24..25, 700 x 11008 13 / 22; 10000 x 5120 30..33 / 27, 4096 x 14336 35 / 31,
-//     4096 x 8192 25 / 22
-//     33 to 64: 512 x 14336 17..18 / 26, 1024 x 14336 20..21 / 26, 2048 x 6144 19..20 / 20..22, 4096 x 4096 18..19 / 20..22; 2048 x 14336 34..36 / 27..29, 8192 x
-//     4096 26..29 / 25, 6144 x 3072 22 / 20..22. Above: 4096 x 4096 at 96 28 / 26, 1024 x 6144 23 / 22
-// `bench.py --workload rows-sweep` prints the table for a shape.
+// Rows the matrix-unit rows kernels take before the tiled matmul does. A rows kernel reads the weights straight from HBM, once for
+// every 16 or 32 activation rows; its time steps up once its workgroups (`items` above 32 rows, n / 16 up to 16) are more than the
+// CUs. The f16 tiles cut K and read the weights once per 32 to 128 rows. Whole calls of forward on MI355X, rows kernel / f16 tiles
+// (us; Q5_K like Q4_K):
+//                          9             16            24            32            64            128
+//   Q4_K  512 x 4096       5.7 / 12.2    5.7 / 12.9    14.9 / 13.0   16.0 / 13.2   16.0 / 13.9   16.6 / 15.7
+//         4096 x 4096      7.2 / 14.0    7.6 / 14.6    15.3 / 15.1   16.4 / 15.5   16.7 / 19.3   25.6 / 23.3
+//         8192 x 4096      9.5 / 17.5    9.8 / 18.0    16.0 / 19.4   17.2 / 20.4   26.0 / 23.0   40.2 / 29.8
+//         14336 x 4096     16.6 / 20.8   17.6 / 21.2   22.7 / 21.6   25.1 / 22.2   40.6 / 29.0   66.3 / 39.9
+//         2048 x 5120      7.6 / 13.6    7.7 / 14.3    17.3 / 14.8   18.3 / 15.1   18.6 / 18.1   19.4 / 21.4
+//         8192 x 8192      15.0 / 22.5   15.1 / 22.8   26.3 / 23.3   28.6 / 23.9   44.9 / 29.6   69.2 / 43.0
+//         14336 x 8192     29.5 / 28.6   35.5 / 29.7   37.1 / 30.1   41.8 / 30.9   68.5 / 41.4   118 / 67.4
+//         4096 x 14336     15.9 / 23.6   17.7 / 23.9   39.9 / 24.7   43.1 / 25.1   43.9 / 29.1   70.4 / 40.9
+//   Q6_K  1024 x 2048      4.8 / 14.1    4.7 / 14.2    6.5 / 14.5    6.6 / 14.4    7.4 / 14.7    14.1 / 15.7
+//         4096 x 4096      10.7 / 17.1   11.0 / 17.5   16.1 / 17.9   15.8 / 18.3   19.1 / 22.3   29.4 / 26.3
+//         8192 x 4096      16.2 / 22.7   17.0 / 22.8   19.0 / 23.5   20.2 / 23.9   29.9 / 25.5   46.3 / 36.5
+//         2048 x 5120      8.9 / 16.4    9.1 / 17.1    11.3 / 17.5   11.3 / 17.7   18.4 / 20.4   21.9 / 24.0
+//         14336 x 5120     30.8 / 32.6   32.1 / 33.4   35.0 / 33.8   37.2 / 34.4   57.2 / 41.4   98.0 / 61.1
+//         1024 x 8192      11.6 / 19.1   11.7 / 19.6   11.9 / 20.1   12.2 / 20.3   14.8 / 21.2   28.9 / 24.5
+//         8192 x 8192      27.0 / 29.8   28.0 / 30.3   29.9 / 31.0   32.3 / 31.4   51.4 / 37.6   82.5 / 54.8
+//         4096 x 14336     21.4 / 34.0   22.0 / 34.1   35.8 / 34.5   36.7 / 35.2   48.5 / 34.8   82.2 / 52.1
+// Of 810 such calls (512 to 14336 matrix rows of 2048 to 14336 values, 9 to 400 rows, the three formats) 43 are more than a
+// microsecond and 6 % behind the other side, by 4 at most: mostly Q4_K and Q5_K at 24 to 96 rows of 4096 values over few matrix rows.
 static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K) return false;
     if (rows <= 8) return true;
     const long long results = (long long)n * rows, weights = (long long)n * k;
-    // (few matrix rows yield few tiles whatever the cut: the int8 tiles' line)
+    // few matrix rows yield few tiles whatever the cut, and under 512 they are the int8 ones
     if (n < 512) return rows <= 16 || results * (k > 4096 ? k : 4096) <= 450000ll * 4096 * (n > 0 ? 2048 / n : 2048);
     const long long items = (n + 31ll) / 32 * ((rows + 31) / 32);
     if (dtype == LK_TYPE_Q6_K) {
@@ -117,14 +146,25 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     return items <= 256 || (k <= 2048 && results <= 450000);
 }
 
-// The K-quants at 3 to 8 f32 rows: the 16-row tiles of the matrix-unit kernels (their time hardly moves
-// with the row count) against mat-vec launches (whose dot work grows with every row). Up to 4096 values a row the rows kernel takes the rows
-// themselves, one launch where the mat-vec kernels need the quantizer's too, rows kernel / mat-vec at 3, 5, 8 rows: Q4_K 256 x 256 3.6, 3.7, 3.7 / 7.4, 9.3, 12.2; 2000 x
-// 1024 3.6 / 7.4, 9.3, 12.2; 256 x 2048 4.1 / 6.6, 8.1, 10.0; 8192 x 4096 7.6, 7.8, 7.9 / 9.9, 11.6, 14.1; Q6_K 1024 x 1024 4.0 / 7.9, 9.7, 12.6; 4096 x 4096 8.4, 8.3, 8.5 /
-// 8.9, 10.3, 12.1 (fewer than 256 matrix rows have not been moved: 64 x 1024 3.6 / 7.0, 9.0, 12.0, Q6_K 200 x 4096 7.0 / 6.5, 7.4, 8.8). Longer rows: measured on MI355X, mat-vec against rows kernel, quantizer included (us): Q4_K / Q5_K 4096 x 8192 at 4 / 5 / 8 rows 10.7, 11.7, 14.1 / 10.2,
-// 10.5, 10.0, 4096 x 14336 at 3 / 8 13.8, 24.0 / 13.5, 14.1, 8192 x 4096 at 4 / 5 10.8, 11.6 / 10.8, 10.1, 1024 x 14336 at 6 / 8 13.3, 15.5 / 12.0, 12.2; 2048 x 8192 at 8 10.8 / 9.8;
-// k = 2048: 2048 rows from 4, 6144 and 151936 from 3. Q6_K 4096 x 8192 at 5 / 6 13.1, 13.8 / 12.9, 12.9, 6144 x 2048 at 5 / 6 10.6, 11.5 / 10.0, 9.9, 1024 x 14336 at
-// 5 / 8 13.8, 22.1 / 14.6, 14.7, 700 x 5120 at 8 12.2 / 10.0, 512 x 4096 at 8 10.0 / 9.8, 4096 x 14336 at 3 / 4 16.6, 18.8 / 16.8, 16.8.
+// The K-quants at 3 to 8 rows: the 16-row tiles of the matrix-unit kernels, whose time hardly moves with the row count, against
+// mat-vec launches, whose dot work grows with every row. Up to 4096 values a row the rows kernel takes the rows themselves, one
+// launch where the mat-vec kernels need the quantizer's too. Rows kernel / mat-vec (us):
+//                          3 rows        5 rows        8 rows
+//   Q4_K  256 x 256        3.6 / 7.4     3.7 / 9.3     3.7 / 12.2
+//         2000 x 1024      3.6 / 7.4     3.6 / 9.3     3.6 / 12.2
+//         256 x 2048       4.1 / 6.6     4.1 / 8.1     4.1 / 10.0
+//         8192 x 4096      7.6 / 9.9     7.8 / 11.6    7.9 / 14.1
+//   Q6_K  1024 x 1024      4.0 / 7.9     4.0 / 9.7     4.0 / 12.6
+//         1024 x 4096      7.2 / 6.6     7.2 / 7.6     7.3 / 9.1
+//         4096 x 4096      8.4 / 8.9     8.3 / 10.3    8.5 / 12.1
+//         8192 x 4096      - / 11.7      13.7 / 13.6   13.9 / 16.9
+// (fewer than 256 matrix rows have not been moved: 64 x 1024 3.6 / 7.0, 3.7 / 9.0, 3.6 / 12.0; Q6_K 200 x 4096 7.0 / 6.5, 7.0 / 7.4, 7.1 / 8.8).
+// Longer rows, by way of the quantizer on both sides:
+//   Q4_K and Q5_K  2048 x 8192 at 8 rows 9.8 / 10.8; 4096 x 8192 at 4 / 5 / 8 10.2 / 10.7, 10.5 / 11.7, 10.0 / 14.1; 8192 x 4096 at 4 / 5
+//                  10.8 / 10.8, 10.1 / 11.6; 1024 x 14336 at 6 / 8 12.0 / 13.3, 12.2 / 15.5; 4096 x 14336 at 3 / 8 13.5 / 13.8, 14.1 / 24.0;
+//                  of 2048 values more than 16384 matrix rows from 3 (151936 x 2048)
+//   Q6_K           512 x 4096 at 8 9.8 / 10.0; 700 x 5120 at 8 10.0 / 12.2; 4096 x 8192 at 5 / 6 12.9 / 13.1, 12.9 / 13.8; 6144 x 2048 at 5 / 6
+//                  10.0 / 10.6, 9.9 / 11.5; 1024 x 14336 at 5 / 8 14.6 / 13.8, 14.7 / 22.1; 4096 x 14336 at 3 / 4 16.8 / 16.6, 16.8 / 18.8
 static bool small_rows_kernel_pays(int dtype, int n, int k, int rows) {
     if (rows < 3 || rows > 8 || k % 256 != 0 || (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K)) return false;
     const long long weights = (long long)n * k;
@@ -135,7 +175,7 @@ static bool small_rows_kernel_pays(int dtype, int n, int k, int rows) {
 }
 
 // Matrices whose 3 to 8 rows are refused as rows quantized beforehand, as they have been since the 16-row tiles took them over; the
-// smaller ones small_rows_kernel_pays names are served from Q8_1 rows too.
+// smaller ones of small_rows_kernel_pays are served from Q8_1 rows too.
 static bool large_for_few_rows(int dtype, int n, int k, int rows) {
     if (dtype == LK_TYPE_Q6_K) return k % 2048 == 0 && ((long long)n * k >= (48ll << 20) || (rows >= 7 && n >= 1024));
     return (long long)n * rows >= (k <= 2048 ? 8192 : 57344);
@@ -146,9 +186,9 @@ static bool fits_rows_kernel(int dtype, int k, const void* blob) {
     return k % 256 == 0 && ((uintptr_t)blob & (dtype == LK_TYPE_Q6_K ? 1 : 15)) == 0;
 }
 
-// Three to eight rows go to the rows kernels by the lines of the 16-row tiles, which take weights from a 16-byte boundary on. Q6_K weights off it (a
-// matrix that starts at some row of another one) would get the 32-row tiles: 3 / 8 rows, those / mat-vec: 2048 x 3840 13.6, 14.0 / 7.1, 10.2; 4096 x 8448
-// at 5 / 8 24.8, 25.3 / 18.4, 23.6; 256 x 1280 at 3 / 8 7.9, 8.1 / 7.4, 11.4.
+// Three to eight rows go to the rows kernels by the lines of the 16-row tiles, which take weights from a 16-byte boundary on. Q6_K
+// weights off it (a matrix that starts at some row of another one) would get the 32-row tiles. Those / mat-vec: 2048 x 3840 at 3 / 8
+// rows 13.6 / 7.1, 14.0 / 10.2; 4096 x 8448 at 5 / 8 24.8 / 18.4, 25.3 / 23.6; 256 x 1280 at 3 / 8 7.9 / 7.4, 8.1 / 11.4.
 static bool few_rows_to_kernel(int dtype, int n, int k, int rows, const void* blob) {
     return ((uintptr_t)blob & 15) == 0 && small_rows_kernel_pays(dtype, n, k, rows);
 }
@@ -191,7 +231,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
             const int nn[1] = {n_};
             return lk_mmvq_fused(dtype_, 1, vx, (const float*)x, k_, dst, x_type, k_, nn, rows, n_, nullptr, stream);
         };
-        const bool can_fuse = !plain && rows <= 2 && k_ <= 8192 && ((uintptr_t)x & (x_type == LK_TYPE_F32 ? 15 : 7)) == 0 && k_ % 4 == 0;
+        const bool can_fuse = !plain && rows <= 2 && k_ <= 8192 && k_ % 4 == 0 && ((uintptr_t)x & (x_type == LK_TYPE_F32 ? 15 : 7)) == 0;
         if (can_fuse && pays_in_one_launch(dtype_, n_, k_, rows)) return in_one_launch();
         const int k_padded = (int)pad_to((size_t)k_, 512), blocks = k_padded / 32;
         LkScratch scratch(stream);
@@ -261,10 +301,11 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     return LK_OK;
 }
 
-// takes_matvec of the reference (kernel_matmul.rs:1069-1075), for rows quantized beforehand: mat-vec counts of rows, but for the K-quants'
-// 3 to 8 rows over a large matrix (large_for_few_rows) and the formats with tiles from nibble_tiles_pay's row counts. Which launch serves the call
-// is forward's choice all the same (forward_quantized). Three products over one activation, forward three times / quantized once (us): Q4_K 4096 x 4096
-// at 4 / 8 rows 18.9, 18.8 / 17.1, 17.2; Q6_K 2048 x 3072 at 8 rows 17.3 / 15.8; Q8_0 4096 x 8192 at 16 81 / 83, 14336 x 4096 at 9 105 / 107.
+// takes_matvec of the reference (kernel_matmul.rs:1069-1075), for rows quantized beforehand: mat-vec counts of rows, but for the
+// K-quants' 3 to 8 rows over a large matrix (large_for_few_rows) and the formats with tiles from nibble_tiles_pay's row counts. Which
+// launch serves the call is forward's choice all the same (forward_quantized). Three products over one activation, forward three
+// times / quantized once (us): Q4_K 4096 x 4096 at 4 / 8 rows 18.9 / 17.1, 18.8 / 17.2; Q6_K 2048 x 3072 at 8 17.3 / 15.8; Q8_0 4096 x 8192
+// at 16 81 / 83, 14336 x 4096 at 9 105 / 107.
 bool QKernelMatMul::takes_quantized(int rows, bool decode_order) const {
     if (!blob_ || rows < 1) return false;
     if (decode_order && rows > 1) return true;

@@ -5,12 +5,12 @@
   gemv-4096   one Q4_K 4096x4096 mat-vec at one row, over rotating copies of the weight (more
               than twice the 256 MB last-level cache) and over one hot copy; the Q8_1 quantizer
               launch timed by itself and the two-launch call timed as a whole
-  mmq         the tiled int8-MFMA matmul: `--shape 2a` = 512 rows x 4096 -> 14336 in Q4_K,
+  mmq         the tiled matmul: `--shape 2a` = 512 rows x 4096 -> 14336 in Q4_K,
               `--shape 2b` = 2048 rows x 14336 -> 4096 in Q6_K; quantizer + matmul per step
   moe         one Qwen3-30B-A3B-shaped expert block (128 experts, 2048 -> 768 -> 2048, top-8,
               Q4_K) at `--tokens` rows, path chosen as the layer code chooses it
   decode-1p7b every quantized linear of a Qwen3-1.7B-shaped decode step at `--batch` rows:
-              mat-vec launches up to 8 rows, the tiled matmul above
+              mat-vec launches at one row, the rows kernels or the tiled matmul above
 
 Timing: 20 warm-up launches, then `--launches` (default 200) launches each bracketed by its own
 pair of events on the launch stream; median, p10, p90, min and max are reported (the protocol of
@@ -457,7 +457,7 @@ def decode_1p7b(args, dev):
     matvec = b <= 8
     used = {"rows": 0, "matvec": 0, "tiled": 0}
 
-    def rows_kernel_serves(wtype, n, k, rows):   # the rule of host_qmatmul.hip
+    def rows_kernel_serves(wtype, n, k, rows):   # this workload's own line above 16 rows (the host linear's, host_qmatmul.hip, is finer)
         if wtype != Q6K and 8 < rows <= 16 and k >= 8192 and n >= 2048:
             return False
         return rows <= 16 or n * rows * max(k, 4096) <= 450000 * 4096 * (2048 // max(n, 1) if n < 2048 else 1)
@@ -763,8 +763,8 @@ def brief_mmq(shape, launches=200):
 def rows_sweep(args, dev):
     """One weight matrix at a ladder of row counts: quantizer + matrix-unit rows kernel against
     quantizer + tiled matmul, each as a graph replay of the two launches, and the path the host
-    mirror of QKernelMatMul::forward takes. The crossover constants in host_qmatmul.hip come from
-    these tables."""
+    mirror of QKernelMatMul::forward takes. (Forward itself quantizes few rows in the rows kernel's launch
+    and writes the tiles' operands straight from the rows; its lines, host_qmatmul.hip, go by whole calls.)"""
     L = lib.load()
     wtype = {"q4_k": Q4K, "q5_k": WTYPES["q5_k"], "q6_k": Q6K}.get(args.wtype)
     if wtype is None:
