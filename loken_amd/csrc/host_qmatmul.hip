@@ -342,6 +342,8 @@ int QKernelMatMul::forward_quantized(const QuantizedActivation& a, void* out, vo
     last_path_ = Path::None;
     if (!a.q81 || !out) return LK_ERR_ARG;
     if (a.k != k_ || a.device != device_ || !takes_quantized(a.rows, decode_order)) return LK_NOT_TAKEN;
+    if (a.x_type != LK_TYPE_F32 && a.x_type != LK_TYPE_F16 && a.x_type != LK_TYPE_BF16) return LK_ERR_TYPE;   // (as every mat-vec launch)
+    if (((uintptr_t)a.q81 & 3) != 0) return LK_ERR_ARG;
     int current = -1;
     if (hipGetDevice(&current) != hipSuccess || current != device_) {
         (void)hipGetLastError();

@@ -468,6 +468,7 @@ def test_rows_quantized_beforehand_are_served_by_the_launches_of_forward(name, r
         assert l.lkh_qkernel_matmul_quantize_for_matvec(lin.h, x.data_ptr(), X_TYPES[xt], rows, q81.data_ptr(), s, 0) == 0
         assert l.lkh_qkernel_matmul_forward_quantized(lin.h, q81.data_ptr(), X_TYPES[xt], rows, out.data_ptr(), s, 0) == 0
         assert lin.path == expect and torch.equal(torch.nan_to_num(out), torch.nan_to_num(want))
+        assert l.lkh_qkernel_matmul_forward_quantized(lin.h, q81.data_ptr() + 2, X_TYPES[xt], rows, out.data_ptr(), s, 0) == lib.LK_ERR_ARG
         if not bad:
             pick = np.arange(0, n, 7)
             eps = 0.0 if xt == torch.float32 else 2.0 ** -8   # one rounding to the narrow type
