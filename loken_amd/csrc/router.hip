@@ -48,7 +48,7 @@ static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], floa
         sum += e < n_experts ? p[i] : 0.f;
     }
     sum = wave_sum(sum);
-    float picked_sum = 0.f, my_weight = 0.f;
+    float my_weight = 0.f;
     uint32_t my_id = 0;
     for (int j = 0; j < topk; ++j) {
         float best = p[0];
@@ -64,13 +64,16 @@ static __device__ __forceinline__ void select_topk_softmax(float (&p)[PER], floa
             const unsigned long long at = __ballot(p[i] == wanted);
             if (at) e = 64 * i + __ffsll((long long)at) - 1;
         }
-        const float prob = best / sum;
-        picked_sum += prob;
-        if (lane == j) { my_weight = prob; my_id = (uint32_t)e; }
+        if (lane == j) { my_weight = best; my_id = (uint32_t)e; }
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             if (lane + 64 * i == e) p[i] = -1.f;
     }
+    // the divisions of all choices at once, after the rounds that only depend on each other's maxima
+    my_weight /= sum;
+    float picked_sum = 0.f;
+    if (with_norm)
+        for (int j = 0; j < topk; ++j) picked_sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_weight), j));
     if (lane < topk) {
         weights[lane] = with_norm ? my_weight / picked_sum : my_weight;
         ids[lane] = my_id;
@@ -95,7 +98,7 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(const float* __restric
 
 // ---------------------------------------------------------------------------------------------
 // The gate product, softmax and top-k of every token (loken_gate_topk_softmax, cuda/moe/gate_topk.cu:253-295,
-// 366-403), in two launches: the logits as an f32 product on the matrix unit, then a wave per token that adds
+// 366-403), in two launches (a few tokens in one): the logits as an f32 product on the matrix unit, then a wave per token that adds
 // the partial sums and selects. One workgroup per token (the kernel after these, still the one for rows that do
 // not start on 16 bytes and for streams that record a graph before their scratch exists) reads the whole gate
 // for each token through one CU: 28 us at one token of 2048 x 128, where the bytes take a microsecond, and 69 us
@@ -109,16 +112,13 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(const float* __restric
 constexpr int LOGIT_WAVES = 4;
 constexpr int LOGIT_SPREAD = 768;   // workgroups a launch aims at: loads wait a microsecond each, so three per CU
 
-// Up to sixteen tokens: 16 x 16 tiles, rows straight from memory.
-__global__ __launch_bounds__(64 * LOGIT_WAVES) void gate_logits16_kernel(const float* __restrict__ x_in, const float* __restrict__ gate_w,
-                                                                         float* __restrict__ part, int hidden, int n_rows,
-                                                                         int n_experts) {
+// A wave's share of the product of a 16 x 16 tile, rows straight from memory: lane (group, column), register v: token 4 grp + v,
+// expert e0 + column.
+static __device__ __forceinline__ v4f logits16_share(const float* __restrict__ x_in, const float* __restrict__ gate_w, int hidden, int n_rows,
+                                                     int n_experts, int e0, int share, int shares) {
     constexpr int M = 16, UNIT = 16, AHEAD = 4;   // UNIT: values of K a load of the wave covers; AHEAD: loads per operand in flight
-    __shared__ __align__(16) float meet[LOGIT_WAVES - 1][M * M];
     const int lane = threadIdx.x & 63, at = lane % M, grp = lane / M;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int e0 = blockIdx.y * M;
-    const int units = (hidden + UNIT - 1) / UNIT, shares = gridDim.z * LOGIT_WAVES, share = blockIdx.z * LOGIT_WAVES + wave;
+    const int units = (hidden + UNIT - 1) / UNIT;
     const int u0 = (int)((int64_t)units * share / shares), u1 = (int)((int64_t)units * (share + 1) / shares);
     const float* xr = x_in + (size_t)min(at, n_rows - 1) * hidden;
     const float* wr = gate_w + (size_t)min(e0 + at, n_experts - 1) * hidden;
@@ -127,32 +127,126 @@ __global__ __launch_bounds__(64 * LOGIT_WAVES) void gate_logits16_kernel(const f
         float4 a[AHEAD], b[AHEAD];
         bool live[AHEAD];
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            // past the share (or the row's end, in its last unit): a repeat of the row's start, multiplied by zero
-            const int k = (u + i) * UNIT + 4 * grp;
-            live[i] = u + i < u1 && k < hidden;
-            a[i] = *(const float4*)(xr + (live[i] ? k : 0));
-            b[i] = *(const float4*)(wr + (live[i] ? k : 0));
-        }
+        for (int i = 0; i < AHEAD; ++i)
+            if (u + i < u1) {   // (the same for the whole wave: nothing is loaded past its share)
+                const int k = (u + i) * UNIT + 4 * grp;
+                live[i] = k < hidden;   // past the row's end, in its last unit: a repeat of the row's start, multiplied by zero
+                a[i] = *(const float4*)(xr + (live[i] ? k : 0));
+                b[i] = *(const float4*)(wr + (live[i] ? k : 0));
+            }
         __builtin_amdgcn_sched_barrier(0);   // all of them out before the first is waited for
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            if (!live[i]) a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].x, b[i].x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].y, b[i].y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].z, b[i].z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].w, b[i].w, acc, 0, 0, 0);
-        }
+        for (int i = 0; i < AHEAD; ++i)
+            if (u + i < u1) {
+                if (!live[i]) a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].x, b[i].x, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].y, b[i].y, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].z, b[i].z, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].w, b[i].w, acc, 0, 0, 0);
+            }
     }
+    return acc;
+}
+
+// Up to sixteen tokens.
+__global__ __launch_bounds__(64 * LOGIT_WAVES) void gate_logits16_kernel(const float* __restrict__ x_in, const float* __restrict__ gate_w,
+                                                                         float* __restrict__ part, int hidden, int n_rows,
+                                                                         int n_experts) {
+    constexpr int M = 16;
+    __shared__ __align__(16) float meet[LOGIT_WAVES - 1][M * M];
+    const int lane = threadIdx.x & 63, at = lane % M, grp = lane / M;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e0 = blockIdx.y * M;
+    v4f acc = logits16_share(x_in, gate_w, hidden, n_rows, n_experts, e0, blockIdx.z * LOGIT_WAVES + wave, gridDim.z * LOGIT_WAVES);
     if (wave > 0) *(v4f*)(meet[wave - 1] + lane * 4) = acc;
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
     for (int w = 0; w < LOGIT_WAVES - 1; ++w) acc += *(const v4f*)(meet[w] + lane * 4);
-    // lane (group, column), register v: token 4 grp + v, expert `at` of the tile
 #pragma unroll
     for (int v = 0; v < 4; ++v)
         if (4 * grp + v < n_rows && e0 + at < n_experts) part[((size_t)blockIdx.z * n_rows + 4 * grp + v) * n_experts + e0 + at] = acc[v];
+}
+
+// A few tokens: 16 x 16 tiles, rows straight from memory, the choice in the same launch. A workgroup is twice the four waves
+// that share a partial sum; the last one of the launch to arrive (its stream's counter, which wraps to zero with it)
+// reads all partial sums and gives a wave to each token. Its tail (the stores' way to memory, the counter, the partial sums, the choice:
+// 3 us) takes what the second launch takes, so what it saves is the host's time for that launch, which bounds a call of so little work: one to eight
+// tokens called one by one 11.0 -> 8.6 us. Replayed in a graph, one launch against two (128 experts of 2048, 1 / 4 / 8 / 16 tokens):
+// 6.1 / 6.2 / 7.1 / 10.4 us against 5.4 / 5.7 / 5.9 / 6.0; 128 of 3072 6.4 / 6.6 / 7.6 / 10.9 against 5.6 / 5.9 / 6.2 / 6.3. So up to
+// CHOICE_TOKENS tokens take it, outside a recording. Sums in the order of the two launches, hence the same bits.
+__device__ uint32_t g_arrived[LK_SCRATCH_TICKETS];
+constexpr int CHOICE_GROUPS = 2, CHOICE_THREADS = 64 * LOGIT_WAVES * CHOICE_GROUPS, CHOICE_TOKENS = 4;
+
+// FRESH: partial sums of other XCDs' workgroups of this launch, read past this XCD's cache.
+template <int PER, bool FRESH>
+static __device__ __forceinline__ void sum_partials(float (&p)[PER], const float* part, int splits, int64_t row, int n_rows, int n_experts, int lane) {
+    // partial sums in flight (one after the other they took 10 us of a one-token call, eight at a time a microsecond more than sixteen)
+    constexpr int AHEAD = PER <= 2 ? 16 : 8;
+    const int64_t step = (int64_t)n_rows * n_experts;
+    const float* from = part + row * n_experts;   // uniform: a load is a scalar base and the lane's offset
+    int at[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        at[i] = min(lane + 64 * i, n_experts - 1);
+        p[i] = 0.f;
+    }
+    for (int z0 = 0; z0 < splits; z0 += AHEAD) {
+        float v[AHEAD][PER];
+#pragma unroll
+        for (int z = 0; z < AHEAD; ++z) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) v[z][i] = FRESH ? __hip_atomic_load(from + at[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : from[at[i]];
+            if (z0 + z + 1 < splits) from += step;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int z = 0; z < AHEAD; ++z)
+#pragma unroll
+            for (int i = 0; i < PER; ++i) p[i] += z0 + z < splits ? v[z][i] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (lane + 64 * i >= n_experts) p[i] = -INFINITY;
+}
+
+template <int PER>
+__global__ __launch_bounds__(CHOICE_THREADS) void gate_topk16_kernel(const float* __restrict__ x_in, const float* __restrict__ gate_w,
+                                                                     float* part, float* __restrict__ weights, uint32_t* __restrict__ ids,
+                                                                     int hidden, int n_rows, int n_experts, int splits, int topk, int with_norm,
+                                                                     int ticket) {
+    constexpr int M = 16;
+    __shared__ __align__(16) float meet[CHOICE_THREADS / 64][M * M];
+    __shared__ int is_last;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e0 = blockIdx.x * M, z0 = blockIdx.y * CHOICE_GROUPS, share = z0 * LOGIT_WAVES + wave;
+    if (share < splits * LOGIT_WAVES)
+        *(v4f*)(meet[wave] + lane * 4) = logits16_share(x_in, gate_w, hidden, n_rows, n_experts, e0, share, splits * LOGIT_WAVES);
+    __syncthreads();
+    {   // register v of lane (group, column): token 4 grp + v, expert `at` of the tile
+        const int g = threadIdx.x / (M * M), i = threadIdx.x % (M * M), t = 4 * (i / 64) + i % 4, e = e0 + i / 4 % M, z = z0 + g;
+        if (z < splits && t < n_rows && e < n_experts) {
+            float sum = meet[LOGIT_WAVES * g][i];
+#pragma unroll
+            for (int w = 1; w < LOGIT_WAVES; ++w) sum += meet[LOGIT_WAVES * g + w][i];
+            __hip_atomic_store(part + ((size_t)z * n_rows + t) * n_experts + e, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    // Stores of agent scope go through the XCD's cache to where every XCD reads; once each wave has waited for its own, one thread
+    // counts the workgroup in.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t last = gridDim.x * gridDim.y - 1;
+        is_last = atomicInc(&g_arrived[ticket], last) == last;
+    }
+    __syncthreads();
+    if (!is_last) return;
+    if (wave >= n_rows) return;
+    float p[PER];
+    sum_partials<PER, true>(p, part, splits, wave, n_rows, n_experts, lane);
+    select_topk_softmax<PER>(p, weights + (size_t)wave * topk, ids + (size_t)wave * topk, n_experts, topk, with_norm, lane);
 }
 
 // More tokens: 32 x 32 tiles. Taken from memory in operand order (a lane per row) a load touches 32 cache lines
@@ -232,25 +326,7 @@ __global__ __launch_bounds__(256) void gate_select_kernel(const float* __restric
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= n_rows) return;
     float p[PER];
-#pragma unroll
-    for (int i = 0; i < PER; ++i) p[i] = 0.f;
-    constexpr int AHEAD = 8;   // partial sums in flight (one after the other they took 10 us of a one-token call)
-    for (int z0 = 0; z0 < splits; z0 += AHEAD) {
-        float v[AHEAD][PER];
-#pragma unroll
-        for (int z = 0; z < AHEAD; ++z)
-#pragma unroll
-            for (int i = 0; i < PER; ++i)
-                v[z][i] = part[((size_t)min(z0 + z, splits - 1) * n_rows + row) * n_experts + min(lane + 64 * i, n_experts - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int z = 0; z < AHEAD; ++z)
-#pragma unroll
-            for (int i = 0; i < PER; ++i) p[i] += z0 + z < splits ? v[z][i] : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-        if (lane + 64 * i >= n_experts) p[i] = -INFINITY;
+    sum_partials<PER, false>(p, part, splits, row, n_rows, n_experts, lane);
     select_topk_softmax<PER>(p, weights + row * topk, ids + row * topk, n_experts, topk, with_norm, lane);
 }
 
@@ -393,6 +469,7 @@ extern "C" void loken_gate_topk_softmax(const float* x_in, const float* gate_w, 
     if (!router_sizes_ok(n_rows, n_experts, n_expert_used)) return;
     hipStream_t s = (hipStream_t)stream;
     if (hidden % 4 == 0 && (((uintptr_t)x_in | (uintptr_t)gate_w) & 15) == 0) {
+        LkScratch scratch(s);
         const int m = n_rows <= 16 ? 16 : 32;
         const int t_tiles = (n_rows + m - 1) / m, e_tiles = (n_experts + m - 1) / m;
         // K split until the launch has LOGIT_SPREAD workgroups, while a wave keeps at least two units of K
@@ -401,9 +478,15 @@ extern "C" void loken_gate_topk_softmax(const float* x_in, const float* gate_w, 
         if (splits > units / (2 * LOGIT_WAVES)) splits = units / (2 * LOGIT_WAVES);
         if (splits > 16) splits = 16;
         if (splits < 1) splits = 1;
-        LkScratch scratch(s);
         float* part = (float*)scratch.get(LK_SCRATCH_ROUTER, (size_t)splits * n_rows * n_experts * 4);
         if (part) {
+            if (n_rows <= CHOICE_TOKENS && scratch.ticket() >= 0) {
+                auto choice = n_experts <= 64 ? gate_topk16_kernel<1> : n_experts <= 128 ? gate_topk16_kernel<2> : n_experts <= 256 ? gate_topk16_kernel<4> : gate_topk16_kernel<8>;
+                hipLaunchKernelGGL(choice, dim3(e_tiles, (splits + CHOICE_GROUPS - 1) / CHOICE_GROUPS), dim3(CHOICE_THREADS), 0, s, x_in, gate_w, part,
+                                   weights_out, ids_out, hidden, n_rows, n_experts, splits, n_expert_used, with_norm, scratch.ticket());
+                (void)hipGetLastError();
+                return;
+            }
             auto logits = m == 16 ? gate_logits16_kernel : gate_logits32_kernel;
             hipLaunchKernelGGL(logits, dim3(t_tiles, e_tiles, splits), dim3(64 * LOGIT_WAVES), 0, s, x_in, gate_w, part, hidden, n_rows,
                                n_experts);

@@ -46,6 +46,11 @@ class LkScratch {
     // asks for more of the same use), or kept until the release where a graph's nodes hold its address.
     void* get(LkScratchUse use, size_t bytes);
 
+    // A number below LK_SCRATCH_TICKETS that no other stream's scratch has: which of an array of counters in device memory a kernel
+    // may count its workgroups in. A launch finds its counter at zero and leaves it there. -1 where all are taken, and while the stream
+    // records a graph.
+    int ticket() const;
+
   private:
     hipStream_t stream_;
     std::shared_ptr<LkScratchPool> pool_;
@@ -54,6 +59,8 @@ class LkScratch {
 
 // Streams of a device with buffers of their own.
 constexpr int LK_SCRATCH_STREAMS = 32;
+// Streams' scratches with a counter of their own.
+constexpr int LK_SCRATCH_TICKETS = 4096;
 // What all recorded graphs of a device may hold together.
 constexpr size_t LK_SCRATCH_GRAPH_BYTES = (size_t)32 << 30;
 // The uses of the host linears, and those of everything else: each side gives back its own.

@@ -29,14 +29,26 @@ struct Owner {
 std::mutex g_mu;   // of what follows; taken inside a pool's lock, never around one
 std::vector<std::shared_ptr<LkScratchPool>>& g_streams = *new std::vector<std::shared_ptr<LkScratchPool>>;   // never destroyed: the
 std::vector<std::shared_ptr<LkScratchPool>>& g_graphs = *new std::vector<std::shared_ptr<LkScratchPool>>;    // process may end after its runtime
+std::vector<int>& g_tickets = *new std::vector<int>;   // given back
+int g_next_ticket = 0;
 
 }  // namespace
 
 struct LkScratchPool {
-    explicit LkScratchPool(const Owner& o) : owner(o) {}
-    ~LkScratchPool() {
+    explicit LkScratchPool(const Owner& o) : owner(o) {   // caller holds g_mu
+        if (o.recording) return;
+        if (!g_tickets.empty()) {
+            ticket = g_tickets.back();
+            g_tickets.pop_back();
+        } else if (g_next_ticket < LK_SCRATCH_TICKETS) {
+            ticket = g_next_ticket++;
+        }
+    }
+    ~LkScratchPool() {   // its kernels are over: a pool leaves the tables after the device was waited for
         free_blocks(take_blocks(EVERY_USE));
         if (last_use && hipEventDestroy(last_use) != hipSuccess) (void)hipGetLastError();
+        std::lock_guard<std::mutex> lock(g_mu);
+        if (ticket >= 0) g_tickets.push_back(ticket);
     }
 
     std::vector<Block> take_blocks(unsigned uses) {   // caller holds mu and g_mu, or has the last reference
@@ -64,6 +76,7 @@ struct LkScratchPool {
     }
 
     const Owner owner;
+    int ticket = -1;
     std::recursive_mutex mu;
     bool retired = false;   // out of the table: the stream's next call gets another one
     // written under mu and g_mu, so either is enough to read
@@ -197,6 +210,8 @@ void* LkScratch::get(LkScratchUse use, size_t bytes) {
     own = Block{fresh, want, use};
     return fresh;
 }
+
+int LkScratch::ticket() const { return pool_->ticket; }
 
 void lk_stream_scratch_release(int device, unsigned uses) {
     int current = 0;

@@ -210,6 +210,26 @@ static void threads_hold_what_they_use() {
     CHECK(fake::held() == 0);
 }
 
+static void a_counter_belongs_to_one_stream() {
+    static ihipStream_t many[LK_SCRATCH_STREAMS + 2];
+    std::map<int, int> seen;
+    for (int i = 0; i < LK_SCRATCH_STREAMS; ++i) {
+        const int t = LkScratch(&many[i]).ticket();
+        CHECK(t >= 0 && t < LK_SCRATCH_TICKETS && seen[t]++ == 0 && LkScratch(&many[i]).ticket() == t);
+    }
+    const int shared = LkScratch(&many[LK_SCRATCH_STREAMS]).ticket();   // one set of buffers, one counter, in order
+    CHECK(shared >= 0 && !seen[shared] && LkScratch(&many[LK_SCRATCH_STREAMS + 1]).ticket() == shared);
+    {
+        Recording r(&many[0], 5);
+        CHECK(LkScratch(&many[0]).ticket() == -1);
+    }
+    for (int i = 0; i < 2 * LK_SCRATCH_TICKETS; ++i) {                 // a release gives them back
+        take(&many[i % LK_SCRATCH_STREAMS], LK_SCRATCH_ROUTER, 10);
+        if (i % 7 == 6) lk_stream_scratch_release(-1, ~0u);
+    }
+    CHECK(LkScratch(&many[3]).ticket() >= 0);
+}
+
 int main(int argc, char** argv) {
     const struct { const char* name; void (*run)(); } cases[] = {
 #define CASE(f) {#f, f}
@@ -218,6 +238,7 @@ int main(int argc, char** argv) {
         CASE(an_outgrown_buffer_goes_unless_a_graph_has_it),
         CASE(a_release_frees_its_own_part), CASE(streams_past_the_bound_share_in_order),
         CASE(without_an_event_the_shared_buffers_wait_on_the_host), CASE(threads_hold_what_they_use),
+        CASE(a_counter_belongs_to_one_stream),
     };
     for (auto& c : cases) {
         if (argc < 2) puts(c.name);

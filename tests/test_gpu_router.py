@@ -119,3 +119,34 @@ def test_stable_sorts_match_numpy(n, experts, small):
     want_order = np.argsort(keys, kind="stable")
     assert np.array_equal(order.cpu().numpy().view(np.uint32), want_order.astype(np.uint32))
     assert np.array_equal(got.cpu().numpy().view(np.uint32), keys[want_order])
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,k", [(1, 2048, 128, 8), (4, 2048, 128, 8), (5, 512, 17, 2), (4, 132, 512, 64), (2, 8192, 60, 4), (3, 64, 200, 1)])
+def test_a_few_tokens_choose_alike_on_every_stream_and_in_graphs(tokens, hidden, experts, k):
+    # up to four tokens one launch, whose workgroups count themselves in a counter of the stream: whatever ran before, it is at zero;
+    # more tokens, and recorded calls, two launches with the same bits
+    x, gate = dev(synth.normal(31, 1, tokens * hidden).reshape(tokens, hidden)), dev(synth.normal(31, 2, experts * hidden).reshape(experts, hidden) * 0.05)
+    logits = x.double() @ gate.double().T
+    want_w, want_ids = moe.topk_softmax(logits.float(), k)
+    ranked = logits.softmax(1).sort(dim=1, descending=True).values
+    gap = (ranked[:, :k] - ranked[:, 1:k + 1]).min() if k < experts else (ranked[:, :-1] - ranked[:, 1:]).min()
+    first = moe.gate_topk_softmax(x, gate, k)
+    if gap > 1e-5 * ranked.max():
+        assert torch.equal(first[1], want_ids)
+    assert (first[0].sort(dim=1).values - want_w.sort(dim=1).values).abs().max() < 2e-5
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        recorded = moe.gate_topk_softmax(x, gate, k)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        graph.replay()
+        results = []
+        for s in streams:
+            with torch.cuda.stream(s):
+                results += [moe.gate_topk_softmax(x, gate, k), moe.gate_topk_softmax(x[:1], gate, k)]
+        torch.cuda.synchronize()
+        for w, ids in results:
+            assert torch.equal(w, first[0][:w.shape[0]]) and torch.equal(ids, first[1][:w.shape[0]])
+        assert torch.equal(recorded[0], first[0]) and torch.equal(recorded[1], first[1])
