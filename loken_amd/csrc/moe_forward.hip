@@ -62,8 +62,8 @@ int block_on_tiles(const Format& fg, const Format& fd, const float* x, const voi
     float* pairs = (float*)(base + pairs_at);
     const LkTokenOperands tokens_in = lk_operands_at(base + x_at, tokens, nb), h = lk_operands_at(base + h_at, rows, nb2);
 
-    if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, s)) return rc;
-    if (int rc = lk_operands_quantize(x, LK_TYPE_F32, tokens_in, hidden, tokens, s)) return rc;
+    const LkMoeRows quantized{x, tokens, hidden, nullptr, tokens_in};
+    if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, &quantized, s)) return rc;
     MmqProblem gu{(const uint8_t*)gate, nullptr, nullptr, nullptr, nb, hidden / fg.block_len, rows, 0, ffn, 0, 0};
     const MmqTileExperts first{bounds, src, (const uint8_t*)up, 0, stack_bytes(fg, ffn, hidden), longest, n_experts, &h};
     if (int rc = lk_mmq_tiles_moe(fg.type, gu, tokens_in, first, s)) return rc;
@@ -214,9 +214,9 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
         launch_mmq_quantize_q8_1_DS4(from, gather, to, LK_TYPE_F32, k, k, 0, 0, (k + 511) / 512 * 512, rows, 1, 1, stream);
     };
 
-    if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, s)) return rc;
+    const LkMoeRows quantized{x, tokens, hidden, y, {}};
+    if (int rc = lk_moe_route(choices, rows, topk, n_experts, nullptr, bounds, slots, src, rows_gu ? &quantized : nullptr, s)) return rc;
     if (rows_gu) {
-        if (int rc = lk_quantize_q8_1(x, LK_TYPE_F32, y, hidden, hidden, tokens, stream)) return rc;
         if (int rc = lk_moe_q4k_rows_grouped(gate, up, 0, y, hidden / 32, bounds, src, nullptr, h, ffn, n_experts,
                                              (int64_t)ffn * (hidden / 256) * Q4K_BYTES, ffn, hidden, longest, stream)) return rc;
     } else {

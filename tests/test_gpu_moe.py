@@ -611,6 +611,20 @@ def test_block_in_one_call_is_the_block_launch_by_launch(tokens, topk, n_experts
         assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
 
 
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,rows_gu", [(41, 2, 8, 768, 256, lib.TYPE_Q4_K, True), (9, 4, 16, 256, 256, lib.TYPE_Q5_K, False),
+                                                                        (67, 4, 32, 768, 256, lib.TYPE_Q5_K, False), (333, 1, 8, 1280, 512, lib.TYPE_Q6_K, False)])
+def test_tokens_that_start_between_pieces_give_the_block_of_aligned_ones(tokens, topk, n_experts, hidden, ffn, gu, rows_gu):
+    # the routing launch quantizes them too: rows of any number of 256-value blocks, from any float on
+    gate, up, down, x, ids, w = make_layer(tokens, hidden, ffn, n_experts, topk, 77, gu, dt_gu=gu)
+    path = lib.load().lk_moe_block_path(gu, gu, tokens, topk, n_experts, hidden, ffn)
+    assert bool(path & lib.MOE_ROWS_GATE_UP) == rows_gu and bool(path & (lib.MOE_TILES | lib.MOE_ROWS_GATE_UP))
+    args = [dev(a) for a in (gate, up, down, ids, w)]
+    want = moe.moe_forward(gu, gu, dev(x), *args, n_experts, ffn)
+    odd = torch.empty(x.size + 1, device="cuda")
+    odd[1:].copy_(dev(x).reshape(-1))
+    assert torch.equal(moe.moe_forward(gu, gu, odd[1:].view(tokens, hidden), *args, n_experts, ffn), want)
+
+
 @pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,dn,rows_gu", [
     (105, 2, 8, 512, 256, lib.TYPE_Q6_K, True), (115, 2, 8, 512, 256, lib.TYPE_Q6_K, False),   # longest run 36 / 39, down tiled
     (500, 4, 128, 2304, 256, lib.TYPE_Q4_K, False), (115, 2, 8, 2304, 256, lib.TYPE_Q4_K, True)])   # long rows: tiles fill the chip, or not
