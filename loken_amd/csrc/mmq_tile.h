@@ -742,19 +742,20 @@ static __device__ __forceinline__ void store_gated(const v16f& gate, const v16f&
 }
 
 // Workgroup id -> (n tile, K range, m tile): the m tiles of one n tile re-read the same weight rows, so they are issued back
-// to back on one XCD (ids are dealt round robin over the 8 XCDs). splits > 1: the tile over one of `splits` ranges of K, the
-// partial tile to part[range].
+// to back on one XCD (ids are dealt round robin over the 8 XCDs). Each XCD takes an eighth of all tiles in that order, give or take one: dealt
+// whole n tiles, those of 1213 rows, ten, left six XCDs with half the work of the other two. splits > 1: the tile over one of `splits`
+// ranges of K, the partial tile to part[range].
 template <class F, int TT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void tile_dense_kernel(MmqProblem pb, LkTokenOperands ops, int n_tiles,
                                                                                     int m_tiles, int splits, float* part) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int ROWS = 32 * WAVES;
-    const int xcd = blockIdx.x & 7;
-    int seq = blockIdx.x >> 3;
-    const int m_tile = seq % m_tiles;
-    seq /= m_tiles;
-    const int split = seq % splits, n_tile = (seq / splits) * 8 + xcd;
-    if (n_tile >= n_tiles) return;
+    const uint32_t xcd = blockIdx.x & 7, all = (uint32_t)n_tiles * m_tiles * splits;
+    if (blockIdx.x >> 3 >= all / 8 + (xcd < all % 8)) return;
+    uint32_t at = (blockIdx.x >> 3) + all / 8 * xcd + min(xcd, all % 8);
+    const int m_tile = at % m_tiles;
+    at /= m_tiles;
+    const int split = at % splits, n_tile = at / splits;
     if (splits > 1) {
         const int64_t kb0 = pb.nb * split / splits, kb1 = pb.nb * (split + 1) / splits;
         pb.w += kb0 * F::BYTES;
@@ -876,7 +877,7 @@ static int launch_dense(const MmqProblem& pb, const LkTokenOperands& ops, int sp
     auto kernel = tile_dense_kernel<F, TT, WAVES>;
     if (int rc = mmq_prepare_kernel(kernel, LDS)) return rc;
     const int n_tiles = (pb.n + 32 * WAVES - 1) / (32 * WAVES), m_tiles = (pb.m_end + 32 * TT - 1) / (32 * TT);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((n_tiles + 7) / 8 * 8 * m_tiles * splits)), dim3(64 * WAVES), LDS, s, pb, ops, n_tiles, m_tiles,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(((int64_t)n_tiles * m_tiles * splits + 7) / 8 * 8)), dim3(64 * WAVES), LDS, s, pb, ops, n_tiles, m_tiles,
                        splits, part);
     return lk_launch_status();
 }
