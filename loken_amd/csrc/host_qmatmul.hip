@@ -16,7 +16,6 @@ namespace {
 
 constexpr int Q81_BLOCK = 36;
 constexpr size_t MMQ_RECORD = 144;                      // bytes per 128 padded values per row
-constexpr size_t FIXUP_BYTES = 256u * 128u * 128u * 4u;  // kernel_matmul/mmq.rs:42
 
 size_t pad_to(size_t v, size_t m) { return (v + m - 1) / m * m; }
 
@@ -277,7 +276,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     const size_t k_padded = pad_to(pad_to((size_t)k_, 512), 128);
     const size_t ws_bytes = (size_t)rows * (k_padded / 128) * MMQ_RECORD + 128 * MMQ_RECORD;
     LkScratch scratch(stream);
-    void* fixup = scratch.get(LK_SCRATCH_FIXUP, FIXUP_BYTES);
+    void* fixup = scratch.get(LK_SCRATCH_FIXUP, MMQ_HOST_FIXUP_BYTES);
     if (!fixup) return LK_ERR_NOMEM;
     // The f16 tiles' operands straight from x where the product takes those tiles (Q6_K 4096 x 14336 at 2048 rows 527 ->
     // 502 us, Q4_K 14336 x 4096 at 512 rows 100 -> 96 against records in between); without memory for them, by way of the records.
@@ -359,7 +358,7 @@ int QKernelMatMul::forward_quantized(const QuantizedActivation& a, void* out, vo
     }
     if (!one_order && few_rows_to_tiles(dtype_, n_, k_, a.rows, blob_)) {
         LkScratch scratch((hipStream_t)stream);
-        void* fixup = scratch.get(LK_SCRATCH_FIXUP, FIXUP_BYTES);
+        void* fixup = scratch.get(LK_SCRATCH_FIXUP, MMQ_HOST_FIXUP_BYTES);
         const int width = fixup ? lk_mmq_tiles_linear_q8_1(dtype_, fixup, blob_, a.q81, blocks, a.x_type, out, k_, n_, a.rows, (hipStream_t)stream) : -1;
         if (width == 0) return LK_ERR_ARG;
         if (width > 0) {

@@ -89,38 +89,40 @@ const Tiles* tiles_of(int wtype) {
     return nullptr;
 }
 
-// What a launch takes, fitted to 3000 calls on MI355X (7 shapes of 2048 x 2048 to 14336 x 4096 and 4096 x 14336, 33 to 2048 rows,
-// every tile width with K whole and cut into 2 to 12 ranges; the fit is off by 3 to 4 %, the plan it picks takes 1 to 2 % longer than
-// the best one of the sweep). alone / full: nanoseconds an item (32 x 32 x 32 product) takes a SIMD with one workgroup on its CU or two, by token
-// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items. (Q8_ITEM, Q4_ITEM: Q8_0 and Q4_0, from
-// 14336 x 4096 at 33, 128 and 512 rows at every width.)
+// What a launch takes, fitted to 1300 shapes on MI355X (those of the benchmark's models and drawn ones of 512 to 16384 x 1024 to 14336, 12 to 2048 rows, each at
+// every tile width with K whole and cut into 2 to 8 ranges) for the plan it picks: 0.9 % longer in the mean than the best one of the sweep (the items' times
+// are what makes it pick well, no more: a plan of each kind measured alone gives others). alone /
+// full: nanoseconds an item (32 x 32 x 32 product) takes a SIMD with one workgroup on its CU or two, by token
+// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items. (As fitted to whole launches whose workgroups
+// were dealt unevenly to the XCDs, with K cut into even ranges only, the picks were 3.8 % behind.)
 struct ItemTimes {
     double alone[4], full[4], wide, start;
 };
-constexpr ItemTimes ONE_TERM = {{164, 105, 104, 89}, {129, 98, 87.5, 82.7}, 80, 0.6}, TWO_TERMS = {{263, 144, 159, 143}, {194, 134, 122.5, 118}, 0, 3.1},
-                    Q8_ITEM = {{340, 180, 178, 0}, {220, 148, 135, 0}, 0, 1.0}, Q4_ITEM = {{315, 170, 172, 142}, {190, 138, 121, 107}, 0, 1.0};
+constexpr ItemTimes ONE_TERM = {{164, 110, 119, 92.1}, {120, 91.5, 80.5, 75.8}, 72.3, 0.73}, TWO_TERMS = {{265, 150, 168, 139}, {241, 138, 128, 122}, 0, 1.73},
+                    Q8_ITEM = {{264, 159, 184, 0}, {259, 148, 123, 0}, 0, 2.81}, Q4_ITEM = {{240, 164, 167, 152}, {193, 144, 125, 101}, 0, 0.06};
 
 // The tile and the cut of K with the shortest estimated launch. Up to 2 * cus workgroups run at once, and a CU that holds two takes
-// nearly the time of a full chip; past that the rounds blur (0.6 of whole rounds, 0.4 of their share). A cut costs a launch and
-// its partial products, written, read and added.
-MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup) {
+// nearly the time of a full chip; past that the rounds blur (two thirds of whole rounds, one of their share). Of two workgroups on a CU with ranges
+// of unequal length not both are the longest: two thirds of it, one of the mean. A cut costs a launch and its
+// partial products, written, read and added.
+MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup, int64_t fixup_bytes) {
     const ItemTimes& t = f.type == LK_TYPE_Q6_K ? TWO_TERMS : f.type == LK_TYPE_Q8_0 ? Q8_ITEM : f.type == LK_TYPE_Q4_0 ? Q4_ITEM : ONE_TERM;
     const int cus = lk_device().cus;
     const int forced_tt = lk_tune_env("LK_TUNE_MMQ_TT"), forced_splits = lk_tune_env("LK_TUNE_MMQ_SPLITS");   // measurement runs
-    const int most = forced_splits < 0 ? 1 : std::min(mmq_splits_most(pb, fixup, true), 12);
+    const int most = forced_splits < 0 ? 1 : std::min(mmq_splits_most(pb, fixup, true, fixup_bytes), 12);
     MmqTilePlan best{f.tt_most, 4, 1};
     double least = 1e30;
     for (int tt = 1; tt <= f.tt_most; ++tt) {
         if (forced_tt > 0 && tt != forced_tt) continue;
         const int64_t tiles = ((pb.n + 127ll) / 128) * ((pb.m_end + 32ll * tt - 1) / (32 * tt));
         for (int splits = forced_splits > 0 ? std::min(forced_splits, most) : 1; splits <= most; ++splits) {
-            const double items = 8e-3 * tt * ((pb.nb + splits - 1) / splits);
-            const double one = t.start + items * t.alone[tt - 1], two = t.start + 2 * items * t.full[tt - 1];
+            const double longest = (double)((pb.nb + splits - 1) / splits), mean = (double)pb.nb / splits, block = 8e-3 * tt;   // blocks; thousands of items
+            const double one = t.start + block * longest * t.alone[tt - 1], two = t.start + 2 * block * (0.68 * longest + 0.32 * mean) * t.full[tt - 1];
             const int64_t groups = tiles * splits, rounds = groups / (2 * cus), rest = groups % (2 * cus);
             double us = rounds * two;
-            if (rest > 0) us += rest <= cus ? one : one + (two - one) * (0.55 + 0.45 * (rest - cus) / cus);
-            if (rounds > 0) us = 0.6 * us + 0.4 * two * groups / (2 * cus);
-            if (splits > 1) us += 2.2 + 0.13e-6 * (splits + 1) * pb.m_end * pb.n * 4;
+            if (rest > 0) us += rest <= cus ? one : one + (two - one) * (0.775 + 0.225 * (rest - cus) / cus);
+            if (rounds > 0) us = 0.663 * us + 0.337 * two * groups / (2 * cus);
+            if (splits > 1) us += 1.88 + 0.211e-6 * (splits + 1) * pb.m_end * pb.n * 4;
             if (us < least) least = us, best = {tt, 4, splits};
             if (forced_splits > 0) break;
         }
@@ -128,7 +130,7 @@ MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup) 
     if (t.wide > 0 && forced_splits <= 0 && (forced_tt <= 0 || forced_tt == 8)) {
         const int64_t tiles = ((pb.n + 255ll) / 256) * ((pb.m_end + 127ll) / 128), rest = tiles % cus;
         const double round = 64e-3 * pb.nb * t.wide;
-        if (round * (tiles / cus + (rest > 0 ? 0.85 + 0.15 * rest / cus : 0.0)) < least) best = {4, 8, 1};
+        if (round * (tiles / cus + (rest > 0 ? 0.947 + 0.053 * rest / cus : 0.0)) < least) best = {4, 8, 1};
     }
     return best;
 }
@@ -142,7 +144,7 @@ int64_t rows_of_pass(int64_t blocks) { return OPERANDS_CAP / (blocks * (LK_OPERA
 
 // The product in passes; fill(operands, first row, rows) launches what writes a pass's operands. Returns as lk_mmq_tiles_dense.
 template <class Fill>
-int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, Fill fill) {
+int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, int64_t fixup_bytes, Fill fill) {
     if ((uintptr_t)pb.w % f.align != 0 || (f.align != 16 && pb.n < 128)) return -1;
     // lane offsets inside a tile are 32-bit
     if (pb.row_blocks * f.unit * 256 > (int64_t)INT32_MAX || pb.m_begin != 0) return -1;
@@ -158,7 +160,7 @@ int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, 
         pass.m_end = std::min(per_pass, pb.m_end - m0);
         pass.dst = (float*)((uint8_t*)pb.dst + (int64_t)m0 * pb.ldd * (pb.out_type == LK_TYPE_F32 ? 4 : 2));
         const LkTokenOperands ops = lk_operands_at(buffer, pass.m_end, pb.nb);
-        const MmqTilePlan plan = plan_dense(f, pass, fixup);
+        const MmqTilePlan plan = plan_dense(f, pass, fixup, fixup_bytes);
         fill(ops, m0, pass.m_end);
         if (f.dense(pass, ops, plan, (float*)fixup, s) != LK_OK) return 0;
         if (plan.splits > 1 && lk_mmq_split_sum((const float*)fixup, plan.splits, pass, s) != LK_OK) return 0;
@@ -172,7 +174,7 @@ int run_dense(const Tiles& f, const MmqProblem& pb, hipStream_t s, void* fixup, 
 int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup) {
     const Tiles* f = tiles_of(wtype);
     if (!f || !f->dense || (uintptr_t)pb.y % 16 != 0) return -1;
-    return run_dense(*f, pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int rows) {
+    return run_dense(*f, pb, s, fixup, MMQ_FIXUP_BYTES, [&](const LkTokenOperands& ops, int m0, int rows) {
         hipLaunchKernelGGL(operands_from_records_kernel, dim3((unsigned)pb.nb, (unsigned)((rows + 31) / 32)), dim3(256), 0, s, pb.y, ops,
                            pb.rows_total, m0, rows);
     });
@@ -186,7 +188,7 @@ extern "C" int lk_mmq_f16_tiles(int wtype, int64_t n, int64_t rows) {
 int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {
     if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
-    return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
+    return run_dense(*tiles_of(wtype), pb, s, fixup, MMQ_HOST_FIXUP_BYTES, [&](const LkTokenOperands& ops, int m0, int count) {
         (void)lk_operands_quantize((const uint8_t*)x + (int64_t)m0 * k * (type == LK_TYPE_F32 ? 4 : 2), type, ops, k, count, s);
     });
 }
@@ -195,7 +197,7 @@ int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, const void* w, const void* 
                              hipStream_t s) {
     if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
-    return run_dense(*tiles_of(wtype), pb, s, fixup, [&](const LkTokenOperands& ops, int m0, int count) {
+    return run_dense(*tiles_of(wtype), pb, s, fixup, MMQ_HOST_FIXUP_BYTES, [&](const LkTokenOperands& ops, int m0, int count) {
         hipLaunchKernelGGL(operands_from_q8_1_kernel, dim3((unsigned)pb.nb, (unsigned)((count + 31) / 32)), dim3(256), 0, s,
                            (const uint8_t*)q8_1 + (int64_t)m0 * stride * Q81_BYTES, ops, stride, count);
     });
