@@ -123,8 +123,15 @@ int matvec_rows(int dtype, int k) {
 //         1024 x 8192      11.6 / 19.1   11.7 / 19.6   11.9 / 20.1   12.2 / 20.3   14.8 / 21.2   28.9 / 24.5
 //         8192 x 8192      27.0 / 29.8   28.0 / 30.3   29.9 / 31.0   32.3 / 31.4   51.4 / 37.6   82.5 / 54.8
 //         4096 x 14336     21.4 / 34.0   22.0 / 34.1   35.8 / 34.5   36.7 / 35.2   48.5 / 34.8   82.2 / 52.1
-// Of 810 such calls (512 to 14336 matrix rows of 2048 to 14336 values, 9 to 400 rows, the three formats) 43 are more than a
-// microsecond and 6 % behind the other side, by 4 at most: mostly Q4_K and Q5_K at 24 to 96 rows of 4096 values over few matrix rows.
+// Once the tiles were dealt evenly to the XCDs they took over (rows kernel / tiles):
+//   Q6_K, 17 to 32 rows, more than 2048 matrix rows of more than 4352 values, or past 20 M weights where the 16-row tiles have no
+//     granules: 3018 x 6144 at 27 28.3 / 19.6; 4708 x 5376 at 26 26.7 / 21.0; 2165 x 7424 at 21 21.1 / 19.0; 6412 x 3584 at 29 23.3 / 19.8
+//     (4145 x 4096 at 21 16.7 / 18.6; 2977 x 4352 at 31 16.5 / 18.1; 9054 x 1792 at 19 16.6 / 17.2; 1833 x 11264 at 24 18.3 / 22.8)
+//   Q6_K, 33 to 64 rows of fewer than 3072 values, past 320000 results: 9987 x 1536 at 36 23.9 / 18.5 (6621 x 1536 at 46 16.2 / 17.3)
+//   Q4_K and Q5_K, rows of 3328 to 4096 values, 17 to 32 over fewer than 4096 matrix rows, and more where there are at most 128 items:
+//     2077 x 3584 at 26 14.6 / 13.2; 962 x 3840 at 27 14.6 / 13.2; 627 x 4096 at 71 17.0 / 14.4; 1184 x 3584 at 58 14.8 / 13.4
+//     (5246 x 3840 at 28 15.6 / 16.0; 1462 x 3584 at 124 15.6 / 17.6)
+// Left where they were: Q6_K, 65 rows and more over fewer than 1024 matrix rows of 2560 to 5632 values (548 x 3584 at 154 23.0 / 17.4).
 static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K) return false;
     if (rows <= 8) return true;
@@ -134,14 +141,15 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     const long long items = (n + 31ll) / 32 * ((rows + 31) / 32);
     if (dtype == LK_TYPE_Q6_K) {
         if (rows <= 16) return k % 2048 == 0 || k < 4608 || n <= 12288;
-        if (rows <= 32) return weights <= (24ll << 20) || n <= 2048 || (k <= 6144 && weights <= (40ll << 20));
-        if (rows <= 64) return n <= 1024 || (k < 3072 ? results <= 450000 : k <= 6144 && weights <= (17ll << 20));
+        if (rows <= 32) return n <= 2048 || (k <= 4352 && weights <= (k % 2048 == 0 ? 40ll << 20 : 20ll << 20));
+        if (rows <= 64) return n <= 1024 || (k < 3072 ? results <= 320000 : k <= 6144 && weights <= (17ll << 20));
         if (k < 5632 && n < 1024 && rows > 128 && items <= 256) return true;
         return (k < 3072 || (n < 1024 && k < 4608)) && results <= 450000;
     }
     if (rows <= 16) return k < 7168 || n <= 8192;
-    if (k >= 4608) return k < 5632 && items > 128 && items <= 256 && rows > 32;
-    if (rows <= 32) return n < 12288 || k < 4096 || rows < 20;
+    if (k >= 3328 && rows > 32) return k < 5632 && items > 128 && items <= 256;
+    if (k >= 4608) return false;
+    if (rows <= 32) return (n < 12288 || k < 4096 || rows < 20) && (k < 3328 || k > 4096 || n >= 4096);
     return items <= 256 || (k <= 2048 && results <= 450000);
 }
 

@@ -548,3 +548,12 @@ def test_operands_straight_from_the_rows_are_those_of_the_records(name, rows, n,
     got = lin(x)
     assert lin.path == "tiled" and torch.equal(got, ops.mmq_forward(DT[name], w, x.clone(), n))
     lin.close()
+
+
+@pytest.mark.parametrize("name,n,k,rows,expect", [
+    ("q6_k", 2056, 4608, 17, "tiled"), ("q6_k", 2056, 4352, 32, "rows-on-matrix-unit"), ("q6_k", 8200, 2560, 17, "tiled"),
+    ("q6_k", 5200, 4096, 17, "rows-on-matrix-unit"), ("q6_k", 9700, 768, 33, "tiled"), ("q6_k", 9696, 768, 33, "rows-on-matrix-unit"),
+    ("q4_k", 4088, 3328, 17, "tiled"), ("q5_k", 4096, 3328, 17, "rows-on-matrix-unit"), ("q4_k", 600, 4096, 32, "tiled"),
+    ("q5_k", 520, 3328, 161, "tiled"), ("q4_k", 2080, 3328, 65, "rows-on-matrix-unit")])
+def test_the_lines_that_moved_to_the_tiles_dealt_evenly(name, n, k, rows, expect):
+    test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
