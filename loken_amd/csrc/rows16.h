@@ -20,10 +20,10 @@ struct LkRows16 {
 // True when the launch takes `size_m` activation rows of `nb` super-blocks (their codes fit in LDS).
 bool lk_rows16_serves(int size_m, int nb);
 int lk_rows16_launch(const LkRows16& a, bool dual, bool q5, hipStream_t stream);
-// The same (rows16_short.hip) for matrices of few row tiles: a tile to a workgroup, any number of super-blocks.
+// The same (rows16_short.hip) for matrices of few row tiles and up to 128 activation rows: any number of super-blocks.
 // Its sums do not depend on what else the launch holds, nor on `dual`, so all launches over a matrix choose by lk_rows16_short_pays.
 int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream);
-bool lk_rows16_short_pays(int m, int n, int nb);
+bool lk_rows16_short_pays(int m, int n, int nb, bool q5);
 // The short launch straight over the rows (one launch instead of two). -1: a call it does not serve.
 int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream);
 

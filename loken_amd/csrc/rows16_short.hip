@@ -1,4 +1,4 @@
-// Q4_K / Q5_K weights x at most sixteen Q8_1 activation rows where there are few 16-row tiles: the short launch of the
+// Q4_K / Q5_K weights x up to 128 Q8_1 activation rows, in sets of eight or sixteen, where there are few 16-row tiles: the short launch of the
 // 16-row family (rows16_core.h has the arithmetic's layout, rows16_mfma.hip the launches for many tiles).
 //
 // What bounds it: the o projection of a small model (2048 x 2048, 2.4 MB) is 128 row tiles. rows16_mfma.hip gives a workgroup of
@@ -19,7 +19,7 @@ using namespace rows16_direct;
 using rows16::TILE;
 using rows16::WFrag;
 
-constexpr int MAX_TOKS = 16;             // activation rows a launch serves
+constexpr int SET = 16;                  // activation rows a workgroup takes at most; more are sets over grid.y
 constexpr int GROUPS = 16;               // of a tile's super-blocks at most, each summed by one wave
 constexpr int PART_BYTES = 4 * 64 * 4;   // a wave's partial tile; the first one holds its scales until then, [8][TOKS] floats
 enum Out { F32, ANY, DUAL_F32, DUAL_Q81 };   // plain: f32 or p.out_type; act(gate) * up: f32 or the Q8_1 rows that the next linear reads
@@ -33,28 +33,29 @@ static __device__ __forceinline__ T pick3(const T (&a)[3], int i) { return i == 
 struct TileRef {
     int mat, tile;
 };
-// Tile i of workgroup `wg`'s NT: plain: of the matrices' tiles one after another; dual: gate and up of the same rows by turns.
+// Tile i of workgroup `wg`'s NT: plain: of the matrices' groups of NT tiles one after another (a matrix's last group may have tiles past its
+// rows, which store nothing); dual: gate and up of the same rows by turns.
 template <int OUT, int NT>
 static __device__ __forceinline__ TileRef tile_of(const LkRows16& p, int wg, int i) {
     if (OUT >= DUAL_F32) return {i & 1, wg * (NT / 2) + (i >> 1)};
-    int mat = 0, tile = wg * NT + i;
+    int mat = 0;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-        const int tiles = (p.n[m] + TILE - 1) / TILE;
-        if (mat == m && m + 1 < p.count && tile >= tiles) tile -= tiles, mat = m + 1;
+        const int groups = (p.n[m] + NT * TILE - 1) / (NT * TILE);
+        if (mat == m && m + 1 < p.count && wg >= groups) wg -= groups, mat = m + 1;
     }
-    return {mat, tile};
+    return {mat, wg * NT + i};
 }
 
 static __host__ __device__ constexpr int lds_bytes_for(int waves, int nt, bool q81, bool rows = false) {
-    return waves * (nt * PART_BYTES + (rows ? CODE_BYTES : 0)) + (q81 ? MAX_TOKS * nt / 4 * 32 * 4 : 0);
+    return waves * (nt * PART_BYTES + (rows ? CODE_BYTES : 0)) + (q81 ? SET * nt / 4 * 32 * 4 : 0);
 }
 
 // grid.x workgroups of NT row tiles each (one; two where one would be more workgroups than CUs, and for a gate and its up; four for
 // the 32 rows of a Q8_1 block), 64 * waves threads: wave w takes super-blocks w, w + waves, ... of every one of them, against one reading of the
 // activation.
 template <bool Q5, int TOKS, int OUT, int NT, int SRC>
-__global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows16 p, int n_tiles) {
+__global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows16 p, int groups) {
     static_assert(TOKS == 8 || TOKS == 16, "eight or sixteen activation rows");
     static_assert(SRC == Q81 || (TOKS == 8 && OUT <= ANY), "rows of values: eight at a time, dense");
     static_assert(NT == 1 || NT % 2 == 0, "tiles in turn through two sets of weight registers");
@@ -70,13 +71,20 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
     // code before and after (8192 x 14336 at 8 rows 19.1 us -> 17.5, 5000 x 12288 14.9 -> 12.4; sixteen rows with four tiles spill and go 7.5 -> 9.8)
     constexpr bool IN_ORDER = !T16 || (NT == 2 && !Q5);
     const int w_tile_row = IN_ORDER ? lane >> 2 : l16, w_piece = IN_ORDER ? lane & 3 : grp;
-    const uint8_t* w_base[NT];   // each tile's matrix, and the lane's row in it (past the last tile: of the last)
-    uint32_t w_row[NT];
+    const uint8_t* w_base[NT];   // each tile's matrix, and the lane's row in it (past the last row: the last)
+    // Sixteen rows with four tiles: a row's offset is made at each load from the matrix's (uniform) first row. Kept for the four tiles, they were what
+    // spilled 28 registers: 8192 x 4096 at 48 rows 26.8 us -> 17.7.
+    constexpr bool ROW_AT_LOAD = !DUAL && T16 && NT == 4;
+    uint32_t w_row[ROW_AT_LOAD ? 1 : NT];
+    int w_first = 0, w_last = 0;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-        const TileRef r = DUAL ? tile_of<OUT, NT>(p, blockIdx.x, i) : tile_of<OUT, 1>(p, min((int)blockIdx.x * NT + i, n_tiles - 1), 0);
+        // (the minimum, which changes nothing, keeps what follows apart from the results' tiles at the end: without it qwen's q + k + v at 8 rows
+        // takes 0.2 us longer)
+        const TileRef r = tile_of<OUT, NT>(p, NT == 1 ? min((int)blockIdx.x, groups - 1) : (int)blockIdx.x, i);
         w_base[i] = (const uint8_t*)to_gbytes(pick3(p.w, r.mat));
-        w_row[i] = (uint32_t)min(r.tile * TILE + w_tile_row, pick3(p.n, r.mat) - 1) * (uint32_t)(p.nb * Blk<Q5>::BYTES);
+        if (i == 0) w_first = r.tile * TILE, w_last = pick3(p.n, r.mat) - 1;
+        if (!ROW_AT_LOAD) w_row[i] = (uint32_t)min(r.tile * TILE + w_tile_row, pick3(p.n, r.mat) - 1) * (uint32_t)(p.nb * Blk<Q5>::BYTES);
     }
     const int tok = l16 & (TOKS - 1);
     // The activation is asked for in the order it lies in, a row's pieces by neighbouring lanes, and handed to the operand's lanes by a
@@ -123,7 +131,10 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
         for (int u = 0; u < LOADS; ++u) b.raw[u] = *(const u32x4_a4*)(y_codes + at + (T16 ? 4 * (u >> 1) + (u & 1) : 4 * u) * Q81_BYTES);
     };
     auto load_w = [&](WFrag& w, int i, int kb) {
-        const uint32_t at = w_row[i] + (uint32_t)(kb * Blk<Q5>::BYTES), at_q = at + 16 * w_piece;
+        int tile_row = w_tile_row;
+        if (ROW_AT_LOAD) asm volatile("" : "+v"(tile_row));   // (or the compiler makes the four before the loop)
+        const uint32_t row = ROW_AT_LOAD ? (uint32_t)min(w_first + TILE * i + tile_row, w_last) * (uint32_t)(p.nb * Blk<Q5>::BYTES) : w_row[i];
+        const uint32_t at = row + (uint32_t)(kb * Blk<Q5>::BYTES), at_q = at + 16 * w_piece;
         w.hdr = *(const uint4*)(w_base[i] + at);
         if (Q5) w.qh = *(const uint4*)(w_base[i] + (at + 16 * (w_piece & 1)) + 16);
         w.q[0] = *(const uint4*)(w_base[i] + at_q + Blk<Q5>::QS);
@@ -342,77 +353,111 @@ __global__ __launch_bounds__(64 * GROUPS, 1) void q4k_rows16_short_kernel(LkRows
 }
 
 template <bool Q5, int TOKS, int OUT, int NT, int SRC = Q81>
-int launch(const LkRows16& a, int tiles, hipStream_t stream) {
+int launch(const LkRows16& a, hipStream_t stream) {
     static const bool ok = hipFuncSetAttribute((const void*)q4k_rows16_short_kernel<Q5, TOKS, OUT, NT, SRC>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                lds_bytes_for(GROUPS, NT, OUT == DUAL_Q81, SRC != Q81)) == hipSuccess;
     if (!ok) return LK_ERR_ARG;
     const int steps = (a.nb + GROUPS - 1) / GROUPS, waves = (a.nb + steps - 1) / steps;   // as equal a share of super-blocks as they allow
-    const int per_wg = OUT >= DUAL_F32 ? NT / 2 : NT;
-    hipLaunchKernelGGL((q4k_rows16_short_kernel<Q5, TOKS, OUT, NT, SRC>), dim3((tiles + per_wg - 1) / per_wg, (a.m + TOKS - 1) / TOKS), dim3(64 * waves),
-                       lds_bytes_for(waves, NT, OUT == DUAL_Q81, SRC != Q81), stream, a, tiles);
+    constexpr int ROWS = (OUT >= DUAL_F32 ? NT / 2 : NT) * TILE;   // of a matrix, to a workgroup
+    int groups = 0;
+    for (int i = 0; i < (OUT >= DUAL_F32 ? 1 : a.count); ++i) groups += (a.n[i] + ROWS - 1) / ROWS;
+    const int sets = (a.m + TOKS - 1) / TOKS;
+    if (sets > 65535) return LK_ERR_ARG;
+    hipLaunchKernelGGL((q4k_rows16_short_kernel<Q5, TOKS, OUT, NT, SRC>), dim3(groups, sets), dim3(64 * waves),
+                       lds_bytes_for(waves, NT, OUT == DUAL_Q81, SRC != Q81), stream, a, groups);
     return lk_launch_status();
 }
 
-// Tiles to a workgroup: as many as bring the launch to a workgroup to the CU; past two of a matrix to the CU only up to eight rows (registers).
+template <bool Q5, int TOKS, int NT>
+int launch_plain(const LkRows16& a, hipStream_t stream) {
+    return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, NT>(a, stream) : launch<Q5, TOKS, ANY, NT>(a, stream);
+}
+
+// Tiles to a workgroup. Up to eight rows as many as bring the launch to a workgroup to the CU. With sets of sixteen rows a workgroup of one, two, four
+// tiles is there for 3.5, 4.8, 6.6 us of 2048 values, 4.5, 6.8, 9.6 of 4096, 7.5, 8.8, 13.4 of 6144, and each further one of its CU adds what the
+// fit below says, so the least of the three (Q5_K has no registers for four: 13 spilled, level with two; gate and up: as up to eight rows).
 template <bool Q5, int TOKS>
 int launch_out(const LkRows16& a, bool dual, int tiles, hipStream_t stream) {
-    const int cus = lk_device().cus;
+    const int cus = lk_device().cus, sets = (a.m + TOKS - 1) / TOKS;
     if constexpr (TOKS == 8) {
         if (tiles > 2 * cus) {
-            if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 8>(a, tiles, stream);
-            if (dual) return launch<Q5, TOKS, DUAL_F32, 8>(a, tiles, stream);
-            return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 4>(a, tiles, stream) : launch<Q5, TOKS, ANY, 4>(a, tiles, stream);
+            if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 8>(a, stream);
+            return dual ? launch<Q5, TOKS, DUAL_F32, 8>(a, stream) : launch_plain<Q5, TOKS, 4>(a, stream);
         }
     }
-    if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 4>(a, tiles, stream);
-    if (tiles > cus) {
-        if (dual) return launch<Q5, TOKS, DUAL_F32, 4>(a, tiles, stream);
-        return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 2>(a, tiles, stream) : launch<Q5, TOKS, ANY, 2>(a, tiles, stream);
-    }
-    if (dual) return launch<Q5, TOKS, DUAL_F32, 2>(a, tiles, stream);
-    return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, 1>(a, tiles, stream) : launch<Q5, TOKS, ANY, 1>(a, tiles, stream);
+    if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 4>(a, stream);
+    if (dual) return (int64_t)tiles * sets > cus ? launch<Q5, TOKS, DUAL_F32, 4>(a, stream) : launch<Q5, TOKS, DUAL_F32, 2>(a, stream);
+    if constexpr (TOKS == 8) return tiles > cus ? launch_plain<Q5, TOKS, 2>(a, stream) : launch_plain<Q5, TOKS, 1>(a, stream);
+    auto us = [&](int nt, float base, float block) {
+        const int64_t wgs = (int64_t)((tiles + nt - 1) / nt) * sets;
+        return base + block * (float)(a.nb * ((wgs + cus - 1) / cus));
+    };
+    const float one = us(1, 2.2f, 0.2f), two = us(2, 2.8f, 0.255f);
+    if constexpr (!Q5)
+        if (us(4, 3.4f, 0.435f) < (one < two ? one : two)) return launch_plain<Q5, TOKS, 4>(a, stream);
+    return two < one ? launch_plain<Q5, TOKS, 2>(a, stream) : launch_plain<Q5, TOKS, 1>(a, stream);
 }
 
 template <bool Q5, int OUT, int SRC>
 int launch_rows(const LkRows16& a, int tiles, hipStream_t stream) {
     const int cus = lk_device().cus;
-    return tiles > 2 * cus ? launch<Q5, 8, OUT, 4, SRC>(a, tiles, stream) : tiles > cus ? launch<Q5, 8, OUT, 2, SRC>(a, tiles, stream) : launch<Q5, 8, OUT, 1, SRC>(a, tiles, stream);
+    return tiles > 2 * cus ? launch<Q5, 8, OUT, 4, SRC>(a, stream) : tiles > cus ? launch<Q5, 8, OUT, 2, SRC>(a, stream) : launch<Q5, 8, OUT, 1, SRC>(a, stream);
 }
 
 }  // namespace
 
 int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
-    if (a.m < 1 || a.m > MAX_TOKS || a.nb < 1 || a.count < 1 || a.count > 3) return LK_ERR_ARG;
+    if (a.m < 1 || a.nb < 1 || a.count < 1 || a.count > 3) return LK_ERR_ARG;
     if ((dual && (a.count != 2 || a.n[0] != a.n[1])) || (a.q81_dst && (!dual || a.n[0] % 32 != 0 || a.q81_stride < a.n[0] / 32))) return LK_ERR_ARG;
     int tiles = 0;
     for (int i = 0; i < (dual ? 1 : a.count); ++i) tiles += (a.n[i] + TILE - 1) / TILE;
     if (tiles == 0) return LK_OK;
-    // more than eight rows: two sets of eight where both are resident at once (Q4_K 1024 x 2048 at 16 rows 4.2 us against 4.4 with sixteen)
-    const bool eight = a.m <= 8 || (!dual && 2 * tiles <= lk_device().cus);
+    // nine to sixteen rows: two sets of eight where both are resident at once (Q4_K 1024 x 2048 at 16 rows 4.2 us against 4.4 with sixteen)
+    const bool eight = a.m <= 8 || (a.m <= 16 && !dual && 2 * tiles <= lk_device().cus);
     if (eight) return q5 ? launch_out<true, 8>(a, dual, tiles, stream) : launch_out<false, 8>(a, dual, tiles, stream);
     return q5 ? launch_out<true, 16>(a, dual, tiles, stream) : launch_out<false, 16>(a, dual, tiles, stream);
 }
 
-// Matrices of up to four row tiles to the CU, two above eight rows: with more the launches that stage the activation once and walk many tiles are level
-// or ahead; above a tile to the CU rows of 2048 values or more. A choice by the matrix and the class of row counts alone, so that several
-// matrices in one launch carry the bits of one launch each, and not above sixteen rows, where a row carries the 32-row tiles' bits whatever rides with
-// it. Measured in a graph, Q4_K, us, staged launches against this:
+// Matrices of up to four row tiles to the CU, fewer or more by the class of row counts: beyond, the launches that stage the activation once and walk
+// many tiles are level or ahead; above a tile to the CU rows of 2048 values or more. A choice by the matrix and the class of row counts alone (up to
+// 8, 16, 32, 64, 96, 128), so that several matrices in one launch carry the bits of one launch each and a row carries the same bits whatever rides
+// with it in its class. Measured in a graph, Q4_K, us, staged launches against this:
 //   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.7, 3.7; 4096 x 4096 7.7, 8.1 / 5.1, 5.0; 4096 x 14336 17.9, 19.4 / 12.0, 11.9; 6144 x 2048 5.5, 5.5 / 4.9, 4.9;
 //                8192 x 4096 8.8, 9.1 / 7.3, 7.2; 5000 x 12288 16.7, 17.8 / 14.7, 15.0; 14336 x 4096 12.6, 13.3 / 10.6, 10.5; 8192 x 1024 4.2, 4.1 / 4.0, 4.2;
 //                18944 x 3584 (five to the CU) 14.1, 14.4 / 15.2, 15.4
 //   9 / 16 rows  2048 x 2048 5.9, 6.4 / 4.0, 3.9; 4096 x 4096 9.4, 10.2 / 5.6, 5.6; 2048 x 6144 12.1, 13.2 / 6.4, 6.4; 4096 x 14336 28.8, 32.2 / 13.6, 14.7;
 //                8192 x 4096 10.3, 11.0 / 7.9, 8.0; 5000 x 12288 25.9, 28.6 / 16.9, 16.9; 8192 x 1024 4.2, 4.3 / 4.9, 5.1; 14336 x 4096 14.4, 15.4 / 16.0, 16.6
+//   (with the weights from HBM, which the figures above have in a cache; in brackets gate and up to Q8_1 rows) 12288 x 2048 9.0, 9.7 / 7.9, 8.1 (12.6, 12.7 /
+//                11.1, 11.4); 24576 x 2048 13.4, 12.9 / 10.9, 11.3 (17.2, 16.7 / 15.6, 16.5); 9216 x 4096 14.1, 14.9 / 10.7, 11.6 (20.4, 21.3 / 19.5,
+//                20.8); 14336 x 4096 14.9, 15.7 / 11.4, 12.2 (20.7, 21.7 / 20.3, 21.8, and 1.2 more than that between a step's other launches);
+//                10240 x 8192 28.6, 34.6 / 18.9, 20.1; 28672 x 8192 48.6, 56.8 / 38.0, 40.1. Q5_K, four tiles to the CU, is level (16, 27 / 14, 29)
+// Above sixteen rows against the 32-row tiles, where a wave's share of a tile's super-blocks is a chain of matrix instructions and fix-up (1 us a super-
+// block) behind a table that is built first, on a chip that a layer's 64 to 400 tiles do not fill. Weights from HBM:
+//   17 / 32 rows    2048 x 2048 7.5, 8.4 / 4.1, 4.1 (13.0, 14.0 / 6.6, 6.7); 4096 x 4096 12.4, 13.9 / 7.4, 7.7 (21.7, 23.3 / 10.8, 11.6); 8192 x 4096
+//                   12.9, 14.7 / 10.7, 11.2 (22.1, 24.0 / 20.4, 20.5); 4096 x 14336 35.2, 39.4 / 18.0, 19.4; 12288 x 2048 11.5, 13.3 / 10.0, 10.1
+//                   (19.8, 22.9 / 15.1, 15.4); 14336 x 4096 18.7, 23.7 / 19.6, 20.0 (31.4, 38.6 / 38.2, 38.6)
+//   48 / 64         2048 x 2048 8.3, 8.4 / 5.1, 5.2; 4096 x 4096 13.3, 14.3 / 11.1, 11.1 (22.6, 23.8 / 19.2, 19.6); 8192 x 4096 20.6, 23.2 / 17.7, 19.3
+//                   (34.3, 37.9 / 29.2, 37.9); 14336 x 4096 34.1, 37.7 / 27.9, 35.7 (60.1, 65.7 / 55.5, 65.5); 32768 x 2048 34.9, 37.3 / 26.6, 33.1
+//   96 / 128        2048 x 2048 8.6, 8.7 / 6.7, 6.7; 4096 x 4096 21.1, 22.9 / 17.0, 19.0 (35.1, 37.5 / 27.9, 36.3); 8192 x 4096 34.3, 36.9 / 27.1, 35.0
+//                   (62.0, 64.6 / 55.3, 72.5); 14336 x 4096 51.2, 63.3 / 51.5, 60.1 (93.1, 118.6 / 99.3, 126.6)
+//   Q5_K, 32 / 64   2048 x 2048 8.8, 8.8 / 4.6, 5.8; 4096 x 4096 14.7, 15.1 / 9.3, 15.2 (24.8, 25.2 / 17.9, 30.2); 8192 x 2048 10.0, 14.2 / 9.2, 13.9 (16.3,
+//                   23.9 / 17.2, 28.3)
 // (Rows of up to 32768 values: longer ones are the other launches' to take or refuse.)
-bool lk_rows16_short_pays(int m, int n, int nb) {
+bool lk_rows16_short_pays(int m, int n, int nb, bool q5) {
     const int tiles = (n + TILE - 1) / TILE, cus = lk_device().cus;
-    return m >= 1 && m <= MAX_TOKS && !lk_rows16_off(m) && nb <= 128 && (tiles <= cus || (tiles <= (m <= 8 ? 4 : 2) * cus && nb >= 8));
+    if (m < 1 || lk_rows16_off(m) || nb > 128) return false;
+    if (m <= 16) return tiles <= cus || (nb >= 8 && tiles <= (m <= 8 ? 4 : q5 ? 2 : nb <= 8 ? 6 : nb <= 16 ? 3 : 8) * cus);
+    if (m > 128) return false;
+    if (q5) return (int64_t)tiles * (m <= 32 ? 2 : m <= 64 ? 4 : 8) <= 2 * cus;
+    if (nb <= 8) return tiles <= 16 * cus;
+    return tiles <= (m <= 32 ? 2 : m <= 64 ? 4 : m <= 96 ? 2 : 1) * cus;
 }
 
 // Up to eight rows of up to 4096 values (sixteen as two sets where both are resident at once), a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the
 // chip (2 us), and the host is through with one launch where it was with two: up to 8192 x 4096 9.4 us a call -> 6.8, 14336 x 4096 11.1 -> 9.4.
 int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream) {
     const int tiles = (a.n[0] + TILE - 1) / TILE;
-    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || !lk_rows16_short_pays(a.m, a.n[0], a.nb) || (a.m > 8 && 2 * tiles > lk_device().cus)) return -1;
+    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || a.m > 16 || !lk_rows16_short_pays(a.m, a.n[0], a.nb, q5) || (a.m > 8 && 2 * tiles > lk_device().cus)) return -1;
     if (a.x_type == LK_TYPE_F32) return q5 ? launch_rows<true, F32, ROWS_F32>(a, tiles, stream) : launch_rows<false, F32, ROWS_F32>(a, tiles, stream);
     if (a.x_type == LK_TYPE_F16) return q5 ? launch_rows<true, ANY, ROWS_F16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_F16>(a, tiles, stream);
     return q5 ? launch_rows<true, ANY, ROWS_BF16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_BF16>(a, tiles, stream);

@@ -783,7 +783,7 @@ int launch_any(const Args& a, hipStream_t stream) {
     r.count = DUAL ? 2 : 1;
     r.y = a.y; r.nb = a.nb; r.m = a.m; r.stride_y = a.stride_y; r.gelu = a.gelu;
     // few row tiles: each one's super-blocks over the waves of a workgroup (rows16_short.hip)
-    if (lk_rows16_short_pays(a.m, a.n, a.nb)) return lk_rows16_short(r, DUAL, Q5, stream);
+    if (lk_rows16_short_pays(a.m, a.n, a.nb, Q5)) return lk_rows16_short(r, DUAL, Q5, stream);
     if (a.m <= 16) {
         // 16-row tiles (rows16_mfma.hip): half the matrix-unit time per weight, twice the tiles
         if (lk_rows16_serves(a.m, a.nb) && !lk_rows16_off(a.m)) return lk_rows16_launch(r, DUAL, Q5, stream);
@@ -880,7 +880,7 @@ extern "C" void loken_dense_q4k_imma_m8_actmul(const void* gate, const void* up,
 // decode step): outputs[i] is [size_m, sizes_n[i]] f32. The reference issues one
 // loken_dense_q4k_imma_m8_plain per matrix (dense_q4k_imma_m8_matmul, src/inference/moe_cuda/dense/
 // imma.rs:82-135); the results equal those launches' bit for bit. One launch at any row count (the 16-row
-// tiles up to 16 rows, the 32-row tiles above); rows too long for the kernels' LDS tables fall back to one
+// tiles up to 16 rows, above them the short launch's sets or the 32-row tiles); rows too long for the kernels' LDS tables fall back to one
 // launch per matrix.
 extern "C" int lk_dense_q4k_rows_multi(const void* const* weights, float* const* outputs, const int* sizes_n, int count,
                                        const void* q8_1, int size_m, int size_k, int q5, void* stream) {
@@ -898,7 +898,7 @@ extern "C" int lk_dense_q4k_rows_multi(const void* const* weights, float* const*
         int rest_n[3], rest = 0;
         for (int i = 0; i < count; ++i) {
             if (sizes_n[i] <= 0) continue;
-            if (!lk_rows16_short_pays(size_m, sizes_n[i], nb)) {
+            if (!lk_rows16_short_pays(size_m, sizes_n[i], nb, q5 != 0)) {
                 rest_w[rest] = weights[i], rest_out[rest] = outputs[i], rest_n[rest++] = sizes_n[i];
                 continue;
             }
@@ -956,7 +956,7 @@ extern "C" int lk_dense_q4k_rows_multi(const void* const* weights, float* const*
 // Gate and up in one launch with the result handed on as Q8_1: q8_1_out[m][size_n / 32] blocks =
 // lk_quantize_q8_1(act(gate . x) * (up . x)), byte for byte, so the down projection of a layer reads it
 // without the f32 round trip and the quantizer launch in between (what lk_mmvq_pair_act_q8_1 is to the
-// mat-vec pair launch). Up to 16 rows the 16-row-tile kernels (few row tiles: rows16_short.hip), above them the 32-row tiles (a tile's rows are one block; any row length its tables hold). Up to 16 rows k is 2048 or 4096,
+// mat-vec pair launch). Up to 16 rows the 16-row-tile kernels, above them the 32-row tiles (a tile's rows are one block; any row length its tables hold), few row tiles at up to 128 rows rows16_short.hip. Up to 16 rows k is 2048 or 4096,
 // size_n a multiple of 32; anything else returns LK_ERR_ARG (take the f32 form and the quantizer). q5 != 0: Q5_K. No counterpart in the reference, whose dense_q4k_imma_m8_act_mul writes f32
 // (src/inference/moe_cuda/dense/imma.rs:320-400).
 extern "C" int lk_dense_q4k_rows_actmul_q8_1(const void* gate, const void* up, const void* q8_1, void* q8_1_out, int size_m,
@@ -974,7 +974,7 @@ extern "C" int lk_dense_q4k_rows_actmul_q8_1(const void* gate, const void* up, c
     r.count = 2;
     r.y = (const uint8_t*)q8_1; r.nb = nb; r.m = size_m; r.stride_y = size_k / 32; r.gelu = use_gelu ? 1 : 0;
     r.q81_dst = (uint8_t*)q8_1_out; r.q81_stride = size_n / 32;
-    if (lk_rows16_short_pays(size_m, size_n, nb)) return lk_rows16_short(r, true, q5 != 0, (hipStream_t)stream);
+    if (lk_rows16_short_pays(size_m, size_n, nb, q5 != 0)) return lk_rows16_short(r, true, q5 != 0, (hipStream_t)stream);
     if (size_m > 16) {   // the 32-row tiles: a tile's rows are one block
         Args a{(const uint8_t*)gate, (const uint8_t*)q8_1, nullptr, nb, size_n, size_m, size_k / 32, size_n,
                (const uint8_t*)up, use_gelu ? 1 : 0};

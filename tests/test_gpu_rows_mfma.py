@@ -258,6 +258,26 @@ def test_eight_rows_emit_the_exact_integers_on_crafted_inputs(m):
     assert np.array_equal(got.astype(np.int64), want) and np.array_equal(got, got.astype(np.int64))
 
 
+# one, two and four tiles to a workgroup, last sets of one row and of sixteen, a last group of tiles past the matrix's rows
+@pytest.mark.parametrize("wtype,m,k,n", [(Q4K, 16, 2048, 24560), (Q4K, 16, 8192, 10001), (Q4K, 17, 256, 1), (Q4K, 31, 768, 33), (Q4K, 64, 2048, 4100), (Q4K, 100, 2048, 8190), (Q4K, 64, 4096, 4120),
+                                         (Q4K, 17, 4096, 8190), (Q4K, 128, 1024, 4090), (Q4K, 48, 14336, 1000), (Q4K, 65, 32768, 40),
+                                         (lib.TYPE_Q5_K, 17, 256, 1), (lib.TYPE_Q5_K, 33, 1024, 200), (lib.TYPE_Q5_K, 64, 2048, 2000),
+                                         (lib.TYPE_Q5_K, 128, 4096, 1000)])
+def test_sets_of_sixteen_rows_carry_the_bits_of_launches_of_their_own(wtype, m, k, n):
+    """Sets of sixteen rows over the second grid axis (rows16_short.hip): the sums are a launch of each set's, plain and gated, and the first and
+    last rows of the matrix the oracle's."""
+    w = synth.weight(wtype, 64, k, seed=78).reshape(64, -1).repeat((n + 63) // 64, axis=0)[:n]
+    x = synth.activation(m, k, seed=78)
+    wd, xd, q5 = dev(w), dev(x), wtype != Q4K
+    got = ops.dense_q4k_rows(wd, xd, n, q5=q5)
+    gated = ops.dense_q4k_rows_actmul(wd, wd, xd, n, False, q5=q5)
+    for i in range(0, m, 16):
+        assert torch.equal(got[i:i + 16], ops.dense_q4k_rows(wd, xd[i:i + 16].contiguous(), n, q5=q5))
+        assert torch.equal(gated[i:i + 16], ops.dense_q4k_rows_actmul(wd, wd, xd[i:i + 16].contiguous(), n, False, q5=q5))
+    ends = np.unique(np.r_[0:min(n, 20), max(0, n - 20):n])
+    assert_close(got.cpu().numpy()[:, ends], oracle.ob_matmul(wtype, x, w[ends], len(ends)))
+
+
 @pytest.mark.parametrize("m", [1, 5, 8, 11, 16, 19, 32, 33, 70])
 @pytest.mark.parametrize("q5", [False, True])
 def test_three_matrices_in_one_launch_carry_the_single_launches_bits(m, q5):
