@@ -47,7 +47,7 @@ int lk_rows16_launch_experts(const LkRows16& a, const LkRows16Experts& m, int n_
 // multiple of 2048, rows whose codes do not fit in LDS, above 16 rows a matrix of more than 64 MB or of more 16-row tiles than CUs).
 int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                   hipStream_t stream, int out_type);
-// The same at up to 64 rows and any number of super-blocks where there are few row tiles (rows16_q6k_short.hip). -1: does not pay, or
+// The same at up to 128 rows and any number of super-blocks where there are few row tiles (rows16_q6k_short.hip). -1: does not pay, or
 // weights off a 16-byte boundary.
 int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                         hipStream_t stream, int out_type);

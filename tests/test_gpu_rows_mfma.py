@@ -278,6 +278,21 @@ def test_sets_of_sixteen_rows_carry_the_bits_of_launches_of_their_own(wtype, m, 
     assert_close(got.cpu().numpy()[:, ends], oracle.ob_matmul(wtype, x, w[ends], len(ends)))
 
 
+# two sets of sixteen rows to a workgroup with a second set of one row, of sixteen and of none, waves with no super-block of their own, odd phases
+@pytest.mark.parametrize("m,k,n", [(17, 4096, 4090), (32, 256, 4096), (26, 2816, 3000), (41, 6144, 2048), (64, 4352, 2040), (40, 14336, 1040), (96, 4096, 1300),
+                                   (73, 2048, 1000), (128, 5120, 1024), (65, 256, 16)])
+def test_q6k_sets_of_sixteen_rows_carry_the_bits_of_launches_of_their_own(m, k, n):
+    w = synth.weight(lib.TYPE_Q6_K, 64, k, seed=79).reshape(64, -1).repeat((n + 63) // 64, axis=0)[:n]
+    x = synth.activation(m, k, seed=79)
+    wd, xd = dev(w), dev(x)
+    got = ops.dense_q6k_rows(wd, xd, n)
+    for i in range(0, m, 16):
+        i = max(0, min(i, m - 9))   # (up to eight rows long granules are another launch's)
+        assert torch.equal(got[i:i + 16], ops.dense_q6k_rows(wd, xd[i:i + 16].contiguous(), n))
+    ends = np.unique(np.r_[0:min(n, 20), max(0, n - 20):n])
+    assert_close(got.cpu().numpy()[:, ends], oracle.ob_matmul(lib.TYPE_Q6_K, x, w[ends], len(ends)))
+
+
 @pytest.mark.parametrize("m", [1, 5, 8, 11, 16, 19, 32, 33, 70])
 @pytest.mark.parametrize("q5", [False, True])
 def test_three_matrices_in_one_launch_carry_the_single_launches_bits(m, q5):
