@@ -89,8 +89,8 @@ const Tiles* tiles_of(int wtype) {
     return nullptr;
 }
 
-// What a launch takes, fitted to 1300 shapes on MI355X (those of the benchmark's models and drawn ones of 512 to 16384 x 1024 to 14336, 12 to 2048 rows, each at
-// every tile width with K whole and cut into 2 to 8 ranges) for the plan it picks: 0.9 % longer in the mean than the best one of the sweep (the items' times
+// What a launch takes, fitted to 2200 shapes on MI355X (those of the benchmark's models and drawn ones of 512 to 16384 x 1024 to 14336, 9 to 2048 rows, each at
+// every tile width with K whole and cut into 2 to 12 ranges) for the plan it picks: 0.7 % longer in the mean than the best one of the sweep (the items' times
 // are what makes it pick well, no more: a plan of each kind measured alone gives others). alone /
 // full: nanoseconds an item (32 x 32 x 32 product) takes a SIMD with one workgroup on its CU or two, by token
 // tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items. (As fitted to whole launches whose workgroups
@@ -98,11 +98,12 @@ const Tiles* tiles_of(int wtype) {
 struct ItemTimes {
     double alone[4], full[4], wide, start;
 };
-constexpr ItemTimes ONE_TERM = {{164, 110, 119, 92.1}, {120, 91.5, 80.5, 75.8}, 72.3, 0.73}, TWO_TERMS = {{265, 150, 168, 139}, {241, 138, 128, 122}, 0, 1.73},
-                    Q8_ITEM = {{264, 159, 184, 0}, {259, 148, 123, 0}, 0, 2.81}, Q4_ITEM = {{240, 164, 167, 152}, {193, 144, 125, 101}, 0, 0.06};
+constexpr ItemTimes ONE_TERM = {{162, 111, 121, 93.8}, {137, 93.6, 82.2, 75.7}, 72.6, 0.357}, TWO_TERMS = {{239, 146, 166, 152}, {221, 140, 124, 122}, 0, 1.30},
+                    Q8_ITEM = {{265, 159, 181, 0}, {253, 149, 124, 0}, 0, 1.71}, Q4_ITEM = {{250, 164, 181, 146}, {216, 144, 125, 114}, 0, 0.0919};
 
 // The tile and the cut of K with the shortest estimated launch. Up to 2 * cus workgroups run at once, and a CU that holds two takes
-// nearly the time of a full chip; past that the rounds blur (two thirds of whole rounds, one of their share). Of two workgroups on a CU with ranges
+// nearly the time of a full chip; past that the rounds blur (two thirds of whole rounds, one of their share)
+// but for the start of each, without which Q6_K 9675 x 9728 at 23 rows was cut into ten (52 us; into six, the most that is one round, 42). Of two workgroups on a CU with ranges
 // of unequal length not both are the longest: two thirds of it, one of the mean. A cut costs a launch and its
 // partial products, written, read and added.
 MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup, int64_t fixup_bytes) {
@@ -117,12 +118,13 @@ MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup, 
         const int64_t tiles = ((pb.n + 127ll) / 128) * ((pb.m_end + 32ll * tt - 1) / (32 * tt));
         for (int splits = forced_splits > 0 ? std::min(forced_splits, most) : 1; splits <= most; ++splits) {
             const double longest = (double)((pb.nb + splits - 1) / splits), mean = (double)pb.nb / splits, block = 8e-3 * tt;   // blocks; thousands of items
-            const double one = t.start + block * longest * t.alone[tt - 1], two = t.start + 2 * block * (0.68 * longest + 0.32 * mean) * t.full[tt - 1];
+            const double one = t.start + block * longest * t.alone[tt - 1], two = t.start + 2 * block * (0.639 * longest + 0.361 * mean) * t.full[tt - 1];
             const int64_t groups = tiles * splits, rounds = groups / (2 * cus), rest = groups % (2 * cus);
             double us = rounds * two;
-            if (rest > 0) us += rest <= cus ? one : one + (two - one) * (0.775 + 0.225 * (rest - cus) / cus);
-            if (rounds > 0) us = 0.663 * us + 0.337 * two * groups / (2 * cus);
-            if (splits > 1) us += 1.88 + 0.211e-6 * (splits + 1) * pb.m_end * pb.n * 4;
+            if (rest > 0) us += rest <= cus ? one : one + (two - one) * (0.779 + 0.221 * (rest - cus) / cus);
+            if (rounds > 0) us = 0.655 * us + 0.345 * two * groups / (2 * cus);
+            us += 2.38 * (double)((groups - 1) / (2 * cus));
+            if (splits > 1) us += 1.85 + 0.227e-6 * (splits + 1) * pb.m_end * pb.n * 4;
             if (us < least) least = us, best = {tt, 4, splits};
             if (forced_splits > 0) break;
         }
@@ -130,7 +132,7 @@ MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup, 
     if (t.wide > 0 && forced_splits <= 0 && (forced_tt <= 0 || forced_tt == 8)) {
         const int64_t tiles = ((pb.n + 255ll) / 256) * ((pb.m_end + 127ll) / 128), rest = tiles % cus;
         const double round = 64e-3 * pb.nb * t.wide;
-        if (round * (tiles / cus + (rest > 0 ? 0.947 + 0.053 * rest / cus : 0.0)) < least) best = {4, 8, 1};
+        if (round * (tiles / cus + (rest > 0 ? 0.972 + 0.028 * rest / cus : 0.0)) < least) best = {4, 8, 1};
     }
     return best;
 }
