@@ -24,6 +24,7 @@ int lk_rows16_launch(const LkRows16& a, bool dual, bool q5, hipStream_t stream);
 // Its sums do not depend on what else the launch holds, nor on `dual`, so all launches over a matrix choose by lk_rows16_short_pays.
 int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream);
 bool lk_rows16_short_pays(int m, int n, int nb, bool q5);
+float lk_rows16_short_us(int m, int n, int nb, bool q5);   // about what it takes, us, above sixteen rows; -1: another launch's
 // The short launch straight over the rows (one launch instead of two). -1: a call it does not serve.
 int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream);
 

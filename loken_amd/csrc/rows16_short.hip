@@ -373,9 +373,24 @@ int launch_plain(const LkRows16& a, hipStream_t stream) {
     return a.out_type == LK_TYPE_F32 ? launch<Q5, TOKS, F32, NT>(a, stream) : launch<Q5, TOKS, ANY, NT>(a, stream);
 }
 
-// Tiles to a workgroup. Up to eight rows as many as bring the launch to a workgroup to the CU. With sets of sixteen rows a workgroup of one, two, four
-// tiles is there for 3.5, 4.8, 6.6 us of 2048 values, 4.5, 6.8, 9.6 of 4096, 7.5, 8.8, 13.4 of 6144, and each further one of its CU adds what the
-// fit below says, so the least of the three (Q5_K has no registers for four: 13 spilled, level with two; gate and up: as up to eight rows).
+// Time of a launch of sets of sixteen rows, us, with `nt` tiles to a workgroup: a workgroup of one, two, four tiles is there for 3.5, 4.8, 6.6 us of 2048
+// values, 4.5, 6.8, 9.6 of 4096, 7.5, 8.8, 13.4 of 6144, and each further one of its CU adds what the fit says. (Five to seven super-blocks take the time
+// of eight: waves come four to the CU. 14592 x 1280 at 64 rows 20.2 us with two tiles, 14592 x 2048 18.8.)
+float set_us(int nt, int tiles, int sets, int nb) {
+    const int cus = lk_device().cus;
+    const float base = nb <= 4 ? 1.6f + 1.2f * (float)(nt == 4 ? 3 : nt) : 1.6f + 0.6f * (float)(nt == 4 ? 3 : nt), block = nt == 1 ? 0.2f : nt == 2 ? 0.255f : 0.435f;
+    const int64_t wgs = (int64_t)((tiles + nt - 1) / nt) * sets;
+    return base + block * (float)((nb > 4 && nb < 8 ? 8 : nb) * ((wgs + cus - 1) / cus));
+}
+
+// Tiles to a workgroup of sets of sixteen: the least of the three (Q5_K has no registers for four: 13 spilled, level with two).
+int set_tiles(int tiles, int sets, int nb, bool q5) {
+    const float one = set_us(1, tiles, sets, nb), two = set_us(2, tiles, sets, nb);
+    if (!q5 && set_us(4, tiles, sets, nb) < (one < two ? one : two)) return 4;
+    return two < one ? 2 : 1;
+}
+
+// Tiles to a workgroup: up to eight rows as many as bring the launch to a workgroup to the CU, and so for a gate and its up.
 template <bool Q5, int TOKS>
 int launch_out(const LkRows16& a, bool dual, int tiles, hipStream_t stream) {
     const int cus = lk_device().cus, sets = (a.m + TOKS - 1) / TOKS;
@@ -388,14 +403,10 @@ int launch_out(const LkRows16& a, bool dual, int tiles, hipStream_t stream) {
     if (a.q81_dst) return launch<Q5, TOKS, DUAL_Q81, 4>(a, stream);
     if (dual) return (int64_t)tiles * sets > cus ? launch<Q5, TOKS, DUAL_F32, 4>(a, stream) : launch<Q5, TOKS, DUAL_F32, 2>(a, stream);
     if constexpr (TOKS == 8) return tiles > cus ? launch_plain<Q5, TOKS, 2>(a, stream) : launch_plain<Q5, TOKS, 1>(a, stream);
-    auto us = [&](int nt, float base, float block) {
-        const int64_t wgs = (int64_t)((tiles + nt - 1) / nt) * sets;
-        return base + block * (float)(a.nb * ((wgs + cus - 1) / cus));
-    };
-    const float one = us(1, 2.2f, 0.2f), two = us(2, 2.8f, 0.255f);
+    const int nt = set_tiles(tiles, sets, a.nb, Q5);
     if constexpr (!Q5)
-        if (us(4, 3.4f, 0.435f) < (one < two ? one : two)) return launch_plain<Q5, TOKS, 4>(a, stream);
-    return two < one ? launch_plain<Q5, TOKS, 2>(a, stream) : launch_plain<Q5, TOKS, 1>(a, stream);
+        if (nt == 4) return launch_plain<Q5, TOKS, 4>(a, stream);
+    return nt == 2 ? launch_plain<Q5, TOKS, 2>(a, stream) : launch_plain<Q5, TOKS, 1>(a, stream);
 }
 
 template <bool Q5, int OUT, int SRC>
@@ -449,8 +460,17 @@ bool lk_rows16_short_pays(int m, int n, int nb, bool q5) {
     if (m <= 16) return tiles <= cus || (nb >= 8 && tiles <= (m <= 8 ? 4 : q5 ? 2 : nb <= 8 ? 6 : nb <= 16 ? 3 : 8) * cus);
     if (m > 128) return false;
     if (q5) return (int64_t)tiles * (m <= 32 ? 2 : m <= 64 ? 4 : 8) <= 2 * cus;
+    // (five and six super-blocks: 14592 x 1280 at 48 / 64 / 128 rows 14.9, 15.3, 24.3 / 13.6, 19.5, 30.0; 8192 x 1280 8.5, 8.8, 13.7 / 8.5, 8.7, 19.0;
+    // with the quantizer 2767 x 1280 at 113 11.2 / 12.1)
+    if (nb == 5 || nb == 6) return (int64_t)tiles * (m <= 32 ? 2 : m <= 64 ? 4 : m <= 96 ? 6 : 8) <= (m <= 64 ? 12 : 4) * cus;
     if (nb <= 8) return tiles <= 16 * cus;
     return tiles <= (m <= 32 ? 2 : m <= 64 ? 4 : m <= 96 ? 2 : 1) * cus;
+}
+
+float lk_rows16_short_us(int m, int n, int nb, bool q5) {
+    if (m <= 16 || !lk_rows16_short_pays(m, n, nb, q5)) return -1.f;
+    const int tiles = (n + TILE - 1) / TILE, sets = (m + SET - 1) / SET;
+    return set_us(set_tiles(tiles, sets, nb, q5), tiles, sets, nb);
 }
 
 // Up to eight rows of up to 4096 values (sixteen as two sets where both are resident at once), a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the

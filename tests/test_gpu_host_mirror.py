@@ -551,9 +551,32 @@ def test_operands_straight_from_the_rows_are_those_of_the_records(name, rows, n,
 
 
 @pytest.mark.parametrize("name,n,k,rows,expect", [
-    ("q6_k", 2056, 4608, 17, "tiled"), ("q6_k", 2056, 4352, 32, "rows-on-matrix-unit"), ("q6_k", 8200, 2560, 17, "tiled"),
+    ("q6_k", 4112, 4608, 17, "tiled"), ("q6_k", 2056, 4352, 32, "rows-on-matrix-unit"), ("q6_k", 8200, 2560, 17, "tiled"),
     ("q6_k", 5200, 4096, 17, "rows-on-matrix-unit"), ("q6_k", 9700, 768, 33, "tiled"), ("q6_k", 9696, 768, 33, "rows-on-matrix-unit"),
-    ("q4_k", 4088, 3328, 17, "tiled"), ("q5_k", 4096, 3328, 17, "rows-on-matrix-unit"), ("q4_k", 600, 4096, 32, "tiled"),
-    ("q5_k", 520, 3328, 161, "tiled"), ("q4_k", 2080, 3328, 65, "rows-on-matrix-unit")])
+    ("q5_k", 4096, 3328, 17, "rows-on-matrix-unit"), ("q5_k", 520, 3328, 161, "tiled"), ("q4_k", 2080, 3328, 65, "rows-on-matrix-unit")])
 def test_the_lines_that_moved_to_the_tiles_dealt_evenly(name, n, k, rows, expect):
     test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
+
+
+@pytest.mark.parametrize("name,n,k,rows,expect", [
+    ("q4_k", 2986, 6144, 26, "rows-on-matrix-unit"), ("q4_k", 2064, 14336, 40, "rows-on-matrix-unit"), ("q4_k", 1030, 4096, 128, "rows-on-matrix-unit"),
+    ("q4_k", 1030, 5632, 128, "tiled"), ("q4_k", 14336, 5120, 64, "tiled"), ("q5_k", 3456, 5632, 19, "rows-on-matrix-unit"),
+    ("q5_k", 8208, 5632, 19, "tiled"), ("q6_k", 4096, 6144, 17, "rows-on-matrix-unit"), ("q6_k", 4097, 6144, 17, "tiled"),
+    ("q6_k", 2048, 6912, 48, "rows-on-matrix-unit"), ("q6_k", 2049, 6912, 48, "tiled"), ("q6_k", 1360, 4096, 96, "rows-on-matrix-unit"),
+    ("q6_k", 1361, 5632, 96, "tiled"), ("q6_k", 1024, 5632, 128, "rows-on-matrix-unit"), ("q5_k", 1152, 4864, 40, "rows-on-matrix-unit")])
+def test_the_lines_that_moved_to_sets_of_rows(name, n, k, rows, expect):
+    test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
+
+
+def test_q6k_weights_off_a_piece_keep_the_tiles_where_sets_of_rows_would_pay():
+    n, k, rows = 4000, 6144, 24
+    w, x = synth.weight(DT["q6_k"], 50, k, seed=98, stream=3).reshape(50, -1), synth.activation(rows, k, seed=98)
+    want = np.tile(oracle.ob_matmul(DT["q6_k"], x, w, 50), (1, n // 50))
+    flat = torch.zeros(n * w.shape[1] + 32, dtype=torch.uint8, device="cuda")
+    for shift, expect in ((0, "rows-on-matrix-unit"), (2, "tiled")):
+        blob = flat[shift:shift + n * w.shape[1]]
+        blob.view(n // 50, -1)[:] = dev(w).reshape(1, -1)
+        lin = Linear(DT["q6_k"], blob, n, k)
+        got, path = lin(dev(x)), lin.path
+        lin.close()
+        assert path == expect and close(got.cpu().numpy(), want)
