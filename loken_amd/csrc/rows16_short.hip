@@ -473,11 +473,16 @@ float lk_rows16_short_us(int m, int n, int nb, bool q5) {
     return set_us(set_tiles(tiles, sets, nb, q5), tiles, sets, nb);
 }
 
-// Up to eight rows of up to 4096 values (sixteen as two sets where both are resident at once), a super-block to a wave: every workgroup makes the codes again, in less time than a quantizer launch takes on the
-// chip (2 us), and the host is through with one launch where it was with two: up to 8192 x 4096 9.4 us a call -> 6.8, 14336 x 4096 11.1 -> 9.4.
+// Rows of up to 4096 values, a super-block to a wave: up to eight rows, and more as sets of eight where these are a workgroup to the CU, two of rows of up
+// to 2048 values, three of up to 1024. Every workgroup makes the codes again, in less time than a quantizer launch takes on the chip (2 us), and the host is
+// through with one launch where it was with two: up to 8192 x 4096 9.4 us a call -> 6.8, 14336 x 4096 11.1 -> 9.4. Above sixteen rows, called eagerly and on the
+// chip, with a quantizer / without: 690 x 3584 at 22 9.2, 7.0 / 6.7, 6.2; 806 x 1536 at 47 9.0, 6.2 / 6.6, 6.0; 536 x 512 at 89 9.0, 5.7 / 6.7, 4.4. Past
+// the lines the chip is behind: 1222 x 3328 at 28 9.5, 7.2 / 8.6, 8.7; 1120 x 2816 at 41 8.9, 6.8 / 7.6, 7.8.
 int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream) {
     const int tiles = (a.n[0] + TILE - 1) / TILE;
-    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || a.m > 16 || !lk_rows16_short_pays(a.m, a.n[0], a.nb, q5) || (a.m > 8 && 2 * tiles > lk_device().cus)) return -1;
+    if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || !lk_rows16_short_pays(a.m, a.n[0], a.nb, q5)) return -1;
+    if (a.m > 16 && a.n[0] < 512) return -1;   // (a call recorded with nothing reserved stays refused over the smallest matrices)
+    if (a.m > 8 && tiles * ((a.m + 7) / 8) > (a.nb <= 4 ? 3 : a.nb <= 8 ? 2 : 1) * lk_device().cus) return -1;
     if (a.x_type == LK_TYPE_F32) return q5 ? launch_rows<true, F32, ROWS_F32>(a, tiles, stream) : launch_rows<false, F32, ROWS_F32>(a, tiles, stream);
     if (a.x_type == LK_TYPE_F16) return q5 ? launch_rows<true, ANY, ROWS_F16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_F16>(a, tiles, stream);
     return q5 ? launch_rows<true, ANY, ROWS_BF16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_BF16>(a, tiles, stream);

@@ -358,6 +358,14 @@ def test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n,
     lin.close()
 
 
+# a workgroup to the CU, two, three and one more than that; last sets of one row and of eight
+@pytest.mark.parametrize("half", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name,n,k,rows", [("q4_k", 512, 4096, 64), ("q4_k", 511, 4096, 64), ("q5_k", 1030, 2304, 25), ("q4_k", 2040, 2048, 31), ("q5_k", 512, 1792, 97), ("q4_k", 768, 1024, 128),
+                                           ("q5_k", 2050, 768, 41), ("q4_k", 4090, 512, 17), ("q6_k", 640, 4096, 44), ("q6_k", 1360, 1024, 24), ("q6_k", 520, 768, 65)])
+def test_sets_of_eight_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n, k, rows, half):
+    test_a_few_rows_straight_into_the_launch_carry_the_quantizers_codes(name, n, k, rows, half)
+
+
 @pytest.mark.parametrize("half", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name,n,k,rows", [("q4_k", 260, 4096, 3), ("q5_k", 2030, 2048, 9), ("q6_k", 2050, 3072, 8), ("q6_k", 1030, 1024, 16),
                                            ("q4_k", 128, 1024, 12), ("q5_k", 17, 256, 9), ("q6_k", 255, 4096, 16)])
