@@ -123,6 +123,10 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
 //   Q4_K, whose short runs have the rows launch, from 20 rows (128 of 2048 -> 768 at 19 / 26 / 42 rows 123 / 128 / 152 against 117 / 145 / 202,
 //     64 of 1536 -> 1024 at 15 / 22 / 42 rows 64 / 66 / 82 against 59 / 81 / 138); from 9 where that launch reads rows of more than
 //     eight super-blocks and the tiles fill the chip (60 of 2560 -> 1280 at 7 / 9 / 17 / 26 rows 116 / 120 / 117 / 123 against 114 / 141 / 195 / 182)
+//     Rows of one, five to seven or more than eight super-blocks have no wave-per-tile launch (rows16_moe.hip) and go through the 32-row tiles: gate and up of such
+//     rows leave from 9 rows where down's are such too, from 13 up to 2048 values where down's are of two or three (8 of 1792 -> 512 at 19 rows 35 against 60, 8 of
+//     1536 -> 1536 at 16 41 / 58, 8 of 1792 -> 1280 at 12 40 / 50, 60 of 1792 -> 512 at 19 56 / 72, 128 of 1792 -> 1536 at 11 202 / 208; past the
+//     lines 60 of 1280 -> 1024 at 14 70 / 64, 8 of 2816 -> 512 at 14 41 / 36)
 // and with workgroups of 64 gate and up rows for a quarter of the CUs at least.
 static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int hidden, int ffn) {
     auto always = [](int type) { return type == LK_TYPE_Q5_K || type == LK_TYPE_Q8_0 || type == LK_TYPE_Q4_0; };
@@ -132,6 +136,8 @@ static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int 
     if (always(gu) || always(down)) return true;
     if (of_levels(gu) || of_levels(down)) return longest > 32 || n_experts < 60;
     if (gu == LK_TYPE_Q6_K && down == LK_TYPE_Q6_K) return longest > 22 || n_experts < 60;
+    auto wave_a_tile = [](int k) { return k == 512 || k == 768 || k == 1024 || k == 2048; };
+    if (gu == down && !wave_a_tile(hidden) && (wave_a_tile(ffn) ? longest >= 13 && hidden <= 2048 && ffn < 1024 : longest >= 9)) return true;
     return longest >= 20 || (longest >= 9 && hidden > 2048 && 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus);
 }
 

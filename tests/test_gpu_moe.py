@@ -611,6 +611,21 @@ def test_block_in_one_call_is_the_block_launch_by_launch(tokens, topk, n_experts
         assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
 
 
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,tiles", [(24, 2, 8, 1280, 1536, True), (12, 2, 8, 1280, 1536, False), (40, 2, 8, 1792, 512, True),
+                                                                    (24, 2, 8, 1792, 512, False), (40, 2, 8, 1280, 1024, False), (24, 2, 8, 2304, 1280, True),
+                                                                    (40, 2, 8, 1024, 1280, False)])
+def test_short_runs_of_rows_without_a_wave_a_tile_go_on_the_tiles(tokens, topk, n_experts, hidden, ffn, tiles):
+    # Q4_K blocks on both sides of the line, against the same tokens one at a time (a mat-vec per routed pair)
+    gate, up, down, x, ids, w = make_layer(tokens, hidden, ffn, n_experts, topk, 83, lib.TYPE_Q4_K, dt_gu=lib.TYPE_Q4_K)
+    path = lib.load().lk_moe_block_path(lib.TYPE_Q4_K, lib.TYPE_Q4_K, tokens, topk, n_experts, hidden, ffn)
+    assert bool(path & lib.MOE_TILES) == tiles
+    g, u, d, xd, idd, wd = (dev(a) for a in (gate, up, down, x, ids, w))
+    got = moe.moe_forward(lib.TYPE_Q4_K, lib.TYPE_Q4_K, xd, g, u, d, idd, wd, n_experts, ffn)
+    want = torch.cat([moe.moe_forward(lib.TYPE_Q4_K, lib.TYPE_Q4_K, xd[i:i + 1].contiguous(), g, u, d, idd[i:i + 1].contiguous(),
+                                      wd[i:i + 1].contiguous(), n_experts, ffn) for i in range(tokens)])
+    assert ((got - want).abs() <= 1e-3 * want.abs() + 1e-3 * want.abs().max()).all()
+
+
 @pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,rows_gu", [(41, 2, 8, 768, 256, lib.TYPE_Q4_K, True), (9, 4, 16, 256, 256, lib.TYPE_Q5_K, False),
                                                                         (67, 4, 32, 768, 256, lib.TYPE_Q5_K, False), (333, 1, 8, 1280, 512, lib.TYPE_Q6_K, False)])
 def test_tokens_that_start_between_pieces_give_the_block_of_aligned_ones(tokens, topk, n_experts, hidden, ffn, gu, rows_gu):
