@@ -141,6 +141,21 @@ static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int 
     return longest >= 20 || (longest >= 9 && hidden > 2048 && 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus);
 }
 
+// lk_moe_grouped_pays by the weights as well: the expert-batched launches take 28 to 50 us however little there is to read, a mat-vec per pair the time
+// of the pairs' matrices (`bytes`, of which the L2s and the last cache hold what other pairs read). Whole block, pairs / batched, us, 8 experts unless said, at
+// up to six rows each:
+//   Q4_K 1.77 MB an expert, 24 pairs 19.3 / 28.4; 2.65, 26 24.6 / 31.6; 1.99, 44 27.1 / 39.6; (3.32, 48 35.0 / 32.5); Q4_K and Q6_K 2.55, 22 25.6 / 38.8; 3.44,
+//   24 27.9 / 37.9; MXFP4 0.8 to 0.9 of the time under 100 MB; Q5_K under 80 MB 0.73; Q8_0 under 250 MB 0.64 to 0.75
+// and where there is much to read the batched ones pay sooner: Q5_K from 1.25 rows past 300 MB (0.87 of the time over eight blocks), Q8_0 from
+// 2.25 past 400 (0.85 over eight).
+static bool grouped_pays_over(int64_t pairs, int n_experts, int line, int64_t bytes) {
+    const int64_t experts = n_experts > 1 ? n_experts : 1, mb = 1000000;
+    if (pairs <= 6 * experts && bytes < (line == LK_TYPE_Q8_0 ? 250 : line == LK_TYPE_Q5_K ? 80 : 100) * mb) return false;
+    if (line == LK_TYPE_Q5_K && 4 * pairs >= 5 * experts && bytes > 300 * mb) return true;
+    if (line == LK_TYPE_Q8_0 && 4 * pairs >= 9 * experts && bytes > 400 * mb) return true;
+    return lk_moe_grouped_pays(pairs, n_experts, line);
+}
+
 // Which launches the block is made of: LK_MOE_GROUPED (expert-batched products; else a mat-vec per routed pair),
 // and in it LK_MOE_TILES (both products on the f16 tiles), or LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN
 // (lk_moe_q4k_rows_grouped; else the tiled launch). The one place that decides: lk_moe_forward and a caller that issues the
@@ -154,7 +169,8 @@ extern "C" int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int t
     if (!fg || !fd || tokens <= 0 || topk <= 0 || n_experts <= 0) return 0;
     auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K; };
     const int line = wtype_gu == wtype_down ? wtype_gu : has_tiles(wtype_gu) && has_tiles(wtype_down) ? LK_TYPE_Q6_K : -1;
-    if (!lk_moe_grouped_pays((int64_t)tokens * topk, n_experts, line) || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
+    const int64_t pairs = (int64_t)tokens * topk;
+    if (!grouped_pays_over(pairs, n_experts, line, pairs * (2 * stack_bytes(*fg, ffn, hidden) + stack_bytes(*fd, hidden, ffn))) || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
     if (block_takes_tiles(wtype_gu, wtype_down, longest, n_experts, hidden, ffn)) return LK_MOE_GROUPED | LK_MOE_TILES;
     const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);

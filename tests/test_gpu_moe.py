@@ -611,6 +611,22 @@ def test_block_in_one_call_is_the_block_launch_by_launch(tokens, topk, n_experts
         assert torch.equal(moe_forward(*args), moe_forward(*args, return_rows=True)[0])
 
 
+@pytest.mark.parametrize("gu,dn,tokens,topk,n_experts,hidden,ffn,grouped", [
+    (lib.TYPE_Q4_K, lib.TYPE_Q4_K, 12, 2, 8, 2048, 512, False), (lib.TYPE_Q4_K, lib.TYPE_Q4_K, 24, 2, 8, 2048, 1024, True), (lib.TYPE_Q4_K, lib.TYPE_Q6_K, 11, 4, 8, 2048, 1024, True),
+    (lib.TYPE_Q4_K, lib.TYPE_Q4_K, 25, 2, 8, 512, 256, True), (lib.TYPE_Q5_K, lib.TYPE_Q5_K, 10, 8, 64, 3072, 1536, True), (lib.TYPE_Q5_K, lib.TYPE_Q5_K, 10, 8, 64, 1024, 1024, False),
+    (lib.TYPE_Q8_0, lib.TYPE_Q8_0, 20, 8, 64, 1536, 768, True), (lib.TYPE_Q8_0, lib.TYPE_Q8_0, 12, 4, 8, 2048, 768, False)])
+def test_the_pairs_or_the_batch_by_the_weights_too(gu, dn, tokens, topk, n_experts, hidden, ffn, grouped):
+    # both sides of the lines by the bytes of the pairs' matrices, against the same tokens one at a time
+    # (rows small enough that the f16 scale of a Q8_1 block holds every product)
+    gate, up, down, x, ids, w = make_layer(tokens, hidden, ffn, n_experts, topk, 84, dn, x_scale=3.0, dt_gu=gu)
+    assert bool(lib.load().lk_moe_block_path(gu, dn, tokens, topk, n_experts, hidden, ffn) & lib.MOE_GROUPED) == grouped
+    g, u, d, xd, idd, wd = (dev(a) for a in (gate, up, down, x, ids, w))
+    got = moe.moe_forward(gu, dn, xd, g, u, d, idd, wd, n_experts, ffn)
+    want = torch.cat([moe.moe_forward(gu, dn, xd[i:i + 1].contiguous(), g, u, d, idd[i:i + 1].contiguous(), wd[i:i + 1].contiguous(), n_experts, ffn)
+                      for i in range(tokens)])
+    assert ((got - want).abs() <= 1e-3 * want.abs() + 1e-3 * want.abs().max()).all()
+
+
 @pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,tiles", [(24, 2, 8, 1280, 1536, True), (12, 2, 8, 1280, 1536, False), (40, 2, 8, 1792, 512, True),
                                                                     (24, 2, 8, 1792, 512, False), (40, 2, 8, 1280, 1024, False), (24, 2, 8, 2304, 1280, True),
                                                                     (40, 2, 8, 1024, 1280, False)])
@@ -626,7 +642,7 @@ def test_short_runs_of_rows_without_a_wave_a_tile_go_on_the_tiles(tokens, topk, 
     assert ((got - want).abs() <= 1e-3 * want.abs() + 1e-3 * want.abs().max()).all()
 
 
-@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,rows_gu", [(41, 2, 8, 768, 256, lib.TYPE_Q4_K, True), (9, 4, 16, 256, 256, lib.TYPE_Q5_K, False),
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,gu,rows_gu", [(41, 2, 8, 768, 256, lib.TYPE_Q4_K, True), (27, 4, 16, 256, 256, lib.TYPE_Q5_K, False),
                                                                         (67, 4, 32, 768, 256, lib.TYPE_Q5_K, False), (333, 1, 8, 1280, 512, lib.TYPE_Q6_K, False)])
 def test_tokens_that_start_between_pieces_give_the_block_of_aligned_ones(tokens, topk, n_experts, hidden, ffn, gu, rows_gu):
     # the routing launch quantizes them too: rows of any number of 256-value blocks, from any float on
