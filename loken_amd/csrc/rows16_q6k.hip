@@ -441,7 +441,7 @@ int launch(const Args& a, hipStream_t stream, int sets = 1) {
 
 int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                   hipStream_t stream, int out_type) {
-    if (size_m < 1 || size_m > 32 || size_n < 1 || size_k < 256) return -1;
+    if (size_m < 1 || size_m > 16 || size_n < 1 || size_k < 256) return -1;
     // rows of whole granules, on 16-byte boundaries; a tile's granules within one workgroup
     if (size_k % (256 * GRAN) != 0 || size_k / (256 * GRAN) > MAX_WAVES || (((uintptr_t)w) & 15) != 0) return -1;
     if (lk_rows16_off(size_m)) return -1;
@@ -457,17 +457,12 @@ int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, in
         const int rc = 2 * n_tiles <= lk_device().cus || weight_bytes <= ((size_t)22 << 20) ? -1 : launch<8>(a, stream);
         return rc != -1 ? rc : launch<4>(a, stream, 2);   // (eight rows too long for LDS: the sums four or fewer of them have)
     }
-    // 9..32 rows. Sixteen at once when their codes fit LDS and the row tiles are several to the CU; else the
+    // 9..16 rows. Sixteen at once when their codes fit LDS and the row tiles are several to the CU; else the
     // rows in sets of eight, a set per workgroup (grid.y), in one launch: rows too long for sixteen in LDS (k =
-    // 14336: 229 KB), up to two tiles to the CU, where twice the workgroups with half the staging each
+    // 14336: 229 KB), or up to two tiles to the CU, where twice the workgroups with half the staging each
     // finish sooner (16 rows: 8192 x 2048 10.4 us against 13.2, 8192 x 4096 14.5 against 15.7; 11008 x 4096 28.2 against 23.8 and 14336 x
-    // 4096 27.2 against 25.7 stay with sixteen at once), or 17..32 rows (4096 x 4096 13.8 against 17.4 on the 32-row tiles, 4096 x 8192
-    // 24.8 against 31.1). Every set reads the weights again, from L2 while they fit there, and three or four sets of more than a
-    // tile to the CU are too many workgroups: above 16 rows a matrix of more than 64 MB or of more tiles
-    // than CUs stays with the 32-row tiles (at 32 rows 151936 x 2048 173 us against 99, 6144 x 4096 25.8
-    // against 18.4, 14336 x 4096 39.7 against 32.4).
-    if (size_m > 16 && (n_tiles > lk_device().cus || weight_bytes > ((size_t)64 << 20))) return -1;
-    if (size_m <= 16 && n_tiles > 2 * lk_device().cus) {
+    // 4096 27.2 against 25.7 stay with sixteen at once). Every set reads the weights again, from L2 while they fit there.
+    if (n_tiles > 2 * lk_device().cus) {
         const int rc = launch<16>(a, stream);
         if (rc != -1) return rc;
     }
