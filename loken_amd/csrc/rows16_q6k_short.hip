@@ -152,8 +152,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         return u32x4{__builtin_amdgcn_alignbyte(lo[1], lo[0], sh), __builtin_amdgcn_alignbyte(lo[2], lo[1], sh),
                      __builtin_amdgcn_alignbyte(lo[3], lo[2], sh), __builtin_amdgcn_alignbyte(past, lo[3], sh)};
     };
-    u32x4 ql, qhp;
-    auto codes_of = [&](int unit, uint32_t sh) {   // the lane's sixteen signed codes: group 4 unit + grp of the row (units in turn)
+    auto codes_of = [&](int unit, uint32_t sh, u32x4& ql, u32x4& qhp) {   // the lane's sixteen signed codes: group 4 unit + grp of the row (units in turn)
         uint32_t past;
         if (unit % 2 == 0) {
             ql = piece_at(32 * unit + 16 * grp, sh, past);
@@ -242,10 +241,11 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
         }
         const uint32_t sh = (my_at + (uint32_t)(kb * Q6K_BYTES)) & 2u;
         uint32_t past;
+        u32x4 ql, qhp;
         const u32x4 sc = piece_at(192, sh, past);
         const float d = f16_bits_to_f32((past >> (8 * sh)) & 0xFFFFu);
 #pragma unroll
-        for (int unit = 0; unit < 4; ++unit) unit_of(unit, act, codes_of(unit, sh), d, sc[unit]);
+        for (int unit = 0; unit < 4; ++unit) unit_of(unit, act, codes_of(unit, sh, ql, qhp), d, sc[unit]);
         settle();
     };
 
@@ -265,13 +265,14 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
             load_w(w, next);
             const uint32_t sh = (my_at + (uint32_t)(kb * Q6K_BYTES)) & 2u;
             uint32_t past;
+            u32x4 ql, qhp;
             const u32x4 sc = piece_at(192, sh, past);
             const float d = f16_bits_to_f32((past >> (8 * sh)) & 0xFFFFu);
             u32x4 act[SETS][4];
 #pragma unroll
             for (int i = 0; i < SETS; ++i) turn(act_of[i], act[i]), load_act(act_of[i], i, next);
 #pragma unroll
-            for (int unit = 0; unit < 4; ++unit) unit_of(unit, act, codes_of(unit, sh), d, sc[unit]);
+            for (int unit = 0; unit < 4; ++unit) unit_of(unit, act, codes_of(unit, sh, ql, qhp), d, sc[unit]);
             settle();
         }
     } else if constexpr (SRC != Q81) {   // one in flight (registers)
