@@ -106,7 +106,7 @@ int matvec_rows(int dtype, int k) {
 // Rows the matrix-unit rows kernels take before the tiled matmul does. A rows kernel reads the weights straight from HBM, once for
 // every 16 or 32 activation rows; its time steps up once its workgroups (`items` above 32 rows, n / 16 up to 16) are more than the
 // CUs. The f16 tiles cut K and read the weights once per 32 to 128 rows. Whole calls of forward on MI355X, rows kernel / f16 tiles
-// (us; Q5_K like Q4_K):
+// (us; Q5_K like Q4_K; above sixteen rows with the 32-row tiles, before the sets below):
 //                          9             16            24            32            64            128
 //   Q4_K  512 x 4096       5.7 / 12.2    5.7 / 12.9    14.9 / 13.0   16.0 / 13.2   16.0 / 13.9   16.6 / 15.7
 //         4096 x 4096      7.2 / 14.0    7.6 / 14.6    15.3 / 15.1   16.4 / 15.5   16.7 / 19.3   25.6 / 23.3
@@ -148,6 +148,7 @@ static bool sets_of_rows_pay(int dtype, int n, int k, int rows, const void* blob
     if (rows < 17 || rows > 128 || n < 512 || k % 256 != 0 || ((uintptr_t)blob & 15) != 0) return false;   // (off a 16-byte boundary: the 32-row tiles)
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K) return false;
     if (dtype == LK_TYPE_Q6_K) {
+        if (k > 32768) return false;   // (not the short launch's)
         if (rows <= 32) return n <= 4096 && (k <= 12288 || k % 2048 == 0);
         if (rows <= 64) return n <= 2048 && (n >= 1152 || k <= 6144);
         return n <= (rows <= 96 ? 1360 : 1024) && (n >= 1152 || k <= 5632);

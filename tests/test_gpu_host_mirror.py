@@ -571,7 +571,7 @@ def test_the_lines_that_moved_to_the_tiles_dealt_evenly(name, n, k, rows, expect
     ("q4_k", 1030, 5632, 128, "tiled"), ("q4_k", 14336, 5120, 64, "tiled"), ("q5_k", 3456, 5632, 19, "rows-on-matrix-unit"),
     ("q5_k", 8208, 5632, 19, "tiled"), ("q6_k", 4096, 6144, 17, "rows-on-matrix-unit"), ("q6_k", 4097, 6144, 17, "tiled"),
     ("q6_k", 2048, 6912, 48, "rows-on-matrix-unit"), ("q6_k", 2049, 6912, 48, "tiled"), ("q6_k", 1360, 4096, 96, "rows-on-matrix-unit"),
-    ("q6_k", 1361, 5632, 96, "tiled"), ("q6_k", 1024, 5632, 128, "rows-on-matrix-unit"), ("q5_k", 1152, 4864, 40, "rows-on-matrix-unit")])
+    ("q6_k", 1361, 5632, 96, "tiled"), ("q6_k", 1024, 5632, 128, "rows-on-matrix-unit"), ("q6_k", 2056, 34816, 18, "tiled"), ("q5_k", 1152, 4864, 40, "rows-on-matrix-unit")])
 def test_the_lines_that_moved_to_sets_of_rows(name, n, k, rows, expect):
     test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
 
