@@ -170,7 +170,10 @@ extern "C" int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int t
     auto has_tiles = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K; };
     const int line = wtype_gu == wtype_down ? wtype_gu : has_tiles(wtype_gu) && has_tiles(wtype_down) ? LK_TYPE_Q6_K : -1;
     const int64_t pairs = (int64_t)tokens * topk;
-    if (!grouped_pays_over(pairs, n_experts, line, pairs * (2 * stack_bytes(*fg, ffn, hidden) + stack_bytes(*fd, hidden, ffn))) || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
+    // (Q4_0 and Q4_1 have no mat-vec per pair: no choice by the weights)
+    const bool grouped = fg->wire < 0 || fd->wire < 0 ? lk_moe_grouped_pays(pairs, n_experts, line)
+                                                      : grouped_pays_over(pairs, n_experts, line, pairs * (2 * stack_bytes(*fg, ffn, hidden) + stack_bytes(*fd, hidden, ffn)));
+    if (!grouped || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
     if (block_takes_tiles(wtype_gu, wtype_down, longest, n_experts, hidden, ffn)) return LK_MOE_GROUPED | LK_MOE_TILES;
     const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);

@@ -627,6 +627,21 @@ def test_the_pairs_or_the_batch_by_the_weights_too(gu, dn, tokens, topk, n_exper
     assert ((got - want).abs() <= 1e-3 * want.abs() + 1e-3 * want.abs().max()).all()
 
 
+@pytest.mark.parametrize("gu,dn", [(lib.TYPE_Q4_0, lib.TYPE_Q4_0), (lib.TYPE_Q4_1, lib.TYPE_Q4_1), (lib.TYPE_Q8_0, lib.TYPE_Q4_0), (lib.TYPE_Q4_1, lib.TYPE_Q4_K)])
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn", [(12, 2, 8, 512, 256), (23, 2, 8, 1024, 512), (25, 8, 60, 256, 256)])
+def test_formats_without_a_mat_vec_per_pair_at_three_to_six_rows_an_expert(gu, dn, tokens, topk, n_experts, hidden, ffn):
+    # small weights, where other formats take a mat-vec per routed pair
+    gate, up, down, x, ids, w = make_layer(tokens, hidden, ffn, n_experts, topk, 85, dn, x_scale=4.0, dt_gu=gu)
+    args = (gu, dn, dev(x), dev(gate), dev(up), dev(down), dev(ids), dev(w), n_experts, ffn)
+    got, rows = moe_forward(*args, return_rows=True)
+    want, want_h = oracle.moe_forward(1, gu, dn, x, gate, up, down, ids, w, n_experts, ffn, want_h=True)
+    check_block(got.cpu().numpy(), rows.cpu().numpy(), want, slot_order(want_h, ids), dn, down, ids, w, n_experts, hidden)
+    out = torch.empty(tokens, hidden, device="cuda")
+    status = lib.load().lk_moe_forward(gu, dn, *(a.data_ptr() for a in args[2:8]), out.data_ptr(), tokens, topk, n_experts, hidden, ffn,
+                                       torch.cuda.current_stream().cuda_stream)
+    assert status == lib.LK_OK and torch.equal(out, got)
+
+
 @pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,tiles", [(24, 2, 8, 1280, 1536, True), (12, 2, 8, 1280, 1536, False), (40, 2, 8, 1792, 512, True),
                                                                     (24, 2, 8, 1792, 512, False), (40, 2, 8, 1280, 1024, False), (24, 2, 8, 2304, 1280, True),
                                                                     (40, 2, 8, 1024, 1280, False)])
