@@ -146,11 +146,17 @@ static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int 
 // up to six rows each:
 //   Q4_K 1.77 MB an expert, 24 pairs 19.3 / 28.4; 2.65, 26 24.6 / 31.6; 1.99, 44 27.1 / 39.6; (3.32, 48 35.0 / 32.5); Q4_K and Q6_K 2.55, 22 25.6 / 38.8; 3.44,
 //   24 27.9 / 37.9; MXFP4 0.8 to 0.9 of the time under 100 MB; Q5_K under 80 MB 0.73; Q8_0 under 250 MB 0.64 to 0.75
-// and where there is much to read the batched ones pay sooner: Q5_K from 1.25 rows past 300 MB (0.87 of the time over eight blocks), Q8_0 from
+// Only while there are few pairs: many of short rows take their own time however few their bytes (batched / pairs: 64 experts of 512 -> 256 in Q4_K, 304 pairs 22 /
+// 33; 128 of 256 -> 256 in IQ3_S, 706 pairs 30 / 154; 60 of 512 -> 512 in IQ2_S, 314 39 / 127; 128 of 256 -> 256 in Q8_0, 760 34 / 74). Over drawn blocks of
+// fifteen formats, 4 to 128 experts, the pairs are ahead or level (one block of 4000 drawn ones was 9 % behind) up to 40 of the K-quants Q4_K to Q6_K, 64 of Q8_0 and 20 of the others, at
+// 1.4 to 2.2 times the batched speed in the mean.
+// And where there is much to read the batched ones pay sooner: Q5_K from 1.25 rows past 300 MB (0.87 of the time over eight blocks), Q8_0 from
 // 2.25 past 400 (0.85 over eight).
-static bool grouped_pays_over(int64_t pairs, int n_experts, int line, int64_t bytes) {
+static bool grouped_pays_over(int64_t pairs, int n_experts, int gu, int down, int line, int64_t bytes) {
     const int64_t experts = n_experts > 1 ? n_experts : 1, mb = 1000000;
-    if (pairs <= 6 * experts && bytes < (line == LK_TYPE_Q8_0 ? 250 : line == LK_TYPE_Q5_K ? 80 : 100) * mb) return false;
+    auto large_blocks = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K || type == LK_TYPE_Q8_0; };
+    const int64_t few = line == LK_TYPE_Q8_0 ? 64 : large_blocks(gu) && large_blocks(down) ? 40 : 20;
+    if (pairs <= 6 * experts && pairs <= few && bytes < (line == LK_TYPE_Q8_0 ? 250 : line == LK_TYPE_Q5_K ? 80 : 100) * mb) return false;
     if (line == LK_TYPE_Q5_K && 4 * pairs >= 5 * experts && bytes > 300 * mb) return true;
     if (line == LK_TYPE_Q8_0 && 4 * pairs >= 9 * experts && bytes > 400 * mb) return true;
     return lk_moe_grouped_pays(pairs, n_experts, line);
@@ -172,7 +178,7 @@ extern "C" int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int t
     const int64_t pairs = (int64_t)tokens * topk;
     // (Q4_0 and Q4_1 have no mat-vec per pair: no choice by the weights)
     const bool grouped = fg->wire < 0 || fd->wire < 0 ? lk_moe_grouped_pays(pairs, n_experts, line)
-                                                      : grouped_pays_over(pairs, n_experts, line, pairs * (2 * stack_bytes(*fg, ffn, hidden) + stack_bytes(*fd, hidden, ffn)));
+                                                      : grouped_pays_over(pairs, n_experts, wtype_gu, wtype_down, line, pairs * (2 * stack_bytes(*fg, ffn, hidden) + stack_bytes(*fd, hidden, ffn)));
     if (!grouped || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);
     if (block_takes_tiles(wtype_gu, wtype_down, longest, n_experts, hidden, ffn)) return LK_MOE_GROUPED | LK_MOE_TILES;

@@ -17,3 +17,15 @@ def path(gu, dn, tokens, topk, n_experts, hidden, ffn):
 def test_formats_without_a_mat_vec_per_pair_are_batched_from_three_rows_an_expert(gu, dn, tokens, topk, n_experts, hidden, ffn):
     assert path(gu, dn, tokens, topk, n_experts, hidden, ffn) & GROUPED
     assert not path(gu, dn, tokens // 4, topk, n_experts, hidden, ffn) & GROUPED   # fewer rows: refused, as ever
+
+
+# both sides of the lines in pairs, at weights of a few MB: Q4_K to Q6_K and Q8_0 together, Q8_0 alone, the other formats
+@pytest.mark.parametrize("gu,dn,few", [(lib.TYPE_Q4_K, lib.TYPE_Q4_K, 40), (lib.TYPE_Q4_K, lib.TYPE_Q6_K, 40), (lib.TYPE_Q5_K, lib.TYPE_Q5_K, 40),
+                                       (lib.TYPE_Q6_K, lib.TYPE_Q6_K, 40), (lib.TYPE_Q8_0, lib.TYPE_Q4_K, 40), (lib.TYPE_Q8_0, lib.TYPE_Q8_0, 64),
+                                       (lib.TYPE_MXFP4, lib.TYPE_MXFP4, 20), (lib.TYPE_MXFP4, lib.TYPE_Q8_0, 20), (lib.TYPE_IQ3_S, lib.TYPE_IQ3_S, 20),
+                                       (lib.TYPE_Q2_0, lib.TYPE_Q2_0, 20), (lib.TYPE_Q3_K, lib.TYPE_Q3_K, 20), (lib.TYPE_Q5_1, lib.TYPE_IQ4_XS, 20)])
+def test_many_pairs_of_small_matrices_are_batched(gu, dn, few):
+    n_experts = few // 4   # four rows an expert: past the line of lk_moe_grouped_pays in every format
+    assert not path(gu, dn, few, 1, n_experts, 256, 256) & GROUPED
+    assert path(gu, dn, few + 1, 1, n_experts, 256, 256) & GROUPED
+    assert path(gu, dn, 6 * 128 // 2, 2, 128, 256, 256) & GROUPED
