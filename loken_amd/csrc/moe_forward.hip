@@ -150,15 +150,16 @@ static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int 
 // 33; 128 of 256 -> 256 in IQ3_S, 706 pairs 30 / 154; 60 of 512 -> 512 in IQ2_S, 314 39 / 127; 128 of 256 -> 256 in Q8_0, 760 34 / 74). Over drawn blocks of
 // fifteen formats, 4 to 128 experts, the pairs are ahead or level (one block of 4000 drawn ones was 9 % behind) up to 40 of the K-quants Q4_K to Q6_K, 64 of Q8_0 and 20 of the others, at
 // 1.4 to 2.2 times the batched speed in the mean.
-// And where there is much to read the batched ones pay sooner: Q5_K from 1.25 rows past 300 MB (0.87 of the time over eight blocks), Q8_0 from
-// 2.25 past 400 (0.85 over eight).
+// And where there is much to read the batched ones pay sooner: Q5_K from 1.25 rows past 600 MB and from 1.75 past 300 (0.83 of the time over 409 drawn blocks,
+// 1.09 at most; fewer of either 0.95, up to 1.24: 32 experts of 2048 -> 1792, 40 pairs, 63.3 / 78.3), Q8_0 from 2.25 past 400 and 160 pairs (0.84 over
+// 418, 1.10 at most; fewer pairs 1.03, up to 1.35: 32 of 2560 -> 1280, 72 pairs, 139 / 183).
 static bool grouped_pays_over(int64_t pairs, int n_experts, int gu, int down, int line, int64_t bytes) {
     const int64_t experts = n_experts > 1 ? n_experts : 1, mb = 1000000;
     auto large_blocks = [](int type) { return type == LK_TYPE_Q4_K || type == LK_TYPE_Q5_K || type == LK_TYPE_Q6_K || type == LK_TYPE_Q8_0; };
     const int64_t few = line == LK_TYPE_Q8_0 ? 64 : large_blocks(gu) && large_blocks(down) ? 40 : 20;
     if (pairs <= 6 * experts && pairs <= few && bytes < (line == LK_TYPE_Q8_0 ? 250 : line == LK_TYPE_Q5_K ? 80 : 100) * mb) return false;
-    if (line == LK_TYPE_Q5_K && 4 * pairs >= 5 * experts && bytes > 300 * mb) return true;
-    if (line == LK_TYPE_Q8_0 && 4 * pairs >= 9 * experts && bytes > 400 * mb) return true;
+    if (line == LK_TYPE_Q5_K && ((4 * pairs >= 5 * experts && bytes > 600 * mb) || (4 * pairs >= 7 * experts && bytes > 300 * mb))) return true;
+    if (line == LK_TYPE_Q8_0 && 4 * pairs >= 9 * experts && bytes > 400 * mb && pairs >= 160) return true;
     return lk_moe_grouped_pays(pairs, n_experts, line);
 }
 

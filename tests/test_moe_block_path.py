@@ -29,3 +29,12 @@ def test_many_pairs_of_small_matrices_are_batched(gu, dn, few):
     assert not path(gu, dn, few, 1, n_experts, 256, 256) & GROUPED
     assert path(gu, dn, few + 1, 1, n_experts, 256, 256) & GROUPED
     assert path(gu, dn, 6 * 128 // 2, 2, 128, 256, 256) & GROUPED
+
+
+@pytest.mark.parametrize("wtype,tokens,topk,n_experts,hidden,ffn,grouped", [
+    (lib.TYPE_Q5_K, 10, 8, 64, 2048, 1536, False), (lib.TYPE_Q5_K, 10, 8, 64, 2048, 2048, True), (lib.TYPE_Q5_K, 5, 8, 32, 2048, 1792, False),
+    (lib.TYPE_Q5_K, 14, 8, 64, 1024, 1536, True), (lib.TYPE_Q5_K, 13, 8, 64, 1024, 1536, False), (lib.TYPE_Q5_K, 14, 8, 64, 1024, 1024, False),
+    (lib.TYPE_Q8_0, 9, 8, 32, 2560, 1280, False), (lib.TYPE_Q8_0, 20, 8, 64, 2048, 768, True), (lib.TYPE_Q8_0, 19, 8, 64, 2048, 768, False),
+    (lib.TYPE_Q8_0, 36, 8, 128, 512, 768, False)])
+def test_large_matrices_are_batched_sooner_where_there_are_pairs_enough(wtype, tokens, topk, n_experts, hidden, ffn, grouped):
+    assert bool(path(wtype, wtype, tokens, topk, n_experts, hidden, ffn) & GROUPED) == grouped
