@@ -124,9 +124,12 @@ extern "C" int lk_moe_rows_launch_pays(int wtype, int k, int longest_run) {
 //     64 of 1536 -> 1024 at 15 / 22 / 42 rows 64 / 66 / 82 against 59 / 81 / 138); from 9 where that launch reads rows of more than
 //     eight super-blocks and the tiles fill the chip (60 of 2560 -> 1280 at 7 / 9 / 17 / 26 rows 116 / 120 / 117 / 123 against 114 / 141 / 195 / 182)
 //     Rows of one, five to seven or more than eight super-blocks have no wave-per-tile launch (rows16_moe.hip) and go through the 32-row tiles: gate and up of such
-//     rows leave from 9 rows where down's are such too, from 13 up to 2048 values where down's are of two or three (8 of 1792 -> 512 at 19 rows 35 against 60, 8 of
-//     1536 -> 1536 at 16 41 / 58, 8 of 1792 -> 1280 at 12 40 / 50, 60 of 1792 -> 512 at 19 56 / 72, 128 of 1792 -> 1536 at 11 202 / 208; past the
-//     lines 60 of 1280 -> 1024 at 14 70 / 64, 8 of 2816 -> 512 at 14 41 / 36)
+//     rows leave from 9 rows where down's are such too, from 14 up to 2048 values where down's are of two or three (8 of 1792 -> 512 at 19 rows 35 against 60, 8 of
+//     1536 -> 1536 at 16 41 / 58, 8 of 1792 -> 1280 at 12 40 / 50, 60 of 1792 -> 512 at 19 56 / 72; past the lines 60 of 1280 -> 1024 at 14 70 / 64, 8 of
+//     2816 -> 512 at 14 41 / 36, 128 of 1536 -> 512 at 13 77 / 72). Where the rows launch reads so few super-blocks that its 32-row tiles are through as soon, the
+//     line is later or none: 1792 of down from 12 rows (64 of 1792 -> 1792 at 9 128 / 119), hidden 256 up to 1280 (128 of 256 -> 1792 at 12 65 / 57), longer rows
+//     than 2048 from eight experts on and down's of more than one super-block (4 of 3072 -> 1536 at 9 46 / 41, 16 of 3072 -> 256 at 10 38 / 34). Over 408 drawn
+//     blocks past these lines 0.80 of the time in the mean, 1.05 at most
 // and with workgroups of 64 gate and up rows for a quarter of the CUs at least.
 static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int hidden, int ffn) {
     auto always = [](int type) { return type == LK_TYPE_Q5_K || type == LK_TYPE_Q8_0 || type == LK_TYPE_Q4_0; };
@@ -137,7 +140,11 @@ static bool block_takes_tiles(int gu, int down, int longest, int n_experts, int 
     if (of_levels(gu) || of_levels(down)) return longest > 32 || n_experts < 60;
     if (gu == LK_TYPE_Q6_K && down == LK_TYPE_Q6_K) return longest > 22 || n_experts < 60;
     auto wave_a_tile = [](int k) { return k == 512 || k == 768 || k == 1024 || k == 2048; };
-    if (gu == down && !wave_a_tile(hidden) && (wave_a_tile(ffn) ? longest >= 13 && hidden <= 2048 && ffn < 1024 : longest >= 9)) return true;
+    if (gu == down && !wave_a_tile(hidden)) {
+        if (wave_a_tile(ffn) ? longest >= 14 && hidden <= 2048 && ffn < 1024
+                             : longest >= (hidden > 256 && hidden <= 2048 && ffn > 1536 ? 12 : 9) && (hidden == 256 ? ffn <= 1280 : hidden <= 2048 || (n_experts >= 8 && ffn > 256)))
+            return true;
+    }
     return longest >= 20 || (longest >= 9 && hidden > 2048 && 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus);
 }
 

@@ -38,3 +38,12 @@ def test_many_pairs_of_small_matrices_are_batched(gu, dn, few):
     (lib.TYPE_Q8_0, 36, 8, 128, 512, 768, False)])
 def test_large_matrices_are_batched_sooner_where_there_are_pairs_enough(wtype, tokens, topk, n_experts, hidden, ffn, grouped):
     assert bool(path(wtype, wtype, tokens, topk, n_experts, hidden, ffn) & GROUPED) == grouped
+
+
+@pytest.mark.parametrize("tokens,topk,n_experts,hidden,ffn,tiles", [
+    (11, 2, 4, 3072, 1536, False), (22, 2, 8, 3072, 1536, True), (39, 2, 16, 3072, 256, False), (39, 2, 16, 1280, 256, True),
+    (60, 4, 64, 1792, 1792, False), (105, 4, 64, 1792, 1792, True), (60, 4, 64, 1792, 1536, True), (107, 4, 128, 256, 1792, False),
+    (107, 4, 128, 256, 1280, True), (88, 8, 128, 1536, 512, False), (110, 8, 128, 1536, 512, True)])
+def test_short_q4k_runs_go_on_the_tiles_where_these_are_ahead(tokens, topk, n_experts, hidden, ffn, tiles):
+    assert 9 <= lib.load().lk_moe_longest_run(tokens, topk, n_experts) < 20
+    assert bool(path(lib.TYPE_Q4_K, lib.TYPE_Q4_K, tokens, topk, n_experts, hidden, ffn) & TILES) == tiles
