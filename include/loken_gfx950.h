@@ -617,9 +617,10 @@ int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gat
 #define LK_MOE_ROWS_DOWN 4
 #define LK_MOE_TILES 8
 int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int topk, int n_experts, int hidden, int ffn);
-/* The rules this goes by, each for one stack alone: whether the expert-batched launches pay at `rows` routed rows (wtype: the stacks' type where
- * all have the same, else -1); the longest run an expert is expected to own (mmq_experts.rs:215-227); whether a stack
- * then takes lk_moe_q4k_rows_grouped. */
+/* Rules it is made of, each for one stack alone: whether the expert-batched launches pay at `rows` routed rows whatever the experts'
+ * size (wtype: the stacks' type where all have the same, else -1); the longest run an expert is expected to own
+ * (mmq_experts.rs:215-227); whether a stack then takes lk_moe_q4k_rows_grouped. The block goes by the bytes of the weights
+ * and by both stacks too, so a caller that wants its launches asks lk_moe_block_path and not these. */
 int lk_moe_grouped_pays(int64_t rows, int n_experts, int wtype);
 int lk_moe_longest_run(int tokens, int topk, int n_experts);
 int lk_moe_rows_launch_pays(int wtype, int k, int longest_run);

@@ -428,7 +428,8 @@ def stable_sort_u32(keys: torch.Tensor, small: bool = False):
 
 def moe_mmq_pays(rows: int, experts: int, wtype: int | None = None) -> bool:
     """Whether the expert-batched launches beat the per-pair kernels at this many routed rows (``wtype``: the
-    stacks' type where all have the same)."""
+    stacks' type where all have the same), whatever the size of the experts. ``moe_forward`` goes by the bytes of the
+    weights too: which launches a block is made of, ``lk_moe_block_path`` alone tells."""
     return bool(_lib.load().lk_moe_grouped_pays(rows, experts, -1 if wtype is None else wtype))
 
 
@@ -436,8 +437,8 @@ def moe_forward(wtype_gu: int, wtype_down: int, x: torch.Tensor, gate: torch.Ten
                 down: torch.Tensor, choices: torch.Tensor, topk_weights: torch.Tensor, n_experts: int,
                 ffn: int, return_rows: bool = False):
     """The expert block of one layer, path chosen as the reference's layer code chooses it
-    (src/inference/generic_transformer/moe_weights.rs:2118-2152): the expert-batched tiled
-    matmuls when there is at least a routed row per expert, else one mat-vec per routed pair.
+    (src/inference/generic_transformer/moe_weights.rs:2118-2152): the expert-batched
+    matmuls from a few routed rows per expert on, else one mat-vec per routed pair (``lk_moe_block_path``).
     A choice outside ``[0, n_experts)`` adds nothing to its token.
     `return_rows`: also the gated rows the second product read, in slot order (token * topk + choice), zeros where a
     choice names no expert."""

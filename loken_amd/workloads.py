@@ -329,6 +329,15 @@ def mmq(args, dev):
 
 
 # ---------------------------------------------------------------------------- moe
+def moe_launches(how, wtype, tokens, topk, experts, hidden, ffn):
+    """The launches of a block as lk_moe_block_path's bits: the library's own choice, or ("tiled", "rows", "pairs") pinned ones."""
+    if how == "auto":
+        return lib.load().lk_moe_block_path(wtype, wtype, tokens, topk, experts, hidden, ffn)
+    if how == "pairs" or not (moe.moe_mmq_serves(wtype, hidden) and moe.moe_mmq_serves(wtype, ffn)):
+        return 0
+    return lib.MOE_GROUPED | (lib.MOE_ROWS_GATE_UP | lib.MOE_ROWS_DOWN if how == "rows" else 0)
+
+
 def moe_block(args, dev):
     experts, hidden, ffn, topk, tokens = 128, 2048, 768, 8, args.tokens
     mk = Maker(dev)
@@ -352,8 +361,8 @@ def moe_block(args, dev):
     choices = choices.to(torch.int32).contiguous()
 
     pairs = tokens * topk
-    tiled = moe.moe_mmq_pays(pairs, experts, wt) if args.moe_path == "auto" else args.moe_path in ("tiled", "rows")
-    tiled = tiled and moe.moe_mmq_serves(wt, hidden) and moe.moe_mmq_serves(wt, ffn)
+    path = moe_launches(args.moe_path, wt, tokens, topk, experts, hidden, ffn)
+    tiled = bool(path & lib.MOE_GROUPED)
     # The routing (the router's side of the boundary) is built once; the timed block is what the
     # expert launchers do with it, recorded into a graph so that the host's cost stays outside.
     rows_launch = False
@@ -362,12 +371,13 @@ def moe_block(args, dev):
         nonlocal rows_launch
         flat_w = weights.reshape(-1)
         if tiled:
-            plan = moe.MmqRouting.from_choices(choices, experts).with_path(args.moe_path if args.moe_path in ("tiled", "rows") else "auto")
-            rows_launch = plan.takes_rows_launch(wt, hidden)
+            plan = moe.MmqRouting.from_choices(choices, experts).with_tile_width(128 if path & lib.MOE_TILES else 0)
+            first, second = ("rows" if path & bit else "tiled" for bit in (lib.MOE_ROWS_GATE_UP, lib.MOE_ROWS_DOWN))
+            rows_launch = plan.with_path(first).takes_rows_launch(wt, hidden)
 
             def block():
-                h = plan.gate_up_silu(wt, x, gate, up, ffn)
-                return plan.down_fold(wt, h, down, hidden, flat_w)
+                h = plan.with_path(first).gate_up_silu(wt, x, gate, up, ffn)
+                return plan.with_path(second).down_fold(wt, h, down, hidden, flat_w)
         else:
             routing = moe.ExpertRouting(choices)
 
@@ -410,7 +420,7 @@ def moe_block(args, dev):
     hbm_floor_us, mfma_floor_us = nbytes / HBM_PEAK_GBS / 1e3, op_count / INT8_PEAK_TOPS / 1e6
     gbs, tops = nbytes / med / 1e3, op_count / med / 1e6
     if tiled:
-        kernel = f"q4k_rows_moe_kernel, {name}" if rows_launch else f"mmq_moe_kernel, {name}"
+        kernel = f"{'q4k_rows_moe_kernel' if rows_launch else 'tile_moe_kernel' if path & lib.MOE_TILES else 'mmq_moe_kernel'}, {name}"
         note = ("whole expert block (quantize, two grouped matmuls with the activation in the first, fold)" if rows_launch
                 else "whole expert block (plan, route, quantize, two grouped matmuls, activation, fold)")
     else:
