@@ -291,11 +291,14 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
         if (rc < 0) {
             LkScratch scratch(stream);
             void* act = scratch.get(LK_SCRATCH_LINEAR, (size_t)rows * blocks * Q81_BLOCK);
-            if (!act) return LK_ERR_NOMEM;
-            if (int r = lk_quantize_q8_1(x, x_type, act, k_, k_, rows, stream)) return r;
             // (rows too long for the kernels' scale tables in LDS launch nothing, and the call goes on to the
-            // mat-vec or the tiled matmul below)
-            rc = lk_rows_linear(dtype_, blob_, act, blocks, out, x_type, rows, n_, k_, stream);
+            // mat-vec or the tiled matmul below; so does one without memory for the quantized rows, a recorded one above all
+            // of which only larger calls ran before, on the tiles, which work in other buffers)
+            rc = LK_ERR_ARG;
+            if (act) {
+                if (int r = lk_quantize_q8_1(x, x_type, act, k_, k_, rows, stream)) return r;
+                rc = lk_rows_linear(dtype_, blob_, act, blocks, out, x_type, rows, n_, k_, stream);
+            }
         }
         if (rc == LK_OK) {
             last_path_ = Path::RowsOnMatrixUnit;

@@ -128,6 +128,31 @@ def test_scratch_that_grows_after_a_recording():
     lin.close()
 
 
+@pytest.mark.parametrize("wtype,n,k,rows", [(lib.TYPE_Q4_K, 2986, 6144, 26), (lib.TYPE_Q6_K, 2048, 6912, 48), (lib.TYPE_Q5_K, 1152, 4864, 40)])
+def test_a_linear_recorded_after_larger_calls_alone_runs_in_their_buffers(wtype, n, k, rows):
+    """Rows kernels and tiles work in different buffers: where only calls on the tiles ran before, the tiles serve the recorded one."""
+    w = synth.weight(wtype, 64, k, seed=82, stream=1).reshape(64, -1).repeat((n + 63) // 64, axis=0)[:n]
+    x = synth.activation(rows, k, seed=82)
+    lin, xd = Linear(wtype, dev(w), n, k), dev(x)
+    lib.load().lkh_release_workspaces()
+    lib.load().loken_stream_scratch_release()
+    lin(dev(synth.activation(700, k, seed=83)))
+    assert lin.path == "tiled"
+    graph, out = record(lambda: lin(xd), torch.cuda.Stream())
+    assert lin.path == "tiled"
+    eager = lin(xd)
+    assert lin.path == "rows-on-matrix-unit"
+    ends = np.r_[:20, n - 20:n]
+    want = oracle.ob_matmul(wtype, x, w[ends], len(ends))
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (np.abs(out.cpu().numpy()[:, ends] - want) <= 1e-3 * np.abs(want) + 1e-4).all()
+        assert (out - eager).abs().max() <= 2e-5 * eager.abs().max()
+    lin.close()
+
+
 def test_dropping_the_linears_workspaces_leaves_the_mixtures_graph():
     tokens, topk, n_experts, hidden, ffn = 64, 4, 8, 512, 256
     gate, up = (dev(synth.weight(lib.TYPE_Q6_K, n_experts * ffn, hidden, seed=81, stream=i)) for i in (1, 2))
