@@ -11,6 +11,8 @@ int lk_moe_pairs_gate_up(int wire, const float* x, const void* gate, const void*
                          int topk, int pairs, int ffn, int hidden, hipStream_t s);
 int lk_moe_pairs_down(int wire, const float* h, const void* down, const int32_t* choices, const float* weights, float* out,
                       int experts, int topk, int pairs, int hidden, int ffn, hipStream_t s);
+// What the two work in besides `h` (LK_SCRATCH_LAUNCHER), bytes.
+size_t lk_moe_pairs_scratch(int wire_gu, int wire_down, const float* x, const float* h, const void* down, int topk, int pairs, int hidden, int ffn);
 
 // Groups the router's choices by expert (moe_mmq.hip): counts [experts] (nullable), bounds [experts + 1], slots and src_rows [n].
 // With `rows` the launch also quantizes `count` rows of k values, k a multiple of 32: to Q8_1 rows of k / 32 blocks where q81 is set,

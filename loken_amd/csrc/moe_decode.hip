@@ -29,6 +29,7 @@ int lk_moe_down_fold(int quant_type, const float* inputs, const void* weights, c
                      const int32_t* expert_ids, const float* topk_weights, float* outputs, int num_experts, int topk,
                      int size_m, int size_n, int size_k, const float* down_bias, const float* add_after,
                      bool write, hipStream_t stream);
+bool lk_moe_down_fold_serves(int quant_type, const float* inputs, const void* weights, bool sorted, int topk, int size_m, int size_k);
 
 namespace {
 
@@ -489,6 +490,14 @@ int lk_moe_pairs_gate_up(int wire, const float* x, const void* gate, const void*
                          int topk, int pairs, int ffn, int hidden, hipStream_t s) {
     return gate_up_impl(x, gate, up, nullptr, choices, h, experts, topk, pairs, ffn, hidden, wire, LkGateAct{}, 0, s, nullptr,
                         LkMoeAlt{}, true);
+}
+
+size_t lk_moe_pairs_scratch(int wire_gu, int wire_down, const float* x, const float* h, const void* down, int topk, int pairs, int hidden, int ffn) {
+    const size_t tokens = rows_stage_as_f32(x, hidden, wire_gu) ? 0 : (size_t)(pairs / topk) * (pad512(hidden) / 32) * Q81_BYTES;
+    if (lk_moe_down_fold_serves(wire_down, h, down, false, topk, pairs, ffn)) return tokens;
+    const size_t acts = rows_stage_as_f32(h, ffn, wire_down) ? 0 : (((size_t)pairs * (pad512(ffn) / 32) * Q81_BYTES) + 255) & ~(size_t)255;
+    const size_t rows = acts + (size_t)pairs * hidden * sizeof(float);
+    return tokens > rows ? tokens : rows;
 }
 
 int lk_moe_pairs_down(int wire, const float* h, const void* down, const int32_t* choices, const float* weights, float* out,

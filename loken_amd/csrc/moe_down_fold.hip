@@ -308,7 +308,6 @@ int launch(const FoldCall& c, FoldDims d) {
 
 template <class L>
 int launch_format(const FoldCall& c, const FoldDims& d, int nb) {
-    if (((uintptr_t)c.w) & (L::ALIGN - 1)) return -1;
     const bool few = d.topk <= 4;
     switch (nb) {
         case 2: return few ? launch<L, 2, 4>(c, d) : launch<L, 2, 8>(c, d);
@@ -320,17 +319,22 @@ int launch_format(const FoldCall& c, const FoldDims& d, int nb) {
 
 }  // namespace
 
+// Whether the launch below takes the call.
+bool lk_moe_down_fold_serves(int quant_type, const float* inputs, const void* weights, bool sorted, int topk, int size_m, int size_k) {
+    if (lk_tune_env("LK_TUNE_DOWN_FOLD_OFF") || (quant_type != 1 && quant_type != 4 && quant_type != 5)) return false;
+    if ((size_k != 512 && size_k != 768 && size_k != 1024) || topk < 1 || topk > 8 || (sorted && size_m > MAX_PAIRS) || size_m % topk != 0) return false;
+    const int tokens = size_m / topk, align = quant_type == 5 ? LaneQ6K::ALIGN : LaneQ4K<false>::ALIGN;
+    return tokens >= 1 && tokens <= 65535 && ((uintptr_t)inputs & 15) == 0 && ((uintptr_t)weights & (align - 1)) == 0;
+}
+
 // Down + fold of Q4_K / Q5_K / Q6_K experts (wire ids 1, 4, 5) in one launch. Returns -1 when this
 // kernel does not serve the call (the caller then takes the two launches), else an LK_* status.
 int lk_moe_down_fold(int quant_type, const float* inputs, const void* weights, const int32_t* sorted_token_ids,
                      const int32_t* expert_ids, const float* topk_weights, float* outputs, int num_experts, int topk,
                      int size_m, int size_n, int size_k, const float* down_bias, const float* add_after,
                      bool write, hipStream_t stream) {
-    if (lk_tune_env("LK_TUNE_DOWN_FOLD_OFF")) return -1;
-    if (size_k % 256 != 0 || topk < 1 || topk > 8 || (sorted_token_ids && size_m > MAX_PAIRS) || size_m % topk != 0) return -1;
-    if (((uintptr_t)inputs) & 15) return -1;
+    if (!lk_moe_down_fold_serves(quant_type, inputs, weights, sorted_token_ids != nullptr, topk, size_m, size_k)) return -1;
     const int tokens = size_m / topk;
-    if (tokens < 1 || tokens > 65535) return -1;
     const FoldDims d{num_experts, topk, size_m, size_n, 1, 0, write && !add_after ? 1 : 0};
     const FoldCall c{(const uint8_t*)weights, inputs, sorted_token_ids, expert_ids, topk_weights, down_bias, add_after,
                      outputs, tokens, stream};

@@ -170,6 +170,17 @@ static bool grouped_pays_over(int64_t pairs, int n_experts, int gu, int down, in
     return lk_moe_grouped_pays(pairs, n_experts, line);
 }
 
+// What a batched block is made of, as lk_moe_block_path's bits.
+static int batched_path(int wtype_gu, int wtype_down, int tokens, int topk, int n_experts, int hidden, int ffn) {
+    const int longest = lk_moe_longest_run(tokens, topk, n_experts);
+    if (block_takes_tiles(wtype_gu, wtype_down, longest, n_experts, hidden, ffn)) return LK_MOE_GROUPED | LK_MOE_TILES;
+    const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
+    const bool tiles_fill = 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus;
+    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest) && (rows_down || longest <= 36) &&
+                         (hidden <= 2048 || !tiles_fill || longest <= 20);
+    return LK_MOE_GROUPED | (rows_gu ? LK_MOE_ROWS_GATE_UP : 0) | (rows_down ? LK_MOE_ROWS_DOWN : 0);
+}
+
 // Which launches the block is made of: LK_MOE_GROUPED (expert-batched products; else a mat-vec per routed pair),
 // and in it LK_MOE_TILES (both products on the f16 tiles), or LK_MOE_ROWS_GATE_UP / LK_MOE_ROWS_DOWN
 // (lk_moe_q4k_rows_grouped; else the tiled launch). The one place that decides: lk_moe_forward and a caller that issues the
@@ -188,13 +199,7 @@ extern "C" int lk_moe_block_path(int wtype_gu, int wtype_down, int tokens, int t
     const bool grouped = fg->wire < 0 || fd->wire < 0 ? lk_moe_grouped_pays(pairs, n_experts, line)
                                                       : grouped_pays_over(pairs, n_experts, wtype_gu, wtype_down, line, pairs * (2 * stack_bytes(*fg, ffn, hidden) + stack_bytes(*fd, hidden, ffn)));
     if (!grouped || !grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return 0;
-    const int longest = lk_moe_longest_run(tokens, topk, n_experts);
-    if (block_takes_tiles(wtype_gu, wtype_down, longest, n_experts, hidden, ffn)) return LK_MOE_GROUPED | LK_MOE_TILES;
-    const bool rows_down = lk_moe_rows_launch_pays(wtype_down, ffn, longest);
-    const bool tiles_fill = 2ll * n_experts * ((ffn + 255) / 256) >= lk_device().cus;
-    const bool rows_gu = lk_moe_rows_launch_pays(wtype_gu, hidden, longest) && (rows_down || longest <= 36) &&
-                         (hidden <= 2048 || !tiles_fill || longest <= 20);
-    return LK_MOE_GROUPED | (rows_gu ? LK_MOE_ROWS_GATE_UP : 0) | (rows_down ? LK_MOE_ROWS_DOWN : 0);
+    return batched_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn);
 }
 
 extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, const void* gate, const void* up, const void* down,
@@ -210,13 +215,19 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     const int rows = tokens * topk;
     LkScratch scratch(s);
 
-    const int path = lk_moe_block_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn);
+    int path = lk_moe_block_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn);
     if (!(path & LK_MOE_GROUPED)) {
         if (fg->wire < 0 || fd->wire < 0) return LK_ERR_TYPE;
         float* h = (float*)scratch.get(LK_SCRATCH_BLOCK, (size_t)rows * ffn * 4);
-        if (!h) return LK_ERR_NOMEM;
-        if (int rc = lk_moe_pairs_gate_up(fg->wire, x, gate, up, choices, h, n_experts, topk, rows, ffn, hidden, s)) return rc;
-        return lk_moe_pairs_down(fd->wire, h, down, choices, topk_weights, out, n_experts, topk, rows, hidden, ffn, s);
+        const size_t more = lk_moe_pairs_scratch(fg->wire, fd->wire, x, h, down, topk, rows, hidden, ffn);
+        if (h && (more == 0 || scratch.get(LK_SCRATCH_LAUNCHER, more))) {
+            if (int rc = lk_moe_pairs_gate_up(fg->wire, x, gate, up, choices, h, n_experts, topk, rows, ffn, hidden, s)) return rc;
+            return lk_moe_pairs_down(fd->wire, h, down, choices, topk_weights, out, n_experts, topk, rows, hidden, ffn, s);
+        }
+        // Without that memory (a recorded call of which only larger ones, batched, ran before) the batched launches where these
+        // serve: they work in the block's buffer alone.
+        if (!grouped_serves(*fg, hidden) || !grouped_serves(*fd, ffn)) return LK_ERR_NOMEM;
+        path = batched_path(wtype_gu, wtype_down, tokens, topk, n_experts, hidden, ffn);
     }
 
     const int longest = lk_moe_longest_run(tokens, topk, n_experts);

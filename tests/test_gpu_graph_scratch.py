@@ -153,6 +153,41 @@ def test_a_linear_recorded_after_larger_calls_alone_runs_in_their_buffers(wtype,
     lin.close()
 
 
+@pytest.mark.parametrize("gu,dn,tokens,n_experts,hidden,ffn", [(lib.TYPE_Q4_K, lib.TYPE_Q4_K, 15, 8, 512, 256), (lib.TYPE_Q8_0, lib.TYPE_Q8_0, 24, 8, 512, 256),
+                                                               (lib.TYPE_MXFP4, lib.TYPE_MXFP4, 9, 6, 256, 512), (lib.TYPE_Q5_K, lib.TYPE_Q5_K, 1, 8, 512, 512)])
+def test_a_block_recorded_after_larger_calls_alone_runs_in_their_buffers(gu, dn, tokens, n_experts, hidden, ffn):
+    """A block of few pairs works in another buffer than a batched one, unless down and fold are one launch: where only batched
+    blocks ran before, the batched launches serve the recorded one."""
+    topk = 2
+    gate, up = (dev(synth.weight(gu, n_experts * ffn, hidden, seed=84, stream=i)) for i in (1, 2))
+    down = dev(synth.weight(dn, n_experts * hidden, ffn, seed=84, stream=3))
+    L = lib.load()
+
+    def call(tokens, seed):
+        ids, w = oracle.topk_softmax(synth.activation(tokens, n_experts, seed=seed, stream=7), topk)
+        x, ids, w = dev(synth.activation(tokens, hidden, seed=seed)), dev(ids), dev(w)
+
+        def run():
+            out = torch.empty((tokens, hidden), device="cuda")
+            lib.check("lk_moe_forward", L.lk_moe_forward(gu, dn, x.data_ptr(), gate.data_ptr(), up.data_ptr(), down.data_ptr(), ids.data_ptr(), w.data_ptr(),
+                                                         out.data_ptr(), tokens, topk, n_experts, hidden, ffn, torch.cuda.current_stream().cuda_stream))
+            return out
+        return run
+
+    assert not L.lk_moe_block_path(gu, dn, tokens, topk, n_experts, hidden, ffn) & lib.MOE_GROUPED
+    assert L.lk_moe_block_path(gu, dn, 300, topk, n_experts, hidden, ffn) & lib.MOE_GROUPED
+    L.loken_stream_scratch_release()
+    call(300, 85)()
+    small = call(tokens, 86)
+    graph, out = record(small, torch.cuda.Stream())
+    eager = small()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((out - eager).abs() <= 1e-3 * eager.abs() + 1e-3 * eager.abs().max()).all()
+
+
 def test_dropping_the_linears_workspaces_leaves_the_mixtures_graph():
     tokens, topk, n_experts, hidden, ffn = 64, 4, 8, 512, 256
     gate, up = (dev(synth.weight(lib.TYPE_Q6_K, n_experts * ffn, hidden, seed=81, stream=i)) for i in (1, 2))
