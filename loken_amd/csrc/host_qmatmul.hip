@@ -93,6 +93,18 @@ bool nibble_tiles_pay(int dtype, int n, int k, int rows) {
     return rows >= 16 || (long long)n * k >= (48ll << 20);
 }
 
+// The buffer of a tiled call's partial products. A graph keeps its own and all graphs together are bounded, so a recorded call takes
+// the larger size only where its plan uses it; a plan that fits the smaller one is the same in both.
+struct Fixup {
+    void* ptr;
+    int64_t bytes;
+};
+Fixup fixup_of(LkScratch& scratch, int dtype, int n, int k, int rows) {
+    if (!scratch.recording() || lk_mmq_tiles_parts(dtype, k, n, rows) > MMQ_FIXUP_BYTES)
+        if (void* large = scratch.get(LK_SCRATCH_FIXUP, MMQ_HOST_FIXUP_BYTES)) return {large, MMQ_HOST_FIXUP_BYTES};
+    return {scratch.get(LK_SCRATCH_FIXUP, MMQ_FIXUP_BYTES), MMQ_FIXUP_BYTES};
+}
+
 size_t elem_bytes(int type) { return type == LK_TYPE_F32 ? 4 : 2; }
 
 }  // namespace
@@ -313,11 +325,11 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
     const size_t k_padded = pad_to(pad_to((size_t)k_, 512), 128);
     const size_t ws_bytes = (size_t)rows * (k_padded / 128) * MMQ_RECORD + 128 * MMQ_RECORD;
     LkScratch scratch(stream);
-    void* fixup = scratch.get(LK_SCRATCH_FIXUP, MMQ_HOST_FIXUP_BYTES);
-    if (!fixup) return LK_ERR_NOMEM;
+    const Fixup fixup = fixup_of(scratch, dtype_, n_, k_, rows);
+    if (!fixup.ptr) return LK_ERR_NOMEM;
     // The f16 tiles' operands straight from x where the product takes those tiles (Q6_K 4096 x 14336 at 2048 rows 527 ->
     // 502 us, Q4_K 14336 x 4096 at 512 rows 100 -> 96 against records in between); without memory for them, by way of the records.
-    const int width = lk_mmq_tiles_linear(dtype_, fixup, blob_, x, x_type, out, k_, n_, rows, stream);
+    const int width = lk_mmq_tiles_linear(dtype_, fixup.ptr, fixup.bytes, blob_, x, x_type, out, k_, n_, rows, stream);
     if (width == 0) return LK_ERR_ARG;
     if (width > 0) {
         last_path_ = Path::Tiled;
@@ -331,7 +343,7 @@ int QKernelMatMul::forward(const void* x, int x_type, int rows, void* out, void*
                          ? launch_mmq_quantize_q8_1_D4
                          : launch_mmq_quantize_q8_1_DS4;
     quantizer(x, nullptr, act, x_type, k_, k_, 0, 0, (int64_t)k_padded, rows, 1, 1, stream);
-    if (lk_mmq_linear(dtype_, fixup, blob_, act, out, x_type, k_, n_, rows, k_ / block_len, stream) == 0)
+    if (lk_mmq_linear(dtype_, fixup.ptr, blob_, act, out, x_type, k_, n_, rows, k_ / block_len, stream) == 0)
         return LK_ERR_ARG;   // "no tile fits, nothing ran": the reference falls back to dequantized
     last_path_ = Path::Tiled;
     return LK_OK;
@@ -395,8 +407,8 @@ int QKernelMatMul::forward_quantized(const QuantizedActivation& a, void* out, vo
     }
     if (!one_order && few_rows_to_tiles(dtype_, n_, k_, a.rows, blob_)) {
         LkScratch scratch((hipStream_t)stream);
-        void* fixup = scratch.get(LK_SCRATCH_FIXUP, MMQ_HOST_FIXUP_BYTES);
-        const int width = fixup ? lk_mmq_tiles_linear_q8_1(dtype_, fixup, blob_, a.q81, blocks, a.x_type, out, k_, n_, a.rows, (hipStream_t)stream) : -1;
+        const Fixup fixup = fixup_of(scratch, dtype_, n_, k_, a.rows);
+        const int width = fixup.ptr ? lk_mmq_tiles_linear_q8_1(dtype_, fixup.ptr, fixup.bytes, blob_, a.q81, blocks, a.x_type, out, k_, n_, a.rows, (hipStream_t)stream) : -1;
         if (width == 0) return LK_ERR_ARG;
         if (width > 0) {
             last_path_ = Path::Tiled;

@@ -76,7 +76,8 @@ constexpr int64_t MMQ_FIXUP_BYTES = 256ll * 128 * 128 * 4;
 // (11003 x 4096 at 77 rows, quantizer included: Q4_K 63 -> 40 us, Q5_K 73 -> 44, Q6_K 89 -> 51).
 __host__ __device__ static inline int64_t mmq_part_stride(const MmqProblem& pb) { return ((int64_t)pb.n + 3) / 4 * 4; }
 // What the host linear keeps for its own products: a product of many rows and columns has too few tiles for the chip at twice the
-// partial products (1186 x 10240 at 1661 rows of Q6_K: 16 MiB leave it whole, 32 allow three ranges; 64 give no call of 1300 more).
+// partial products (1186 x 10240 at 1661 rows of Q6_K: 16 MiB leave it whole, 32 allow three ranges; 64 give no call of 1300 more). A recorded call
+// whose plan has no use for more takes MMQ_FIXUP_BYTES, and so does one that cannot have this much.
 constexpr int64_t MMQ_HOST_FIXUP_BYTES = 2 * MMQ_FIXUP_BYTES;
 // The most ranges K may be cut into: two blocks each, their partial products in the buffer; 1 where it stays whole.
 static inline int mmq_splits_most(const MmqProblem& pb, const void* fixup, bool ragged = false, int64_t fixup_bytes = MMQ_FIXUP_BYTES) {
@@ -155,10 +156,12 @@ int lk_operands_quantize(const void* x, int type, const LkTokenOperands& ops, in
 // 32-bit offsets, no scratch) and the caller should take the int8 tiles.
 int lk_mmq_tiles_dense(int wtype, const MmqProblem& pb, hipStream_t s, void* fixup);
 // lk_mmq_f16_tiles: whether a dense product takes them: 9 token rows or more and 512 weight rows or more (LK_MMQ_I8 unset).
-// The same for `rows` rows of x, k values each, results in x's type: nothing between x and the operands. `fixup`: MMQ_HOST_FIXUP_BYTES.
-int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s);
+// Bytes of partial products that the plan of such a product writes, given MMQ_HOST_FIXUP_BYTES.
+int64_t lk_mmq_tiles_parts(int wtype, int k, int n, int rows);
+// The same for `rows` rows of x, k values each, results in x's type: nothing between x and the operands.
+int lk_mmq_tiles_linear(int wtype, void* fixup, int64_t fixup_bytes, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s);
 // The same from the rows' Q8_1 blocks, `stride` blocks between rows, with the same bits.
-int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
+int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, int64_t fixup_bytes, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
                              hipStream_t s);
 // The expert-batched product over workspace records, same returns as the dense one.
 int lk_mmq_tiles_moe_records(int wtype, const MmqProblem& pb, const uint8_t* w_second, int64_t dst_second, const int32_t* bounds,

@@ -187,19 +187,28 @@ extern "C" int lk_mmq_f16_tiles(int wtype, int64_t n, int64_t rows) {
     return f && f->dense && rows > 8 && n >= 512 && !lk_env_flag("LK_MMQ_I8");
 }
 
-int lk_mmq_tiles_linear(int wtype, void* fixup, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {
+int64_t lk_mmq_tiles_parts(int wtype, int k, int n, int rows) {
+    if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return 0;
+    MmqProblem pb{};
+    pb.nb = k / 256, pb.m_end = rows, pb.n = n;
+    if (rows > rows_of_pass(pb.nb)) return MMQ_HOST_FIXUP_BYTES;   // several passes: the last one's plan is another
+    const int splits = plan_dense(*tiles_of(wtype), pb, (void*)256, MMQ_HOST_FIXUP_BYTES).splits;
+    return splits > 1 ? splits * (int64_t)rows * mmq_part_stride(pb) * 4 : 0;
+}
+
+int lk_mmq_tiles_linear(int wtype, void* fixup, int64_t fixup_bytes, const void* w, const void* x, int type, void* out, int k, int n, int rows, hipStream_t s) {
     if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
-    return run_dense(*tiles_of(wtype), pb, s, fixup, MMQ_HOST_FIXUP_BYTES, [&](const LkTokenOperands& ops, int m0, int count) {
+    return run_dense(*tiles_of(wtype), pb, s, fixup, fixup_bytes, [&](const LkTokenOperands& ops, int m0, int count) {
         (void)lk_operands_quantize((const uint8_t*)x + (int64_t)m0 * k * (type == LK_TYPE_F32 ? 4 : 2), type, ops, k, count, s);
     });
 }
 
-int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
+int lk_mmq_tiles_linear_q8_1(int wtype, void* fixup, int64_t fixup_bytes, const void* w, const void* q8_1, int stride, int type, void* out, int k, int n, int rows,
                              hipStream_t s) {
     if (!lk_mmq_f16_tiles(wtype, n, rows) || k % 256 != 0) return -1;
     const MmqProblem pb{(const uint8_t*)w, nullptr, (float*)out, nullptr, k / 256, k / tiles_of(wtype)->values, rows, n, n, 0, rows, type};
-    return run_dense(*tiles_of(wtype), pb, s, fixup, MMQ_HOST_FIXUP_BYTES, [&](const LkTokenOperands& ops, int m0, int count) {
+    return run_dense(*tiles_of(wtype), pb, s, fixup, fixup_bytes, [&](const LkTokenOperands& ops, int m0, int count) {
         hipLaunchKernelGGL(operands_from_q8_1_kernel, dim3((unsigned)pb.nb, (unsigned)((count + 31) / 32)), dim3(256), 0, s,
                            (const uint8_t*)q8_1 + (int64_t)m0 * stride * Q81_BYTES, ops, stride, count);
     });

@@ -51,6 +51,9 @@ class LkScratch {
     // records a graph.
     int ticket() const;
 
+    // Whether the stream records a graph, which keeps what it takes.
+    bool recording() const;
+
   private:
     hipStream_t stream_;
     std::shared_ptr<LkScratchPool> pool_;

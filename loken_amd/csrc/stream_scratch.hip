@@ -213,6 +213,8 @@ void* LkScratch::get(LkScratchUse use, size_t bytes) {
 
 int LkScratch::ticket() const { return pool_->ticket; }
 
+bool LkScratch::recording() const { return pool_->owner.recording; }
+
 void lk_stream_scratch_release(int device, unsigned uses) {
     int current = 0;
     if (hipGetDevice(&current) != hipSuccess) { (void)hipGetLastError(); return; }

@@ -188,6 +188,37 @@ def test_a_block_recorded_after_larger_calls_alone_runs_in_their_buffers(gu, dn,
         assert ((out - eager).abs() <= 1e-3 * eager.abs() + 1e-3 * eager.abs().max()).all()
 
 
+@pytest.mark.parametrize("wtype,n,k,rows,most", [(lib.TYPE_Q4_K, 4096, 4096, 200, 16), (lib.TYPE_Q6_K, 1186, 10240, 1661, 32)])
+def test_a_recorded_tiled_linear_holds_what_its_partial_products_need(wtype, n, k, rows, most):
+    """16 MiB beside the operands, 32 where the plan cuts K of a product of many rows and columns: the eager call's plan, and its bits."""
+    L = lib.load()
+    blob = dev(synth.weight(wtype, 2, k, seed=87, stream=1)).reshape(2, -1).repeat(n // 2, 1)
+    lin, x = Linear(wtype, blob, n, k), dev(synth.activation(200, k, seed=87)).repeat(9, 1)[:rows].contiguous()
+    want, out = lin(x), torch.empty((rows, n), device="cuda")
+    assert lin.path == "tiled"
+
+    def call():
+        lib.check("forward", L.lkh_qkernel_matmul_forward(lin.h, x.data_ptr(), lib.TYPE_F32, rows, out.data_ptr(), torch.cuda.current_stream().cuda_stream, 0))
+
+    side, graphs = torch.cuda.Stream(), []
+    graphs.append(record(call, side)[0])
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for _ in range(4):
+        graphs.append(record(call, side)[0])
+    torch.cuda.synchronize()
+    operands = (rows + 128) * (k // 256) * 592 * 5 / 4
+    assert free - torch.cuda.mem_get_info()[0] <= 4 * (operands + (most + 6 << 20))
+    for graph in graphs:
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    lin.close()
+    L.lkh_release_workspaces()
+    L.loken_stream_scratch_release()
+
+
 def test_dropping_the_linears_workspaces_leaves_the_mixtures_graph():
     tokens, topk, n_experts, hidden, ffn = 64, 4, 8, 512, 256
     gate, up = (dev(synth.weight(lib.TYPE_Q6_K, n_experts * ffn, hidden, seed=81, stream=i)) for i in (1, 2))
