@@ -160,10 +160,11 @@ static bool sets_of_rows_pay(int dtype, int n, int k, int rows, const void* blob
     if (rows < 17 || rows > 128 || n < 512 || k % 256 != 0 || ((uintptr_t)blob & 15) != 0) return false;   // (off a 16-byte boundary: the 32-row tiles)
     if (dtype != LK_TYPE_Q4_K && dtype != LK_TYPE_Q5_K && dtype != LK_TYPE_Q6_K) return false;
     if (dtype == LK_TYPE_Q6_K) {
-        if (k > 32768) return false;   // (not the short launch's)
-        if (rows <= 32) return n <= 4096 && (k <= 12288 || k % 2048 == 0);
-        if (rows <= 64) return n <= 2048 && (n >= 1152 || k <= 6144);
-        return n <= (rows <= 96 ? 1360 : 1024) && (n >= 1152 || k <= 5632);
+        if (!lk_rows16_q6k_short_pays(rows, n, k)) return false;
+        const int tiles = (n + 15) / 16, cus = lk_device().cus;
+        if (rows <= 32) return tiles <= cus && (k <= 12288 || k % 2048 == 0);
+        if (rows <= 64) return 2 * tiles <= cus && (n >= 1152 || k <= 6144);
+        return n >= 1152 || k <= 5632;
     }
     if (n < 1152 && k >= 4608) return false;
     const float launch = lk_rows16_short_us(rows, n, k / 256, dtype == LK_TYPE_Q5_K), weights = 1e-6f * (float)n * (float)k;

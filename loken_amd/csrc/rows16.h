@@ -52,5 +52,6 @@ int lk_rows16_q6k(const void* w, const void* q8_1, float* output, int size_m, in
 // weights off a 16-byte boundary.
 int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                         hipStream_t stream, int out_type);
+bool lk_rows16_q6k_short_pays(int size_m, int size_n, int size_k);   // (weights on a 16-byte boundary)
 // The same straight over rows of `x_type` (results in it too). -1: a call it does not serve.
 int lk_rows16_q6k_short_rows(const void* w, const void* x, float* output, int size_m, int size_n, int size_k, int x_type, hipStream_t stream);

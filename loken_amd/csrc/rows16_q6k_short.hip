@@ -374,12 +374,15 @@ int set_rows(int size_m, int size_n, int size_k) {
 
 }  // namespace
 
+bool lk_rows16_q6k_short_pays(int size_m, int size_n, int size_k) {
+    // (rows of more than 32768 values: the others' to take or refuse)
+    return size_m >= 1 && size_m <= 128 && size_n >= 1 && size_k >= 256 && size_k <= 32768 && !lk_rows16_off(size_m) && set_rows(size_m, size_n, size_k) != 0;
+}
+
 int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k, int stride_y, int ldd,
                         hipStream_t stream, int out_type) {
-    // (rows of more than 32768 values: the others' to take or refuse)
-    if (size_m < 1 || size_m > 128 || size_n < 1 || size_k < 256 || size_k > 32768 || (((uintptr_t)w) & 15) != 0 || lk_rows16_off(size_m)) return -1;
+    if ((((uintptr_t)w) & 15) != 0 || !lk_rows16_q6k_short_pays(size_m, size_n, size_k)) return -1;
     const int rows = set_rows(size_m, size_n, size_k);
-    if (rows == 0) return -1;
     const Args a{(const uint8_t*)w, (const uint8_t*)q8_1, output, size_k / 256, size_n, size_m, stride_y, ldd, out_type};
     if (rows == 32) return out_type == LK_TYPE_F32 ? launch<16, false, Q81, 2>(a, stream) : launch<16, true, Q81, 2>(a, stream);
     if (rows == 8) return out_type == LK_TYPE_F32 ? launch<8, false>(a, stream) : launch<8, true>(a, stream);
@@ -389,7 +392,8 @@ int lk_rows16_q6k_short(const void* w, const void* q8_1, float* output, int size
 // Rows of up to 4096 values straight from them where sets of eight are a workgroup to the CU, as lk_rows16_short_rows (672 x 1024 at 18 rows 9.6 us a call,
 // 5.8 on the chip / 6.3, 4.2; 640 x 3584 at 44 9.2, 7.9 / 7.4, 7.5).
 int lk_rows16_q6k_short_rows(const void* w, const void* x, float* output, int size_m, int size_n, int size_k, int x_type, hipStream_t stream) {
-    if (size_m < 1 || size_m > 128 || size_n < (size_m > 16 ? 512 : 1) || size_k < 256 || size_k > 4096 || (((uintptr_t)w) & 15) != 0 || lk_rows16_off(size_m) || set_rows(size_m, size_n, size_k) != 8) return -1;
+    if (size_k > 4096 || (((uintptr_t)w) & 15) != 0 || !lk_rows16_q6k_short_pays(size_m, size_n, size_k) || set_rows(size_m, size_n, size_k) != 8) return -1;
+    if (size_m > 16 && size_n < 512) return -1;   // (a call recorded with nothing reserved stays refused there, as in rows16_short.hip)
     const Args a{(const uint8_t*)w, (const uint8_t*)x, output, size_k / 256, size_n, size_m, 0, size_n, x_type};
     if (x_type == LK_TYPE_F32) return launch<8, false, ROWS_F32>(a, stream);
     return x_type == LK_TYPE_F16 ? launch<8, true, ROWS_F16>(a, stream) : launch<8, true, ROWS_BF16>(a, stream);

@@ -588,3 +588,16 @@ def test_q6k_weights_off_a_piece_keep_the_tiles_where_sets_of_rows_would_pay():
         got, path = lin(dev(x)), lin.path
         lin.close()
         assert path == expect and close(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("name,n,k,rows", [("q6_k", 4000, 6144, 24), ("q6_k", 1360, 5632, 96), ("q4_k", 2986, 6144, 26)])
+def test_without_the_short_launches_their_rows_keep_the_tiles(name, n, k, rows, knobs):
+    w, x = np.tile(synth.weight(DT[name], 50, k, seed=99, stream=3).reshape(50, -1), ((n + 49) // 50, 1))[:n], synth.activation(rows, k, seed=99)
+    lin, xd = Linear(DT[name], dev(w), n, k), dev(x)
+    want = np.tile(oracle.ob_matmul(DT[name], x, w[:50], 50), (1, (n + 49) // 50))[:, :n]
+    got = lin(xd)
+    assert lin.path == "rows-on-matrix-unit" and close(got.cpu().numpy(), want)
+    knobs.set("LK_TUNE_ROWS16_OFF")
+    got = lin(xd)
+    assert lin.path == "tiled" and close(got.cpu().numpy(), want)
+    lin.close()
