@@ -61,13 +61,14 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
     // ---- the weights: load u of a super-block is piece 64 u + lane of its 16 x 14 (sixteen rows are whole pieces: a tile is aligned)
     constexpr int LOADS = (TILE * BLOCK_PIECES + 63) / 64;   // 4, the last half used
     const uint8_t* w_tile = (const uint8_t*)(to_gbytes(p.w) + (size_t)tile * TILE * row_bytes);
-    uint32_t w_at[LOADS], w_piece[LOADS];
+    // (w_at with the piece's offset in it, a register a load. With the two apart the kernel over f16 rows took 91 registers for 78 and the compiler
+    // waited for each of its activation loads before the next: 9136 x 2304 at 5 rows 16.8 us, 11.3; sixteen rows spilled one: 3 % at 13 rows.)
+    uint32_t w_at[LOADS];
     int w_to[LOADS];
 #pragma unroll
     for (int u = 0; u < LOADS; ++u) {
         const int id = min(64 * u + lane, TILE * BLOCK_PIECES - 1), row = id / BLOCK_PIECES;
-        w_piece[u] = (uint32_t)(16 * (id % BLOCK_PIECES));
-        w_at[u] = (uint32_t)(min(row, last_row) * row_bytes);
+        w_at[u] = (uint32_t)(min(row, last_row) * row_bytes + 16 * (id % BLOCK_PIECES));
         w_to[u] = row * PITCH + 16 * (id % BLOCK_PIECES) + 16;
     }
     const uint32_t my_at = (uint32_t)(min(l16, last_row) * row_bytes);   // of the lane's own row
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES, 1) void q6k_rows16_short_kernel(Arg
     auto load_w = [&](Weights& b, int kb) {
         const uint32_t at = (uint32_t)(kb * Q6K_BYTES);
 #pragma unroll
-        for (int u = 0; u < LOADS; ++u) b.w[u] = *(const u32x4*)(w_tile + (((w_at[u] + at) & ~15u) + w_piece[u]));
+        for (int u = 0; u < LOADS; ++u) b.w[u] = *(const u32x4*)(w_tile + ((w_at[u] + at) & ~15u));
     };
 
     auto settle = [] {   // the wave's own LDS writes before its reads of other lanes' data
