@@ -219,7 +219,8 @@ extern "C" int lk_moe_forward(int wtype_gu, int wtype_down, const float* x, cons
     if (!(path & LK_MOE_GROUPED)) {
         if (fg->wire < 0 || fd->wire < 0) return LK_ERR_TYPE;
         float* h = (float*)scratch.get(LK_SCRATCH_BLOCK, (size_t)rows * ffn * 4);
-        const size_t more = lk_moe_pairs_scratch(fg->wire, fd->wire, x, h, down, topk, rows, hidden, ffn);
+        // (asked for ahead only where it may be refused for good: a block of one token is bound by the host)
+        const size_t more = scratch.recording() ? lk_moe_pairs_scratch(fg->wire, fd->wire, x, h, down, topk, rows, hidden, ffn) : 0;
         if (h && (more == 0 || scratch.get(LK_SCRATCH_LAUNCHER, more))) {
             if (int rc = lk_moe_pairs_gate_up(fg->wire, x, gate, up, choices, h, n_experts, topk, rows, ffn, hidden, s)) return rc;
             return lk_moe_pairs_down(fd->wire, h, down, choices, topk_weights, out, n_experts, topk, rows, hidden, ffn, s);
