@@ -93,16 +93,19 @@ const Tiles* tiles_of(int wtype) {
 // every tile width with K whole and cut into 2 to 12 ranges) for the plan it picks: 0.7 % longer in the mean than the best one of the sweep (the items' times
 // are what makes it pick well, no more: a plan of each kind measured alone gives others). alone /
 // full: nanoseconds an item (32 x 32 x 32 product) takes a SIMD with one workgroup on its CU or two, by token
-// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items. (As fitted to whole launches whose workgroups
-// were dealt unevenly to the XCDs, with K cut into even ranges only, the picks were 3.8 % behind.)
+// tiles; wide: with eight waves and tt = 4. start: microseconds of a workgroup beside its items. whole: how far rounds of workgroups stay apart
+// (1: whole rounds). (As fitted to whole launches whose workgroups were dealt unevenly to the XCDs, with K cut into even ranges only, the picks were
+// 3.8 % behind.) Q8_0 and Q4_0, whose items are longer, from 3100 shapes of their own (0.5 and 0.3 % behind the best; with the K-quants' blurred rounds 0.8 and 0.4, by more where a
+// vocabulary meets a few rows, as K was left whole: Q8_0 79538 x 3328 at 14 129 us against 116 in two ranges, Q4_0 80340 x 3840 at 13 109 / 101, and in rounds that
+// are just full: Q8_0 16060 x 7424 at 23 65 in two ranges, 56 in four).
 struct ItemTimes {
-    double alone[4], full[4], wide, start;
+    double alone[4], full[4], wide, start, whole;
 };
-constexpr ItemTimes ONE_TERM = {{162, 111, 121, 93.8}, {137, 93.6, 82.2, 75.7}, 72.6, 0.357}, TWO_TERMS = {{239, 146, 166, 152}, {221, 140, 124, 122}, 0, 1.30},
-                    Q8_ITEM = {{265, 159, 181, 0}, {253, 149, 124, 0}, 0, 1.71}, Q4_ITEM = {{250, 164, 181, 146}, {216, 144, 125, 114}, 0, 0.0919};
+constexpr ItemTimes ONE_TERM = {{162, 111, 121, 93.8}, {137, 93.6, 82.2, 75.7}, 67.4, 0.357, 0.655}, TWO_TERMS = {{239, 146, 166, 152}, {221, 140, 124, 122}, 0, 1.30, 0.655},
+                    Q8_ITEM = {{267, 164, 179, 0}, {218, 150, 123, 0}, 0, 0.98, 1}, Q4_ITEM = {{249, 164, 180, 145}, {217, 145, 128, 114}, 0, 0.06, 1};
 
 // The tile and the cut of K with the shortest estimated launch. Up to 2 * cus workgroups run at once, and a CU that holds two takes
-// nearly the time of a full chip; past that the rounds blur (two thirds of whole rounds, one of their share)
+// nearly the time of a full chip; past that the rounds blur (K-quants: two thirds of whole rounds, one of their share)
 // but for the start of each, without which Q6_K 9675 x 9728 at 23 rows was cut into ten (52 us; into six, the most that is one round, 42). Of two workgroups on a CU with ranges
 // of unequal length not both are the longest: two thirds of it, one of the mean. A cut costs a launch and its
 // partial products, written, read and added.
@@ -122,7 +125,7 @@ MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup, 
             const int64_t groups = tiles * splits, rounds = groups / (2 * cus), rest = groups % (2 * cus);
             double us = rounds * two;
             if (rest > 0) us += rest <= cus ? one : one + (two - one) * (0.779 + 0.221 * (rest - cus) / cus);
-            if (rounds > 0) us = 0.655 * us + 0.345 * two * groups / (2 * cus);
+            if (rounds > 0) us = t.whole * us + (1 - t.whole) * two * groups / (2 * cus);
             us += 2.38 * (double)((groups - 1) / (2 * cus));
             if (splits > 1) us += 1.85 + 0.227e-6 * (splits + 1) * pb.m_end * pb.n * 4;
             if (us < least) least = us, best = {tt, 4, splits};
@@ -132,7 +135,8 @@ MmqTilePlan plan_dense(const Tiles& f, const MmqProblem& pb, const void* fixup, 
     if (t.wide > 0 && forced_splits <= 0 && (forced_tt <= 0 || forced_tt == 8)) {
         const int64_t tiles = ((pb.n + 255ll) / 256) * ((pb.m_end + 127ll) / 128), rest = tiles % cus;
         const double round = 64e-3 * pb.nb * t.wide;
-        if (round * (tiles / cus + (rest > 0 ? 0.972 + 0.028 * rest / cus : 0.0)) < least) best = {4, 8, 1};
+        // (4.5 us the start of a round: without it short rows were taken here too, 13367 x 1536 of Q5_K at 1573 rows 131 us, with four waves 125)
+        if (round * (tiles / cus + (rest > 0 ? 0.8 + 0.2 * rest / cus : 0.0)) + 4.5 * ((tiles + cus - 1) / cus) < least) best = {4, 8, 1};
     }
     return best;
 }
