@@ -138,19 +138,23 @@ int matvec_rows(int dtype, int k) {
 //         4096 x 14336     21.4 / 34.0   22.0 / 34.1   35.8 / 34.5   36.7 / 35.2   48.5 / 34.8   82.2 / 52.1
 // Once the tiles were dealt evenly to the XCDs they took over (rows kernel / tiles):
 //   Q6_K, 17 to 32 rows, more than 2048 matrix rows of more than 4352 values, or past 20 M weights where the 16-row tiles have no
-//     granules: 3018 x 6144 at 27 28.3 / 19.6; 4708 x 5376 at 26 26.7 / 21.0; 2165 x 7424 at 21 21.1 / 19.0; 6412 x 3584 at 29 23.3 / 19.8
-//     (4145 x 4096 at 21 16.7 / 18.6; 2977 x 4352 at 31 16.5 / 18.1; 9054 x 1792 at 19 16.6 / 17.2, and of fewer than 2560 values up to 40 M:
-//     14483 x 1792 at 18 16.9 / 20.4; 1833 x 11264 at 24 18.3 / 22.8)
-//   Q6_K, 33 to 64 rows of fewer than 3072 values, past 320000 results: 9987 x 1536 at 36 23.9 / 18.5 (6621 x 1536 at 46 16.2 / 17.3)
+//     granules: 4708 x 5376 at 26 26.7 / 21.0; 2165 x 7424 at 21 21.1 / 19.0; 6412 x 3584 at 29 23.3 / 19.8
+//     (4145 x 4096 at 21 16.7 / 18.6; 2977 x 4352 at 31 16.5 / 18.1; 9054 x 1792 at 19 16.6 / 17.2; 1833 x 11264 at 24 18.3 / 22.8)
+//     The 32-row tiles stay up to 40 M where a row is less than ten super-blocks, twelve or sixteen (14483 x 1792 at 18 16.9 / 20.4; 11261 x 3072 at 25 21.7 / 23.5;
+//     ten from 9216 matrix rows on: 13147 x 2560 at 20 20.5 / 22.0, 8239 x 2560 at 27 20.4 / 21.2), and of rows of up to 24 where they are one round and the 16-row tiles
+//     three or more to two CUs (6881 x 4608 at 30 19.7 / 22.6; 8073 x 4352 at 17 20.3 / 22.3; 5325 x 4608 at 24, 16-row tiles, 25.0 / 19.4)
+//   Q6_K, 33 to 64 rows of fewer than 3072 values, past 320000 results: 9987 x 1536 at 36 23.9 / 18.5 (6621 x 1536 at 46 16.2 / 17.3); not where
+//     they are two rounds at most of 2048 values or fewer (7315 x 1024 at 60 11.6 / 16.2; 6829 x 1536 at 52 16.0 / 17.4; 5062 x 2304 at 64 21.9 / 18.2)
 //   Q4_K and Q5_K, rows of 3328 to 4096 values, 17 to 32 over fewer than 4096 matrix rows, and more where there are at most 128 items:
 //     2077 x 3584 at 26 14.6 / 13.2; 962 x 3840 at 27 14.6 / 13.2; 627 x 4096 at 71 17.0 / 14.4; 1184 x 3584 at 58 14.8 / 13.4
 //     (5246 x 3840 at 28 15.6 / 16.0; 1462 x 3584 at 124 15.6 / 17.6)
-// Left where they were: Q6_K, 65 rows and more over fewer than 1024 matrix rows of 2560 to 5632 values (548 x 3584 at 154 23.0 / 17.4).
+// Left where they were: Q6_K, 65 rows and more over fewer than 1024 matrix rows of 2560 to 5632 values (548 x 3584 at 154 23.0 / 17.4); 17 to 32 over
+// 4097 to 6144 of 6144 (4642 x 6144 at 18 21.2 / 22.9).
 //
 // 17 to 128 rows as sets of sixteen in the short launches (rows16_short.hip, rows16_q6k_short.hip) moved lines the other way, quantizer and
 // rows kernel / tiles:
 //   Q4_K and Q5_K, where 1.1 times what the launch and its quantizer take (5.3 us and 0.81 of the launch in a graph, fitted to 1460 shapes) is under what the tiles
-//     take (fitted too, 9 %): 2986 x 6144 at 26 11.3 / 18.3; 2665 x 6144 at 36 11.5 / 19.4; 805 x 3840 at 60 9.1 / 13.9; 1256 x 5120 at 70 10.7 /
+//     take (fitted too, 9 %), 1.2 times past 22 us and at 512 values, where both fits are at their ends (7930 x 11264 at 64 48.5 / 36.4, 6102 x 512 at 125 10.1 / 9.1): 2986 x 6144 at 26 11.3 / 18.3; 2665 x 6144 at 36 11.5 / 19.4; 805 x 3840 at 60 9.1 / 13.9; 1256 x 5120 at 70 10.7 /
 //     17.3; 932 x 4096 at 127 10.2 / 16.2; 4060 x 14336 at 46 31.1 / 27.8; Q5_K 3456 x 5632 at 19 12.1 / 18.4, 1344 x 6144 at 44 11.2 / 17.8
 //   Q6_K, where the launch takes the call: 3840 x 6656 at 26 15.2 / 21.7; 1664 x 7168 at 36 15.3 / 21.1, at 58 15.8 / 22.4; 1344 x 4096 at 95 12.9 /
 //     20.2
@@ -168,7 +172,8 @@ static bool sets_of_rows_pay(int dtype, int n, int k, int rows, const void* blob
     }
     if (n < 1152 && k >= 4608) return false;
     const float launch = lk_rows16_short_us(rows, n, k / 256, dtype == LK_TYPE_Q5_K), weights = 1e-6f * (float)n * (float)k;
-    return launch >= 0.f && 1.1f * (5.3f + 0.81f * launch) < 10.2f + 0.00063f * (float)k + weights * (0.026f + 0.0041f * (float)rows);
+    const float rows_us = 5.3f + 0.81f * launch;
+    return launch >= 0.f && (rows_us > 22.f || k <= 512 ? 1.2f : 1.1f) * rows_us < 10.2f + 0.00063f * (float)k + weights * (0.026f + 0.0041f * (float)rows);
 }
 
 static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
@@ -180,8 +185,11 @@ static bool rows_kernel_serves(int dtype, int n, int k, int rows) {
     const long long items = (n + 31ll) / 32 * ((rows + 31) / 32);
     if (dtype == LK_TYPE_Q6_K) {
         if (rows <= 16) return k % 2048 == 0 || k < 4608 || n <= 12288;
-        if (rows <= 32) return n <= 2048 || (k <= 4352 && weights <= (k % 2048 == 0 || k < 2560 ? 40ll << 20 : 20ll << 20));
-        if (rows <= 64) return n <= 1024 || (k < 3072 ? results <= 320000 : k <= 6144 && weights <= (17ll << 20));
+        if (rows <= 32) {
+            if (n <= 2048 || (k > 4096 && k <= 6144 && n > 6144 && items <= 256)) return true;
+            return k <= 4352 && weights <= (k % 2048 == 0 || k < 2560 || k == 3072 || (k == 2560 && n >= 9216) ? 40ll << 20 : 20ll << 20);
+        }
+        if (rows <= 64) return n <= 1024 || (k < 3072 ? results <= 320000 || (k <= 2048 && items <= 512) : k <= 6144 && weights <= (17ll << 20));
         if (k < 5632 && n < 1024 && rows > 128 && items <= 256) return true;
         return (k < 3072 || (n < 1024 && k < 4608)) && results <= 450000;
     }

@@ -576,6 +576,17 @@ def test_the_lines_that_moved_to_sets_of_rows(name, n, k, rows, expect):
     test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
 
 
+
+@pytest.mark.parametrize("name,n,k,rows,expect", [
+    ("q6_k", 8192, 1024, 64, "rows-on-matrix-unit"), ("q6_k", 8196, 1024, 64, "tiled"), ("q6_k", 7000, 2048, 49, "rows-on-matrix-unit"),
+    ("q6_k", 6000, 2304, 60, "tiled"), ("q6_k", 6145, 4608, 30, "rows-on-matrix-unit"), ("q6_k", 6144, 4608, 30, "tiled"),
+    ("q6_k", 8192, 6144, 17, "rows-on-matrix-unit"), ("q6_k", 8196, 4352, 17, "tiled"), ("q6_k", 11264, 3072, 25, "rows-on-matrix-unit"),
+    ("q6_k", 13660, 3072, 25, "tiled"), ("q6_k", 9216, 2560, 20, "rows-on-matrix-unit"), ("q6_k", 9215, 2560, 20, "tiled"),
+    ("q4_k", 7930, 11264, 64, "tiled"), ("q4_k", 6102, 512, 125, "tiled"), ("q4_k", 2986, 6144, 26, "rows-on-matrix-unit")])
+def test_the_lines_where_the_tiles_or_the_sets_had_been_slower(name, n, k, rows, expect):
+    test_both_sides_of_the_lines_around_the_rows_kernels(name, n, k, rows, expect)
+
+
 def test_q6k_weights_off_a_piece_keep_the_tiles_where_sets_of_rows_would_pay():
     n, k, rows = 4000, 6144, 24
     w, x = synth.weight(DT["q6_k"], 50, k, seed=98, stream=3).reshape(50, -1), synth.activation(rows, k, seed=98)
