@@ -697,8 +697,8 @@ int lk_moe_q4k_rows_grouped(const void* weights, const void* weights_second, int
  * cuda/moe/gguf.cuh:782-816); the host mirror of QKernelMatMul::forward uses it between the mat-vec
  * kernels and the tiled matmul. LK_ERR_ARG, and nothing launched, for rows too long for the kernel's
  * scale table in LDS.
- * A row's result depends on the matrix and on whether the call has up to 8, 16, 32, 48, 64 or more rows (Q4_K and Q5_K
- * above: 8, 16 or more), not on how many or which the other rows are; from one class to another the sums' order may differ. */
+ * A row's result depends on the matrix and on whether the call has up to 8, 16, 32, 48, 64, 96, 128 or more rows (Q4_K and Q5_K
+ * above alike), not on how many or which the other rows are; from one class to another the sums' order may differ. */
 int lk_dense_q6k_rows(const void* w, const void* q8_1, float* output, int size_m, int size_n, int size_k,
                       void* stream);
 /* Q4_K weight [nrows_x, ncols_x] x ONE plain Q8_1 row -> dst [nrows_x] f32. Name and arguments of the

@@ -431,7 +431,7 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
 
 // Matrices of up to four row tiles to the CU, fewer or more by the class of row counts: beyond, the launches that stage the activation once and walk
 // many tiles are level or ahead; above a tile to the CU rows of 2048 values or more. A choice by the matrix and the class of row counts alone (up to
-// 8, 16, 32, 64, 96, 128), so that several matrices in one launch carry the bits of one launch each and a row carries the same bits whatever rides
+// 8, 16, 32, 48, 64, 96, 128), so that several matrices in one launch carry the bits of one launch each and a row carries the same bits whatever rides
 // with it in its class. Measured in a graph, Q4_K, us, staged launches against this:
 //   3 / 8 rows   1024 x 2048 5.1, 5.2 / 3.7, 3.7; 4096 x 4096 7.7, 8.1 / 5.1, 5.0; 4096 x 14336 17.9, 19.4 / 12.0, 11.9; 6144 x 2048 5.5, 5.5 / 4.9, 4.9;
 //                8192 x 4096 8.8, 9.1 / 7.3, 7.2; 5000 x 12288 16.7, 17.8 / 14.7, 15.0; 14336 x 4096 12.6, 13.3 / 10.6, 10.5; 8192 x 1024 4.2, 4.1 / 4.0, 4.2;
@@ -448,7 +448,9 @@ int lk_rows16_short(const LkRows16& a, bool dual, bool q5, hipStream_t stream) {
 //                   12.9, 14.7 / 10.7, 11.2 (22.1, 24.0 / 20.4, 20.5); 4096 x 14336 35.2, 39.4 / 18.0, 19.4; 12288 x 2048 11.5, 13.3 / 10.0, 10.1
 //                   (19.8, 22.9 / 15.1, 15.4); 14336 x 4096 18.7, 23.7 / 19.6, 20.0 (31.4, 38.6 / 38.2, 38.6)
 //   48 / 64         2048 x 2048 8.3, 8.4 / 5.1, 5.2; 4096 x 4096 13.3, 14.3 / 11.1, 11.1 (22.6, 23.8 / 19.2, 19.6); 8192 x 4096 20.6, 23.2 / 17.7, 19.3
-//                   (34.3, 37.9 / 29.2, 37.9); 14336 x 4096 34.1, 37.7 / 27.9, 35.7 (60.1, 65.7 / 55.5, 65.5); 32768 x 2048 34.9, 37.3 / 26.6, 33.1
+//                   (34.3, 37.9 / 29.2, 37.9); 14336 x 4096 34.1, 37.7 / 27.9, 35.7 (60.1, 65.7 / 55.5, 65.5); 32768 x 2048 34.9, 37.3 / 26.6, 33.1;
+//                   at 49 to 64 rows past three tiles to the CU not those of more than 4096 values: 15880 x 5632 at 56 41.2 / 46.2, 13850 x 13568 at 51
+//                   82.5 / 89.4 (8342 x 13568 at 60 85.6 / 67.9; at 38 rows 9304 x 11776 70.1 / 41.5)
 //   96 / 128        2048 x 2048 8.6, 8.7 / 6.7, 6.7; 4096 x 4096 21.1, 22.9 / 17.0, 19.0 (35.1, 37.5 / 27.9, 36.3); 8192 x 4096 34.3, 36.9 / 27.1, 35.0
 //                   (62.0, 64.6 / 55.3, 72.5); 14336 x 4096 51.2, 63.3 / 51.5, 60.1 (93.1, 118.6 / 99.3, 126.6)
 //   Q5_K, 32 / 64   2048 x 2048 8.8, 8.8 / 4.6, 5.8; 4096 x 4096 14.7, 15.1 / 9.3, 15.2 (24.8, 25.2 / 17.9, 30.2); 8192 x 2048 10.0, 14.2 / 9.2, 13.9 (16.3,
@@ -464,7 +466,7 @@ bool lk_rows16_short_pays(int m, int n, int nb, bool q5) {
     // with the quantizer 2767 x 1280 at 113 11.2 / 12.1)
     if (nb == 5 || nb == 6) return (int64_t)tiles * (m <= 32 ? 2 : m <= 64 ? 4 : m <= 96 ? 6 : 8) <= (m <= 64 ? 12 : 4) * cus;
     if (nb <= 8) return tiles <= 16 * cus;
-    return tiles <= (m <= 32 ? 2 : m <= 64 ? 4 : m <= 96 ? 2 : 1) * cus;
+    return tiles <= (m <= 32 ? 2 : m <= 48 ? 4 : m <= 64 ? (nb <= 16 ? 4 : 3) : m <= 96 ? 2 : 1) * cus;
 }
 
 float lk_rows16_short_us(int m, int n, int nb, bool q5) {
