@@ -171,8 +171,8 @@ __global__ __launch_bounds__(64 * LOGIT_WAVES) void gate_logits16_kernel(const f
 // A few tokens: 16 x 16 tiles, rows straight from memory, the choice in the same launch. A workgroup is twice the four waves
 // that share a partial sum; the last one of the launch to arrive (its stream's counter, which wraps to zero with it)
 // reads all partial sums and gives a wave to each token. Its tail (the stores' way to memory, the counter, the partial sums, the choice:
-// 3 us) takes what the second launch takes, so what it saves is the host's time for that launch, which bounds a call of so little work: one to eight
-// tokens called one by one 11.0 -> 8.6 us. Replayed in a graph, one launch against two (128 experts of 2048, 1 / 4 / 8 / 16 tokens):
+// 3 us) takes what the second launch takes, so what it saves is the host's time for that launch, which bounds a call of so little work: one to four
+// tokens called one by one 11.0 -> 8.6 us. Replayed in a graph, one launch against the two as they are now (128 experts of 2048, 1 / 4 / 8 / 16 tokens):
 // 6.1 / 6.2 / 7.1 / 10.4 us against 5.4 / 5.7 / 5.9 / 6.0; 128 of 3072 6.4 / 6.6 / 7.6 / 10.9 against 5.6 / 5.9 / 6.2 / 6.3. So up to
 // CHOICE_TOKENS tokens take it, outside a recording. Sums in the order of the two launches, hence the same bits.
 __device__ uint32_t g_arrived[LK_SCRATCH_TICKETS];

@@ -483,7 +483,9 @@ float lk_rows16_short_us(int m, int n, int nb, bool q5) {
 int lk_rows16_short_rows(const LkRows16& a, bool q5, hipStream_t stream) {
     const int tiles = (a.n[0] + TILE - 1) / TILE;
     if (a.count != 1 || a.nb < 1 || a.nb > GROUPS || !lk_rows16_short_pays(a.m, a.n[0], a.nb, q5)) return -1;
-    if (a.m > 16 && a.n[0] < 512) return -1;   // (a call recorded with nothing reserved stays refused over the smallest matrices)
+    // Fewer than 512 matrix rows keep the quantizer's launch above sixteen rows though one launch is faster (a call of 17 to 48 rows 6.8 us, 4.0 to 5.8): a
+    // program that records such a call with nothing reserved is refused, and goes on being refused.
+    if (a.m > 16 && a.n[0] < 512) return -1;
     if (a.m > 8 && tiles * ((a.m + 7) / 8) > (a.nb <= 4 ? 3 : a.nb <= 8 ? 2 : 1) * lk_device().cus) return -1;
     if (a.x_type == LK_TYPE_F32) return q5 ? launch_rows<true, F32, ROWS_F32>(a, tiles, stream) : launch_rows<false, F32, ROWS_F32>(a, tiles, stream);
     if (a.x_type == LK_TYPE_F16) return q5 ? launch_rows<true, ANY, ROWS_F16>(a, tiles, stream) : launch_rows<false, ANY, ROWS_F16>(a, tiles, stream);
