@@ -13,9 +13,13 @@
 // (r, j, q) of a wave then holds, for the whole launch, the Q8_1 codes of quarter q of every
 // super-block of activation row j in registers, and per pass loads the matching quarter of weight
 // row r of expert e_j: 4 lanes per (row, expert), 4 * TKP lanes per output row. The four lanes'
-// shares meet over DPP, the topk pair totals are weighted and summed in slot order, exactly the
-// order of the fold kernel, and one lane stores the output element. No scratch, no atomics, and
+// shares meet over DPP, the topk pair totals are weighted and wait in LDS, and at the end a lane sums a row's in slot order,
+// exactly the order of the fold kernel, and stores the output element. No scratch, no atomics, and
 // the same bits as the two launches give.
+//
+// What bounds it: vector issue (sixteen tokens of 768 -> 2048, top-8: two workgroups a CU, the vector unit active 70 % of the time). Hence the
+// totals' way through LDS and Q4_K's high nibbles left in place (q4k_dots_biased): 2985 vector instructions a wave -> 2527, the launch 18.2 us -> 15.3
+// with the weights in a cache, the whole block with them from HBM 59.5 -> 58.5, at 20 tokens 78.9 -> 76.7.
 
 #include "mmvq_core.h"
 
@@ -43,7 +47,8 @@ struct LaneQ4K {
     };
     struct A {
         uint4 a00, a01, a10, a11;
-        float4 s4;
+        float4 s4;     // Q4_K: the second d over 16 (q4k_dots_biased)
+        int hi_init;   // and what its high nibbles' dot starts from
     };
     static __device__ __forceinline__ void load(W& f, const uint8_t* bp, int q) {
         f.hdr = *(const uint4*)(bp);
@@ -61,6 +66,11 @@ struct LaneQ4K {
         a.a10 = *(const uint4*)(codes + 32);
         a.a11 = *(const uint4*)(codes + 48);
         a.s4 = *(const float4*)(rowl + table + (b * 8 + 2 * q) * 8);
+        if (!Q5) {
+            const uint4 ones = make_uint4(0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u);
+            a.hi_init = 128 * dot16(ones, a.a11, dot16(ones, a.a10, 0));
+            a.s4.z *= 0.0625f;
+        }
     }
     static __device__ __forceinline__ float share(const W& f, const A& a, int q) {
         const Q4KScaleSel sel(q);
@@ -72,8 +82,11 @@ struct LaneQ4K {
             q5k_dots(f.q0, shr4(f.h0, 2 * q), a.a00, a.a10, d_lo, d_hi);
             q5k_dots(f.q1, shr4(f.h1, 2 * q), a.a01, a.a11, d_lo, d_hi);
         } else {
-            q4k_dots(f.q0, a.a00, a.a10, d_lo, d_hi);
-            q4k_dots(f.q1, a.a01, a.a11, d_lo, d_hi);
+            uint32_t flip = 0x80808080u;
+            asm("" : "+v"(flip));   // in a register: the bit instruction takes no literal
+            d_hi = a.hi_init;
+            q4k_dots_biased(f.q0, a.a00, a.a10, flip, d_lo, d_hi);
+            q4k_dots_biased(f.q1, a.a01, a.a11, flip, d_lo, d_hi);
         }
         return q4k_pair_share(dd, dmin, (float)(sc & 0xFFu), (float)(sc >> 8), (float)(mn & 0xFFu), (float)(mn >> 8),
                               a.s4.x, a.s4.z, a.s4.y, a.s4.w, (float)d_lo, (float)d_hi);
@@ -129,11 +142,12 @@ struct FoldDims {
 
 constexpr int SCAN_ROUNDS = 2;              // sorted routing entries a lane looks at: pairs <= 2 * 256
 constexpr int MAX_PAIRS = SCAN_ROUNDS * WG;
+constexpr int MAX_PASSES = 16;
 
 template <class L, int NB>
 struct FoldFrag {
     typename L::W w[NB];
-    float prev, bias;
+    float bias;
 };
 
 template <class L, int NB, int TKP>
@@ -156,6 +170,8 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
     constexpr int ACT_LOADS = (TKP * QUADS + WG - 1) / WG;
     __shared__ __align__(16) uint8_t lds[TKP * PITCH];
     __shared__ int e_of[TKP];
+    // the pairs' totals, [wave][row][slot], in the slot order that the sum takes them in
+    __shared__ __align__(16) float totals[WAVES][MAX_PASSES * RPW][TKP];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -208,13 +224,16 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
     const float* before = add_after ? add_after : out;
     auto load = [&](FoldFrag<L, NB>& f, int p) {
         const int row = min((group0 + p) * RPG + wave * RPW + r, d.cols - 1);
-        const uint8_t* bp = (const uint8_t*)(slab + (size_t)row * (NB * L::BYTES));
+        const uint8_t* bp = (const uint8_t*)(slab + (size_t)(uint32_t)row * (NB * L::BYTES));
 #pragma unroll
         for (int b = 0; b < NB; ++b) L::load(f.w[b], bp + b * L::BYTES, q);
-        f.prev = d.write ? 0.f : before[out_at + row];
         f.bias = down_bias ? down_bias[(size_t)(routed ? e : 0) * d.cols + row] : 0.f;
     };
     FoldFrag<L, NB> fa, fb;
+    // at the end lane i sums the wave's i-th row (row i % RPW of pass i / RPW)
+    const int my_row = (group0 + lane / RPW) * RPG + wave * RPW + lane % RPW;
+    const bool mine = lane < d.passes * RPW && my_row < d.cols;
+    const float prev = d.write || !mine ? 0.f : before[out_at + my_row];
     load(fa, 0);
     load_fence(w);
 
@@ -246,17 +265,19 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
         const float acc = (quad[0] + quad[1]) + (quad[2] + quad[3]);
         float v = acc * scale;
         if (down_bias) v += scale * f.bias;
-        const int bits = __float_as_int(routed ? v : 0.f);
-        const int prev_bits = __float_as_int(f.prev);
+        if (q == 0) totals[wave][p * RPW + r][j] = routed ? v : 0.f;
+    };
+    // (Read from other lanes' registers and added in every pass they were 44 vector instructions of its 300, for two rows.)
+    auto finish = [&] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (!mine) return;
+        const float* t = totals[wave][lane];
+        float sum = add_after ? 0.f : prev;
 #pragma unroll
-        for (int rr = 0; rr < RPW; ++rr) {
-            float sum = add_after ? 0.f : __int_as_float(__builtin_amdgcn_readlane(prev_bits, rr * LPR));
-#pragma unroll
-            for (int jj = 0; jj < TKP; ++jj) sum += __int_as_float(__builtin_amdgcn_readlane(bits, rr * LPR + 4 * jj));
-            if (add_after) sum += __int_as_float(__builtin_amdgcn_readlane(prev_bits, rr * LPR));
-            const int row = (group0 + p) * RPG + wave * RPW + rr;
-            if (lane == rr * LPR && row < d.cols) out[out_at + row] = sum;
-        }
+        for (int jj = 0; jj < TKP; ++jj) sum += t[jj];
+        if (add_after) sum += prev;
+        out[out_at + my_row] = sum;
     };
 
     // Passes ping-pong between two fragments; a load past the last pass re-reads it (never a branch
@@ -264,6 +285,7 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
     const int last = d.passes - 1;
     if (last == 0) {
         compute(fa, 0);
+        finish();
         return;
     }
     for (int p = 0;; p += 2) {
@@ -274,6 +296,7 @@ __global__ __launch_bounds__(WG) void moe_down_fold_kernel(const uint8_t* __rest
         compute(fb, p + 1);
         if (p + 2 > last) break;
     }
+    finish();
 }
 
 struct FoldCall {
@@ -297,7 +320,7 @@ int launch(const FoldCall& c, FoldDims d) {
     int passes = (int)(((int64_t)c.tokens * groups + 2 * lk_device().cus - 1) / (2 * lk_device().cus));
     passes = passes <= 1 ? 1 : passes <= 2 ? 2 : passes <= 5 ? 4 : 8;   // (12 passes: 57 us at 16 tokens, 88 at 24 against 81)
     if (const int t = lk_tune_env("LK_TUNE_DOWN_FOLD_PASSES")) passes = t;
-    passes = passes < 1 ? 1 : passes > 16 ? 16 : passes;
+    passes = passes < 1 ? 1 : passes > MAX_PASSES ? MAX_PASSES : passes;
     d.passes = passes;
     d.slab_bytes = (int64_t)d.cols * NB * L::BYTES;
     const dim3 grid((groups + passes - 1) / passes, c.tokens);
