@@ -417,7 +417,13 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
 // The gate / up pair per routed (token, expert) pair of an MoE layer: grid.y names the pair, whose
 // expert picks the two slabs, whose token picks the f32 activation row and whose slot picks the
 // output row (the conventions of loken_moe_gemm_gguf_gate_up_silu_mul, cuda/moe/moe_gguf.cu:896-1060
-// of the reference). Everything else is the pair kernel above.
+// of the reference). Everything else is the pair kernel above, but for two things, because this launch is bound by vector
+// issue (sixteen tokens, 128 pairs of 768 x 2048: four workgroups on every CU, the vector unit active 80 % of the time, a
+// wave's six tiles 1290 instructions): a row's place is a 32-bit offset from the slab, where 64-bit products were sixteen issue
+// slots a tile, and a tile's totals wait in lanes of their own, so that the activation (an exponential and a division, a
+// fifth of a tile) runs once for up to GROUP / 4 tiles instead of once a tile for two lanes of it: 1290 -> 1078. Whole block of 128 experts of 2048 -> 768, top-8, weights
+// from HBM, before and after, with the grid's rule in launch_moe_pair: 4 / 9 / 12 tokens 27.0 / 58.7 / 54.0 us -> 24.8 / 57.2 / 53.7 (9: a Q6_K down), 60 experts of
+// 1536 -> 1024, top-4, at 12 tokens 35.0 -> 31.2; 16 tokens, which the weights' bytes bound, 59.0 -> 59.5.
 struct RegMoeArgs {
     const int32_t* sorted_token_ids;   // null: pair i is slot i
     const int32_t* expert_ids;
@@ -439,30 +445,49 @@ __global__ __launch_bounds__(RT) void q4k_reg_moe_pair_kernel(const uint8_t* __r
     const Geo<RP> g(nb);
     const Q4KScaleSel sel(g.p);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const size_t row_stride = (size_t)nb * Q4K_BYTES;
+    const uint32_t row_bytes = (uint32_t)nb * Q4K_BYTES;
     const gbytes_t wg = to_gbytes(gate) + (int64_t)e * m.slab_bytes, wu = to_gbytes(up) + (int64_t)e * m.slab_bytes;
     const gbytes_t act = to_gbytes(acts) + (size_t)(slot / m.topk) * nb * (256 * sizeof(float));
     float* dst = out + (size_t)slot * n;
     uint32_t flip = 0x80808080u;
     asm volatile("" : "+v"(flip));
     const bool odd = g.lane & 1;
-    RowFrag fg, fu;
-    auto load = [&](int row) {
-        const size_t at = (size_t)min(row, n - 1) * row_stride;
-        row_load(fg, wg + at, g.hdr_off, g.qs_off);
-        row_load(fu, wu + at, g.hdr_off, g.qs_off);
-    };
+    // the lane group's row of tile t, in bytes from the slab: 32 bits (the launcher sees to that), and it moves by the same step every time
     const int tiles = (n + RP - 1) / RP, step = (int)gridDim.x * waves;
     int t = (int)blockIdx.x * waves + wave;
+    const uint32_t last_at = (uint32_t)(n - 1) * row_bytes, step_at = (uint32_t)(step * RP) * row_bytes;
+    uint32_t row_at = (uint32_t)(t * RP + g.rp) * row_bytes;
+    RowFrag fg, fu;
+    auto load = [&] {
+        const uint32_t at = min(row_at, last_at), hdr = at + g.hdr_off, qs = at + g.qs_off;
+        const uint8_t *gate_p = (const uint8_t*)wg, *up_p = (const uint8_t*)wu;
+        fg.h = *(const uint4*)(gate_p + hdr);
+        fg.q0 = *(const uint4*)(gate_p + qs);
+        fg.q1 = *(const uint4*)(gate_p + qs + 16);
+        fu.h = *(const uint4*)(up_p + hdr);
+        fu.q0 = *(const uint4*)(up_p + qs);
+        fu.q1 = *(const uint4*)(up_p + qs + 16);
+    };
     Slice s[1];
-    slice_load<true, 1>(s, act, 0, nb, g.unit, g.valid, lds, [&] { load(min(t, tiles - 1) * RP + g.rp); });
+    slice_load<true, 1>(s, act, 0, nb, g.unit, g.valid, lds, load);
+    // Tile i of a batch waits in the i-th pair of lanes that group_sum2 defines: 0 1, 2 3, 8 9, 10 11 of each row of 16.
+    constexpr int SLOTS = Geo<RP>::GROUP / 4;
+    const int in_group = g.lane & (Geo<RP>::GROUP - 1);
+    const int my_slot = (in_group & 4) ? -1 : (in_group >> 4) * 4 + ((in_group >> 2) & 2) + ((in_group >> 1) & 1);
+    float kept = 0.f;
+    int first = t, held = 0;   // the batch's first tile, and how many it holds
     while (t < tiles) {
-        const int row = t * RP + g.rp;
         const float both = group_sum2<Geo<RP>::GROUP>(row_share(fg, s[0], sel, g.valid, flip), row_share(fu, s[0], sel, g.valid, flip), odd);
-        const float u = dpp_f32<0xB1>(both);   // the odd neighbour's total
-        if ((g.lane & (Geo<RP>::GROUP - 1)) == 0 && row < n) dst[row] = lk_gated(m.act, both, u, (size_t)e * n + row);
         t += step;
-        if (t < tiles) load(t * RP + g.rp);
+        row_at += step_at;
+        if (t < tiles) load();
+        kept = my_slot == held ? both : kept;
+        if (++held < SLOTS && t < tiles) continue;
+        const float u = dpp_f32<0xB1>(kept);   // the odd neighbour's total
+        const int row = (first + my_slot * step) * RP + g.rp;
+        if (!odd && my_slot >= 0 && my_slot < held && row < n) dst[row] = lk_gated(m.act, kept, u, (size_t)e * n + row);
+        first = t;
+        held = 0;
     }
 }
 
@@ -582,6 +607,10 @@ static int launch_moe_pair(const uint8_t* gate, const uint8_t* up, const float* 
     const int tiles = (n + RP - 1) / RP, need = (tiles + RW - 1) / RW;
     int share = lk_device().cus * (forced_per_cu > 0 ? forced_per_cu : 4) / m.pairs;
     if (share < 1) share = 1;
+    // The fewest workgroups that leave a wave as many tiles as `share` would: 32 pairs of 384 tiles go two to a wave over 24 workgroups a pair, where
+    // 32 would leave half the waves with one (four tokens, whole block 25.9 us against 24.3).
+    const int steps = (tiles + share * RW - 1) / (share * RW);
+    share = (tiles + steps * RW - 1) / (steps * RW);
     const dim3 grid(need < share ? need : share, m.pairs);
     hipLaunchKernelGGL((q4k_reg_moe_pair_kernel<RP>), grid, dim3(RT), 0, s, gate, up, acts, out, nb, n, m, RW);
     return lk_launch_status();
@@ -592,6 +621,8 @@ int lk_q4k_reg_moe_pair(const uint8_t* gate, const uint8_t* up, const float* act
                         int64_t slab_bytes, const LkGateAct& act, hipStream_t stream) {
     const int off = lk_tune_env("LK_TUNE_NO_REG_MOE");
     if (off || !lk_q4k_reg_serves(nb) || pairs < 1 || pairs > 65535 || n < 1) return -1;
+    // a row's offset in a slab is 32-bit, and so is a step's past the last (the grid steps by no more rows than a slab has, and a workgroup's)
+    if (((int64_t)n + 64) * nb * Q4K_BYTES > INT32_MAX) return -1;
     if ((((uintptr_t)gate) | ((uintptr_t)up) | ((uintptr_t)acts)) & 15) return -1;
     const RegMoeArgs m{sorted_token_ids, expert_ids, experts, topk, pairs, slab_bytes, act};
     switch (q4k_rows_per_pass(nb)) {

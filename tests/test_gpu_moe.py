@@ -287,6 +287,28 @@ TABLE_TAIL = {"q2_k": lib.TYPE_Q2_K, "q3_k": lib.TYPE_Q3_K, "q5_0": lib.TYPE_Q5_
               "q5_k": lib.TYPE_Q5_K}   # and Q5_K on the K-quant engine, short rows and long
 
 
+@pytest.mark.parametrize("hidden,ffn", [(256, 331), (1024, 129), (1024, 128), (2048, 331), (2048, 512), (2560, 331), (4096, 257)])
+def test_gated_launch_of_many_tiles_a_wave(hidden, ffn):
+    """1024 routed pairs leave a pair one workgroup, whose waves walk 4 to 42 tiles: more than, as many as and fewer than the
+    totals that wait in a wave's lanes at a time (4, 8 or 16 tiles of 4, 2 or 1 rows), and a last one cut by the row count."""
+    n_experts, topk, tokens = 3, 2, 512
+    gate = synth.weight(lib.TYPE_Q4_K, n_experts * ffn, hidden, seed=61, stream=1)
+    up = synth.weight(lib.TYPE_Q4_K, n_experts * ffn, hidden, seed=61, stream=2)
+    x = synth.activation(tokens, hidden, seed=61) * np.float32(4.0)
+    ids = np.stack([np.random.default_rng(t).choice(n_experts, topk, replace=False) for t in range(tokens)]).astype(np.int32)
+    got = moe_gemm_gguf_gate_up_silu_mul(lib.TYPE_Q4_K, dev(x), dev(gate), dev(up), ExpertRouting(dev(ids)), n_experts, ffn).cpu().numpy()
+    some = np.r_[0, 1, tokens // 2, tokens - 1]
+    g = oracle.ob_matmul(lib.TYPE_Q4_K, x[some], gate, n_experts * ffn).reshape(len(some), n_experts, ffn).astype(np.float64)
+    u = oracle.ob_matmul(lib.TYPE_Q4_K, x[some], up, n_experts * ffn).reshape(len(some), n_experts, ffn).astype(np.float64)
+    h = g / (1.0 + np.exp(-g)) * u
+    for i, t in enumerate(some):
+        for j in range(topk):
+            # 1e-3 of each factor, as the mat-vec's bound (1e-3 relative + 1e-4 absolute): both factors' errors add up, silu's slope is at most 1.1
+            e = ids[t, j]
+            bound = (1.1 * (1e-3 * np.abs(g[i, e]) + 1e-4)) * np.abs(u[i, e]) + np.abs(g[i, e]) * (1e-3 * np.abs(u[i, e]) + 1e-4) + 1e-6
+            assert (np.abs(got[t * topk + j] - h[i, e]) <= bound).all()
+
+
 @pytest.mark.parametrize("tokens,hidden,ffn,n_experts,topk", [(1, 1024, 768, 16, 4), (3, 512, 256, 6, 2), (2, 2560, 512, 4, 2)])
 @pytest.mark.parametrize("name", sorted(TABLE_TAIL))
 def test_per_pair_decode_block_in_the_tail_formats_matches_oracle(name, tokens, hidden, ffn, n_experts, topk):
