@@ -38,8 +38,12 @@ struct FmtLinear {
 };
 
 // What lane q (0..3) of a super-block loads, keeps of the activation and makes of the two.
-template <bool Q5>
+// IN_PLACE: Q4_K's high nibbles stay where they are (q4k_dots_biased), for a register more per super-block: with four
+// super-blocks 260 registers, one wave a SIMD, where the shifted form keeps two (60 experts of 1024 -> 1536, top-4, at
+// 3 / 5 / 8 / 20 tokens, the launch alone, weights from HBM: in place 7.6 / 8.2 / 10.4 / 15.7 us, shifted 6.4 / 6.8 / 8.3 / 13.4).
+template <bool Q5, bool IN_PLACE>
 struct LaneQ4K {
+    static_assert(!(Q5 && IN_PLACE), "Q5_K's codes are put together from two places");
     using Fmt = FmtLinear<2>;
     static constexpr int BYTES = Q5 ? Q5K_BYTES : Q4K_BYTES, QS0 = Q5 ? 48 : 16, ALIGN = 16;
     struct W {
@@ -47,8 +51,8 @@ struct LaneQ4K {
     };
     struct A {
         uint4 a00, a01, a10, a11;
-        float4 s4;     // Q4_K: the second d over 16 (q4k_dots_biased)
-        int hi_init;   // and what its high nibbles' dot starts from
+        float4 s4;     // IN_PLACE: the second d over 16
+        int hi_init;   // and what the high nibbles' dot starts from
     };
     static __device__ __forceinline__ void load(W& f, const uint8_t* bp, int q) {
         f.hdr = *(const uint4*)(bp);
@@ -66,7 +70,7 @@ struct LaneQ4K {
         a.a10 = *(const uint4*)(codes + 32);
         a.a11 = *(const uint4*)(codes + 48);
         a.s4 = *(const float4*)(rowl + table + (b * 8 + 2 * q) * 8);
-        if (!Q5) {
+        if (IN_PLACE) {
             const uint4 ones = make_uint4(0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u);
             a.hi_init = 128 * dot16(ones, a.a11, dot16(ones, a.a10, 0));
             a.s4.z *= 0.0625f;
@@ -81,6 +85,9 @@ struct LaneQ4K {
         if (Q5) {
             q5k_dots(f.q0, shr4(f.h0, 2 * q), a.a00, a.a10, d_lo, d_hi);
             q5k_dots(f.q1, shr4(f.h1, 2 * q), a.a01, a.a11, d_lo, d_hi);
+        } else if (!IN_PLACE) {
+            q4k_dots(f.q0, a.a00, a.a10, d_lo, d_hi);
+            q4k_dots(f.q1, a.a01, a.a11, d_lo, d_hi);
         } else {
             uint32_t flip = 0x80808080u;
             asm("" : "+v"(flip));   // in a register: the bit instruction takes no literal
@@ -329,13 +336,14 @@ int launch(const FoldCall& c, FoldDims d) {
     return lk_launch_status();
 }
 
-template <class L>
+// L4: the lane's form for rows of four super-blocks
+template <class L, class L4 = L>
 int launch_format(const FoldCall& c, const FoldDims& d, int nb) {
     const bool few = d.topk <= 4;
     switch (nb) {
         case 2: return few ? launch<L, 2, 4>(c, d) : launch<L, 2, 8>(c, d);
         case 3: return few ? launch<L, 3, 4>(c, d) : launch<L, 3, 8>(c, d);
-        case 4: return few ? launch<L, 4, 4>(c, d) : launch<L, 4, 8>(c, d);
+        case 4: return few ? launch<L4, 4, 4>(c, d) : launch<L4, 4, 8>(c, d);
         default: return -1;
     }
 }
@@ -346,7 +354,7 @@ int launch_format(const FoldCall& c, const FoldDims& d, int nb) {
 bool lk_moe_down_fold_serves(int quant_type, const float* inputs, const void* weights, bool sorted, int topk, int size_m, int size_k) {
     if (lk_tune_env("LK_TUNE_DOWN_FOLD_OFF") || (quant_type != 1 && quant_type != 4 && quant_type != 5)) return false;
     if ((size_k != 512 && size_k != 768 && size_k != 1024) || topk < 1 || topk > 8 || (sorted && size_m > MAX_PAIRS) || size_m % topk != 0) return false;
-    const int tokens = size_m / topk, align = quant_type == 5 ? LaneQ6K::ALIGN : LaneQ4K<false>::ALIGN;
+    const int tokens = size_m / topk, align = quant_type == 5 ? LaneQ6K::ALIGN : LaneQ4K<false, true>::ALIGN;
     return tokens >= 1 && tokens <= 65535 && ((uintptr_t)inputs & 15) == 0 && ((uintptr_t)weights & (align - 1)) == 0;
 }
 
@@ -362,8 +370,8 @@ int lk_moe_down_fold(int quant_type, const float* inputs, const void* weights, c
     const FoldCall c{(const uint8_t*)weights, inputs, sorted_token_ids, expert_ids, topk_weights, down_bias, add_after,
                      outputs, tokens, stream};
     switch (quant_type) {
-        case 1: return launch_format<LaneQ4K<false>>(c, d, size_k / 256);
-        case 4: return launch_format<LaneQ4K<true>>(c, d, size_k / 256);
+        case 1: return launch_format<LaneQ4K<false, true>, LaneQ4K<false, false>>(c, d, size_k / 256);
+        case 4: return launch_format<LaneQ4K<true, false>>(c, d, size_k / 256);
         case 5: return launch_format<LaneQ6K>(c, d, size_k / 256);
         default: return -1;
     }
