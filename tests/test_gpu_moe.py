@@ -575,6 +575,35 @@ def test_down_and_fold_in_one_launch_gives_the_bits_of_the_two_launches(name, to
     assert_close(one[0].cpu().numpy(), want, atol=1e-4 * max(1.0, np.abs(want).max()))
 
 
+@pytest.mark.parametrize("tokens,hidden,ffn,n_experts,topk", [(3, 331, 512, 6, 8), (2, 100, 768, 5, 4), (3, 331, 1024, 6, 4), (2, 203, 1024, 9, 8),
+                                                              (2, 1031, 768, 4, 3)])
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+def test_down_and_fold_over_several_passes_and_a_cut_last_workgroup(name, tokens, hidden, ffn, n_experts, topk, knobs):
+    """A workgroup takes 16 (up to four pairs a token) or 8 rows a pass and sums a row's pairs after its last one: one to sixteen
+    passes, odd counts, and rows that end inside a workgroup's first, middle or last pass, against the mat-vec per pair and the sum."""
+    dt = {"q4_k": lib.TYPE_Q4_K, "q5_k": lib.TYPE_Q5_K, "q6_k": lib.TYPE_Q6_K}[name]
+    down = dev(synth.weight(dt, n_experts * hidden, ffn, seed=65, stream=3))
+    ids = np.stack([np.arange(topk) % n_experts for _ in range(tokens)]).astype(np.int32)
+    ids = np.stack([np.random.default_rng(t).permutation(row) for t, row in enumerate(ids)])
+    w = synth.activation(tokens, topk, seed=65, stream=7)
+    h = dev(synth.activation(tokens * topk, ffn, seed=65, stream=4) * np.float32(5.0))
+    routing, w = ExpertRouting(dev(ids)), dev(w.reshape(-1))
+    bias = torch.randn((n_experts, hidden), device="cuda", generator=torch.Generator(device="cuda").manual_seed(11))
+    res = torch.randn((tokens, hidden), device="cuda", generator=torch.Generator(device="cuda").manual_seed(12))
+    kinds = ({}, {"residual": res}, {"add_after": res}, {"down_bias": bias}, {"down_bias": bias, "add_after": res})
+
+    def run():
+        return [moe_gemm_gguf_down_reduce(dt, h, down, routing, w, n_experts, hidden, **kw) for kw in kinds]
+
+    knobs.set("LK_TUNE_DOWN_FOLD_OFF")
+    want = run()
+    knobs.clear("LK_TUNE_DOWN_FOLD_OFF")
+    for passes in (1, 2, 3, 4, 7, 16):
+        knobs.set("LK_TUNE_DOWN_FOLD_PASSES", str(passes))
+        for got, two in zip(run(), want):
+            assert torch.equal(got, two), passes
+
+
 def test_pairs_the_routing_leaves_out_add_nothing():
     tokens, hidden, ffn, n_experts, topk = 3, 256, 256, 4, 2
     gate, up, down, x, ids, w = make_layer(tokens, hidden, ffn, n_experts, topk, seed=60)
