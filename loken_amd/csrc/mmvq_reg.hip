@@ -431,6 +431,10 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
 // fifth of a tile) runs once for up to GROUP / 4 tiles instead of once a tile for two lanes of it: 1290 -> 1078. Whole block of 128 experts of 2048 -> 768, top-8, weights
 // from HBM, before and after, with the grid's rule in launch_moe_pair: 4 / 9 / 12 tokens 27.0 / 58.7 / 54.0 us -> 24.8 / 57.2 / 53.7 (9: a Q6_K down), 60 experts of
 // 1536 -> 1024, top-4, at 12 tokens 35.0 -> 31.2; 16 tokens, which the weights' bytes bound, 59.0 -> 59.5.
+// ONE: no wave has more than one tile. Then there is nothing to step on to and nothing to wait for: no loop, a row's place
+// as a 64-bit product, the activation at once. The launch alone, weights from HBM, through the loop and without it: 60
+// experts of 1536 -> 1024, top-4, at 2 / 3 tokens 6.47 / 7.49 us, 6.05 / 7.08; 64 of 1024 -> 512, top-8, at 1 / 6 tokens
+// 4.02 / 6.74, 3.75 / 6.40; 128 of 2048 -> 768, top-8, at 2 tokens 9.68, 9.28.
 struct RegMoeArgs {
     const int32_t* sorted_token_ids;   // null: pair i is slot i
     const int32_t* expert_ids;
@@ -438,7 +442,7 @@ struct RegMoeArgs {
     int64_t slab_bytes;
     LkGateAct act;
 };
-template <int RP>
+template <int RP, bool ONE>
 __global__ __launch_bounds__(RT) void q4k_reg_moe_pair_kernel(const uint8_t* __restrict__ gate, const uint8_t* __restrict__ up,
                                                               const float* __restrict__ acts, float* __restrict__ out, int nb,
                                                               int n, RegMoeArgs m, int waves) {
@@ -459,12 +463,26 @@ __global__ __launch_bounds__(RT) void q4k_reg_moe_pair_kernel(const uint8_t* __r
     uint32_t flip = 0x80808080u;
     asm volatile("" : "+v"(flip));
     const bool odd = g.lane & 1;
-    // the lane group's row of tile t, in bytes from the slab: 32 bits (the launcher sees to that), and it moves by the same step every time
     const int tiles = (n + RP - 1) / RP, step = (int)gridDim.x * waves;
     int t = (int)blockIdx.x * waves + wave;
+    RowFrag fg, fu;
+    Slice s[1];
+    if (ONE) {
+        slice_load<true, 1>(s, act, 0, nb, g.unit, g.valid, lds, [&] {
+            const size_t at = (size_t)min(min(t, tiles - 1) * RP + g.rp, n - 1) * row_bytes;
+            row_load(fg, wg + at, g.hdr_off, g.qs_off);
+            row_load(fu, wu + at, g.hdr_off, g.qs_off);
+        });
+        if (t >= tiles) return;
+        const float both = group_sum2<Geo<RP>::GROUP>(row_share(fg, s[0], sel, g.valid, flip), row_share(fu, s[0], sel, g.valid, flip), odd);
+        const float u = dpp_f32<0xB1>(both);   // the odd neighbour's total
+        const int row = t * RP + g.rp;
+        if ((g.lane & (Geo<RP>::GROUP - 1)) == 0 && row < n) dst[row] = lk_gated(m.act, both, u, (size_t)e * n + row);
+        return;
+    }
+    // the lane group's row of tile t, in bytes from the slab: 32 bits (the launcher sees to that), and it moves by the same step every time
     const uint32_t last_at = (uint32_t)(n - 1) * row_bytes, step_at = (uint32_t)(step * RP) * row_bytes;
     uint32_t row_at = (uint32_t)(t * RP + g.rp) * row_bytes;
-    RowFrag fg, fu;
     auto load = [&] {
         const uint32_t at = min(row_at, last_at), hdr = at + g.hdr_off, qs = at + g.qs_off;
         const uint8_t *gate_p = (const uint8_t*)wg, *up_p = (const uint8_t*)wu;
@@ -475,7 +493,6 @@ __global__ __launch_bounds__(RT) void q4k_reg_moe_pair_kernel(const uint8_t* __r
         fu.q0 = *(const uint4*)(up_p + qs);
         fu.q1 = *(const uint4*)(up_p + qs + 16);
     };
-    Slice s[1];
     slice_load<true, 1>(s, act, 0, nb, g.unit, g.valid, lds, load);
     constexpr int SLOTS = Geo<RP>::GROUP / 4;
     const int my_slot = total_slot<RP>(g.lane);
@@ -617,7 +634,8 @@ static int launch_moe_pair(const uint8_t* gate, const uint8_t* up, const float* 
     const int steps = (tiles + share * RW - 1) / (share * RW);
     share = (tiles + steps * RW - 1) / (steps * RW);
     const dim3 grid(need < share ? need : share, m.pairs);
-    hipLaunchKernelGGL((q4k_reg_moe_pair_kernel<RP>), grid, dim3(RT), 0, s, gate, up, acts, out, nb, n, m, RW);
+    hipLaunchKernelGGL((steps == 1 ? q4k_reg_moe_pair_kernel<RP, true> : q4k_reg_moe_pair_kernel<RP, false>), grid, dim3(RT), 0, s, gate, up,
+                       acts, out, nb, n, m, RW);
     return lk_launch_status();
 }
 

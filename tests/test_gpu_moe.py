@@ -289,8 +289,8 @@ TABLE_TAIL = {"q2_k": lib.TYPE_Q2_K, "q3_k": lib.TYPE_Q3_K, "q5_0": lib.TYPE_Q5_
 
 @pytest.mark.parametrize("hidden,ffn", [(256, 331), (1024, 129), (1024, 128), (2048, 331), (2048, 512), (2560, 331), (4096, 257)])
 def test_gated_launch_of_many_tiles_a_wave(hidden, ffn):
-    """1024 routed pairs leave a pair one workgroup, whose waves walk 4 to 42 tiles: more than, as many as and fewer than the
-    totals that wait in a wave's lanes at a time (4, 8 or 16 tiles of 4, 2 or 1 rows), and a last one cut by the row count."""
+    """1024 routed pairs leave a pair one workgroup, whose waves walk 4 to 42 tiles: one or several times the totals that wait in a
+    wave's lanes at a time (4, 8 or 16 tiles of 4, 2 or 1 rows), a short last batch, and a last tile cut by the row count."""
     n_experts, topk, tokens = 3, 2, 512
     gate = synth.weight(lib.TYPE_Q4_K, n_experts * ffn, hidden, seed=61, stream=1)
     up = synth.weight(lib.TYPE_Q4_K, n_experts * ffn, hidden, seed=61, stream=2)
@@ -307,6 +307,37 @@ def test_gated_launch_of_many_tiles_a_wave(hidden, ffn):
             e = ids[t, j]
             bound = (1.1 * (1e-3 * np.abs(g[i, e]) + 1e-4)) * np.abs(u[i, e]) + np.abs(g[i, e]) * (1e-3 * np.abs(u[i, e]) + 1e-4) + 1e-6
             assert (np.abs(got[t * topk + j] - h[i, e]) <= bound).all()
+
+
+@pytest.mark.parametrize("hidden,rows", [(256, 4), (1024, 4), (1280, 2), (2048, 2), (2560, 1), (4096, 1)])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 17])
+def test_gated_register_launch_gives_the_bits_of_the_staged_one(hidden, rows, tiles, knobs):
+    """1024 routed pairs leave a pair one workgroup of eight waves, so that a wave walks the given number of tiles of `rows` rows: one
+    (a form of its own), fewer than the totals that wait in a wave's lanes at a time, and more; with the last wave cut and whole. The
+    biases are read at rows that the lanes rebuild, so every activation goes through both."""
+    from loken_amd.moe import (moe_gemm_gguf_gate_up_gelu_mul_concat, moe_gemm_gguf_gate_up_swiglu_limited,
+                               moe_gemm_gguf_gate_up_swiglu_oai)
+    n_experts, topk, tokens, dt = 3, 2, 512, lib.TYPE_Q4_K
+    x = dev(synth.activation(tokens, hidden, seed=66) * np.float32(4.0))
+    ids = np.stack([np.random.default_rng(t).choice(n_experts, topk, replace=False) for t in range(tokens)]).astype(np.int32)
+    routing = ExpertRouting(dev(ids))
+    for ffn in (8 * rows * tiles, 8 * rows * tiles - 1, 8 * rows * (tiles - 1) + 1):
+        gate, up = (dev(synth.weight(dt, n_experts * ffn, hidden, seed=66, stream=i)) for i in (1, 2))
+        both = dev(synth.weight(dt, n_experts * 2 * ffn, hidden, seed=66, stream=3))
+        gb, ub = (dev(synth.normal(66, i, n_experts * ffn).reshape(n_experts, ffn)) for i in (11, 12))
+
+        def run():
+            return [moe_gemm_gguf_gate_up_silu_mul(dt, x, gate, up, routing, n_experts, ffn),
+                    moe_gemm_gguf_gate_up_swiglu_oai(dt, x, gate, up, routing, n_experts, ffn, 1.702, 7.0, gb, ub),
+                    moe_gemm_gguf_gate_up_swiglu_limited(dt, x, gate, up, routing, n_experts, ffn, 5.0),
+                    moe_gemm_gguf_gate_up_gelu_mul_concat(dt, x, both, routing, n_experts, ffn)]
+
+        one = run()
+        knobs.set("LK_TUNE_NO_REG_MOE")
+        two = run()
+        knobs.clear("LK_TUNE_NO_REG_MOE")
+        for a, b in zip(one, two):
+            assert torch.equal(a, b), ffn
 
 
 @pytest.mark.parametrize("tokens,hidden,ffn,n_experts,topk", [(1, 1024, 768, 16, 4), (3, 512, 256, 6, 2), (2, 2560, 512, 4, 2)])
