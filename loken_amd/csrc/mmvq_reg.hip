@@ -644,8 +644,9 @@ int lk_q4k_reg_moe_pair(const uint8_t* gate, const uint8_t* up, const float* act
                         int64_t slab_bytes, const LkGateAct& act, hipStream_t stream) {
     const int off = lk_tune_env("LK_TUNE_NO_REG_MOE");
     if (off || !lk_q4k_reg_serves(nb) || pairs < 1 || pairs > 65535 || n < 1) return -1;
-    // a row's offset in a slab is 32-bit, and so is a step's past the last (the grid steps by no more rows than a slab has, and a workgroup's)
-    if (((int64_t)n + 64) * nb * Q4K_BYTES > INT32_MAX) return -1;
+    // A wave of several tiles keeps its rows' places in 32 bits without a sign (64 rows past the last cover a first tile that
+    // the grid deals beyond it). A slab of 4 GiB and more goes to the staged launch, which gives the same bits.
+    if (((int64_t)n + 64) * nb * Q4K_BYTES > (int64_t)UINT32_MAX) return -1;
     if ((((uintptr_t)gate) | ((uintptr_t)up) | ((uintptr_t)acts)) & 15) return -1;
     const RegMoeArgs m{sorted_token_ids, expert_ids, experts, topk, pairs, slab_bytes, act};
     switch (q4k_rows_per_pass(nb)) {

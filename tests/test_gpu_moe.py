@@ -340,6 +340,20 @@ def test_gated_register_launch_gives_the_bits_of_the_staged_one(hidden, rows, ti
             assert torch.equal(a, b), ffn
 
 
+@pytest.mark.parametrize("gib", [2.5, 4.5])
+def test_gated_launch_over_a_slab_of_more_than_31_and_than_32_bits(gib):
+    # 2.5 GiB an expert is the register launch's (offsets of 32 bits), 4.5 GiB the staged one's. A period of rows over and over:
+    # its outputs repeat.
+    hidden, period, dt = 4096, 4093, lib.TYPE_Q4_K
+    times = int(gib * 2**30) // (period * 16 * 144)
+    one_gate, one_up = (dev(synth.weight(dt, period, hidden, seed=67, stream=i)) for i in (1, 2))
+    x, routing = dev(synth.activation(1, hidden, seed=67) * np.float32(4.0)), ExpertRouting(dev(np.zeros((1, 1), np.int32)))
+    want = moe_gemm_gguf_gate_up_silu_mul(dt, x, one_gate, one_up, routing, 1, period)
+    gate, up = (w.reshape(-1).repeat(times) for w in (one_gate, one_up))
+    got = moe_gemm_gguf_gate_up_silu_mul(dt, x, gate, up, routing, 1, period * times)
+    assert torch.equal(got.reshape(times, period), want.expand(times, period))
+
+
 @pytest.mark.parametrize("tokens,hidden,ffn,n_experts,topk", [(1, 1024, 768, 16, 4), (3, 512, 256, 6, 2), (2, 2560, 512, 4, 2)])
 @pytest.mark.parametrize("name", sorted(TABLE_TAIL))
 def test_per_pair_decode_block_in_the_tail_formats_matches_oracle(name, tokens, hidden, ffn, n_experts, topk):
