@@ -388,6 +388,23 @@ def test_pair_launch_writes_the_quantizers_q8_1_of_its_own_f32_result(name, n, k
         assert torch.equal(got, want)
 
 
+# Q4_K at one row, and at two while the blocks of 32 rows fit a workgroup each (the last case is past that): a wave's totals wait by
+# activation row and pass, in one, two or four passes (rows of up to 4, 8 and 16 super-blocks), and a workgroup has one block or,
+# past 512, a second one.
+@pytest.mark.parametrize("n,k,b,act", [(6144, 2048, 1, "silu"), (6144, 2048, 2, "silu"), (96, 1280, 2, "gelu"), (64, 512, 2, "gelu"),
+                                       (8192, 1024, 2, "silu"), (96, 4096, 2, "silu"), (160, 2304, 2, "gelu"), (22400, 512, 1, "silu"),
+                                       (22400, 2048, 1, "gelu"), (16416, 4096, 1, "silu"), (22400, 1024, 2, "silu")])
+def test_q4_k_pair_launch_q8_1_by_rows_and_passes(n, k, b, act, knobs):
+    gate, up = (dev(synth.weight(lib.TYPE_Q4_K, n, k, seed=72, stream=i)) for i in (1, 2))
+    x = dev(synth.activation(b, k, seed=72))
+    q = ops.quantize_q8_1_rows(x)
+    want = ops.quantize_q8_1_rows(ops.mmvq_pair_act(lib.TYPE_Q4_K, gate, up, q, k, n, act=act), k_padded=n)
+    got = [ops.mmvq_pair_act_q8_1(lib.TYPE_Q4_K, gate, up, src, k, n, act=act) for src in (x, q)]
+    knobs.set("LK_TUNE_NO_REG")   # the staged engine's launch
+    got.append(ops.mmvq_pair_act_q8_1(lib.TYPE_Q4_K, gate, up, q, k, n, act=act))
+    assert all(torch.equal(g, want) for g in got)
+
+
 def test_pair_q8_1_launch_declines_partial_blocks():
     gate = dev(synth.weight(lib.TYPE_Q4_K, 40, 256, seed=71))
     x = dev(synth.activation(1, 256, seed=71))
