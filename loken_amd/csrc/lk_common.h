@@ -131,11 +131,11 @@ static __device__ __forceinline__ void lk_store_q8_1_block_by_lane(float x, int 
 }
 
 // Two values at once: the even lanes of a group return the group's sum of `x0`, the odd lanes that
-// of `x1`, each with the additions of group_sum in the same order as far as lanes 0 .. 3 and 8 .. 11 of the
-// group's rows of 16 are concerned, the only lanes whose result is defined (the first step hands every lane its
-// neighbour's value of the row it keeps, the later steps move by even distances only: rotations by 4
-// and 8 inside a row of 16, so lane 0 adds (Q0 + Q1) + (Q2 + Q3) over the row's quads as
-// group_sum's mirrors do, and lane 8 (Q2 + Q3) + (Q0 + Q1)).
+// of `x1`, each with the additions of group_sum in the same order as far as lanes 0 .. 3 and 8 .. 11
+// of the group's rows of 16 are concerned, the only lanes whose result is defined (the first step
+// hands every lane its neighbour's value of the row it keeps, the later steps move by even distances
+// only: rotations by 4 and 8 inside a row of 16, so lane 0 adds (Q0 + Q1) + (Q2 + Q3) over the row's
+// quads as group_sum's mirrors do, and lane 8 (Q2 + Q3) + (Q0 + Q1)).
 template <int LANES>
 static __device__ __forceinline__ float group_sum2(float x0, float x1, bool odd) {
     const float keep = odd ? x1 : x0, send = odd ? x0 : x1;

@@ -186,7 +186,8 @@ struct Geo {
     }
 };
 
-// Total i of a lane group waits in the i-th pair of lanes that group_sum2 defines: 0 1, 2 3, 8 9, 10 11 of each row of 16. The lane's i, or -1.
+// Total i of a lane group waits in the i-th pair of lanes that group_sum2 defines: 0 1, 2 3, 8 9, 10 11 of each row of 16.
+// The lane's i, or -1.
 template <int RP>
 static __device__ __forceinline__ int total_slot(int lane) {
     const int at = lane & (Geo<RP>::GROUP - 1);
@@ -375,8 +376,9 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
         for (int i = 0; i < D; ++i) load_pass(i, min(b, blocks - 1), i);
     });
     int half = 0;
-    // The passes' totals wait in lanes of their own (total_slot), so that the activation runs once a block and not ahead of every pass's loads: five
-    // layers' launches of a decode step, weights from HBM, Llama-3-8B at one row 186.8 us -> 185.6, Qwen3-1.7B at one and two 100.6 -> 100.1, 119.0 -> 117.0.
+    // The passes' totals wait in lanes of their own (total_slot), so that the activation runs once a block and not ahead of
+    // every pass's loads. Five layers' launches of a decode step, weights from HBM: Llama-3-8B at one row 186.8 us -> 185.6,
+    // Qwen3-1.7B at one and two rows 100.6 -> 100.1, 119.0 -> 117.0.
     const int my_slot = total_slot<RP>(g.lane), my_r = my_slot / PASSES, my_pass = my_slot % PASSES;
     static_assert(B * PASSES <= Geo<RP>::GROUP / 4, "lanes for the totals");
     for (; b < blocks; b += gridDim.x) {
@@ -394,8 +396,8 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
             else if (nb_next < blocks) load_pass(i % D, nb_next, i + D - PASSES);
         }
         const float u = dpp_f32<0xB1>(kept);   // the odd neighbour's total
-        const float value = (act_fn == 0 ? act_silu(kept) : act_gelu_tanh(kept)) * u;
-        if (!odd && my_slot >= 0 && my_slot < B * PASSES) meet[(my_r * 2 + half) * 32 + 4 * wave + my_pass * RP + g.rp] = value;
+        const float gated = (act_fn == 0 ? act_silu(kept) : act_gelu_tanh(kept)) * u;
+        if (!odd && my_slot >= 0 && my_slot < B * PASSES) meet[(my_r * 2 + half) * 32 + 4 * wave + my_pass * RP + g.rp] = gated;
         __syncthreads();   // every wave of the workgroup has delivered its four
         if (wave == 0 && g.lane < 8 * B) {
             const int l8 = g.lane & 7, r = g.lane >> 3;
@@ -424,13 +426,15 @@ __global__ __launch_bounds__(RT) void q4k_reg_pair_kernel(const uint8_t* __restr
 // The gate / up pair per routed (token, expert) pair of an MoE layer: grid.y names the pair, whose
 // expert picks the two slabs, whose token picks the f32 activation row and whose slot picks the
 // output row (the conventions of loken_moe_gemm_gguf_gate_up_silu_mul, cuda/moe/moe_gguf.cu:896-1060
-// of the reference). Everything else is the pair kernel above, but for two things, because this launch is bound by vector
-// issue (sixteen tokens, 128 pairs of 768 x 2048: four workgroups on every CU, the vector unit active 80 % of the time, a
-// wave's six tiles 1290 instructions): a row's place is a 32-bit offset from the slab, where 64-bit products were sixteen issue
-// slots a tile, and a tile's totals wait in lanes of their own, so that the activation (an exponential and a division, a
-// fifth of a tile) runs once for up to GROUP / 4 tiles instead of once a tile for two lanes of it: 1290 -> 1078. Whole block of 128 experts of 2048 -> 768, top-8, weights
-// from HBM, before and after, with the grid's rule in launch_moe_pair: 4 / 9 / 12 tokens 27.0 / 58.7 / 54.0 us -> 24.8 / 57.2 / 53.7 (9: a Q6_K down), 60 experts of
-// 1536 -> 1024, top-4, at 12 tokens 35.0 -> 31.2; 16 tokens, which the weights' bytes bound, 59.0 -> 59.5.
+// of the reference). Everything else is the pair kernel above, but for two things where a wave has several tiles: a row's
+// place is a 32-bit offset from the slab, where 64-bit products were sixteen issue slots a tile, and a tile's totals wait in
+// lanes of their own, so that the activation (an exponential and a division, a fifth of a tile) runs once for up to
+// GROUP / 4 tiles instead of once a tile for two lanes of it. At sixteen tokens of 128 experts of 2048 -> 768, top-8, a
+// wave's six tiles are 1290 vector instructions without the two and 1078 with them, the vector unit is active 80 and 67 %
+// of the time, and the launch takes 30.6 and 29.4 us: issue alone is not what bounds it there. With the grid's rule in
+// launch_moe_pair, the launch alone, weights from HBM, neither / the rule / the two things / all: 128 experts, 4 tokens
+// 12.9 / 11.8 / 12.7 / 11.7 us, 8 tokens 19.1 / 19.1 / 18.8 / 18.8, 14 tokens 34.4 / 26.2 / 34.7 / 25.6; 60 of
+// 1536 -> 1024, top-4, 12 tokens 18.0 / 14.4 / 17.4 / 13.6; 32 of 3072 -> 1536, top-4, 10 tokens 36.8 / 32.0 / 34.7 / 29.7.
 // ONE: no wave has more than one tile. Then there is nothing to step on to and nothing to wait for: no loop, a row's place
 // as a 64-bit product, the activation at once. The launch alone, weights from HBM, through the loop and without it: 60
 // experts of 1536 -> 1024, top-4, at 2 / 3 tokens 6.47 / 7.49 us, 6.05 / 7.08; 64 of 1024 -> 512, top-8, at 1 / 6 tokens
@@ -480,7 +484,7 @@ __global__ __launch_bounds__(RT) void q4k_reg_moe_pair_kernel(const uint8_t* __r
         if ((g.lane & (Geo<RP>::GROUP - 1)) == 0 && row < n) dst[row] = lk_gated(m.act, both, u, (size_t)e * n + row);
         return;
     }
-    // the lane group's row of tile t, in bytes from the slab: 32 bits (the launcher sees to that), and it moves by the same step every time
+    // the lane group's row of tile t, in bytes from the slab: 32 bits (the launcher sees to that), by the same step every time
     const uint32_t last_at = (uint32_t)(n - 1) * row_bytes, step_at = (uint32_t)(step * RP) * row_bytes;
     uint32_t row_at = (uint32_t)(t * RP + g.rp) * row_bytes;
     auto load = [&] {
@@ -626,14 +630,16 @@ template <int RP>
 static int launch_moe_pair(const uint8_t* gate, const uint8_t* up, const float* acts, float* out, int nb, int n,
                            const RegMoeArgs& m, hipStream_t s) {
     const int forced_per_cu = lk_tune_env("LK_TUNE_REG_MOE_PER_CU");
-    const int tiles = (n + RP - 1) / RP, need = (tiles + RW - 1) / RW;
+    const int tiles = (n + RP - 1) / RP;
     int share = lk_device().cus * (forced_per_cu > 0 ? forced_per_cu : 4) / m.pairs;
     if (share < 1) share = 1;
-    // The fewest workgroups that leave a wave as many tiles as `share` would: 32 pairs of 384 tiles go two to a wave over 24 workgroups a pair, where
-    // 32 would leave half the waves with one (four tokens, whole block 25.9 us against 24.3).
+    // The fewest workgroups that leave a wave as many tiles as `share` would: 32 pairs of 384 tiles go two to a wave over 24
+    // workgroups a pair, where 32 would leave half the waves with one. Of 49 launches of 2 to 160 pairs, weights from HBM, 22
+    // are 3 to 26 % faster by it (24 pairs of those tiles, 42 workgroups a pair -> 24: 12.5 us -> 11.6), 25 level, and two
+    // slower (18 pairs of 2560 -> 1280 12.9 us -> 13.5, 36 pairs of 2304 -> 1024 18.9 -> 19.5).
     const int steps = (tiles + share * RW - 1) / (share * RW);
     share = (tiles + steps * RW - 1) / (steps * RW);
-    const dim3 grid(need < share ? need : share, m.pairs);
+    const dim3 grid(share, m.pairs);
     hipLaunchKernelGGL((steps == 1 ? q4k_reg_moe_pair_kernel<RP, true> : q4k_reg_moe_pair_kernel<RP, false>), grid, dim3(RT), 0, s, gate, up,
                        acts, out, nb, n, m, RW);
     return lk_launch_status();

@@ -13,13 +13,14 @@
 // (r, j, q) of a wave then holds, for the whole launch, the Q8_1 codes of quarter q of every
 // super-block of activation row j in registers, and per pass loads the matching quarter of weight
 // row r of expert e_j: 4 lanes per (row, expert), 4 * TKP lanes per output row. The four lanes'
-// shares meet over DPP, the topk pair totals are weighted and wait in LDS, and at the end a lane sums a row's in slot order,
-// exactly the order of the fold kernel, and stores the output element. No scratch, no atomics, and
-// the same bits as the two launches give.
+// shares meet over DPP, the topk pair totals are weighted and wait in LDS, and at the end a lane sums
+// a row's in slot order, exactly the order of the fold kernel, and stores the output element. No
+// scratch, no atomics, and the same bits as the two launches give.
 //
-// What bounds it: vector issue (sixteen tokens of 768 -> 2048, top-8: two workgroups a CU, the vector unit active 70 % of the time). Hence the
-// totals' way through LDS and Q4_K's high nibbles left in place (q4k_dots_biased): 2985 vector instructions a wave -> 2527, the launch 18.2 us -> 15.3
-// with the weights in a cache, the whole block with them from HBM 59.5 -> 58.5, at 20 tokens 78.9 -> 76.7.
+// What bounds it: vector issue with the weights in a cache (sixteen tokens of 768 -> 2048, top-8: two
+// workgroups a CU, the vector unit active 69 % of the time). Hence the totals' way through LDS and
+// Q4_K's high nibbles left in place (q4k_dots_biased): 2985 vector instructions a wave -> 2527, the
+// unit active 67 %, 18.2 us -> 15.3; with the weights from HBM 20.4 -> 19.3, at 20 tokens 28.5 -> 25.5.
 
 #include "mmvq_core.h"
 
